@@ -563,6 +563,24 @@ struct RingCfg {
   static_assert(A_INSTR == 4 && B_INSTR == 4, "load schedule assumes 4 + 4");
 };
 
+// Position of tile `rem` of an expert where its row tiles are many: 32
+// consecutive logical tiles (what an XCD holds at any moment) form a block of 8
+// row tiles x 4 column tiles: 12 operand panels for 32 tiles.  With the plain
+// order they would be 32 row tiles of one column tile: 33 panels, every row
+// panel fetched once per column tile.  Blocks follow each other along N, so the
+// next 32 tiles share the 8 row panels.  (8 row tiles: both orders are the
+// same.)  Leaves (tm, tn) alone where it does not apply.
+__device__ __forceinline__ void ring_tile_blocks(int rem, int tiles_m,
+                                                 int tiles_n, int& tm, int& tn) {
+  if (tiles_m > 8 && (tiles_m & 7) == 0 && (tiles_n & 3) == 0) {
+    const int sup = rem >> 5, within = rem & 31;
+    const int per_row = tiles_n >> 2;
+    const int sm = sup / per_row, sn = sup - sm * per_row;
+    tm = sm * 8 + (within & 7);
+    tn = sn * 4 + (within >> 3);
+  }
+}
+
 // GATHER: the rows of expert e's first operand are not A[e][r] but rows of a
 // shared token matrix, A[row_map[e * R + r]] (row_map < 0: the all-zero row
 // `zero_row`): the dispatch of the Mixture-of-Experts layer folded into the
@@ -620,7 +638,8 @@ struct RingCfg {
 static __device__ __attribute__((aligned(256))) bf16_t kmajor_zero_row[256];
 
 template <bool RELU, bool GATHER = false, bool KMAJOR = false,
-          bool MASKED = false, bool LISTED = false, bool TAILS = false>
+          bool MASKED = false, bool LISTED = false, bool TAILS = false,
+          bool SPLIT = false>
 __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
     bf16_t* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
@@ -629,7 +648,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const bf16_t* __restrict__ mask_src = nullptr,
     const int32_t* __restrict__ tile_list = nullptr,
     const int32_t* __restrict__ row_count = nullptr,
-    float mask_scale = 1.0f) {
+    float mask_scale = 1.0f, float* __restrict__ partial = nullptr,
+    int whole_tiles = 0, int split = 1) {
   using Cfg = RingCfg;
   // row_count [E], optional: KMAJOR kernels take it as the reduction extent
   // per expert (k_extent)
@@ -682,6 +702,9 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // (KMAJOR) the expert's first k_extent[e] reduction rows only
   int nk = KMAJOR ? (K + BK - 1) / BK : K / BK;
   bool tile_empty = false;   // k_extent[e] == 0: the result is zero
+  // SPLIT: first K tile of the current unit, and its place among the partial
+  // results (-1: the unit is a whole tile)
+  int kt0 = 0, unit = -1;
 
   // per-tile state
   int row0, col0;
@@ -698,20 +721,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int rem = logical - e * tiles_per_e;
     tn = rem / tiles_m;
     tm = rem - tn * tiles_m;
-    if (!LISTED && !TAILS && tiles_m > 8 && (tiles_m & 7) == 0 &&
-        (tiles_n & 3) == 0) {
-      // 32 consecutive logical tiles (what an XCD holds at any moment) form a
-      // block of 8 row tiles x 4 column tiles: 12 operand panels for 32 tiles.
-      // With the plain order and many row tiles they would be 32 row tiles of
-      // one column tile: 33 panels, every row panel fetched once per column
-      // tile.  Blocks follow each other along N, so the next 32 tiles share
-      // the 8 row panels.  (8 row tiles: both orders are the same.)
-      const int sup = rem >> 5, within = rem & 31;
-      const int per_row = tiles_n >> 2;
-      const int sm = sup / per_row, sn = sup - sm * per_row;
-      tm = sm * 8 + (within & 7);
-      tn = sn * 4 + (within >> 3);
-    }
+    if (!LISTED && !TAILS) ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
   };
   // GATHER: the slot -> token map entries of the four rows this lane loads in
   // a tile.  fetch_map issues the four loads back to back without waiting
@@ -733,6 +743,15 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     }
   };
   auto set_tile = [&](int logical) {
+    int part = 0;
+    if constexpr (SPLIT) {
+      unit = logical - whole_tiles;
+      if (unit >= 0) {
+        const int split_tiles = (total_tiles - whole_tiles) / split;
+        part = unit / split_tiles;
+        logical = whole_tiles + unit - part * split_tiles;
+      }
+    }
     int e, tm, tn;
     tile_coords(logical, e, tm, tn);
     if constexpr (TAILS) {
@@ -748,6 +767,23 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         const int used = k_extent[e];
         tile_empty = used == 0;
         nk = max(1, min((K + BK - 1) / BK, (used + BK - 1) / BK));
+      }
+    }
+    if constexpr (SPLIT) {
+      if (KMAJOR && k_extent == nullptr) nk = (K + BK - 1) / BK;
+      if constexpr (KMAJOR) {
+        if (k_extent == nullptr) tile_empty = false;
+      }
+      kt0 = 0;
+      if (unit >= 0) {
+        const int all = nk;
+        kt0 = (int)((int64_t)all * part / split);
+        nk = (int)((int64_t)all * (part + 1) / split) - kt0;
+        if (nk == 0) {     // fewer K tiles than parts
+          nk = 1;
+          kt0 = 0;
+          tile_empty = true;
+        }
       }
     }
     Ae = GATHER ? A : A + (int64_t)e * R * K;
@@ -785,12 +821,12 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // KMAJOR: load j of a tile fills reduction rows 2 (wave + WAVES j) and + 1
   // (lanes 32-63) of it; past the last reduction row they are zeros
   auto kmajor_past_end = [&](int kt, int j) {
-    return kt * BK + (wave + Cfg::WAVES * j) * 2 + (lane >> 5) >= K;
+    return (kt0 + kt) * BK + (wave + Cfg::WAVES * j) * 2 + (lane >> 5) >= K;
   };
   auto load_a = [&](int kt, int j) {
     const int slot = kt & 1;
     kt = min(kt, nk - 1);
-    const bf16_t* src = Ae + kt * (KMAJOR ? BK * R : BK) + a_off[j];
+    const bf16_t* src = Ae + (kt0 + kt) * (KMAJOR ? BK * R : BK) + a_off[j];
     if constexpr (KMAJOR) {
       if (kmajor_past_end(kt, j)) src = kmajor_zero_row + (lane & 31) * 8;
     }
@@ -801,7 +837,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   };
   auto load_b = [&](int kt, int slot, int j) {
     kt = min(kt, nk - 1);
-    const bf16_t* src = Be + kt * (KMAJOR ? BK * N : BK) + b_off[j];
+    const bf16_t* src = Be + (kt0 + kt) * (KMAJOR ? BK * N : BK) + b_off[j];
     if constexpr (KMAJOR) {
       if (kmajor_past_end(kt, j)) src = kmajor_zero_row + (lane & 31) * 8;
     }
@@ -1060,7 +1096,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     __syncthreads();
     const int out_row0 = row0, out_col0 = col0;
     bf16_t* out_c = Ce;
-    if constexpr (KMAJOR) {
+    const int out_unit = unit;
+    if constexpr (KMAJOR || SPLIT) {
       // an expert without reduction rows: its one K tile held rows that
       // nobody wrote
       if (tile_empty) {
@@ -1076,6 +1113,29 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       // the next tile's first loads fly while this tile is written out
       set_tile(next);
       prologue_head();
+    }
+    if constexpr (SPLIT) {
+      if (out_unit >= 0) {
+        // a part of a tile's reduction: the accumulators as they lie, 16
+        // bytes per lane and register group; split_reduce_kernel adds the
+        // parts and knows the layout
+        float* dst = partial + (int64_t)out_unit * (BM * BN) + tid * 4;
+#pragma unroll
+        for (int i = 0; i < Cfg::TM; ++i)
+#pragma unroll
+          for (int j = 0; j < Cfg::TN; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              *reinterpret_cast<float4*>(
+                  dst + ((i * Cfg::TN + j) * 4 + q) * (Cfg::THREADS * 4)) =
+                  make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
+                              acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        if (!has_next) break;
+        tile = next;
+        ++round;
+        prologue_tail();
+        continue;
+      }
     }
     // round (and relu), stage in LDS, coalesced 16-byte stores.  Nothing here
     // waits for vector memory: the next tile's first loads and this tile's
@@ -1161,6 +1221,53 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     ++round;
     prologue_tail();   // the staging area is free again
   }
+}
+
+// Sums the parts of the split tiles of a ring launch, in part order, rounds
+// once and writes the tiles.  One block per (tile, MFMA tile of the
+// wavefronts); the parts lie in accumulator order (see the kernel above).
+__global__ __launch_bounds__(RingCfg::THREADS) void split_reduce_kernel(
+    const float* __restrict__ partial, bf16_t* __restrict__ Cout, int R, int N,
+    int tiles_m, int tiles_n, int whole_tiles, int split_tiles, int split) {
+  using Cfg = RingCfg;
+  constexpr int GROUPS = Cfg::TM * Cfg::TN;
+  const int t = blockIdx.x / GROUPS, ij = blockIdx.x - t * GROUPS;
+  const int tiles_per_e = tiles_m * tiles_n;
+  const int logical = whole_tiles + t;
+  const int e = logical / tiles_per_e, rem = logical - e * tiles_per_e;
+  int tn = rem / tiles_m, tm = rem - tn * tiles_m;
+  ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
+  const int i = ij / Cfg::TN, j = ij - i * Cfg::TN;
+  float4 sum[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+  const float* src = partial + (int64_t)t * (Cfg::BM * Cfg::BN) +
+                     (int64_t)ij * 4 * (Cfg::THREADS * 4) + tid * 4;
+  const int64_t part_stride = (int64_t)split_tiles * (Cfg::BM * Cfg::BN);
+#pragma unroll 2
+  for (int p = 0; p < split; ++p, src += part_stride) {
+    float4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      v[q] = *reinterpret_cast<const float4*>(src + q * (Cfg::THREADS * 4));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      sum[q].x += v[q].x; sum[q].y += v[q].y;
+      sum[q].z += v[q].z; sum[q].w += v[q].w;
+    }
+  }
+  const int row = tm * Cfg::BM + wm * Cfg::WTM + i * 32 + (lane & 31);
+  const int col = tn * Cfg::BN + wn * Cfg::WTN + j * 32 + (lane >> 5) * 4;
+  if (row >= R) return;
+  bf16_t* dst = Cout + ((int64_t)e * R + row) * N + col;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (col + 8 * q < N)
+      *reinterpret_cast<uint2*>(dst + 8 * q) =
+          make_uint2(f32x2_to_bf16x2(sum[q].x, sum[q].y),
+                     f32x2_to_bf16x2(sum[q].z, sum[q].w));
 }
 
 // ---------------------------------------------------------------------------
@@ -1694,9 +1801,51 @@ static bool kmajor_path_applies(const void* A, const void* B, const void* C,
          (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
 }
 
+// A weight gradient of few tiles and a long reduction (a dense layer's: one
+// "expert", every token of the batch) leaves most compute units idle, each
+// busy one walking the whole reduction: the K tiles of the last, partly filled
+// round of tiles are then cut into `split` parts, which are units of work of
+// their own (SPLIT), and split_reduce_kernel adds the parts.  Measured for 768 x
+// 768 from 16000 rows (9 tiles of 250 K tiles), both launches: 277 us in one
+// part, 81 in 4, 46 in 10, 40 in 14 - 20, 42 in 28; 768 x 3072 (36 tiles): 275
+// in one, 97 in 4, 84 in 7.  The count comes from what these runs and those at
+// 512 x 512 x 4000 and 1024 x 4096 x 2000 fit: 1.15 us per K tile, 0.07 us per part (256
+// KB written and read back), 7 us for the second launch.
+struct SplitPlan {
+  int whole_tiles = 0;   // tiles computed whole, before the split ones
+  int split = 1;         // parts of each of the others (1: none is split)
+  size_t bytes = 0;      // scratch for the parts
+};
+static SplitPlan kmajor_split_plan(int E, int R, int N, int K) {
+  using Cfg = RingCfg;
+  SplitPlan plan;
+  const int64_t tiles = (int64_t)((R + Cfg::BM - 1) / Cfg::BM) *
+                        ((N + Cfg::BN - 1) / Cfg::BN) * E;
+  const int cus = compute_units();
+  if (cus == 0 || tiles > 0x7fffffffLL) return plan;
+  const int tail = (int)(tiles % cus), nk = (K + Cfg::BK - 1) / Cfg::BK;
+  if (tail == 0) return plan;
+  const double per_k_tile = 1.15, per_part = 0.07, second_launch = 7.0;
+  double best = nk * per_k_tile;
+  for (int split = 2; split * tail <= cus && split <= nk; ++split) {
+    const double cost = ((nk + split - 1) / split) * per_k_tile +
+                        split * tail * per_part + second_launch;
+    if (cost < best) {
+      best = cost;
+      plan.split = split;
+    }
+  }
+  if (plan.split == 1) return plan;
+  plan.whole_tiles = (int)tiles - tail;
+  plan.bytes = (size_t)tail * plan.split * Cfg::BM * Cfg::BN * sizeof(float);
+  return plan;
+}
+
+// scratch: kmajor_split_plan(...).bytes for the parts (null: nothing is split)
 static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
                               int E, int R, int N, int K, hipStream_t st,
-                              const int32_t* k_extent = nullptr) {
+                              const int32_t* k_extent = nullptr,
+                              void* scratch = nullptr) {
   using Cfg = RingCfg;
   const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
@@ -1706,11 +1855,32 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
   const int cus = compute_units();
   if (cus == 0) return MESH_MOE_E_HIP;
   const unsigned blocks = (unsigned)(tiles < cus ? tiles : cus);
+  const SplitPlan plan =
+      scratch == nullptr ? SplitPlan() : kmajor_split_plan(E, R, N, K);
+  if (plan.split > 1) {
+    const int tail = (int)tiles - plan.whole_tiles;
+    const int units = plan.whole_tiles + tail * plan.split;
+    // (a multiple of 8 blocks: the XCDs then hold runs of consecutive units,
+    // which share operand panels; blocks without a unit end at once)
+    const unsigned split_blocks = (unsigned)(units < cus ? (units + 7) & ~7 : cus);
+    auto k = grouped_gemm_bf16_ring_kernel<false, false, true, false, false,
+                                           false, true>;
+    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
+    k<<<split_blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
+        A, B, C, R, N, K, tiles_m, tiles_n, units, nullptr, nullptr, nullptr,
+        nullptr, k_extent, 1.0f, (float*)scratch, plan.whole_tiles, plan.split);
+    MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands, split)");
+    split_reduce_kernel<<<(unsigned)tail * Cfg::TM * Cfg::TN, Cfg::THREADS, 0,
+                          st>>>((const float*)scratch, C, R, N, tiles_m,
+                                tiles_n, plan.whole_tiles, tail, plan.split);
+    MOE_CHECK_LAUNCH("expert_ffn_backward (sum of the parts)");
+    return 0;
+  }
   auto k = grouped_gemm_bf16_ring_kernel<false, false, true>;
   MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
   k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
       A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-      nullptr, nullptr, k_extent, 1.0f);
+      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1);
   MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
   return 0;
 }
@@ -1738,7 +1908,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-        mask_src, tile_list, nullptr, mask_scale);
+        mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, listed tiles, masked result)");
     return 0;
   }
@@ -1750,7 +1920,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);                                          \
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(                           \
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,     \
-        nullptr, tile_list, nullptr, 1.0f);                                    \
+        nullptr, tile_list, nullptr, 1.0f, nullptr, 0, 1);                     \
   } while (0)
     if (row_map != nullptr) {
       if (relu) MOE_RING_LISTED(true, true);
@@ -1770,7 +1940,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-        mask_src, nullptr, nullptr, mask_scale);
+        mask_src, nullptr, nullptr, mask_scale, nullptr, 0, 1);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, masked result)");
     return 0;
   }
@@ -1784,7 +1954,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);                                          \
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(                           \
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,     \
-        nullptr, nullptr, nullptr, 1.0f);                                      \
+        nullptr, nullptr, nullptr, 1.0f, nullptr, 0, 1);                       \
   } while (0)
 #define MOE_RING_PLAIN_T(RELU_, GATHER_)                                       \
   do {                                                                         \
@@ -2401,7 +2571,10 @@ extern "C" size_t mesh_moe_expert_linear_backward_workspace_bytes(int E, int R,
                                                                   int K, int N,
                                                                   int dtype) {
   if (E < 1 || R < 1 || K < 1 || N < 1 || !valid_dtype(dtype)) return 0;
-  return ((size_t)E * R * K + (size_t)E * R * N) * dtype_size(dtype) + 2 * 256;
+  const size_t transposed =
+      ((size_t)E * R * K + (size_t)E * R * N) * dtype_size(dtype) + 2 * 256;
+  const size_t parts = kmajor_split_plan(E, K, N, R).bytes + 256;
+  return transposed > parts ? transposed : parts;
 }
 
 extern "C" int mesh_moe_expert_linear_backward(
@@ -2420,6 +2593,7 @@ extern "C" int mesh_moe_expert_linear_backward(
                                                                   dtype),
               MESH_MOE_E_ARG, "expert_linear_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
+  auto up = [](uintptr_t v) { return (v + 255) & ~(uintptr_t)255; };
   int rc;
   if (da != nullptr) {
     // da = dy . w^T  (w in its variable layout [E, K, N] is K-contiguous here);
@@ -2437,9 +2611,9 @@ extern "C" int mesh_moe_expert_linear_backward(
   // dw [E, K, N] = a^T . dy: the reduction runs over the rows of both operands
   if (kmajor_path_applies(a, dy, dw, K, N, R, dtype))
     return launch_ring_kmajor((const bf16_t*)a, (const bf16_t*)dy, (bf16_t*)dw,
-                              E, K, N, R, st);
+                              E, K, N, R, st, nullptr,
+                              (void*)up((uintptr_t)workspace));
   const size_t es = dtype_size(dtype);
-  auto up = [](uintptr_t v) { return (v + 255) & ~(uintptr_t)255; };
   unsigned char* tr_a = (unsigned char*)up((uintptr_t)workspace);
   unsigned char* tr_dy =
       (unsigned char*)up((uintptr_t)(tr_a + (size_t)E * R * K * es));
@@ -2465,7 +2639,13 @@ extern "C" size_t mesh_moe_expert_ffn_backward_workspace_bytes(int E, int R,
                                                                int dtype) {
   if (E < 1 || R < 1 || M < 1 || H < 1 || N < 1 || !valid_dtype(dtype))
     return 0;
-  return ffn_backward_elems(E, R, M, H, N) * dtype_size(dtype) + 3 * 256;
+  const size_t p1 = kmajor_split_plan(E, H, N, R).bytes;
+  const size_t p2 = kmajor_split_plan(E, M, H, R).bytes;
+  const size_t hidden = (size_t)E * R * H * dtype_size(dtype);
+  const size_t parts = hidden + (p1 > p2 ? p1 : p2) + 2 * 256;
+  const size_t transposed =
+      ffn_backward_elems(E, R, M, H, N) * dtype_size(dtype) + 3 * 256;
+  return transposed > parts ? transposed : parts;
 }
 
 extern "C" int mesh_moe_expert_ffn_backward(
@@ -2533,11 +2713,12 @@ extern "C" int mesh_moe_expert_ffn_backward(
   // reduction runs over token rows, the outermost index of both operands
   if (kmajor_path_applies(h, dy, dwo, H, N, R, dtype) &&
       kmajor_path_applies(expert_in, dh, dwi, M, H, R, dtype)) {
+    // (the parts of split reductions lie behind dh)
     rc = launch_ring_kmajor((const bf16_t*)h, (const bf16_t*)dy, (bf16_t*)dwo,
-                            E, H, N, R, st);
+                            E, H, N, R, st, nullptr, tr_h);
     if (rc != 0) return rc;
     return launch_ring_kmajor((const bf16_t*)expert_in, (const bf16_t*)dh,
-                              (bf16_t*)dwi, E, M, H, R, st);
+                              (bf16_t*)dwi, E, M, H, R, st, nullptr, tr_h);
   }
   // otherwise: both operands transposed to token-contiguous copies first
   rc = mesh_moe_pack_weights(h, tr_h, E, R, H, dtype, dtype, stream);

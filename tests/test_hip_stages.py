@@ -1388,6 +1388,30 @@ def test_expert_linear_many_row_tiles(hip, shape):
                                atol=1e-2 * float(wnt.abs().max()), err_msg=name)
 
 
+@pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
+                                   (2, 6144, 776, 256), (29, 3000, 520, 760)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_of_split_reductions(hip, shape):
+  """Weight gradients whose last round of tiles is cut into parts along the
+  reduction (few tiles, many rows; the last shape has whole tiles before the
+  split ones; row counts that leave part of a K tile, edges of the output
+  inside a tile).  The bound: one bf16 rounding, and for each of the two
+  float32 sums of R products R / 2 ulps of the sum of magnitudes."""
+  e, rows, k, n = shape
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(shape))
+  a, dy, w = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16)
+              for s in ((e, rows, k), (e, rows, n), (e, k, n)))
+  dw = hip.expert_linear_backward(a, dy, w, want_da=False)[1]
+  assert torch.equal(dw, hip.expert_linear_backward(a, dy, w, want_da=False)[1])
+  for i in range(0, e, max(1, e // 3)):
+    at = a[i].float().t().contiguous()
+    want = at @ dy[i].float()
+    magnitude = at.abs() @ dy[i].float().abs()
+    bound = 2.0 ** -8 * want.abs() + rows * 2.0 ** -24 * magnitude
+    assert bool(((dw[i].float() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(2, 256, 512, 128), (1, 100, 72, 40),
                                    (1, 4096, 1024, 256)],
