@@ -1172,6 +1172,31 @@ def test_block_backward_entries(hip, act_dtype):
                                rtol=1e-5 if act_dtype == "float32" else 2e-2)
 
 
+@pytest.mark.parametrize("rows,m", [(37, 8), (700, 768), (33, 1000), (9, 2056),
+                                    (2049, 520), (5, 4088)])
+def test_rms_norm_backward_widths(hip, rows, m):
+  """bf16 rows that end inside the 512 columns of a wavefront's load, against
+  float64.  Bounds: dx one bf16 rounding of a value whose float32 terms are
+  sums of m products; dscale one rounding and a float32 sum over the rows."""
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(rows + m)
+  x, dy = (torch.randn((rows, m), generator=gen, device="cuda").bfloat16()
+           for _ in range(2))
+  scale = (1 + 0.2 * torch.randn(m, generator=gen, device="cuda")).bfloat16()
+  dx, ds = hip.rms_norm_backward(x, scale, dy)
+  eps = float(torch.tensor(1e-6, dtype=torch.bfloat16))
+  xd, g = x.double(), dy.double() * scale.double()
+  r = (xd.square().mean(-1, keepdim=True) + eps).rsqrt()
+  want_dx = r * g - xd * r ** 3 * (g * xd).mean(-1, keepdim=True)
+  terms = (r * g).abs() + xd.abs() * r ** 3 * (g * xd).abs().mean(-1, keepdim=True)
+  assert bool(((dx.double() - want_dx).abs()
+               <= 2.0 ** -8 * want_dx.abs() + m * 2.0 ** -23 * terms).all())
+  want_ds = (dy.double() * xd * r).sum(0)
+  magnitude = (dy.double() * xd * r).abs().sum(0)
+  assert bool(((ds.double() - want_ds).abs() <= 2.0 ** -8 * want_ds.abs()
+               + (rows + m) * 2.0 ** -23 * magnitude).all())
+
+
 @pytest.mark.parametrize("bsz,length,heads,d,causal", [
     (1, 8, 1, 64, True), (2, 72, 2, 64, False), (1, 200, 3, 128, True),
     (1, 328, 2, 128, False), (2, 256, 2, 64, True), (1, 776, 1, 128, True),
