@@ -341,9 +341,11 @@ __global__ __launch_bounds__(256) void dispatch_backward_router4_kernel(
 // float32 (over the kernel rows, which are no longer needed) so that the
 // second phase -- half a wavefront per token row, 16 bytes per lane, the rows
 // of d(expert_in) added -- reads and writes whole rows.  The rows' loads are
-// issued before the first phase, whose latency they hide.  KS = E / 16.
-// Needs M % 256 == 0, E % 16 == 0, E <= DBM_MAX_E, S % 32 == 0 (the 32 tokens
-// share a group).
+// issued before the first phase, whose latency they hide.  KS = E / 16 rounded
+// up (the experts past E count as zeros).
+// Needs M % 8 == 0, E % 8 == 0, E <= DBM_MAX_E and 32 tokens of one router
+// (S * groups_per_router a multiple of 32, or one router for all).  9000 x
+// 768, 16 experts: 12 us, dispatch_backward_router4_kernel 25.
 constexpr int DBM_TOK = 32, DBM_COLS = 256, DBM_MAX_E = 128;
 constexpr int DBM_LD = DBM_COLS + 4;     // floats per LDS row of the share
 typedef __attribute__((ext_vector_type(8))) __bf16 dbm_bf16x8_t;
@@ -352,6 +354,7 @@ typedef uint32_t dbm_u32x4_t __attribute__((ext_vector_type(4)));
 
 // LDS bytes: [kernel rows | share] then the d(logits) rows
 static size_t dbm_lds_bytes(int E) {
+  E = (E + 15) / 16 * 16;
   const size_t wbytes = (size_t)DBM_COLS * (E * 2 + 16);
   const size_t sbytes = sizeof(float) * DBM_TOK * DBM_LD;
   return (wbytes > sbytes ? wbytes : sbytes) + (size_t)DBM_TOK * (E * 4 + 16);
@@ -376,12 +379,12 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
     const bf16_t* __restrict__ dxe, const int32_t* __restrict__ idx,
     const int32_t* __restrict__ pos, const float* __restrict__ gate,
     const uint8_t* __restrict__ kept, const float* __restrict__ dlogits,
-    const bf16_t* __restrict__ wg, bf16_t* __restrict__ dx, int G, int S,
+    const bf16_t* __restrict__ wg, bf16_t* __restrict__ dx, int G, int S, int E,
     int C, int M, int64_t T_tokens, int groups_per_router,
     const int32_t* __restrict__ row_offsets,
     const int16_t* __restrict__ tok_slot = nullptr) {
-  constexpr int E = KS * 16;
-  constexpr int WROW = E * 2 + 16, DROW = E * 4 + 16;   // padded LDS rows, bytes
+  constexpr int EP = KS * 16;                             // E, padded
+  constexpr int WROW = EP * 2 + 16, DROW = EP * 4 + 16;   // padded LDS rows, bytes
   constexpr int WBYTES = DBM_COLS * WROW;
   constexpr int SBYTES = (int)sizeof(float) * DBM_TOK * DBM_LD;
   extern __shared__ __attribute__((aligned(16))) unsigned char dbm_smem[];
@@ -392,12 +395,14 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
   const int half = lane >> 5, l32 = lane & 31;
   const int64_t t0 = (int64_t)blockIdx.y * DBM_TOK;
   const int m0 = blockIdx.x * DBM_COLS;
-  const int g = (int)(t0 / S);
-  wg += (int64_t)(g / groups_per_router) * M * E;
+  wg += (t0 / S / groups_per_router) * M * E;
+  // this lane's 8 columns of a token row (the last tile may reach past M)
+  const bool col_in = m0 + 8 * l32 < M;
+  const int col_at = col_in ? m0 + 8 * l32 : 0;
 
-  constexpr int WPR = E / 8;                  // 16-byte pieces per kernel row
-  constexpr int WP = DBM_COLS * WPR / 256;    // pieces per thread (= E / 8)
-  constexpr int DPR = E / 4;                  // pieces per d(logits) row
+  constexpr int WPR = EP / 8;                 // 16-byte pieces per kernel row
+  constexpr int WP = DBM_COLS * WPR / 256;    // pieces per thread (= EP / 8)
+  constexpr int DPR = EP / 4;                 // pieces per d(logits) row
   constexpr int DP = (DBM_TOK * DPR + 255) / 256;
   constexpr int RP = DBM_TOK / 8;
   const uint4 z = make_uint4(0, 0, 0, 0);
@@ -432,8 +437,10 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
   dbm_u32x4_t wv[WP];
 #pragma unroll
   for (int i = 0; i < WP; ++i) {
-    const uint4* src =
-        reinterpret_cast<const uint4*>(wg + (int64_t)m0 * E) + tid + 256 * i;
+    const int p = tid + 256 * i;
+    const int row = min(m0 + p / WPR, M - 1), piece = p % WPR;
+    const uint4* src = reinterpret_cast<const uint4*>(
+        wg + (int64_t)row * E + (piece * 8 < E ? piece * 8 : 0));
     asm volatile("global_load_dwordx4 %0, %1, off"
                  : "=&v"(wv[i]) : "v"(src) : "memory");
   }
@@ -442,8 +449,10 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
 #pragma unroll
   for (int i = 0; i < DP; ++i) {
     const int p = tid + 256 * i;
-    dv_used[i] = p < DBM_TOK * DPR && t0 + p / DPR < T_tokens;
-    dv[i] = reinterpret_cast<const float4*>(dlogits + t0 * E)[dv_used[i] ? p : 0];
+    dv_used[i] = p < DBM_TOK * DPR && t0 + p / DPR < T_tokens &&
+                 (p % DPR) * 4 < E;
+    dv[i] = *reinterpret_cast<const float4*>(
+        dlogits + t0 * E + (dv_used[i] ? (p / DPR) * E + (p % DPR) * 4 : 0));
   }
   __builtin_amdgcn_sched_barrier(0);
   // the rows this lane adds in phase 2: 8 columns from column 8 l32 of the tile
@@ -453,7 +462,10 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
   if constexpr (!SLOT) {
     int64_t base[RP][2];
 #pragma unroll
-    for (int j = 0; j < RP; ++j)
+    for (int j = 0; j < RP; ++j) {
+      int64_t t = t0 + wave * 8 + 2 * j + half;
+      t = t < T_tokens ? t : T_tokens - 1;
+      const int64_t g = t / S;
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int64_t e = k ? idx2[j].y : idx2[j].x;
@@ -462,6 +474,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
         else
           base[j][k] = (e * G + g) * C;
       }
+    }
 #pragma unroll
     for (int j = 0; j < RP; ++j) {
       const bool in_range = t0 + wave * 8 + 2 * j + half < T_tokens;
@@ -473,7 +486,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
         used |= (u ? 1u : 0u) << (2 * j + k);
         const int64_t slot = u ? base[j][k] + (k ? pos2[j].y : pos2[j].x) : 0;
         v[j][k] = load_streaming(
-            reinterpret_cast<const uint4*>(dxe + slot * M + m0) + l32);
+            reinterpret_cast<const uint4*>(dxe + slot * M + col_at));
       }
     }
   }
@@ -486,11 +499,15 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   else
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(2 * RP) : "memory");
+  // (the values pass through here so that nothing made from them moves up)
+#pragma unroll
+  for (int i = 0; i < WP; ++i) asm volatile("" : "+v"(wv[i]));
 #pragma unroll
   for (int i = 0; i < WP; ++i) {
     const int p = tid + 256 * i;
+    const dbm_u32x4_t zero = {0, 0, 0, 0};
     *reinterpret_cast<dbm_u32x4_t*>(wl + (p / WPR) * WROW + (p % WPR) * 16) =
-        wv[i];
+        (p % WPR) * 8 < E ? wv[i] : zero;
   }
 #pragma unroll
   for (int i = 0; i < DP; ++i) {
@@ -559,6 +576,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
       if constexpr (SLOT) {
         // this half-wavefront's token: lane l32 looks at experts l32, l32 + 32,
         // ..; the rows are added in expert order
+        const int64_t g = t / S;
 #pragma unroll
         for (int q = 0; q < 8; ++q) { a[q] = 0.f; b[q] = 0.f; }
         for (int e0 = 0; e0 < E; e0 += 32) {
@@ -571,7 +589,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
             const int64_t slot = ((int64_t)(e0 + el) * G + g) * C + cc;
             float r[8];
             unpack16(load_streaming(reinterpret_cast<const uint4*>(
-                         dxe + slot * M + m0) + l32), r, bf16_t());
+                         dxe + slot * M + col_at)), r, bf16_t());
 #pragma unroll
             for (int q = 0; q < 8; ++q) a[q] += r[q];
           }
@@ -588,8 +606,9 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
       const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
 #pragma unroll
       for (int q = 0; q < 8; ++q) o[q] = (a[q] + b[q]) + sv[q];
-      store_streaming(reinterpret_cast<uint4*>(dx + t * M + m0) + l32,
-                      pack16(o, bf16_t()));
+      if (col_in)
+        store_streaming(reinterpret_cast<uint4*>(dx + t * M + col_at),
+                        pack16(o, bf16_t()));
     }
   }
 }
@@ -639,14 +658,15 @@ __device__ __forceinline__ float gb_prob(float logit, float neglse, bool bf) {
 constexpr int GB_MAX_K = 8;
 
 template <typename IT>
-__global__ __launch_bounds__(256) void gate_count_kernel(
+__global__ __launch_bounds__(1024) void gate_count_kernel(
     GateBackwardParams p, const float* __restrict__ logits,
     const int32_t* __restrict__ idx, const IT* __restrict__ importance,
     int32_t* __restrict__ counts, float* __restrict__ n_one) {
   extern __shared__ int32_t cnt[];  // [E] + 1 + [E]
   int32_t* cnt2 = cnt + p.E + 1;    // second choices (second-place loss)
-  // block (g, chunk): its share of the group's tokens, added to the group's
-  // counters (zero before the launch) with integer-valued atomics
+  // block (g, chunk): its share of the group's tokens.  One block per group
+  // writes the group's counters; several add to them (zero before the launch)
+  // with integer-valued atomics.
   const int g = blockIdx.x;
   const int per = (p.S + gridDim.y - 1) / gridDim.y;
   const int s_lo = blockIdx.y * per, s_hi = min(p.S, s_lo + per);
@@ -697,12 +717,115 @@ __global__ __launch_bounds__(256) void gate_count_kernel(
       atomicAdd(&cnt2[idx[t * 2 + 1]], 1);
   }
   __syncthreads();
+  if (gridDim.y == 1) {
+    for (int e = threadIdx.x; e < p.E; e += blockDim.x) {
+      counts[(int64_t)g * p.E + e] = cnt[e];
+      counts[((int64_t)p.G + g) * p.E + e] = cnt2[e];
+    }
+    if (threadIdx.x == 0) n_one[g] = (float)cnt[p.E];
+    return;
+  }
   for (int e = threadIdx.x; e < p.E; e += blockDim.x) {
     if (cnt[e]) atomicAdd(&counts[(int64_t)g * p.E + e], cnt[e]);
     if (cnt2[e]) atomicAdd(&counts[((int64_t)p.G + g) * p.E + e], cnt2[e]);
   }
   if (threadIdx.x == 0 && cnt[p.E]) atomicAdd(&n_one[g], (float)cnt[p.E]);
 }
+
+// What a token's d(probabilities) are made of, beside the group's counts.
+template <typename IT>
+struct GateBackwardToken {
+  int i1, i2, router;
+  float m1;              // importance == 1
+  float add1, add2;      // d(p[i1]), d(p[i2]) from the gates
+  float coef;            // d(p[e]) = coef * counts[g,e] from the loss
+  bool loss2;
+  float coef2, rq, aq;   // second-place loss
+
+  __device__ __forceinline__ GateBackwardToken(
+      const GateBackwardParams& p, const float* row, const IT* importance,
+      const int32_t* idx, const uint8_t* kept, const float* dgate,
+      const float* d_loss, const float* n_one, int64_t t, int g, float neglse) {
+    const bool bf = p.softmax_bf16 != 0;
+    const int E = p.E, S = p.S;
+    router = p.router;
+    m1 = 1.0f;
+    if (importance != nullptr) {
+      const float imp = load_f32<IT>(importance + t);
+      m1 = (p.importance_from_slot_gate ? imp > 0.5f : imp == 1.0f) ? 1.0f : 0.0f;
+    }
+    const int2 id = *reinterpret_cast<const int2*>(idx + t * 2);
+    i1 = id.x;
+    i2 = id.y;
+    const float k1 = kept[t * 2] ? 1.0f : 0.0f, k2 = kept[t * 2 + 1] ? 1.0f : 0.0f;
+    const float mb =
+        p.num_microbatches > 1 ? (float)(1.0 / (double)p.num_microbatches) : 1.0f;
+    const float dl = d_loss[0] * p.loss_scale;
+    const float inv_s = (float)(1.0 / (double)S);
+    const float ee = (float)((double)E * (double)E);
+    add1 = add2 = 0.f;
+    if (router == 0) {
+      const float p1 = gb_prob(row[i1], neglse, bf);
+      const float p2 = gb_prob(row[i2], neglse, bf);
+      const float g1 = p1 * m1;
+      const float same = (i2 == i1) ? m1 : 0.0f;
+      const float g2 = p2 * (1.0f - same);
+      const float dg1n = dgate[t * 2] * k1, dg2n = dgate[t * 2 + 1] * k2;
+      const float rec = 1.0f / ((g1 + g2) + 1e-9f);
+      const float common = (dg1n * g1 + dg2n * g2) * rec * rec;
+      add1 = (dg1n * rec - common) * m1;
+      add2 = (dg2n * rec - common) * (1.0f - same);
+      // loss = mean_{g,e}(mean_s(p * m1) * density_1) * E^2, density = count / S
+      coef = dl * mb * ee * (float)(1.0 / ((double)p.G * (double)E)) * inv_s *
+             inv_s * m1;
+    } else {
+      // switch: the gate is the arg-max probability; ntlb: the probability of
+      // the candidate that took the token, and the loss averages over the
+      // top_k passes as well (moe.py:845-856)
+      add1 = dgate[t * 2] * k1 * m1;
+      const double terms =
+          (double)p.G * (double)E * (router == 2 ? (double)p.top_k : 1.0);
+      if (p.has_importance)
+        coef = dl * mb * ee * (float)(1.0 / (terms * (double)S)) * n_one[g] *
+               inv_s * inv_s;
+      else
+        coef = dl * mb * ee * (float)(1.0 / terms) * inv_s * inv_s;
+    }
+    // Second-place loss (moe.py:1426-1438): 0.5 * E^2 * mean_{g,e}(mean_s(n) *
+    // density_2) with n = q / (sum(q) + 1e-9), q = p * (1 - mask_1):
+    // d/dq[e] = c2[e] * rq - (sum_f c2[f] q[f]) * rq^2, c2 = coef2 * count_2.
+    loss2 = router == 0 && p.use_second_place_loss;
+    coef2 = rq = aq = 0.f;
+    if (loss2)
+      coef2 = dl * mb * 0.5f * ee * (float)(1.0 / ((double)p.G * (double)E)) *
+              inv_s * inv_s;
+  }
+  // q = sum(q), a = sum_f c2[f] q[f]
+  __device__ __forceinline__ void second_place(float q, float a) {
+    rq = 1.0f / (q + 1e-9f);
+    aq = a * rq * rq;
+  }
+  __device__ __forceinline__ float dprob(int e, int count, int count2) const {
+    float dp = coef * (float)count;
+    if (e == i1) dp += add1;
+    if (router == 0 && e == i2) dp += add2;
+    if (loss2)
+      dp += (e == i1 ? 1.0f - m1 : 1.0f) * (coef2 * (float)count2 * rq - aq);
+    return dp;
+  }
+  // d/dx of z_coef * sum(lse^2 * m1) / (n * microbatches)
+  __device__ __forceinline__ float z_factor(const GateBackwardParams& p,
+                                            const float* d_loss,
+                                            const float* n_one,
+                                            float lse) const {
+    if (!p.use_z_loss) return 0.f;
+    float n = 0.f;
+    for (int gg = 0; gg < p.G; ++gg) n += n_one[gg];
+    const float mbz = (float)(p.num_microbatches > 0 ? p.num_microbatches : 1);
+    return (d_loss[0] * p.loss_scale * p.z_loss_coef * 2.0f) * lse * m1 /
+           (n * mbz);
+  }
+};
 
 template <typename IT>
 __global__ __launch_bounds__(256) void gating_backward_kernel(
@@ -737,86 +860,27 @@ __global__ __launch_bounds__(256) void gating_backward_kernel(
   const bool bf = p.softmax_bf16 != 0;
   const float lse = gb_logsumexp(row, E, bf);
   const float neglse = -lse;
-  float m1 = 1.0f;
-  if (importance != nullptr) {
-    const float imp = load_f32<IT>(importance + t);
-    m1 = (p.importance_from_slot_gate ? imp > 0.5f : imp == 1.0f) ? 1.0f : 0.0f;
-  }
-  const int i1 = idx[t * 2], i2 = idx[t * 2 + 1];
-  const float k1 = kept[t * 2] ? 1.0f : 0.0f, k2 = kept[t * 2 + 1] ? 1.0f : 0.0f;
-  const float mb =
-      p.num_microbatches > 1 ? (float)(1.0 / (double)p.num_microbatches) : 1.0f;
-  const float dl = d_loss[0] * p.loss_scale;
-  const float inv_s = (float)(1.0 / (double)S);
-  const float ee = (float)((double)E * (double)E);
-  float add1 = 0.f, add2 = 0.f;  // d(p[i1]), d(p[i2]) from the gates
-  float coef;                    // d(p[e]) = coef * counts[g,e] from the loss
-  if (p.router == 0) {
-    const float p1 = gb_prob(row[i1], neglse, bf);
-    const float p2 = gb_prob(row[i2], neglse, bf);
-    const float g1 = p1 * m1;
-    const float same = (i2 == i1) ? m1 : 0.0f;
-    const float g2 = p2 * (1.0f - same);
-    const float dg1n = dgate[t * 2] * k1, dg2n = dgate[t * 2 + 1] * k2;
-    const float rec = 1.0f / ((g1 + g2) + 1e-9f);
-    const float common = (dg1n * g1 + dg2n * g2) * rec * rec;
-    add1 = (dg1n * rec - common) * m1;
-    add2 = (dg2n * rec - common) * (1.0f - same);
-    // loss = mean_{g,e}(mean_s(p * m1) * density_1) * E^2, density = count / S
-    coef = dl * mb * ee * (float)(1.0 / ((double)p.G * (double)E)) * inv_s *
-           inv_s * m1;
-  } else {
-    // switch: the gate is the arg-max probability; ntlb: the probability of
-    // the candidate that took the token, and the loss averages over the
-    // top_k passes as well (moe.py:845-856)
-    add1 = dgate[t * 2] * k1 * m1;
-    const double terms =
-        (double)p.G * (double)E * (p.router == 2 ? (double)p.top_k : 1.0);
-    if (p.has_importance)
-      coef = dl * mb * ee * (float)(1.0 / (terms * (double)S)) * n_one[g] *
-             inv_s * inv_s;
-    else
-      coef = dl * mb * ee * (float)(1.0 / terms) * inv_s * inv_s;
-  }
+  GateBackwardToken<IT> tok(p, row, importance, idx, kept, dgate, d_loss, n_one,
+                            t, g, neglse);
   const int32_t* cg = counts + (int64_t)g * E;
-  // Second-place loss (moe.py:1426-1438): 0.5 * E^2 * mean_{g,e}(mean_s(n) *
-  // density_2) with n = q / (sum(q) + 1e-9), q = p * (1 - mask_1):
-  // d/dq[e] = c2[e] * rq - (sum_f c2[f] q[f]) * rq^2, c2 = coef2 * count_2.
   const int32_t* cg2 = counts + ((int64_t)p.G + g) * E;
-  const bool loss2 = p.router == 0 && p.use_second_place_loss;
-  float coef2 = 0.f, rq = 0.f, aq = 0.f;
-  if (loss2) {
-    coef2 = dl * mb * 0.5f * ee * (float)(1.0 / ((double)p.G * (double)E)) *
-            inv_s * inv_s;
+  if (tok.loss2) {
     float q = 0.f, a = 0.f;
     for (int e = 0; e < E; ++e) {
       const float qe =
-          gb_prob(row[e], neglse, bf) * (e == i1 ? 1.0f - m1 : 1.0f);
+          gb_prob(row[e], neglse, bf) * (e == tok.i1 ? 1.0f - tok.m1 : 1.0f);
       q += qe;
-      a += coef2 * (float)cg2[e] * qe;
+      a += tok.coef2 * (float)cg2[e] * qe;
     }
-    rq = 1.0f / (q + 1e-9f);
-    aq = a * rq * rq;
+    tok.second_place(q, a);
   }
   auto dprob = [&](int e) {
-    float dp = coef * (float)cg[e];
-    if (e == i1) dp += add1;
-    if (p.router == 0 && e == i2) dp += add2;
-    if (loss2)
-      dp += (e == i1 ? 1.0f - m1 : 1.0f) * (coef2 * (float)cg2[e] * rq - aq);
-    return dp;
+    return tok.dprob(e, cg[e], tok.loss2 ? cg2[e] : 0);
   };
   // inner = sum_e p[e] * dp[e]
   float inner = 0.f;
   for (int e = 0; e < E; ++e) inner += gb_prob(row[e], neglse, bf) * dprob(e);
-  float zfac = 0.f;
-  if (p.use_z_loss) {  // d/dx of z_coef * sum(lse^2 * m1) / (n * microbatches)
-    float n = 0.f;
-    for (int gg = 0; gg < p.G; ++gg) n += n_one[gg];
-    const float mbz = (float)(p.num_microbatches > 0 ? p.num_microbatches : 1);
-    zfac = (d_loss[0] * p.loss_scale * p.z_loss_coef * 2.0f) * lse * m1 /
-           (n * mbz);
-  }
+  const float zfac = tok.z_factor(p, d_loss, n_one, lse);
   for (int e = 0; e < E; ++e) {
     const float pe = gb_prob(row[e], neglse, bf);
     out[e] = pe * (dprob(e) - inner) + zfac * pe;
@@ -830,28 +894,143 @@ __global__ __launch_bounds__(256) void gating_backward_kernel(
   }
 }
 
+// The same with four lanes per token, for E % 4 == 0 and E <= 4 PER: lane q of
+// a token's four holds `chunk` consecutive logits (a multiple of 4, so that
+// they are read and written 16 bytes at a time; the four lanes of a token
+// cover its row and 16 tokens per wavefront whole lines) and their
+// probabilities in registers, so that every probability is formed once and no
+// LDS is needed.  One thread per token has E dependent steps in each of four
+// passes and 1 / 4 of the wavefronts (32768 tokens, 64 experts: 69 us; this 14).
+template <typename IT, int PER>
+__global__ __launch_bounds__(256) void gating_backward_rows_kernel(
+    GateBackwardParams p, const float* __restrict__ logits,
+    const IT* __restrict__ importance, const int32_t* __restrict__ idx,
+    const uint8_t* __restrict__ kept, const float* __restrict__ dgate,
+    const float* __restrict__ d_loss, const int32_t* __restrict__ counts,
+    const float* __restrict__ n_one, float* __restrict__ dlogits, int chunk) {
+  const int E = p.E, S = p.S;
+  const int64_t T_tokens = (int64_t)p.G * p.S;
+  const int64_t t_at = (int64_t)blockIdx.x * 64 + (threadIdx.x >> 2);
+  // (lanes past the last token follow it, for the shuffles, and store nothing)
+  const int64_t t = t_at < T_tokens ? t_at : T_tokens - 1;
+  const int e0 = (threadIdx.x & 3) * chunk;
+  const int n = max(0, min(chunk, E - e0));      // a multiple of 4
+  const float* row = logits + t * E;
+  const int g = (int)(t / S);
+  float pr[PER];
+#pragma unroll
+  for (int i = 0; i < PER; i += 4) {
+    float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    if (i < n) v = *reinterpret_cast<const float4*>(row + e0 + i);
+    pr[i] = v.x; pr[i + 1] = v.y; pr[i + 2] = v.z; pr[i + 3] = v.w;
+  }
+  auto quad_sum = [](float v) {
+    v += __shfl_xor(v, 1);
+    return v + __shfl_xor(v, 2);
+  };
+  const bool bf = p.softmax_bf16 != 0;
+  float lse;
+  if (bf) {
+    // the roundings of the forward's sum depend on its order
+    lse = gb_logsumexp(row, E, true);
+  } else {
+    float m = pr[0];
+#pragma unroll
+    for (int i = 1; i < PER; ++i) m = fmaxf(m, pr[i]);
+    m = fmaxf(m, __shfl_xor(m, 1));
+    m = fmaxf(m, __shfl_xor(m, 2));
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) s += expf(pr[i] - m);
+    lse = logf(quad_sum(s)) + m;
+  }
+  const float neglse = -lse;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) pr[i] = i < n ? gb_prob(pr[i], neglse, bf) : 0.f;
+  GateBackwardToken<IT> tok(p, row, importance, idx, kept, dgate, d_loss, n_one,
+                            t, g, neglse);
+  const int32_t* cg = counts + (int64_t)g * E + e0;
+  const int32_t* cg2 = counts + ((int64_t)p.G + g) * E + e0;
+  if (tok.loss2) {
+    float q = 0.f, a = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (i < n) {
+        const float qe = pr[i] * (e0 + i == tok.i1 ? 1.0f - tok.m1 : 1.0f);
+        q += qe;
+        a += tok.coef2 * (float)cg2[i] * qe;
+      }
+    tok.second_place(quad_sum(q), quad_sum(a));
+  }
+  float inner = 0.f;
+  float dp[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    dp[i] = 0.f;
+    if (i < n)
+      dp[i] = tok.dprob(e0 + i, cg[i], tok.loss2 ? cg2[i] : 0);
+    inner += pr[i] * dp[i];
+  }
+  inner = quad_sum(inner);
+  const float zfac = tok.z_factor(p, d_loss, n_one, lse);
+  if (t_at >= T_tokens) return;
+  float* out = dlogits + t * E + e0;
+#pragma unroll
+  for (int i = 0; i < PER; i += 4)
+    if (i < n) {
+      float o[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        o[j] = pr[i + j] * (dp[i + j] - inner) + zfac * pr[i + j];
+      *reinterpret_cast<float4*>(out + i) = make_float4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 // ---------------------------------------------------------------------------
-// The same product on the float32 matrix cores (v_mfma_f32_32x32x2_f32: two
-// tokens per instruction, lanes 0-31 bring the first, lanes 32-63 the second;
-// x as the row operand, dlogits as the column operand, both read as they lie
-// in memory).  Block = 128 kernel rows x 64 experts x 512 tokens, 32 tokens
-// staged in LDS at a time as float32 (rows padded by 32 floats so that the two
-// half-waves hit different banks); a wavefront owns 32 rows x 64 experts.
-// Needs M % 128 == 0, E % 8 == 0 and 16-byte aligned rows.
+// dw[m,e] = sum_t x[t,m] * dlogits[t,e] on the float32 matrix cores
+// (v_mfma_f32_32x32x2_f32: two tokens per instruction, lanes 0-31 bring the
+// first, lanes 32-63 the second; x as the row operand, dlogits as the column
+// operand, both read as they lie in memory).  Block = 128 kernel rows x 64
+// experts x `chunk` tokens, 32 tokens staged in LDS at a time as float32 (rows
+// padded by 32 floats so that the two half-waves hit different banks); a
+// wavefront owns 32 rows x 64 experts.  The next 32 tokens are loaded while
+// the staged ones are multiplied.  Every block writes its sums to its token
+// chunk's [M, E] plane of the workspace and router_wgrad_reduce_kernel adds
+// the planes in chunk order: the same bits on every run.
+// Needs M % 4 == 0, E % 4 == 0 and 16-byte aligned rows.
+//
+// The product is short of blocks, not of bandwidth: 2048 tokens per block
+// left 30 blocks of 64 dependent steps for 9000 x 768 tokens and 16 experts
+// (bf16 kernel 79 us; 10 us in blocks of 96 tokens, sum of the planes 6).
+// 32768 x 1024, 64 experts: 82 -> 42 us; float32 2048 x 512, 8 experts: 32 + 10
+// us for clearing and converting -> 12 + 5.  router_wgrad_chunk() picks the tokens per block.
 // ---------------------------------------------------------------------------
-constexpr int WM_M = 128, WM_TOK = 512, WM_KT = 32;
+constexpr int WM_M = 128, WM_KT = 32;
 typedef float wm_f32x16_t __attribute__((ext_vector_type(16)));
 
-template <typename T>
+// Tokens per block of the two kernels below: about 512 blocks (two per compute
+// unit), but at least 4 E tokens (a plane of the workspace, 4 E bytes per
+// kernel row written and read, then stays below the tokens' own bytes) and
+// between 64 and 2048.
+static int router_wgrad_chunk(int64_t tokens, int M, int E) {
+  const int64_t tiles = (int64_t)((M + WM_M - 1) / WM_M) * ((E + 63) / 64);
+  const int64_t chunks = tiles >= 512 ? 1 : 512 / tiles;
+  int64_t tok = (tokens + chunks - 1) / chunks;
+  if (tok < 4 * E) tok = 4 * E;
+  if (tok < 64) tok = 64;
+  if (tok > 2048) tok = 2048;
+  return (int)((tok + WM_KT - 1) / WM_KT * WM_KT);
+}
+
 __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
-    const T* __restrict__ x, const float* __restrict__ dlogits,
-    float* __restrict__ acc_out, int64_t T_tokens, int M, int E) {
-  constexpr int VN = Vec16B<T>::N;            // elements per 16-byte piece
+    const float* __restrict__ x, const float* __restrict__ dlogits,
+    float* __restrict__ planes, int64_t T_tokens, int M, int E, int chunk) {
+  constexpr int VN = 4;                       // elements per 16-byte piece
   __shared__ float xs[WM_KT][WM_M + 32];
   __shared__ float ds[WM_KT][64 + 32];
   const int m0 = blockIdx.x * WM_M, e0 = blockIdx.z * 64;
-  const int64_t t0 = (int64_t)blockIdx.y * WM_TOK;
-  const int64_t t1 = t0 + WM_TOK < T_tokens ? t0 + WM_TOK : T_tokens;
+  const int64_t t0 = (int64_t)blockIdx.y * chunk;
+  const int64_t t1 = t0 + chunk < T_tokens ? t0 + chunk : T_tokens;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = lane >> 5, l32 = lane & 31;
   wm_f32x16_t acc0, acc1;
@@ -859,41 +1038,34 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
   for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
   // staging: thread -> (token row tid / 8, 16 kernel rows / 8 experts)
   const int sr = tid >> 3, sc = tid & 7;
-  for (int64_t tb = t0; tb < t1; tb += WM_KT) {
+  const uint4 z4 = make_uint4(0, 0, 0, 0);
+  uint4 xraw[16 / VN], draw[2];
+  auto load = [&](int64_t tb) {
     const int64_t t = tb + sr;
-    float xv[16], dv[8];
-    if (t < t1) {
-      const T* xp = x + t * M + m0 + sc * 16;
 #pragma unroll
-      for (int u = 0; u < 16 / VN; ++u) {
-        float f[VN];
-        unpack16(*reinterpret_cast<const uint4*>(xp + u * VN), f, T());
+    for (int u = 0; u < 16 / VN; ++u)
+      xraw[u] = t < t1 && m0 + sc * 16 + u * VN < M
+                    ? *reinterpret_cast<const uint4*>(x + t * M + m0 + sc * 16 +
+                                                      u * VN)
+                    : z4;
 #pragma unroll
-        for (int j = 0; j < VN; ++j) xv[u * VN + j] = f[j];
-      }
-      if (e0 + sc * 8 < E) {
-        const float4 a = *reinterpret_cast<const float4*>(dlogits + t * E + e0 + sc * 8);
-        const float4 b = *reinterpret_cast<const float4*>(dlogits + t * E + e0 + sc * 8 + 4);
-        dv[0] = a.x; dv[1] = a.y; dv[2] = a.z; dv[3] = a.w;
-        dv[4] = b.x; dv[5] = b.y; dv[6] = b.z; dv[7] = b.w;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) dv[j] = 0.f;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) xv[j] = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) dv[j] = 0.f;
-    }
+    for (int u = 0; u < 2; ++u)
+      draw[u] = t < t1 && e0 + sc * 8 + u * 4 < E
+                    ? *reinterpret_cast<const uint4*>(dlogits + t * E + e0 +
+                                                      sc * 8 + u * 4)
+                    : z4;
+  };
+  load(t0);
+  for (int64_t tb = t0; tb < t1; tb += WM_KT) {
     __syncthreads();                 // the previous batch has been consumed
 #pragma unroll
-    for (int j = 0; j < 16; j += 4)
-      *reinterpret_cast<float4*>(&xs[sr][sc * 16 + j]) =
-          make_float4(xv[j], xv[j + 1], xv[j + 2], xv[j + 3]);
-    *reinterpret_cast<float4*>(&ds[sr][sc * 8]) = make_float4(dv[0], dv[1], dv[2], dv[3]);
-    *reinterpret_cast<float4*>(&ds[sr][sc * 8 + 4]) = make_float4(dv[4], dv[5], dv[6], dv[7]);
+    for (int u = 0; u < 16 / VN; ++u)
+      *reinterpret_cast<uint4*>(&xs[sr][sc * 16 + u * VN]) = xraw[u];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      *reinterpret_cast<uint4*>(&ds[sr][sc * 8 + u * 4]) = draw[u];
     __syncthreads();
+    if (tb + WM_KT < t1) load(tb + WM_KT);
 #pragma unroll
     for (int ks = 0; ks < WM_KT / 2; ++ks) {
       const float a = xs[2 * ks + half][wave * 32 + l32];
@@ -903,12 +1075,13 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
       acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b1, acc1, 0, 0, 0);
     }
   }
+  float* part = planes + (int64_t)blockIdx.y * M * E;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int m = m0 + wave * 32 + 8 * (r / 4) + 4 * half + (r % 4);
-    if (e0 + l32 < E) atomicAdd(acc_out + (int64_t)m * E + e0 + l32, acc0[r]);
-    if (e0 + 32 + l32 < E)
-      atomicAdd(acc_out + (int64_t)m * E + e0 + 32 + l32, acc1[r]);
+    if (m >= M) continue;
+    if (e0 + l32 < E) part[(int64_t)m * E + e0 + l32] = acc0[r];
+    if (e0 + 32 + l32 < E) part[(int64_t)m * E + e0 + 32 + l32] = acc1[r];
   }
 }
 
@@ -923,15 +1096,12 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
 // operands (8 consecutive tokens of one kernel row / one expert per lane) are
 // read with ds_read_b64_tr_b16: within 16 lanes, lane t addresses the 8 bytes
 // at (row t / 4, elements 4 (t % 4) ..) of a 4 x 16 block and lane i receives
-// the block's column i.  Block = 128 kernel rows x 64 experts x WB_TOK tokens,
+// the block's column i.  Block = 128 kernel rows x 64 experts x `chunk` tokens,
 // 32 tokens staged at a time; a wavefront owns 32 rows x 64 experts.  Rows are
-// padded so that the four rows of a block lie in different banks.  Every
-// block writes its sums to its token chunk's [M, E] plane of the workspace
-// and router_wgrad_reduce_kernel adds the planes in chunk order: the same
-// bits on every run (the other kernels add with float atomics).
-// Needs M % 128 == 0, E % 8 == 0 and 16-byte aligned rows.
+// padded so that the four rows of a block lie in different banks.  Planes as
+// above; needs M % 8 == 0.
 // ---------------------------------------------------------------------------
-constexpr int WB_M = 128, WB_TOK = 2048, WB_KT = 32;
+constexpr int WB_M = WM_M, WB_KT = WM_KT;
 constexpr int WB_XS = (WB_M + 32) * 2;   // bytes per staged token row of x
 constexpr int WB_DS = (64 + 16) * 2;     // ... of one half of d(logits)
 typedef __attribute__((ext_vector_type(8))) __bf16 wb_bf16x8_t;
@@ -953,13 +1123,13 @@ __device__ __forceinline__ wb_bf16x8_t lds_read_tr8(uint32_t addr) {
 
 __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     const bf16_t* __restrict__ x, const float* __restrict__ dlogits,
-    float* __restrict__ acc_out, int64_t T_tokens, int M, int E) {
+    float* __restrict__ planes, int64_t T_tokens, int M, int E, int chunk) {
   __shared__ __attribute__((aligned(16))) unsigned char xs[WB_KT * WB_XS];
   __shared__ __attribute__((aligned(16))) unsigned char dhs[WB_KT * WB_DS];
   __shared__ __attribute__((aligned(16))) unsigned char dls[WB_KT * WB_DS];
   const int m0 = blockIdx.x * WB_M, e0 = blockIdx.z * 64;
-  const int64_t t0 = (int64_t)blockIdx.y * WB_TOK;
-  const int64_t t1 = t0 + WB_TOK < T_tokens ? t0 + WB_TOK : T_tokens;
+  const int64_t t0 = (int64_t)blockIdx.y * chunk;
+  const int64_t t1 = t0 + chunk < T_tokens ? t0 + chunk : T_tokens;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = lane >> 5, l32 = lane & 31;
   wm_f32x16_t acc0, acc1;
@@ -978,30 +1148,34 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
   const uint32_t la = (uint32_t)(size_t)(wb_lds_void_t*)dls + rrow * WB_DS +
                       rcol * 2;
   const uint4 z4 = make_uint4(0, 0, 0, 0);
-  for (int64_t tb = t0; tb < t1; tb += WB_KT) {
+  uint4 xv0, xv1, da, db;
+  auto load = [&](int64_t tb) {
     const int64_t t = tb + sr;
-    uint4 xv0 = z4, xv1 = z4, dh = z4, dl = z4;
-    if (t < t1) {
-      const uint4* xp = reinterpret_cast<const uint4*>(x + t * M + m0 + sc * 16);
-      xv0 = xp[0];
-      xv1 = xp[1];
-      if (e0 + sc * 8 < E) {
-        const float4 a = *reinterpret_cast<const float4*>(dlogits + t * E + e0 + sc * 8);
-        const float4 b = *reinterpret_cast<const float4*>(dlogits + t * E + e0 + sc * 8 + 4);
-        const float d[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        float lo[8];
+    const bool in = t < t1;
+    const int m = m0 + sc * 16, e = e0 + sc * 8;
+    const uint4* xp = reinterpret_cast<const uint4*>(x + t * M + m);
+    const uint4* dp = reinterpret_cast<const uint4*>(dlogits + t * E + e);
+    xv0 = in && m < M ? xp[0] : z4;
+    xv1 = in && m + 8 < M ? xp[1] : z4;
+    da = in && e < E ? dp[0] : z4;
+    db = in && e + 4 < E ? dp[1] : z4;
+  };
+  load(t0);
+  for (int64_t tb = t0; tb < t1; tb += WB_KT) {
+    const uint32_t dw[8] = {da.x, da.y, da.z, da.w, db.x, db.y, db.z, db.w};
+    float d[8], lo[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) lo[j] = d[j] - round_to<bf16_t>(d[j]);
-        dh = pack16(d, bf16_t());
-        dl = pack16(lo, bf16_t());
-      }
+    for (int j = 0; j < 8; ++j) {
+      d[j] = __uint_as_float(dw[j]);
+      lo[j] = d[j] - round_to<bf16_t>(d[j]);
     }
     __syncthreads();                 // the previous batch has been consumed
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32) = xv0;
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32 + 16) = xv1;
-    *reinterpret_cast<uint4*>(dhs + sr * WB_DS + sc * 16) = dh;
-    *reinterpret_cast<uint4*>(dls + sr * WB_DS + sc * 16) = dl;
+    *reinterpret_cast<uint4*>(dhs + sr * WB_DS + sc * 16) = pack16(d, bf16_t());
+    *reinterpret_cast<uint4*>(dls + sr * WB_DS + sc * 16) = pack16(lo, bf16_t());
     __syncthreads();
+    if (tb + WB_KT < t1) load(tb + WB_KT);
     // 16 tokens per step: the x operand and, per 32 experts, hi and lo
     const wb_bf16x8_t a0 = lds_read_tr8<0, 4 * WB_XS>(xa);
     const wb_bf16x8_t h00 = lds_read_tr8<0, 4 * WB_DS>(ha);
@@ -1026,11 +1200,11 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, l10, acc0, 0, 0, 0);
     acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, l11, acc1, 0, 0, 0);
   }
-  // this block's partial sums: chunk blockIdx.y of acc_out [chunks][M][E]
-  float* part = acc_out + (int64_t)blockIdx.y * M * E;
+  float* part = planes + (int64_t)blockIdx.y * M * E;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int m = m0 + wave * 32 + 8 * (r / 4) + 4 * half + (r % 4);
+    if (m >= M) continue;
     if (e0 + l32 < E) part[(int64_t)m * E + e0 + l32] = acc0[r];
     if (e0 + 32 + l32 < E) part[(int64_t)m * E + e0 + 32 + l32] = acc1[r];
   }
@@ -1044,7 +1218,15 @@ __global__ void router_wgrad_reduce_kernel(const float* __restrict__ part,
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float sum = 0.f;
-  for (int c = 0; c < chunks; ++c) sum += part[(int64_t)c * n + i];
+  int c = 0;
+  for (; c + 8 <= chunks; c += 8) {          // eight loads in flight
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)(c + u) * n + i];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += v[u];
+  }
+  for (; c < chunks; ++c) sum += part[(int64_t)c * n + i];
   store_f32<T>(dw + i, sum);
 }
 
@@ -1187,23 +1369,22 @@ bool launch_slot_dispatch_backward_mfma(
   *rc = 0;
   if (!(dtype == MESH_MOE_BF16 && dlogits != nullptr && w_gate != nullptr &&
         bw_aligned16(dexpert_in) && bw_aligned16(dx) && bw_aligned16(w_gate) &&
-        bw_aligned16(dlogits) && E % 16 == 0 && E <= DBM_MAX_E &&
-        M % DBM_COLS == 0 && S % DBM_TOK == 0 &&
-        (T_tokens + DBM_TOK - 1) / DBM_TOK <= 65535))
+        bw_aligned16(dlogits) && E % 8 == 0 && E <= DBM_MAX_E &&
+        M % 8 == 0 && (T_tokens + DBM_TOK - 1) / DBM_TOK <= 65535))
     return false;
-  dim3 grid((unsigned)(M / DBM_COLS),
+  dim3 grid((unsigned)((M + DBM_COLS - 1) / DBM_COLS),
             (unsigned)((T_tokens + DBM_TOK - 1) / DBM_TOK));
   const size_t lds = dbm_lds_bytes(E);
   auto run = [&](auto k) -> int {
     MOE_ALLOW_LDS(k, lds);
     k<<<grid, 256, lds, st>>>(
         (const bf16_t*)dexpert_in, nullptr, nullptr, nullptr, nullptr, dlogits,
-        (const bf16_t*)w_gate, (bf16_t*)dx, G, S, C, M, T_tokens, G, nullptr,
+        (const bf16_t*)w_gate, (bf16_t*)dx, G, S, E, C, M, T_tokens, G, nullptr,
         tok_slot);
     MOE_CHECK_LAUNCH("slot_dispatch_backward (router share on the matrix cores)");
     return 0;
   };
-  switch (E / 16) {
+  switch ((E + 15) / 16) {
     case 1: *rc = run(dispatch_backward_mfma_kernel<1, true>); break;
     case 2: *rc = run(dispatch_backward_mfma_kernel<2, true>); break;
     case 3: *rc = run(dispatch_backward_mfma_kernel<3, true>); break;
@@ -1342,10 +1523,11 @@ static int run_dispatch_backward(
   hipStream_t st = (hipStream_t)stream;
   if (vec && dlogits != nullptr && w_gate != nullptr &&
       dtype == MESH_MOE_BF16 && bw_aligned16(w_gate) &&
-      bw_aligned16(dlogits) && E % 16 == 0 && E <= DBM_MAX_E &&
-      M % DBM_COLS == 0 && S % DBM_TOK == 0 &&
+      bw_aligned16(dlogits) && E % 8 == 0 && E <= DBM_MAX_E && M % 8 == 0 &&
+      (groups_per_router == G ||
+       ((int64_t)groups_per_router * S) % DBM_TOK == 0) &&
       (T_tokens + DBM_TOK - 1) / DBM_TOK <= 65535) {
-    dim3 grid((unsigned)(M / DBM_COLS),
+    dim3 grid((unsigned)((M + DBM_COLS - 1) / DBM_COLS),
               (unsigned)((T_tokens + DBM_TOK - 1) / DBM_TOK));
     const size_t lds = dbm_lds_bytes(E);
 #define MOE_DBM(KS_)                                                         \
@@ -1356,10 +1538,10 @@ static int run_dispatch_backward(
     MOE_ALLOW_LDS(k, lds);                                                   \
     k<<<grid, 256, lds, st>>>(                                               \
         (const bf16_t*)dexpert_in, idx, pos, gate, kept, dlogits,            \
-        (const bf16_t*)w_gate, (bf16_t*)dx, G, S, C, M, T_tokens,            \
+        (const bf16_t*)w_gate, (bf16_t*)dx, G, S, E, C, M, T_tokens,         \
         groups_per_router, row_offsets, nullptr);                            \
   } while (0)
-    switch (E / 16) {
+    switch ((E + 15) / 16) {
       case 1: MOE_DBM(1); break;
       case 2: MOE_DBM(2); break;
       case 3: MOE_DBM(3); break;
@@ -1408,6 +1590,45 @@ extern "C" size_t mesh_moe_gating_backward_workspace_bytes(int G, int E) {
   return sizeof(int32_t) * 2 * (size_t)G * E + sizeof(float) * (size_t)G + 256;
 }
 
+template <typename IT>
+static int launch_gating_backward(
+    const GateBackwardParams& p, dim3 cgrid, unsigned cthreads, size_t smem,
+    const float* logits, const IT* importance, const int32_t* idx,
+    const uint8_t* kept, const float* dgate, const float* d_loss,
+    int32_t* counts, float* n_one, float* dlogits, hipStream_t st) {
+  gate_count_kernel<IT><<<cgrid, cthreads, smem, st>>>(p, logits, idx,
+                                                       importance, counts, n_one);
+  MOE_CHECK_LAUNCH("gating_backward (count)");
+  const int E = p.E;
+  const int64_t T_tokens = (int64_t)p.G * p.S;
+  if (E % 4 == 0 && E <= 128 && bw_aligned16(logits) && bw_aligned16(dlogits)) {
+    const int chunk = (E / 4 + 3) / 4 * 4;
+    const unsigned blocks = (unsigned)((T_tokens + 63) / 64);
+    auto run = [&](auto k) {
+      k<<<blocks, 256, 0, st>>>(p, logits, importance, idx, kept, dgate, d_loss,
+                                counts, n_one, dlogits, chunk);
+    };
+    if (chunk <= 4) run(gating_backward_rows_kernel<IT, 4>);
+    else if (chunk <= 8) run(gating_backward_rows_kernel<IT, 8>);
+    else if (chunk <= 16) run(gating_backward_rows_kernel<IT, 16>);
+    else run(gating_backward_rows_kernel<IT, 32>);
+    MOE_CHECK_LAUNCH("gating_backward (four lanes per token)");
+    return 0;
+  }
+  // rows through LDS where a block's rows fit: 256 threads up to 64 experts,
+  // 128 threads up to 128
+  const int staged = E <= 128;
+  const unsigned threads = (staged && E > 64) ? 128 : 256;
+  const size_t tile = staged ? sizeof(float) * threads * (E + 1) : 0;
+  auto k = gating_backward_kernel<IT>;
+  MOE_ALLOW_LDS(k, tile);
+  k<<<(unsigned)((T_tokens + threads - 1) / threads), threads, tile, st>>>(
+      p, logits, importance, idx, kept, dgate, d_loss, counts, n_one, dlogits,
+      staged);
+  MOE_CHECK_LAUNCH("gating_backward");
+  return 0;
+}
+
 extern "C" int mesh_moe_gating_backward(
     const float* logits, const void* importance, int importance_dtype,
     int importance_from_slot_gate, const int32_t* idx, const uint8_t* kept,
@@ -1452,53 +1673,43 @@ extern "C" int mesh_moe_gating_backward(
   const int64_t T_tokens = (int64_t)G * S;
   // rows through LDS where a block's rows fit: 256 threads up to 64 experts,
   // 128 threads up to 128
-  const int staged = E <= 128;
-  const unsigned gb_threads = (staged && E > 64) ? 128 : 256;
-  const size_t gb_smem = staged ? sizeof(float) * gb_threads * (E + 1) : 0;
-  const unsigned blocks =
-      (unsigned)((T_tokens + gb_threads - 1) / gb_threads);
-  // the counters (int32 counts, then float n_one: all-zero bits either way)
-  const int64_t n_cnt = 2 * (int64_t)G * E + G;
-  fill_f32_kernel<<<(unsigned)((n_cnt + 255) / 256 < 1024 ? (n_cnt + 255) / 256
-                                                          : 1024),
-                    256, 0, st>>>((float*)counts, n_cnt, 0.0f);
-  MOE_CHECK_LAUNCH("gating_backward (clear)");
-  // up to 16 blocks per group, 256 tokens or more each
-  const dim3 cgrid((unsigned)G, (unsigned)((S + 255) / 256 < 16 ? (S + 255) / 256
-                                                               : 16));
-  if (importance && importance_dtype == MESH_MOE_BF16) {
-    gate_count_kernel<bf16_t><<<cgrid, 256, smem, st>>>(
-        p, logits, idx, (const bf16_t*)importance, counts, n_one);
-    MOE_CHECK_LAUNCH("gating_backward (count)");
-    auto k = gating_backward_kernel<bf16_t>;
-    MOE_ALLOW_LDS(k, gb_smem);
-    k<<<blocks, gb_threads, gb_smem, st>>>(
-        p, logits, (const bf16_t*)importance, idx, kept, dgate, d_loss, counts,
-        n_one, dlogits, staged);
-  } else {
-    gate_count_kernel<float><<<cgrid, 256, smem, st>>>(
-        p, logits, idx, (const float*)importance, counts, n_one);
-    MOE_CHECK_LAUNCH("gating_backward (count)");
-    auto k = gating_backward_kernel<float>;
-    MOE_ALLOW_LDS(k, gb_smem);
-    k<<<blocks, gb_threads, gb_smem, st>>>(
-        p, logits, (const float*)importance, idx, kept, dgate, d_loss, counts,
-        n_one, dlogits, staged);
+  // Counting: one block per group.  (ntlb recomputes every token's candidates:
+  // up to 16 blocks per group, 256 tokens or more each.)
+  const unsigned chunks =
+      router == 2 ? (unsigned)((S + 255) / 256 < 16 ? (S + 255) / 256 : 16) : 1;
+  const unsigned cthreads =
+      router == 2 ? 256 : (unsigned)(S >= 1024 ? 1024 : (S + 63) / 64 * 64);
+  if (chunks > 1) {
+    // the counters (int32 counts, then float n_one: all-zero bits either way)
+    const int64_t n_cnt = 2 * (int64_t)G * E + G;
+    fill_f32_kernel<<<(unsigned)((n_cnt + 255) / 256 < 1024 ? (n_cnt + 255) / 256
+                                                            : 1024),
+                      256, 0, st>>>((float*)counts, n_cnt, 0.0f);
+    MOE_CHECK_LAUNCH("gating_backward (clear)");
   }
-  MOE_CHECK_LAUNCH("gating_backward");
-  return 0;
+  const dim3 cgrid((unsigned)G, chunks);
+  if (importance && importance_dtype == MESH_MOE_BF16)
+    return launch_gating_backward<bf16_t>(
+        p, cgrid, cthreads, smem, logits, (const bf16_t*)importance, idx, kept,
+        dgate, d_loss, counts, n_one, dlogits, st);
+  return launch_gating_backward<float>(
+      p, cgrid, cthreads, smem, logits, (const float*)importance, idx, kept,
+      dgate, d_loss, counts, n_one, dlogits, st);
 }
 
-static bool router_wgrad_bf16_applies(int64_t tokens, int M, int E, int dtype) {
-  return dtype == MESH_MOE_BF16 && ((size_t)M * 2) % 16 == 0 && E % 8 == 0 &&
-         M % WB_M == 0 && (tokens + WB_TOK - 1) / WB_TOK <= 65535;
+// the matrix-core kernels take the sizes (operands still have to be aligned)
+static bool router_wgrad_mfma_applies(int64_t tokens, int M, int E, int dtype) {
+  const int chunk = router_wgrad_chunk(tokens, M, E);
+  return ((size_t)M * dtype_size(dtype)) % 16 == 0 && E % 4 == 0 &&
+         (tokens + chunk - 1) / chunk <= 65535 && (E + 63) / 64 <= 65535;
 }
 
 extern "C" size_t mesh_moe_router_backward_weights_workspace_bytes(
     int64_t tokens, int M, int E, int dtype) {
   if (tokens < 1 || M < 1 || E < 1 || !valid_dtype(dtype)) return 0;
-  const size_t planes = router_wgrad_bf16_applies(tokens, M, E, dtype)
-                            ? (size_t)((tokens + WB_TOK - 1) / WB_TOK) : 1;
+  const int chunk = router_wgrad_chunk(tokens, M, E);
+  const size_t planes = router_wgrad_mfma_applies(tokens, M, E, dtype)
+                            ? (size_t)((tokens + chunk - 1) / chunk) : 1;
   return sizeof(float) * planes * (size_t)M * E;
 }
 
@@ -1522,21 +1733,31 @@ extern "C" int mesh_moe_router_backward_weights(const void* x,
               (long long)tokens);
   hipStream_t st = (hipStream_t)stream;
   const int64_t n = (int64_t)M * E;
-  const unsigned fb = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
-  if (router_wgrad_bf16_applies(tokens, M, E, dtype) && bw_aligned16(x) &&
-      bw_aligned16(dlogits)) {
-    const int bchunks = (int)((tokens + WB_TOK - 1) / WB_TOK);
-    dim3 bgrid((unsigned)(M / WB_M), (unsigned)bchunks,
-               (unsigned)((E + 63) / 64));
-    router_wgrad_bf16_kernel<<<bgrid, 256, 0, st>>>(
-        (const bf16_t*)x, dlogits, workspace, tokens, M, E);
-    MOE_CHECK_LAUNCH("router_backward_weights (mfma, bf16 terms)");
-    router_wgrad_reduce_kernel<bf16_t><<<(unsigned)((n + 255) / 256), 256, 0,
-                                         st>>>(workspace, (bf16_t*)dw_gate, n,
-                                               bchunks);
+  const bool aligned = bw_aligned16(x) && bw_aligned16(dlogits);
+  if (router_wgrad_mfma_applies(tokens, M, E, dtype) && aligned) {
+    const int chunk = router_wgrad_chunk(tokens, M, E);
+    const int planes = (int)((tokens + chunk - 1) / chunk);
+    const dim3 mgrid((unsigned)((M + WM_M - 1) / WM_M), (unsigned)planes,
+                     (unsigned)((E + 63) / 64));
+    const unsigned rb = (unsigned)((n + 255) / 256);
+    if (dtype == MESH_MOE_F32) {
+      router_wgrad_mfma_kernel<<<mgrid, 256, 0, st>>>(
+          (const float*)x, dlogits, workspace, tokens, M, E, chunk);
+      MOE_CHECK_LAUNCH("router_backward_weights (mfma)");
+      router_wgrad_reduce_kernel<float><<<rb, 256, 0, st>>>(
+          workspace, (float*)dw_gate, n, planes);
+    } else {
+      router_wgrad_bf16_kernel<<<mgrid, 256, 0, st>>>(
+          (const bf16_t*)x, dlogits, workspace, tokens, M, E, chunk);
+      MOE_CHECK_LAUNCH("router_backward_weights (mfma, bf16 terms)");
+      router_wgrad_reduce_kernel<bf16_t><<<rb, 256, 0, st>>>(
+          workspace, (bf16_t*)dw_gate, n, planes);
+    }
     MOE_CHECK_LAUNCH("router_backward_weights (sum of the chunks)");
     return 0;
   }
+  // other sizes and unaligned operands: float32 sums with atomics
+  const unsigned fb = (unsigned)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096);
   fill_f32_kernel<<<fb, 256, 0, st>>>(workspace, n, 0.0f);
   MOE_CHECK_LAUNCH("router_backward_weights (clear)");
   dim3 grid((unsigned)((M + WG_M - 1) / WG_M), (unsigned)chunks,
@@ -1544,29 +1765,7 @@ extern "C" int mesh_moe_router_backward_weights(const void* x,
   // 16-byte loads: rows of x and of dlogits start 16-byte aligned and hold
   // whole pieces
   const bool vec = ((size_t)M * dtype_size(dtype)) % 16 == 0 && E % 4 == 0 &&
-                   bw_aligned16(x) && bw_aligned16(dlogits);
-  if (vec && M % WM_M == 0 && E % 8 == 0) {
-    const int64_t mchunks = (tokens + WM_TOK - 1) / WM_TOK;
-    MOE_REQUIRE(mchunks <= 65535, MESH_MOE_E_UNSUPPORTED,
-                "router_backward_weights: too many tokens (%lld)",
-                (long long)tokens);
-    dim3 mgrid((unsigned)(M / WM_M), (unsigned)mchunks, (unsigned)((E + 63) / 64));
-    if (dtype == MESH_MOE_F32) {
-      router_wgrad_mfma_kernel<float><<<mgrid, 256, 0, st>>>(
-          (const float*)x, dlogits, workspace, tokens, M, E);
-      MOE_CHECK_LAUNCH("router_backward_weights (mfma)");
-      convert_f32_kernel<float><<<fb, 256, 0, st>>>(workspace, (float*)dw_gate, n);
-    } else {
-      // (unaligned bf16 operands: the float32 matrix cores)
-      router_wgrad_mfma_kernel<bf16_t><<<mgrid, 256, 0, st>>>(
-          (const bf16_t*)x, dlogits, workspace, tokens, M, E);
-      MOE_CHECK_LAUNCH("router_backward_weights (mfma)");
-      convert_f32_kernel<bf16_t><<<fb, 256, 0, st>>>(workspace, (bf16_t*)dw_gate,
-                                                    n);
-    }
-    MOE_CHECK_LAUNCH("router_backward_weights (convert)");
-    return 0;
-  }
+                   aligned;
   if (dtype == MESH_MOE_F32) {
     router_wgrad_kernel<float><<<grid, 256, 0, st>>>(
         (const float*)x, dlogits, workspace, tokens, M, E, vec);

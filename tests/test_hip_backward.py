@@ -364,6 +364,36 @@ def test_dispatch_backward_router_share_on_matrix_cores(hip, shape):
   assert float((step > 0).float().mean()) < 0.02
 
 
+@pytest.mark.parametrize("shape", [(3, 50, 776, 24, 5), (2, 100, 200, 8, 3),
+                                   (1, 33, 264, 40, 2), (5, 31, 1032, 120, 1)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_dispatch_backward_router_share_ragged_sizes(hip, shape):
+  """The same at sizes inside a tile of 32 tokens x 256 columns x 16 experts,
+  32 tokens that span groups included."""
+  test_dispatch_backward_router_share_on_matrix_cores(hip, shape)
+
+
+@pytest.mark.parametrize("case", [
+    ("top_2", 3, 50, 24, 40, 12, 1.25, "float32", True),
+    ("top_2", 2, 65, 16, 24, 68, 1.0, "float32", False),
+    ("switch", 2, 70, 16, 24, 24, 1.0, "float32", True),
+    ("switch_max", 1, 1030, 16, 24, 128, 1.0, "float32", True),
+    ("ntlb", 2, 96, 16, 24, 32, 1.0, "float32", True)],
+    ids=lambda c: "%s-%d" % (c[0], c[5]))
+def test_backward_expert_counts(hip, case):
+  """Numbers of experts around the 4, 8, 16 and 32 logits that a lane of the
+  gating backward holds, and a group longer than a block of its counting."""
+  test_backward_matches_oracle(hip, case)
+
+
+@pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("shape", [(63, 8, 4), (9001, 72, 12), (65, 1984, 68),
+                                   (4097, 136, 128)])
+def test_router_backward_weights_sizes(hip, shape, act_dtype):
+  """Kernel widths, expert counts and token chunks that end inside a tile."""
+  test_router_backward_weights(hip, shape, act_dtype)
+
+
 def test_full_size_router_terms_on_matrix_cores(hip):
   """Configuration 4's token count and widths (65536 tokens, d_model 4096, 64
   experts).  The router kernel's gradient from bfloat16 tokens (d(logits) as
