@@ -230,6 +230,103 @@ __global__ __launch_bounds__(256) void grouped_gemm_bf16_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// bf16 MFMA kernel for a few rows per expert (decoding steps, small batches):
+// the launch is a stream over the weights.
+//
+// A block owns 16 NT columns of one expert and all of its rows (MT tiles of 16);
+// its wavefronts cut the reduction into contiguous parts and add their sums in
+// LDS, in wavefront order.  Operands go from global memory to registers as the
+// instruction (16 x 16 x 32) wants them: lane l brings row l % 16, 16 bytes at k =
+// 8 (l / 16), i.e. 64-byte pieces of 16 rows per load.  That is a quarter of what
+// the load path can do for whole lines and four times what the weights need
+// (each weight byte is read by one block, once); the tokens come from the L2.
+// No LDS in the loop, no barrier: a wavefront has U (MT + NT) loads in flight.
+// 32 rows: 1024 x 1024 6.5 us, 1024 x 4096 6.9, 4096 x 1024 15.8; the 128 x 128
+// tile kernel, one block per 128 columns walking all of K: 20.4, 20.7, 69.9.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+template <int MT, int NT>
+__global__ __launch_bounds__(1024) void skinny_gemm_bf16_kernel(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+    bf16_t* __restrict__ C, int R, int N, int K, int groups_n, int relu) {
+  constexpr int U = MT <= 2 ? 4 : 2;       // k steps of 32 loaded together
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int waves = blockDim.x >> 6;
+  const int e = blockIdx.x / groups_n, n0 = (blockIdx.x - e * groups_n) * 16 * NT;
+  const int r16 = lane & 15, kq = (lane >> 4) * 8;
+  const bf16_t* bp[NT];
+  const bf16_t* ap[MT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    bp[j] = B + ((int64_t)e * N + min(n0 + 16 * j + r16, N - 1)) * K + kq;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    ap[i] = A + ((int64_t)e * R + min(16 * i + r16, R - 1)) * K + kq;
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[i][j][q] = 0.f;
+  const int steps = K / 32;
+  const int s1 = (int)((int64_t)steps * (wave + 1) / waves);
+  int s = (int)((int64_t)steps * wave / waves);
+  auto block_of = [&](auto u_tag) {
+    constexpr int UU = decltype(u_tag)::value;
+    bf16x8_t bf[UU][NT], af[UU][MT];
+#pragma unroll
+    for (int u = 0; u < UU; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        bf[u][j] = __builtin_nontemporal_load(
+            reinterpret_cast<const bf16x8_t*>(bp[j] + (s + u) * 32));
+#pragma unroll
+    for (int u = 0; u < UU; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        af[u][i] = *reinterpret_cast<const bf16x8_t*>(ap[i] + (s + u) * 32);
+#pragma unroll
+    for (int u = 0; u < UU; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              bf[u][j], af[u][i], acc[i][j], 0, 0, 0);
+    s += UU;
+  };
+  while (s + U <= s1) block_of(std::integral_constant<int, U>{});
+  while (s < s1) block_of(std::integral_constant<int, 1>{});
+  // lane: row 16 i + l % 16, columns 16 j + 4 (l / 16) ..
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(smem_raw);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      part[(wave * (MT * NT) + i * NT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  for (int t = wave; t < MT * NT; t += waves) {
+    f32x4_t sum = part[t * 64 + lane];
+    for (int w = 1; w < waves; ++w) {
+      const f32x4_t v = part[(w * (MT * NT) + t) * 64 + lane];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum[q] += v[q];
+    }
+    const int row = t / NT * 16 + r16, col = n0 + t % NT * 16 + (lane >> 4) * 4;
+    if (row < R && col < N) {
+      uint2 v;
+      v.x = pack2_bf16(sum[0], sum[1], relu != 0);
+      v.y = pack2_bf16(sum[2], sum[3], relu != 0);
+      *reinterpret_cast<uint2*>(C + ((int64_t)e * R + row) * N + col) = v;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // bf16 MFMA kernel with direct global -> LDS loads and an NS-stage ring.
 //
 // Same tiling and MFMA operand roles as the kernel above, but the K loop is fed
@@ -546,6 +643,152 @@ __device__ __forceinline__ void lds_read_tr16_pair(uint32_t addr, i16x4_t& lo,
                : "=v"(lo) : "v"(addr), "n"(OFF));
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
                : "=v"(hi) : "v"(addr), "n"(OFF + 2048));
+}
+
+// ---------------------------------------------------------------------------
+// bf16 MFMA kernel for few rows per expert and many experts (a decoding step's
+// experts): the launch is a stream over the weights, every byte of which one
+// block reads once.
+//
+// Block tile: all rows of an expert (MT tiles of 32) x 128 columns, K step 64,
+// 4 wavefronts of 32 columns each, direct-to-LDS loads (whole 128-byte lines,
+// the same swizzled LDS image as above) into a ring of NS slots: NS - 1 K
+// tiles in flight per block, two blocks per compute unit.  One barrier per K
+// tile: it publishes the oldest tile and frees the slot that the next loads go
+// to.
+//
+// row_map (optional, [E, R]): the slot -> token map.  An expert without an
+// occupied slot is left out, its rows of C unwritten (nothing reads them).
+// With `gather` row r of expert e is A[row_map[e, r]], zeros where that is
+// negative.
+//
+// 64 experts, 512 MB of weights: 4 rows each 89 - 93 us (5.8 - 6.0 TB/s), 32 rows
+// 100, 64 rows 107 (K = 1024) and 113 (K = 4096); the 128 x 128 register-staged
+// kernel before: 112 / 123 at 4 rows, 106 at 32, 110 / 130 at 64.  (8
+// wavefronts and 256 columns: the same at 4 rows, 121 / 106 at 64.  65 to 128
+// rows: 149 / 124 at 128 against 134 / 139 of the 128 x 128 kernel, which keeps
+// them.)
+// ---------------------------------------------------------------------------
+template <int MT>        // tiles of 32 rows
+struct StreamCfg {
+  static constexpr int BN = 128, BK = 64, ROW_BYTES = BK * 2;
+  static constexpr int A_BYTES = 32 * MT * ROW_BYTES, B_BYTES = BN * ROW_BYTES;
+  static constexpr int SLOT_BYTES = A_BYTES + B_BYTES;
+  static constexpr int NS = 80 * 1024 / SLOT_BYTES;
+  static constexpr size_t LDS_BYTES = (size_t)NS * SLOT_BYTES;
+  static constexpr int LOADS = MT + 4;     // per wavefront and K tile
+  static_assert(NS >= 3, "a ring");
+};
+
+template <int MT, bool MAPPED>
+__global__ __launch_bounds__(256) void stream_gemm_bf16_kernel(
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+    bf16_t* __restrict__ C, int R, int N, int K, int tiles_n, int relu,
+    const int32_t* __restrict__ row_map, int gather,
+    const bf16_t* __restrict__ zero_row) {
+  using Cfg = StreamCfg<MT>;
+  constexpr int BN = Cfg::BN, BK = Cfg::BK, NS = Cfg::NS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int e = blockIdx.x / tiles_n, tn = blockIdx.x - e * tiles_n;
+  const int col0 = tn * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bf16_t* asrc[MT];
+  const bf16_t* bsrc[4];
+  bool any = !MAPPED;
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int row = (wave + 4 * j) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ lds_swizzle(row);
+    const bf16_t* base = A + ((int64_t)e * R + min(row, R - 1)) * K;
+    if constexpr (MAPPED) {
+      const int src = row_map[(int64_t)e * R + min(row, R - 1)];
+      any |= src >= 0;
+      if (gather) base = src >= 0 ? A + (int64_t)src * K : zero_row;
+    }
+    asrc[j] = base + chunk * 8;
+  }
+  if constexpr (MAPPED) {
+    if (!__syncthreads_or(any)) return;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = (wave + 4 * j) * 8 + (lane >> 3);
+    const int chunk = (lane & 7) ^ lds_swizzle(row);
+    bsrc[j] = B + ((int64_t)e * N + min(col0 + row, N - 1)) * K + chunk * 8;
+  }
+  const int nk = K / BK;
+  // Blocks start their walk along K at different K tiles: rows of a weight
+  // matrix are a power of two apart in many models, and blocks in step would
+  // all read from the same few memory channels (64 experts of 1024 x 4096, 4
+  // rows: 113 us in step, 90 like this).
+  // (Past the end of K a tile is fetched again into a slot nobody reads: every
+  // K tile then has the same number of loads in flight behind it.)
+  const int first = (int)((blockIdx.x * 5u) % (unsigned)nk);
+  auto issue = [&](int kt, int slot) {
+    int t = min(kt, nk - 1) + first;
+    t = t >= nk ? t - nk : t;
+    const int at = t * BK;
+    unsigned char* sa = smem_raw + slot * Cfg::SLOT_BYTES;
+    unsigned char* sb = sa + Cfg::A_BYTES;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(bsrc[j] + at),
+                                       (lds_void_t*)(sb + (wave + 4 * j) * 1024),
+                                       16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(asrc[j] + at),
+                                       (lds_void_t*)(sa + (wave + 4 * j) * 1024),
+                                       16, 0, 0);
+  };
+  f32x16_t acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.f;
+#pragma unroll
+  for (int t = 0; t < NS - 1; ++t) issue(t, t);
+  const int fr = lane & 31, fc = lane >> 5;
+  int slot = 0, free_slot = NS - 1;
+  for (int kt = 0; kt < nk; ++kt) {
+    wait_vmcnt<(NS - 2) * Cfg::LOADS>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(kt + NS - 1, free_slot);
+    const unsigned char* sa = smem_raw + slot * Cfg::SLOT_BYTES;
+    const unsigned char* sb = sa + Cfg::A_BYTES + wave * 32 * Cfg::ROW_BYTES;
+#pragma unroll
+    for (int kk = 0; kk < BK / 16; ++kk) {
+      const int at = fr * Cfg::ROW_BYTES + (((kk * 2 + fc) ^ lds_swizzle(fr)) * 16);
+      const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(sb + at);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(
+            sa + i * 32 * Cfg::ROW_BYTES + at);
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, acc[i], 0, 0, 0);
+      }
+    }
+    free_slot = slot;
+    slot = slot + 1 == NS ? 0 : slot + 1;
+  }
+  // no direct-to-LDS load may outlive the block
+  wait_vmcnt<0>();
+  // lane: row 32 i + l % 32, columns 8 q + 4 (l / 32) .. of the wavefront's 32
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int row = i * 32 + fr;
+    if (row >= R) continue;
+    bf16_t* dst = C + ((int64_t)e * R + row) * N + col0 + wave * 32 + fc * 4;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (col0 + wave * 32 + fc * 4 + 8 * q < N) {
+        uint2 v;
+        v.x = pack2_bf16(acc[i][4 * q], acc[i][4 * q + 1], relu != 0);
+        v.y = pack2_bf16(acc[i][4 * q + 2], acc[i][4 * q + 3], relu != 0);
+        *reinterpret_cast<uint2*>(dst + 8 * q) = v;
+      }
+  }
 }
 
 struct RingCfg {
@@ -1728,6 +1971,23 @@ static int launch_activation(void* h, int64_t n, int act, int dtype,
   return 0;
 }
 
+// Compute units of the current device (one persistent block per CU: a block
+// takes all of a CU's LDS); 0 on failure.
+static int compute_units() {
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) !=
+            hipSuccess || n < 1) {
+      set_error("expert_ffn: cannot query the number of compute units");
+      return 0;
+    }
+    cus = n;
+  }
+  return cus;
+}
+
 template <int BM, int BN, int BK>
 static int launch_mfma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                        int R, int N, int K, bool relu, hipStream_t st) {
@@ -1751,6 +2011,90 @@ static int launch_mfma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
   return 0;
 }
 
+constexpr int SKINNY_ROWS = 128;
+
+static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
+                         int R, int N, int K, bool relu, hipStream_t st) {
+  // 32 columns per block (half the token reads of 16), 16 while that leaves
+  // compute units without a block
+  const int nt = (int64_t)E * ((N + 31) / 32) >= 512 ? 2 : 1;
+  const int groups_n = (N + 16 * nt - 1) / (16 * nt);
+  const int64_t blocks = (int64_t)E * groups_n;
+  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: too many tiles (%lld)", (long long)blocks);
+  // wavefronts along the reduction: 16 per compute unit in all, while each
+  // keeps 4 steps of 32
+  int waves = 2;
+  while (waves < 16 && blocks * waves < 4096 && K / 32 / (2 * waves) >= 4)
+    waves *= 2;
+  int mt = (R + 15) / 16;              // 1, 2, 3, 4, 6 or 8 tiles of 16 rows
+  mt = mt == 5 || mt == 7 ? mt + 1 : mt;
+  const size_t lds = (size_t)waves * mt * nt * 64 * 16;
+  auto run = [&](auto k) -> int {
+    MOE_ALLOW_LDS(k, lds);
+    k<<<(unsigned)blocks, 64 * waves, lds, st>>>(A, B, C, R, N, K, groups_n,
+                                                 relu ? 1 : 0);
+    MOE_CHECK_LAUNCH("expert_ffn (mfma, few rows)");
+    return 0;
+  };
+#define MOE_SKINNY(MT_)                                                        \
+  return nt == 2 ? run(skinny_gemm_bf16_kernel<MT_, 2>)                        \
+                 : run(skinny_gemm_bf16_kernel<MT_, 1>)
+  switch (mt) {
+    case 1: MOE_SKINNY(1);
+    case 2: MOE_SKINNY(2);
+    case 3: MOE_SKINNY(3);
+    case 4: MOE_SKINNY(4);
+    case 6: MOE_SKINNY(6);
+    default: MOE_SKINNY(8);
+  }
+#undef MOE_SKINNY
+}
+
+// The two kernels for a few rows per expert.  Where the launch has a 128-column
+// tile for half of the compute units, the stream of whole lines; below, the
+// skinny kernel, which cuts the reduction so that every unit has work (one
+// expert of 32 rows, 4096 x 1024: 15 us against 22 for the stream's 8 blocks; 8
+// experts of 64 rows, 1024 x 2048, 128 tiles: 16 against 12).
+constexpr int STREAM_ROWS = 64;
+static bool stream_applies(int E, int R, int N, int K) {
+  const int cus = compute_units();
+  return R <= STREAM_ROWS && K % 64 == 0 && N % 8 == 0 && cus > 0 &&
+         (int64_t)E * ((N + 127) / 128) * 2 >= cus;
+}
+static bool skinny_applies(int E, int R, int N, int K) {
+  const int cus = compute_units();
+  return R <= SKINNY_ROWS && N % 16 == 0 && K % 32 == 0 && cus > 0 &&
+         (int64_t)E * ((N + 127) / 128) * 2 < cus;
+}
+
+// row_map / gather / zero_row: see the kernel (null: rows as they lie)
+static int launch_stream(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
+                         int R, int N, int K, bool relu, hipStream_t st,
+                         const int32_t* row_map = nullptr, bool gather = false,
+                         const bf16_t* zero_row = nullptr) {
+  auto run = [&](auto k, auto cfg) -> int {
+    using Cfg = decltype(cfg);
+    const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+    const int64_t blocks = (int64_t)E * tiles_n;
+    MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+                "expert_ffn: too many tiles (%lld)", (long long)blocks);
+    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
+    k<<<(unsigned)blocks, 256, Cfg::LDS_BYTES, st>>>(
+        A, B, C, R, N, K, tiles_n, relu ? 1 : 0, row_map, gather ? 1 : 0,
+        zero_row);
+    MOE_CHECK_LAUNCH("expert_ffn (mfma, few rows per expert)");
+    return 0;
+  };
+#define MOE_STREAM(MT_)                                                        \
+  return row_map != nullptr                                                    \
+             ? run(stream_gemm_bf16_kernel<MT_, true>, StreamCfg<MT_>())       \
+             : run(stream_gemm_bf16_kernel<MT_, false>, StreamCfg<MT_>())
+  if (R <= 32) MOE_STREAM(1);
+  MOE_STREAM(2);
+#undef MOE_STREAM
+}
+
 template <int BM, int BN, int WN, int WM = 2>
 static int launch_dma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                       int R, int N, int K, bool relu, hipStream_t st) {
@@ -1772,23 +2116,6 @@ static int launch_dma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
   }
   MOE_CHECK_LAUNCH("expert_ffn (mfma, direct-to-LDS)");
   return 0;
-}
-
-// Compute units of the current device (one persistent block per CU: a block
-// takes all of a CU's LDS); 0 on failure.
-static int compute_units() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) !=
-            hipSuccess || n < 1) {
-      set_error("expert_ffn: cannot query the number of compute units");
-      return 0;
-    }
-    cus = n;
-  }
-  return cus;
 }
 
 // C[e] [R, N] = A[e]^T . B[e] with A[e] [K, R] and B[e] [K, N] (both with the
@@ -2077,6 +2404,12 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
     if (!mfma_ok)
       rc = launch_simple<bf16_t>((const bf16_t*)A, (const bf16_t*)B,
                                  (bf16_t*)C, E, R, N, K, relu, st);
+    else if (stream_applies(E, R, N, K))
+      rc = launch_stream((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
+                         N, K, relu, st);
+    else if (skinny_applies(E, R, N, K))
+      rc = launch_skinny((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
+                         N, K, relu, st);
     else if (N >= 256 && R >= 128 && K % 64 == 0 &&
              (int64_t)R * K < (1LL << 31) && (int64_t)N * K < (1LL << 31)) {
       // direct-to-LDS kernels; the persistent 256-row kernel unless 128-row
@@ -2199,6 +2532,28 @@ __global__ void slot_map_kernel(const int32_t* __restrict__ idx,
   map[(int64_t)idx[i] * rows_per_expert + g * C + pos[i]] = (int32_t)t;
 }
 
+// The same map in one launch for few rows per expert (at most STREAM_ROWS): a
+// block per expert looks through the record for its slots.
+__global__ __launch_bounds__(256) void slot_map_rows_kernel(
+    const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
+    const float* __restrict__ gate, const uint8_t* __restrict__ kept,
+    int32_t* __restrict__ map, int tokens, int S, int C, int rows,
+    bf16_t* zero_row, int m) {
+  __shared__ int32_t own[STREAM_ROWS];
+  const int e = blockIdx.x, tid = threadIdx.x;
+  if (tid < rows) own[tid] = -1;
+  if (e == 0)
+    for (int i = tid; i < m; i += 256) zero_row[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < tokens * 2; i += 256) {
+    if (idx[i] != e || !kept[i] || round_to<bf16_t>(gate[i]) == 0.0f) continue;
+    const int t = i >> 1;
+    own[t / S * C + pos[i]] = t;
+  }
+  __syncthreads();
+  if (tid < rows) map[(int64_t)e * rows + tid] = own[tid];
+}
+
 // ---------------------------------------------------------------------------
 // Compacted rows: expert e's occupied slots, groups in order, slots in order,
 // become rows 0 .. rows_used[e] - 1 of its row range.
@@ -2315,13 +2670,17 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
               MESH_MOE_E_ARG, "dispatched_expert_ffn: unknown activation %d",
               activation);
   const int64_t rows = (int64_t)G * C;
+  const bool few_rows =
+      rows <= STREAM_ROWS && (int64_t)G * S < (1 << 30) &&
+      stream_applies(E, (int)rows, H, M) &&
+      ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
   MOE_REQUIRE(dtype == MESH_MOE_BF16 && rows <= 0x7fffffffLL &&
                   (int64_t)G * S <= 0x7fffffffLL &&
-                  ring_path_applies((int)rows, H, M) &&
+                  (few_rows || ring_path_applies((int)rows, H, M)) &&
                   (((uintptr_t)x | (uintptr_t)wi_packed | (uintptr_t)h) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,
-              "dispatched_expert_ffn: needs bf16 and a first GEMM the 256 x 256 "
-              "direct-to-LDS kernel takes (rows=%lld M=%d H=%d)",
+              "dispatched_expert_ffn: needs bf16 and a first GEMM that one of "
+              "the direct-to-LDS kernels takes (rows=%lld M=%d H=%d)",
               (long long)rows, M, H);
   MOE_REQUIRE(workspace_bytes >=
                   mesh_moe_dispatched_expert_ffn_workspace_bytes(G, E, C, M),
@@ -2331,6 +2690,26 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
   int32_t* map = (int32_t*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   bf16_t* zero_row =
       (bf16_t*)(((uintptr_t)(map + (size_t)E * R) + 255) & ~(uintptr_t)255);
+  const bool relu = activation == MESH_MOE_ACT_RELU;
+  if (few_rows) {
+    slot_map_rows_kernel<<<E, 256, 0, st>>>(idx, pos, gate, kept, map, G * S, S,
+                                            C, R, zero_row, M);
+    MOE_CHECK_LAUNCH("dispatched_expert_ffn (slot map, few rows)");
+    int rc = launch_stream((const bf16_t*)x, (const bf16_t*)wi_packed,
+                           (bf16_t*)h, E, R, H, M, relu, st, map, true,
+                           zero_row);
+    if (rc != 0) return rc;
+    if (!relu && activation != MESH_MOE_ACT_LINEAR) {
+      // (also over the rows of experts that were left out: nothing reads them)
+      rc = launch_activation(h, (int64_t)E * R * H, activation, dtype, st);
+      if (rc != 0) return rc;
+    }
+    if (stream_applies(E, R, N, H))
+      return launch_stream((const bf16_t*)h, (const bf16_t*)wo_packed,
+                           (bf16_t*)y, E, R, N, H, false, st, map);
+    return grouped_gemm(h, wo_packed, y, E, R, N, H, MESH_MOE_ACT_LINEAR, dtype,
+                        st);
+  }
   const int64_t n_map = (int64_t)E * R;
   const unsigned cb = (unsigned)((n_map + 255) / 256 < 4096 ? (n_map + 255) / 256
                                                             : 4096);
@@ -2340,7 +2719,6 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
   slot_map_kernel<<<(unsigned)((pairs + 255) / 256), 256, 0, st>>>(
       idx, pos, gate, kept, map, (int64_t)G * S, S, C, rows);
   MOE_CHECK_LAUNCH("dispatched_expert_ffn (slot map)");
-  const bool relu = activation == MESH_MOE_ACT_RELU;
   int rc = launch_ring((const bf16_t*)x, (const bf16_t*)wi_packed, (bf16_t*)h,
                        E, R, H, M, relu, st, map, zero_row);
   if (rc != 0) return rc;

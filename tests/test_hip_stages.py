@@ -1388,6 +1388,77 @@ def test_expert_linear_many_row_tiles(hip, shape):
                                atol=1e-2 * float(wnt.abs().max()), err_msg=name)
 
 
+def _check_linear(hip, shape, activation):
+  """expert_linear against float32 products.  The bound: one bf16 rounding and
+  the float32 sums of K products in another order."""
+  e, rows, k, n = shape
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(shape))
+  a = torch.randn((e, rows, k), generator=gen, device="cuda").to(torch.bfloat16)
+  w = torch.randn((e, n, k), generator=gen, device="cuda").to(torch.bfloat16)
+  y = hip.expert_linear(a, w, activation)
+  assert torch.equal(y, hip.expert_linear(a, w, activation))
+  for i in range(0, e, max(1, e // 4)):
+    wt = w[i].float().t().contiguous()
+    want = a[i].float() @ wt
+    bound = 2.0 ** -8 * want.abs() + k * 2.0 ** -24 * (a[i].float().abs() @ wt.abs())
+    want = want.relu() if activation == "relu" else want
+    assert bool(((y[i].float() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 1, 32, 16), (1, 17, 96, 48), (1, 33, 2080, 80), (2, 64, 512, 1040),
+    (3, 65, 4096, 112), (1, 97, 1056, 2064), (1, 128, 768, 768)],
+    ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("activation", ["linear", "relu"])
+def test_linear_of_few_rows_and_columns(hip, shape, activation):
+  """Few rows, and fewer column tiles than compute units: the reduction is cut
+  over the wavefronts of a block.  One to eight tiles of 16 rows; reductions of
+  1 to 130 steps over 2 to 16 wavefronts; columns inside a block's 16 or 32."""
+  _check_linear(hip, shape, activation)
+
+
+@pytest.mark.parametrize("shape", [
+    (130, 1, 64, 72), (64, 32, 192, 256), (43, 33, 320, 400), (128, 64, 1024, 128),
+    (16, 5, 128, 1032)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("activation", ["linear", "relu"])
+def test_linear_of_few_rows_many_experts(hip, shape, activation):
+  """At most 64 rows for each of many column tiles: reductions shorter than the
+  ring of K tiles, columns that end inside a 128-column tile."""
+  _check_linear(hip, shape, activation)
+
+
+@pytest.mark.parametrize("case", [(1, 64, 64, 4, 256, 512), (3, 40, 32, 5, 128, 1088),
+                                  (8, 32, 48, 8, 64, 384)],
+                         ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("activation", ["relu", "gelu"])
+def test_dispatched_ffn_of_few_rows(hip, case, activation):
+  """dispatch + experts in one call with at most 64 rows per expert, some of
+  the experts without a token: the slots that the combine reads equal those of
+  the two calls bit for bit."""
+  g, s, e, c, m, h = case
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(case))
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  logits = mk(g, s, e)
+  logits[..., e // 2:e // 2 + 3] -= 100.0       # experts that nobody chooses
+  r = hip.top2_gating(logits, c)
+  x = mk(g, s, m).to(torch.bfloat16)
+  wi = mk(e, h, m).to(torch.bfloat16) / m ** 0.5
+  wo = mk(e, m, h).to(torch.bfloat16) / h ** 0.5
+  y = hip.dispatched_expert_ffn(x, r, wi, wo, activation)
+  assert y is not None
+  want = hip.expert_ffn(hip.dispatch(x, r).reshape(e, g * c, m), wi, wo, activation)
+  assert not bool((r.fill.sum(0) > 0).all())
+  for gi in range(g):
+    for ei in range(e):
+      n = int(r.fill[gi, ei])
+      at = slice(gi * c, gi * c + n)
+      assert torch.equal(y[ei, at], want[ei, at])
+  out = hip.combine(y.reshape(e, g, c, m), r, s)
+  assert torch.equal(out, hip.combine(want.reshape(e, g, c, m), r, s))
+
+
 @pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
                                    (2, 6144, 776, 256), (29, 3000, 520, 760)],
                          ids=lambda s: "x".join(map(str, s)))
