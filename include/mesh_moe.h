@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 34
+#define MESH_MOE_ABI_VERSION 35
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -989,6 +989,17 @@ int mesh_moe_attention_decode(const void* q, const void* k_new, const void* v_ne
                               int H, int D, const void* rel_values,
                               const int32_t* rel_bucket, int num_buckets,
                               int dtype, void* stream);
+
+/*
+ * The same with the recurrent states as values: new_k, new_v [B,Lm,H*D] receive
+ * old_k, old_v with row position[b] replaced, in the pass that reads them.  The
+ * old states are not changed; no operand may overlap the new ones.
+ */
+int mesh_moe_attention_decode_states(
+    const void* q, const void* k_new, const void* v_new, const void* old_k,
+    const void* old_v, void* new_k, void* new_v, const int32_t* position,
+    void* out, int B, int Lm, int H, int D, const void* rel_values,
+    const int32_t* rel_bucket, int num_buckets, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -36,6 +36,9 @@ class HipMeshImpl(mtf.MeshImpl):
           "HipMeshImpl needs a GPU: torch.cuda.is_available() is False "
           "(there is no CPU path)")
     self._device = torch.device(device or "cuda:%d" % torch.cuda.current_device())
+    self._device_index = self._device.index
+    if self._device_index is None:
+      self._device_index = torch.cuda.current_device()
     moe_hip.load_library()  # fail now, not at the first kernel, if not built
 
   device = property(lambda self: self._device)
@@ -190,14 +193,18 @@ class HipMeshImpl(mtf.MeshImpl):
   def slicewise(self, fn, *inputs):
     """Calls fn once on the single slice of each input
     (mesh_tensorflow/placement_mesh_impl.py:159-178)."""
-    inputs = mtf.convert_args_to_laid_out_tensors(inputs)
-    args = [x.tensor_list[0] if isinstance(x, self.LaidOutTensor) else x
-            for x in inputs]
-    with torch.cuda.device(self._device):
+    laid_out = self.LaidOutTensor
+    args = []
+    for x in mtf.convert_args_to_laid_out_tensors(inputs):
+      args.append(x.tensor_list[0] if isinstance(x, laid_out) else x)
+    if torch.cuda.current_device() == self._device_index:
       ret = fn(*args)
+    else:
+      with torch.cuda.device(self._device):
+        ret = fn(*args)
     if isinstance(ret, tuple):
-      return tuple(self.LaidOutTensor([t]) for t in ret)
-    return self.LaidOutTensor([ret])
+      return tuple(laid_out([t]) for t in ret)
+    return laid_out([ret])
 
   def einsum(self, equation, *slices):
     """The hook the reference documents "for custom einsum implementation"

@@ -138,11 +138,10 @@ class DenseOperation(mtf.Operation):
     x, kernel = self.inputs
     mesh_impl = lowering.mesh_impl(self)
     packed = lowering.variables[kernel.operation].packed(x.dtype)
-    sizes = self.outputs[0].shape.to_integer_list
     act = self._activation
 
     def fn(xs):
-      return moe_hip.dense(xs.contiguous(), packed, act).reshape(sizes)
+      return moe_hip.dense(xs.contiguous(), packed, act)
     lowering.set_tensor_lowering(
         self.outputs[0], mesh_impl.slicewise(fn, lowering.tensors[x]))
 

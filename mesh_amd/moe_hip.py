@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 34
+ABI_VERSION = 35
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -229,6 +229,10 @@ _SIGNATURES = {
     "mesh_moe_attention_decode": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, _vp, _vp, ctypes.c_int, ctypes.c_int, _vp]),
+    "mesh_moe_attention_decode_states": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp, _vp, ctypes.c_int,
+        ctypes.c_int, _vp]),
 }
 EXPORTS = sorted(_SIGNATURES)
 
@@ -282,14 +286,21 @@ def _dev(t, name, dtype=None, shape=None):
     raise MoeHipError("%s must be contiguous" % name)
   if dtype is not None and t.dtype != dtype:
     raise MoeHipError("%s: dtype %s, expected %s" % (name, t.dtype, dtype))
-  if shape is not None and tuple(t.shape) != tuple(shape):
+  if shape is not None and t.shape != tuple(shape):
     raise MoeHipError("%s: shape %s, expected %s"
                       % (name, tuple(t.shape), tuple(shape)))
   return t.data_ptr()
 
 
+# The handle of the current stream without a torch.cuda.Stream object around it
+# (6 us per library call on the benchmark machine's host, this 0.3).
+_current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-  return torch.cuda.current_stream().cuda_stream
+  if _current_raw_stream is None:
+    return torch.cuda.current_stream().cuda_stream
+  return _current_raw_stream(torch.cuda.current_device())
 
 
 class StageTimer(object):
@@ -335,16 +346,36 @@ class StageTimer(object):
 _timer = None
 
 
-class _stage(object):
+class _UntimedStage(object):
+  """What brackets a stage while no timer is set."""
+
+  def __enter__(self):
+    return self
+
+  def __exit__(self, *exc):
+    return False
+
+  def call(self, keep, fn, *args):
+    del keep
+    return fn(*args)
+
+
+_UNTIMED = _UntimedStage()
+
+
+def _stage(name):
   """Context manager bracketing one stage with events if a timer is set."""
+  return _UNTIMED if _timer is None else _TimedStage(name)
+
+
+class _TimedStage(object):
 
   def __init__(self, name):
     self.name = name
 
   def __enter__(self):
-    if _timer is not None:
-      self.start = torch.cuda.Event(enable_timing=True)
-      self.start.record()
+    self.start = torch.cuda.Event(enable_timing=True)
+    self.start.record()
     return self
 
   def __exit__(self, *exc):
@@ -1369,10 +1400,20 @@ def rms_norm(x, scale, epsilon=1e-6):
 def dense(x, w_packed, activation=None):
   """x [..., K] times a packed kernel [1, N, K] -> [..., N]
   (mtf.layers.dense without bias: one einsum, ops.py / layers.py:112-160)."""
-  k = x.shape[-1]
+  lib = load_library()
+  if activation not in ACTIVATIONS:
+    raise ValueError("unsupported expert activation %r" % (activation,))
+  sizes = x.shape
+  k = sizes[-1]
   n = w_packed.shape[1]
-  y = expert_linear(x.reshape(1, -1, k), w_packed, activation)
-  return y.reshape(tuple(x.shape[:-1]) + (n,))
+  dt = x.dtype
+  y = torch.empty(sizes[:-1] + (n,), dtype=dt, device=x.device)
+  with _stage("expert_linear"):
+    _check(lib.mesh_moe_expert_linear(
+        _dev(x, "a"), _dev(w_packed, "w_packed", dt, (1, n, k)), y.data_ptr(), 1,
+        x.numel() // k, k, n, ACTIVATIONS[activation], dtype_code(dt),
+        _stream()), "expert_linear")
+  return y
 
 
 def fused_attention_applies(q, num_heads):
@@ -1439,6 +1480,31 @@ def attention_decode(q, k_new, v_new, k_cache, v_cache, position, num_heads,
         *_relative_bias_ptrs(relative_bias, q.dtype, num_heads, lm),
         dtype_code(q.dtype), _stream()), "attention_decode")
   return out
+
+
+def attention_decode_states(q, k_new, v_new, old_k, old_v, position, num_heads,
+                            relative_bias=None):
+  """attention_decode with the states as values: (out, new_k, new_v), the old
+  states with row position[b] replaced, as tensors of their own."""
+  lib = load_library()
+  b, hd = q.shape
+  lm = old_k.shape[1]
+  if hd % num_heads:
+    raise MoeHipError("q channels %d not divisible by %d heads"
+                      % (hd, num_heads))
+  out = torch.empty_like(q)
+  new_k, new_v = torch.empty_like(old_k), torch.empty_like(old_v)
+  with _stage("attention_decode"):
+    _check(lib.mesh_moe_attention_decode_states(
+        _dev(q, "q"), _dev(k_new, "k_new", q.dtype, (b, hd)),
+        _dev(v_new, "v_new", q.dtype, (b, hd)),
+        _dev(old_k, "old_k", q.dtype, (b, lm, hd)),
+        _dev(old_v, "old_v", q.dtype, (b, lm, hd)), new_k.data_ptr(),
+        new_v.data_ptr(), _dev(position, "position", torch.int32, (b,)),
+        out.data_ptr(), b, lm, num_heads, hd // num_heads,
+        *_relative_bias_ptrs(relative_bias, q.dtype, num_heads, lm),
+        dtype_code(q.dtype), _stream()), "attention_decode_states")
+  return out, new_k, new_v
 
 
 def slot_combine_backward(dout, y, r):

@@ -615,6 +615,9 @@ class Lowering(object):
     self.variables = {}    # {Variable: LaidOutVariable}
     self.initial_values = dict(initial_values or {})
     self._feeds = {}
+    # {Tensor: its slice shape}: a Tensor's Shape and a mesh's layout do not
+    # change, and every step checks every tensor against it
+    self._slice_shapes = {}
     self.scalar_summaries = {}   # {name: 0-d torch tensor} of the last run
     for op in graph.operations:
       op.lower(self)
@@ -718,7 +721,10 @@ class Lowering(object):
     self.tensors[tensor] = laid_out_tensor
 
   def verify_slice_shapes(self, tensor, laid_out_tensor):
-    correct_shape = self.mesh_impl(tensor).slice_shape(tensor.shape)
+    correct_shape = self._slice_shapes.get(tensor)
+    if correct_shape is None:
+      correct_shape = self.mesh_impl(tensor).slice_shape(tensor.shape)
+      self._slice_shapes[tensor] = correct_shape
     actual_shape = list(laid_out_tensor.slice_shape)
     if actual_shape != correct_shape:
       raise ValueError(

@@ -342,7 +342,7 @@ class AttentionDecodeOperation(mtf.Operation):
   step, the recurrent states old_k, old_v [batch..., memory_length,
   heads * d_kv] and position [batch...] (int32) -> the attention outputs
   [batch..., heads * d_kv] and the updated states.  The states are new tensors
-  (the graph stays functional); the library call updates a copy in place.
+  (the graph stays functional), written in the pass that reads the old ones.
   relative_values [heads, buckets]: the relative attention bias of the memory
   positions against the step's position (transformer_layers.py:317-352)."""
 
@@ -380,14 +380,15 @@ class AttentionDecodeOperation(mtf.Operation):
 
     def fn(q, k, v, old_k, old_v, position, *extra):
       q2, k2, v2 = (t.reshape(-1, channels).contiguous() for t in (q, k, v))
-      kc = old_k.reshape(-1, memory, channels).clone()
-      vc = old_v.reshape(-1, memory, channels).clone()
+      kc, vc = (t.reshape(-1, memory, channels).contiguous()
+                for t in (old_k, old_v))
       pos = position.reshape(-1).to(torch.int32).contiguous()
       _, rel = _attention_extras(extra, None, 3 if extra else None, memory,
                                  bidirectional, q.dtype)
-      out = moe_hip.attention_decode(q2, k2, v2, kc, vc, pos, heads,
-                                     relative_bias=rel)
-      return out.reshape(q_sizes), kc.reshape(s_sizes), vc.reshape(s_sizes)
+      out, new_k, new_v = moe_hip.attention_decode_states(
+          q2, k2, v2, kc, vc, pos, heads, relative_bias=rel)
+      return (out.reshape(q_sizes), new_k.reshape(s_sizes),
+              new_v.reshape(s_sizes))
     outs = mesh_impl.slicewise(fn, *[lowering.tensors[t] for t in self.inputs])
     for tensor, value in zip(self.outputs, outs):
       lowering.set_tensor_lowering(tensor, value)

@@ -271,6 +271,40 @@ def test_attention_decode(hip, case, act_dtype):
 
 
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("case", [(2, 12, 2, 4), (3, 300, 4, 64), (33, 511, 16, 64),
+                                  (1, 77, 3, 24), (2, 600, 1, 320), (1, 1, 1, 8)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_attention_decode_states(hip, case, act_dtype):
+  """The step with the states as values: outputs and new states are those of
+  the in-place call bit for bit (rows behind the position included, whatever
+  they hold), the old states stay as they were."""
+  b, lm, heads, d = case
+  dt = H.ACT_TORCH[act_dtype]
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(case))
+  mk = lambda *s: torch.randn(s, generator=gen, device="cuda").to(dt)
+  q, kn, vn = (mk(b, heads * d) for _ in range(3))
+  kc, vc = mk(b, lm, heads * d), mk(b, lm, heads * d)
+  pos = torch.randint(0, lm, (b,), generator=gen, device="cuda", dtype=torch.int32)
+  pos[0] = lm - 1
+  behind = torch.arange(lm, device="cuda")[None] > pos[:, None]
+  vc[behind] = float("nan")          # never read into the output
+  values = mk(heads, 16)
+  bucket = torch.from_numpy(B.relative_position_bucket(
+      np.arange(-(lm - 1), lm), False, 16).astype(np.int32)).cuda()
+  for rel in (None, (values, bucket)):
+    k1, v1 = kc.clone(), vc.clone()
+    want = hip.attention_decode(q, kn, vn, k1, v1, pos, heads, relative_bias=rel)
+    k0, v0 = kc.clone(), vc.clone()
+    got, k2, v2 = hip.attention_decode_states(q, kn, vn, k0, v0, pos, heads,
+                                              relative_bias=rel)
+    assert torch.equal(got, want) and bool(torch.isfinite(got.float()).all())
+    bits = torch.int32 if dt == torch.float32 else torch.int16
+    for a, w in ((k2, k1), (v2, v1), (k0, kc), (v0, vc)):
+      assert torch.equal(a.view(bits), w.view(bits))
+
+
+@pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("case", [(2, 40, 2, 16, 8), (2, 200, 3, 64, 32),
                                   (1, 328, 2, 128, 32), (1, 1024, 2, 64, 32),
