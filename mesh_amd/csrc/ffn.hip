@@ -327,14 +327,10 @@ __global__ __launch_bounds__(1024) void skinny_gemm_bf16_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// bf16 MFMA kernel with direct global -> LDS loads and an NS-stage ring.
-//
-// Same tiling and MFMA operand roles as the kernel above, but the K loop is fed
-// by global_load_lds_dwordx4: every lane names its own 16 global bytes and the
+// Direct global -> LDS loads, which feed the K loops of the kernels below
+// (global_load_lds_dwordx4): every lane names its own 16 global bytes and the
 // wavefront's 64 x 16 bytes land contiguously in LDS without passing through
-// registers.  The loads for K tile kt+NS-1 are issued while tile kt is being
-// multiplied; a partial vmcnt wait plus one bare s_barrier per K tile publishes
-// the oldest tile.
+// registers.
 //
 // One load instruction fetches 8 rows x 128 bytes (BK = 64 bf16): 8 consecutive
 // lanes read one full 128-byte line of a row, which is what the memory
@@ -387,237 +383,16 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-template <int BM, int BN, int WN, int WM = 2>  // WM x WN wavefronts
-struct DmaCfg {
-  static constexpr int BK = 64;
-  static constexpr int NS = 2;                         // LDS slots
-  static constexpr int WAVES = WM * WN;
-  static constexpr int THREADS = 64 * WAVES;
-  static constexpr int WTM = BM / WM, WTN = BN / WN;
-  static constexpr int TM = WTM / 32, TN = WTN / 32;
-  static constexpr int ROW_BYTES = BK * 2;             // 128
-  static constexpr int A_INSTR = (BM / 8) / WAVES;     // per wavefront
-  static constexpr int B_INSTR = (BN / 8) / WAVES;
-  static constexpr int A_BYTES = BM * ROW_BYTES, B_BYTES = BN * ROW_BYTES;
-  static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
-  static constexpr int LDC = BN + 4;
-  static constexpr size_t LOOP_BYTES = (size_t)NS * STAGE_BYTES;
-  static constexpr size_t EPI_BYTES = (size_t)BM * LDC * sizeof(bf16_t);
-  static constexpr size_t LDS_BYTES =
-      LOOP_BYTES > EPI_BYTES ? LOOP_BYTES : EPI_BYTES;
-};
-
 __device__ __forceinline__ int lds_swizzle(int row) {
   return (row & 7) ^ ((row >> 3) & 1);
-}
-
-template <int BM, int BN, int WN, bool RELU, int WM = 2>
-__global__ __launch_bounds__(64 * WM * WN) void grouped_gemm_bf16_dma_kernel(
-    const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-    bf16_t* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n) {
-  using Cfg = DmaCfg<BM, BN, WN, WM>;
-  constexpr int BK = Cfg::BK;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-
-  const int nblk = gridDim.x;
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  const int per_xcd = nblk >> 3, extra = nblk & 7;
-  const int logical = xcd * per_xcd + min(xcd, extra) + local;
-  const int tiles_per_e = tiles_m * tiles_n;
-  const int e = logical / tiles_per_e;
-  const int rem = logical - e * tiles_per_e;
-  const int tn = rem / tiles_m;
-  const int tm = rem - tn * tiles_m;
-  const int row0 = tm * BM, col0 = tn * BN;
-  const bf16_t* Ae = A + (int64_t)e * R * K;
-  const bf16_t* Be = B + (int64_t)e * N * K;
-  bf16_t* Ce = Cout + (int64_t)e * R * N;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-
-  // Element offsets of the 16 bytes this lane fetches in each of its load
-  // instructions.  Instruction q of an operand covers tile rows 8q .. 8q+7;
-  // lane l fills LDS slot (row 8q + l/8, column l%8).  Wavefront w issues
-  // q = w, w + 4, ...
-  int a_off[Cfg::A_INSTR], b_off[Cfg::B_INSTR];
-#pragma unroll
-  for (int j = 0; j < Cfg::A_INSTR; ++j) {
-    const int row = (wave + Cfg::WAVES * j) * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ lds_swizzle(row);
-    a_off[j] = min(row0 + row, R - 1) * K + chunk * 8;
-  }
-#pragma unroll
-  for (int j = 0; j < Cfg::B_INSTR; ++j) {
-    const int row = (wave + Cfg::WAVES * j) * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ lds_swizzle(row);
-    b_off[j] = min(col0 + row, N - 1) * K + chunk * 8;
-  }
-  auto issue_stage = [&](int kt, int slot) {
-    unsigned char* sa = smem_raw + slot * Cfg::STAGE_BYTES;
-    unsigned char* sb = sa + Cfg::A_BYTES;
-    const bf16_t* ak = Ae + kt * BK;
-    const bf16_t* bk = Be + kt * BK;
-#pragma unroll
-    for (int j = 0; j < Cfg::A_INSTR; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (glb_void_t*)(ak + a_off[j]),
-          (lds_void_t*)(sa + (wave + Cfg::WAVES * j) * 1024), 16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < Cfg::B_INSTR; ++j)
-      __builtin_amdgcn_global_load_lds(
-          (glb_void_t*)(bk + b_off[j]),
-          (lds_void_t*)(sb + (wave + Cfg::WAVES * j) * 1024), 16, 0, 0);
-  };
-
-  f32x16_t acc[Cfg::TM][Cfg::TN];
-#pragma unroll
-  for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  // Fragment reads: this lane reads row l % 32 of each 32-row MFMA tile of its
-  // wavefront's sub-tile, chunk 2*kk + l/32 of the K tile, at the swizzled
-  // column.  The swizzle depends only on the low four row bits, which every
-  // MFMA tile of the sub-tile shares.
-  const int fr = lane & 31, fc = lane >> 5;
-  int a_frag[BK / 16], b_frag[BK / 16];
-#pragma unroll
-  for (int kk = 0; kk < BK / 16; ++kk) {
-    const int col = ((kk * 2 + fc) ^ lds_swizzle(fr)) * 16;
-    a_frag[kk] = (wm * Cfg::WTM + fr) * Cfg::ROW_BYTES + col;
-    b_frag[kk] = (wn * Cfg::WTN + fr) * Cfg::ROW_BYTES + col;
-  }
-
-  // K loop, NS = 2 slots.  The MFMA fragments are double buffered in registers:
-  // while the 16 MFMAs of step kk run, the 8 fragment reads of step kk+1 are in
-  // flight.  The hand-over to the next K tile happens before the MFMAs of the
-  // LAST step of a tile: once this lane holds that step's fragments it no
-  // longer needs the tile's LDS slot, so it waits for its own loads of the next
-  // tile, meets the other wavefronts at a bare s_barrier (__syncthreads() would
-  // add a fence that also drains the loads that are meant to stay in flight),
-  // issues the loads of tile kt+2 into the slot just freed and reads the first
-  // fragments of tile kt+1 -- all of it hidden behind the last 16 MFMAs.
-  constexpr int KSTEPS = BK / 16;
-  const int nk = K / BK;
-  bf16x8_t fa[2][Cfg::TM], fb[2][Cfg::TN];
-  auto read_frags = [&](int slot, int kk, int buf) {
-    const unsigned char* sa = smem_raw + slot * Cfg::STAGE_BYTES;
-    const unsigned char* sb = sa + Cfg::A_BYTES;
-#pragma unroll
-    for (int i = 0; i < Cfg::TM; ++i)
-      fa[buf][i] = *reinterpret_cast<const bf16x8_t*>(sa + a_frag[kk] + i * 32 * Cfg::ROW_BYTES);
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j)
-      fb[buf][j] = *reinterpret_cast<const bf16x8_t*>(sb + b_frag[kk] + j * 32 * Cfg::ROW_BYTES);
-  };
-
-  issue_stage(0, 0);
-  wait_vmcnt<0>();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  if (nk > 1) issue_stage(1, 1);
-  read_frags(0, 0, 0);
-  // One K tile.  LAST = the final tile (no hand-over).  The body is free of
-  // branches so that the scheduling hints below see one basic block; past the
-  // end of K the hand-over simply re-fetches the last tile into the free slot.
-  auto k_tile = [&](int kt, auto last_tag) {
-    constexpr bool LAST = decltype(last_tag)::value;
-    const int slot = kt & 1;
-#pragma unroll
-    for (int kk = 0; kk < KSTEPS; ++kk) {
-      const int cur = kk & 1, nxt = cur ^ 1;
-      if (kk + 1 < KSTEPS) {
-        read_frags(slot, kk + 1, nxt);
-      } else if (!LAST) {
-        // fragments of the last step are in registers (lgkmcnt 0) and this
-        // lane's loads of tile kt+1 have landed (vmcnt 0)
-        __builtin_amdgcn_s_waitcnt(0x0070);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        issue_stage(min(kt + 2, nk - 1), slot);
-        read_frags(slot ^ 1, 0, nxt);
-      }
-#pragma unroll
-      for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < Cfg::TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[cur][j], fa[cur][i], acc[i][j], 0, 0, 0);
-      // Spread the memory instructions of this step between its MFMAs instead
-      // of letting them queue up in front (masks: 0x8 MFMA, 0x20 VMEM read,
-      // 0x100 LDS read).
-      constexpr int READS = Cfg::TM + Cfg::TN;
-      constexpr int MFMA_PER_READ = Cfg::TM * Cfg::TN / READS;
-      constexpr int LOADS = Cfg::A_INSTR + Cfg::B_INSTR;
-      if (kk + 1 < KSTEPS) {
-#pragma unroll
-        for (int g = 0; g < READS; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, MFMA_PER_READ, 0);
-        }
-      } else if (!LAST) {
-#pragma unroll
-        for (int g = 0; g < READS; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x020, (LOADS + READS - 1) / READS, 0);
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-      }
-    }
-  };
-  for (int kt = 0; kt + 1 < nk; ++kt) k_tile(kt, std::false_type{});
-  k_tile(nk - 1, std::true_type{});
-  // the epilogue reuses the ring: no direct-to-LDS load may still be in flight
-  // (the last hand-over re-fetches a tile nobody reads)
-  wait_vmcnt<0>();
-  __syncthreads();
-
-  // epilogue: round (and relu), stage the tile in LDS, coalesced stores
-  bf16_t* Cs = reinterpret_cast<bf16_t*>(smem_raw);  // [BM][LDC]
-  const int m_l = lane & 31;
-  const int n_l = (lane >> 5) * 4;
-#pragma unroll
-  for (int i = 0; i < Cfg::TM; ++i) {
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row = wm * Cfg::WTM + i * 32 + m_l;
-        const int col = wn * Cfg::WTN + j * 32 + 8 * q + n_l;
-        uint2 v;
-        v.x = pack2_bf16(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], RELU);
-        v.y = pack2_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3], RELU);
-        *reinterpret_cast<uint2*>(Cs + row * Cfg::LDC + col) = v;
-      }
-    }
-  }
-  __syncthreads();
-  constexpr int CPR_C = BN / 8;  // 16-byte chunks per output row
-#pragma unroll 4
-  for (int c = tid; c < BM * CPR_C; c += Cfg::THREADS) {
-    const int r = c / CPR_C, cc = (c % CPR_C) * 8;
-    const int grow = row0 + r, gcol = col0 + cc;
-    if (grow < R && gcol < N) {
-      const uint2* s = reinterpret_cast<const uint2*>(Cs + r * Cfg::LDC + cc);
-      uint2 lo = s[0], hi = s[1];
-      *reinterpret_cast<uint4*>(Ce + (int64_t)grow * N + gcol) =
-          make_uint4(lo.x, lo.y, hi.x, hi.y);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
 // bf16 MFMA kernel for 256 x 256 tiles with SPREAD direct-to-LDS loads.
 //
-// Same tile, wavefront grid (2 x 4, 128 x 64 sub-tiles), LDS image and
-// fragment reads as grouped_gemm_bf16_dma_kernel<256, 256, 4, RELU, 2>; the
-// difference is when the loads are issued.  A wavefront that issues its eight
+// 8 wavefronts in a 2 x 4 grid, two per SIMD, each a 128 x 64 sub-tile = 4 x 2
+// MFMA tiles; operand roles as in the first kernel of this file.  What shapes
+// the kernel is when the loads are issued.  A wavefront that issues its eight
 // loads of a K tile back to back sits in that burst for ~0.7 us (the memory
 // pipeline accepts them only as fast as earlier requests drain), and because
 // the wavefronts of a block hand over together, the MFMA pipes idle meanwhile.
@@ -863,19 +638,17 @@ __device__ __forceinline__ void ring_tile_blocks(int rem, int tiles_m,
 // slower, although nothing was added to the path of the full tiles but a
 // second copy of the K loop next to it.)
 //
-// TAILS (R not a multiple of the 256-row tile): in an expert's last row tile
-// a wavefront multiplies only the 32-row pieces of its 128-row sub-tile that
-// hold rows below R -- the piece count is the same for the whole K loop, so
-// the wavefront runs the copy of the loop written for that count (0 to 4
-// pieces; with 0 it only loads and meets the barriers).  The two wavefronts of
-// a SIMD own the upper and the lower half of the tile, so a tile with 144
-// valid rows costs the SIMD 4 + 1 pieces instead of 8.  (Numbering the
-// experts' last row tiles after all full ones, so that the persistent blocks
-// end on the cheaper tiles, separates the row tiles that share a weight panel:
-// with 400 rows per expert the weights were then read twice from memory and
-// the launches took 14 % longer; moving only as many last row tiles as the
-// final, partly filled round holds to the end cost 5 % where it applied, 640
-// rows per expert with 384 tiles, for the same reason.)
+// TAILS (row tiles of `tile_rows` <= 256 rows, see ring_tile_rows, and a last
+// one that may hold fewer): a wavefront multiplies only 32-row pieces that hold
+// rows -- their count is the same for the whole K loop, so the wavefront runs
+// the copy of the loop written for that count (0 to 4 pieces; with 0 it only
+// loads and meets the barriers).  The two wavefronts of a SIMD own the upper
+// and the lower half of the LDS tile; the tile's pieces are dealt out evenly
+// between them (rows 0 .. 32 p0 - 1 to the upper half, the others to the lower),
+// so that neither waits for the other at the hand-overs.  (Numbering the
+// experts' last row tiles after all full ones separates the row tiles that
+// share a weight panel: with 400 rows per expert the weights were then read
+// twice from memory and the launches took 14 % longer.)
 // 512 bytes that stay zero (nothing writes them): where a K-major tile reaches
 // past the last reduction row, its rows are loaded from here
 static __device__ __attribute__((aligned(256))) bf16_t kmajor_zero_row[256];
@@ -892,7 +665,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int32_t* __restrict__ tile_list = nullptr,
     const int32_t* __restrict__ row_count = nullptr,
     float mask_scale = 1.0f, float* __restrict__ partial = nullptr,
-    int whole_tiles = 0, int split = 1) {
+    int whole_tiles = 0, int split = 1, int tile_rows = RingCfg::BM) {
   using Cfg = RingCfg;
   // row_count [E], optional: KMAJOR kernels take it as the reduction extent
   // per expert (k_extent)
@@ -955,8 +728,18 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   bf16_t* Ce;
   typename std::conditional<GATHER, int64_t, int>::type a_off[Cfg::A_INSTR];
   int b_off[Cfg::B_INSTR];
-  // TAILS: 32-row pieces of this wavefront's sub-tile that hold rows below R
-  int pieces = Cfg::TM;
+  // TAILS: 32-row pieces of this wavefront's sub-tile that hold rows of the
+  // tile, and of the sub-tiles of the upper half
+  int pieces = Cfg::TM, pieces0 = Cfg::TM;
+  // first row of row tile tm, and the place in it of LDS tile row `row`
+  auto tile_row0 = [&](int tm) { return TAILS ? tm * tile_rows : tm * BM; };
+  auto tile_pieces0 = [&](int tm) {
+    const int valid = min(tile_rows, R - tm * tile_rows);
+    return (((valid + 31) >> 5) + 1) >> 1;
+  };
+  auto row_in_tile = [&](int row, int p0) {
+    return TAILS && row >= BM / 2 ? row - BM / 2 + 32 * p0 : row;
+  };
   // logical tile -> expert, row tile, column tile
   auto tile_coords = [&](int logical, int& e, int& tm, int& tn) {
     if constexpr (LISTED) logical = tile_list[logical];
@@ -964,7 +747,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int rem = logical - e * tiles_per_e;
     tn = rem / tiles_m;
     tm = rem - tn * tiles_m;
-    if (!LISTED && !TAILS) ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
+    if (!LISTED) ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
   };
   // GATHER: the slot -> token map entries of the four rows this lane loads in
   // a tile.  fetch_map issues the four loads back to back without waiting
@@ -976,10 +759,12 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     if constexpr (GATHER) {
       int e, tm, tn;
       tile_coords(logical, e, tm, tn);
+      const int p0 = TAILS ? tile_pieces0(tm) : 0;
 #pragma unroll
       for (int j = 0; j < Cfg::A_INSTR; ++j) {
-        const int row = (wave + Cfg::WAVES * j) * 8 + (lane >> 3);
-        const int32_t* p = row_map + ((int64_t)e * R + min(tm * BM + row, R - 1));
+        const int row = row_in_tile((wave + Cfg::WAVES * j) * 8 + (lane >> 3), p0);
+        const int32_t* p =
+            row_map + ((int64_t)e * R + min(tile_row0(tm) + row, R - 1));
         asm volatile("global_load_dword %0, %1, off"
                      : "=&v"(map_src[j]) : "v"(p) : "memory");
       }
@@ -998,12 +783,13 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     int e, tm, tn;
     tile_coords(logical, e, tm, tn);
     if constexpr (TAILS) {
-      const int valid = min(BM, R - tm * BM);
+      const int valid = min(tile_rows, R - tm * tile_rows);
       const int blocks = (valid + 31) >> 5;
-      pieces = __builtin_amdgcn_readfirstlane(
-          wm == 0 ? min(blocks, Cfg::TM) : max(blocks - Cfg::TM, 0));
+      pieces0 = (blocks + 1) >> 1;
+      pieces = __builtin_amdgcn_readfirstlane(wm == 0 ? pieces0
+                                                      : blocks - pieces0);
     }
-    row0 = tm * BM;
+    row0 = tile_row0(tm);
     col0 = tn * BN;
     if constexpr (KMAJOR) {
       if (k_extent != nullptr) {
@@ -1052,7 +838,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         a_off[j] = (src >= 0 ? (int64_t)src * K : (int64_t)(zero_row - A)) +
                    chunk * 8;
       } else {
-        a_off[j] = min(row0 + row, R - 1) * K + chunk * 8;
+        a_off[j] = min(row0 + row_in_tile(row, pieces0), R - 1) * K + chunk * 8;
       }
       b_off[j] = min(col0 + row, N - 1) * K + chunk * 8;
     }
@@ -1337,7 +1123,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     wait_vmcnt<0>();
     asm volatile("" ::: "memory");
     __syncthreads();
-    const int out_row0 = row0, out_col0 = col0;
+    const int out_row0 = row0, out_col0 = col0, out_pieces0 = pieces0;
     bf16_t* out_c = Ce;
     const int out_unit = unit;
     if constexpr (KMAJOR || SPLIT) {
@@ -1431,9 +1217,14 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         const int c = e_tid + n * Cfg::THREADS;
         const int srow = c / CPR_C, chunk = c % CPR_C;
         // staging row -> tile row: 64 rows of each half of the tile
-        const int grow = out_row0 + (srow >> 6) * 128 + pass * 64 + (srow & 63);
+        const int half_row = pass * 64 + (srow & 63);
+        const int grow =
+            out_row0 + (srow >> 6) * (TAILS ? 32 * out_pieces0 : 128) + half_row;
         const int gcol = out_col0 + chunk * 8;
-        if (grow < R && gcol < N) {
+        // (TAILS: a half's rows past its pieces belong to the other half or to
+        // the next tile)
+        if (grow < (TAILS ? min(R, out_row0 + tile_rows) : R) && gcol < N &&
+            !(TAILS && srow < 64 && half_row >= 32 * out_pieces0)) {
           u32x4_t v = piece[n];
           if constexpr (MASKED) {
             const u32x4_t hm = *reinterpret_cast<const u32x4_t*>(
@@ -2095,29 +1886,6 @@ static int launch_stream(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
 #undef MOE_STREAM
 }
 
-template <int BM, int BN, int WN, int WM = 2>
-static int launch_dma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
-                      int R, int N, int K, bool relu, hipStream_t st) {
-  using Cfg = DmaCfg<BM, BN, WN, WM>;
-  const int tiles_m = (R + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int64_t blocks = (int64_t)tiles_m * tiles_n * E;
-  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
-              "expert_ffn: too many tiles (%lld)", (long long)blocks);
-  if (relu) {
-    auto k = grouped_gemm_bf16_dma_kernel<BM, BN, WN, true, WM>;
-    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
-    k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(A, B, C, R, N, K, tiles_m,
-                                                      tiles_n);
-  } else {
-    auto k = grouped_gemm_bf16_dma_kernel<BM, BN, WN, false, WM>;
-    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
-    k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(A, B, C, R, N, K, tiles_m,
-                                                      tiles_n);
-  }
-  MOE_CHECK_LAUNCH("expert_ffn (mfma, direct-to-LDS)");
-  return 0;
-}
-
 // C[e] [R, N] = A[e]^T . B[e] with A[e] [K, R] and B[e] [K, N] (both with the
 // reduction index outermost); true if the K-major ring kernel takes the shape.
 static bool kmajor_path_applies(const void* A, const void* B, const void* C,
@@ -2195,7 +1963,8 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<split_blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, units, nullptr, nullptr, nullptr,
-        nullptr, k_extent, 1.0f, (float*)scratch, plan.whole_tiles, plan.split);
+        nullptr, k_extent, 1.0f, (float*)scratch, plan.whole_tiles, plan.split,
+        Cfg::BM);
     MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands, split)");
     split_reduce_kernel<<<(unsigned)tail * Cfg::TM * Cfg::TN, Cfg::THREADS, 0,
                           st>>>((const float*)scratch, C, R, N, tiles_m,
@@ -2207,9 +1976,43 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
   MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
   k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
       A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1);
+      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, Cfg::BM);
   MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
   return 0;
+}
+
+// Rows per row tile (a multiple of 32, at most 256) for R rows per expert.
+// The persistent blocks take whole rounds of tiles, so what counts is rounds
+// times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
+// 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
+// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside
+// the K loop.  Rows are spread evenly over the row tiles: 640 rows per expert are
+// three tiles of 224 or four of 160, not 256 + 256 + 128.  Measured, tiles of
+// 256 and a shorter last one -> the rule's choice (both sides bit-identical):
+//   32 x 640 rows, 4096 x 1024 (384 tiles -> 512 of 160 rows)   203 -> 166 us
+//   16 x 705 rows, 768 x 3072 / 3072 x 768 (192 rows)       73 / 67 -> 60 / 55
+//   8 x 900 rows, 1536 x 4608 (192 rows)                        117 -> 100
+//   64 x 320 rows, 1024 x 4096 (160 rows; 128-row kernel before) 268 -> 207
+//   5000 rows, 1280 x 1280 (128 rows, 200 tiles instead of 100)  31 -> 25
+//   128 x 400 rows, 2048 x 8192 (224 rows)                     1729 -> 1680
+static int ring_tile_rows(int E, int R, int N, int K, int cus) {
+  const int tiles_n = (N + RingCfg::BN - 1) / RingCfg::BN;
+  const int nk = (K + RingCfg::BK - 1) / RingCfg::BK;
+  int best_rows = RingCfg::BM;
+  double best = 0;
+  for (int rows = RingCfg::BM; rows >= 32; rows -= 32) {
+    const int tiles_m = (R + rows - 1) / rows;
+    const int even = ((R + tiles_m - 1) / tiles_m + 31) / 32 * 32;
+    const int64_t tiles = (int64_t)E * ((R + even - 1) / even) * tiles_n;
+    const double per_k_tile = 0.45 + 0.14 * (even / 32);
+    const double cost = (double)((tiles + cus - 1) / cus) *
+                        (nk * (per_k_tile < 0.6 ? 0.6 : per_k_tile) + 6.5);
+    if (rows == RingCfg::BM || cost < 0.98 * best) {
+      best = cost;
+      best_rows = even;
+    }
+  }
+  return best_rows;
 }
 
 static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
@@ -2220,86 +2023,52 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                        const int32_t* tile_list = nullptr,
                        float mask_scale = 1.0f) {
   using Cfg = RingCfg;
-  const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  // (listed tiles are 256 rows high)
+  const int tile_rows =
+      tile_list != nullptr ? Cfg::BM : ring_tile_rows(E, R, N, K, cus);
+  const int tiles_m = (R + tile_rows - 1) / tile_rows;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n * E;
   MOE_REQUIRE(tiles <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
               "expert_ffn: too many tiles (%lld)", (long long)tiles);
-  const int cus = compute_units();
-  if (cus == 0) return MESH_MOE_E_HIP;
+  MOE_REQUIRE(mask_src == nullptr || (!relu && row_map == nullptr),
+              MESH_MOE_E_ARG,
+              "expert_ffn: masked result with relu or gathered rows");
   const unsigned blocks = (unsigned)(tiles < cus ? tiles : cus);
-  if (tile_list != nullptr && mask_src != nullptr) {
-    MOE_REQUIRE(!relu && row_map == nullptr, MESH_MOE_E_ARG,
-                "expert_ffn: masked result with relu or gathered rows");
-    auto k = grouped_gemm_bf16_ring_kernel<false, false, false, true, true>;
+  auto run = [&](auto k) -> int {
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
-        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-        mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1);
-    MOE_CHECK_LAUNCH("expert_ffn (mfma, listed tiles, masked result)");
+        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,
+        mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1, tile_rows);
+    MOE_CHECK_LAUNCH("expert_ffn (mfma, 256-column direct-to-LDS tiles)");
     return 0;
-  }
+  };
+#define MOE_RING(RELU_, GATHER_, MASKED_, LISTED_, TAILS_)                     \
+  run(grouped_gemm_bf16_ring_kernel<RELU_, GATHER_, false, MASKED_, LISTED_,   \
+                                    TAILS_>)
   if (tile_list != nullptr) {
-    // listed tiles: the first GEMM gathers its rows, the second does not
-#define MOE_RING_LISTED(RELU_, GATHER_)                                        \
-  do {                                                                         \
-    auto k = grouped_gemm_bf16_ring_kernel<RELU_, GATHER_, false, false, true>; \
-    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);                                          \
-    k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(                           \
-        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,     \
-        nullptr, tile_list, nullptr, 1.0f, nullptr, 0, 1);                     \
-  } while (0)
-    if (row_map != nullptr) {
-      if (relu) MOE_RING_LISTED(true, true);
-      else MOE_RING_LISTED(false, true);
-    } else {
-      if (relu) MOE_RING_LISTED(true, false);
-      else MOE_RING_LISTED(false, false);
-    }
-#undef MOE_RING_LISTED
-    MOE_CHECK_LAUNCH("expert_ffn (mfma, listed tiles)");
-    return 0;
+    if (mask_src != nullptr) return MOE_RING(false, false, true, true, false);
+    // the first GEMM gathers its rows, the second does not
+    if (row_map != nullptr)
+      return relu ? MOE_RING(true, true, false, true, false)
+                  : MOE_RING(false, true, false, true, false);
+    return relu ? MOE_RING(true, false, false, true, false)
+                : MOE_RING(false, false, false, true, false);
   }
-  if (mask_src != nullptr) {
-    MOE_REQUIRE(!relu && row_map == nullptr, MESH_MOE_E_ARG,
-                "expert_ffn: masked result with relu or gathered rows");
-    auto k = grouped_gemm_bf16_ring_kernel<false, false, false, true>;
-    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
-    k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
-        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-        mask_src, nullptr, nullptr, mask_scale, nullptr, 0, 1);
-    MOE_CHECK_LAUNCH("expert_ffn (mfma, masked result)");
-    return 0;
-  }
-  // an expert's last row tile is partly empty: the instantiation that skips
-  // its empty 32-row pieces
-  const bool tails = R % Cfg::BM != 0;
-#define MOE_RING_PLAIN(RELU_, GATHER_, TAILS_)                                 \
-  do {                                                                         \
-    auto k = grouped_gemm_bf16_ring_kernel<RELU_, GATHER_, false, false,       \
-                                           false, TAILS_>;                     \
-    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);                                          \
-    k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(                           \
-        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,     \
-        nullptr, nullptr, nullptr, 1.0f, nullptr, 0, 1);                       \
-  } while (0)
-#define MOE_RING_PLAIN_T(RELU_, GATHER_)                                       \
-  do {                                                                         \
-    if (tails) MOE_RING_PLAIN(RELU_, GATHER_, true);                           \
-    else MOE_RING_PLAIN(RELU_, GATHER_, false);                                \
-  } while (0)
-  if (row_map != nullptr) {
-    if (relu) MOE_RING_PLAIN_T(true, true);
-    else MOE_RING_PLAIN_T(false, true);
-    MOE_CHECK_LAUNCH("expert_ffn (mfma, gathered rows)");
-    return 0;
-  }
-  if (relu) MOE_RING_PLAIN_T(true, false);
-  else MOE_RING_PLAIN_T(false, false);
-#undef MOE_RING_PLAIN_T
-#undef MOE_RING_PLAIN
-  MOE_CHECK_LAUNCH("expert_ffn (mfma, spread direct-to-LDS loads)");
-  return 0;
+  // row tiles of fewer than 256 rows, or an expert's last one partly empty: the
+  // instantiation that skips empty 32-row pieces
+  const bool tails = R % tile_rows != 0 || tile_rows != Cfg::BM;
+#define MOE_RING_T(RELU_, GATHER_, MASKED_)                                    \
+  (tails ? MOE_RING(RELU_, GATHER_, MASKED_, false, true)                      \
+         : MOE_RING(RELU_, GATHER_, MASKED_, false, false))
+  if (mask_src != nullptr) return MOE_RING_T(false, false, true);
+  if (row_map != nullptr)
+    return relu ? MOE_RING_T(true, true, false) : MOE_RING_T(false, true, false);
+  return relu ? MOE_RING_T(true, false, false) : MOE_RING_T(false, false, false);
+#undef MOE_RING_T
+#undef MOE_RING
 }
 
 template <int TM, int TN>
@@ -2378,6 +2147,17 @@ static int launch_simple(const T* A, const T* B, T* C, int E, int R, int N,
   return 0;
 }
 
+static bool ring_shape(int R, int N, int K) {
+  return N >= 256 && R >= 128 && K % 64 == 0 && N % 8 == 0 &&
+         (int64_t)N * K < (1LL << 31);
+}
+// The calls that fold the dispatch into their first GEMM decline row counts
+// whose whole 256-row tiles would be more than a fifth padding.
+static bool ring_path_applies(int R, int N, int K) {
+  const int pad256 = (R + 255) / 256 * 256, pad128 = (R + 127) / 128 * 128;
+  return ring_shape(R, N, K) && pad128 * 5 >= pad256 * 4;
+}
+
 // C[e] = act(A[e] . B[e]^T) for every expert.
 // relu_mask_src (same shape and dtype as C): the kernels that can zero the
 // elements of C whose mask_src element is not positive while they write C do so
@@ -2410,27 +2190,16 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
     else if (skinny_applies(E, R, N, K))
       rc = launch_skinny((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
                          N, K, relu, st);
-    else if (N >= 256 && R >= 128 && K % 64 == 0 &&
-             (int64_t)R * K < (1LL << 31) && (int64_t)N * K < (1LL << 31)) {
-      // direct-to-LDS kernels; the persistent 256-row kernel unless 128-row
-      // tiles save more than a fifth of the padded rows (at 640 rows per
-      // expert, 3 x 256 against 5 x 128, the persistent kernel still wins:
-      // 0.43 against 0.50 ms for both GEMMs of benchmark config 2)
-      const bf16_t *a = (const bf16_t*)A, *b = (const bf16_t*)B;
-      bf16_t* c = (bf16_t*)C;
-      const int pad256 = (R + 255) / 256 * 256, pad128 = (R + 127) / 128 * 128;
-      // 256 x 256 tiles run 8 wavefronts (two per SIMD, 128 x 64 sub-tiles)
-      // with the loads spread over the MFMA steps
-      if (pad128 * 5 < pad256 * 4) {
-        rc = launch_dma<128, 256, 2>(a, b, c, E, R, N, K, relu, st);
-      } else if (relu_mask_src != nullptr && mask_applied != nullptr && !relu &&
-                 ((uintptr_t)relu_mask_src % 16) == 0) {
-        rc = launch_ring(a, b, c, E, R, N, K, false, st, nullptr, nullptr,
-                         (const bf16_t*)relu_mask_src, nullptr, mask_scale);
-        *mask_applied = rc == 0;
-      } else {
-        rc = launch_ring(a, b, c, E, R, N, K, relu, st);
-      }
+    else if (ring_shape(R, N, K) && (int64_t)R * K < (1LL << 31)) {
+      // 256-column tiles in persistent blocks of 8 wavefronts (two per SIMD),
+      // the loads spread over the MFMA steps
+      const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
+                         !relu && ((uintptr_t)relu_mask_src % 16) == 0;
+      rc = launch_ring((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R, N,
+                       K, relu, st, nullptr, nullptr,
+                       masks ? (const bf16_t*)relu_mask_src : nullptr, nullptr,
+                       masks ? mask_scale : 1.0f);
+      if (masks) *mask_applied = rc == 0;
     } else if (R >= 1024 && N >= 1024)
       rc = launch_mfma<256, 256, 64>((const bf16_t*)A, (const bf16_t*)B,
                                      (bf16_t*)C, E, R, N, K, relu, st);
@@ -2639,12 +2408,6 @@ __global__ void rows_used_kernel(const int32_t* __restrict__ fill,
   if (e < E)
     rows_used[e] = row_offsets[(int64_t)e * G + G - 1] +
                    fill[(int64_t)(G - 1) * E + e];
-}
-
-static bool ring_path_applies(int R, int N, int K) {
-  const int pad256 = (R + 255) / 256 * 256, pad128 = (R + 127) / 128 * 128;
-  return N >= 256 && R >= 128 && K % 64 == 0 && K % 8 == 0 && N % 8 == 0 &&
-         pad128 * 5 >= pad256 * 4 && (int64_t)N * K < (1LL << 31);
 }
 
 }  // namespace mesh_moe

@@ -1459,6 +1459,28 @@ def test_dispatched_ffn_of_few_rows(hip, case, activation):
   assert torch.equal(out, hip.combine(want.reshape(e, g, c, m), r, s))
 
 
+@pytest.mark.parametrize("shape", [
+    (3, 640, 128, 4096), (32, 640, 512, 1024), (5, 705, 192, 768), (1, 129, 64, 256),
+    (2, 320, 1088, 264), (1, 2000, 256, 776), (1, 5000, 128, 1280), (7, 257, 64, 520)],
+    ids=lambda s: "x".join(map(str, s)))
+def test_linear_row_tiles(hip, shape):
+  """Row counts that are spread over row tiles of 32 to 256 rows, the pieces of
+  a tile dealt out between its two halves: plain, with ReLU, and with the ReLU
+  mask of a gradient on the stores."""
+  for activation in ("linear", "relu"):
+    _check_linear(hip, shape, activation)
+  e, rows, k, n = shape
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(1)
+  dy = torch.randn((e, rows, k), generator=gen, device="cuda").to(torch.bfloat16)
+  w = torch.randn((e, n, k), generator=gen, device="cuda").to(torch.bfloat16)
+  mask = torch.randn((e, rows, n), generator=gen, device="cuda").to(torch.bfloat16)
+  da, _ = hip.expert_linear_backward(mask, dy, w)
+  masked, _ = hip.expert_linear_backward(mask, dy, w, da_relu_mask=mask)
+  assert torch.equal(masked, da * (mask > 0))
+  assert torch.equal(da, hip.expert_linear(dy, w))
+
+
 @pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
                                    (2, 6144, 776, 256), (29, 3000, 520, 760)],
                          ids=lambda s: "x".join(map(str, s)))
