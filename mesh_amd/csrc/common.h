@@ -13,6 +13,10 @@ namespace mesh_moe {
 // Per-thread error text returned by mesh_moe_last_error().
 void set_error(const char* fmt, ...);
 
+// Compute units of the current device (ffn.hip); 0 on failure, with the error
+// text set.
+int compute_units();
+
 // Batched C[e] = A[e] . B[e]^T (ffn.hip): A [E,R,K], B [E,N,K] of `dtype`
 // (MESH_MOE_F32 / MESH_MOE_BF16), C [E,R,N] of `dtype`, or float32 when
 // out_f32.  Float32 accumulation on the matrix cores for bf16.

@@ -1505,6 +1505,37 @@ def test_weight_gradient_of_split_reductions(hip, shape):
     assert bool(((dw[i].float() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("shape", [
+    (8, 320, 2048, 512), (8, 320, 512, 2048), (2, 33, 36, 100), (1, 32, 32, 32),
+    (1, 2000, 260, 1028), (40, 65, 68, 132), (3, 161, 1000, 64), (5, 97, 64, 300)],
+    ids=lambda s: "x".join(map(str, s)))
+def test_linear_float32_tiles(hip, shape):
+  """The float32 kernel's block tiles, with their edges inside a tile and a last
+  K tile that is partly there: products, with ReLU, with a gradient's ReLU mask
+  on the stores, and weight gradients from rows as they lie.  The bound: K / 2
+  ulps of the sum of magnitudes for a sum of K products."""
+  e, rows, k, n = shape
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(shape))
+  a, dy, w = (torch.randn(s, generator=gen, device="cuda")
+              for s in ((e, rows, n), (e, rows, k), (e, n, k)))
+
+  def check(got, x, y, terms, keep=None):
+    want = x.double() @ y.double()
+    bound = terms * 2.0 ** -24 * (x.double().abs() @ y.double().abs())
+    if keep is not None:
+      want = want * keep
+      assert not bool(got[~keep].any())
+    assert bool(((got.double() - want).abs() <= bound).all())
+  wt = w.transpose(1, 2)
+  y = hip.expert_linear(dy, w)
+  check(y, dy, wt, k)
+  assert torch.equal(hip.expert_linear(dy, w, activation="relu"), y.clamp(min=0))
+  da, dw = hip.expert_linear_backward(a, dy, w, da_relu_mask=a)
+  check(da, dy, wt, k, a > 0)
+  check(dw, a.transpose(1, 2), dy, rows)
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(2, 256, 512, 128), (1, 100, 72, 40),
                                    (1, 4096, 1024, 256)],
