@@ -14,11 +14,15 @@ namespace mesh_moe {
 
 // ---------------------------------------------------------------------------
 // Router logits: logits[b,t,e] = sum_m x[b,t,m] * w[b,m,e] (+ bias[e]).
-// One block = 64 tokens; thread (tok = tid % 64, eg = tid / 64) accumulates
-// experts eg*EPT .. eg*EPT+EPT-1 with EPT = ceil(E / 4) <= 32.  x and w are
-// staged through LDS as float32 in chunks of KC columns of M.
+// One block = TOK tokens; thread (tok = tid % TOK, eg = tid / TOK) accumulates
+// experts eg*ept .. eg*ept+ept-1 with ept = ceil(E / (256 / TOK)) <= 32, in the
+// order of m.  x and w are staged through LDS as float32 in chunks of KC columns
+// of M; the next chunk is loaded while one is multiplied.
+//
+// Bound by the latency of that chain of chunks: blocks of 64 tokens are kept
+// for calls that fill the compute units with them, smaller calls take 16 tokens
+// a block.  2048 tokens x 512, 8 experts, float32: 22.9 -> 11.5 us.
 // ---------------------------------------------------------------------------
-constexpr int RL_TOK = 64;
 constexpr int RL_KC = 64;
 constexpr int RL_MAX_EPT = 32;
 
@@ -26,55 +30,68 @@ constexpr int RL_MAX_EPT = 32;
 // experts is unrolled without conditions: with EPT = 32 and a condition per
 // expert the 64 x 32 scalar branches per chunk were the whole run time at
 // E = 8; the surplus products read the next group's weights and are dropped)
-template <typename T, int EPT>
+template <typename T, int EPT, int TOK>
 __global__ __launch_bounds__(256) void router_logits_kernel(
     const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ bias, float* __restrict__ logits,
     int64_t tokens, int M, int E, int ept) {
+  constexpr int GROUPS = 256 / TOK;
+  constexpr int XV = TOK * RL_KC / 256;            // loads per thread and chunk
+  constexpr int WV = EPT * GROUPS * RL_KC / 256;
   extern __shared__ float smem[];
-  float* xs = smem;                       // [RL_TOK][RL_KC + 1]
-  float* ws = smem + RL_TOK * (RL_KC + 1);  // [RL_KC][E] + 4 EPT
+  float* xs = smem;                       // [TOK][RL_KC + 1]
+  float* ws = smem + TOK * (RL_KC + 1);   // [RL_KC][E] + GROUPS EPT
   const int b = blockIdx.y;
-  const int64_t t0 = (int64_t)blockIdx.x * RL_TOK;
+  const int64_t t0 = (int64_t)blockIdx.x * TOK;
   const int tid = threadIdx.x;
-  const int tok = tid & 63;
-  const int eg = tid >> 6;
+  const int tok = tid % TOK;
+  const int eg = tid / TOK;
   const T* xb = x + ((int64_t)b * tokens) * M;
   const T* wb = w + (int64_t)b * M * E;
+  const int wn = RL_KC * E;               // weights of a chunk, contiguous
   float acc[EPT];
 #pragma unroll
   for (int j = 0; j < EPT; ++j) acc[j] = 0.f;
 
-  for (int k0 = 0; k0 < M; k0 += RL_KC) {
-    // x tile: 64 tokens x KC, coalesced along M; a thread's 16 loads are all
-    // issued before the first LDS write (one at a time, each waited for, the
-    // staging took 30 us per chunk)
-    float xv[RL_TOK * RL_KC / 256];
+  // all loads of a chunk are issued together (one at a time, each waited for,
+  // the staging took 30 us per chunk)
+  float xv[XV], wv[WV];
+  auto load = [&](int k0) {
 #pragma unroll
-    for (int u = 0; u < RL_TOK * RL_KC / 256; ++u) {
+    for (int u = 0; u < XV; ++u) {
       const int i = tid + u * 256;
-      const int r = i / RL_KC, c = i % RL_KC;
-      const int64_t t = t0 + r;
-      xv[u] = (t < tokens && k0 + c < M) ? load_f32<T>(xb + t * M + k0 + c) : 0.f;
+      const int64_t t = t0 + i / RL_KC;
+      const int c = k0 + i % RL_KC;
+      xv[u] = (t < tokens && c < M) ? load_f32<T>(xb + t * M + c) : 0.f;
     }
+    const int left = (int)min((int64_t)wn, (int64_t)(M - k0) * E);
 #pragma unroll
-    for (int u = 0; u < RL_TOK * RL_KC / 256; ++u) {
+    for (int u = 0; u < WV; ++u) {
+      const int i = tid + u * 256;
+      wv[u] = i < left ? load_f32<T>(wb + (int64_t)k0 * E + i) : 0.f;
+    }
+  };
+  load(0);
+  for (int k0 = 0; k0 < M; k0 += RL_KC) {
+#pragma unroll
+    for (int u = 0; u < XV; ++u) {
       const int i = tid + u * 256;
       xs[(i / RL_KC) * (RL_KC + 1) + i % RL_KC] = xv[u];
     }
-    for (int i = tid; i < RL_KC * E; i += 256) {
-      int r = i / E, c = i % E;
-      float v = 0.f;
-      if (k0 + r < M) v = load_f32<T>(wb + (int64_t)(k0 + r) * E + c);
-      ws[i] = v;
+#pragma unroll
+    for (int u = 0; u < WV; ++u) {
+      const int i = tid + u * 256;
+      if (i < wn) ws[i] = wv[u];
     }
     __syncthreads();
+    if (k0 + RL_KC < M) load(k0 + RL_KC);
     const int e0 = eg * ept;
+#pragma unroll 8
     for (int k = 0; k < RL_KC; ++k) {
-      float xv = xs[tok * (RL_KC + 1) + k];
+      float xk = xs[tok * (RL_KC + 1) + k];
       const float* wr = ws + k * E + e0;
 #pragma unroll
-      for (int j = 0; j < EPT; ++j) acc[j] = fmaf(xv, wr[j], acc[j]);
+      for (int j = 0; j < EPT; ++j) acc[j] = fmaf(xk, wr[j], acc[j]);
     }
     __syncthreads();
   }
@@ -272,8 +289,7 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(
 // ---------------------------------------------------------------------------
 // Gating step 1: per token softmax, top-2, gate normalisation, second-place
 // policy; per block column sums of the balancing-loss proxies.
-// Grid (blocks per group, G); one thread per token; the logits tile is staged
-// in LDS with row stride E+1 so that per-thread row walks are conflict-free.
+// Grid (blocks per group, G).
 // ---------------------------------------------------------------------------
 // Accesses that are coherent across the GPU's compute dies without a cache
 // flush.  Each die (XCD) has its own L2; an ordinary store may sit there, and
@@ -335,181 +351,18 @@ constexpr int GATE_MAX_GROUP = 16384;
 // bit 0 of the step-1 `kept` byte: the token competes for a slot (mask_k after
 // importance and policy); bit 1 (second choice only): mask_2 before the policy,
 // which is what the second-place loss counts (moe.py:1430).
-//
-// gate_select_tile does the work for `ntok` tokens (tokens t0 .. of group g,
-// block `blk` of the group) whose logits already sit in LDS as tile[ntok][ld];
-// every thread of the block must call it.
-//
-// With `ch` (LDS, 3 * ch_stride int16) the expert a token competes for with
-// its first / second choice, and the expert the loss's extra count sees, also
-// go there (-1 = none) for the in-block ranking of the single-launch kernel,
-// which then writes `pos` itself.
-template <typename IT>
-__device__ __forceinline__ void gate_select_tile(
-    float* tile, float* isone, int ld, int ntok, int g, int blk, int t0,
-    const IT* __restrict__ importance, const float* __restrict__ second_uniform,
-    const GateParams& p, int32_t* __restrict__ idx, int32_t* __restrict__ pos,
-    float* __restrict__ gate, uint8_t* __restrict__ kept,
-    float* __restrict__ part1, float* __restrict__ part2,
-    int16_t* ch = nullptr, int ch_stride = 0) {
-  const int E = p.E, S = p.S;
-  const int tid = threadIdx.x;
-  float qscale = 0.f, zterm = 0.f;
-  int i1 = 0;
-  bool sel1 = false;
-  if (tid < ntok) {
-    float* row = tile + tid * ld;
-    const int64_t t = (int64_t)g * S + t0 + tid;
-    float m = row[0];
-    for (int e = 1; e < E; ++e) m = fmaxf(m, row[e]);       // reduce_max
-    const float negm = -m;
-    float s = 0.f;
-    for (int e = 0; e < E; ++e) s += expf(row[e] + negm);   // exp, reduce_sum
-    const float neglse = -(logf(s) + m);                    // log + max
-    float g1 = -1.f;
-    for (int e = 0; e < E; ++e) {
-      float pe = expf(row[e] + neglse);                     // exp(log_softmax)
-      row[e] = pe;
-      if (pe > g1) { g1 = pe; i1 = e; }                     // first argmax
-    }
-    sel1 = true;
-    if (p.router == ROUTER_SWITCH && second_uniform != nullptr) {
-      // policy "sample" (moe.py:1213-1216): the expert is the first arg-max of
-      // the caller's choice logits [G,S,E] (router logits plus Gumbel noise
-      // times the temperature, ops.py:5070-5086), which arrive through the
-      // pointer the top-2 mode uses for its uniform samples; the gate is the
-      // softmax probability of that expert (mtf.gather of raw_gates)
-      const float* ch = second_uniform + t * E;
-      float best = ch[0];
-      i1 = 0;
-      for (int e = 1; e < E; ++e) {
-        const float v = ch[e];
-        if (v > best) { best = v; i1 = e; }
-      }
-      g1 = row[i1];
-    }
-    if (p.router == ROUTER_SWITCH) {
-      // one choice, raw probability as the gate (moe.py:1207-1228); the load
-      // balancing loss counts every token's arg-max (density_1 is taken
-      // before the importance mask, moe.py:1224) and an unmasked proxy
-      if (importance != nullptr)
-        sel1 = (load_f32<IT>(importance + t) == 1.0f);
-      if (!sel1) g1 = g1 * 0.0f;
-      idx[t * 2 + 0] = i1;
-      idx[t * 2 + 1] = 0;
-      if (ch == nullptr) {
-        pos[t * 2 + 0] = 0;
-        pos[t * 2 + 1] = 0;
-      } else {
-        ch[tid] = sel1 ? (int16_t)i1 : (int16_t)-1;
-        ch[ch_stride + tid] = -1;
-        ch[2 * ch_stride + tid] = (int16_t)i1;
-      }
-      gate[t * 2 + 0] = g1;
-      gate[t * 2 + 1] = 0.0f;
-      kept[t * 2 + 0] = (sel1 ? 1 : 0) | 2;   // bit 1: counted by density_1
-      kept[t * 2 + 1] = 0;
-      isone[tid] = 1.0f;
-      const float lse = -neglse;                            // reduce_logsumexp
-      zterm = sel1 ? lse * lse : 0.0f;                      // moe.py:1256-1259
-    } else {
-    bool sel2 = true;
-    if (importance != nullptr) {
-      float imp = load_f32<IT>(importance + t);
-      if (p.importance_from_slot_gate)                      // moe.py:725-727
-        imp = 0.5f * ((imp > 0.5f ? 1.0f : 0.0f) + (imp > 0.0f ? 1.0f : 0.0f));
-      sel1 = (imp == 1.0f);                                 // moe.py:1402-1404
-      sel2 = (imp > 0.0f);                                  // moe.py:1411
-    }
-    if (!sel1) g1 = g1 * 0.0f;
-    // gates_without_top_1 = raw_gates * (1 - mask_1); its first argmax.
-    float g2 = -1.f, qsum = 0.f;
-    int i2 = 0;
-    for (int e = 0; e < E; ++e) {
-      float keep = (sel1 && e == i1) ? 0.0f : 1.0f;         // 1 + (-mask_1)
-      float q = row[e] * keep;
-      qsum += q;
-      if (q > g2) { g2 = q; i2 = e; }
-    }
-    const float denom = (g1 + g2) + 1e-9f;                  // moe.py:1413
-    const float r = 1.0f / denom;                           // reciprocal
-    const float g1n = g1 * r, g2n = g2 * r;
-    const bool sel2_loss = sel2;
-    if (p.policy == MESH_MOE_SECOND_NONE) {
-      sel2 = false;
-    } else if (p.policy == MESH_MOE_SECOND_THRESHOLD) {
-      sel2 = sel2 && (g2n > p.threshold);
-    } else if (p.policy == MESH_MOE_SECOND_RANDOM) {
-      sel2 = sel2 && (second_uniform[t] < g2n * p.inv_threshold);
-    }
-    idx[t * 2 + 0] = i1;
-    idx[t * 2 + 1] = i2;
-    if (ch == nullptr) {
-      pos[t * 2 + 0] = 0;
-      pos[t * 2 + 1] = 0;
-    } else {
-      ch[tid] = sel1 ? (int16_t)i1 : (int16_t)-1;
-      ch[ch_stride + tid] = sel2 ? (int16_t)i2 : (int16_t)-1;
-      ch[2 * ch_stride + tid] = sel2_loss ? (int16_t)i2 : (int16_t)-1;
-    }
-    gate[t * 2 + 0] = g1n;
-    gate[t * 2 + 1] = g2n;
-    kept[t * 2 + 0] = sel1 ? 1 : 0;
-    kept[t * 2 + 1] = (sel2 ? 1 : 0) | (sel2_loss ? 2 : 0);
-    isone[tid] = sel1 ? 1.0f : 0.0f;
-    qscale = 1.0f / (qsum + 1e-9f);                         // moe.py:1433-1434
-    }
-  }
-  __syncthreads();
-  // density_1_proxy partial: sum over the block's tokens of p * (imp == 1)
-  for (int e = tid; e < E; e += blockDim.x) {
-    float s = 0.f;
-    for (int r = 0; r < ntok; ++r) s += tile[r * ld + e] * isone[r];
-    part1[((int64_t)g * p.nblk + blk) * E + e] = s;
-  }
-  if (p.router == ROUTER_SWITCH) {
-    // per-block sums for the z-loss: column 0 = sum of logsumexp^2 over the
-    // tokens with importance 1, column 1 = how many those are
-    __syncthreads();
-    if (tid < ntok) {
-      tile[tid * ld + 0] = zterm;
-      tile[tid * ld + 1] = sel1 ? 1.0f : 0.0f;
-    }
-    __syncthreads();
-    if (tid < 2) {
-      float s = 0.f;
-      for (int r = 0; r < ntok; ++r) s += tile[r * ld + tid];
-      part2[((int64_t)g * p.nblk + blk) * E + tid] = s;
-    }
-  } else if (p.use_second_place_loss) {
-    __syncthreads();
-    if (tid < ntok) {
-      float* row = tile + tid * ld;
-      for (int e = 0; e < E; ++e) {
-        float keep = (sel1 && e == i1) ? 0.0f : 1.0f;
-        row[e] = (row[e] * keep) * qscale;
-      }
-    }
-    __syncthreads();
-    for (int e = tid; e < E; e += blockDim.x) {
-      float s = 0.f;
-      for (int r = 0; r < ntok; ++r) s += tile[r * ld + e];
-      part2[((int64_t)g * p.nblk + blk) * E + e] = s;
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
-// gate_select_tile for the projection kernel, straight from the matrix-core
-// accumulators: 256 threads, 128 tokens, two lanes per token.  After the
-// 32x32x16 MFMAs lane l of a wavefront holds, for token l % 32 and per
+// gate_select_kernel's work for the projection kernel, straight from the
+// matrix-core accumulators: 256 threads, 128 tokens, two lanes per token.
+// After the 32x32x16 MFMAs lane l of a wavefront holds, for token l % 32 and per
 // 32-expert tile j, the logits of experts 32 j + 8 q + 4 (l / 32) + r (q, r =
 // 0..3): lanes l and l + 32 together hold the token's whole row, in alternating
 // groups of four experts.  Each lane does the exponentials of its half (two per
 // expert, the bulk of the work); every float32 sum still runs in expert order
 // (the running sum changes lanes after every group of four) and a tie between
 // the two lanes' arg-max candidates goes to the lower expert, so every
-// per-token result is bit for bit that of gate_select_tile.  The probabilities
+// per-token result is bit for bit that of gate_select_kernel.  The probabilities
 // go to LDS (tile [128][ld], ld % 4 == 0) for the per-block column sums of the
 // loss, which are split over four row ranges; colpart: LDS [4][E] floats.
 // ---------------------------------------------------------------------------
@@ -813,31 +666,221 @@ __device__ __forceinline__ void gate_select_acc_tile(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Step 1 from logits in memory.  A block has SELECT_TOKENS tokens and sixteen
+// lanes per token; lane l does the exponentials and comparisons of experts l,
+// l + 16, ...  The two sums over a token's experts that decide its gates still
+// run in expert order, read back from LDS (every lane of the token runs the
+// same chain), and a tie between two lanes' candidates goes to the lower
+// expert: the per-token results do not depend on the split.  One thread per
+// token walking its row was a chain of four passes of E dependent steps, and
+// 256 tokens per block left most compute units without one: 64 tokens of 64
+// experts 17.6 -> 8.2 us, 6 groups of 1500 tokens, 16 experts 16.5 -> 6.8 us.
+// ---------------------------------------------------------------------------
+constexpr int SELECT_TOKENS = 64;
+constexpr int SELECT_LANES = 16;
+constexpr int SELECT_THREADS = SELECT_TOKENS * SELECT_LANES;
+
+__host__ __device__ constexpr int select_row_floats(int E) {
+  return (E + 3) / 4 * 4 + 4;            // 16-byte rows, odd in units of 16 bytes
+}                                        // for E = 8 n
+
 template <typename IT>
-__global__ __launch_bounds__(256) void gate_select_kernel(
+__global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     const float* __restrict__ logits, const IT* __restrict__ importance,
     const float* __restrict__ second_uniform, GateParams p,
     int32_t* __restrict__ idx, int32_t* __restrict__ pos,
     float* __restrict__ gate, uint8_t* __restrict__ kept,
     float* __restrict__ part1, float* __restrict__ part2) {
-  extern __shared__ float smem[];
+  extern __shared__ __attribute__((aligned(16))) float smem[];
   const int E = p.E, S = p.S;
-  const int ld = E + 1;
-  float* tile = smem;                                  // [tt][E+1]
-  float* isone = smem + (size_t)p.tt * ld;             // [tt]
-  const int g = blockIdx.y;
-  const int blk = blockIdx.x;
-  const int t0 = blk * p.tt;
-  const int ntok = min(p.tt, S - t0);
-  const int tid = threadIdx.x;
-  const float* src = logits + ((int64_t)g * S + t0) * E;
-  for (int i = tid; i < ntok * E; i += blockDim.x) {
-    int r = i / E, c = i - r * E;
-    tile[r * ld + c] = src[i];
+  const int ld = select_row_floats(E);
+  float* tile = smem;                                  // [SELECT_TOKENS][ld]
+  float* isone = tile + SELECT_TOKENS * ld;            // [SELECT_TOKENS]
+  float* cols = isone + SELECT_TOKENS;                 // [SELECT_THREADS]
+  const int g = blockIdx.y, blk = blockIdx.x;
+  const int t0 = blk * SELECT_TOKENS;
+  const int ntok = min(SELECT_TOKENS, S - t0);
+  const int tid = threadIdx.x, lane = tid % SELECT_LANES;
+  const int tok = tid / SELECT_LANES;
+  const bool live = tok < ntok;
+  // experts this lane walks: none for a token that does not exist
+  const int e_end = live ? E : 0;
+  const int64_t t = (int64_t)g * S + t0 + (live ? tok : 0);
+  const float* src = logits + t * E;
+  float* row = tile + tok * ld;
+  const bool sw = p.router == ROUTER_SWITCH;
+
+  float m = -INFINITY;
+  for (int e = lane; e < e_end; e += SELECT_LANES) m = fmaxf(m, src[e]);
+#pragma unroll
+  for (int d = 1; d < SELECT_LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+  const float negm = -m;                                    // reduce_max
+  for (int e = lane; e < e_end; e += SELECT_LANES)
+    row[e] = expf(src[e] + negm);
+  __syncthreads();
+  // exp, reduce_sum: in expert order
+  float s = 0.f;
+  if (live) {
+    int e = 0;
+    for (; e + 4 <= E; e += 4) {
+      const float4 v = *reinterpret_cast<const float4*>(row + e);
+      s += v.x; s += v.y; s += v.z; s += v.w;
+    }
+    for (; e < E; ++e) s += row[e];
   }
   __syncthreads();
-  gate_select_tile<IT>(tile, isone, ld, ntok, g, blk, t0, importance,
-                       second_uniform, p, idx, pos, gate, kept, part1, part2);
+  // the larger value, of equal ones the lower expert
+  auto first_max = [&](float& v, int& i) {
+#pragma unroll
+    for (int d = 1; d < SELECT_LANES; d *= 2) {
+      const float v2 = __shfl_xor(v, d);
+      const int i2 = __shfl_xor(i, d);
+      if (v2 > v || (v2 == v && i2 < i)) { v = v2; i = i2; }
+    }
+  };
+  const float neglse = -(logf(s) + m);                      // log + max
+  float g1 = -1.f;
+  int i1 = 0;
+  for (int e = lane; e < e_end; e += SELECT_LANES) {
+    const float pe = expf(src[e] + neglse);                 // exp(log_softmax)
+    row[e] = pe;
+    if (pe > g1) { g1 = pe; i1 = e; }                       // first argmax
+  }
+  first_max(g1, i1);
+  __syncthreads();
+  bool sel1 = live;
+  float qscale = 0.f;
+  if (sw) {
+    if (second_uniform != nullptr) {
+      // policy "sample" (moe.py:1213-1216): the expert is the first arg-max of
+      // the caller's choice logits [G,S,E] (router logits plus Gumbel noise
+      // times the temperature, ops.py:5070-5086), which arrive through the
+      // pointer the top-2 mode uses for its uniform samples; the gate is the
+      // softmax probability of that expert (mtf.gather of raw_gates)
+      const float* ch = second_uniform + t * E;
+      float best = -INFINITY;
+      i1 = 0;
+      for (int e = lane; e < e_end; e += SELECT_LANES) {
+        const float v = ch[e];
+        if (v > best) { best = v; i1 = e; }
+      }
+      first_max(best, i1);
+      // (nothing compares greater than a NaN in the first place)
+      if (live && ch[0] != ch[0]) i1 = 0;
+      if (live) g1 = row[i1];
+    }
+    // one choice, raw probability as the gate (moe.py:1207-1228); the load
+    // balancing loss counts every token's arg-max (density_1 is taken
+    // before the importance mask, moe.py:1224) and an unmasked proxy
+    if (live && importance != nullptr)
+      sel1 = (load_f32<IT>(importance + t) == 1.0f);
+    if (!sel1) g1 = g1 * 0.0f;
+    if (live && lane == 0) {
+      idx[t * 2 + 0] = i1;
+      idx[t * 2 + 1] = 0;
+      pos[t * 2 + 0] = 0;
+      pos[t * 2 + 1] = 0;
+      gate[t * 2 + 0] = g1;
+      gate[t * 2 + 1] = 0.0f;
+      kept[t * 2 + 0] = (sel1 ? 1 : 0) | 2;   // bit 1: counted by density_1
+      kept[t * 2 + 1] = 0;
+      isone[tok] = 1.0f;
+    }
+  } else {
+    bool sel2 = live;
+    if (live && importance != nullptr) {
+      float imp = load_f32<IT>(importance + t);
+      if (p.importance_from_slot_gate)                      // moe.py:725-727
+        imp = 0.5f * ((imp > 0.5f ? 1.0f : 0.0f) + (imp > 0.0f ? 1.0f : 0.0f));
+      sel1 = (imp == 1.0f);                                 // moe.py:1402-1404
+      sel2 = (imp > 0.0f);                                  // moe.py:1411
+    }
+    if (!sel1) g1 = g1 * 0.0f;
+    // gates_without_top_1 = raw_gates * (1 - mask_1); its first argmax.
+    const int masked = sel1 ? i1 : -1;                      // 1 + (-mask_1)
+    float g2 = -1.f;
+    int i2 = 0;
+    for (int e = lane; e < e_end; e += SELECT_LANES) {
+      const float q = row[e] * (e == masked ? 0.0f : 1.0f);
+      if (q > g2) { g2 = q; i2 = e; }
+    }
+    first_max(g2, i2);
+    if (p.use_second_place_loss && live) {
+      float qsum = 0.f;
+      for (int e = 0; e < E; ++e) qsum += row[e] * (e == masked ? 0.0f : 1.0f);
+      qscale = 1.0f / (qsum + 1e-9f);                       // moe.py:1433-1434
+    }
+    const float denom = (g1 + g2) + 1e-9f;                  // moe.py:1413
+    const float r = 1.0f / denom;                           // reciprocal
+    const float g1n = g1 * r, g2n = g2 * r;
+    const bool sel2_loss = sel2;
+    if (live && lane == 0) {
+      if (p.policy == MESH_MOE_SECOND_NONE) {
+        sel2 = false;
+      } else if (p.policy == MESH_MOE_SECOND_THRESHOLD) {
+        sel2 = sel2 && (g2n > p.threshold);
+      } else if (p.policy == MESH_MOE_SECOND_RANDOM) {
+        sel2 = sel2 && (second_uniform[t] < g2n * p.inv_threshold);
+      }
+      idx[t * 2 + 0] = i1;
+      idx[t * 2 + 1] = i2;
+      pos[t * 2 + 0] = 0;
+      pos[t * 2 + 1] = 0;
+      gate[t * 2 + 0] = g1n;
+      gate[t * 2 + 1] = g2n;
+      kept[t * 2 + 0] = sel1 ? 1 : 0;
+      kept[t * 2 + 1] = (sel2 ? 1 : 0) | (sel2_loss ? 2 : 0);
+      isone[tok] = sel1 ? 1.0f : 0.0f;
+    }
+  }
+  // sums over the block's tokens, per expert: part[e] = sum of tile[r][e] *
+  // (weights ? weights[r] : 1); the rows in up to SELECT_LANES ranges, whose
+  // sums are added in order
+  auto column_sums = [&](const float* weights, float* part) {
+    int el = 2;
+    while (el < E) el *= 2;
+    const int ranges = min(SELECT_LANES, SELECT_THREADS / el);
+    const int e = tid % el, c = tid / el;
+    const int per = SELECT_TOKENS / ranges;
+    __syncthreads();
+    if (e < E && c < ranges) {
+      float a = 0.f;
+      for (int r = c * per; r < min(ntok, (c + 1) * per); ++r)
+        a += weights != nullptr ? tile[r * ld + e] * weights[r]
+                                : tile[r * ld + e];
+      cols[c * el + e] = a;
+    }
+    __syncthreads();
+    if (tid < E) {
+      float a = 0.f;
+      for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
+      part[((int64_t)g * p.nblk + blk) * E + tid] = a;
+    }
+  };
+  // density_1_proxy partial: sum over the block's tokens of p * (imp == 1)
+  column_sums(isone, part1);
+  if (sw) {
+    // per-block sums for the z-loss: column 0 = sum of logsumexp^2 over the
+    // tokens with importance 1, column 1 = how many those are
+    __syncthreads();
+    if (lane == 0) {
+      const float lse = -neglse;                            // reduce_logsumexp
+      cols[tok] = sel1 ? lse * lse : 0.0f;                  // moe.py:1256-1259
+      cols[SELECT_TOKENS + tok] = sel1 ? 1.0f : 0.0f;
+    }
+    __syncthreads();
+    if (tid < 2) {
+      float a = 0.f;
+      for (int r = 0; r < ntok; ++r) a += cols[tid * SELECT_TOKENS + r];
+      part2[((int64_t)g * p.nblk + blk) * E + tid] = a;
+    }
+  } else if (p.use_second_place_loss) {
+    __syncthreads();
+    for (int e = lane; e < e_end; e += SELECT_LANES)
+      row[e] = (row[e] * (sel1 && e == i1 ? 0.0f : 1.0f)) * qscale;
+    column_sums(nullptr, part2);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -911,7 +954,7 @@ __device__ __forceinline__ bool arrive_is_last(unsigned long long* word,
 }
 
 // Ranks of the block's choices.  ch [3][128] int16 in LDS as written by
-// gate_select_tile; wcnt [3][2][E] int32 in LDS.  Wavefront w ranks choice
+// gate_select_kernel; wcnt [3][2][E] int32 in LDS.  Wavefront w ranks choice
 // w / 2 of tokens 64 (w % 2) ..; with `loss2` wavefronts 0 and 1 also count
 // the third array.  A lane's rank is the number of lower lanes of its
 // wavefront that name the same expert.  Writes pos (rank within the block)
@@ -1174,7 +1217,7 @@ __device__ __forceinline__ void gate_group_tail(
 // ---------------------------------------------------------------------------
 // Router projection fused with gating step 1: the K loop of router_mfma_kernel,
 // then the block's 128 x E logits go from the accumulators to LDS (never to
-// HBM unless `logits` is given) and gate_select_tile runs on them.  Needs the
+// HBM unless `logits` is given) and step 1 runs on them.  Needs the
 // group size to be a multiple of 128 so that a block's tokens share a group.
 // ---------------------------------------------------------------------------
 template <int NT, typename IT>
@@ -1340,6 +1383,57 @@ __global__ __launch_bounds__(256) void router_gate_kernel(
   (void)tokens_total;
 }
 
+// The balancing loss from the groups' terms; one thread.  COHERENT: the terms
+// were written by other blocks of the same launch (see st_dev).
+template <bool COHERENT>
+__device__ __forceinline__ void gate_loss_value(const GateParams& p,
+                                                const float* gsum_in,
+                                                float* loss) {
+  struct Terms {
+    const float* q;
+    __device__ float operator[](int i) const {
+      return COHERENT ? ld_dev(q + i) : q[i];
+    }
+  } gsum = {gsum_in};
+  float s1 = 0.f, s2 = 0.f;
+  for (int g = 0; g < p.G; ++g) {
+    s1 += gsum[g * GSUM];
+    s2 += gsum[g * GSUM + 1];
+  }
+  const float inv_ge = (float)(1.0 / ((double)p.G * (double)p.E));
+  const float ee = (float)((double)p.E * (double)p.E);
+  float l;
+  if (p.router == ROUTER_SWITCH) {
+    if (p.has_importance) {
+      // mean over [G,E,S] of proxy[g,e] * (imp[g,s] == 1) * density[g,e]
+      // (moe.py:1229-1234): each group's term counts once per such token
+      float sm = 0.f;
+      for (int g = 0; g < p.G; ++g) sm += gsum[g * GSUM] * gsum[g * GSUM + 2];
+      l = (sm * (float)(1.0 / ((double)p.G * (double)p.E * (double)p.S))) * ee;
+    } else {
+      l = (s1 * inv_ge) * ee;
+    }
+    if (p.num_microbatches > 1)
+      l = l * (float)(1.0 / (double)p.num_microbatches);     // moe.py:1235-1238
+    if (p.use_z_loss) {                                      // moe.py:1253-1266
+      float z = 0.f, n = 0.f;
+      for (int g = 0; g < p.G; ++g) {
+        z += gsum[g * GSUM + 3];
+        n += gsum[g * GSUM + 2];
+      }
+      const float mb = (float)(p.num_microbatches > 0 ? p.num_microbatches : 1);
+      l = l + p.z_loss_coef * (z / (n * mb));
+    }
+    loss[0] = l;
+    return;
+  }
+  l = (s1 * inv_ge) * ee;                                    // moe.py:1423-1424
+  if (p.use_second_place_loss) l = l + ((s2 * inv_ge) * ee) * 0.5f;
+  if (p.num_microbatches > 1)
+    l = l * (float)(1.0 / (double)p.num_microbatches);       // moe.py:1439-1442
+  loss[0] = l;
+}
+
 // ---------------------------------------------------------------------------
 // Gating step 2: capacity positions for one group per block (moe.py:1472-1496).
 // Thread (e = tid % EL, chunk = tid / EL) counts, over its chunk of the
@@ -1366,13 +1460,25 @@ __device__ __forceinline__ int cap_match8(const uint4& v, int e) {
 }
 
 // Number of entries of ch[s_begin, s_end) equal to e; with `vec` the range
-// starts 16-byte aligned and is read eight ids at a time.
+// starts 16-byte aligned and is read eight ids at a time, up to the next
+// multiple of eight.
 __device__ __forceinline__ int cap_count(const int16_t* ch, int s_begin,
                                          int s_end, int e, bool vec) {
   int c = 0, s = s_begin;
-  if (vec)
+  if (vec) {
     for (; s + 8 <= s_end; s += 8)
       c += cap_match8(*reinterpret_cast<const uint4*>(ch + s), e);
+    const int n = s_end - s;             // of the next eight only the first n
+    if (n > 0) {
+      const uint4 v = *reinterpret_cast<const uint4*>(ch + s);
+      auto only = [&](uint32_t w, int at) {
+        return n >= at + 2 ? w : n == at + 1 ? w | 0xffff0000u : 0xffffffffu;
+      };
+      c += cap_match8(make_uint4(only(v.x, 0), only(v.y, 2), only(v.z, 4),
+                                 only(v.w, 6)), e);
+    }
+    return c;
+  }
   for (; s < s_end; ++s) c += (ch[s] == e);
   return c;
 }
@@ -1381,19 +1487,20 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     GateParams p, const int32_t* __restrict__ idx, int32_t* __restrict__ pos,
     float* __restrict__ gate, uint8_t* __restrict__ kept,
     int32_t* __restrict__ fill, const float* __restrict__ part1,
-    const float* __restrict__ part2, float* __restrict__ gsum, int el) {
+    const float* __restrict__ part2, float* __restrict__ gsum, int el, int ss,
+    float* __restrict__ loss) {
   extern __shared__ __attribute__((aligned(16))) int32_t smem_i[];
   const int S = p.S, E = p.E, C = p.C;
   int32_t* cnt = smem_i;                        // [nchunks][el] = CAP_THREADS
   int32_t* pre = cnt + CAP_THREADS;             // [nchunks][el]: first slots
   int32_t* tot = pre + CAP_THREADS;             // [3][el]: total1,total2,loss2
   float* prod = reinterpret_cast<float*>(tot + 3 * el);  // [2][el]
-  int16_t* c1 = reinterpret_cast<int16_t*>(prod + 2 * el);  // [S]
-  int16_t* c2 = c1 + S;                                      // [S]
-  int16_t* c2l = c2 + S;                                     // [S] (loss only)
+  int16_t* c1 = reinterpret_cast<int16_t*>(prod + 2 * el);  // [ss], ss >= S
+  int16_t* c2 = c1 + ss;                                     // [ss]
+  int16_t* c2l = c2 + ss;                                    // [ss] (loss only)
   // first-choice gates of the group, for the by-gate slot order; float-aligned
-  // because 3 * S int16 may end on an odd 2-byte boundary
-  float* gl = reinterpret_cast<float*>(c2l + S + (S & 1));    // [S]
+  // because 3 * ss int16 may end on an odd 2-byte boundary
+  float* gl = reinterpret_cast<float*>(c2l + ss + (ss & 1));  // [S]
   // by-gate order only: the first-choice gates listed per expert (token order
   // within an expert), every token's place in that list, the experts' first
   // places
@@ -1421,12 +1528,21 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
   const int e = tid % el;
   const int chunk = tid / el;
   const int nchunks = CAP_THREADS / el;
-  const int clen = (S + nchunks - 1) / nchunks;
+  // 16-byte reads of the id arrays: c1 starts 8192 + 20 * el bytes into LDS,
+  // c2 and c2l ss and 2 ss ids later, a chunk clen ids after the previous one
+  const bool vec = (el % 4 == 0) && (ss % 8 == 0);
+  int clen = (S + nchunks - 1) / nchunks;
+  if (vec) clen = (clen + 7) / 8 * 8;
   const int s_begin = min(S, chunk * clen);
   const int s_end = min(S, s_begin + clen);
-  // 16-byte reads of the id arrays: c1 starts 8192 + 20 * el bytes into LDS,
-  // c2 and c2l S and 2 S ids later, a chunk clen ids after the previous one
-  const bool vec = (el % 4 == 0) && (S % 8 == 0) && (clen % 8 == 0);
+  // The prefix over the chunks in two levels of about sqrt(nchunks) each
+  // (nchunks and q are powers of two): one walk over all of them by all 1024
+  // threads was much of the kernel (2 groups of 1024 tokens, 8 experts: 15.6 ->
+  // 10.1 us; 6 groups of 1500, 16 experts, ids now padded for wide reads: 18.3
+  // -> 14.2 us).
+  int q = 1;
+  while (q * q < nchunks) q *= 2;
+  const int super = chunk / q;
 
   int count1 = 0;  // kept first choices of expert e (valid after choice 0)
   for (int choice = 0; choice < 2; ++choice) {
@@ -1434,11 +1550,20 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     cnt[chunk * el + e] = cap_count(ch, s_begin, s_end, e, vec);
     __syncthreads();
     int before = 0, total = 0;
-    for (int k = 0; k < nchunks; ++k) {
-      int v = cnt[k * el + e];
+    for (int k = super * q; k < (super + 1) * q; ++k) {
+      const int v = cnt[k * el + e];
       total += v;
       if (k < chunk) before += v;
     }
+    if (chunk == super * q) pre[super * el + e] = total;
+    __syncthreads();
+    total = 0;
+    for (int k = 0; k < nchunks / q; ++k) {
+      const int v = pre[k * el + e];
+      total += v;
+      if (k < super) before += v;
+    }
+    __syncthreads();
     pre[chunk * el + e] = before + (choice == 0 ? 0 : count1);
     if (chunk == 0 && e < E) tot[choice * el + e] = total;
     if (choice == 0) count1 = min(total, C);
@@ -1565,70 +1690,15 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     gsum[g * GSUM + 1] = s2;
     gsum[g * GSUM + 2] = sw ? n_one_sum : 0.f;
     gsum[g * GSUM + 3] = sw ? zsum : 0.f;
+    // a single group's block needs no launch after it for the loss
+    if (p.G == 1) gate_loss_value<false>(p, gsum, loss);
   }
-}
-
-// The balancing loss from the groups' terms; one thread.  COHERENT: the terms
-// were written by other blocks of the same launch (see st_dev).
-template <bool COHERENT>
-__device__ __forceinline__ void gate_loss_value(const GateParams& p,
-                                                const float* gsum_in,
-                                                float* loss) {
-  struct Terms {
-    const float* q;
-    __device__ float operator[](int i) const {
-      return COHERENT ? ld_dev(q + i) : q[i];
-    }
-  } gsum = {gsum_in};
-  float s1 = 0.f, s2 = 0.f;
-  for (int g = 0; g < p.G; ++g) {
-    s1 += gsum[g * GSUM];
-    s2 += gsum[g * GSUM + 1];
-  }
-  const float inv_ge = (float)(1.0 / ((double)p.G * (double)p.E));
-  const float ee = (float)((double)p.E * (double)p.E);
-  float l;
-  if (p.router == ROUTER_SWITCH) {
-    if (p.has_importance) {
-      // mean over [G,E,S] of proxy[g,e] * (imp[g,s] == 1) * density[g,e]
-      // (moe.py:1229-1234): each group's term counts once per such token
-      float sm = 0.f;
-      for (int g = 0; g < p.G; ++g) sm += gsum[g * GSUM] * gsum[g * GSUM + 2];
-      l = (sm * (float)(1.0 / ((double)p.G * (double)p.E * (double)p.S))) * ee;
-    } else {
-      l = (s1 * inv_ge) * ee;
-    }
-    if (p.num_microbatches > 1)
-      l = l * (float)(1.0 / (double)p.num_microbatches);     // moe.py:1235-1238
-    if (p.use_z_loss) {                                      // moe.py:1253-1266
-      float z = 0.f, n = 0.f;
-      for (int g = 0; g < p.G; ++g) {
-        z += gsum[g * GSUM + 3];
-        n += gsum[g * GSUM + 2];
-      }
-      const float mb = (float)(p.num_microbatches > 0 ? p.num_microbatches : 1);
-      l = l + p.z_loss_coef * (z / (n * mb));
-    }
-    loss[0] = l;
-    return;
-  }
-  l = (s1 * inv_ge) * ee;                                    // moe.py:1423-1424
-  if (p.use_second_place_loss) l = l + ((s2 * inv_ge) * ee) * 0.5f;
-  if (p.num_microbatches > 1)
-    l = l * (float)(1.0 / (double)p.num_microbatches);       // moe.py:1439-1442
-  loss[0] = l;
 }
 
 __global__ void gate_loss_kernel(GateParams p, const float* __restrict__ gsum,
                                  float* __restrict__ loss) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   gate_loss_value<false>(p, gsum, loss);
-}
-
-static int gate_tokens_per_block(int E) {
-  if (E <= 128) return 256;
-  if (E <= 256) return 128;
-  return 64;
 }
 
 }  // namespace mesh_moe
@@ -1675,27 +1745,41 @@ extern "C" int mesh_moe_router_logits(const void* x, const void* w,
       return launch_router_mfma<2>(xb, wp, bias, logits, batch, (int)tokens, M, E, s2);
     return launch_router_mfma<4>(xb, wp, bias, logits, batch, (int)tokens, M, E, s2);
   }
-  const int ept = (E + 3) / 4;
-  dim3 grid((unsigned)((tokens + RL_TOK - 1) / RL_TOK), (unsigned)batch);
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  const int tok = (tokens + 63) / 64 * batch < cus ? 16 : 64;
+  const int groups = 256 / tok;
+  const int ept = (E + groups - 1) / groups;
+  dim3 grid((unsigned)((tokens + tok - 1) / tok), (unsigned)batch);
   int eptp = 1;
   while (eptp < ept) eptp *= 2;
-  size_t smem = sizeof(float) * (RL_TOK * (RL_KC + 1) + (size_t)RL_KC * E + 4 * eptp);
+  size_t smem = sizeof(float) * (tok * (RL_KC + 1) + (size_t)RL_KC * E +
+                                 groups * eptp);
   hipStream_t st = (hipStream_t)stream;
-#define MOE_ROUTER_LOGITS(T, P)                                                \
+#define MOE_ROUTER_LOGITS(T, P, TOK)                                           \
   do {                                                                         \
-    auto kern = router_logits_kernel<T, P>;                                    \
+    auto kern = router_logits_kernel<T, P, TOK>;                               \
     MOE_ALLOW_LDS(kern, smem);                                                 \
     kern<<<grid, 256, smem, st>>>((const T*)x, (const T*)w, bias, logits,      \
                                   tokens, M, E, ept);                          \
   } while (0)
 #define MOE_ROUTER_LOGITS_T(T)                                                 \
-  switch (eptp) {                                                              \
-    case 1: MOE_ROUTER_LOGITS(T, 1); break;                                    \
-    case 2: MOE_ROUTER_LOGITS(T, 2); break;                                    \
-    case 4: MOE_ROUTER_LOGITS(T, 4); break;                                    \
-    case 8: MOE_ROUTER_LOGITS(T, 8); break;                                    \
-    case 16: MOE_ROUTER_LOGITS(T, 16); break;                                  \
-    default: MOE_ROUTER_LOGITS(T, 32); break;                                  \
+  if (tok == 16) {                                                             \
+    switch (eptp) {                                                            \
+      case 1: MOE_ROUTER_LOGITS(T, 1, 16); break;                              \
+      case 2: MOE_ROUTER_LOGITS(T, 2, 16); break;                              \
+      case 4: MOE_ROUTER_LOGITS(T, 4, 16); break;                              \
+      default: MOE_ROUTER_LOGITS(T, 8, 16); break;                             \
+    }                                                                          \
+  } else {                                                                     \
+    switch (eptp) {                                                            \
+      case 1: MOE_ROUTER_LOGITS(T, 1, 64); break;                              \
+      case 2: MOE_ROUTER_LOGITS(T, 2, 64); break;                              \
+      case 4: MOE_ROUTER_LOGITS(T, 4, 64); break;                              \
+      case 8: MOE_ROUTER_LOGITS(T, 8, 64); break;                              \
+      case 16: MOE_ROUTER_LOGITS(T, 16, 64); break;                            \
+      default: MOE_ROUTER_LOGITS(T, 32, 64); break;                            \
+    }                                                                          \
   }
   if (dtype == MESH_MOE_F32) {
     MOE_ROUTER_LOGITS_T(float);
@@ -1716,14 +1800,21 @@ static int launch_capacity_and_loss(const GateParams& p, int32_t* idx,
                                     float* gsum, hipStream_t st) {
   int el = 2;
   while (el < p.E) el *= 2;
-  size_t smem = sizeof(int32_t) * (2 * CAP_THREADS + 3 * (size_t)el) +
-                sizeof(float) * 2 * (size_t)el +
-                sizeof(int16_t) * (3 * (size_t)p.S + 1) +
-                (p.rank_by_gate ? sizeof(float) * (3 * (size_t)p.S + el) : 0);
+  // the id arrays padded to multiples of eight ids, for 16-byte reads, unless
+  // a group as large as LDS takes leaves no room for it
+  auto lds_bytes = [&](size_t ss) {
+    return sizeof(int32_t) * (2 * CAP_THREADS + 3 * (size_t)el) +
+           sizeof(float) * 2 * (size_t)el + sizeof(int16_t) * (3 * ss + 1) +
+           (p.rank_by_gate ? sizeof(float) * (3 * (size_t)p.S + el) : 0);
+  };
+  const int padded = (p.S + 7) / 8 * 8;
+  const int ss = lds_bytes(padded) <= 160 * 1024 ? padded : p.S;
+  const size_t smem = lds_bytes(ss);
   MOE_ALLOW_LDS(gate_capacity_kernel, smem);
   gate_capacity_kernel<<<p.G, CAP_THREADS, smem, st>>>(
-      p, idx, pos, gate, kept, fill, part1, part2, gsum, el);
+      p, idx, pos, gate, kept, fill, part1, part2, gsum, el, ss, loss);
   MOE_CHECK_LAUNCH("gate_capacity");
+  if (p.G == 1) return 0;
   gate_loss_kernel<<<1, 64, 0, st>>>(p, gsum, loss);
   MOE_CHECK_LAUNCH("gate_loss");
   return 0;
@@ -1848,17 +1939,19 @@ static int run_gating(const GateParams& p, const float* logits,
   float* part2 = part1 + (size_t)G * p.nblk * E;
   float* gsum = part2 + (size_t)G * p.nblk * E;
   dim3 grid((unsigned)p.nblk, (unsigned)G);
-  size_t smem = sizeof(float) * ((size_t)p.tt * (E + 1) + p.tt);
+  const size_t smem =
+      sizeof(float) * ((size_t)SELECT_TOKENS * select_row_floats(E) +
+                       SELECT_TOKENS + SELECT_THREADS);
   if (importance && importance_dtype == MESH_MOE_BF16) {
     auto k = gate_select_kernel<bf16_t>;
     MOE_ALLOW_LDS(k, smem);
-    k<<<grid, p.tt, smem, st>>>(logits, (const bf16_t*)importance,
+    k<<<grid, SELECT_THREADS, smem, st>>>(logits, (const bf16_t*)importance,
                                 second_uniform, p, idx, pos, gate, kept, part1,
                                 part2);
   } else {
     auto k = gate_select_kernel<float>;
     MOE_ALLOW_LDS(k, smem);
-    k<<<grid, p.tt, smem, st>>>(logits, (const float*)importance,
+    k<<<grid, SELECT_THREADS, smem, st>>>(logits, (const float*)importance,
                                 second_uniform, p, idx, pos, gate, kept, part1,
                                 part2);
   }
@@ -2026,7 +2119,7 @@ extern "C" int mesh_moe_top2_gating(
   GateParams p = make_gate_params(G, S, E, C, policy, threshold,
                                   use_second_place_loss, num_microbatches,
                                   importance_from_slot_gate,
-                                  gate_tokens_per_block(E));
+                                  SELECT_TOKENS);
   return run_gating(p, logits, importance, importance_dtype, second_uniform,
                     idx, pos, gate, kept, fill, loss, workspace,
                     (hipStream_t)stream);
@@ -2070,7 +2163,7 @@ extern "C" int mesh_moe_switch_gating(
     return rc;
   GateParams p = make_switch_params(G, S, E, C, importance, slots_by_gate,
                                     use_z_loss, z_loss_coef, num_microbatches,
-                                    gate_tokens_per_block(E));
+                                    SELECT_TOKENS);
   return run_gating(p, logits, importance, importance_dtype, choice_logits,
                     idx, pos, gate, kept, fill, loss, workspace,
                     (hipStream_t)stream);

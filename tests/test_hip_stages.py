@@ -40,6 +40,25 @@ def test_gating_random_logits(hip, shape):
   np.testing.assert_allclose(got["loss"], want["loss"], rtol=2e-5)
 
 
+# group sizes around the 64-token blocks and the eight ids of a wide read, expert
+# counts around the 16 lanes of a token and the groups of four of its sums, the
+# most experts and a group whose ids fill most of LDS
+@pytest.mark.parametrize("shape", [
+    (2, 63, 17, 5), (1, 64, 16, 6), (3, 65, 3, 30), (1, 129, 33, 8),
+    (2, 71, 512, 2), (1, 1500, 16, 100), (1, 15999, 6, 3000)])
+@pytest.mark.parametrize("second_place_loss", [False, True])
+def test_gating_edges(hip, shape, second_place_loss):
+  g, s, e, c = shape
+  rng = np.random.default_rng(sum(shape))
+  logits = H.safe_logits(rng, g, s, e, scale=1.5)
+  want = O.top_2_gating(logits, c, use_second_place_loss=second_place_loss)
+  r = hip.top2_gating(torch.from_numpy(logits).cuda(), c,
+                      use_second_place_loss=second_place_loss)
+  got = H.routing_to_np(r)
+  H.assert_routing_equal(got, want)
+  np.testing.assert_allclose(got["loss"], want["loss"], rtol=2e-5)
+
+
 @pytest.mark.parametrize("shape", [(2, 256, 8, 40), (3, 500, 64, 9)])
 def test_gating_exact_ties(hip, shape):
   """Logits on a coarse grid: many exact ties, where the lowest index must win
@@ -100,7 +119,8 @@ def test_gating_second_policy(hip, policy):
 
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(2, 1024, 512, 8), (3, 100, 72, 5),
-                                   (1, 640, 1024, 128)])
+                                   (1, 640, 1024, 128), (1, 15, 4, 17),
+                                   (1, 16401, 40, 5)])
 def test_router_logits(hip, act_dtype, shape):
   g, s, m, e = shape
   rng = np.random.default_rng(17)
