@@ -141,6 +141,46 @@ def _packed_sequence_ids(rng, b, l, mean_len):
   return ids
 
 
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("case", [(64, 64), (129, 64), (515, 64), (513, 128)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_self_attention_sequence_ids_in_any_order(hip, case, causal, with_bias):
+  """Ids that come back later in the row, that are equal modulo 64, negative
+  ones and a single position of its own, in the fused kernels: which tiles of
+  keys or queries are walked must not hang on ids lying in order."""
+  l, d = case
+  b, heads, nb = 3, 1, 8
+  rng = np.random.default_rng(l + d + causal)
+  at = np.arange(l)
+  ids = np.stack([np.where(at // 100 % 2 == 0, 3, 67),
+                  np.where(at < l // 2, -1, np.where(at < l - 40, 63, 5)),
+                  at // 70]).astype(np.int32)
+  ids[0, l // 3] = 9
+  mk = lambda *sizes: O.cast_act(
+      (rng.standard_normal(sizes) * 0.5).astype(np.float32), "bfloat16")
+  q, k, v, do = (mk(b, l, heads * d) for _ in range(4))
+  g = lambda a: H.to_gpu(a, "bfloat16")
+  values, rel = None, None
+  if with_bias:
+    values = mk(heads, nb)
+    bucket = B.relative_position_bucket(np.arange(-(l - 1), l), not causal, nb)
+    rel = (g(values), torch.from_numpy(bucket.astype(np.int32)).cuda())
+  sid = torch.from_numpy(ids).cuda()
+  got = H.to_np(hip.self_attention(g(q), g(k), g(v), heads, causal,
+                                   sequence_id=sid, relative_bias=rel))
+  want = B._attention_core(q, k, v, heads, causal, "bfloat16", sequence_id=ids,
+                           relative_values=values)
+  np.testing.assert_allclose(got, want, **_tol("bfloat16"))
+  grads = hip.self_attention_backward(g(q), g(k), g(v), g(do), heads, causal,
+                                      sequence_id=sid, relative_bias=rel)
+  want = B.attention_core_backward(q, k, v, do, heads, causal, "bfloat16",
+                                   sequence_id=ids, relative_values=values)
+  for gt, wnt in zip(grads, want):
+    scale = max(1.0, float(np.abs(wnt).max()))
+    np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("case", [(2, 40, 2, 16, 5), (2, 200, 2, 64, 37),
