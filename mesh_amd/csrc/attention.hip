@@ -104,19 +104,33 @@ __device__ __forceinline__ float fa_exp2(float x) {
 // Which (tile, batch * head) a block works on.  Workgroups go to the 8 XCDs
 // round-robin in launch order (x fastest), so with the plain mapping the tiles
 // of one (batch, head) land on all of them and every XCD's L2 fetches that
-// head's K and V for itself.  Here XCD x takes the heads x, x + 8, ... and runs
-// all tiles of a head back to back: a head's K and V enter one L2 once.
+// head's K and V for itself.  Here XCD x takes the heads x, x + 8, ..., whose K
+// and V then enter one L2 once.
+// Without a causal mask a head's tiles run back to back.  With one the tiles are
+// of very different length (the caller numbers the long ones first), and head
+// after head the last head's long tiles start when everything else is nearly
+// done: 8 heads of 16 tiles on the 64 places of an XCD then take 59 units of
+// time instead of 34.  So heads are taken in groups large enough for two tiles
+// per place, the longest tiles of all of a group's heads first; larger groups
+// would only spread an L2 over more heads.
+// 8 x 2048 positions, 8 heads of 128, causal, forward: 155 -> 127 us with the
+// loads' addresses worked out once; 16 packed rows of 1000, 12 heads of 64:
+// forward 72 -> 55, dv, dk, dq 88, 125, 173 -> 62, 95, 125 us.
+template <bool CAUSAL>
 __device__ __forceinline__ void fa_block_to_work(int n_tiles, int& tile, int& bh) {
   const int nbh = (int)gridDim.y;
-  if (nbh % 8 == 0) {
-    const int id = (int)blockIdx.x + n_tiles * (int)blockIdx.y;
-    const int slot = id >> 3;
-    bh = (slot / n_tiles) * 8 + (id & 7);
-    tile = slot % n_tiles;
-  } else {
-    tile = (int)blockIdx.x;
-    bh = (int)blockIdx.y;
+  const int lanes = nbh % 8 == 0 ? 8 : 1;
+  const int id = (int)blockIdx.x + n_tiles * (int)blockIdx.y;
+  const int slot = id / lanes, heads = nbh / lanes;
+  int size = 1;                                    // heads of a group
+  if (CAUSAL) {
+    const int groups = max(1, (int)((int64_t)heads * n_tiles / (1024 / lanes)));
+    size = (heads + groups - 1) / groups;
   }
+  const int group = slot / (size * n_tiles), at = slot - group * size * n_tiles;
+  const int here = min(size, heads - group * size);
+  tile = at / here;
+  bh = (group * size + at - tile * here) * lanes + id % lanes;
 }
 
 // Shrinks the streamed tiles [t_begin, t_end) of BT rows to those between the
@@ -129,7 +143,8 @@ __device__ __forceinline__ void fa_block_to_work(int n_tiles, int& tile, int& bh
 // loops over consecutive tiles.  Every wavefront calls it; scratch: the start
 // of the tile ring, free again afterwards.  A row's own id is always found.
 // 16 rows of 1000 positions, two sequences and padding in each, 12 heads of 64:
-// forward 98 -> 72 us; dv, dk, dq 99, 152, 211 -> 88, 125, 173 us.
+// forward 98 -> 72 us; dv, dk, dq 99, 152, 211 -> 88, 125, 173 us (with the
+// blocks still head after head, see above).
 template <int WAVES>
 __device__ __forceinline__ void fa_visible_tiles(
     const int32_t* __restrict__ seq_b, int L, int BT, int my_sid, bool uniform,
@@ -201,7 +216,7 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
   const int half = lane >> 5, l32 = lane & 31;
   const int nq = (L + Cfg::BQ - 1) / Cfg::BQ;
   int tile_x, bh;
-  fa_block_to_work(nq, tile_x, bh);
+  fa_block_to_work<CAUSAL>(nq, tile_x, bh);
   const int qt = nq - 1 - tile_x;            // long (late) query tiles first
   const int b = bh / H, h = bh % H;
   const int q0 = qt * Cfg::BQ;
@@ -242,31 +257,36 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
       qf[s] = *reinterpret_cast<const fa_bf16x8_t*>(qr + s * 16);
   }
 
-  // direct-to-LDS loads of one K tile and one V tile
+  // direct-to-LDS loads of one K tile and one V tile: a lane's places in a tile
+  // (row and swizzled chunk) are offsets that never change, the tile's is a
+  // scalar; rows past the end repeat the last
+  static_assert(Cfg::K_RPI == Cfg::V_RPI && Cfg::KCH == Cfg::VCH, "one row shape");
+  const uint32_t rs = (uint32_t)row_stride;
+  uint32_t k_chunk[Cfg::K_INSTR], v_chunk[Cfg::K_INSTR], row_off[Cfg::K_INSTR];
+#pragma unroll
+  for (int j = 0; j < Cfg::K_INSTR; ++j) {
+    const int row = (wave * Cfg::K_INSTR + j) * Cfg::K_RPI + lane / Cfg::KCH;
+    const int p = lane % Cfg::KCH;
+    k_chunk[j] = (uint32_t)(p ^ fa_kswz<Cfg::KCH>(row)) * 8;
+    v_chunk[j] =
+        (uint32_t)((((p >> 2) ^ fa_vswz<Cfg::V_UNITS>(row)) << 2) | (p & 3)) * 8;
+    row_off[j] = (uint32_t)row * rs;
+  }
   auto load_tile = [&](int kt, int buf) {
     const int key0 = kt * Cfg::BK;
     unsigned char* base = fa_smem + buf * Cfg::STAGE;
+    const bf16_t* kt0 = kb + (int64_t)key0 * row_stride;
+    const bf16_t* vt0 = vb + (int64_t)key0 * row_stride;
+    const uint32_t last_row = (uint32_t)(L - 1 - key0) * rs;
 #pragma unroll
     for (int j = 0; j < Cfg::K_INSTR; ++j) {
+      const uint32_t row = min(row_off[j], last_row);
       const int g = wave * Cfg::K_INSTR + j;
-      const int row = g * Cfg::K_RPI + lane / Cfg::KCH;
-      const int c = (lane % Cfg::KCH) ^ fa_kswz<Cfg::KCH>(row);
-      const bf16_t* src =
-          kb + (int64_t)min(key0 + row, L - 1) * row_stride + c * 8;
-      __builtin_amdgcn_global_load_lds((fa_glb_void_t*)src,
+      __builtin_amdgcn_global_load_lds((fa_glb_void_t*)(kt0 + (row + k_chunk[j])),
                                        (fa_lds_void_t*)(base + g * 1024), 16, 0,
                                        0);
-    }
-#pragma unroll
-    for (int j = 0; j < Cfg::V_INSTR; ++j) {
-      const int g = wave * Cfg::V_INSTR + j;
-      const int row = g * Cfg::V_RPI + lane / Cfg::VCH;     // key
-      const int p = lane % Cfg::VCH;
-      const int c = (((p >> 2) ^ fa_vswz<Cfg::V_UNITS>(row)) << 2) | (p & 3);
-      const bf16_t* src =
-          vb + (int64_t)min(key0 + row, L - 1) * row_stride + c * 8;
       __builtin_amdgcn_global_load_lds(
-          (fa_glb_void_t*)src,
+          (fa_glb_void_t*)(vt0 + (row + v_chunk[j])),
           (fa_lds_void_t*)(base + Cfg::K_BYTES + g * 1024), 16, 0, 0);
     }
     if constexpr (SEQ) {
@@ -685,7 +705,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
   const int n_own = (L + Cfg::BOWN - 1) / Cfg::BOWN;
   // long tiles first: late queries, early keys
   int tile_x, bh;
-  fa_block_to_work(n_own, tile_x, bh);
+  fa_block_to_work<CAUSAL>(n_own, tile_x, bh);
   const int ot = OWN_Q && CAUSAL ? n_own - 1 - tile_x : tile_x;
   const int own0 = ot * Cfg::BOWN;
   const int b = bh / H, h = bh % H;
@@ -737,20 +757,30 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
   }
 
   // one tile copy: rows of `src` from row0, chunk-swizzled for row reads
-  // (TR = false) or unit-swizzled for transposing reads (TR = true)
+  // (TR = false) or unit-swizzled for transposing reads (TR = true); a lane's
+  // places in a tile are offsets that never change
+  const uint32_t rs = (uint32_t)row_stride;
+  uint32_t row_off[Cfg::INSTR], chunk_off[2][Cfg::INSTR];
+#pragma unroll
+  for (int j = 0; j < Cfg::INSTR; ++j) {
+    const int row = (wave * Cfg::INSTR + j) * Cfg::RPI + lane / Cfg::CH;
+    const int p = lane % Cfg::CH;
+    chunk_off[0][j] = (uint32_t)(p ^ fa_kswz<Cfg::CH>(row)) * 8;
+    chunk_off[1][j] =
+        (uint32_t)((((p >> 2) ^ fa_vswz<Cfg::UNITS>(row)) << 2) | (p & 3)) * 8;
+    row_off[j] = (uint32_t)row * rs;
+  }
   auto load_copy = [&](const bf16_t* src, int row0, unsigned char* dst,
                        auto tr_c) {
     constexpr bool TR = decltype(tr_c)::value;
+    const bf16_t* first = src + (int64_t)row0 * row_stride;
+    const uint32_t last_row = (uint32_t)(L - 1 - row0) * rs;
 #pragma unroll
     for (int j = 0; j < Cfg::INSTR; ++j) {
-      const int g = wave * Cfg::INSTR + j;
-      const int row = g * Cfg::RPI + lane / Cfg::CH;
-      const int p = lane % Cfg::CH;
-      const int c = TR ? ((((p >> 2) ^ fa_vswz<Cfg::UNITS>(row)) << 2) | (p & 3))
-                       : (p ^ fa_kswz<Cfg::CH>(row));
-      const bf16_t* a = src + (int64_t)min(row0 + row, L - 1) * row_stride + c * 8;
-      __builtin_amdgcn_global_load_lds((fa_glb_void_t*)a,
-                                       (fa_lds_void_t*)(dst + g * 1024), 16, 0, 0);
+      const uint32_t row = min(row_off[j], last_row);
+      __builtin_amdgcn_global_load_lds(
+          (fa_glb_void_t*)(first + (row + chunk_off[TR ? 1 : 0][j])),
+          (fa_lds_void_t*)(dst + (wave * Cfg::INSTR + j) * 1024), 16, 0, 0);
     }
   };
   auto load_tile = [&](int t, int buf) {
