@@ -1403,6 +1403,7 @@ def dense(x, w_packed, activation=None):
   lib = load_library()
   if activation not in ACTIVATIONS:
     raise ValueError("unsupported expert activation %r" % (activation,))
+  x = x.contiguous()
   sizes = x.shape
   k = sizes[-1]
   n = w_packed.shape[1]

@@ -66,6 +66,22 @@ def test_dense(hip, shape, act_dtype):
                                **_tol(act_dtype))
 
 
+def test_dense_takes_any_strides(hip):
+  """Rows that do not lie one behind the other, broadcast ones among them, give
+  what their copies give."""
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(3)
+  mk = lambda *sizes: torch.randn(sizes, generator=gen, device="cuda").to(
+      torch.bfloat16)
+  w = mk(1, 40, 64)
+  for x in (mk(5, 3, 64).transpose(0, 1), mk(64, 7).t(), mk(4, 6, 128)[..., 1::2],
+            mk(1, 64).expand(9, 64)):
+    assert not x.is_contiguous()
+    got = hip.dense(x, w, "relu")
+    assert got.shape == x.shape[:-1] + (40,)
+    assert torch.equal(got, hip.dense(x.contiguous(), w, "relu"))
+
+
 ATT_CASES = [
     # B, L, heads, d_kv, d_model; bf16 with d_kv 64 / 128 runs the fused kernel
     (2, 12, 3, 4, 16), (1, 128, 4, 32, 64), (2, 200, 2, 64, 48),
