@@ -2402,12 +2402,19 @@ namespace mesh_moe {
 // ---------------------------------------------------------------------------
 // Dispatch folded into the first expert GEMM: slot -> token map.
 // ---------------------------------------------------------------------------
+// threads first, first + stride, ... of those that clear the map
+__device__ __forceinline__ void clear_slot_map(int32_t* map, int64_t n,
+                                               bf16_t* zero_row, int m,
+                                               int64_t first, int64_t stride) {
+  for (int64_t i = first; i < n; i += stride) map[i] = -1;
+  for (int64_t i = first; i < m; i += stride) zero_row[i] = 0;
+}
+
 __global__ void slot_map_clear_kernel(int32_t* map, int64_t n, bf16_t* zero_row,
                                       int m) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (int64_t i = i0; i < n; i += stride) map[i] = -1;
-  for (int64_t i = i0; i < m; i += stride) zero_row[i] = 0;
+  clear_slot_map(map, n, zero_row, m,
+                 (int64_t)blockIdx.x * blockDim.x + threadIdx.x,
+                 (int64_t)gridDim.x * blockDim.x);
 }
 
 // one thread per (token, choice): a kept choice whose activation-dtype gate is
@@ -2452,46 +2459,119 @@ __global__ __launch_bounds__(256) void slot_map_rows_kernel(
 // ---------------------------------------------------------------------------
 // Compacted rows: expert e's occupied slots, groups in order, slots in order,
 // become rows 0 .. rows_used[e] - 1 of its row range.
-// row_offsets[e][g] = sum over g' < g of fill[g'][e]; one block per expert.
+//
+// Two launches prepare a call's GEMMs: compact_rows_kernel (the row offsets, and
+// the map cleared) and compact_map_kernel (the map from the offsets, and both
+// GEMMs' tile lists); the backward takes one (compact_lists_kernel).  Each is
+// bound by being a launch, about 5 us.  As a launch per task they were five and
+// three: 32768 tokens, 64 experts, 572 -> 566 us a pass, and 2253 -> 2233 in
+// training with one choice per token.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void row_offsets_kernel(
+// The sum of v over the threads before this one; `total` over all.  (Callers
+// synchronise before they use wave_sums, NT / 64 values, again.)
+template <int NT>
+__device__ __forceinline__ int block_prefix(int v, int* wave_sums, int& total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int sum = v;
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const int before = __shfl_up(sum, d);
+    if (lane >= d) sum += before;
+  }
+  if (lane == 63) wave_sums[wave] = sum;
+  __syncthreads();
+  int first = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    const int s = wave_sums[w];
+    if (w < wave) first += s;
+    total += s;
+  }
+  return first + sum - v;
+}
+
+// Blocks 0 .. E - 1: row_offsets[e][g] = sum over g' < g of fill[g'][e].  The
+// blocks behind them clear the map.
+__global__ __launch_bounds__(256) void compact_rows_kernel(
     const int32_t* __restrict__ fill, int32_t* __restrict__ row_offsets,
-    int32_t* __restrict__ rows_used, int G, int E) {
-  __shared__ int32_t part[256];
+    int32_t* __restrict__ rows_used, int G, int E, int32_t* __restrict__ map,
+    int64_t n_map, bf16_t* __restrict__ zero_row, int m) {
+  __shared__ int wave_sums[4];
   const int e = blockIdx.x, tid = threadIdx.x;
+  if (e >= E) {
+    clear_slot_map(map, n_map, zero_row, m, (int64_t)(e - E) * 256 + tid,
+                   (int64_t)((int)gridDim.x - E) * 256);
+    return;
+  }
   const int per = (G + 255) / 256;
   const int g0 = min(G, tid * per), g1 = min(G, g0 + per);
   int sum = 0;
   for (int g = g0; g < g1; ++g) sum += fill[(int64_t)g * E + e];
-  part[tid] = sum;
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int i = 0; i < 256; ++i) {
-      const int v = part[i];
-      part[i] = run;
-      run += v;
-    }
-    rows_used[e] = run;
-  }
-  __syncthreads();
-  int run = part[tid];
+  int total;
+  int run = block_prefix<256>(sum, wave_sums, total);
+  if (tid == 0) rows_used[e] = total;
   for (int g = g0; g < g1; ++g) {
     row_offsets[(int64_t)e * G + g] = run;
     run += fill[(int64_t)g * E + e];
   }
 }
 
-// One thread per (token, choice), as slot_map_kernel, onto the compacted rows.
-__global__ void slot_map_compact_kernel(const int32_t* __restrict__ idx,
-                                        const int32_t* __restrict__ pos,
-                                        const float* __restrict__ gate,
-                                        const uint8_t* __restrict__ kept,
-                                        const int32_t* __restrict__ row_offsets,
-                                        int32_t* __restrict__ map,
-                                        int64_t tokens, int S, int G,
-                                        int64_t rows_per_expert) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// The tiles that hold occupied rows, in the order of the full tile numbering
+// ((expert, N tile, M tile), M tile fastest), of up to two GEMMs over the same
+// rows: list[-1] = their number.  E <= 1024 (a thread per expert).
+constexpr int LIST_THREADS = 1024;
+struct TileLists {
+  int32_t* list[2];
+  int tiles_n[2];
+  int E, tiles_m, bm;
+  int parts;             // blocks per list
+};
+// a block per 8 tiles a thread, no more than a list needs and at most 16
+static int tile_list_parts(int E, int tiles_m, int tn1, int tn2) {
+  const int64_t tiles = (int64_t)E * tiles_m * (tn1 > tn2 ? tn1 : tn2);
+  const int64_t parts = (tiles + 8 * LIST_THREADS - 1) / (8 * LIST_THREADS);
+  return (int)(parts < 16 ? parts : 16);
+}
+// block `block` of 2 L.parts; used: the occupied rows of expert threadIdx.x
+__device__ __forceinline__ void write_tile_list(const TileLists& L, int used,
+                                                int block) {
+  __shared__ int32_t mt[LIST_THREADS], pre[LIST_THREADS];
+  __shared__ int wave_sums[LIST_THREADS / 64];
+  const int tid = threadIdx.x, part = block >> 1;
+  const bool second = (block & 1) != 0;
+  int32_t* list = second ? L.list[1] : L.list[0];
+  const int tiles_n = second ? L.tiles_n[1] : L.tiles_n[0];
+  const int own = tid < L.E ? min(L.tiles_m, (used + L.bm - 1) / L.bm) : 0;
+  int total_m;
+  pre[tid] = block_prefix<LIST_THREADS>(own, wave_sums, total_m);
+  mt[tid] = own;
+  if (part == 0 && tid == 0) list[-1] = total_m * tiles_n;
+  __syncthreads();
+  const int64_t total = (int64_t)L.E * tiles_n * L.tiles_m;
+  for (int64_t at = (int64_t)part * LIST_THREADS + tid; at < total;
+       at += (int64_t)L.parts * LIST_THREADS) {
+    const int i = (int)at;
+    const int tm = i % L.tiles_m, rest = i / L.tiles_m;
+    const int tn = rest % tiles_n, e = rest / tiles_n;
+    if (tm < mt[e]) list[tiles_n * pre[e] + tn * mt[e] + tm] = i;
+  }
+}
+
+// Blocks 0 .. 2 parts - 1: the tile lists.  Behind them one thread per (token,
+// choice), as slot_map_kernel, onto the compacted rows.
+__global__ __launch_bounds__(LIST_THREADS) void compact_map_kernel(
+    const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
+    const float* __restrict__ gate, const uint8_t* __restrict__ kept,
+    const int32_t* __restrict__ row_offsets,
+    const int32_t* __restrict__ rows_used, int32_t* __restrict__ map,
+    int64_t tokens, int S, int G, int64_t rows_per_expert, TileLists lists) {
+  const int list_blocks = 2 * lists.parts, tid = threadIdx.x;
+  if ((int)blockIdx.x < list_blocks) {
+    write_tile_list(lists, tid < lists.E ? rows_used[tid] : 0, blockIdx.x);
+    return;
+  }
+  const int64_t i = (int64_t)(blockIdx.x - list_blocks) * LIST_THREADS + tid;
   if (i >= tokens * 2) return;
   if (!kept[i] || round_to<bf16_t>(gate[i]) == 0.0f) return;
   const int64_t t = i >> 1;
@@ -2501,39 +2581,18 @@ __global__ void slot_map_compact_kernel(const int32_t* __restrict__ idx,
       (int32_t)t;
 }
 
-// The tiles that hold occupied rows, in the order of the full tile numbering
-// ((expert, N tile, M tile), M tile fastest): list[-1] = their number.  One
-// block; E <= 1024.
-__global__ __launch_bounds__(1024) void tile_list_kernel(
-    const int32_t* __restrict__ rows_used, int32_t* __restrict__ list, int E,
-    int tiles_m, int tiles_n, int bm) {
-  __shared__ int32_t mt[1024], pre[1025];
-  const int tid = threadIdx.x;
-  if (tid < E) mt[tid] = min(tiles_m, (rows_used[tid] + bm - 1) / bm);
-  __syncthreads();
-  if (tid == 0) {
-    int run = 0;
-    for (int e = 0; e < E; ++e) { pre[e] = run; run += mt[e]; }
-    pre[E] = run;
-    list[-1] = run * tiles_n;
-  }
-  __syncthreads();
-  const int total = E * tiles_n * tiles_m;
-  for (int i = tid; i < total; i += blockDim.x) {
-    const int tm = i % tiles_m, rest = i / tiles_m;
-    const int tn = rest % tiles_n, e = rest / tiles_n;
-    if (tm < mt[e]) list[tiles_n * pre[e] + tn * mt[e] + tm] = i;
-  }
-}
-
-// rows_used[e] from the row offsets of the last group and its fill count
-__global__ void rows_used_kernel(const int32_t* __restrict__ fill,
-                                 const int32_t* __restrict__ row_offsets,
-                                 int32_t* __restrict__ rows_used, int G, int E) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < E)
-    rows_used[e] = row_offsets[(int64_t)e * G + G - 1] +
-                   fill[(int64_t)(G - 1) * E + e];
+// The backward's tile lists, and rows_used[e] from the row offsets of the last
+// group and its fill count.
+__global__ __launch_bounds__(LIST_THREADS) void compact_lists_kernel(
+    const int32_t* __restrict__ fill, const int32_t* __restrict__ row_offsets,
+    int32_t* __restrict__ rows_used, int G, TileLists lists) {
+  const int e = threadIdx.x;
+  int used = 0;
+  if (e < lists.E)
+    used = row_offsets[(int64_t)e * G + G - 1] +
+           fill[(int64_t)(G - 1) * lists.E + e];
+  if (blockIdx.x == 0 && e < lists.E) rows_used[e] = used;
+  write_tile_list(lists, used, blockIdx.x);
 }
 
 }  // namespace mesh_moe
@@ -2683,23 +2742,21 @@ extern "C" int mesh_moe_compact_expert_ffn(
   int32_t* list1 = (int32_t*)up((uintptr_t)(rows_used + E)) + 64;
   int32_t* list2 = (int32_t*)up((uintptr_t)(list1 + (size_t)E * tiles_m * tn1)) + 64;
   bf16_t* zero_row = (bf16_t*)up((uintptr_t)(list2 + (size_t)E * tiles_m * tn2));
-  row_offsets_kernel<<<E, 256, 0, st>>>(fill, row_offsets, rows_used, G, E);
-  MOE_CHECK_LAUNCH("compact_expert_ffn (row offsets)");
   const int64_t n_map = (int64_t)E * R;
   const unsigned cb = (unsigned)((n_map + 255) / 256 < 4096 ? (n_map + 255) / 256
                                                             : 4096);
-  slot_map_clear_kernel<<<cb, 256, 0, st>>>(map, n_map, zero_row, M);
-  MOE_CHECK_LAUNCH("compact_expert_ffn (clear)");
+  compact_rows_kernel<<<(unsigned)E + cb, 256, 0, st>>>(
+      fill, row_offsets, rows_used, G, E, map, n_map, zero_row, M);
+  MOE_CHECK_LAUNCH("compact_expert_ffn (row offsets)");
+  const TileLists lists = {{list1, list2}, {tn1, tn2}, E, tiles_m, RingCfg::BM,
+                           tile_list_parts(E, tiles_m, tn1, tn2)};
   const int64_t pairs = (int64_t)G * S * 2;
-  slot_map_compact_kernel<<<(unsigned)((pairs + 255) / 256), 256, 0, st>>>(
-      idx, pos, gate, kept, row_offsets, map, (int64_t)G * S, S, G, rows);
-  MOE_CHECK_LAUNCH("compact_expert_ffn (slot map)");
-  tile_list_kernel<<<1, 1024, 0, st>>>(rows_used, list1, E, tiles_m, tn1,
-                                       RingCfg::BM);
-  MOE_CHECK_LAUNCH("compact_expert_ffn (tile list 1)");
-  tile_list_kernel<<<1, 1024, 0, st>>>(rows_used, list2, E, tiles_m, tn2,
-                                       RingCfg::BM);
-  MOE_CHECK_LAUNCH("compact_expert_ffn (tile list 2)");
+  compact_map_kernel<<<(unsigned)(2 * lists.parts +
+                                  (pairs + LIST_THREADS - 1) / LIST_THREADS),
+                       LIST_THREADS, 0, st>>>(
+      idx, pos, gate, kept, row_offsets, rows_used, map, (int64_t)G * S, S, G,
+      rows, lists);
+  MOE_CHECK_LAUNCH("compact_expert_ffn (slot map, tile lists)");
   const bool relu = activation == MESH_MOE_ACT_RELU;
   int rc = launch_ring((const bf16_t*)x, (const bf16_t*)wi_packed, (bf16_t*)h,
                        E, R, H, M, relu, st, map, zero_row, nullptr, list1);
@@ -3088,15 +3145,12 @@ extern "C" int mesh_moe_compact_expert_ffn_backward(
   int32_t* list_h = (int32_t*)up((uintptr_t)(rows_used + E)) + 64;
   int32_t* list_m =
       (int32_t*)up((uintptr_t)(list_h + (size_t)E * tiles_m * tn_h)) + 64;
-  rows_used_kernel<<<(E + 255) / 256, 256, 0, st>>>(fill, row_offsets,
-                                                    rows_used, G, E);
-  MOE_CHECK_LAUNCH("compact_expert_ffn_backward (rows used)");
-  tile_list_kernel<<<1, 1024, 0, st>>>(rows_used, list_h, E, tiles_m, tn_h,
-                                       RingCfg::BM);
-  MOE_CHECK_LAUNCH("compact_expert_ffn_backward (tile list 1)");
-  tile_list_kernel<<<1, 1024, 0, st>>>(rows_used, list_m, E, tiles_m, tn_m,
-                                       RingCfg::BM);
-  MOE_CHECK_LAUNCH("compact_expert_ffn_backward (tile list 2)");
+  const TileLists lists = {{list_h, list_m}, {tn_h, tn_m}, E, tiles_m,
+                           RingCfg::BM,
+                           tile_list_parts(E, tiles_m, tn_h, tn_m)};
+  compact_lists_kernel<<<2 * lists.parts, LIST_THREADS, 0, st>>>(
+      fill, row_offsets, rows_used, G, lists);
+  MOE_CHECK_LAUNCH("compact_expert_ffn_backward (tile lists)");
   // dh = dy . wo^T on the listed row tiles, the ReLU mask on its stores (the
   // rows of a listed tile past the expert's occupied ones have h = 0 and
   // dy = 0)

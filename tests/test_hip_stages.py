@@ -1240,6 +1240,33 @@ def test_compact_expert_ffn_equals_two_calls(hip, case):
       assert torch.equal(y[ei, o:o + k], y_all[ei, gi * c:gi * c + k])
 
 
+@pytest.mark.parametrize("case", [
+    (1, 300, 2, 256, 64, 256, 256), (300, 16, 8, 2, 64, 256, 264),
+    (257, 16, 65, 2, 64, 320, 256), (2, 1024, 512, 128, 64, 4352, 256)],
+    ids=lambda c: "x".join(map(str, c)))
+def test_compact_rows_map_and_lists(hip, case):
+  """The compacted rows' offsets, map and tile lists at their edges: one group
+  and two experts, more groups than a block has threads, more experts than a
+  wavefront, more tiles than one block lists, experts without a token."""
+  g, s, e, c, m, h, n = case
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(case))
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  logits = mk(g, s, e)
+  logits[..., e // 2] -= 100.0
+  r = hip.switch_gating(logits, c)
+  x = mk(g, s, m).to(torch.bfloat16)
+  wi = mk(e, h, m).to(torch.bfloat16) / m ** 0.5
+  wo = mk(e, n, h).to(torch.bfloat16) / h ** 0.5
+  y, row_offsets = hip.compact_expert_ffn(x, r, wi, wo, "relu")
+  fill = r.fill.long()
+  assert torch.equal(row_offsets, (fill.t().cumsum(1) - fill.t()).to(torch.int32))
+  want = hip.expert_ffn(hip.dispatch(x, r).reshape(e, g * c, m), wi, wo, "relu")
+  assert torch.equal(
+      hip.combine(y.reshape(e, g, c, n), r, s, row_offsets=row_offsets),
+      hip.combine(want.reshape(e, g, c, n), r, s))
+
+
 def test_dispatched_expert_ffn_equals_two_calls_cfg4(hip):
   """The same identity at the full size of benchmark configuration 4 (32 groups
   of 2048 tokens, 64 experts, capacity 64, d_model 4096, hidden 16384), where
