@@ -526,7 +526,11 @@ __global__ __launch_bounds__(256) void stream_gemm_bf16_kernel(
   const int fr = lane & 31, fc = lane >> 5;
   int slot = 0, free_slot = NS - 1;
   for (int kt = 0; kt < nk; ++kt) {
+    // the oldest tile has landed, and this wavefront's reads of the slot that
+    // is about to be loaded again have returned: the multiplications that use
+    // them need not be issued yet
     wait_vmcnt<(NS - 2) * Cfg::LOADS>();
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");

@@ -1467,11 +1467,13 @@ def test_linear_of_few_rows_and_columns(hip, shape, activation):
 
 @pytest.mark.parametrize("shape", [
     (130, 1, 64, 72), (64, 32, 192, 256), (43, 33, 320, 400), (128, 64, 1024, 128),
-    (16, 5, 128, 1032)], ids=lambda s: "x".join(map(str, s)))
+    (16, 5, 128, 1032), (160, 20, 4096, 256), (160, 64, 4160, 256)],
+    ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("activation", ["linear", "relu"])
 def test_linear_of_few_rows_many_experts(hip, shape, activation):
   """At most 64 rows for each of many column tiles: reductions shorter than the
-  ring of K tiles, columns that end inside a 128-column tile."""
+  ring of K tiles, and ones that go round it many times while two blocks share a
+  compute unit; columns that end inside a 128-column tile."""
   _check_linear(hip, shape, activation)
 
 
