@@ -326,6 +326,28 @@ __global__ __launch_bounds__(256) void dispatch_backward_router4_kernel(
   }
 }
 
+// Eight float32 as three bfloat16 terms each, term[0] + term[1] + term[2] == d
+// exactly: the leading 8 significant bits, the next 8 and the last 8.  (Terms are
+// cut off, not rounded, so that none is larger than d.  Only bits below the
+// smallest bfloat16, 2^-133, can be lost.)
+__device__ __forceinline__ void split_bf16x3(const float (&d)[8],
+                                             uint4 (&term)[3]) {
+  uint32_t t[3][8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float rest = d[j];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      t[i][j] = __float_as_uint(rest) & 0xffff0000u;
+      if (i < 2) rest -= __uint_as_float(t[i][j]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    term[i] = make_uint4(t[i][1] | t[i][0] >> 16, t[i][3] | t[i][2] >> 16,
+                         t[i][5] | t[i][4] >> 16, t[i][7] | t[i][6] >> 16);
+}
+
 // The same for bfloat16 with the router's share on the matrix cores
 // (v_mfma_f32_32x32x16_bf16).  The share of 32 tokens x 256 columns,
 // sum_e dlogits[t][e] * w_gate[m][e], is a product whose two operands both lie
@@ -334,9 +356,10 @@ __global__ __launch_bounds__(256) void dispatch_backward_router4_kernel(
 // d(logits) rows to LDS with whole-line loads (lanes reading their 8
 // consecutive e straight from global memory touch 32 lines per instruction and
 // ask for every line four times: 0.59 against 0.49 ms for 65536 tokens of 4096)
-// and the lanes take their operands from there.  The float32 d(logits) go in as two bfloat16 terms
-// (hi = bf16(d), lo = bf16(d - hi): the products are exact in the float32
-// accumulator, what is dropped is below 2^-17 |d|).  The instruction leaves a
+// and the lanes take their operands from there.  The float32 d(logits) go in as
+// three bfloat16 terms that add up to them exactly (split_bf16x3): every product
+// is exact in the float32 accumulator, as those of the one-token and four-token
+// kernels are.  The instruction leaves a
 // lane with 4 consecutive columns of one token; the tile goes through LDS as
 // float32 (over the kernel rows, which are no longer needed) so that the
 // second phase -- half a wavefront per token row, 16 bytes per lane, the rows
@@ -536,17 +559,15 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
       const float4 d0 = *reinterpret_cast<const float4*>(dl + l32 * DROW + ks * 64 + half * 32);
       const float4 d1 = *reinterpret_cast<const float4*>(dl + l32 * DROW + ks * 64 + half * 32 + 16);
       const float d[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
-      float lo[8];
+      uint4 term[3];
+      split_bf16x3(d, term);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) lo[j] = d[j] - round_to<bf16_t>(d[j]);
-      const dbm_bf16x8_t bh = __builtin_bit_cast(dbm_bf16x8_t, pack16(d, bf16_t()));
-      const dbm_bf16x8_t bl = __builtin_bit_cast(dbm_bf16x8_t, pack16(lo, bf16_t()));
+      for (int i = 0; i < 3; ++i)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const dbm_bf16x8_t a = __builtin_bit_cast(dbm_bf16x8_t, afrag[b][ks]);
-        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bh, acc[b], 0, 0, 0);
-        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bl, acc[b], 0, 0, 0);
-      }
+        for (int b = 0; b < 2; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(dbm_bf16x8_t, afrag[b][ks]),
+              __builtin_bit_cast(dbm_bf16x8_t, term[i]), acc[b], 0, 0, 0);
     }
     // (the share goes over the kernel rows: every wavefront has its operands
     // in registers before the first write)
@@ -1088,10 +1109,9 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
 // ---------------------------------------------------------------------------
 // The same product for bfloat16 tokens on the bfloat16 matrix cores
 // (v_mfma_f32_32x32x16_bf16, 16 tokens per instruction instead of 2).  The
-// float32 d(logits) go in as two bfloat16 terms, hi = bf16(d) and
-// lo = bf16(d - hi): x * hi and x * lo are exact in the float32 accumulator and
-// what is left of d, at most 2^-17 |d|, is below the rounding of the sum
-// itself.  Both operands lie in memory with the reduction index (the token)
+// float32 d(logits) go in as three bfloat16 terms that add up to them exactly
+// (split_bf16x3), so that every product is exact in the float32 accumulator.
+// Both operands lie in memory with the reduction index (the token)
 // outermost; they are staged in LDS as they lie and the instruction's
 // operands (8 consecutive tokens of one kernel row / one expert per lane) are
 // read with ds_read_b64_tr_b16: within 16 lanes, lane t addresses the 8 bytes
@@ -1103,7 +1123,8 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
 // ---------------------------------------------------------------------------
 constexpr int WB_M = WM_M, WB_KT = WM_KT;
 constexpr int WB_XS = (WB_M + 32) * 2;   // bytes per staged token row of x
-constexpr int WB_DS = (64 + 16) * 2;     // ... of one half of d(logits)
+constexpr int WB_DS = (64 + 16) * 2;     // ... of one term of d(logits)
+constexpr int WB_DT = WB_KT * WB_DS;     // ... from one term to the next
 typedef __attribute__((ext_vector_type(8))) __bf16 wb_bf16x8_t;
 typedef short wb_i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void wb_lds_void_t;
@@ -1125,8 +1146,7 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     const bf16_t* __restrict__ x, const float* __restrict__ dlogits,
     float* __restrict__ planes, int64_t T_tokens, int M, int E, int chunk) {
   __shared__ __attribute__((aligned(16))) unsigned char xs[WB_KT * WB_XS];
-  __shared__ __attribute__((aligned(16))) unsigned char dhs[WB_KT * WB_DS];
-  __shared__ __attribute__((aligned(16))) unsigned char dls[WB_KT * WB_DS];
+  __shared__ __attribute__((aligned(16))) unsigned char ds[3 * WB_DT];
   const int m0 = blockIdx.x * WB_M, e0 = blockIdx.z * 64;
   const int64_t t0 = (int64_t)blockIdx.y * chunk;
   const int64_t t1 = t0 + chunk < T_tokens ? t0 + chunk : T_tokens;
@@ -1143,10 +1163,8 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
   const int rcol = (g16 & 1) * 16 + 4 * (t16 & 3);
   const uint32_t xa = (uint32_t)(size_t)(wb_lds_void_t*)xs + rrow * WB_XS +
                       (wave * 32 + rcol) * 2;
-  const uint32_t ha = (uint32_t)(size_t)(wb_lds_void_t*)dhs + rrow * WB_DS +
-                      rcol * 2;
-  const uint32_t la = (uint32_t)(size_t)(wb_lds_void_t*)dls + rrow * WB_DS +
-                      rcol * 2;
+  const uint32_t dsa = (uint32_t)(size_t)(wb_lds_void_t*)ds + rrow * WB_DS +
+                       rcol * 2;
   const uint4 z4 = make_uint4(0, 0, 0, 0);
   uint4 xv0, xv1, da, db;
   auto load = [&](int64_t tb) {
@@ -1162,43 +1180,41 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
   };
   load(t0);
   for (int64_t tb = t0; tb < t1; tb += WB_KT) {
-    const uint32_t dw[8] = {da.x, da.y, da.z, da.w, db.x, db.y, db.z, db.w};
-    float d[8], lo[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      d[j] = __uint_as_float(dw[j]);
-      lo[j] = d[j] - round_to<bf16_t>(d[j]);
-    }
+    const float d[8] = {__uint_as_float(da.x), __uint_as_float(da.y),
+                        __uint_as_float(da.z), __uint_as_float(da.w),
+                        __uint_as_float(db.x), __uint_as_float(db.y),
+                        __uint_as_float(db.z), __uint_as_float(db.w)};
+    uint4 term[3];
+    split_bf16x3(d, term);
     __syncthreads();                 // the previous batch has been consumed
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32) = xv0;
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32 + 16) = xv1;
-    *reinterpret_cast<uint4*>(dhs + sr * WB_DS + sc * 16) = pack16(d, bf16_t());
-    *reinterpret_cast<uint4*>(dls + sr * WB_DS + sc * 16) = pack16(lo, bf16_t());
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      *reinterpret_cast<uint4*>(ds + i * WB_DT + sr * WB_DS + sc * 16) = term[i];
     __syncthreads();
     if (tb + WB_KT < t1) load(tb + WB_KT);
-    // 16 tokens per step: the x operand and, per 32 experts, hi and lo
-    const wb_bf16x8_t a0 = lds_read_tr8<0, 4 * WB_XS>(xa);
-    const wb_bf16x8_t h00 = lds_read_tr8<0, 4 * WB_DS>(ha);
-    const wb_bf16x8_t l00 = lds_read_tr8<0, 4 * WB_DS>(la);
-    const wb_bf16x8_t h01 = lds_read_tr8<64, 4 * WB_DS>(ha);
-    const wb_bf16x8_t l01 = lds_read_tr8<64, 4 * WB_DS>(la);
-    const wb_bf16x8_t a1 = lds_read_tr8<16 * WB_XS, 4 * WB_XS>(xa);
-    const wb_bf16x8_t h10 = lds_read_tr8<16 * WB_DS, 4 * WB_DS>(ha);
-    const wb_bf16x8_t l10 = lds_read_tr8<16 * WB_DS, 4 * WB_DS>(la);
-    const wb_bf16x8_t h11 = lds_read_tr8<16 * WB_DS + 64, 4 * WB_DS>(ha);
-    const wb_bf16x8_t l11 = lds_read_tr8<16 * WB_DS + 64, 4 * WB_DS>(la);
+    // 16 tokens per step: the x operand and, per 32 experts, the three terms
+    const wb_bf16x8_t a[2] = {lds_read_tr8<0, 4 * WB_XS>(xa),
+                              lds_read_tr8<16 * WB_XS, 4 * WB_XS>(xa)};
+    wb_bf16x8_t d0[2][3], d1[2][3];
+#define MOE_WB_READ(K_, I_)                                                    \
+  d0[K_][I_] = lds_read_tr8<I_ * WB_DT + K_ * 16 * WB_DS, 4 * WB_DS>(dsa);     \
+  d1[K_][I_] = lds_read_tr8<I_ * WB_DT + K_ * 16 * WB_DS + 64, 4 * WB_DS>(dsa)
+    MOE_WB_READ(0, 0); MOE_WB_READ(0, 1); MOE_WB_READ(0, 2);
+    MOE_WB_READ(1, 0); MOE_WB_READ(1, 1); MOE_WB_READ(1, 2);
+#undef MOE_WB_READ
     // the compiler does not count the asm reads: wait for them here
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_sched_barrier(0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, h00, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, h01, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, l00, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, l01, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, h10, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, h11, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, l10, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, l11, acc1, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], d0[k][i], acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], d1[k][i], acc1, 0, 0, 0);
+      }
   }
   float* part = planes + (int64_t)blockIdx.y * M * E;
 #pragma unroll

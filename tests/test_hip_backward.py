@@ -333,7 +333,7 @@ def test_compact_gradient_calls_edge_fills(hip):
                          ids=lambda s: "x".join(map(str, s)))
 def test_dispatch_backward_router_share_on_matrix_cores(hip, shape):
   """d(tokens) = the rows of d(expert_in) + d(logits) . w_gate^T with the
-  second term on the bfloat16 matrix cores (d(logits) as two bfloat16 terms):
+  second term on the bfloat16 matrix cores (d(logits) as three bfloat16 terms):
   against float64 arithmetic rounded once, and against the kernel that does
   the term in float32 multiply-adds (equal up to one rounding step of the
   result)."""
@@ -373,6 +373,36 @@ def test_dispatch_backward_router_share_ragged_sizes(hip, shape):
   test_dispatch_backward_router_share_on_matrix_cores(hip, shape)
 
 
+@pytest.mark.parametrize("shape", [(2, 50, 776, 24), (1, 64, 256, 16),
+                                   (1, 96, 136, 12), (3, 333, 640, 40)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_router_terms_keep_all_bits_of_the_logit_gradients(hip, shape):
+  """Gradients that cancel down to their last bits: 1 + 2^-10 + 2^-20 less
+  1 + 2^-10, over two tokens in the router kernel's gradient and over two
+  experts in the router's share of d(tokens).  Every sum is exact in float32,
+  in any order."""
+  g, s, m, e = shape
+  dt = torch.bfloat16
+  scale = 2.0 ** (torch.arange(e, device="cuda") % 7 - 3.0)
+  whole, part = 1 + 2.0 ** -10 + 2.0 ** -20, 1 + 2.0 ** -10
+  d = torch.zeros(g * s, e, device="cuda")
+  d[3] = whole * scale
+  d[g * s - 2] = -part * scale
+  x = torch.zeros(g * s, m, dtype=dt, device="cuda")
+  x[3] = x[g * s - 2] = 0.5
+  dw = hip.router_backward_weights(x, d)
+  assert torch.equal(dw.float(), (2.0 ** -21 * scale).expand(m, e))
+  r = hip.top2_gating(torch.randn(g, s, e, device="cuda"), 4)
+  dxe = torch.zeros(e, g, 4, m, dtype=dt, device="cuda")
+  d = torch.zeros(g, s, e, device="cuda")
+  d[..., 1], d[..., e - 1] = whole, -part
+  w = torch.zeros(m, e, dtype=dt, device="cuda")
+  w[:, 1] = w[:, e - 1] = 2.0
+  w_p = hip.pack_weights(w.reshape(1, m, e), dt).reshape(e, m)
+  dx = hip.dispatch_backward(dxe, r, s, d, w_p, w_gate=w)
+  assert bool((dx.float() == 2.0 ** -19).all())
+
+
 @pytest.mark.parametrize("case", [
     ("top_2", 3, 50, 24, 40, 12, 1.25, "float32", True),
     ("top_2", 2, 65, 16, 24, 68, 1.0, "float32", False),
@@ -397,7 +427,7 @@ def test_router_backward_weights_sizes(hip, shape, act_dtype):
 def test_full_size_router_terms_on_matrix_cores(hip):
   """Configuration 4's token count and widths (65536 tokens, d_model 4096, 64
   experts).  The router kernel's gradient from bfloat16 tokens (d(logits) as
-  two bfloat16 terms on the bfloat16 matrix cores) against the same product
+  three bfloat16 terms on the bfloat16 matrix cores) against the same product
   from the tokens widened to float32 (float32 matrix cores); the router's
   share of d(tokens) on the matrix cores against the kernel with float32
   multiply-adds.  Each pair equal up to one rounding step of the bfloat16
