@@ -329,23 +329,28 @@ __global__ __launch_bounds__(256) void dispatch_backward_router4_kernel(
 // Eight float32 as three bfloat16 terms each, term[0] + term[1] + term[2] == d
 // exactly: the leading 8 significant bits, the next 8 and the last 8.  (Terms are
 // cut off, not rounded, so that none is larger than d.  Only bits below the
-// smallest bfloat16, 2^-133, can be lost.)
+// smallest bfloat16, 2^-133, can be lost.)  An infinity or a NaN is the first
+// term, the others are 0.  (The other operand of the products below is finite
+// wherever d is: a token or router kernel that is not gives NaN logits.)
 __device__ __forceinline__ void split_bf16x3(const float (&d)[8],
                                              uint4 (&term)[3]) {
   uint32_t t[3][8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    float rest = d[j];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      t[i][j] = __float_as_uint(rest) & 0xffff0000u;
-      if (i < 2) rest -= __uint_as_float(t[i][j]);
-    }
+    const uint32_t bits = __float_as_uint(d[j]), size = bits & 0x7fffffffu;
+    t[0][j] = bits & 0xffff0000u;
+    if (size > 0x7f800000u) t[0][j] |= 0x00400000u;   // still a NaN when cut off
+    const float rest =
+        size < 0x7f800000u ? d[j] - __uint_as_float(t[0][j]) : 0.f;
+    t[1][j] = __float_as_uint(rest) & 0xffff0000u;
+    t[2][j] = __float_as_uint(rest - __uint_as_float(t[1][j]));
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i)
-    term[i] = make_uint4(t[i][1] | t[i][0] >> 16, t[i][3] | t[i][2] >> 16,
-                         t[i][5] | t[i][4] >> 16, t[i][7] | t[i][6] >> 16);
+    term[i] = make_uint4((t[i][1] & 0xffff0000u) | t[i][0] >> 16,
+                         (t[i][3] & 0xffff0000u) | t[i][2] >> 16,
+                         (t[i][5] & 0xffff0000u) | t[i][4] >> 16,
+                         (t[i][7] & 0xffff0000u) | t[i][6] >> 16);
 }
 
 // The same for bfloat16 with the router's share on the matrix cores

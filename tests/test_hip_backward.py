@@ -403,6 +403,40 @@ def test_router_terms_keep_all_bits_of_the_logit_gradients(hip, shape):
   assert bool((dx.float() == 2.0 ** -19).all())
 
 
+@pytest.mark.parametrize("shape", [(2, 50, 776, 24), (1, 64, 256, 16),
+                                   (1, 96, 136, 12)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_router_terms_of_overflowed_logit_gradients(hip, shape):
+  """d(logits) of +-inf give +-inf where the other factor is not 0, NaN gives
+  NaN, and a finite one above the largest bfloat16 stays finite; other tokens
+  and experts are not touched."""
+  g, s, m, e = shape
+  dt = torch.bfloat16
+  inf, nan = float("inf"), float("nan")
+  huge = 3.4028234e38                  # rounds to inf in bfloat16
+  low_nan = torch.tensor([0x7f800001], dtype=torch.int32).view(torch.float32)
+  d = torch.zeros(g * s, e, device="cuda")
+  d[5, 0], d[6, 1], d[7, 2], d[8, 3], d[9, 5] = inf, -inf, nan, huge, 1.0
+  d[10, 4] = low_nan.cuda()[0]
+  x = torch.full((g * s, m), 2.0 ** -10, dtype=dt, device="cuda")
+  dw = hip.router_backward_weights(x, d).float()
+  assert bool((dw[:, 0] == inf).all() and (dw[:, 1] == -inf).all())
+  assert bool(dw[:, 2].isnan().all() and dw[:, 4].isnan().all())
+  want = torch.tensor(huge * 2.0 ** -10, device="cuda").to(dt).float()
+  assert bool((dw[:, 3] == want).all() and (dw[:, 5] == 2.0 ** -10).all())
+  assert not bool(dw[:, 6:].any())
+  r = hip.top2_gating(torch.randn(g, s, e, device="cuda"), 4)
+  dxe = torch.zeros(e, g, 4, m, dtype=dt, device="cuda")
+  w = torch.full((m, e), 2.0 ** -10, dtype=dt, device="cuda")
+  w_p = hip.pack_weights(w.reshape(1, m, e), dt).reshape(e, m)
+  dx = hip.dispatch_backward(dxe, r, s, d.reshape(g, s, e), w_p, w_gate=w)
+  dx = dx.reshape(g * s, m).float()
+  assert bool((dx[5] == inf).all() and (dx[6] == -inf).all())
+  assert bool(dx[7].isnan().all() and dx[10].isnan().all())
+  assert bool((dx[8] == want).all() and (dx[9] == 2.0 ** -10).all())
+  assert not bool(dx[:5].any() or dx[11:].any())
+
+
 @pytest.mark.parametrize("case", [
     ("top_2", 3, 50, 24, 40, 12, 1.25, "float32", True),
     ("top_2", 2, 65, 16, 24, 68, 1.0, "float32", False),
