@@ -358,20 +358,24 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void lds_write_b64_asm(uint32_t addr, u32x2_t v) {
   asm volatile("ds_write_b64 %0, %1" :: "v"(addr), "v"(v) : "memory");
 }
-__device__ __forceinline__ u32x4_t lds_read_b128_asm(uint32_t addr) {
-  u32x4_t v;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
-  return v;
-}
-// Waits for the LDS reads above; the values pass through it so that nothing
-// that uses them is scheduled ahead of the wait.
-template <int N>
-__device__ __forceinline__ void lds_wait_pieces(u32x4_t (&p)[N]) {
-  static_assert(N == 8, "eight pieces per pass");
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]),
-                 "+v"(p[5]), "+v"(p[6]), "+v"(p[7])
-               :: "memory");
+// Eight 16-byte reads, 8192 bytes apart, the even and the odd ones each from an
+// address of their own, and the wait for them: in one asm, whose outputs then
+// hold what the compiler takes them for.
+__device__ __forceinline__ void lds_read_pieces(u32x4_t (&p)[8], uint32_t even,
+                                                uint32_t odd) {
+  asm volatile("ds_read_b128 %0, %8\n\t"
+               "ds_read_b128 %1, %9 offset:8192\n\t"
+               "ds_read_b128 %2, %8 offset:16384\n\t"
+               "ds_read_b128 %3, %9 offset:24576\n\t"
+               "ds_read_b128 %4, %8 offset:32768\n\t"
+               "ds_read_b128 %5, %9 offset:40960\n\t"
+               "ds_read_b128 %6, %8 offset:49152\n\t"
+               "ds_read_b128 %7, %9 offset:57344\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]), "=&v"(p[4]),
+                 "=&v"(p[5]), "=&v"(p[6]), "=&v"(p[7])
+               : "v"(even), "v"(odd)
+               : "memory");
 }
 
 // Block barrier that publishes LDS writes and waits for nothing else: vector
@@ -754,24 +758,32 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     if (!LISTED) ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
   };
   // GATHER: the slot -> token map entries of the four rows this lane loads in
-  // a tile.  fetch_map issues the four loads back to back without waiting
-  // (written as asm: the compiler would wait for each before issuing the
-  // next, four round trips per tile); the caller waits with vmcnt(0) before
-  // set_tile of the same tile reads map_src.
+  // a tile.  fetch_map issues the four loads back to back and waits for them
+  // with everything else in flight (written as asm: the compiler would wait for
+  // each before issuing the next, four round trips per tile; the wait belongs
+  // to the same asm, whose outputs then hold what the compiler takes them for).
   int map_src[Cfg::A_INSTR];
   auto fetch_map = [&](int logical) {
     if constexpr (GATHER) {
       int e, tm, tn;
       tile_coords(logical, e, tm, tn);
       const int p0 = TAILS ? tile_pieces0(tm) : 0;
+      const int32_t* p[Cfg::A_INSTR];
 #pragma unroll
       for (int j = 0; j < Cfg::A_INSTR; ++j) {
         const int row = row_in_tile((wave + Cfg::WAVES * j) * 8 + (lane >> 3), p0);
-        const int32_t* p =
-            row_map + ((int64_t)e * R + min(tile_row0(tm) + row, R - 1));
-        asm volatile("global_load_dword %0, %1, off"
-                     : "=&v"(map_src[j]) : "v"(p) : "memory");
+        p[j] = row_map + ((int64_t)e * R + min(tile_row0(tm) + row, R - 1));
       }
+      static_assert(Cfg::A_INSTR == 4, "four map entries per lane");
+      asm volatile("global_load_dword %0, %4, off\n\t"
+                   "global_load_dword %1, %5, off\n\t"
+                   "global_load_dword %2, %6, off\n\t"
+                   "global_load_dword %3, %7, off\n\t"
+                   "s_waitcnt vmcnt(0)"
+                   : "=&v"(map_src[0]), "=&v"(map_src[1]), "=&v"(map_src[2]),
+                     "=&v"(map_src[3])
+                   : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3])
+                   : "memory");
     }
   };
   auto set_tile = [&](int logical) {
@@ -1077,10 +1089,6 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   constexpr int CPR_C = BN / 8;  // 16-byte chunks per output row
 
   fetch_map(tile);
-  if constexpr (GATHER) {
-    wait_vmcnt<0>();
-    asm volatile("" ::: "memory");
-  }
   set_tile(tile);
   prologue_head();
   prologue_tail();
@@ -1208,14 +1216,12 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       constexpr int PIECES = EPI_ROWS * CPR_C / Cfg::THREADS;
       static_assert(EPI_ROWS * CPR_C % Cfg::THREADS == 0, "whole pieces");
       u32x4_t piece[PIECES];
-#pragma unroll
-      for (int n = 0; n < PIECES; ++n) {
-        const int c = e_tid + n * Cfg::THREADS;
-        const int srow = c / CPR_C, chunk = c % CPR_C;
-        piece[n] = lds_read_b128_asm(cs0 + srow * EPI_ROW_BYTES +
-                                     ((chunk ^ (srow & 31)) * 16));
-      }
-      lds_wait_pieces(piece);
+      // piece n: staging row (e_tid / CPR_C) + 16 n
+      static_assert(PIECES == 8 && Cfg::THREADS / CPR_C == 16 &&
+                        16 * EPI_ROW_BYTES == 8192, "offsets of the reads");
+      const uint32_t row_at = cs0 + e_tid / CPR_C * EPI_ROW_BYTES;
+      const uint32_t at = (e_tid % CPR_C) ^ (e_tid / CPR_C);
+      lds_read_pieces(piece, row_at + at * 16, row_at + (at ^ 16) * 16);
 #pragma unroll
       for (int n = 0; n < PIECES; ++n) {
         const int c = e_tid + n * Cfg::THREADS;
