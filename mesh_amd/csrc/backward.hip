@@ -1034,6 +1034,17 @@ __global__ __launch_bounds__(256) void gating_backward_rows_kernel(
 constexpr int WM_M = 128, WM_KT = 32;
 typedef float wm_f32x16_t __attribute__((ext_vector_type(16)));
 
+// *p, or zeros.  (As `in ? *p : zero` both sides are places in memory, the
+// compiler chooses between their addresses, and what follows are flat loads word
+// by word, for which the wait for LDS reads waits too: nothing is loaded ahead.
+// 65536 x 4096, 64 experts: 271 us like that, 178 like this; 4096 x 1024, 512
+// experts: 105, 62.)
+__device__ __forceinline__ uint4 load_or_zero(const uint4* p, bool in) {
+  uint4 v = make_uint4(0, 0, 0, 0);
+  if (in) v = *p;
+  return v;
+}
+
 // Tokens per block of the two kernels below: about 512 blocks (two per compute
 // unit), but at least 4 E tokens (a plane of the workspace, 4 E bytes per
 // kernel row written and read, then stays below the tokens' own bytes) and
@@ -1064,22 +1075,19 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
   for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
   // staging: thread -> (token row tid / 8, 16 kernel rows / 8 experts)
   const int sr = tid >> 3, sc = tid & 7;
-  const uint4 z4 = make_uint4(0, 0, 0, 0);
   uint4 xraw[16 / VN], draw[2];
   auto load = [&](int64_t tb) {
     const int64_t t = tb + sr;
 #pragma unroll
     for (int u = 0; u < 16 / VN; ++u)
-      xraw[u] = t < t1 && m0 + sc * 16 + u * VN < M
-                    ? *reinterpret_cast<const uint4*>(x + t * M + m0 + sc * 16 +
-                                                      u * VN)
-                    : z4;
+      xraw[u] = load_or_zero(
+          reinterpret_cast<const uint4*>(x + t * M + m0 + sc * 16 + u * VN),
+          t < t1 && m0 + sc * 16 + u * VN < M);
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      draw[u] = t < t1 && e0 + sc * 8 + u * 4 < E
-                    ? *reinterpret_cast<const uint4*>(dlogits + t * E + e0 +
-                                                      sc * 8 + u * 4)
-                    : z4;
+      draw[u] = load_or_zero(
+          reinterpret_cast<const uint4*>(dlogits + t * E + e0 + sc * 8 + u * 4),
+          t < t1 && e0 + sc * 8 + u * 4 < E);
   };
   load(t0);
   for (int64_t tb = t0; tb < t1; tb += WM_KT) {
@@ -1170,7 +1178,6 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
                       (wave * 32 + rcol) * 2;
   const uint32_t dsa = (uint32_t)(size_t)(wb_lds_void_t*)ds + rrow * WB_DS +
                        rcol * 2;
-  const uint4 z4 = make_uint4(0, 0, 0, 0);
   uint4 xv0, xv1, da, db;
   auto load = [&](int64_t tb) {
     const int64_t t = tb + sr;
@@ -1178,10 +1185,10 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     const int m = m0 + sc * 16, e = e0 + sc * 8;
     const uint4* xp = reinterpret_cast<const uint4*>(x + t * M + m);
     const uint4* dp = reinterpret_cast<const uint4*>(dlogits + t * E + e);
-    xv0 = in && m < M ? xp[0] : z4;
-    xv1 = in && m + 8 < M ? xp[1] : z4;
-    da = in && e < E ? dp[0] : z4;
-    db = in && e + 4 < E ? dp[1] : z4;
+    xv0 = load_or_zero(xp, in && m < M);
+    xv1 = load_or_zero(xp + 1, in && m + 8 < M);
+    da = load_or_zero(dp, in && e < E);
+    db = load_or_zero(dp + 1, in && e + 4 < E);
   };
   load(t0);
   for (int64_t tb = t0; tb < t1; tb += WB_KT) {
@@ -1239,15 +1246,14 @@ __global__ void router_wgrad_reduce_kernel(const float* __restrict__ part,
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float sum = 0.f;
-  int c = 0;
-  for (; c + 8 <= chunks; c += 8) {          // eight loads in flight
-    float v[8];
+  for (int c = 0; c < chunks; c += 16) {     // sixteen loads in flight
+    float v[16];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)(c + u) * n + i];
+    for (int u = 0; u < 16; ++u)
+      v[u] = c + u < chunks ? part[(int64_t)(c + u) * n + i] : 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) sum += v[u];
+    for (int u = 0; u < 16; ++u) sum += v[u];
   }
-  for (; c < chunks; ++c) sum += part[(int64_t)c * n + i];
   store_f32<T>(dw + i, sum);
 }
 
