@@ -458,6 +458,19 @@ def test_router_backward_weights_sizes(hip, shape, act_dtype):
   test_router_backward_weights(hip, shape, act_dtype)
 
 
+@pytest.mark.parametrize("e", [8, 512])
+def test_router_backward_weights_float32_sums_stay_short(hip, e):
+  """No float32 sum runs over more than 512 tokens before the chunks' sums are
+  added: 256 times 1 + 2^-14 and 256 times 1 still have a sum that float32
+  holds, and so do the chunks' sums together."""
+  t, m = 4096, 128
+  x = torch.ones(t, m, device="cuda")
+  d = torch.ones(t, e, device="cuda")
+  d[::2] += 2.0 ** -14
+  dw = hip.router_backward_weights(x, d)
+  assert bool((dw == t + t // 2 * 2.0 ** -14).all())
+
+
 def test_full_size_router_terms_on_matrix_cores(hip):
   """Configuration 4's token count and widths (65536 tokens, d_model 4096, 64
   experts).  The router kernel's gradient from bfloat16 tokens (d(logits) as
