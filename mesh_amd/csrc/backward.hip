@@ -326,31 +326,43 @@ __global__ __launch_bounds__(256) void dispatch_backward_router4_kernel(
   }
 }
 
-// Eight float32 as three bfloat16 terms each, term[0] + term[1] + term[2] == d
-// exactly: the leading 8 significant bits, the next 8 and the last 8.  (Terms are
-// cut off, not rounded, so that none is larger than d.  Only bits below the
-// smallest bfloat16, 2^-133, can be lost.)  An infinity or a NaN is the first
-// term, the others are 0.  (The other operand of the products below is finite
-// wherever d is: a token or router kernel that is not gives NaN logits.)
-__device__ __forceinline__ void split_bf16x3(const float (&d)[8],
-                                             uint4 (&term)[3]) {
-  uint32_t t[3][8];
+// N float32 as TERMS bfloat16 terms each.  Three add up to d exactly: the leading
+// 8 significant bits, the next 8 and the last 8, cut off and not rounded, so that
+// none is larger than d (only bits below the smallest bfloat16, 2^-133, can be
+// lost).  Two are d rounded and what that leaves, rounded: 17 bits.  An infinity
+// or a NaN is the first term, the others are 0.  (The other operand of the
+// products below is finite wherever d is: a token or router kernel that is not
+// gives NaN logits.)
+template <int TERMS, int N>
+__device__ __forceinline__ void split_bf16(const float (&d)[N],
+                                           uint32_t (&term)[TERMS][N / 2]) {
+  static_assert(TERMS == 2 || TERMS == 3, "two or three terms");
+  uint32_t first[N];
+  float rest[N];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < N; ++j) {
     const uint32_t bits = __float_as_uint(d[j]), size = bits & 0x7fffffffu;
-    t[0][j] = bits & 0xffff0000u;
-    if (size > 0x7f800000u) t[0][j] |= 0x00400000u;   // still a NaN when cut off
-    const float rest =
-        size < 0x7f800000u ? d[j] - __uint_as_float(t[0][j]) : 0.f;
-    t[1][j] = __float_as_uint(rest) & 0xffff0000u;
-    t[2][j] = __float_as_uint(rest - __uint_as_float(t[1][j]));
+    first[j] = bits & 0xffff0000u;
+    if (size > 0x7f800000u) first[j] |= 0x00400000u;  // still a NaN when cut off
+    // (rounded only where that does not make an infinity of it)
+    if (TERMS == 2 && size < 0x7f7f8000u)
+      first[j] = __float_as_uint(round_to<bf16_t>(d[j]));
+    rest[j] = size < 0x7f800000u ? d[j] - __uint_as_float(first[j]) : 0.f;
   }
 #pragma unroll
-  for (int i = 0; i < 3; ++i)
-    term[i] = make_uint4((t[i][1] & 0xffff0000u) | t[i][0] >> 16,
-                         (t[i][3] & 0xffff0000u) | t[i][2] >> 16,
-                         (t[i][5] & 0xffff0000u) | t[i][4] >> 16,
-                         (t[i][7] & 0xffff0000u) | t[i][6] >> 16);
+  for (int j = 0; j < N / 2; ++j) {
+    term[0][j] = first[2 * j + 1] | first[2 * j] >> 16;
+    if constexpr (TERMS == 2) {
+      term[1][j] = f32x2_to_bf16x2(rest[2 * j], rest[2 * j + 1]);
+    } else {
+      const uint32_t a = __float_as_uint(rest[2 * j]) & 0xffff0000u;
+      const uint32_t b = __float_as_uint(rest[2 * j + 1]) & 0xffff0000u;
+      term[1][j] = b | a >> 16;
+      term[2][j] =
+          (__float_as_uint(rest[2 * j + 1] - __uint_as_float(b)) & 0xffff0000u) |
+          __float_as_uint(rest[2 * j] - __uint_as_float(a)) >> 16;
+    }
+  }
 }
 
 // The same for bfloat16 with the router's share on the matrix cores
@@ -362,9 +374,12 @@ __device__ __forceinline__ void split_bf16x3(const float (&d)[8],
 // consecutive e straight from global memory touch 32 lines per instruction and
 // ask for every line four times: 0.59 against 0.49 ms for 65536 tokens of 4096)
 // and the lanes take their operands from there.  The float32 d(logits) go in as
-// three bfloat16 terms that add up to them exactly (split_bf16x3): every product
-// is exact in the float32 accumulator, as those of the one-token and four-token
-// kernels are.  The instruction leaves a
+// three bfloat16 terms that add up to them exactly (split_bf16): every product is
+// exact in the float32 accumulator, as those of the one-token and four-token
+// kernels are.  Where every tile is whole (WHOLE) they go in as two: these sizes
+// have had this kernel from the start, and with three they are slower (32 x 1024
+// tokens of 2048, 128 experts: 145 us, 159 with three terms and the ragged sizes'
+// addresses; 112 experts, width 1024: 51, 81).  The instruction leaves a
 // lane with 4 consecutive columns of one token; the tile goes through LDS as
 // float32 (over the kernel rows, which are no longer needed) so that the
 // second phase -- half a wavefront per token row, 16 bytes per lane, the rows
@@ -381,11 +396,15 @@ typedef float dbm_f32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t dbm_u32x4_t __attribute__((ext_vector_type(4)));
 
 // LDS bytes: [kernel rows | share] then the d(logits) rows
-static size_t dbm_lds_bytes(int E) {
+static size_t dbm_lds_bytes(int E, bool whole) {
   E = (E + 15) / 16 * 16;
   const size_t wbytes = (size_t)DBM_COLS * (E * 2 + 16);
   const size_t sbytes = sizeof(float) * DBM_TOK * DBM_LD;
-  return (wbytes > sbytes ? wbytes : sbytes) + (size_t)DBM_TOK * (E * 4 + 16);
+  return (wbytes > sbytes ? wbytes : sbytes) + (size_t)DBM_TOK * (E * (whole ? 4 : 6) + 16);
+}
+
+static bool dbm_whole(int S, int E, int M) {
+  return M % DBM_COLS == 0 && E % 16 == 0 && S % DBM_TOK == 0;
 }
 
 // Block barrier that waits for this wavefront's LDS accesses only.
@@ -402,17 +421,22 @@ __device__ __forceinline__ void dbm_lds_barrier() {
 // expert-selection router (tok_slot [T, E] int16, -1 = not chosen by that
 // expert; any number of rows per token) instead of the per-token record.
 // COMPACT: the rows lie in the compacted order (row_offsets given).
-template <int KS, bool SLOT = false, bool COMPACT = false>
+// WHOLE: M % 256 == 0, E % 16 == 0 and S % 32 == 0 (a block's tokens share a
+// group).
+template <int KS, bool WHOLE, bool SLOT = false, bool COMPACT = false>
 __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
     const bf16_t* __restrict__ dxe, const int32_t* __restrict__ idx,
     const int32_t* __restrict__ pos, const float* __restrict__ gate,
     const uint8_t* __restrict__ kept, const float* __restrict__ dlogits,
-    const bf16_t* __restrict__ wg, bf16_t* __restrict__ dx, int G, int S, int E,
-    int C, int M, int64_t T_tokens, int groups_per_router,
+    const bf16_t* __restrict__ wg, bf16_t* __restrict__ dx, int G, int S,
+    int experts, int C, int M, int64_t T_tokens, int groups_per_router,
     const int32_t* __restrict__ row_offsets,
     const int16_t* __restrict__ tok_slot = nullptr) {
   constexpr int EP = KS * 16;                             // E, padded
-  constexpr int WROW = EP * 2 + 16, DROW = EP * 4 + 16;   // padded LDS rows, bytes
+  constexpr int TERMS = WHOLE ? 2 : 3;
+  // padded LDS rows, bytes
+  constexpr int WROW = EP * 2 + 16, DROW = EP * 2 * TERMS + 16;
+  const int E = WHOLE ? EP : experts;
   constexpr int WBYTES = DBM_COLS * WROW;
   constexpr int SBYTES = (int)sizeof(float) * DBM_TOK * DBM_LD;
   extern __shared__ __attribute__((aligned(16))) unsigned char dbm_smem[];
@@ -423,9 +447,14 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
   const int half = lane >> 5, l32 = lane & 31;
   const int64_t t0 = (int64_t)blockIdx.y * DBM_TOK;
   const int m0 = blockIdx.x * DBM_COLS;
-  wg += (t0 / S / groups_per_router) * M * E;
+  // (the caller has at most 65535 blocks of tokens: their numbers fit in 32 bits)
+  const uint32_t g0 = (uint32_t)t0 / (uint32_t)S;
+  auto group_of = [&](int64_t t) {
+    return (int64_t)(WHOLE ? g0 : (uint32_t)t / (uint32_t)S);
+  };
+  wg += (int64_t)(g0 / (uint32_t)groups_per_router) * M * E;
   // this lane's 8 columns of a token row (the last tile may reach past M)
-  const bool col_in = m0 + 8 * l32 < M;
+  const bool col_in = WHOLE || m0 + 8 * l32 < M;
   const int col_at = col_in ? m0 + 8 * l32 : 0;
 
   constexpr int WPR = EP / 8;                 // 16-byte pieces per kernel row
@@ -466,7 +495,8 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
 #pragma unroll
   for (int i = 0; i < WP; ++i) {
     const int p = tid + 256 * i;
-    const int row = min(m0 + p / WPR, M - 1), piece = p % WPR;
+    const int row = WHOLE ? m0 + p / WPR : min(m0 + p / WPR, M - 1);
+    const int piece = p % WPR;
     const uint4* src = reinterpret_cast<const uint4*>(
         wg + (int64_t)row * E + (piece * 8 < E ? piece * 8 : 0));
     asm volatile("global_load_dwordx4 %0, %1, off"
@@ -478,7 +508,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
   for (int i = 0; i < DP; ++i) {
     const int p = tid + 256 * i;
     dv_used[i] = p < DBM_TOK * DPR && t0 + p / DPR < T_tokens &&
-                 (p % DPR) * 4 < E;
+                 (WHOLE || (p % DPR) * 4 < E);
     dv[i] = *reinterpret_cast<const float4*>(
         dlogits + t0 * E + (dv_used[i] ? (p / DPR) * E + (p % DPR) * 4 : 0));
   }
@@ -493,7 +523,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
     for (int j = 0; j < RP; ++j) {
       int64_t t = t0 + wave * 8 + 2 * j + half;
       t = t < T_tokens ? t : T_tokens - 1;
-      const int64_t g = t / S;
+      const int64_t g = group_of(t);
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int64_t e = k ? idx2[j].y : idx2[j].x;
@@ -535,14 +565,21 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
     const int p = tid + 256 * i;
     const dbm_u32x4_t zero = {0, 0, 0, 0};
     *reinterpret_cast<dbm_u32x4_t*>(wl + (p / WPR) * WROW + (p % WPR) * 16) =
-        (p % WPR) * 8 < E ? wv[i] : zero;
+        WHOLE || (p % WPR) * 8 < E ? wv[i] : zero;
   }
 #pragma unroll
   for (int i = 0; i < DP; ++i) {
     const int p = tid + 256 * i;
-    if (p < DBM_TOK * DPR)
-      *reinterpret_cast<float4*>(dl + (p / DPR) * DROW + (p % DPR) * 16) =
-          dv_used[i] ? dv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    if (p < DBM_TOK * DPR) {
+      const float d[4] = {dv_used[i] ? dv[i].x : 0.f, dv_used[i] ? dv[i].y : 0.f,
+                          dv_used[i] ? dv[i].z : 0.f, dv_used[i] ? dv[i].w : 0.f};
+      uint32_t term[TERMS][2];
+      split_bf16(d, term);
+#pragma unroll
+      for (int n = 0; n < TERMS; ++n)
+        *reinterpret_cast<uint2*>(dl + (p / DPR) * DROW + n * EP * 2 +
+                                  (p % DPR) * 8) = make_uint2(term[n][0], term[n][1]);
+    }
   }
   dbm_lds_barrier();
   uint4 afrag[2][KS];
@@ -561,18 +598,16 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
       for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const float4 d0 = *reinterpret_cast<const float4*>(dl + l32 * DROW + ks * 64 + half * 32);
-      const float4 d1 = *reinterpret_cast<const float4*>(dl + l32 * DROW + ks * 64 + half * 32 + 16);
-      const float d[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
-      uint4 term[3];
-      split_bf16x3(d, term);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
+      for (int i = 0; i < TERMS; ++i) {
+        const uint4 term = *reinterpret_cast<const uint4*>(
+            dl + l32 * DROW + i * EP * 2 + ks * 32 + half * 16);
 #pragma unroll
         for (int b = 0; b < 2; ++b)
           acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               __builtin_bit_cast(dbm_bf16x8_t, afrag[b][ks]),
-              __builtin_bit_cast(dbm_bf16x8_t, term[i]), acc[b], 0, 0, 0);
+              __builtin_bit_cast(dbm_bf16x8_t, term), acc[b], 0, 0, 0);
+      }
     }
     // (the share goes over the kernel rows: every wavefront has its operands
     // in registers before the first write)
@@ -602,7 +637,7 @@ __global__ __launch_bounds__(256) void dispatch_backward_mfma_kernel(
       if constexpr (SLOT) {
         // this half-wavefront's token: lane l32 looks at experts l32, l32 + 32,
         // ..; the rows are added in expert order
-        const int64_t g = t / S;
+        const int64_t g = group_of(t);
 #pragma unroll
         for (int q = 0; q < 8; ++q) { a[q] = 0.f; b[q] = 0.f; }
         for (int e0 = 0; e0 < E; e0 += 32) {
@@ -1037,8 +1072,8 @@ typedef float wm_f32x16_t __attribute__((ext_vector_type(16)));
 // *p, or zeros.  (As `in ? *p : zero` both sides are places in memory, the
 // compiler chooses between their addresses, and what follows are flat loads word
 // by word, for which the wait for LDS reads waits too: nothing is loaded ahead.
-// 65536 x 4096, 64 experts: 271 us like that, 178 like this; 4096 x 1024, 512
-// experts: 105, 62.)
+// 65536 x 4096, 64 experts: 269 us like that, 156 like this; 4096 x 1024, 512
+// experts: 97, 61.)
 __device__ __forceinline__ uint4 load_or_zero(const uint4* p, bool in) {
   uint4 v = make_uint4(0, 0, 0, 0);
   if (in) v = *p;
@@ -1126,7 +1161,10 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
 // The same product for bfloat16 tokens on the bfloat16 matrix cores
 // (v_mfma_f32_32x32x16_bf16, 16 tokens per instruction instead of 2).  The
 // float32 d(logits) go in as three bfloat16 terms that add up to them exactly
-// (split_bf16x3), so that every product is exact in the float32 accumulator.
+// (split_bf16), so that every product is exact in the float32 accumulator, or as
+// two for M % 128 == 0 and E % 8 == 0: sizes that have had this kernel from the
+// start and are slower with three (65536 x 4096, 64 experts: 156 us, 178 with
+// three).
 // Both operands lie in memory with the reduction index (the token)
 // outermost; they are staged in LDS as they lie and the instruction's
 // operands (8 consecutive tokens of one kernel row / one expert per lane) are
@@ -1158,11 +1196,12 @@ __device__ __forceinline__ wb_bf16x8_t lds_read_tr8(uint32_t addr) {
       wb_bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
+template <int TERMS>
 __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     const bf16_t* __restrict__ x, const float* __restrict__ dlogits,
     float* __restrict__ planes, int64_t T_tokens, int M, int E, int chunk) {
   __shared__ __attribute__((aligned(16))) unsigned char xs[WB_KT * WB_XS];
-  __shared__ __attribute__((aligned(16))) unsigned char ds[3 * WB_DT];
+  __shared__ __attribute__((aligned(16))) unsigned char ds[TERMS * WB_DT];
   const int m0 = blockIdx.x * WB_M, e0 = blockIdx.z * 64;
   const int64_t t0 = (int64_t)blockIdx.y * chunk;
   const int64_t t1 = t0 + chunk < T_tokens ? t0 + chunk : T_tokens;
@@ -1199,25 +1238,29 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
                         __uint_as_float(da.z), __uint_as_float(da.w),
                         __uint_as_float(db.x), __uint_as_float(db.y),
                         __uint_as_float(db.z), __uint_as_float(db.w)};
-    uint4 term[3];
-    split_bf16x3(d, term);
+    uint32_t term[TERMS][4];
+    split_bf16(d, term);
     __syncthreads();                 // the previous batch has been consumed
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32) = xv0;
     *reinterpret_cast<uint4*>(xs + sr * WB_XS + sc * 32 + 16) = xv1;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      *reinterpret_cast<uint4*>(ds + i * WB_DT + sr * WB_DS + sc * 16) = term[i];
+    for (int i = 0; i < TERMS; ++i)
+      *reinterpret_cast<uint4*>(ds + i * WB_DT + sr * WB_DS + sc * 16) =
+          make_uint4(term[i][0], term[i][1], term[i][2], term[i][3]);
     __syncthreads();
     if (tb + WB_KT < t1) load(tb + WB_KT);
-    // 16 tokens per step: the x operand and, per 32 experts, the three terms
+    // 16 tokens per step: the x operand and, per 32 experts, the terms
     const wb_bf16x8_t a[2] = {lds_read_tr8<0, 4 * WB_XS>(xa),
                               lds_read_tr8<16 * WB_XS, 4 * WB_XS>(xa)};
-    wb_bf16x8_t d0[2][3], d1[2][3];
+    wb_bf16x8_t d0[2][TERMS], d1[2][TERMS];
 #define MOE_WB_READ(K_, I_)                                                    \
   d0[K_][I_] = lds_read_tr8<I_ * WB_DT + K_ * 16 * WB_DS, 4 * WB_DS>(dsa);     \
   d1[K_][I_] = lds_read_tr8<I_ * WB_DT + K_ * 16 * WB_DS + 64, 4 * WB_DS>(dsa)
-    MOE_WB_READ(0, 0); MOE_WB_READ(0, 1); MOE_WB_READ(0, 2);
-    MOE_WB_READ(1, 0); MOE_WB_READ(1, 1); MOE_WB_READ(1, 2);
+    MOE_WB_READ(0, 0); MOE_WB_READ(0, 1);
+    MOE_WB_READ(1, 0); MOE_WB_READ(1, 1);
+    if constexpr (TERMS == 3) {
+      MOE_WB_READ(0, 2); MOE_WB_READ(1, 2);
+    }
 #undef MOE_WB_READ
     // the compiler does not count the asm reads: wait for them here
     __builtin_amdgcn_sched_barrier(0);
@@ -1226,7 +1269,7 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
+      for (int i = 0; i < TERMS; ++i) {
         acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], d0[k][i], acc0, 0, 0, 0);
         acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k], d1[k][i], acc1, 0, 0, 0);
       }
@@ -1404,7 +1447,8 @@ bool launch_slot_dispatch_backward_mfma(
     return false;
   dim3 grid((unsigned)((M + DBM_COLS - 1) / DBM_COLS),
             (unsigned)((T_tokens + DBM_TOK - 1) / DBM_TOK));
-  const size_t lds = dbm_lds_bytes(E);
+  const bool whole = dbm_whole(S, E, M);
+  const size_t lds = dbm_lds_bytes(E, whole);
   auto run = [&](auto k) -> int {
     MOE_ALLOW_LDS(k, lds);
     k<<<grid, 256, lds, st>>>(
@@ -1415,14 +1459,18 @@ bool launch_slot_dispatch_backward_mfma(
     return 0;
   };
   switch ((E + 15) / 16) {
-    case 1: *rc = run(dispatch_backward_mfma_kernel<1, true>); break;
-    case 2: *rc = run(dispatch_backward_mfma_kernel<2, true>); break;
-    case 3: *rc = run(dispatch_backward_mfma_kernel<3, true>); break;
-    case 4: *rc = run(dispatch_backward_mfma_kernel<4, true>); break;
-    case 5: *rc = run(dispatch_backward_mfma_kernel<5, true>); break;
-    case 6: *rc = run(dispatch_backward_mfma_kernel<6, true>); break;
-    case 7: *rc = run(dispatch_backward_mfma_kernel<7, true>); break;
-    default: *rc = run(dispatch_backward_mfma_kernel<8, true>); break;
+#define MOE_DBM(KS_)                                                         \
+  *rc = whole ? run(dispatch_backward_mfma_kernel<KS_, true, true>)          \
+              : run(dispatch_backward_mfma_kernel<KS_, false, true>)
+    case 1: MOE_DBM(1); break;
+    case 2: MOE_DBM(2); break;
+    case 3: MOE_DBM(3); break;
+    case 4: MOE_DBM(4); break;
+    case 5: MOE_DBM(5); break;
+    case 6: MOE_DBM(6); break;
+    case 7: MOE_DBM(7); break;
+    default: MOE_DBM(8); break;
+#undef MOE_DBM
   }
   return true;
 }
@@ -1559,31 +1607,34 @@ static int run_dispatch_backward(
       (T_tokens + DBM_TOK - 1) / DBM_TOK <= 65535) {
     dim3 grid((unsigned)((M + DBM_COLS - 1) / DBM_COLS),
               (unsigned)((T_tokens + DBM_TOK - 1) / DBM_TOK));
-    const size_t lds = dbm_lds_bytes(E);
+    const bool whole = dbm_whole(S, E, M);
+    const size_t lds = dbm_lds_bytes(E, whole);
+    auto run = [&](auto k) -> int {
+      MOE_ALLOW_LDS(k, lds);
+      k<<<grid, 256, lds, st>>>(
+          (const bf16_t*)dexpert_in, idx, pos, gate, kept, dlogits,
+          (const bf16_t*)w_gate, (bf16_t*)dx, G, S, E, C, M, T_tokens,
+          groups_per_router, row_offsets, nullptr);
+      MOE_CHECK_LAUNCH("dispatch_backward (router share on the matrix cores)");
+      return 0;
+    };
 #define MOE_DBM(KS_)                                                         \
-  do {                                                                       \
-    auto k = row_offsets != nullptr                                          \
-                 ? dispatch_backward_mfma_kernel<KS_, false, true>           \
-                 : dispatch_backward_mfma_kernel<KS_, false, false>;         \
-    MOE_ALLOW_LDS(k, lds);                                                   \
-    k<<<grid, 256, lds, st>>>(                                               \
-        (const bf16_t*)dexpert_in, idx, pos, gate, kept, dlogits,            \
-        (const bf16_t*)w_gate, (bf16_t*)dx, G, S, E, C, M, T_tokens,         \
-        groups_per_router, row_offsets, nullptr);                            \
-  } while (0)
+  return row_offsets != nullptr                                              \
+             ? whole ? run(dispatch_backward_mfma_kernel<KS_, true, false, true>) \
+                     : run(dispatch_backward_mfma_kernel<KS_, false, false, true>) \
+         : whole ? run(dispatch_backward_mfma_kernel<KS_, true>)             \
+                 : run(dispatch_backward_mfma_kernel<KS_, false>)
     switch ((E + 15) / 16) {
-      case 1: MOE_DBM(1); break;
-      case 2: MOE_DBM(2); break;
-      case 3: MOE_DBM(3); break;
-      case 4: MOE_DBM(4); break;
-      case 5: MOE_DBM(5); break;
-      case 6: MOE_DBM(6); break;
-      case 7: MOE_DBM(7); break;
-      default: MOE_DBM(8); break;
+      case 1: MOE_DBM(1);
+      case 2: MOE_DBM(2);
+      case 3: MOE_DBM(3);
+      case 4: MOE_DBM(4);
+      case 5: MOE_DBM(5);
+      case 6: MOE_DBM(6);
+      case 7: MOE_DBM(7);
+      default: MOE_DBM(8);
     }
 #undef MOE_DBM
-    MOE_CHECK_LAUNCH("dispatch_backward (router share on the matrix cores)");
-    return 0;
   }
   if (vec && dlogits != nullptr && E <= DBR_MAX_E && S % DBR_TOK == 0) {
     const int64_t nb4 = (T_tokens + 4 * DBR_TOK - 1) / (4 * DBR_TOK);
@@ -1777,8 +1828,10 @@ extern "C" int mesh_moe_router_backward_weights(const void* x,
       router_wgrad_reduce_kernel<float><<<rb, 256, 0, st>>>(
           workspace, (float*)dw_gate, n, planes);
     } else {
-      router_wgrad_bf16_kernel<<<mgrid, 256, 0, st>>>(
-          (const bf16_t*)x, dlogits, workspace, tokens, M, E, chunk);
+      auto k = M % WB_M == 0 && E % 8 == 0 ? router_wgrad_bf16_kernel<2>
+                                           : router_wgrad_bf16_kernel<3>;
+      k<<<mgrid, 256, 0, st>>>((const bf16_t*)x, dlogits, workspace, tokens, M,
+                               E, chunk);
       MOE_CHECK_LAUNCH("router_backward_weights (mfma, bf16 terms)");
       router_wgrad_reduce_kernel<bf16_t><<<rb, 256, 0, st>>>(
           workspace, (bf16_t*)dw_gate, n, planes);
