@@ -1918,12 +1918,16 @@ static int launch_mfma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
 }
 
 constexpr int SKINNY_ROWS = 128;
+// Columns of a block of the kernel for few rows and few columns.
+static int skinny_columns(int E, int N) {
+  return (int64_t)E * ((N + 15) / 16) <= compute_units() ? 16 : 32;
+}
 
 static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                          int R, int N, int K, bool relu, hipStream_t st) {
-  // 32 columns per block (half the token reads of 16), 16 while that leaves
-  // compute units without a block
-  const int nt = (int64_t)E * ((N + 31) / 32) >= 512 ? 2 : 1;
+  // 16 columns per block while no compute unit gets a second block, else 32
+  // (half the token reads)
+  const int nt = skinny_columns(E, N) / 16;
   const int groups_n = (N + 16 * nt - 1) / (16 * nt);
   const int64_t blocks = (int64_t)E * groups_n;
   MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
@@ -1935,6 +1939,7 @@ static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     waves *= 2;
   int mt = (R + 15) / 16;              // 1, 2, 3, 4, 6 or 8 tiles of 16 rows
   mt = mt == 5 || mt == 7 ? mt + 1 : mt;
+  while (waves * mt * nt > 128) waves /= 2;    // 128 KB of LDS
   const size_t lds = (size_t)waves * mt * nt * 64 * 16;
   auto run = [&](auto k) -> int {
     MOE_ALLOW_LDS(k, lds);
@@ -1957,21 +1962,39 @@ static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
 #undef MOE_SKINNY
 }
 
-// The two kernels for a few rows per expert.  Where the launch has a 128-column
-// tile for half of the compute units, the stream of whole lines; below, the
-// skinny kernel, which cuts the reduction so that every unit has work (one
-// expert of 32 rows, 4096 x 1024: 15 us against 22 for the stream's 8 blocks; 8
-// experts of 64 rows, 1024 x 2048, 128 tiles: 16 against 12).
+// The two kernels for a few rows per expert.  The skinny one cuts the reduction
+// so that every compute unit has work; it is the faster one while no unit gets a
+// second block of 32 columns (blocks that do not fit in one round, each with all
+// of the token rows to read, cost up to twice the tile kernels' time: 128 rows,
+// 16000 x 4096: 135 us, 128 x 128 tiles 75).  Above, up to 64 rows, the stream of
+// whole lines.  us, one expert, K = 4096, by columns: 16 a block / 32 a block /
+// stream / best tile kernel:
+//    64 rows   4096: 25, 28, 33, 57   8192: 46, 29, 34, 58  10240: 66, 52, 34, 57
+//    96 rows   4096: 30, 36, -, 56    8192: 55, 37, -, 57   10240: 84, 70, -, 57
+//   128 rows   4096: 37, 47, -, 56    8192: 70, 48, -, 57   10240: 102, 91, -, 57
+// Above 96 rows, blocks of 32 columns win with long reductions only (8192 columns,
+// K = 1024: 16.2, tiles 14.8; 2048: 27, 32).  Reductions that the stream does not
+// take (K % 64 != 0) keep to 32 columns a block (64 rows, 16000 x 1024: 16, 128 x
+// 128 tiles 22).
 constexpr int STREAM_ROWS = 64;
-static bool stream_applies(int E, int R, int N, int K) {
-  const int cus = compute_units();
-  return R <= STREAM_ROWS && K % 64 == 0 && N % 8 == 0 && cus > 0 &&
-         (int64_t)E * ((N + 127) / 128) * 2 >= cus;
+static bool skinny_rounds(int E, int N) {
+  return (int64_t)E * ((N + 31) / 32) <= compute_units();
+}
+// a 128-column tile for half of the compute units
+static bool many_column_tiles(int E, int N) {
+  return (int64_t)E * ((N + 127) / 128) * 2 >= compute_units();
 }
 static bool skinny_applies(int E, int R, int N, int K) {
-  const int cus = compute_units();
-  return R <= SKINNY_ROWS && N % 16 == 0 && K % 32 == 0 && cus > 0 &&
-         (int64_t)E * ((N + 127) / 128) * 2 < cus;
+  if (compute_units() == 0 || N % 16 != 0 || K % 32 != 0 || R > SKINNY_ROWS ||
+      many_column_tiles(E, N))
+    return false;
+  if (R <= STREAM_ROWS) return skinny_rounds(E, N) || K % 64 != 0;
+  return skinny_rounds(E, N) &&
+         (R <= 96 || K > 1024 || skinny_columns(E, N) == 16);
+}
+static bool stream_applies(int E, int R, int N, int K) {
+  return compute_units() > 0 && R <= STREAM_ROWS && K % 64 == 0 && N % 8 == 0 &&
+         (many_column_tiles(E, N) || !skinny_rounds(E, N));
 }
 
 // row_map / gather / zero_row: see the kernel (null: rows as they lie)
@@ -2630,7 +2653,7 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
   const int64_t rows = (int64_t)G * C;
   const bool few_rows =
       rows <= STREAM_ROWS && (int64_t)G * S < (1 << 30) &&
-      stream_applies(E, (int)rows, H, M) &&
+      stream_applies(E, (int)rows, H, M) && many_column_tiles(E, H) &&
       ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
   MOE_REQUIRE(dtype == MESH_MOE_BF16 && rows <= 0x7fffffffLL &&
                   (int64_t)G * S <= 0x7fffffffLL &&

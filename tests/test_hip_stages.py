@@ -1455,19 +1455,29 @@ def _check_linear(hip, shape, activation):
 
 @pytest.mark.parametrize("shape", [
     (1, 1, 32, 16), (1, 17, 96, 48), (1, 33, 2080, 80), (2, 64, 512, 1040),
-    (3, 65, 4096, 112), (1, 97, 1056, 2064), (1, 128, 768, 768)],
+    (3, 65, 4096, 112), (1, 97, 1056, 2064), (1, 128, 768, 768),
+    # 32 columns a block: one to eight tiles of rows, the last columns a half
+    # block; the longest reduction with eight tiles (LDS holds 8 wavefronts' sums)
+    (1, 1, 64, 8192), (3, 30, 480, 2736), (1, 40, 4128, 4112), (5, 64, 1024, 1616),
+    (7, 96, 352, 1040), (1, 97, 1088, 8176), (1, 128, 8192, 4112),
+    # more blocks of 32 columns than compute units, K % 64 != 0
+    (1, 50, 96, 16000), (30, 64, 160, 400),
+    # neither kernel's any more: too many columns for the rows
+    (1, 65, 192, 10240), (1, 128, 256, 16000), (60, 100, 128, 256)],
     ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("activation", ["linear", "relu"])
 def test_linear_of_few_rows_and_columns(hip, shape, activation):
   """Few rows, and fewer column tiles than compute units: the reduction is cut
   over the wavefronts of a block.  One to eight tiles of 16 rows; reductions of
-  1 to 130 steps over 2 to 16 wavefronts; columns inside a block's 16 or 32."""
+  1 to 256 steps over 2 to 16 wavefronts; columns inside a block's 16 or 32."""
   _check_linear(hip, shape, activation)
 
 
 @pytest.mark.parametrize("shape", [
     (130, 1, 64, 72), (64, 32, 192, 256), (43, 33, 320, 400), (128, 64, 1024, 128),
-    (16, 5, 128, 1032), (160, 20, 4096, 256), (160, 64, 4160, 256)],
+    (16, 5, 128, 1032), (160, 20, 4096, 256), (160, 64, 4160, 256),
+    # fewer than 128 column tiles, more than 256 blocks of 32 columns
+    (1, 64, 1024, 10248), (9, 17, 320, 936), (33, 48, 64, 256)],
     ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("activation", ["linear", "relu"])
 def test_linear_of_few_rows_many_experts(hip, shape, activation):
