@@ -1520,7 +1520,9 @@ def test_dispatched_ffn_of_few_rows(hip, case, activation):
 
 @pytest.mark.parametrize("shape", [
     (3, 640, 128, 4096), (32, 640, 512, 1024), (5, 705, 192, 768), (1, 129, 64, 256),
-    (2, 320, 1088, 264), (1, 2000, 256, 776), (1, 5000, 128, 1280), (7, 257, 64, 520)],
+    (2, 320, 1088, 264), (1, 2000, 256, 776), (1, 5000, 128, 1280), (7, 257, 64, 520),
+    # tiles that are no multiple of the 8 XCDs, in one round and in two
+    (42, 384, 1024, 512), (43, 400, 320, 512)],
     ids=lambda s: "x".join(map(str, s)))
 def test_linear_row_tiles(hip, shape):
   """Row counts that are spread over row tiles of 32 to 256 rows, the pieces of
