@@ -2295,6 +2295,23 @@ static bool ring_shape(int R, int N, int K) {
   return N >= 256 && R >= 128 && K % 64 == 0 && N % 8 == 0 &&
          (int64_t)N * K < (1LL << 31);
 }
+// Products for which the 128 x 128 tiles are faster than the ring's 256 columns
+// (same bits):
+// short reductions in at most two blocks per compute unit (the ring's first loads,
+// its hand-over and its epilogue through LDS take longer than the K loop: 30
+// experts, 384 x 512, K = 64: 7.0 against 8.7 us; 320 x 2048, K = 128: 5.6, 6.9;
+// from three blocks on the ring wins: 30 x 640 x 512, K = 128: 12.1, 10.6), and
+// one row tile per expert in a few blocks per compute unit, where a ring tile of
+// 128 rows has no second row tile to share its weights with (64 experts, 128 x
+// 1024: K = 256 14.8 against 17.2 us, K = 1024 33.9, 38.5; 256 experts, 128 x 512,
+// K = 512 38.5, 42.9; 64 experts, 128 x 4096, K = 1024 148, 137).
+static bool small_tiles_apply(int E, int R, int N, int K) {
+  const int64_t tiles =
+      (int64_t)E * ((R + 127) / 128) * ((N + 127) / 128);
+  const int cus = compute_units();
+  if (R <= 128 && tiles > cus) return tiles <= 2 * cus || K <= 512;
+  return (K <= 128 && tiles <= 2 * cus) || (K <= 256 && tiles <= cus);
+}
 // The calls that fold the dispatch into their first GEMM decline row counts
 // whose whole 256-row tiles would be more than a fifth padding.
 static bool ring_path_applies(int R, int N, int K) {
@@ -2330,6 +2347,8 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
     const bool mfma_ok =
         (K % 8 == 0) && (N % 8 == 0) &&
         (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0);
+    const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
+                       !relu && ((uintptr_t)relu_mask_src % 16) == 0;
     if (!mfma_ok)
       rc = launch_simple<bf16_t>((const bf16_t*)A, (const bf16_t*)B,
                                  (bf16_t*)C, E, R, N, K, relu, st);
@@ -2339,17 +2358,16 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
     else if (skinny_applies(E, R, N, K))
       rc = launch_skinny((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
                          N, K, relu, st);
-    else if (ring_shape(R, N, K) && (int64_t)R * K < (1LL << 31)) {
+    else if (ring_shape(R, N, K) && (int64_t)R * K < (1LL << 31) &&
+             (masks || !small_tiles_apply(E, R, N, K))) {
       // 256-column tiles in persistent blocks of 8 wavefronts (two per SIMD),
       // the loads spread over the MFMA steps
-      const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
-                         !relu && ((uintptr_t)relu_mask_src % 16) == 0;
       rc = launch_ring((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R, N,
                        K, relu, st, nullptr, nullptr,
                        masks ? (const bf16_t*)relu_mask_src : nullptr, nullptr,
                        masks ? mask_scale : 1.0f);
       if (masks) *mask_applied = rc == 0;
-    } else if (R >= 1024 && N >= 1024)
+    } else if (R >= 1024 && N >= 1024 && !small_tiles_apply(E, R, N, K))
       rc = launch_mfma<256, 256, 64>((const bf16_t*)A, (const bf16_t*)B,
                                      (bf16_t*)C, E, R, N, K, relu, st);
     else

@@ -1522,12 +1522,16 @@ def test_dispatched_ffn_of_few_rows(hip, case, activation):
     (3, 640, 128, 4096), (32, 640, 512, 1024), (5, 705, 192, 768), (1, 129, 64, 256),
     (2, 320, 1088, 264), (1, 2000, 256, 776), (1, 5000, 128, 1280), (7, 257, 64, 520),
     # tiles that are no multiple of the 8 XCDs, in one round and in two
-    (42, 384, 1024, 512), (43, 400, 320, 512)],
+    (42, 384, 1024, 512), (43, 400, 320, 512),
+    # 128 x 128 tiles for short reductions and single row tiles, either side
+    (30, 384, 64, 512), (30, 640, 128, 512), (1, 1100, 256, 1032), (1, 4096, 256, 1024),
+    (64, 128, 1024, 1024), (130, 128, 576, 520)],
     ids=lambda s: "x".join(map(str, s)))
 def test_linear_row_tiles(hip, shape):
   """Row counts that are spread over row tiles of 32 to 256 rows, the pieces of
   a tile dealt out between its two halves: plain, with ReLU, and with the ReLU
-  mask of a gradient on the stores."""
+  mask of a gradient on the stores.  (The masked product always takes these
+  tiles; where the plain one takes 128 x 128 tiles its bits are the same.)"""
   for activation in ("linear", "relu"):
     _check_linear(hip, shape, activation)
   e, rows, k, n = shape
