@@ -313,9 +313,9 @@ size_t mesh_moe_dispatched_expert_ffn_workspace_bytes(int G, int E, int C,
  * kept choices whose gate rounds to 0 read a zero row).  Same h and y as the
  * two calls.  For callers that do not need expert_in afterwards (inference;
  * the backward reads it).  bf16 only, and only where the first GEMM
- * ([G*C, M] x [M, H] per expert) fits the 256 x 256 direct-to-LDS kernel or the
- * one for at most 64 rows per expert; otherwise MESH_MOE_E_UNSUPPORTED with
- * nothing launched: make the two calls.  With at most 64 rows per expert, an
+ * ([G*C, M] x [M, H] per expert) fits the 256 x 256 direct-to-LDS kernel or, for
+ * at most 512 tokens, the one for at most 64 rows per expert; otherwise
+ * MESH_MOE_E_UNSUPPORTED with nothing launched: make the two calls.  With at most 64 rows per expert, an
  * expert without an occupied slot is left out (its weights are not read) and
  * its rows of h and y hold unspecified values.
  *   x [G,S,M] dtype; idx, pos, gate, kept as written by the gating calls

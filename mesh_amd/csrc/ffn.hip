@@ -2484,8 +2484,15 @@ __global__ void slot_map_kernel(const int32_t* __restrict__ idx,
   map[(int64_t)idx[i] * rows_per_expert + g * C + pos[i]] = (int32_t)t;
 }
 
-// The same map in one launch for few rows per expert (at most STREAM_ROWS): a
-// block per expert looks through the record for its slots.
+// The same map in one launch for few rows per expert (at most STREAM_ROWS) and at
+// most MAP_SCAN_TOKENS tokens: a block per expert looks through the whole record
+// for its slots, 128 tokens a round.  From about 512 tokens on that takes longer
+// than the launch it saves, and with the map in two launches the call takes longer
+// than a dispatch and the two products (64 experts of 256 -> 512 -> 256: 256 tokens
+// 15.1 us, two launches 16.1, dispatch 14.0 to 16; 2048 tokens 28, 21, 19; 16384
+// tokens 64, 21, 21.  64 experts of 1024 -> 4096 -> 1024, 1024 tokens: two launches
+// 219, dispatch 213).
+constexpr int MAP_SCAN_TOKENS = 512;
 __global__ __launch_bounds__(256) void slot_map_rows_kernel(
     const int32_t* __restrict__ idx, const int32_t* __restrict__ pos,
     const float* __restrict__ gate, const uint8_t* __restrict__ kept,
@@ -2669,7 +2676,7 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
               activation);
   const int64_t rows = (int64_t)G * C;
   const bool few_rows =
-      rows <= STREAM_ROWS && (int64_t)G * S < (1 << 30) &&
+      rows <= STREAM_ROWS && (int64_t)G * S <= MAP_SCAN_TOKENS &&
       stream_applies(E, (int)rows, H, M) && many_column_tiles(E, H) &&
       ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
   MOE_REQUIRE(dtype == MESH_MOE_BF16 && rows <= 0x7fffffffLL &&

@@ -845,7 +845,9 @@ def dispatched_expert_ffn(x, r, wi_packed, wo_packed, activation="relu",
   """dispatch + expert_ffn without materialising expert_in: x [G, S, M], the
   Routing r -> y [E, G*C, N], or None where the library has no such kernel for
   the case (the caller then makes the two calls).  h [E, G*C, H], if given,
-  receives the hidden tensor."""
+  receives the hidden tensor.  With at most 64 rows per expert the rows of y and
+  h of an expert that no token goes to are unspecified (combine reads none of
+  them)."""
   lib = load_library()
   if activation not in ACTIVATIONS:
     raise ValueError("unsupported expert activation %r" % (activation,))

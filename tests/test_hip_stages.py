@@ -1518,6 +1518,25 @@ def test_dispatched_ffn_of_few_rows(hip, case, activation):
   assert torch.equal(out, hip.combine(want.reshape(e, g, c, m), r, s))
 
 
+@pytest.mark.parametrize("tokens", [512, 513])
+def test_dispatched_ffn_of_few_rows_and_many_tokens(hip, tokens):
+  """The map is made by a walk over all tokens for every expert: above 512 tokens
+  the call is declined."""
+  e, c, m, h = 64, 16, 64, 256
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(tokens)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  r = hip.top2_gating(mk(1, tokens, e), c)
+  x = mk(1, tokens, m).to(torch.bfloat16)
+  wi, wo = mk(e, h, m).to(torch.bfloat16), mk(e, m, h).to(torch.bfloat16)
+  y = hip.dispatched_expert_ffn(x, r, wi, wo, "relu")
+  assert (y is not None) == (tokens <= 512)
+  if y is not None:
+    want = hip.expert_ffn(hip.dispatch(x, r).reshape(e, c, m), wi, wo, "relu")
+    assert torch.equal(hip.combine(y.reshape(e, 1, c, m), r, tokens),
+                       hip.combine(want.reshape(e, 1, c, m), r, tokens))
+
+
 @pytest.mark.parametrize("shape", [
     (3, 640, 128, 4096), (32, 640, 512, 1024), (5, 705, 192, 768), (1, 129, 64, 256),
     (2, 320, 1088, 264), (1, 2000, 256, 776), (1, 5000, 128, 1280), (7, 257, 64, 520),
