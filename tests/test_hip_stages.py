@@ -1477,7 +1477,9 @@ def test_linear_of_few_rows_and_columns(hip, shape, activation):
     (130, 1, 64, 72), (64, 32, 192, 256), (43, 33, 320, 400), (128, 64, 1024, 128),
     (16, 5, 128, 1032), (160, 20, 4096, 256), (160, 64, 4160, 256),
     # fewer than 128 column tiles, more than 256 blocks of 32 columns
-    (1, 64, 1024, 10248), (9, 17, 320, 936), (33, 48, 64, 256)],
+    (1, 64, 1024, 10248), (9, 17, 320, 936), (33, 48, 64, 256),
+    # more blocks than compute units: 48 rows, 49, longer reductions, more columns
+    (130, 48, 512, 264), (130, 49, 512, 264), (130, 49, 576, 264), (33, 64, 64, 1032)],
     ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("activation", ["linear", "relu"])
 def test_linear_of_few_rows_many_experts(hip, shape, activation):
