@@ -667,42 +667,55 @@ __device__ __forceinline__ void gate_select_acc_tile(
 }
 
 // ---------------------------------------------------------------------------
-// Step 1 from logits in memory.  A block has SELECT_TOKENS tokens and sixteen
-// lanes per token; lane l does the exponentials and comparisons of experts l,
-// l + 16, ...  The two sums over a token's experts that decide its gates still
-// run in expert order, read back from LDS (every lane of the token runs the
-// same chain), and a tie between two lanes' candidates goes to the lower
-// expert: the per-token results do not depend on the split.  One thread per
-// token walking its row was a chain of four passes of E dependent steps, and
-// 256 tokens per block left most compute units without one: 64 tokens of 64
-// experts 17.6 -> 8.2 us, 6 groups of 1500 tokens, 16 experts 16.5 -> 6.8 us.
+// Step 1 from logits in memory.  A block of 1024 threads has LANES lanes per token;
+// lane l does the exponentials and comparisons of experts l, l + LANES, ...  The two
+// sums over a token's experts that decide its gates still run in expert order, read
+// back from LDS (every lane of the token runs the same chain), and a tie between two
+// lanes' candidates goes to the lower expert: the per-token results do not depend on
+// the split.  One thread per token walking its row was a chain of four passes of E
+// dependent steps, and 256 tokens per block left most compute units without one:
+// 64 tokens of 64 experts 17.6 -> 8.2 us with sixteen lanes, 6 groups of 1500 tokens,
+// 16 experts 16.5 -> 6.8 us.
+// Launches that fill the chip anyway pay for what the lanes of a token do alike (the
+// chain), the more of it the fewer experts there are.  The whole gating in us, 16 / 8
+// / 4 lanes (one thread per token before): 65536 tokens, 16 experts 28.9, 22.7, 23.5
+// (28), 64 experts 36, 32, 34; 131072 tokens, 16 experts 44, 36, 32; 524288 tokens, 8
+// experts 141, 106, 92 (94), 16 experts 138, 99, 88 (93), 32 experts 150, 127, 129
+// (113), 64 experts 184, 161, 171, 128 experts 310, 280, 271.
 // ---------------------------------------------------------------------------
-constexpr int SELECT_TOKENS = 64;
-constexpr int SELECT_LANES = 16;
-constexpr int SELECT_THREADS = SELECT_TOKENS * SELECT_LANES;
+constexpr int SELECT_THREADS = 1024;
+
+// Tokens per block of step 1 from logits in memory: SELECT_THREADS / LANES.  (The
+// probabilities of 128 tokens lie in LDS twice per compute unit up to 128 experts.)
+static int select_tokens(int G, int S, int E) {
+  const int64_t tokens = (int64_t)G * S;
+  if (tokens < 65536 || E > 128) return 64;
+  return tokens >= 131072 && E <= 24 ? 256 : 128;
+}
 
 __host__ __device__ constexpr int select_row_floats(int E) {
   return (E + 3) / 4 * 4 + 4;            // 16-byte rows, odd in units of 16 bytes
 }                                        // for E = 8 n
 
-template <typename IT>
+template <typename IT, int LANES>
 __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     const float* __restrict__ logits, const IT* __restrict__ importance,
     const float* __restrict__ second_uniform, GateParams p,
     int32_t* __restrict__ idx, int32_t* __restrict__ pos,
     float* __restrict__ gate, uint8_t* __restrict__ kept,
     float* __restrict__ part1, float* __restrict__ part2) {
+  constexpr int TOKENS = SELECT_THREADS / LANES;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int E = p.E, S = p.S;
   const int ld = select_row_floats(E);
-  float* tile = smem;                                  // [SELECT_TOKENS][ld]
-  float* isone = tile + SELECT_TOKENS * ld;            // [SELECT_TOKENS]
-  float* cols = isone + SELECT_TOKENS;                 // [SELECT_THREADS]
+  float* tile = smem;                                  // [TOKENS][ld]
+  float* isone = tile + TOKENS * ld;            // [TOKENS]
+  float* cols = isone + TOKENS;                 // [SELECT_THREADS]
   const int g = blockIdx.y, blk = blockIdx.x;
-  const int t0 = blk * SELECT_TOKENS;
-  const int ntok = min(SELECT_TOKENS, S - t0);
-  const int tid = threadIdx.x, lane = tid % SELECT_LANES;
-  const int tok = tid / SELECT_LANES;
+  const int t0 = blk * TOKENS;
+  const int ntok = min(TOKENS, S - t0);
+  const int tid = threadIdx.x, lane = tid % LANES;
+  const int tok = tid / LANES;
   const bool live = tok < ntok;
   // experts this lane walks: none for a token that does not exist
   const int e_end = live ? E : 0;
@@ -712,11 +725,11 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   const bool sw = p.router == ROUTER_SWITCH;
 
   float m = -INFINITY;
-  for (int e = lane; e < e_end; e += SELECT_LANES) m = fmaxf(m, src[e]);
+  for (int e = lane; e < e_end; e += LANES) m = fmaxf(m, src[e]);
 #pragma unroll
-  for (int d = 1; d < SELECT_LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+  for (int d = 1; d < LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
   const float negm = -m;                                    // reduce_max
-  for (int e = lane; e < e_end; e += SELECT_LANES)
+  for (int e = lane; e < e_end; e += LANES)
     row[e] = expf(src[e] + negm);
   __syncthreads();
   // exp, reduce_sum: in expert order
@@ -733,7 +746,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   // the larger value, of equal ones the lower expert
   auto first_max = [&](float& v, int& i) {
 #pragma unroll
-    for (int d = 1; d < SELECT_LANES; d *= 2) {
+    for (int d = 1; d < LANES; d *= 2) {
       const float v2 = __shfl_xor(v, d);
       const int i2 = __shfl_xor(i, d);
       if (v2 > v || (v2 == v && i2 < i)) { v = v2; i = i2; }
@@ -742,7 +755,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   const float neglse = -(logf(s) + m);                      // log + max
   float g1 = -1.f;
   int i1 = 0;
-  for (int e = lane; e < e_end; e += SELECT_LANES) {
+  for (int e = lane; e < e_end; e += LANES) {
     const float pe = expf(src[e] + neglse);                 // exp(log_softmax)
     row[e] = pe;
     if (pe > g1) { g1 = pe; i1 = e; }                       // first argmax
@@ -761,7 +774,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
       const float* ch = second_uniform + t * E;
       float best = -INFINITY;
       i1 = 0;
-      for (int e = lane; e < e_end; e += SELECT_LANES) {
+      for (int e = lane; e < e_end; e += LANES) {
         const float v = ch[e];
         if (v > best) { best = v; i1 = e; }
       }
@@ -801,7 +814,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     const int masked = sel1 ? i1 : -1;                      // 1 + (-mask_1)
     float g2 = -1.f;
     int i2 = 0;
-    for (int e = lane; e < e_end; e += SELECT_LANES) {
+    for (int e = lane; e < e_end; e += LANES) {
       const float q = row[e] * (e == masked ? 0.0f : 1.0f);
       if (q > g2) { g2 = q; i2 = e; }
     }
@@ -835,14 +848,14 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     }
   }
   // sums over the block's tokens, per expert: part[e] = sum of tile[r][e] *
-  // (weights ? weights[r] : 1); the rows in up to SELECT_LANES ranges, whose
+  // (weights ? weights[r] : 1); the rows in up to 16 ranges, whose
   // sums are added in order
   auto column_sums = [&](const float* weights, float* part) {
     int el = 2;
     while (el < E) el *= 2;
-    const int ranges = min(SELECT_LANES, SELECT_THREADS / el);
+    const int ranges = min(16, SELECT_THREADS / el);
     const int e = tid % el, c = tid / el;
-    const int per = SELECT_TOKENS / ranges;
+    const int per = TOKENS / ranges;
     __syncthreads();
     if (e < E && c < ranges) {
       float a = 0.f;
@@ -867,17 +880,17 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     if (lane == 0) {
       const float lse = -neglse;                            // reduce_logsumexp
       cols[tok] = sel1 ? lse * lse : 0.0f;                  // moe.py:1256-1259
-      cols[SELECT_TOKENS + tok] = sel1 ? 1.0f : 0.0f;
+      cols[TOKENS + tok] = sel1 ? 1.0f : 0.0f;
     }
     __syncthreads();
     if (tid < 2) {
       float a = 0.f;
-      for (int r = 0; r < ntok; ++r) a += cols[tid * SELECT_TOKENS + r];
+      for (int r = 0; r < ntok; ++r) a += cols[tid * TOKENS + r];
       part2[((int64_t)g * p.nblk + blk) * E + tid] = a;
     }
   } else if (p.use_second_place_loss) {
     __syncthreads();
-    for (int e = lane; e < e_end; e += SELECT_LANES)
+    for (int e = lane; e < e_end; e += LANES)
       row[e] = (row[e] * (sel1 && e == i1 ? 0.0f : 1.0f)) * qscale;
     column_sums(nullptr, part2);
   }
@@ -1946,23 +1959,27 @@ static int run_gating(const GateParams& p, const float* logits,
   float* part2 = part1 + (size_t)G * p.nblk * E;
   float* gsum = part2 + (size_t)G * p.nblk * E;
   dim3 grid((unsigned)p.nblk, (unsigned)G);
-  const size_t smem =
-      sizeof(float) * ((size_t)SELECT_TOKENS * select_row_floats(E) +
-                       SELECT_TOKENS + SELECT_THREADS);
-  if (importance && importance_dtype == MESH_MOE_BF16) {
-    auto k = gate_select_kernel<bf16_t>;
+  const size_t smem = sizeof(float) * ((size_t)p.tt * select_row_floats(E) +
+                                       p.tt + SELECT_THREADS);
+  auto run = [&](auto k, auto* imp) -> int {
     MOE_ALLOW_LDS(k, smem);
-    k<<<grid, SELECT_THREADS, smem, st>>>(logits, (const bf16_t*)importance,
-                                second_uniform, p, idx, pos, gate, kept, part1,
-                                part2);
-  } else {
-    auto k = gate_select_kernel<float>;
-    MOE_ALLOW_LDS(k, smem);
-    k<<<grid, SELECT_THREADS, smem, st>>>(logits, (const float*)importance,
-                                second_uniform, p, idx, pos, gate, kept, part1,
-                                part2);
-  }
-  MOE_CHECK_LAUNCH("gate_select");
+    k<<<grid, SELECT_THREADS, smem, st>>>(logits, imp, second_uniform, p, idx,
+                                          pos, gate, kept, part1, part2);
+    MOE_CHECK_LAUNCH("gate_select");
+    return 0;
+  };
+  auto run_lanes = [&](auto* imp) -> int {
+    using IT = std::remove_const_t<std::remove_pointer_t<decltype(imp)>>;
+    switch (p.tt) {
+      case 64: return run(gate_select_kernel<IT, 16>, imp);
+      case 128: return run(gate_select_kernel<IT, 8>, imp);
+      default: return run(gate_select_kernel<IT, 4>, imp);
+    }
+  };
+  const int rc = importance && importance_dtype == MESH_MOE_BF16
+                     ? run_lanes((const bf16_t*)importance)
+                     : run_lanes((const float*)importance);
+  if (rc != 0) return rc;
   return launch_capacity_and_loss(p, idx, pos, gate, kept, fill, loss, part1,
                                   part2, gsum, st);
 }
@@ -2126,7 +2143,7 @@ extern "C" int mesh_moe_top2_gating(
   GateParams p = make_gate_params(G, S, E, C, policy, threshold,
                                   use_second_place_loss, num_microbatches,
                                   importance_from_slot_gate,
-                                  SELECT_TOKENS);
+                                  select_tokens(G, S, E));
   return run_gating(p, logits, importance, importance_dtype, second_uniform,
                     idx, pos, gate, kept, fill, loss, workspace,
                     (hipStream_t)stream);
@@ -2170,7 +2187,7 @@ extern "C" int mesh_moe_switch_gating(
     return rc;
   GateParams p = make_switch_params(G, S, E, C, importance, slots_by_gate,
                                     use_z_loss, z_loss_coef, num_microbatches,
-                                    SELECT_TOKENS);
+                                    select_tokens(G, S, E));
   return run_gating(p, logits, importance, importance_dtype, choice_logits,
                     idx, pos, gate, kept, fill, loss, workspace,
                     (hipStream_t)stream);

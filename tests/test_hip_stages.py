@@ -1435,6 +1435,48 @@ def test_expert_linear_many_row_tiles(hip, shape):
                                atol=1e-2 * float(wnt.abs().max()), err_msg=name)
 
 
+@pytest.mark.parametrize("shape", [(64, 1024, 16), (66, 1001, 128), (9, 16384, 32),
+                                   (130, 1009, 24), (1400, 97, 3), (2048, 64, 10)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("with_importance", [False, True])
+def test_gating_of_many_tokens_equals_its_parts(hip, shape, with_importance):
+  """Sixteen, eight or four lanes select for a token, by the number of tokens and
+  experts: routing, gates and counts are bit for bit those of the groups gated in
+  two calls of half the tokens.  The loss is the mean of theirs with its sums of
+  positive terms in another order: at most 16 terms, 16 ranges, 256 blocks and 2048
+  groups after each other, half a rounding of 2^-23 each."""
+  g, s, e = shape
+  half = 131072 if e <= 24 and g * s >= 131072 else 65536
+  assert g * s >= half > (g - g // 2) * s or e == 32
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(shape))
+  logits = torch.randn((g, s, e), generator=gen, device="cuda")
+  logits[::3, 5] = 1.0                           # ties
+  imp = None
+  if with_importance:
+    imp = torch.tensor([0.0, 0.5, 1.0], device="cuda")[
+        torch.randint(0, 3, (g, s), generator=gen, device="cuda")].to(torch.bfloat16)
+  c = max(1, s // e)
+  parts = [slice(0, g // 2), slice(g // 2, g)]
+  choice = torch.randn((g, s, e), generator=gen, device="cuda")
+  for run in (lambda p: hip.top2_gating(logits[p], c, use_second_place_loss=True,
+                                        importance=None if imp is None else imp[p]),
+              lambda p: hip.switch_gating(logits[p], c, z_loss=1e-3,
+                                          importance=None if imp is None else imp[p]),
+              lambda p: hip.switch_gating(logits[p], c, choice_logits=choice[p])):
+    whole, halves = run(slice(0, g)), [run(p) for p in parts]
+    for name in ("idx", "pos", "kept", "fill"):
+      assert torch.equal(getattr(whole, name),
+                         torch.cat([getattr(h, name) for h in halves])), name
+    gates = torch.cat([h.gate for h in halves])
+    assert torch.equal(whole.gate.view(torch.int32), gates.view(torch.int32))
+    if imp is None:
+      mean = sum(float(h.loss) * (p.stop - p.start)
+                 for h, p in zip(halves, parts)) / g
+      assert abs(float(whole.loss) - mean) <= 2336 * 2.0 ** -24 * mean
+
+
+
 def _check_linear(hip, shape, activation):
   """expert_linear against float32 products.  The bound: one bf16 rounding and
   the float32 sums of K products in another order."""
