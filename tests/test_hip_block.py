@@ -163,8 +163,8 @@ def _packed_sequence_ids(rng, b, l, mean_len):
                          ids=lambda c: "x".join(map(str, c)))
 def test_self_attention_sequence_ids_in_any_order(hip, case, causal, with_bias):
   """Ids that come back later in the row, that are equal modulo 64, negative
-  ones and a single position of its own, in the fused kernels: which tiles of
-  keys or queries are walked must not hang on ids lying in order."""
+  ones and a single position of its own, at lengths of a single tile or that the
+  fused kernels do not take (no multiple of 8: the three-step form)."""
   l, d = case
   b, heads, nb = 3, 1, 8
   rng = np.random.default_rng(l + d + causal)
@@ -190,6 +190,53 @@ def test_self_attention_sequence_ids_in_any_order(hip, case, causal, with_bias):
   np.testing.assert_allclose(got, want, **_tol("bfloat16"))
   grads = hip.self_attention_backward(g(q), g(k), g(v), g(do), heads, causal,
                                       sequence_id=sid, relative_bias=rel)
+  want = B.attention_core_backward(q, k, v, do, heads, causal, "bfloat16",
+                                   sequence_id=ids, relative_values=values)
+  for gt, wnt in zip(grads, want):
+    scale = max(1.0, float(np.abs(wnt).max()))
+    np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
+
+
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("case", [(136, 64), (520, 64), (520, 128), (1000, 64),
+                                  (1000, 128)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_fused_attention_skips_tiles_of_other_sequences(hip, case, causal, with_bias):
+  """The fused kernels walk the tiles between the first and the last row of a
+  block's own sequences.  Rows of one sequence (both ends are the block's own);
+  sequences whose first tile is not tile 0 and whose last is not the last; ids
+  that come back, alias modulo 64 or are negative; single positions at both ends
+  that belong to a block in the middle."""
+  l, d = case
+  b, heads, nb = 5, 1, 8
+  rng = np.random.default_rng(l + d + causal)
+  at = np.arange(l)
+  ids = np.stack([np.full(l, 7), at // 150 + 1,
+                  np.where(at // 100 % 2 == 0, 3, 67),
+                  np.where(at < l // 2, -1, np.where(at < l - 40, 63, 5)),
+                  at // 130]).astype(np.int32)
+  ids[1, -24:] = 0
+  ids[4, 0] = ids[4, -1] = ids[4, l // 2]
+  mk = lambda *sizes: O.cast_act(
+      (rng.standard_normal(sizes) * 0.5).astype(np.float32), "bfloat16")
+  q, k, v, do = (mk(b, l, heads * d) for _ in range(4))
+  g = lambda a: H.to_gpu(a, "bfloat16")
+  assert hip.fused_attention_applies(g(q), heads)
+  values, rel = None, None
+  if with_bias:
+    values = mk(heads, nb)
+    bucket = B.relative_position_bucket(np.arange(-(l - 1), l), not causal, nb)
+    rel = (g(values), torch.from_numpy(bucket.astype(np.int32)).cuda())
+  sid = torch.from_numpy(ids).cuda()
+  got = H.to_np(hip.self_attention(g(q), g(k), g(v), heads, causal,
+                                   sequence_id=sid, relative_bias=rel))
+  want = B._attention_core(q, k, v, heads, causal, "bfloat16", sequence_id=ids,
+                           relative_values=values)
+  np.testing.assert_allclose(got, want, **_tol("bfloat16"))
+  grads = hip.self_attention_backward(g(q), g(k), g(v), g(do), heads, causal,
+                                      fused=True, sequence_id=sid,
+                                      relative_bias=rel)
   want = B.attention_core_backward(q, k, v, do, heads, causal, "bfloat16",
                                    sequence_id=ids, relative_values=values)
   for gt, wnt in zip(grads, want):
