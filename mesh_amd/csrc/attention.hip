@@ -119,18 +119,21 @@ __device__ __forceinline__ float fa_exp2(float x) {
 template <bool CAUSAL>
 __device__ __forceinline__ void fa_block_to_work(int n_tiles, int& tile, int& bh) {
   const int nbh = (int)gridDim.y;
-  const int lanes = nbh % 8 == 0 ? 8 : 1;
+  const int shift = nbh % 8 == 0 ? 3 : 0;          // XCDs, as a power of two
   const int id = (int)blockIdx.x + n_tiles * (int)blockIdx.y;
-  const int slot = id / lanes, heads = nbh / lanes;
-  int size = 1;                                    // heads of a group
-  if (CAUSAL) {
-    const int groups = max(1, (int)((int64_t)heads * n_tiles / (1024 / lanes)));
-    size = (heads + groups - 1) / groups;
+  const int slot = id >> shift, heads = nbh >> shift;
+  // heads of a group; one group where everything is in flight at once
+  int size = CAUSAL ? heads : 1, first = 0, at = slot;
+  const int groups = (heads * n_tiles) >> (10 - shift);
+  if (CAUSAL && groups > 1) size = (heads + groups - 1) / groups;
+  if (!CAUSAL || groups > 1) {
+    const int group = slot / (size * n_tiles);
+    first = group * size;
+    at = slot - first * n_tiles;
   }
-  const int group = slot / (size * n_tiles), at = slot - group * size * n_tiles;
-  const int here = min(size, heads - group * size);
+  const int here = CAUSAL ? min(size, heads - first) : 1;
   tile = at / here;
-  bh = (group * size + at - tile * here) * lanes + id % lanes;
+  bh = ((first + at - tile * here) << shift) + (id & ((1 << shift) - 1));
 }
 
 // Shrinks the streamed tiles [t_begin, t_end) of BT rows to those between the
@@ -142,13 +145,21 @@ __device__ __forceinline__ void fa_block_to_work(int n_tiles, int& tile, int& bh
 // multiplied; a first and a last tile are enough for that, and the loops stay
 // loops over consecutive tiles.  Every wavefront calls it; scratch: the start
 // of the tile ring, free again afterwards.  A row's own id is always found.
+// There is nothing to find in a range of no more tiles than the block's own rows
+// have (own_tiles), nor where both its ends carry one of the ids, as in a row of
+// one sequence (one sequence, searched anyway / now: 8 heads of 64 positions,
+// backward 21.4 / 17.8 us; 64 x 8 heads of 128 positions 55.5 / 49.7; 2 x 16 heads
+// of 512 positions 66.8 / 63.6; without the ids 60).
 // 16 rows of 1000 positions, two sequences and padding in each, 12 heads of 64:
 // forward 98 -> 72 us; dv, dk, dq 99, 152, 211 -> 88, 125, 173 us (with the
 // blocks still head after head, see above).
 template <int WAVES>
 __device__ __forceinline__ void fa_visible_tiles(
-    const int32_t* __restrict__ seq_b, int L, int BT, int my_sid, bool uniform,
-    unsigned char* scratch, int& t_begin, int& t_end) {
+    const int32_t* __restrict__ seq_b, int L, int BT, int own_tiles, int my_sid,
+    bool uniform, unsigned char* scratch, int& t_begin, int& t_end) {
+  if (t_end - t_begin <= own_tiles) return;
+  const int end = min(t_end * BT, L);
+  const int first_sid = seq_b[t_begin * BT], last_sid = seq_b[end - 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   unsigned long long* masks = reinterpret_cast<unsigned long long*>(scratch);
   int* firsts = reinterpret_cast<int*>(masks + WAVES);
@@ -161,8 +172,11 @@ __device__ __forceinline__ void fa_visible_tiles(
   __syncthreads();
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) own |= masks[w];
+  if ((own >> (first_sid & 63)) & (own >> (last_sid & 63)) & 1) {
+    __syncthreads();
+    return;
+  }
   int first = L, last = -1;
-  const int end = min(t_end * BT, L);
 #pragma unroll 4
   for (int i = t_begin * BT + tid; i < end; i += WAVES * 64)
     if ((own >> (seq_b[i] & 63)) & 1) {
@@ -242,8 +256,8 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
     own_uniform = __ballot(my_sid != own_first) == 0ull;
   }
   if constexpr (SEQ)
-    fa_visible_tiles<Cfg::WAVES>(seq_b, L, Cfg::BK, my_sid, own_uniform, fa_smem,
-                                 kt_begin, n_ktiles);
+    fa_visible_tiles<Cfg::WAVES>(seq_b, L, Cfg::BK, Cfg::BQ / Cfg::BK, my_sid,
+                                 own_uniform, fa_smem, kt_begin, n_ktiles);
   // key ids of the two tile stages, behind the K / V ring; then the two
   // stages' windows of the bias table (192 floats each)
   int32_t* sid_s = reinterpret_cast<int32_t*>(fa_smem + Cfg::LDS_BYTES);
@@ -324,8 +338,9 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
   __syncthreads();
 
   const int qw_first = q0 + wave * 32;
-  for (int kt = kt_begin; kt < n_ktiles; ++kt) {
-    const int buf = (kt - kt_begin) & 1;
+  const int kt_count = n_ktiles - kt_begin;
+  for (int it = 0; it < kt_count; ++it) {
+    const int kt = kt_begin + it, buf = it & 1;
     if (kt + 1 < n_ktiles) load_tile(kt + 1, buf ^ 1);
     const int key0 = kt * Cfg::BK;
     // (a wavefront whose queries all precede this tile still runs it: every
@@ -752,8 +767,8 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     my_sid = seq_b[my_c];
     own_first = __builtin_amdgcn_readfirstlane(my_sid);
     own_uniform = __ballot(my_sid != own_first) == 0ull;
-    fa_visible_tiles<Cfg::WAVES>(seq_b, L, Cfg::BT, my_sid, own_uniform, fb_smem,
-                                 t_begin, t_end);
+    fa_visible_tiles<Cfg::WAVES>(seq_b, L, Cfg::BT, Cfg::BOWN / Cfg::BT, my_sid,
+                                 own_uniform, fb_smem, t_begin, t_end);
   }
 
   // one tile copy: rows of `src` from row0, chunk-swizzled for row reads
