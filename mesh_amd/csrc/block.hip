@@ -1349,8 +1349,15 @@ static int run_attention_decode(const void* q, const void* k_new,
                     (uintptr_t)v_new | (uintptr_t)k_out | (uintptr_t)v_out) %
                    16) == 0;
   const bool copy = k_out != k_cache || v_out != v_cache;
-  // few blocks: four times the threads, i.e. the loads in flight, per block
-  const bool wide = vec && (int64_t)H * B <= 512 && Lm >= 512 &&
+  // few blocks: four times the threads, i.e. the loads in flight, per block.  In
+  // place only the rows up to the position are read: with two blocks per compute
+  // unit the smaller blocks are the faster ones up to 2048 rows (32 x 16 heads of
+  // 64, 512 rows, position 3, 128, 511: 6.3, 9.0, 19.5 us against 9.9, 13.0, 16.8);
+  // with one, sixteen wavefronts lose little early and gain more later (32 x 8
+  // heads of 128, 1024 rows, position 3, 256, 1023: 7.4, 11.6, 27 against 6.0,
+  // 18.4, 55).
+  const bool wide = vec && (int64_t)H * B <= 512 &&
+                    Lm >= (copy || (int64_t)H * B <= 256 ? 512 : 2048) &&
                     ((size_t)Lm + D + 16 + 8 * 1024) * sizeof(float) <= 150 * 1024;
   const int nt = wide ? 1024 : 256;
   const size_t floats =
