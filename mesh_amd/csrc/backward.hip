@@ -1292,14 +1292,20 @@ __global__ void router_wgrad_reduce_kernel(const float* __restrict__ part,
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float sum = 0.f;
-  for (int c = 0; c < chunks; c += 16) {     // sixteen loads in flight
-    float v[16];
+  int c = 0;
+  auto add = [&](auto loads_c) {               // that many loads in flight
+    constexpr int LOADS = decltype(loads_c)::value;
+    for (; c + LOADS <= chunks; c += LOADS) {
+      float v[LOADS];
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      v[u] = c + u < chunks ? part[(int64_t)(c + u) * n + i] : 0.f;
+      for (int u = 0; u < LOADS; ++u) v[u] = part[(int64_t)(c + u) * n + i];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) sum += v[u];
-  }
+      for (int u = 0; u < LOADS; ++u) sum += v[u];
+    }
+  };
+  add(std::integral_constant<int, 16>());
+  add(std::integral_constant<int, 4>());
+  add(std::integral_constant<int, 1>());
   store_f32<T>(dw + i, sum);
 }
 
