@@ -1688,7 +1688,11 @@ static int launch_gating_backward(
   MOE_CHECK_LAUNCH("gating_backward (count)");
   const int E = p.E;
   const int64_t T_tokens = (int64_t)p.G * p.S;
-  if (E % 4 == 0 && E <= 128 && bw_aligned16(logits) && bw_aligned16(dlogits)) {
+  // (four experts are one lane's: three of a token's four lanes idle, which costs
+  // more than it saves in large launches: 65536 tokens 8.9 us, one thread per token
+  // 11.0; 524288 tokens 28, 20)
+  if (E % 4 == 0 && E <= 128 && (E > 4 || T_tokens <= 131072) &&
+      bw_aligned16(logits) && bw_aligned16(dlogits)) {
     const int chunk = (E / 4 + 3) / 4 * 4;
     const unsigned blocks = (unsigned)((T_tokens + 63) / 64);
     auto run = [&](auto k) {

@@ -451,6 +451,24 @@ def test_backward_expert_counts(hip, case):
   test_backward_matches_oracle(hip, case)
 
 
+def test_gating_backward_of_four_experts(hip):
+  """Four experts in a large launch (one thread per token) against its halves (four
+  lanes per token).  The gradient of the gates alone: sums over four experts, in
+  orders that differ; each has at most ten roundings of 2^-24."""
+  g, s, e = 1030, 128, 4
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(4)
+  logits = torch.randn((g, s, e), generator=gen, device="cuda")
+  dgate = torch.randn((g, s, 2), generator=gen, device="cuda")
+  dl = torch.zeros(1, device="cuda")
+  run = lambda p: hip.gating_backward(logits[p], hip.top2_gating(logits[p], 40),
+                                      dgate[p], dl, 1.0)
+  whole = run(slice(0, g))
+  halves = torch.cat([run(slice(0, 500)), run(slice(500, g))])
+  assert bool(whole.any())
+  assert float((whole - halves).abs().max()) <= 20 * 2.0 ** -24 * float(dgate.abs().max()) * 4
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(63, 8, 4), (9001, 72, 12), (65, 1984, 68),
                                    (4097, 136, 128)])
