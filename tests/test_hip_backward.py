@@ -451,6 +451,12 @@ def test_backward_expert_counts(hip, case):
   test_backward_matches_oracle(hip, case)
 
 
+@pytest.mark.parametrize("router", ["top_2", "switch"])
+def test_backward_of_long_groups(hip, router):
+  """Groups whose choices are counted by several blocks."""
+  test_backward_matches_oracle(hip, (router, 2, 5000, 16, 24, 8, 0.1, "float32", True))
+
+
 def test_gating_backward_of_four_experts(hip):
   """Four experts in a large launch (one thread per token) against its halves (four
   lanes per token).  The gradient of the gates alone: sums over four experts, in
