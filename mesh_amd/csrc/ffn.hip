@@ -800,7 +800,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     }
     row0 = tile_row0(tm);
     col0 = tn * BN;
-    if constexpr (KMAJOR) {
+    if constexpr (KMAJOR && !SPLIT) {
       if (k_extent != nullptr) {
         const int used = k_extent[e];
         tile_empty = used == 0;
@@ -808,10 +808,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       }
     }
     if constexpr (SPLIT) {
-      if (KMAJOR && k_extent == nullptr) nk = (K + BK - 1) / BK;
-      if constexpr (KMAJOR) {
-        if (k_extent == nullptr) tile_empty = false;
-      }
+      nk = (K + BK - 1) / BK;
+      tile_empty = false;
       kt0 = 0;
       if (unit >= 0) {
         const int all = nk;
@@ -2081,7 +2079,8 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
   return (unsigned)(((tiles < cus ? tiles : cus) + 7) / 8 * 8);
 }
 
-// scratch: kmajor_split_plan(...).bytes for the parts (null: nothing is split)
+// scratch: kmajor_split_plan(...).bytes for the parts (null: nothing is split;
+// with k_extent nothing is)
 static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
                               int E, int R, int N, int K, hipStream_t st,
                               const int32_t* k_extent = nullptr,
@@ -2096,7 +2095,8 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
   if (cus == 0) return MESH_MOE_E_HIP;
   const unsigned blocks = ring_blocks(tiles, cus);
   const SplitPlan plan =
-      scratch == nullptr ? SplitPlan() : kmajor_split_plan(E, R, N, K);
+      scratch == nullptr || k_extent != nullptr ? SplitPlan()
+                                                : kmajor_split_plan(E, R, N, K);
   if (plan.split > 1) {
     const int tail = (int)tiles - plan.whole_tiles;
     const int units = plan.whole_tiles + tail * plan.split;
@@ -2106,7 +2106,7 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<split_blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, units, nullptr, nullptr, nullptr,
-        nullptr, k_extent, 1.0f, (float*)scratch, plan.whole_tiles, plan.split,
+        nullptr, nullptr, 1.0f, (float*)scratch, plan.whole_tiles, plan.split,
         Cfg::BM);
     MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands, split)");
     split_reduce_kernel<<<(unsigned)tail * Cfg::TM * Cfg::TN, Cfg::THREADS, 0,
