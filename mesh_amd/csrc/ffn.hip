@@ -2319,7 +2319,8 @@ static bool small_tiles_apply(int E, int R, int N, int K) {
   return (K <= 128 && tiles <= 2 * cus) || (K <= 256 && tiles <= cus);
 }
 // The calls that fold the dispatch into their first GEMM decline row counts
-// whose whole 256-row tiles would be more than a fifth padding.
+// whose whole 256-row tiles would be more than a fifth padding.  (The line was drawn
+// for tiles of 256 rows; it has not been measured with lower ones.)
 static bool ring_path_applies(int R, int N, int K) {
   const int pad256 = (R + 255) / 256 * 256, pad128 = (R + 127) / 128 * 128;
   return ring_shape(R, N, K) && pad128 * 5 >= pad256 * 4;

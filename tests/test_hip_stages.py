@@ -1186,8 +1186,8 @@ def test_dispatched_expert_ffn_equals_two_calls(hip, shape):
   got = hip.dispatched_expert_ffn(x, r, wi_p, wo_p, "relu")
   assert got is not None
   assert torch.equal(got, want)
-  # float32, and row counts that 128-row tiles serve better (320 rows here):
-  # the library declines and the caller makes the two calls
+  # float32, and row counts whose whole 256-row tiles would be more than a fifth
+  # padding: the library declines and the caller makes the two calls
   assert hip.dispatched_expert_ffn(x.float(), r, wi_p.float(), wo_p.float(),
                                    "relu") is None
   if g * c == 256:
