@@ -5,8 +5,8 @@
 //
 // Both GEMMs are "TN": A [R, K] and the packed weight B [N, K] are
 // K-contiguous, C [R, N] = A . B^T.  The bf16 kernel uses
-// v_mfma_f32_32x32x16_bf16 with LDS double buffering; float32 and odd shapes
-// use a plain FMA tile kernel.
+// v_mfma_f32_32x32x16_bf16 with LDS double buffering; float32 has its own file
+// (gemm_f32.hip), odd shapes use a plain FMA tile kernel.
 #include <type_traits>
 
 #include "common.h"
@@ -1306,256 +1306,6 @@ __global__ __launch_bounds__(RingCfg::THREADS) void split_reduce_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// float32 on the matrix cores: v_mfma_f32_32x32x2_f32, true float32 operands
-// and accumulation (the float32 configuration of the layer: no narrowing).
-// Four wavefronts; K step 32.  As in the bf16 kernels the weight tile is the
-// MFMA's first operand, so a lane ends up with 4 consecutive output columns
-// per register group.  One MFMA consumes k = 2 s + (lane / 32) for step s; a
-// lane instead takes the four consecutive k = 8 u + 4 (lane / 32) + j for steps
-// 4 u + j (both operands agree on the order, and a sum does not care), which
-// makes its operand reads 16 bytes wide.  Tiles are staged through registers
-// into LDS rows of 32 + 4 floats.  K % 4 == 0 and N % 4 == 0.
-//
-// KMAJOR: the reduction index is the outermost one of both operands (weight
-// gradients: A [K][R], B [K][N], token rows summed over).  They are staged as
-// they lie, [32][tile + 8], and a lane's four k are four reads of 4 bytes; the
-// rows a half-wavefront apart are 4 (tile + 8) = 32 (mod 64) banks apart, so
-// the reads do not meet.  R % 4 == 0 and N % 4 == 0, any K.
-//
-// Bound by the matrix pipes, of whose 64 cycles an MFMA the loop keeps 60 to 75
-// % busy: a step's LDS writes, barrier and first operand reads stand beside its
-// MFMAs unless another block of the compute unit fills in.  Three (128 x 128
-// tiles: two) K tiles are on their way in registers, and the barrier does not
-// wait for them.  Blocks are renumbered so that an XCD works on a contiguous
-// range of tiles, which share weight panels.
-// 8 experts x 320 rows, 5.4 GFLOP a product (34 us at the peak): 512 -> 2048 68
-// -> 62 us; 2048 -> 512 87 -> 67; weight gradients, as they lie instead of
-// through transposed copies, 76 -> 57.
-// ---------------------------------------------------------------------------
-// TM x TN: MFMA tiles per wavefront.  WM x WN x WK: the wavefronts' grid; the
-// WK wavefronts of a sub-tile share out the k of every staged tile and add up
-// their sums in the end, so a small tile keeps all four matrix pipes busy.
-template <int TM, int TN, int WM, int WN, int WK, bool KMAJOR>
-struct F32Cfg {
-  static_assert(WM * WN * WK == 4, "four wavefronts");
-  static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, BK = 32,
-                       THREADS = 256;
-  // floats per LDS row and per stage of an operand
-  static constexpr int LDA = KMAJOR ? BM + 8 : BK + 4;
-  static constexpr int LDB = KMAJOR ? BN + 8 : BK + 4;
-  static constexpr int STAGE_A = (KMAJOR ? BK : BM) * LDA;
-  static constexpr int STAGE_B = (KMAJOR ? BK : BN) * LDB;
-  // 16-byte chunks per staged row
-  static constexpr int CPR_A = (KMAJOR ? BM : BK) / 4;
-  static constexpr int CPR_B = (KMAJOR ? BN : BK) / 4;
-  // K tiles loaded ahead
-  static constexpr int PF = BM * BN >= 128 * 128 ? 2 : 3;
-  static constexpr int A_CHUNKS = BM * BK / 4 / THREADS;
-  static constexpr int B_CHUNKS = BN * BK / 4 / THREADS;
-  static constexpr size_t LDS_BYTES =
-      2ull * (STAGE_A + STAGE_B) * sizeof(float);
-  static_assert(LDS_BYTES >= (WK - 1) * WM * WN * TM * TN * 1024 * sizeof(float),
-                "the partial sums of the other wavefronts fit");
-};
-
-// mask_src (shape of C): elements whose mask_src element is not positive become
-// 0, the others are multiplied by mask_scale.
-template <int TM, int TN, int WM, int WN, int WK, bool KMAJOR>
-__global__ __launch_bounds__(256) void grouped_gemm_f32_mfma_kernel(
-    const float* __restrict__ A, const float* __restrict__ B,
-    float* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
-    int relu, const float* __restrict__ mask_src, float mask_scale) {
-  using Cfg = F32Cfg<TM, TN, WM, WN, WK, KMAJOR>;
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
-  constexpr int LDA = Cfg::LDA, LDB = Cfg::LDB, PF = Cfg::PF;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  float* As = reinterpret_cast<float*>(smem_raw);  // [2][STAGE_A]
-  float* Bs = As + 2 * Cfg::STAGE_A;               // [2][STAGE_B]
-  const int nblk = gridDim.x;
-  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-  const int logical = xcd * (nblk >> 3) + min(xcd, nblk & 7) + local;
-  const int tiles_per_e = tiles_m * tiles_n;
-  const int e = logical / tiles_per_e;
-  const int rem = logical - e * tiles_per_e;
-  const int tn = rem / tiles_m, tm = rem - tn * tiles_m;
-  const int row0 = tm * BM, col0 = tn * BN;
-  const float* Ae = A + (int64_t)e * R * K;
-  const float* Be = B + (int64_t)e * N * K;
-  float* Ce = Cout + (int64_t)e * R * N;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wk = wave / (WM * WN), wmn = wave % (WM * WN);
-  const int wm = wmn / WN, wn = wmn % WN;
-
-  // PF K tiles are on their way in registers beside the one in LDS.  Chunk c of
-  // an operand tile whose first row (KMAJOR: column) is `first` of `rows`;
-  // addresses are clamped into the operand, what lies past the end of k becomes
-  // 0 on its way into LDS.
-  uint4 areg[PF][Cfg::A_CHUNKS], breg[PF][Cfg::B_CHUNKS];
-  auto load_chunk = [&](const float* src, int c, int cpr, int first, int rows,
-                        int k0) {
-    const int r = c / cpr, off = (c % cpr) * 4;
-    const float* p =
-        KMAJOR ? src + (int64_t)min(k0 + r, K - 1) * rows +
-                     min(first + off, rows - 4)
-               : src + (int64_t)min(first + r, rows - 1) * K +
-                     min(k0 + off, K - 4);
-    return *reinterpret_cast<const uint4*>(p);
-  };
-  auto load_global = [&](int k0, auto slot_c) {
-    constexpr int SLOT = decltype(slot_c)::value;
-#pragma unroll
-    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
-      areg[SLOT][i] =
-          load_chunk(Ae, tid + i * Cfg::THREADS, Cfg::CPR_A, row0, R, k0);
-#pragma unroll
-    for (int i = 0; i < Cfg::B_CHUNKS; ++i)
-      breg[SLOT][i] =
-          load_chunk(Be, tid + i * Cfg::THREADS, Cfg::CPR_B, col0, N, k0);
-  };
-  auto store_chunk = [&](float* dst, int c, int cpr, int ld, uint4 v, int k0) {
-    const int r = c / cpr, off = (c % cpr) * 4;
-    if (k0 + BK > K && k0 + (KMAJOR ? r : off) >= K) v = make_uint4(0, 0, 0, 0);
-    *reinterpret_cast<uint4*>(dst + r * ld + off) = v;
-  };
-  auto store_lds = [&](int buf, int k0, auto slot_c) {
-    constexpr int SLOT = decltype(slot_c)::value;
-#pragma unroll
-    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
-      store_chunk(As + buf * Cfg::STAGE_A, tid + i * Cfg::THREADS, Cfg::CPR_A,
-                  LDA, areg[SLOT][i], k0);
-#pragma unroll
-    for (int i = 0; i < Cfg::B_CHUNKS; ++i)
-      store_chunk(Bs + buf * Cfg::STAGE_B, tid + i * Cfg::THREADS, Cfg::CPR_B,
-                  LDB, breg[SLOT][i], k0);
-  };
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nk = (K + BK - 1) / BK;
-  // where this lane's operands start: a row and four k, of its wavefront's k
-  constexpr int US = BK / 8 / WK;                  // groups of 8 k a wavefront
-  const int frag_row = lane & 31, frag_k = (lane >> 5) * 4 + wk * US * 8;
-  const int a_row = wm * 32 * TM + frag_row, b_row = wn * 32 * TN + frag_row;
-  const int a_at = KMAJOR ? frag_k * LDA + a_row : a_row * LDA + frag_k;
-  const int b_at = KMAJOR ? frag_k * LDB + b_row : b_row * LDB + frag_k;
-  auto fragment = [&](const float* src, int ld, int tile, int u) {
-    if constexpr (KMAJOR) {
-      const float* p = src + u * 8 * ld + tile * 32;
-      return make_float4(p[0], p[ld], p[2 * ld], p[3 * ld]);
-    } else {
-      return *reinterpret_cast<const float4*>(src + tile * 32 * ld + u * 8);
-    }
-  };
-  auto step = [&](int kt, auto slot_c) {
-    const int buf = kt & 1;
-    // (the other stage may still be read by wavefronts one step behind; this
-    // one's readers passed the barrier of the step before)
-    store_lds(buf, kt * BK, slot_c);
-    load_global((kt + PF) * BK, slot_c);
-    // the LDS writes of every wavefront are done; the loads stay in flight
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const float* as = As + buf * Cfg::STAGE_A + a_at;
-    const float* bs = Bs + buf * Cfg::STAGE_B + b_at;
-#pragma unroll
-    for (int u = 0; u < US; ++u) {
-      float4 af[TM], bfr[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = fragment(as, LDA, i, u);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bfr[j] = fragment(bs, LDB, j, u);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const float a = q == 0 ? af[i].x : q == 1 ? af[i].y
-                            : q == 2 ? af[i].z : af[i].w;
-            const float b = q == 0 ? bfr[j].x : q == 1 ? bfr[j].y
-                            : q == 2 ? bfr[j].z : bfr[j].w;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b, a, acc[i][j],
-                                                             0, 0, 0);
-          }
-      }
-    }
-  };
-  load_global(0, std::integral_constant<int, 0>());
-  load_global(BK, std::integral_constant<int, 1>());
-  if constexpr (PF > 2) load_global(2 * BK, std::integral_constant<int, PF - 1>());
-  for (int kt = 0; kt < nk; kt += PF) {
-    step(kt, std::integral_constant<int, 0>());
-    if (kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>());
-    if constexpr (PF > 2)
-      if (kt + 2 < nk) step(kt + 2, std::integral_constant<int, PF - 1>());
-  }
-  if constexpr (WK > 1) {
-    // [wk - 1][sub-tile][TM][TN][16][64], where the stages were
-    __syncthreads();
-    float* parts = reinterpret_cast<float*>(smem_raw);
-    constexpr int SUB = TM * TN * 1024, PLANE = WM * WN * SUB;
-    if (wk > 0) {
-      float* dst = parts + (wk - 1) * PLANE + wmn * SUB + lane;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            dst[((i * TN + j) * 16 + r) * 64] = acc[i][j][r];
-    }
-    __syncthreads();
-    if (wk > 0) return;
-#pragma unroll
-    for (int w = 0; w < WK - 1; ++w) {
-      const float* src = parts + w * PLANE + wmn * SUB + lane;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            acc[i][j][r] += src[((i * TN + j) * 16 + r) * 64];
-    }
-  }
-  const int m_l = lane & 31, n_l = (lane >> 5) * 4;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int grow = row0 + (wm * TM + i) * 32 + m_l;
-        const int gcol = col0 + (wn * TN + j) * 32 + 8 * q + n_l;
-        if (grow < R && gcol < N) {
-          float4 v = make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
-                                 acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-          const int64_t at = (int64_t)grow * N + gcol;
-          if (relu) {
-            v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f);
-            v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f);
-          }
-          if (mask_src != nullptr) {
-            const float4 m = *reinterpret_cast<const float4*>(
-                mask_src + (int64_t)e * R * N + at);
-            v.x = m.x > 0.f ? v.x * mask_scale : 0.f;
-            v.y = m.y > 0.f ? v.y * mask_scale : 0.f;
-            v.z = m.z > 0.f ? v.z * mask_scale : 0.f;
-            v.w = m.w > 0.f ? v.w * mask_scale : 0.f;
-          }
-          *reinterpret_cast<float4*>(Ce + at) = v;
-        }
-      }
-}
-
-// ---------------------------------------------------------------------------
 // Plain FMA tile kernel (float32, and bf16 shapes the MFMA kernel rejects):
 // 64 x 64 tile, 16-deep K step, each thread a 4 x 4 patch, float32 accumulate
 // in k order.
@@ -2214,72 +1964,6 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
 #undef MOE_RING
 }
 
-template <int TM, int TN, int WM, int WN, int WK, bool KMAJOR>
-static int launch_f32_mfma_tile(const float* A, const float* B, float* C, int E,
-                                int R, int N, int K, bool relu,
-                                const float* mask_src, float mask_scale,
-                                hipStream_t st) {
-  using Cfg = F32Cfg<TM, TN, WM, WN, WK, KMAJOR>;
-  const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
-  const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
-  const int64_t blocks = (int64_t)tiles_m * tiles_n * E;
-  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
-              "expert_ffn: too many tiles (%lld)", (long long)blocks);
-  auto k = grouped_gemm_f32_mfma_kernel<TM, TN, WM, WN, WK, KMAJOR>;
-  MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
-  k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
-      A, B, C, R, N, K, tiles_m, tiles_n, relu ? 1 : 0, mask_src, mask_scale);
-  MOE_CHECK_LAUNCH("expert_ffn (float32 mfma)");
-  return 0;
-}
-
-// Block tile of the float32 kernel.  The kernel is bound by the float32 matrix
-// pipes (a 32 x 32 x 2 MFMA takes 64 cycles), so its time is rounds of tiles
-// over the compute units times the tile's area; small launches want small tiles
-// (less padding of the row count, fewer idle compute units in the last round).
-// The smallest two pay for it with more LDS and cache traffic per product: the
-// weights.  Measured at 8 experts x 320 rows, per launch (us), in the order of
-// the table: 512 -> 2048 83, 71, 62, 67, 73; 2048 -> 512 151, 85, 85, 73, 67;
-// their weight gradients 57, 60, 60, 66, 72.
-template <bool KMAJOR>
-static int launch_f32_mfma(const float* A, const float* B, float* C, int E,
-                           int R, int N, int K, bool relu, hipStream_t st,
-                           const float* mask_src = nullptr,
-                           float mask_scale = 1.f) {
-  const int cus = compute_units();
-  if (cus == 0) return MESH_MOE_E_HIP;
-  static const int shapes[5][2] = {{128, 128}, {64, 128}, {64, 64}, {32, 64},
-                                   {32, 32}};
-  static const double weight[5] = {1.0, 1.0, 1.0, 1.08, 1.18};
-  int best = 0;
-  double best_cost = 0;
-  int64_t best_tiles = 0;
-  for (int i = 0; i < 5; ++i) {
-    const int bm = shapes[i][0], bn = shapes[i][1];
-    const int64_t tiles = (int64_t)E * ((R + bm - 1) / bm) * ((N + bn - 1) / bn);
-    const double cost = (double)((tiles + cus - 1) / cus) * bm * bn * weight[i];
-    // a smaller tile when it saves time by this count, or costs the same while
-    // the larger one leaves compute units with fewer than two blocks to overlap
-    if (i == 0 || cost < 0.95 * best_cost ||
-        (cost <= best_cost && best_tiles < 2 * (int64_t)cus)) {
-      best = i;
-      best_cost = cost;
-      best_tiles = tiles;
-    }
-  }
-#define MOE_F32_TILE(...)                                                      \
-  launch_f32_mfma_tile<__VA_ARGS__, KMAJOR>(A, B, C, E, R, N, K, relu,         \
-                                            mask_src, mask_scale, st)
-  switch (best) {
-    case 0: return MOE_F32_TILE(2, 2, 2, 2, 1);
-    case 1: return MOE_F32_TILE(1, 2, 2, 2, 1);
-    case 2: return MOE_F32_TILE(1, 1, 2, 2, 1);
-    case 3: return MOE_F32_TILE(1, 1, 1, 2, 2);
-    default: return MOE_F32_TILE(1, 1, 1, 1, 4);
-  }
-#undef MOE_F32_TILE
-}
-
 template <typename T>
 static int launch_simple(const T* A, const T* B, T* C, int E, int R, int N,
                          int K, bool relu, hipStream_t st) {
@@ -2338,14 +2022,13 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
   int rc;
   if (mask_applied) *mask_applied = false;
   if (dtype == MESH_MOE_F32) {
-    if (K % 4 == 0 && N % 4 == 0 && K >= 32 && R >= 32 && N >= 32 &&
+    if (K % 4 == 0 && N % 4 == 0 && f32_gemm_applies(R, N, K) &&
         (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0)) {
       const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
                          !relu && ((uintptr_t)relu_mask_src % 16) == 0;
-      rc = launch_f32_mfma<false>((const float*)A, (const float*)B, (float*)C,
-                                  E, R, N, K, relu, st,
-                                  masks ? (const float*)relu_mask_src : nullptr,
-                                  mask_scale);
+      rc = f32_gemm((const float*)A, (const float*)B, (float*)C, E, R, N, K, false,
+                    relu, masks ? (const float*)relu_mask_src : nullptr,
+                    mask_scale, st);
       if (masks) *mask_applied = rc == 0;
     } else
       rc = launch_simple<float>((const float*)A, (const float*)B, (float*)C, E,
@@ -2387,12 +2070,12 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
   return 0;
 }
 
-// C[e] = A[e]^T . B[e] in float32, A [K, R] and B [K, N]: takes the sizes and
-// alignments of launch_f32_mfma<true>.
+// C[e] = A[e]^T . B[e] in float32, A [K, R] and B [K, N]: what f32_gemm takes with
+// operands as they lie.
 static bool f32_kmajor_applies(const void* A, const void* B, const void* C,
                                int R, int N, int K, int dtype) {
-  return dtype == MESH_MOE_F32 && R % 4 == 0 && N % 4 == 0 && R >= 32 &&
-         N >= 32 && K >= 32 &&
+  return dtype == MESH_MOE_F32 && R % 4 == 0 && N % 4 == 0 &&
+         f32_gemm_applies(R, N, K) &&
          ((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0;
 }
 
@@ -3002,8 +2685,8 @@ extern "C" int mesh_moe_expert_linear_backward(
                               E, K, N, R, st, nullptr,
                               (void*)up((uintptr_t)workspace));
   if (f32_kmajor_applies(a, dy, dw, K, N, R, dtype))
-    return launch_f32_mfma<true>((const float*)a, (const float*)dy, (float*)dw,
-                                 E, K, N, R, false, st);
+    return f32_gemm((const float*)a, (const float*)dy, (float*)dw, E, K, N, R, true,
+                    false, nullptr, 1.f, st);
   const size_t es = dtype_size(dtype);
   unsigned char* tr_a = (unsigned char*)up((uintptr_t)workspace);
   unsigned char* tr_dy =
@@ -3113,11 +2796,11 @@ extern "C" int mesh_moe_expert_ffn_backward(
   }
   if (f32_kmajor_applies(h, dy, dwo, H, N, R, dtype) &&
       f32_kmajor_applies(expert_in, dh, dwi, M, H, R, dtype)) {
-    rc = launch_f32_mfma<true>((const float*)h, (const float*)dy, (float*)dwo,
-                               E, H, N, R, false, st);
+    rc = f32_gemm((const float*)h, (const float*)dy, (float*)dwo, E, H, N, R, true,
+                  false, nullptr, 1.f, st);
     if (rc != 0) return rc;
-    return launch_f32_mfma<true>((const float*)expert_in, (const float*)dh,
-                                 (float*)dwi, E, M, H, R, false, st);
+    return f32_gemm((const float*)expert_in, (const float*)dh, (float*)dwi, E, M, H,
+                    R, true, false, nullptr, 1.f, st);
   }
   // otherwise: both operands transposed to token-contiguous copies first
   rc = mesh_moe_pack_weights(h, tr_h, E, R, H, dtype, dtype, stream);

@@ -1,0 +1,513 @@
+// Grouped float32 products on the bf16 matrix cores of gfx950:
+//   C[e] = act(A[e] . B[e]^T),  or A[e]^T . B[e] (weight gradients)
+// (the float32 configuration of layers.dense_product / layers.dense in
+// mesh_tensorflow/transformer/moe.py:469-486 and of their gradients).
+#include <type_traits>
+#include <utility>
+
+#include "common.h"
+
+namespace mesh_moe {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+// ---------------------------------------------------------------------------
+// Every float32 is the sum of three bf16 terms, x = x1 + x2 + x3: x1 is x
+// rounded to bf16, x2 the remainder rounded, and what is left then has at most
+// 8 significant bits.  (Exactly, down to 2^-133, the last bit of a bf16
+// denormal: what an operand loses below that is less than 2^-134 of the other
+// operand.)  A product a b is then the sum of nine exact products, of which
+// a2 b3, a3 b2 and a3 b3, together below 2^-26 |a b|, are left out; the other six
+// run on v_mfma_f32_16x16x32_bf16, which adds exact products into float32: 96 cycles
+// of the matrix pipe for 16 x 16 outputs and k = 32 instead of 256 of
+// v_mfma_f32_32x32x2_f32.  The six are summed by themselves, small ones first, and
+// added to the accumulator once per 32 k, which rounds a sixteenth as often as
+// those did.  Error against float64 (relative 2-norm; before, with float32 MFMAs,
+// in brackets): K = 512 0.9e-7 (4.1e-7), 2048 1.3e-7 (4.1e-7), 3072 1.9e-7 (9.9e-7),
+// weight gradients from 320 rows 0.75e-7 (3.2e-7), 16000 rows 2.5e-7 (11e-7).
+//
+// Measured (us, float32 MFMAs -> here): 8 experts x 320 rows, 512 -> 2048 64 -> 39,
+// 2048 -> 512 66 -> 42, their weight gradients 54 -> 34; 4096 x 4096, K = 1024 303
+// -> 174 (1.18 PFLOP/s of bf16 products, what a large product reaches here); 64 x
+// 160 rows, 512 -> 2048 241 -> 132; 33 rows x 128, K = 4096, 32 experts 50 -> 28.
+// Bound by the bf16 matrix pipes (and the power cap) in large launches; in small
+// ones by the latency of a block's first loads and of its last stores, and by
+// making terms, 11 vector instructions per pair of values, which run beside the
+// MFMAs.  What stays behind is reductions of few K tiles (K = 200 and 260: 8.4 ->
+// 9.0 and 6.8 -> 7.3).
+//
+// A sum with an infinity, a NaN or an overflow in it is not what the terms give
+// (inf - inf, inf * 0).  Whatever such an operand touches comes out as an
+// infinity or a NaN; a wavefront that finds one among its results computes its
+// sub-tile again with float32 multiply-adds, in order of k.
+//
+// TM x TN MFMA tiles per wavefront; WN wavefronts along N times WK wavefronts
+// that share out the k of every K tile and add up their sums in the end.  All
+// wavefronts of a block work on the same 32 TM rows of A: their terms are made
+// once, on the way from registers into LDS ([3][rows][BK] bf16, rows padded by 16
+// bytes so that fragment reads and writes spread over all banks).  A
+// wavefront's 32 TN columns of B belong to it and its WK partners alone: its
+// lanes load them straight from memory in operand layout and make the terms in
+// registers.  Both operands of K tile t + 2 are on their way in registers, and
+// the terms of tile t + 1 are made beside the MFMAs of tile t.
+//
+// k is taken in an order of its own, the same for both operands: 16-byte piece
+// p of a group of 32 k holds k = 4 p .. 4 p + 3 and 16 + 4 p .. 16 + 4 p + 3, so
+// that the loads of a row are 64 bytes wide.
+//
+// KMAJOR: the reduction index is the outermost one of both operands (A [K][R],
+// B [K][N], token rows summed over); a lane's 8 k of a column are 8 loads, each
+// contiguous over the wavefront.
+// ---------------------------------------------------------------------------
+template <int TM_, int TN_, int WN_, int WK_>
+struct SplitCfg {
+  static constexpr int TM = TM_, TN = TN_, WN = WN_, WK = WK_;
+  static constexpr int THREADS = 64 * WN * WK;
+  static constexpr int BM = 16 * TM, BN = 16 * TN * WN;
+  static constexpr int BK = WK > 1 ? 32 * WK : 32;
+  static constexpr int LDR = BK + 8;           // bf16 per LDS row
+  static constexpr int PLANE = BM * LDR;       // one term of the A tile
+  static constexpr int STAGE = 3 * PLANE;
+  static constexpr int CHUNKS = BK / 8;        // 16-byte pieces per row
+  static constexpr int A_PIECES = BM * CHUNKS;
+  // per thread; where they do not come out even, some pieces are done twice
+  static constexpr int A_CHUNKS = (A_PIECES + THREADS - 1) / THREADS;
+  static constexpr int KS = BK / 32 / WK;      // MFMA steps of a wavefront
+  static constexpr size_t LOOP_BYTES = 2ull * STAGE * sizeof(bf16_t);
+  static constexpr size_t SUM_BYTES =
+      (size_t)(WK - 1) * WN * TM * TN * 256 * sizeof(float);
+  static constexpr size_t LDS_BYTES =
+      LOOP_BYTES > SUM_BYTES ? LOOP_BYTES : SUM_BYTES;
+};
+
+template <typename F, int... I>
+__device__ __forceinline__ void for_each_index(
+    F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>()), ...);
+}
+// f(0), ..., f(COUNT - 1) with constant arguments
+template <int COUNT, typename F>
+__device__ __forceinline__ void for_each_index(F f) {
+  for_each_index(f, std::make_integer_sequence<int, COUNT>());
+}
+
+// The three terms of two values, a's in the low halves.  (The remainders by
+// v_dot2c_f32_bf16 would be one instruction each instead of two, but it waits for
+// the matrix pipe: 8 of them and 2 MFMAs take as long as both by themselves.)
+__device__ __forceinline__ void split_pair(float a, float b,
+                                           uint32_t (&t)[3]) {
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    t[n] = f32x2_to_bf16x2(a, b);
+    if (n == 2) break;
+    a = a - __uint_as_float(t[n] << 16);            // exact
+    b = b - __uint_as_float(t[n] & 0xffff0000u);
+  }
+}
+// the terms of 8 values as MFMA operands
+__device__ __forceinline__ void split_terms(const float (&f)[8],
+                                            uint4 (&t)[3]) {
+  uint32_t w[4][3];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) split_pair(f[2 * p], f[2 * p + 1], w[p]);
+#pragma unroll
+  for (int n = 0; n < 3; ++n)
+    t[n] = make_uint4(w[0][n], w[1][n], w[2][n], w[3][n]);
+}
+
+// mask_src (shape of C): elements whose mask_src element is not positive become
+// 0, the others are multiplied by mask_scale.
+__device__ __forceinline__ float finish_f32(float v, bool relu, bool masked,
+                                            float m, float mask_scale) {
+  if (relu) v = fmaxf(v, 0.f);
+  if (masked) v = m > 0.f ? v * mask_scale : 0.f;
+  return v;
+}
+
+template <int TM, int TN, int WN, int WK, int RAW, bool KMAJOR>
+__global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
+    const float* __restrict__ A, const float* __restrict__ B,
+    float* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
+    int relu, const float* __restrict__ mask_src, float mask_scale) {
+  using Cfg = SplitCfg<TM, TN, WN, WK>;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, LDR = Cfg::LDR;
+  constexpr int KS = Cfg::KS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  bf16_t* As = reinterpret_cast<bf16_t*>(smem_raw);   // [2][3][BM][LDR]
+  // an XCD works on a contiguous range of tiles, which share weight panels
+  const int nblk = gridDim.x;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int logical = xcd * (nblk >> 3) + min(xcd, nblk & 7) + local;
+  const int tiles_per_e = tiles_m * tiles_n;
+  const int e = logical / tiles_per_e;
+  const int rem = logical - e * tiles_per_e;
+  const int tn = rem / tiles_m, tm = rem - tn * tiles_m;
+  const int row0 = tm * BM, col0 = tn * BN;
+  const float* Ae = A + (int64_t)e * R * K;
+  const float* Be = B + (int64_t)e * N * K;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wk = wave / WN, wn = wave % WN;
+
+  // Where this thread's loads lie relative to the K tile's corner (element
+  // (row0, k0) of A, (col0, k0) of B), in bytes.  Rows past the end are read as
+  // the last one and not stored.
+  auto k_of_piece = [](int c) { return (c >> 2) * 32 + (c & 3) * 4; };
+  uint32_t a_off[Cfg::A_CHUNKS], b_off[KS][TN];
+  int a_lds[Cfg::A_CHUNKS], a_k[Cfg::A_CHUNKS], b_k[KS];
+#pragma unroll
+  for (int i = 0; i < Cfg::A_CHUNKS; ++i) {
+    const int c = (tid + i * Cfg::THREADS) % Cfg::A_PIECES;
+    const int r = KMAJOR ? c % BM : c / Cfg::CHUNKS;
+    const int piece = KMAJOR ? c / BM : c % Cfg::CHUNKS;
+    const uint32_t row = min(row0 + r, R - 1) - row0;
+    a_k[i] = k_of_piece(piece);
+    a_off[i] = 4u * (KMAJOR ? (uint32_t)a_k[i] * R + row : row * K + a_k[i]);
+    a_lds[i] = r * LDR + piece * 8;
+  }
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    b_k[s] = k_of_piece((wk * KS + s) * 4 + (lane >> 4));
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int c = (wn * TN + j) * 16 + (lane & 15);
+      const uint32_t col = min(col0 + c, N - 1) - col0;
+      b_off[s][j] = 4u * (KMAJOR ? (uint32_t)b_k[s] * N + col : col * K + b_k[s]);
+    }
+  }
+  // 8 values of one row: k .. k + 3 and k + 16 .. k + 19 from `at` on
+  auto load8 = [&](const float* corner, uint32_t off, int rows, float (&f)[8]) {
+    const char* p = reinterpret_cast<const char*>(corner);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (KMAJOR) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          f[4 * h + q] = *reinterpret_cast<const float*>(
+              p + (int64_t)(16 * h + q) * rows * 4 + off);
+      } else {
+        const float4 v = *reinterpret_cast<const float4*>(p + 64 * h + off);
+        f[4 * h] = v.x; f[4 * h + 1] = v.y; f[4 * h + 2] = v.z; f[4 * h + 3] = v.w;
+      }
+    }
+  };
+  const float* a_corner = Ae + (KMAJOR ? (int64_t)row0 : (int64_t)row0 * K);
+  const float* b_corner = Be + (KMAJOR ? (int64_t)col0 : (int64_t)col0 * K);
+  const int nk = K / BK;          // whole K tiles, at least one
+  // first k of K tile kt; past the whole tiles, the last BK of k
+  auto k_first = [&](int kt) { return (int64_t)min(kt * BK, K - BK); };
+  float a_raw[RAW][Cfg::A_CHUNKS][8], b_raw[RAW][KS][TN][8];
+  auto load_tile = [&](int kt, auto slot_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+    const int64_t k0 = k_first(kt);
+    const float* ac = a_corner + (KMAJOR ? k0 * R : k0);
+    const float* bc = b_corner + (KMAJOR ? k0 * N : k0);
+#pragma unroll
+    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
+      load8(ac, a_off[i], R, a_raw[SLOT % RAW][i]);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) load8(bc, b_off[s][j], N, b_raw[SLOT % RAW][s][j]);
+  };
+  uint4 b_terms[2][KS][TN][3];
+  // the terms of a loaded tile: A's into stage `slot`, B's into registers
+  auto make_terms = [&](auto slot_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+#pragma unroll
+    for (int i = 0; i < Cfg::A_CHUNKS; ++i) {
+      uint4 t[3];
+      split_terms(a_raw[SLOT % RAW][i], t);
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+        *reinterpret_cast<uint4*>(As + SLOT * Cfg::STAGE + n * Cfg::PLANE +
+                                  a_lds[i]) = t[n];
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        split_terms(b_raw[SLOT % RAW][s][j], b_terms[SLOT][s][j]);
+  };
+
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+  // The products of the K tile in stage / registers SLOT.  With NEXT, the terms of
+  // the other slot's loaded tile are made on the way, a pair of values at a time
+  // between the MFMAs, and each piece's registers are loaded again with tile
+  // `ahead`.
+  auto products = [&](auto slot_c, auto next_c, int ahead) {
+    constexpr int SLOT = decltype(slot_c)::value, OTHER = SLOT ^ 1;
+    constexpr bool NEXT = decltype(next_c)::value;
+    // (the small products first)
+    constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
+    constexpr int MFMAS = 6 * TM * TN * KS;
+    constexpr int GROUPS = Cfg::A_CHUNKS + KS * TN, PAIRS = 4 * GROUPS;
+    const int64_t k0 = k_first(ahead);
+    const float* ac = a_corner + (KMAJOR ? k0 * R : k0);
+    const float* bc = b_corner + (KMAJOR ? k0 * N : k0);
+    const bf16_t* src = As + SLOT * Cfg::STAGE + (lane & 15) * LDR +
+                        (wk * KS * 4 + (lane >> 4)) * 8;
+    // the terms of row tile at % TM in MFMA step at / TM
+    bf16x8_t af[2][3];
+    auto read = [&](int at) {
+#pragma unroll
+      for (int n = 0; n < 3; ++n)
+        af[at & 1][n] = *reinterpret_cast<const bf16x8_t*>(
+            src + n * Cfg::PLANE + at % TM * 16 * LDR + at / TM * 32);
+    };
+    uint32_t w[3][4];
+    auto work = [&](auto at_c) {
+      constexpr int g = decltype(at_c)::value >> 2, p = decltype(at_c)::value & 3;
+      constexpr bool of_a = g < Cfg::A_CHUNKS;
+      constexpr int ga = of_a ? g : 0, gb = of_a ? 0 : g - Cfg::A_CHUNKS;
+      constexpr int s = gb / TN, j = gb % TN;
+      float(&raw)[8] = of_a ? a_raw[OTHER % RAW][ga] : b_raw[OTHER % RAW][s][j];
+      uint32_t t[3];
+      split_pair(raw[2 * p], raw[2 * p + 1], t);
+#pragma unroll
+      for (int n = 0; n < 3; ++n) w[n][p] = t[n];
+      if constexpr (p == 3) {
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+          const uint4 v = make_uint4(w[n][0], w[n][1], w[n][2], w[n][3]);
+          if constexpr (of_a)
+            *reinterpret_cast<uint4*>(As + OTHER * Cfg::STAGE + n * Cfg::PLANE +
+                                      a_lds[ga]) = v;
+          else
+            b_terms[OTHER][s][j][n] = v;
+        }
+        if constexpr (of_a) load8(ac, a_off[ga], R, raw);
+        else load8(bc, b_off[s][j], N, raw);
+      }
+    };
+    // the products of 32 k, added to the accumulators while the next row tile's
+    // are on their way
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t sum[2][TN];
+    auto add = [&](int at, int j) { acc[at % TM][j] += sum[at & 1][j]; };
+    read(0);
+    for_each_index<MFMAS>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value;
+      constexpr int j = m % TN, p = m / TN % 6, at = m / (TN * 6), i = at % TM,
+                    s = at / TM;
+      constexpr int ta = TA[p], tb = TB[p];
+      if constexpr (m % (TN * 6) == 0 && at + 1 < TM * KS) read(at + 1);
+      sum[at & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(bf16x8_t, b_terms[SLOT][s][j][tb]), af[at & 1][ta],
+          p == 0 ? zero : sum[at & 1][j], 0, 0, 0);
+      if constexpr (at > 0 && p == 1) add(at - 1, j);
+      if constexpr (NEXT) {
+        constexpr int from = PAIRS * m / MFMAS, to = PAIRS * (m + 1) / MFMAS;
+        for_each_index<to - from>([&](auto at_c) {
+          work(std::integral_constant<int, from + decltype(at_c)::value>());
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+#pragma unroll
+    for (int j = 0; j < TN; ++j) add(TM * KS - 1, j);
+  };
+  // LDS writes and reads of every wavefront are done; loads stay in flight
+  auto barrier = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  load_tile(0, S0());
+  if constexpr (RAW == 2) load_tile(1, S1());
+  make_terms(S0());
+  load_tile(RAW, S0());
+  barrier();
+  // (the stage written here was read in the step before, whose readers have
+  // passed the barrier at its end; past the end it is written for nobody)
+  for (int kt = 0; kt + 1 < nk; kt += 2) {
+    products(S0(), std::true_type(), kt + 1 + RAW);
+    barrier();
+    products(S1(), std::true_type(), kt + 2 + RAW);
+    barrier();
+  }
+  if (nk & 1) {
+    products(S0(), std::false_type(), 0);
+    barrier();
+  }
+  if (nk * BK < K) {
+    // the last BK of k are in the raw registers: the whole tiles' share of them
+    // becomes zeros in A
+    const int old = (nk + 1) * BK - K;
+#pragma unroll
+    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (a_k[i] + (q >> 2) * 16 + (q & 3) < old) a_raw[0][i][q] = 0.f;
+    make_terms(S0());
+    barrier();
+    products(S0(), std::false_type(), 0);
+    barrier();
+  }
+  if constexpr (WK > 1) {
+    // [wk - 1][wn][TM][TN][4][64], where the stages were
+    float* parts = reinterpret_cast<float*>(smem_raw);
+    constexpr int SUB = TM * TN * 256, PART = WN * SUB;
+    if (wk > 0) {
+      float* dst = parts + (wk - 1) * PART + wn * SUB + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            dst[((i * TN + j) * 4 + r) * 64] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int w = 0; w < WK - 1; ++w) {
+      const float* src = parts + w * PART + wn * SUB + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[i][j][r] += src[((i * TN + j) * 4 + r) * 64];
+    }
+  }
+  float* Ce = Cout + (int64_t)e * R * N;
+  const float* mask = mask_src == nullptr ? nullptr : mask_src + (int64_t)e * R * N;
+  const int col_w = col0 + wn * TN * 16;
+  // 0 x is 0 only for finite x
+  float test = 0.f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) test = __builtin_fmaf(acc[i][j][r], 0.f, test);
+  if (__any(!(test == 0.f))) {
+    for (int at = lane; at < BM * TN * 16; at += 64) {
+      const int row = row0 + at / (TN * 16), col = col_w + at % (TN * 16);
+      if (row >= R || col >= N) continue;
+      const int64_t sa = KMAJOR ? R : 1, sb = KMAJOR ? N : 1;
+      const float* pa = Ae + (KMAJOR ? (int64_t)row : (int64_t)row * K);
+      const float* pb = Be + (KMAJOR ? (int64_t)col : (int64_t)col * K);
+      float sum = 0.f;
+      for (int k = 0; k < K; ++k) sum = __builtin_fmaf(pa[k * sa], pb[k * sb], sum);
+      const int64_t c = (int64_t)row * N + col;
+      Ce[c] = finish_f32(sum, relu, mask != nullptr, mask ? mask[c] : 1.f,
+                         mask_scale);
+    }
+    return;
+  }
+  const int m_l = lane & 15, n_l = (lane >> 4) * 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int grow = row0 + i * 16 + m_l, gcol = col_w + j * 16 + n_l;
+      if (grow < R && gcol < N) {
+        const int64_t c = (int64_t)grow * N + gcol;
+        const float4 m = mask == nullptr
+                             ? make_float4(1.f, 1.f, 1.f, 1.f)
+                             : *reinterpret_cast<const float4*>(mask + c);
+        const bool masked = mask != nullptr;
+        *reinterpret_cast<float4*>(Ce + c) = make_float4(
+            finish_f32(acc[i][j][0], relu, masked, m.x, mask_scale),
+            finish_f32(acc[i][j][1], relu, masked, m.y, mask_scale),
+            finish_f32(acc[i][j][2], relu, masked, m.z, mask_scale),
+            finish_f32(acc[i][j][3], relu, masked, m.w, mask_scale));
+      }
+    }
+}
+
+template <int TM, int TN, int WN, int WK, int RAW>
+static int launch_split(const float* A, const float* B, float* C, int E, int R,
+                        int N, int K, bool kmajor, bool relu,
+                        const float* mask_src, float mask_scale, hipStream_t st) {
+  using Cfg = SplitCfg<TM, TN, WN, WK>;
+  const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
+  const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t blocks = (int64_t)tiles_m * tiles_n * E;
+  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: too many tiles (%lld)", (long long)blocks);
+  auto k = kmajor ? grouped_gemm_f32_split_kernel<TM, TN, WN, WK, RAW, true>
+                  : grouped_gemm_f32_split_kernel<TM, TN, WN, WK, RAW, false>;
+  MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
+  k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
+      A, B, C, R, N, K, tiles_m, tiles_n, relu ? 1 : 0, mask_src, mask_scale);
+  MOE_CHECK_LAUNCH("expert_ffn (float32 in bf16 terms)");
+  return 0;
+}
+
+// Block tiles and what a launch of one costs: a + n b us for n = blocks per
+// compute unit (rounded up), plus (c + n d) us per K tile.  Fitted to 38 products
+// of 1 to 64 experts, 33 to 8192 rows, K 36 to 16000, both layouts, each with
+// every tile (root mean square of the deviations 6 to 10 %, 18 % for the smallest
+// tile); the tile the fit picks is 0.6 % slower than the best one on average and 10 %
+// at worst.  Large tiles spend less on making terms (each value of A once per
+// column tile, of B once per row tile), small ones waste less on rows that do not
+// fill a tile and on the last round; the wavefronts of the small ones share out
+// k, so that every SIMD has work.
+struct SplitTile {
+  int rows, cols, k;
+  decltype(&launch_split<8, 2, 8, 1, 1>) launch;
+  double a, b, c, d;
+};
+template <int TM, int TN, int WN, int WK, int RAW>
+static constexpr SplitTile split_tile(double a, double b, double c, double d) {
+  using Cfg = SplitCfg<TM, TN, WN, WK>;
+  return {Cfg::BM, Cfg::BN, Cfg::BK, launch_split<TM, TN, WN, WK, RAW>, a, b, c, d};
+}
+static const SplitTile split_tiles[] = {
+    split_tile<8, 2, 8, 1, 1>(0.0, 5.93, 0.0, 2.08),     // 128 x 256
+    split_tile<10, 2, 8, 1, 1>(0.0, 6.23, 0.0, 2.76),    // 160 x 256
+    split_tile<10, 2, 4, 2, 1>(0.33, 7.41, 0.0, 2.98),   // 160 x 128
+    split_tile<4, 2, 4, 2, 1>(1.71, 3.89, 0.0, 1.39),    // 64 x 128
+    split_tile<5, 2, 2, 4, 1>(1.27, 5.19, 0.0, 2.01),    // 80 x 64
+    split_tile<6, 2, 2, 4, 1>(0.86, 5.74, 0.0, 2.18),    // 96 x 64
+    split_tile<2, 2, 1, 8, 1>(1.71, 3.12, 0.10, 1.36),   // 32 x 32
+    split_tile<1, 2, 1, 4, 2>(4.10, 0.34, 0.0, 0.59),    // 16 x 32
+    split_tile<2, 2, 2, 2, 1>(3.39, 0.52, 0.13, 0.58),   // 32 x 64
+    split_tile<6, 2, 8, 1, 1>(0.0, 5.35, 0.0, 1.75),     // 96 x 256
+    split_tile<4, 2, 8, 1, 1>(0.0, 4.97, 0.0, 1.35),     // 64 x 256
+    split_tile<4, 2, 4, 1, 1>(1.85, 2.07, 0.26, 0.68),   // 64 x 128, K tiles of 32
+    split_tile<1, 2, 4, 1, 2>(2.90, 0.50, 0.13, 0.48)};  // 16 x 128
+
+bool f32_gemm_applies(int R, int N, int K) {
+  // (offsets inside a tile are 32 bits)
+  const int most = 1 << 22;
+  return R >= 32 && N >= 32 && K >= 32 && R <= most && N <= most && K <= most;
+}
+
+int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int K,
+             bool kmajor, bool relu, const float* mask_src, float mask_scale,
+             hipStream_t st) {
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  const SplitTile* best = nullptr;
+  double best_cost = 0;
+  for (const SplitTile& t : split_tiles) {
+    if (t.k > K) continue;
+    const int64_t blocks = (int64_t)E * ((R + t.rows - 1) / t.rows) *
+                           ((N + t.cols - 1) / t.cols);
+    const double n = (double)((blocks + cus - 1) / cus);
+    const double cost =
+        t.a + n * t.b + (double)((K + t.k - 1) / t.k) * (t.c + n * t.d);
+    if (best == nullptr || cost < best_cost) {
+      best = &t;
+      best_cost = cost;
+    }
+  }
+  return best->launch(A, B, C, E, R, N, K, kmajor, relu, mask_src, mask_scale, st);
+}
+
+}  // namespace mesh_moe

@@ -1,0 +1,96 @@
+"""float32 products in three bf16 terms per operand, against float64."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+  from mesh_amd import moe_hip
+  moe_hip.load_library()
+  return moe_hip
+
+
+def _values(gen, *sizes):
+  """Sixteen binary orders of magnitude, signs mixed."""
+  exponent = torch.randint(-8, 8, sizes, generator=gen, device="cuda")
+  return torch.ldexp(torch.randn(sizes, generator=gen, device="cuda"), exponent)
+
+
+def _assert_close(got, a, b):
+  """got [E,R,N] against a [E,R,K] . b [E,K,N].  Per 32 k six matrix products of
+  exact terms and one addition to the sum, and a handful of additions where
+  wavefronts share k out; what the three dropped products of terms leave out is
+  below 2^-26 of |a b|."""
+  a, b = a.double(), b.double()
+  roundings = a.shape[2] // 32 + 20
+  bound = roundings * 2.0 ** -24 * (a.abs() @ b.abs())
+  assert (((got.double() - a @ b).abs()) <= bound).all()
+
+
+# rows and columns around the tiles' edges (16 to 160 rows, 32 to 256 columns), k
+# below, at and above one K tile of 32 to 256 and with remainders, few and many
+# tiles: every tile of the table is picked by one of them
+SHAPES = [
+    (1, 32, 32, 32), (1, 33, 36, 36), (1, 33, 68, 60), (3, 47, 132, 64),
+    (1, 64, 512, 512), (2, 65, 260, 100), (1, 37, 64, 2052), (1, 100, 96, 1028),
+    (8, 161, 1028, 196), (8, 320, 2048, 256), (8, 320, 512, 1028), (7, 95, 508, 260),
+    (4, 330, 516, 644), (16, 97, 1024, 100), (30, 129, 1028, 68), (24, 255, 772, 36),
+    (9, 161, 4096, 64), (1, 2000, 640, 320), (1, 5000, 36, 96), (12, 427, 1024, 128)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_products(hip, shape):
+  e, r, n, k = shape
+  gen = torch.Generator(device="cuda").manual_seed(sum(shape))
+  a, w = _values(gen, e, r, k), _values(gen, e, n, k)
+  got = hip.expert_linear(a, w, "linear")
+  _assert_close(got, a, w.transpose(1, 2).contiguous())
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_products_summed_over_rows(hip, shape):
+  """Weight gradients: both operands with the reduction outermost, any length."""
+  e, m, n, rows = shape
+  m, rows = (m + 3) // 4 * 4, rows + 1
+  gen = torch.Generator(device="cuda").manual_seed(sum(shape))
+  a, dy = _values(gen, e, rows, m), _values(gen, e, rows, n)
+  w = torch.empty(e, m, n, device="cuda")
+  _, got = hip.expert_linear_backward(a, dy, w, want_da=False)
+  _assert_close(got, a.transpose(1, 2).contiguous(), dy)
+
+
+@pytest.mark.parametrize("shape", [(2, 70, 260, 100), (8, 320, 512, 1028)])
+@pytest.mark.parametrize("activation", ["linear", "relu"])
+def test_infinities_nan_and_overflow(hip, shape, activation):
+  """What an infinity, a NaN or an overflow does to a sum is what it does in
+  float32 arithmetic; the rest of its tile keeps its values."""
+  e, r, n, k = shape
+  gen = torch.Generator(device="cuda").manual_seed(5)
+  a, w = _values(gen, e, r, k), _values(gen, e, n, k)
+  a[0, 3, 7] = float("inf")
+  w[0, 9, 7] = -2.0            # -inf
+  w[0, 10, 7] = 1.0            # +inf: no remainder of 1.0 times infinity
+  w[0, 11, 7] = 0.0            # NaN
+  a[0, 5, 1] = float("nan")
+  a[1, 0, 2], a[1, 0, 3] = 3e38, -3e38
+  w[1, 4, 2], w[1, 4, 3] = 2.0, -2.0    # overflows in any order
+  a[1, 1, 0] = 3.402823e38              # rounds to infinity in bf16
+  w[1, :, 0] = 2.0 ** -20
+  got = hip.expert_linear(a, w, activation).double()
+  wt = w.double().transpose(1, 2).contiguous()
+  want, absolute = a.double() @ wt, a.double().abs() @ wt.abs()
+  # (an element of a tile that is computed again is added k by k)
+  bound = (k + 20) * 2.0 ** -24 * absolute
+  want = want.float().double()
+  if activation == "relu":
+    # NaN and negative sums become 0, as in every other kernel here
+    want = torch.where(want > 0, want, torch.zeros_like(want))
+  sure = absolute < 3.4e38              # no partial sum can overflow
+  assert ((got - want).abs() <= bound)[sure].all()
+  sure = ~absolute.isfinite()
+  sure[1, 0, 4] = True
+  assert torch.equal(got[sure].nan_to_num(7.0, 1e300, -1e300),
+                     want[sure].nan_to_num(7.0, 1e300, -1e300))
