@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 35
+#define MESH_MOE_ABI_VERSION 36
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -265,13 +265,25 @@ int mesh_moe_pack_weights(const void* src, void* dst, int E, int K, int N,
  *   expert_in [E,R,M] dtype (R = rows per expert = groups * capacity)
  *   wi_packed [E,H,M] dtype; wo_packed [E,N,H] dtype  (see pack_weights)
  *   h [E,R,H] dtype (caller-provided scratch); y [E,R,N] dtype
- * bf16 with M and H multiples of 8 runs on the MFMA kernel; float32 and other
- * shapes run on a plain FMA tile kernel.
+ * bf16 with M and H multiples of 8 and float32 with M, H and N multiples of 4 run on
+ * the matrix cores (float32 as three bf16 terms per value, with less error than
+ * float32 multiply-adds), other shapes on a plain FMA tile kernel.
  */
 int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
                         const void* wo_packed, void* h, void* y, int E, int R,
                         int M, int H, int N, int activation, int dtype,
                         void* stream);
+
+/*
+ * mesh_moe_expert_ffn for callers that keep h, i.e. for a step whose gradient is
+ * wanted: the same, except that float32 ReLU experts sum h in an order that stays as
+ * it is from one version of the library to the next (which hidden units the ReLU
+ * lets through hangs on sums that may be 0 up to rounding, and so do gradients).
+ */
+int mesh_moe_expert_ffn_kept(const void* expert_in, const void* wi_packed,
+                             const void* wo_packed, void* h, void* y, int E,
+                             int R, int M, int H, int N, int activation,
+                             int dtype, void* stream);
 
 /*
  * One expert projection: y = act(a . w) per expert, float32 accumulate -- the

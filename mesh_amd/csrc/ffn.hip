@@ -2010,6 +2010,13 @@ static bool ring_path_applies(int R, int N, int K) {
   return ring_shape(R, N, K) && pad128 * 5 >= pad256 * 4;
 }
 
+// f32_gemm and f32_gemm_stable take these operands
+static bool f32_nt_applies(const void* A, const void* B, const void* C, int R,
+                           int N, int K) {
+  return K % 4 == 0 && N % 4 == 0 && f32_gemm_applies(R, N, K) &&
+         ((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0;
+}
+
 // C[e] = act(A[e] . B[e]^T) for every expert.
 // relu_mask_src (same shape and dtype as C): the kernels that can zero the
 // elements of C whose mask_src element is not positive while they write C do so
@@ -2022,8 +2029,7 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
   int rc;
   if (mask_applied) *mask_applied = false;
   if (dtype == MESH_MOE_F32) {
-    if (K % 4 == 0 && N % 4 == 0 && f32_gemm_applies(R, N, K) &&
-        (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0)) {
+    if (f32_nt_applies(A, B, C, R, N, K)) {
       const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
                          !relu && ((uintptr_t)relu_mask_src % 16) == 0;
       rc = f32_gemm((const float*)A, (const float*)B, (float*)C, E, R, N, K, false,
@@ -2116,10 +2122,10 @@ int batched_gemm_nt(const void* A, const void* B, void* C, int E, int R, int N,
 
 using namespace mesh_moe;
 
-extern "C" int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
-                                   const void* wo_packed, void* h, void* y,
-                                   int E, int R, int M, int H, int N,
-                                   int activation, int dtype, void* stream) {
+static int expert_ffn(const void* expert_in, const void* wi_packed,
+                      const void* wo_packed, void* h, void* y, int E, int R, int M,
+                      int H, int N, int activation, int dtype, void* stream,
+                      bool hidden_kept) {
   MOE_REQUIRE(expert_in && wi_packed && wo_packed && h && y, MESH_MOE_E_ARG,
               "expert_ffn: null pointer");
   MOE_REQUIRE(valid_dtype(dtype), MESH_MOE_E_ARG, "expert_ffn: bad dtype %d",
@@ -2130,11 +2136,33 @@ extern "C" int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
                   activation <= MESH_MOE_ACT_SWISH,
               MESH_MOE_E_ARG, "expert_ffn: unknown activation %d", activation);
   hipStream_t st = (hipStream_t)stream;
-  int rc = grouped_gemm(expert_in, wi_packed, h, E, R, H, M, activation, dtype,
-                        st);
+  int rc;
+  if (hidden_kept && dtype == MESH_MOE_F32 && activation == MESH_MOE_ACT_RELU &&
+      f32_nt_applies(expert_in, wi_packed, h, R, H, M))
+    rc = f32_gemm_stable((const float*)expert_in, (const float*)wi_packed,
+                         (float*)h, E, R, H, M, true, st);
+  else
+    rc = grouped_gemm(expert_in, wi_packed, h, E, R, H, M, activation, dtype, st);
   if (rc != 0) return rc;
   return grouped_gemm(h, wo_packed, y, E, R, N, H, MESH_MOE_ACT_LINEAR, dtype,
                       st);
+}
+
+extern "C" int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
+                                   const void* wo_packed, void* h, void* y,
+                                   int E, int R, int M, int H, int N,
+                                   int activation, int dtype, void* stream) {
+  return expert_ffn(expert_in, wi_packed, wo_packed, h, y, E, R, M, H, N,
+                    activation, dtype, stream, false);
+}
+
+extern "C" int mesh_moe_expert_ffn_kept(const void* expert_in,
+                                        const void* wi_packed,
+                                        const void* wo_packed, void* h, void* y,
+                                        int E, int R, int M, int H, int N,
+                                        int activation, int dtype, void* stream) {
+  return expert_ffn(expert_in, wi_packed, wo_packed, h, y, E, R, M, H, N,
+                    activation, dtype, stream, true);
 }
 
 namespace mesh_moe {

@@ -510,4 +510,285 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
   return best->launch(A, B, C, E, R, N, K, kmajor, relu, mask_src, mask_scale, st);
 }
 
+// ---------------------------------------------------------------------------
+// Sums that do not change: v_mfma_f32_32x32x2_f32, true float32 operands, the
+// order of k and the tiles these products have always had.
+//
+// For the hidden tensor that a training step keeps.  Its ReLU lets a unit through
+// or not by the sign of a sum, about one in ten million of these sums is 0 up to
+// rounding, and a unit that switches moves its column of the weight gradient by up
+// to 0.6 of the gradient's root mean square.  With other rounding a few units of a
+// step would switch, so that steps of two versions could not be compared; the more
+// exact kernel above is as good an answer, and not the same one.  (All other
+// products of a step are continuous in their operands and go there.)
+//
+// Four wavefronts; K step 32.  The weight tile is the MFMA's first operand, so a
+// lane ends up with 4 consecutive output columns per register group.  One MFMA
+// consumes k = 2 s + (lane / 32) for step s; a lane instead takes the four
+// consecutive k = 8 u + 4 (lane / 32) + j for steps 4 u + j, which makes its operand
+// reads 16 bytes wide.  Tiles are staged through registers into LDS rows of 32 + 4
+// floats.  K % 4 == 0 and N % 4 == 0.
+//
+// Bound by the float32 matrix pipes, of whose 64 cycles an MFMA the loop keeps 60 to
+// 75 % busy.  Three (128 x 128 tiles: two) K tiles are on their way in registers, and
+// the barrier does not wait for them.  8 experts x 320 rows, 5.4 GFLOP (34 us at the
+// peak): 512 -> 2048 62 us, 2048 -> 512 67 us.
+//
+// TM x TN: MFMA tiles per wavefront.  WM x WN x WK: the wavefronts' grid; the
+// WK wavefronts of a sub-tile share out the k of every staged tile and add up
+// their sums in the end, so a small tile keeps all four matrix pipes busy.
+// ---------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
+
+template <int TM, int TN, int WM, int WN, int WK>
+struct F32Cfg {
+  static_assert(WM * WN * WK == 4, "four wavefronts");
+  static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN, BK = 32,
+                       THREADS = 256;
+  // floats per LDS row and per stage of an operand
+  static constexpr int LDR = BK + 4;
+  static constexpr int STAGE_A = BM * LDR, STAGE_B = BN * LDR;
+  static constexpr int CPR = BK / 4;      // 16-byte chunks per staged row
+  // K tiles loaded ahead
+  static constexpr int PF = BM * BN >= 128 * 128 ? 2 : 3;
+  static constexpr int A_CHUNKS = BM * BK / 4 / THREADS;
+  static constexpr int B_CHUNKS = BN * BK / 4 / THREADS;
+  static constexpr size_t LDS_BYTES =
+      2ull * (STAGE_A + STAGE_B) * sizeof(float);
+  static_assert(LDS_BYTES >= (WK - 1) * WM * WN * TM * TN * 1024 * sizeof(float),
+                "the partial sums of the other wavefronts fit");
+};
+
+template <int TM, int TN, int WM, int WN, int WK>
+__global__ __launch_bounds__(256) void grouped_gemm_f32_mfma_kernel(
+    const float* __restrict__ A, const float* __restrict__ B,
+    float* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
+    int relu) {
+  using Cfg = F32Cfg<TM, TN, WM, WN, WK>;
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
+  constexpr int LDR = Cfg::LDR, CPR = Cfg::CPR, PF = Cfg::PF;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  float* As = reinterpret_cast<float*>(smem_raw);  // [2][STAGE_A]
+  float* Bs = As + 2 * Cfg::STAGE_A;               // [2][STAGE_B]
+  const int nblk = gridDim.x;
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int logical = xcd * (nblk >> 3) + min(xcd, nblk & 7) + local;
+  const int tiles_per_e = tiles_m * tiles_n;
+  const int e = logical / tiles_per_e;
+  const int rem = logical - e * tiles_per_e;
+  const int tn = rem / tiles_m, tm = rem - tn * tiles_m;
+  const int row0 = tm * BM, col0 = tn * BN;
+  const float* Ae = A + (int64_t)e * R * K;
+  const float* Be = B + (int64_t)e * N * K;
+  float* Ce = Cout + (int64_t)e * R * N;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wk = wave / (WM * WN), wmn = wave % (WM * WN);
+  const int wm = wmn / WN, wn = wmn % WN;
+
+  // PF K tiles are on their way in registers beside the one in LDS.  Chunk c of
+  // an operand tile whose first row is `first` of `rows`; addresses are clamped
+  // into the operand, what lies past the end of k becomes 0 on its way into LDS.
+  uint4 areg[PF][Cfg::A_CHUNKS], breg[PF][Cfg::B_CHUNKS];
+  auto load_chunk = [&](const float* src, int c, int first, int rows, int k0) {
+    const int r = c / CPR, off = (c % CPR) * 4;
+    return *reinterpret_cast<const uint4*>(
+        src + (int64_t)min(first + r, rows - 1) * K + min(k0 + off, K - 4));
+  };
+  auto load_global = [&](int k0, auto slot_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+#pragma unroll
+    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
+      areg[SLOT][i] = load_chunk(Ae, tid + i * Cfg::THREADS, row0, R, k0);
+#pragma unroll
+    for (int i = 0; i < Cfg::B_CHUNKS; ++i)
+      breg[SLOT][i] = load_chunk(Be, tid + i * Cfg::THREADS, col0, N, k0);
+  };
+  auto store_chunk = [&](float* dst, int c, uint4 v, int k0) {
+    const int r = c / CPR, off = (c % CPR) * 4;
+    if (k0 + BK > K && k0 + off >= K) v = make_uint4(0, 0, 0, 0);
+    *reinterpret_cast<uint4*>(dst + r * LDR + off) = v;
+  };
+  auto store_lds = [&](int buf, int k0, auto slot_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+#pragma unroll
+    for (int i = 0; i < Cfg::A_CHUNKS; ++i)
+      store_chunk(As + buf * Cfg::STAGE_A, tid + i * Cfg::THREADS, areg[SLOT][i],
+                  k0);
+#pragma unroll
+    for (int i = 0; i < Cfg::B_CHUNKS; ++i)
+      store_chunk(Bs + buf * Cfg::STAGE_B, tid + i * Cfg::THREADS, breg[SLOT][i],
+                  k0);
+  };
+
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+  const int nk = (K + BK - 1) / BK;
+  // where this lane's operands start: a row and four k, of its wavefront's k
+  constexpr int US = BK / 8 / WK;                  // groups of 8 k a wavefront
+  const int frag_row = lane & 31, frag_k = (lane >> 5) * 4 + wk * US * 8;
+  const int a_at = (wm * 32 * TM + frag_row) * LDR + frag_k;
+  const int b_at = (wn * 32 * TN + frag_row) * LDR + frag_k;
+  auto fragment = [&](const float* src, int tile, int u) {
+    return *reinterpret_cast<const float4*>(src + tile * 32 * LDR + u * 8);
+  };
+  auto step = [&](int kt, auto slot_c) {
+    const int buf = kt & 1;
+    // (the other stage may still be read by wavefronts one step behind; this
+    // one's readers passed the barrier of the step before)
+    store_lds(buf, kt * BK, slot_c);
+    load_global((kt + PF) * BK, slot_c);
+    // the LDS writes of every wavefront are done; the loads stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const float* as = As + buf * Cfg::STAGE_A + a_at;
+    const float* bs = Bs + buf * Cfg::STAGE_B + b_at;
+#pragma unroll
+    for (int u = 0; u < US; ++u) {
+      float4 af[TM], bfr[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) af[i] = fragment(as, i, u);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) bfr[j] = fragment(bs, j, u);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const float a = q == 0 ? af[i].x : q == 1 ? af[i].y
+                            : q == 2 ? af[i].z : af[i].w;
+            const float b = q == 0 ? bfr[j].x : q == 1 ? bfr[j].y
+                            : q == 2 ? bfr[j].z : bfr[j].w;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b, a, acc[i][j],
+                                                             0, 0, 0);
+          }
+      }
+    }
+  };
+  load_global(0, std::integral_constant<int, 0>());
+  load_global(BK, std::integral_constant<int, 1>());
+  if constexpr (PF > 2) load_global(2 * BK, std::integral_constant<int, PF - 1>());
+  for (int kt = 0; kt < nk; kt += PF) {
+    step(kt, std::integral_constant<int, 0>());
+    if (kt + 1 < nk) step(kt + 1, std::integral_constant<int, 1>());
+    if constexpr (PF > 2)
+      if (kt + 2 < nk) step(kt + 2, std::integral_constant<int, PF - 1>());
+  }
+  if constexpr (WK > 1) {
+    // [wk - 1][sub-tile][TM][TN][16][64], where the stages were
+    __syncthreads();
+    float* parts = reinterpret_cast<float*>(smem_raw);
+    constexpr int SUB = TM * TN * 1024, PLANE = WM * WN * SUB;
+    if (wk > 0) {
+      float* dst = parts + (wk - 1) * PLANE + wmn * SUB + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            dst[((i * TN + j) * 16 + r) * 64] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int w = 0; w < WK - 1; ++w) {
+      const float* src = parts + w * PLANE + wmn * SUB + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] += src[((i * TN + j) * 16 + r) * 64];
+    }
+  }
+  const int m_l = lane & 31, n_l = (lane >> 5) * 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int grow = row0 + (wm * TM + i) * 32 + m_l;
+        const int gcol = col0 + (wn * TN + j) * 32 + 8 * q + n_l;
+        if (grow < R && gcol < N) {
+          float4 v = make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
+                                 acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+          const int64_t at = (int64_t)grow * N + gcol;
+          if (relu) {
+            v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f);
+            v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f);
+          }
+          *reinterpret_cast<float4*>(Ce + at) = v;
+        }
+      }
+}
+
+template <int TM, int TN, int WM, int WN, int WK>
+static int launch_f32_mfma_tile(const float* A, const float* B, float* C, int E,
+                                int R, int N, int K, bool relu, hipStream_t st) {
+  using Cfg = F32Cfg<TM, TN, WM, WN, WK>;
+  const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
+  const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  const int64_t blocks = (int64_t)tiles_m * tiles_n * E;
+  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: too many tiles (%lld)", (long long)blocks);
+  auto k = grouped_gemm_f32_mfma_kernel<TM, TN, WM, WN, WK>;
+  MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
+  k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
+      A, B, C, R, N, K, tiles_m, tiles_n, relu ? 1 : 0);
+  MOE_CHECK_LAUNCH("expert_ffn (float32 mfma)");
+  return 0;
+}
+
+// Block tile of the float32 kernel.  The kernel is bound by the float32 matrix
+// pipes (a 32 x 32 x 2 MFMA takes 64 cycles), so its time is rounds of tiles
+// over the compute units times the tile's area; small launches want small tiles
+// (less padding of the row count, fewer idle compute units in the last round).
+// The smallest two pay for it with more LDS and cache traffic per product: the
+// weights.  Measured at 8 experts x 320 rows, per launch (us), in the order of
+// the table: 512 -> 2048 83, 71, 62, 67, 73; 2048 -> 512 151, 85, 85, 73, 67.
+int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int N,
+                    int K, bool relu, hipStream_t st) {
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  static const int shapes[5][2] = {{128, 128}, {64, 128}, {64, 64}, {32, 64},
+                                   {32, 32}};
+  static const double weight[5] = {1.0, 1.0, 1.0, 1.08, 1.18};
+  int best = 0;
+  double best_cost = 0;
+  int64_t best_tiles = 0;
+  for (int i = 0; i < 5; ++i) {
+    const int bm = shapes[i][0], bn = shapes[i][1];
+    const int64_t tiles = (int64_t)E * ((R + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const double cost = (double)((tiles + cus - 1) / cus) * bm * bn * weight[i];
+    // a smaller tile when it saves time by this count, or costs the same while
+    // the larger one leaves compute units with fewer than two blocks to overlap
+    if (i == 0 || cost < 0.95 * best_cost ||
+        (cost <= best_cost && best_tiles < 2 * (int64_t)cus)) {
+      best = i;
+      best_cost = cost;
+      best_tiles = tiles;
+    }
+  }
+#define MOE_F32_TILE(...)                                                      \
+  launch_f32_mfma_tile<__VA_ARGS__>(A, B, C, E, R, N, K, relu, st)
+  switch (best) {
+    case 0: return MOE_F32_TILE(2, 2, 2, 2, 1);
+    case 1: return MOE_F32_TILE(1, 2, 2, 2, 1);
+    case 2: return MOE_F32_TILE(1, 1, 2, 2, 1);
+    case 3: return MOE_F32_TILE(1, 1, 1, 2, 2);
+    default: return MOE_F32_TILE(1, 1, 1, 1, 4);
+  }
+#undef MOE_F32_TILE
+}
+
 }  // namespace mesh_moe

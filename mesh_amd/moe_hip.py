@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 35
+ABI_VERSION = 36
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -81,6 +81,9 @@ _SIGNATURES = {
         _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp]),
     "mesh_moe_expert_ffn": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
+    "mesh_moe_expert_ffn_kept": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
     "mesh_moe_dispatched_expert_ffn_workspace_bytes": (ctypes.c_size_t, [
@@ -824,6 +827,8 @@ def expert_ffn(expert_in, wi_packed, wo_packed, activation="relu", h=None,
   ip = _dev(expert_in, "expert_in")
   wip = _dev(wi_packed, "wi_packed", dt, (e, hdim, m))
   wop = _dev(wo_packed, "wo_packed", dt, (e, n, hdim))
+  # a caller that brings h keeps it, for a gradient
+  call = lib.mesh_moe_expert_ffn if h is None else lib.mesh_moe_expert_ffn_kept
   if h is None:
     h = torch.empty((e, rows, hdim), dtype=dt, device=expert_in.device)
   if y is None:
@@ -831,9 +836,8 @@ def expert_ffn(expert_in, wi_packed, wo_packed, activation="relu", h=None,
   hp = _dev(h, "h", dt, (e, rows, hdim))
   yp = _dev(y, "y", dt, (e, rows, n))
   with _stage("expert_ffn"):
-    _check(lib.mesh_moe_expert_ffn(ip, wip, wop, hp, yp, e, rows, m, hdim, n,
-                                   ACTIVATIONS[activation], code, _stream()),
-           "expert_ffn")
+    _check(call(ip, wip, wop, hp, yp, e, rows, m, hdim, n,
+                ACTIVATIONS[activation], code, _stream()), "expert_ffn")
   return y
 
 
