@@ -13,96 +13,129 @@
 namespace mesh_moe {
 
 // ---------------------------------------------------------------------------
-// Router logits: logits[b,t,e] = sum_m x[b,t,m] * w[b,m,e] (+ bias[e]).
-// One block = TOK tokens; thread (tok = tid % TOK, eg = tid / TOK) accumulates
-// experts eg*ept .. eg*ept+ept-1 with ept = ceil(E / (256 / TOK)) <= 32, in the
-// order of m.  x and w are staged through LDS as float32 in chunks of KC columns
-// of M; the next chunk is loaded while one is multiplied.
+// Router logits: logits[b,t,e] = sum_m x[b,t,m] * w[b,m,e] (+ bias[e]), float32
+// multiply-adds in the order of m.
 //
-// Bound by the latency of that chain of chunks: blocks of 64 tokens are kept
-// for calls that fill the compute units with them, smaller calls take 16 tokens
-// a block.  2048 tokens x 512, 8 experts, float32: 22.9 -> 11.5 us.
+// A wavefront makes 16 tokens x 16 experts on v_mfma_f32_16x16x4_f32, which
+// adds its four products one after the other: the sums have the bits of fmaf in
+// the order of m.  Operands come straight from memory, PF groups of 16 columns
+// ahead; the wavefronts of a block share the token rows, one expert tile each.
+// VEC: a lane loads four consecutive columns of its token and the four lanes that
+// hold a token's 16 trade them (the MFMA wants column 4 j + lane / 16).
+//
+// Bound by the chain of MFMAs, 8 cycles per column, and the first loads.  Measured
+// (us), in brackets one thread per token and a few experts with the operands
+// through LDS, which waited for every LDS read: 2048 tokens x 512, 8 experts 7.0
+// (11.8), 64 experts 9.3 (43); 64 x 1024, 64 experts 13.5 (82); 16384 x 1024, 128
+// experts 88 (577); 4000 x 320, 24 experts 6.6 (16.6); bf16, 20000 x 700, 64 experts
+// 38 (259).
 // ---------------------------------------------------------------------------
-constexpr int RL_KC = 64;
-constexpr int RL_MAX_EPT = 32;
+constexpr int RL_MAX_EXPERTS = 128;      // of a router_logits call
+typedef __attribute__((ext_vector_type(4))) float rl_f32x4_t;
 
-// EPT: experts per thread, a power of two >= ept (the loop over a thread's
-// experts is unrolled without conditions: with EPT = 32 and a condition per
-// expert the 64 x 32 scalar branches per chunk were the whole run time at
-// E = 8; the surplus products read the next group's weights and are dropped)
-template <typename T, int EPT, int TOK>
+template <typename T>
+__device__ __forceinline__ void load_f32x4(const T* p, float (&v)[4]);
+template <>
+__device__ __forceinline__ void load_f32x4<float>(const float* p,
+                                                  float (&v)[4]) {
+  const float4 q = *reinterpret_cast<const float4*>(p);
+  v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+template <>
+__device__ __forceinline__ void load_f32x4<bf16_t>(const bf16_t* p,
+                                                   float (&v)[4]) {
+  const uint2 q = *reinterpret_cast<const uint2*>(p);
+  v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+  v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+}
+
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void router_logits_kernel(
     const T* __restrict__ x, const T* __restrict__ w,
     const float* __restrict__ bias, float* __restrict__ logits,
-    int64_t tokens, int M, int E, int ept) {
-  constexpr int GROUPS = 256 / TOK;
-  constexpr int XV = TOK * RL_KC / 256;            // loads per thread and chunk
-  constexpr int WV = EPT * GROUPS * RL_KC / 256;
-  extern __shared__ float smem[];
-  float* xs = smem;                       // [TOK][RL_KC + 1]
-  float* ws = smem + TOK * (RL_KC + 1);   // [RL_KC][E] + GROUPS EPT
-  const int b = blockIdx.y;
-  const int64_t t0 = (int64_t)blockIdx.x * TOK;
-  const int tid = threadIdx.x;
-  const int tok = tid % TOK;
-  const int eg = tid / TOK;
-  const T* xb = x + ((int64_t)b * tokens) * M;
-  const T* wb = w + (int64_t)b * M * E;
-  const int wn = RL_KC * E;               // weights of a chunk, contiguous
-  float acc[EPT];
+    int64_t tokens, int M, int E) {
+  constexpr int PF = 8;
+  const int b = blockIdx.z;
+  const int64_t t0 = (int64_t)blockIdx.x * 16;
+  const int lane = threadIdx.x & 63, col = lane & 15, h = lane >> 4;
+  const int e0 = (blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 16;
+  if (e0 >= E) return;
+  // tokens and experts past the end are read as the last ones, not stored
+  const T* xt = x + ((int64_t)b * tokens + min(t0 + col, tokens - 1)) * M;
+  const T* we = w + (int64_t)b * M * E + min(e0 + col, E - 1);
+  float xr[PF][4], wr[PF][4];
+  // a group of 16 columns: WHOLE, or with what lies past M clamped
+  const T* xh = xt + (VEC ? 4 * h : h);
+  const T* wh = we + (int64_t)h * E;
+  auto load = [&](int k0, float (&xv)[4], float (&wv)[4], auto whole_c) {
+    constexpr bool WHOLE = decltype(whole_c)::value;
+    if (VEC) {
+      load_f32x4<T>(WHOLE ? xh + k0 : xt + min(k0 + 4 * h, M - 4), xv);
+    } else {
 #pragma unroll
-  for (int j = 0; j < EPT; ++j) acc[j] = 0.f;
-
-  // all loads of a chunk are issued together (one at a time, each waited for,
-  // the staging took 30 us per chunk)
-  float xv[XV], wv[WV];
-  auto load = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < XV; ++u) {
-      const int i = tid + u * 256;
-      const int64_t t = t0 + i / RL_KC;
-      const int c = k0 + i % RL_KC;
-      xv[u] = (t < tokens && c < M) ? load_f32<T>(xb + t * M + c) : 0.f;
+      for (int j = 0; j < 4; ++j)
+        xv[j] = load_f32<T>(WHOLE ? xh + k0 + 4 * j
+                                  : xt + min(k0 + 4 * j + h, M - 1));
     }
-    const int left = (int)min((int64_t)wn, (int64_t)(M - k0) * E);
 #pragma unroll
-    for (int u = 0; u < WV; ++u) {
-      const int i = tid + u * 256;
-      wv[u] = i < left ? load_f32<T>(wb + (int64_t)k0 * E + i) : 0.f;
+    for (int j = 0; j < 4; ++j)
+      wv[j] = load_f32<T>(WHOLE ? wh + (int64_t)(k0 + 4 * j) * E
+                                : we + (int64_t)min(k0 + 4 * j + h, M - 1) * E);
+  };
+  rl_f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int k0, float (&xv)[4], float (&wv)[4], auto whole_c) {
+    constexpr bool WHOLE = decltype(whole_c)::value;
+    if (VEC) {
+      auto swap = [](auto fn, float& p, float& q) {
+        const auto r = fn(__float_as_uint(p), __float_as_uint(q));
+        p = __uint_as_float(r[0]);
+        q = __uint_as_float(r[1]);
+      };
+      auto swap32 = [](uint32_t p, uint32_t q) {
+        return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+      };
+      auto swap16 = [](uint32_t p, uint32_t q) {
+        return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+      };
+      swap(swap32, xv[0], xv[2]);
+      swap(swap32, xv[1], xv[3]);
+      swap(swap16, xv[0], xv[1]);
+      swap(swap16, xv[2], xv[3]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool in = WHOLE || k0 + 4 * j + h < M;      // past M: 0 * 0
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? wv[j] : 0.f,
+                                                 in ? xv[j] : 0.f, acc, 0, 0, 0);
     }
   };
-  load(0);
-  for (int k0 = 0; k0 < M; k0 += RL_KC) {
+  using Whole = std::true_type;
+  using Rest = std::false_type;
 #pragma unroll
-    for (int u = 0; u < XV; ++u) {
-      const int i = tid + u * 256;
-      xs[(i / RL_KC) * (RL_KC + 1) + i % RL_KC] = xv[u];
-    }
+  for (int u = 0; u < PF; ++u) load(u * 16, xr[u], wr[u], Rest());
+  int k0 = 0;
+  for (; k0 + 32 * PF <= M; k0 += 16 * PF) {
 #pragma unroll
-    for (int u = 0; u < WV; ++u) {
-      const int i = tid + u * 256;
-      if (i < wn) ws[i] = wv[u];
+    for (int u = 0; u < PF; ++u) {
+      multiply(k0 + 16 * u, xr[u], wr[u], Whole());
+      load(k0 + 16 * (u + PF), xr[u], wr[u], Whole());
     }
-    __syncthreads();
-    if (k0 + RL_KC < M) load(k0 + RL_KC);
-    const int e0 = eg * ept;
-#pragma unroll 8
-    for (int k = 0; k < RL_KC; ++k) {
-      float xk = xs[tok * (RL_KC + 1) + k];
-      const float* wr = ws + k * E + e0;
-#pragma unroll
-      for (int j = 0; j < EPT; ++j) acc[j] = fmaf(xk, wr[j], acc[j]);
-    }
-    __syncthreads();
   }
-  int64_t t = t0 + tok;
-  if (t < tokens) {
-    float* out = logits + ((int64_t)b * tokens + t) * E;
+  for (; k0 < M; k0 += 16 * PF) {
 #pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      int e = eg * ept + j;
-      if (j < ept && e < E) out[e] = bias ? acc[j] + bias[e] : acc[j];
+    for (int u = 0; u < PF; ++u) {
+      if (k0 + 16 * u < M) multiply(k0 + 16 * u, xr[u], wr[u], Rest());
+      if (k0 + 16 * (u + PF) < M)
+        load(k0 + 16 * (u + PF), xr[u], wr[u], Rest());
     }
+  }
+  const int64_t t = t0 + col;
+  if (t >= tokens) return;
+  float* out = logits + ((int64_t)b * tokens + t) * E;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int e = e0 + 4 * h + r;
+    if (e < E) out[e] = bias ? acc[r] + bias[e] : acc[r];
   }
 }
 
@@ -1748,8 +1781,8 @@ extern "C" int mesh_moe_router_logits(const void* x, const void* w,
   MOE_REQUIRE(batch >= 1 && tokens >= 0 && M >= 1 && E >= 1, MESH_MOE_E_ARG,
               "router_logits: bad sizes batch=%d tokens=%lld M=%d E=%d", batch,
               (long long)tokens, M, E);
-  MOE_REQUIRE(E <= 4 * RL_MAX_EPT, MESH_MOE_E_UNSUPPORTED,
-              "router_logits: E=%d > %d", E, 4 * RL_MAX_EPT);
+  MOE_REQUIRE(E <= RL_MAX_EXPERTS, MESH_MOE_E_UNSUPPORTED,
+              "router_logits: E=%d > %d", E, RL_MAX_EXPERTS);
   MOE_REQUIRE(batch <= 65535, MESH_MOE_E_UNSUPPORTED,
               "router_logits: batch=%d > 65535", batch);
   if (tokens == 0) return 0;
@@ -1765,49 +1798,24 @@ extern "C" int mesh_moe_router_logits(const void* x, const void* w,
       return launch_router_mfma<2>(xb, wp, bias, logits, batch, (int)tokens, M, E, s2);
     return launch_router_mfma<4>(xb, wp, bias, logits, batch, (int)tokens, M, E, s2);
   }
-  const int cus = compute_units();
-  if (cus == 0) return MESH_MOE_E_HIP;
-  const int tok = (tokens + 63) / 64 * batch < cus ? 16 : 64;
-  const int groups = 256 / tok;
-  const int ept = (E + groups - 1) / groups;
-  dim3 grid((unsigned)((tokens + tok - 1) / tok), (unsigned)batch);
-  int eptp = 1;
-  while (eptp < ept) eptp *= 2;
-  size_t smem = sizeof(float) * (tok * (RL_KC + 1) + (size_t)RL_KC * E +
-                                 groups * eptp);
+  const int tiles = (E + 15) / 16, waves = tiles < 4 ? tiles : 4;
+  const int64_t blocks = (tokens + 15) / 16;
+  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+              "router_logits: too many tokens (%lld)", (long long)tokens);
+  dim3 grid((unsigned)blocks, (unsigned)((tiles + waves - 1) / waves),
+            (unsigned)batch);
   hipStream_t st = (hipStream_t)stream;
-#define MOE_ROUTER_LOGITS(T, P, TOK)                                           \
-  do {                                                                         \
-    auto kern = router_logits_kernel<T, P, TOK>;                               \
-    MOE_ALLOW_LDS(kern, smem);                                                 \
-    kern<<<grid, 256, smem, st>>>((const T*)x, (const T*)w, bias, logits,      \
-                                  tokens, M, E, ept);                          \
-  } while (0)
-#define MOE_ROUTER_LOGITS_T(T)                                                 \
-  if (tok == 16) {                                                             \
-    switch (eptp) {                                                            \
-      case 1: MOE_ROUTER_LOGITS(T, 1, 16); break;                              \
-      case 2: MOE_ROUTER_LOGITS(T, 2, 16); break;                              \
-      case 4: MOE_ROUTER_LOGITS(T, 4, 16); break;                              \
-      default: MOE_ROUTER_LOGITS(T, 8, 16); break;                             \
-    }                                                                          \
-  } else {                                                                     \
-    switch (eptp) {                                                            \
-      case 1: MOE_ROUTER_LOGITS(T, 1, 64); break;                              \
-      case 2: MOE_ROUTER_LOGITS(T, 2, 64); break;                              \
-      case 4: MOE_ROUTER_LOGITS(T, 4, 64); break;                              \
-      case 8: MOE_ROUTER_LOGITS(T, 8, 64); break;                              \
-      case 16: MOE_ROUTER_LOGITS(T, 16, 64); break;                            \
-      default: MOE_ROUTER_LOGITS(T, 32, 64); break;                            \
-    }                                                                          \
-  }
-  if (dtype == MESH_MOE_F32) {
-    MOE_ROUTER_LOGITS_T(float);
-  } else {
-    MOE_ROUTER_LOGITS_T(bf16_t);
-  }
-#undef MOE_ROUTER_LOGITS_T
-#undef MOE_ROUTER_LOGITS
+  const bool vec = M % 4 == 0 && (uintptr_t)x % (4 * dtype_size(dtype)) == 0;
+  auto run = [&](auto kern, const auto* xp, const auto* wp) {
+    kern<<<grid, 64 * waves, 0, st>>>(xp, wp, bias, logits, tokens, M, E);
+  };
+  if (dtype == MESH_MOE_F32)
+    run(vec ? router_logits_kernel<float, true> : router_logits_kernel<float, false>,
+        (const float*)x, (const float*)w);
+  else
+    run(vec ? router_logits_kernel<bf16_t, true>
+            : router_logits_kernel<bf16_t, false>,
+        (const bf16_t*)x, (const bf16_t*)w);
   MOE_CHECK_LAUNCH("router_logits");
   return 0;
 }

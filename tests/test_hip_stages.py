@@ -117,6 +117,27 @@ def test_gating_second_policy(hip, policy):
   np.testing.assert_allclose(got["loss"], want["loss"], rtol=2e-5)
 
 
+# token, expert and column counts around the 16 x 16 tiles, the groups of 16
+# columns and the 128 that are on their way, rows of 16-byte pieces and others
+@pytest.mark.parametrize("shape", [
+    (1, 1, 1, 2), (1, 15, 3, 16), (1, 17, 15, 17), (2, 33, 17, 3), (1, 16, 130, 64),
+    (3, 5, 128, 128), (1, 1000, 255, 33), (1, 40, 256, 8), (2, 70, 260, 100),
+    (1, 31, 516, 15), (1, 300, 63, 1)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_router_logits_edges(hip, shape, dtype):
+  b, t, m, e = shape
+  gen = torch.Generator(device="cuda").manual_seed(sum(shape))
+  x = torch.randn((b, t, m), generator=gen, device="cuda").to(H.ACT_TORCH[dtype])
+  w = torch.randn((b, m, e), generator=gen, device="cuda").to(H.ACT_TORCH[dtype])
+  bias = torch.randn((e,), generator=gen, device="cuda")
+  got = hip.router_logits(x, w, bias).double()
+  want = x.double() @ w.double() + bias.double()
+  # a rounding per column and one for the bias
+  bound = (m + 1) * 2.0 ** -24 * (
+      x.double().abs() @ w.double().abs() + bias.double().abs())
+  assert ((got - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(2, 1024, 512, 8), (3, 100, 72, 5),
                                    (1, 640, 1024, 128), (1, 15, 4, 17),
