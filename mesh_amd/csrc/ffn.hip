@@ -1141,6 +1141,32 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
       }
     }
+    // staging row -> row of the output
+    auto out_row = [&](int pass, int srow) {
+      return out_row0 + (srow >> 6) * (TAILS ? 32 * out_pieces0 : 128) +
+             pass * 64 + (srow & 63);
+    };
+    // MASKED: the mask of a pass's pieces, all loads together and ahead of the
+    // staging.  (In front of its store, each was waited for by itself: what the
+    // mask costs a launch of 64 x 2048 rows, 1024 x 4096, is 108 us instead of 232,
+    // 16000 rows, 768 x 3072, 4 instead of 13.  Touching the mask's lines two K
+    // tiles earlier, for the L2, costs twice what it saves.)
+    constexpr int PIECES = EPI_ROWS * CPR_C / Cfg::THREADS;
+    u32x4_t mask[MASKED ? PIECES : 1];
+    auto load_mask = [&](int pass) {
+      if constexpr (MASKED) {
+        int m_tid = tid;
+        asm volatile("" : "+v"(m_tid));
+        const bf16_t* m = mask_src + (out_c - Cout) +
+                          min(out_col0 + m_tid % CPR_C * 8, N - 8);
+#pragma unroll
+        for (int n = 0; n < PIECES; ++n)
+          mask[n] = *reinterpret_cast<const u32x4_t*>(
+              m + (int64_t)min(out_row(pass, m_tid / CPR_C + 16 * n), R - 1) * N);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    load_mask(0);
     if (has_next) {
       // the next tile's first loads fly while this tile is written out
       set_tile(next);
@@ -1204,7 +1230,6 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       }
       lds_barrier();
       // all staged pieces of this pass first, one wait, then the stores
-      constexpr int PIECES = EPI_ROWS * CPR_C / Cfg::THREADS;
       static_assert(EPI_ROWS * CPR_C % Cfg::THREADS == 0, "whole pieces");
       u32x4_t piece[PIECES];
       // piece n: staging row (e_tid / CPR_C) + 16 n
@@ -1217,10 +1242,9 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       for (int n = 0; n < PIECES; ++n) {
         const int c = e_tid + n * Cfg::THREADS;
         const int srow = c / CPR_C, chunk = c % CPR_C;
-        // staging row -> tile row: 64 rows of each half of the tile
+        // 64 rows of each half of the tile
         const int half_row = pass * 64 + (srow & 63);
-        const int grow =
-            out_row0 + (srow >> 6) * (TAILS ? 32 * out_pieces0 : 128) + half_row;
+        const int grow = out_row(pass, srow);
         const int gcol = out_col0 + chunk * 8;
         // (TAILS: a half's rows past its pieces belong to the other half or to
         // the next tile)
@@ -1228,8 +1252,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
             !(TAILS && srow < 64 && half_row >= 32 * out_pieces0)) {
           u32x4_t v = piece[n];
           if constexpr (MASKED) {
-            const u32x4_t hm = *reinterpret_cast<const u32x4_t*>(
-                mask_src + (out_c - Cout) + (int64_t)grow * N + gcol);
+            const u32x4_t hm = mask[n];
             if (mask_scale != 1.0f) {
 #pragma unroll
               for (int q = 0; q < 4; ++q)
@@ -1249,6 +1272,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
           *reinterpret_cast<u32x4_t*>(out_c + (int64_t)grow * N + gcol) = v;
         }
       }
+      if (pass == 0) load_mask(1);
       lds_barrier();
     }
     if (!has_next) break;
