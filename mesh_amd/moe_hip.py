@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 36
+ABI_VERSION = 37
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -212,6 +212,12 @@ _SIGNATURES = {
     "mesh_moe_slot_combine": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
+    "mesh_moe_residual_rms_norm": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
+        ctypes.c_double, ctypes.c_int, _vp]),
+    "mesh_moe_residual_rms_norm_backward": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
+        ctypes.c_double, ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
     "mesh_moe_rms_norm": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int, ctypes.c_double,
         ctypes.c_int, _vp]),
@@ -1403,6 +1409,35 @@ def rms_norm(x, scale, epsilon=1e-6):
   return out
 
 
+def residual_rms_norm_supported(x):
+  """True if residual_rms_norm and the mask / addend of rms_norm_backward have a
+  kernel for rows like x's."""
+  m = x.shape[-1]
+  return (x.dtype == torch.bfloat16 and m % 8 == 0 and m <= 4096 and
+          x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def residual_rms_norm(x, residual, scale, epsilon=1e-6, row_mask=None):
+  """rms_norm(x + residual) * row_mask in one pass: x, residual (or None) [..., M],
+  row_mask [...] (or None) -> (x + residual or x itself, result)."""
+  lib = load_library()
+  m = x.shape[-1]
+  rows = x.numel() // m
+  shape = tuple(x.shape)
+  total = x if residual is None else torch.empty_like(x)
+  out = torch.empty_like(x)
+  with _stage("rms_norm"):
+    _check(lib.mesh_moe_residual_rms_norm(
+        _dev(x, "x"),
+        None if residual is None else _dev(residual, "residual", x.dtype, shape),
+        _dev(scale, "scale", x.dtype, (m,)),
+        None if row_mask is None else _dev(row_mask, "row_mask", x.dtype,
+                                           shape[:-1]),
+        None if residual is None else total.data_ptr(), out.data_ptr(), rows, m,
+        float(epsilon), dtype_code(x.dtype), _stream()), "residual_rms_norm")
+  return total, out
+
+
 def dense(x, w_packed, activation=None):
   """x [..., K] times a packed kernel [1, N, K] -> [..., N]
   (mtf.layers.dense without bias: one einsum, ops.py / layers.py:112-160)."""
@@ -1585,8 +1620,10 @@ def expert_choice_backward(logits, r, dweight, d_loss, loss_scale,
 
 
 # ---- backward of the block's operations ----------------------------------------
-def rms_norm_backward(x, scale, dy, epsilon=1e-6):
-  """Backward of rms_norm: x, dy [..., M], scale [M] -> (dx, dscale)."""
+def rms_norm_backward(x, scale, dy, epsilon=1e-6, row_mask=None, addend=None):
+  """Backward of rms_norm: x, dy [..., M], scale [M] -> (dx, dscale).  row_mask
+  [...]: dy is multiplied by it first; addend [..., M] is added to dx (both where
+  residual_rms_norm_supported)."""
   lib = load_library()
   m = x.shape[-1]
   rows = x.numel() // m
@@ -1596,11 +1633,18 @@ def rms_norm_backward(x, scale, dy, epsilon=1e-6):
   ws_bytes = lib.mesh_moe_rms_norm_backward_workspace_bytes(rows, m)
   ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device)
   with _stage("rms_norm_backward"):
-    _check(lib.mesh_moe_rms_norm_backward(
-        _dev(x, "x"), _dev(scale, "scale", dt, (m,)),
-        _dev(dy, "dy", dt, tuple(x.shape)), dx.data_ptr(), dscale.data_ptr(),
-        rows, m, float(epsilon), dtype_code(dt), ws.data_ptr(), ws_bytes,
-        _stream()), "rms_norm_backward")
+    shape = tuple(x.shape)
+    tail = (dx.data_ptr(), dscale.data_ptr(), rows, m, float(epsilon),
+            dtype_code(dt), ws.data_ptr(), ws_bytes, _stream())
+    ops = (_dev(x, "x"), _dev(scale, "scale", dt, (m,)), _dev(dy, "dy", dt, shape))
+    if row_mask is None and addend is None:
+      rc = lib.mesh_moe_rms_norm_backward(*ops, *tail)
+    else:
+      rc = lib.mesh_moe_residual_rms_norm_backward(
+          *ops,
+          None if row_mask is None else _dev(row_mask, "row_mask", dt, shape[:-1]),
+          None if addend is None else _dev(addend, "addend", dt, shape), *tail)
+    _check(rc, "rms_norm_backward")
   return dx, dscale
 
 

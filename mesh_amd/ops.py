@@ -619,6 +619,9 @@ class Lowering(object):
     # change, and every step checks every tensor against it
     self._slice_shapes = {}
     self.scalar_summaries = {}   # {name: 0-d torch tensor} of the last run
+    # Operations whose outputs this run already holds, because an operation in
+    # front of them made them in the same kernel
+    self.done_ahead = set()
     for op in graph.operations:
       op.lower(self)
       for out in op.outputs:
@@ -631,6 +634,7 @@ class Lowering(object):
     imported Tensors to new torch tensors of the same shape."""
     self._feeds = dict(feeds or {})
     self.scalar_summaries = {}
+    self.done_ahead = set()
     try:
       for op in self.graph.operations:
         if not isinstance(op, Variable):
@@ -1178,7 +1182,12 @@ def gradients(ys, xs, grad_ys=None, operations=None):
           for inp, grad in zip(op.inputs, input_grads):
             if inp in downstream and grad is not None:
               if inp in tensor_to_gradient:
-                tensor_to_gradient[inp] = tensor_to_gradient[inp] + grad
+                # (an operation that can add to its result while it writes it)
+                add_to = getattr(grad.operation, "add_to_output", None)
+                total = add_to(grad, tensor_to_gradient[inp]) if add_to else None
+                if total is None:
+                  total = tensor_to_gradient[inp] + grad
+                tensor_to_gradient[inp] = total
               else:
                 tensor_to_gradient[inp] = grad
   finally:

@@ -1657,3 +1657,105 @@ def test_layer_stack_gradients_bfloat16_follow_float32():
     assert np.isfinite(g).all(), name
     cos = float(g @ w / (np.linalg.norm(g) * np.linalg.norm(w) + 1e-30))
     assert cos > 0.97, (name, cos)
+
+
+# rows around the four of a block and the wavefronts' strides, columns around the
+# 512 a wavefront takes at once, the shortest and the longest row
+@pytest.mark.parametrize("rows,m", [(1, 8), (3, 504), (4, 512), (5, 520),
+                                    (2049, 768), (33, 1024), (7, 1032),
+                                    (9, 2048), (10, 3592), (2, 4096)])
+@pytest.mark.parametrize("with_residual", [True, False])
+@pytest.mark.parametrize("with_mask", [True, False])
+def test_residual_rms_norm_and_backward(hip, rows, m, with_residual, with_mask):
+  """The same bits as the sum, the norm, the mask and their gradients one after
+  the other."""
+  gen = torch.Generator(device="cuda").manual_seed(rows + m)
+
+  def draw(*sizes):
+    return torch.randn(sizes, generator=gen, device="cuda").bfloat16()
+  x, residual, scale, dy, addend = (draw(rows, m), draw(rows, m), draw(m),
+                                    draw(rows, m), draw(rows, m))
+  mask = (torch.rand((rows,), generator=gen, device="cuda") < 0.7).bfloat16()
+  total, y = hip.residual_rms_norm(
+      x, residual if with_residual else None, scale,
+      row_mask=mask if with_mask else None)
+  want_total = x + residual if with_residual else x
+  want = hip.rms_norm(want_total, scale)
+  assert torch.equal(total, want_total)
+  assert torch.equal(y, want * mask[:, None] if with_mask else want)
+  dx, dscale = hip.rms_norm_backward(
+      x, scale, dy, row_mask=mask if with_mask else None,
+      addend=addend if with_residual else None)
+  want_dx, want_dscale = hip.rms_norm_backward(
+      x, scale, dy * mask[:, None] if with_mask else dy)
+  assert torch.equal(dx, addend + want_dx if with_residual else want_dx)
+  assert torch.equal(dscale, want_dscale)
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layer_stack_second_run(packed, dtype):
+  """The first run of a training step has no norm scales when the residual sums are
+  made and makes sums, norms and masks one by one; the later runs make them
+  together.  Same bits, in the intermediate tensors too, and new inputs count."""
+  b, l, m = 3, 40, 64
+  gen = torch.Generator(device="cuda").manual_seed(11)
+
+  def draw(*sizes):
+    return torch.randn(sizes, generator=gen, device="cuda").to(dtype)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("batch", b), mtf.Dimension("length", l),
+          mtf.Dimension("d_model", m)]
+  ids = torch.ones((b, l), dtype=torch.int32, device="cuda")
+  ids[0, 30:] = 0
+  ids[1, 10:25] = 2
+  x0, dy0 = draw(b, l, m), draw(b, l, m)
+  xt = mtf.import_tf_tensor(mesh, x0, mtf.Shape(dims))
+  dyt = mtf.import_tf_tensor(mesh, dy0, mtf.Shape(dims))
+  idt = mtf.import_tf_tensor(mesh, ids, mtf.Shape(dims[:2])) if packed else None
+  stack = transformer.make_layer_stack(
+      [(transformer_layers.SelfAttention, dict(num_heads=2, key_value_size=32)),
+       (transformer_layers.DenseReluDense, dict(hidden_size=96)),
+       (transformer_layers.DenseReluDense, dict(hidden_size=32))],
+      num_layers=1, block_scope=False)
+  model = transformer.Unitransformer(stack, d_model=m, name="decoder",
+                                     autoregressive=True)
+  y, _ = model.call_layers(xt, mtf.VariableDType(dtype, dtype, dtype),
+                           mode="train", sequence_id=idt)
+  wrt = [xt] + [v.outputs[0] for v in graph.trainable_variables]
+  grads = mtf.gradients([y], wrt, grad_ys=[dyt])
+  init = {}
+  for v in graph.all_variables:
+    sizes = v.shape.to_integer_list
+    init[v.name] = draw(*sizes) * (sizes[0] ** -0.5 if len(sizes) > 1 else 1.0)
+  lowering = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()}, initial_values=init)
+  tensors = [t for op in graph.operations for t in op.outputs
+             if not isinstance(op, mtf.Variable)]
+
+  def everything(low):
+    return {t: low.export_to_tf_tensor(t).clone() for t in tensors}
+  first = everything(lowering)
+  lowering.run()
+  assert lowering.done_ahead or dtype == torch.float32
+  second = everything(lowering)
+  for t in tensors:
+    assert torch.equal(first[t], second[t]), t
+  assert all(g in first for g in grads)
+  # other inputs, other ids: what a new program gives on them
+  feeds = {xt: draw(b, l, m), dyt: draw(b, l, m)}
+  if packed:
+    feeds[idt] = ids.flip(0).contiguous()
+  lowering.run(feeds)
+  third = everything(lowering)
+  for t, value in feeds.items():
+    t.operation._tf_tensor = value     # pylint: disable=protected-access
+  fresh = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()}, initial_values=init)
+  want = everything(fresh)
+  for t in tensors:
+    assert torch.equal(third[t], want[t]), t
+  # and a recorded step
+  step = lowering.capture()
+  step.replay(feeds)
+  for g in grads + [y]:
+    assert torch.equal(lowering.export_to_tf_tensor(g), want[g]), g
