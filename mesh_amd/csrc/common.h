@@ -35,7 +35,8 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
 // A[e] . B[e]^T (the operands and limits of f32_gemm) with sums whose bits do not
 // change from one version of f32_gemm to the next.
 int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int N,
-                    int K, bool relu, hipStream_t st);
+                    int K, bool relu, const float* mask_src, float mask_scale,
+                    hipStream_t st);
 
 // Fused self-attention (attention.hip): q, k, v, out [B,L,H*D] bf16.
 bool flash_attention_supported(int L, int H, int D, int dtype, const void* q,

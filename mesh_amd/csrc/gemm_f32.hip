@@ -520,7 +520,8 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
 // to 0.6 of the gradient's root mean square.  With other rounding a few units of a
 // step would switch, so that steps of two versions could not be compared; the more
 // exact kernel above is as good an answer, and not the same one.  (All other
-// products of a step are continuous in their operands and go there.)
+// products of a step are continuous in their operands and go there, short reductions
+// of little work excepted, which are faster here.)
 //
 // Four wavefronts; K step 32.  The weight tile is the MFMA's first operand, so a
 // lane ends up with 4 consecutive output columns per register group.  One MFMA
@@ -563,7 +564,7 @@ template <int TM, int TN, int WM, int WN, int WK>
 __global__ __launch_bounds__(256) void grouped_gemm_f32_mfma_kernel(
     const float* __restrict__ A, const float* __restrict__ B,
     float* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
-    int relu) {
+    int relu, const float* __restrict__ mask_src, float mask_scale) {
   using Cfg = F32Cfg<TM, TN, WM, WN, WK>;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
   constexpr int LDR = Cfg::LDR, CPR = Cfg::CPR, PF = Cfg::PF;
@@ -727,6 +728,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_mfma_kernel(
             v.x = fmaxf(v.x, 0.f); v.y = fmaxf(v.y, 0.f);
             v.z = fmaxf(v.z, 0.f); v.w = fmaxf(v.w, 0.f);
           }
+          if (mask_src != nullptr) {
+            const float4 m = *reinterpret_cast<const float4*>(
+                mask_src + (int64_t)e * R * N + at);
+            v = make_float4(finish_f32(v.x, false, true, m.x, mask_scale),
+                            finish_f32(v.y, false, true, m.y, mask_scale),
+                            finish_f32(v.z, false, true, m.z, mask_scale),
+                            finish_f32(v.w, false, true, m.w, mask_scale));
+          }
           *reinterpret_cast<float4*>(Ce + at) = v;
         }
       }
@@ -734,7 +743,9 @@ __global__ __launch_bounds__(256) void grouped_gemm_f32_mfma_kernel(
 
 template <int TM, int TN, int WM, int WN, int WK>
 static int launch_f32_mfma_tile(const float* A, const float* B, float* C, int E,
-                                int R, int N, int K, bool relu, hipStream_t st) {
+                                int R, int N, int K, bool relu,
+                                const float* mask_src, float mask_scale,
+                                hipStream_t st) {
   using Cfg = F32Cfg<TM, TN, WM, WN, WK>;
   const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
@@ -744,7 +755,7 @@ static int launch_f32_mfma_tile(const float* A, const float* B, float* C, int E,
   auto k = grouped_gemm_f32_mfma_kernel<TM, TN, WM, WN, WK>;
   MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
   k<<<(unsigned)blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
-      A, B, C, R, N, K, tiles_m, tiles_n, relu ? 1 : 0);
+      A, B, C, R, N, K, tiles_m, tiles_n, relu ? 1 : 0, mask_src, mask_scale);
   MOE_CHECK_LAUNCH("expert_ffn (float32 mfma)");
   return 0;
 }
@@ -757,7 +768,8 @@ static int launch_f32_mfma_tile(const float* A, const float* B, float* C, int E,
 // weights.  Measured at 8 experts x 320 rows, per launch (us), in the order of
 // the table: 512 -> 2048 83, 71, 62, 67, 73; 2048 -> 512 151, 85, 85, 73, 67.
 int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int N,
-                    int K, bool relu, hipStream_t st) {
+                    int K, bool relu, const float* mask_src, float mask_scale,
+                    hipStream_t st) {
   const int cus = compute_units();
   if (cus == 0) return MESH_MOE_E_HIP;
   static const int shapes[5][2] = {{128, 128}, {64, 128}, {64, 64}, {32, 64},
@@ -780,7 +792,8 @@ int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int 
     }
   }
 #define MOE_F32_TILE(...)                                                      \
-  launch_f32_mfma_tile<__VA_ARGS__>(A, B, C, E, R, N, K, relu, st)
+  launch_f32_mfma_tile<__VA_ARGS__>(A, B, C, E, R, N, K, relu, mask_src,       \
+                                    mask_scale, st)
   switch (best) {
     case 0: return MOE_F32_TILE(2, 2, 2, 2, 1);
     case 1: return MOE_F32_TILE(1, 2, 2, 2, 1);
