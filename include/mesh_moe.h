@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 37
+#define MESH_MOE_ABI_VERSION 38
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -391,6 +391,18 @@ int mesh_moe_combine_compact(const void* y, const int32_t* idx,
                              const uint8_t* kept, const int32_t* row_offsets,
                              void* out, int G, int S, int E, int C, int N,
                              int dtype, void* stream);
+
+/*
+ * mesh_moe_combine, or mesh_moe_combine_compact with row_offsets, and the layer's
+ * loss on the way (transformer/moe.py:526-529): loss [1] float32 -> loss_out [2] of
+ * dtype, the loss rounded to dtype and that times loss_coef (a value of dtype),
+ * rounded.
+ */
+int mesh_moe_combine_loss(const void* y, const int32_t* idx, const int32_t* pos,
+                          const float* gate, const uint8_t* kept,
+                          const int32_t* row_offsets, const float* loss,
+                          double loss_coef, void* out, void* loss_out, int G, int S,
+                          int E, int C, int N, int dtype, void* stream);
 
 /*
  * "No token left behind" gating (_ntlb_gating, transformer/moe.py:804-940)

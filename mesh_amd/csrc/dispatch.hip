@@ -178,13 +178,21 @@ __device__ __forceinline__ uint4 combine_vec<bf16_t>(uint4 a, uint4 b, float w1,
   return r;
 }
 
+// loss_out (null: none) [2]: the balancing loss rounded to T, and that times
+// loss_coef.  (By themselves they are two launches of one thread's work, 4 us each.)
 template <typename T>
 __global__ __launch_bounds__(256) void combine_kernel(
     const T* __restrict__ y, const int32_t* __restrict__ idx,
     const int32_t* __restrict__ pos, const float* __restrict__ gate,
     const uint8_t* __restrict__ kept, T* __restrict__ out, int G, int S, int E,
     int C, int N, int64_t T_tokens, bool vec,
-    const int32_t* __restrict__ row_offsets) {
+    const int32_t* __restrict__ row_offsets, const float* __restrict__ loss,
+    float loss_coef, T* __restrict__ loss_out) {
+  if (loss_out != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+    const float l = round_to<T>(loss[0]);
+    store_f32<T>(loss_out, l);
+    store_f32<T>(loss_out + 1, l * loss_coef);
+  }
   const int lane = threadIdx.x & 63;
   const int64_t t = (int64_t)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
   if (t >= T_tokens) return;
@@ -345,7 +353,9 @@ static int run_dispatch(const void* x, const int32_t* idx, const int32_t* pos,
 static int run_combine(const void* y, const int32_t* idx, const int32_t* pos,
                        const float* gate, const uint8_t* kept,
                        const int32_t* row_offsets, void* out, int G, int S,
-                       int E, int C, int N, int dtype, void* stream);
+                       int E, int C, int N, int dtype, void* stream,
+                       const float* loss = nullptr, float loss_coef = 0.f,
+                       void* loss_out = nullptr);
 
 extern "C" int mesh_moe_combine(const void* y, const int32_t* idx,
                                 const int32_t* pos, const float* gate,
@@ -366,10 +376,25 @@ extern "C" int mesh_moe_combine_compact(const void* y, const int32_t* idx,
                      dtype, stream);
 }
 
+extern "C" int mesh_moe_combine_loss(const void* y, const int32_t* idx,
+                                     const int32_t* pos, const float* gate,
+                                     const uint8_t* kept,
+                                     const int32_t* row_offsets,
+                                     const float* loss, double loss_coef,
+                                     void* out, void* loss_out, int G, int S,
+                                     int E, int C, int N, int dtype,
+                                     void* stream) {
+  MOE_REQUIRE(loss && loss_out, MESH_MOE_E_ARG, "combine_loss: null pointer");
+  return run_combine(y, idx, pos, gate, kept, row_offsets, out, G, S, E, C, N,
+                     dtype, stream, loss, (float)loss_coef, loss_out);
+}
+
 static int run_combine(const void* y, const int32_t* idx, const int32_t* pos,
                        const float* gate, const uint8_t* kept,
                        const int32_t* row_offsets, void* out, int G, int S,
-                       int E, int C, int N, int dtype, void* stream) {
+                       int E, int C, int N, int dtype, void* stream,
+                       const float* loss, float loss_coef,
+                       void* loss_out) {
   MOE_REQUIRE(y && idx && pos && gate && kept && out, MESH_MOE_E_ARG,
               "combine: null pointer");
   MOE_REQUIRE(valid_dtype(dtype), MESH_MOE_E_ARG, "combine: bad dtype %d",
@@ -386,11 +411,11 @@ static int run_combine(const void* y, const int32_t* idx, const int32_t* pos,
   if (dtype == MESH_MOE_F32) {
     combine_kernel<float><<<(unsigned)nblocks, 256, 0, st>>>(
         (const float*)y, idx, pos, gate, kept, (float*)out, G, S, E, C, N,
-        T_tokens, vec, row_offsets);
+        T_tokens, vec, row_offsets, loss, loss_coef, (float*)loss_out);
   } else {
     combine_kernel<bf16_t><<<(unsigned)nblocks, 256, 0, st>>>(
         (const bf16_t*)y, idx, pos, gate, kept, (bf16_t*)out, G, S, E, C, N,
-        T_tokens, vec, row_offsets);
+        T_tokens, vec, row_offsets, loss, loss_coef, (bf16_t*)loss_out);
   }
   MOE_CHECK_LAUNCH("combine");
   return 0;

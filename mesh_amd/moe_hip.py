@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 37
+ABI_VERSION = 38
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -100,6 +100,10 @@ _SIGNATURES = {
         ctypes.c_float, _vp, _vp, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         _vp]),
+    "mesh_moe_combine_loss": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_double, _vp, _vp,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, _vp]),
     "mesh_moe_combine_compact": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
@@ -820,8 +824,9 @@ def pack_weights(w, dtype, out=None):
 
 
 def expert_ffn(expert_in, wi_packed, wo_packed, activation="relu", h=None,
-               y=None):
-  """expert_in [E, R, M]; wi_packed [E, H, M]; wo_packed [E, N, H] -> y [E,R,N]."""
+               y=None, for_gradient=False):
+  """expert_in [E, R, M]; wi_packed [E, H, M]; wo_packed [E, N, H] -> y [E,R,N].
+  for_gradient: h is kept for a gradient (mesh_moe_expert_ffn_kept)."""
   lib = load_library()
   if activation not in ACTIVATIONS:
     raise ValueError("unsupported expert activation %r" % (activation,))
@@ -833,14 +838,14 @@ def expert_ffn(expert_in, wi_packed, wo_packed, activation="relu", h=None,
   ip = _dev(expert_in, "expert_in")
   wip = _dev(wi_packed, "wi_packed", dt, (e, hdim, m))
   wop = _dev(wo_packed, "wo_packed", dt, (e, n, hdim))
-  # a caller that brings h keeps it, for a gradient
-  call = lib.mesh_moe_expert_ffn if h is None else lib.mesh_moe_expert_ffn_kept
   if h is None:
     h = torch.empty((e, rows, hdim), dtype=dt, device=expert_in.device)
   if y is None:
     y = torch.empty((e, rows, n), dtype=dt, device=expert_in.device)
   hp = _dev(h, "h", dt, (e, rows, hdim))
   yp = _dev(y, "y", dt, (e, rows, n))
+  call = (lib.mesh_moe_expert_ffn_kept if for_gradient
+          else lib.mesh_moe_expert_ffn)
   with _stage("expert_ffn"):
     _check(call(ip, wip, wop, hp, yp, e, rows, m, hdim, n,
                 ACTIVATIONS[activation], code, _stream()), "expert_ffn")
@@ -969,9 +974,11 @@ def expert_linear(a, w_packed, activation="linear", y=None):
   return y
 
 
-def combine(y, r, group_size, out=None, row_offsets=None):
+def combine(y, r, group_size, out=None, row_offsets=None, loss_coef=None):
   """y [E, G, C, N] -> out [G, S, N].  With row_offsets [E, G] (from
-  compact_expert_ffn) y holds every expert's occupied slots first."""
+  compact_expert_ffn) y holds every expert's occupied slots first.  With loss_coef
+  (a value of y's dtype): (out, r.loss in y's dtype, that times loss_coef), the last
+  two 0-d."""
   lib = load_library()
   e, g, c, n = y.shape
   s = group_size
@@ -983,6 +990,20 @@ def combine(y, r, group_size, out=None, row_offsets=None):
   if out is None:
     out = torch.empty((g, s, n), dtype=y.dtype, device=y.device)
   op = _dev(out, "out", y.dtype, (g, s, n))
+  if loss_coef is not None:
+    losses = torch.empty((2,), dtype=y.dtype, device=y.device)
+    with _stage("combine") as st:
+      _check(st.call(
+          (y, r, row_offsets, out, losses), lib.mesh_moe_combine_loss,
+          yp, _dev(r.idx, "idx", torch.int32, (g, s, 2)),
+          _dev(r.pos, "pos", torch.int32, (g, s, 2)),
+          _dev(r.gate, "gate", torch.float32, (g, s, 2)),
+          _dev(r.kept, "kept", torch.uint8, (g, s, 2)),
+          None if row_offsets is None else _dev(row_offsets, "row_offsets",
+                                                torch.int32, (e, g)),
+          _dev(r.loss, "loss", torch.float32, (1,)), float(loss_coef), op,
+          losses.data_ptr(), g, s, e, c, n, code, _stream()), "combine_loss")
+    return out, losses[0], losses[1]
   if row_offsets is not None:
     with _stage("combine") as st:
       _check(st.call(

@@ -412,6 +412,32 @@ def _release_saved(saved):
     saved.clear()
 
 
+class ScaledLossOperation(mtf.Operation):
+  """The layer's loss times moe_loss_coef (transformer/moe.py:526-529), made by the
+  layer's last kernel where that can (MoEV1Operation)."""
+
+  def __init__(self, loss, coef, name=None):
+    super(ScaledLossOperation, self).__init__([loss], name=name or "scalar_mul")
+    # the scalar as the reference's op sees it, rounded to the tensor's dtype
+    self._unrounded = coef
+    self.coef = torch.tensor(coef, dtype=loss.dtype).item()
+    self._outputs = [mtf.Tensor(self, loss.shape, loss.dtype)]
+    layer = loss.operation
+    if isinstance(layer, MoEV1Operation) and layer.scaled_loss is None:
+      layer.scaled_loss = self
+
+  def gradient(self, grad_ys):
+    return [grad_ys[0] * self._unrounded]
+
+  def lower(self, lowering):
+    if self in lowering.done_ahead:
+      return
+    coef = self.coef
+    lowering.set_tensor_lowering(
+        self.outputs[0], lowering.mesh_impl(self).slicewise(
+            lambda t: t * coef, lowering.tensors[self.inputs[0]]))
+
+
 class MoEV1Operation(mtf.Operation):
   """The whole of transformer_moe_layer_v1 after the reshape to groups:
   inputs [outer_batch, groups, group, d_model] -> (outputs with d_model
@@ -459,6 +485,7 @@ class MoEV1Operation(mtf.Operation):
     out_shape = mtf.Shape(inputs.shape.dims[:-1] + [output_dim])
     self._outputs = [mtf.Tensor(self, out_shape, inputs.dtype, index=0),
                      mtf.Tensor(self, mtf.Shape([]), inputs.dtype, index=1)]
+    self.scaled_loss = None      # a ScaledLossOperation of the loss
     if k_wo is not None:
       self._outputs.append(mtf.Tensor(self, out_shape, inputs.dtype, index=2))
 
@@ -590,7 +617,8 @@ class MoEV1Operation(mtf.Operation):
         if save or kwo_p is not None:
           h = torch.empty((e_, groups * c_, wi_p.shape[1]), dtype=dt,
                           device=xg.device)
-        y = moe_hip.expert_ffn(expert_in, wi_p, wo_p, self._activation, h=h)
+        y = moe_hip.expert_ffn(expert_in, wi_p, wo_p, self._activation, h=h,
+                               for_gradient=save)
       elif y is None:
         # the hidden tensor is worked on between the two projections: the
         # other factors of the product, then the dropout
@@ -615,8 +643,21 @@ class MoEV1Operation(mtf.Operation):
                                          want_noise=keep_noise)
         y = moe_hip.expert_linear(h, wo_p)
       y4 = y.reshape(e_, groups, c_, n_)
-      out = (moe_hip.slot_combine(y4, r, s_) if by_slot
-             else moe_hip.combine(y4, r, s_, row_offsets=row_offsets))
+      scaled = None
+      if by_slot:
+        out = moe_hip.slot_combine(y4, r, s_)
+      elif self.scaled_loss is not None:
+        out, loss, scaled = moe_hip.combine(
+            y4, r, s_, row_offsets=row_offsets,
+            loss_coef=self.scaled_loss.coef)
+      else:
+        out = moe_hip.combine(y4, r, s_, row_offsets=row_offsets)
+      if scaled is None:
+        loss = r.loss.to(dt).reshape(())
+      else:
+        lowering.set_tensor_lowering(self.scaled_loss.outputs[0],
+                                     mesh_impl.LaidOutTensor([scaled]))
+        lowering.done_ahead.add(self.scaled_loss)
       if save:
         # what the gradient operation reads (activations of this step)
         gate_noise = getattr(self._gating, "noise", None)
@@ -625,7 +666,7 @@ class MoEV1Operation(mtf.Operation):
                      expert_in=expert_in, h=h, y=y, row_offsets=row_offsets,
                      w_gate_packed=wg_p,
                      gate_in=gate_in, w_gate=wg_s, hidden_noise=noise)
-      outs = (out.reshape(o_, g_, s_, n_), r.loss.to(dt).reshape(()))
+      outs = (out.reshape(o_, g_, s_, n_), loss)
       if kwo_p is not None:
         # the "k" projection of the same hidden tensor (moe.py:514-520)
         yk = moe_hip.expert_linear(h, kwo_p).reshape(e_, groups, c_, n_)
@@ -945,7 +986,8 @@ def transformer_moe_layer_v1(
         hidden_keep_prob=hidden_keep_prob).outputs
     outputs = [mtf.reshape(t, batch_and_length_dims + [output_dim])
                for t in (q, k)]
-    return outputs, loss * hparams.moe_loss_coef
+    return outputs, ScaledLossOperation(
+        loss, hparams.moe_loss_coef).outputs[0]
   wo = mtf_layers.get_dense_kernel_weights(
       inputs, [output_dim], [hidden_dim], [experts_dim], None, name="wo",
       variable_dtype=variable_dtype)
@@ -954,7 +996,8 @@ def transformer_moe_layer_v1(
       inputs, w_gate, wi, wo, nonpadding, output_dim, expert_capacity, gating,
       act_names, hidden_keep_prob=hidden_keep_prob).outputs
   output = mtf.reshape(output, batch_and_length_dims + [output_dim])
-  return output, loss * hparams.moe_loss_coef
+  return output, ScaledLossOperation(
+      loss, hparams.moe_loss_coef).outputs[0]
 
 
 class MoEV2Operation(mtf.Operation):
@@ -1036,7 +1079,7 @@ class MoEV2Operation(mtf.Operation):
         h = torch.empty((y_e * x_e, h0 * d_, wi_p.shape[1]), dtype=dt,
                         device=xg.device)
       yy = moe_hip.expert_ffn(ein_y.reshape(y_e * x_e, h0 * d_, m_), wi_p,
-                              wo_p, "relu", h=h)
+                              wo_p, "relu", h=h, for_gradient=save)
       out_y = moe_hip.combine(yy.reshape(y_e, x_e * h0, d_, n_), ry, t_)
       out = moe_hip.combine(out_y.reshape(x_e, ag, c_, n_), rx, s_)
       loss = (rx.loss.to(dt) + ry.loss.to(dt)).reshape(())

@@ -1961,3 +1961,19 @@ def test_dropout_noise_from_the_relu_mask(hip):
     with pytest.raises(Exception, match="dh_keep_prob"):
       hip.compact_expert_ffn_backward(xe_c, h_c, dy_c, wi, wo, r, ro, "relu",
                                       keep_prob=bad)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("g,s,n", [(1, 1, 8), (2, 130, 72), (3, 64, 20)])
+def test_combine_with_loss(hip, dtype, g, s, n):
+  """The layer's loss on the way out: the bits of a cast and a scalar product."""
+  e, c = 6, 40
+  gen = torch.Generator(device="cuda").manual_seed(s + n)
+  logits = torch.randn((g, s, e), generator=gen, device="cuda")
+  r = hip.top2_gating(logits, c)
+  y = torch.randn((e, g, c, n), generator=gen, device="cuda").to(dtype)
+  coef = torch.tensor(1e-2, dtype=dtype).item()
+  out, loss, scaled = hip.combine(y, r, s, loss_coef=coef)
+  assert torch.equal(out, hip.combine(y, r, s))
+  want = r.loss.to(dtype).reshape(())
+  assert torch.equal(loss, want) and torch.equal(scaled, want * coef)
