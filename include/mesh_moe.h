@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 38
+#define MESH_MOE_ABI_VERSION 39
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -874,6 +874,20 @@ int mesh_moe_broadcast_dropout(const void* x, const void* uniform,
                                const void* noise_in, float keep_prob, void* out,
                                void* noise_out, int64_t outer, int64_t mid,
                                int64_t inner, int dtype, void* stream);
+
+/*
+ * Dense layers of one input in one launch, as the q, k and v projections of an
+ * attention layer are (transformer/attention.py:481-551): y[e] = a . w[e], and their
+ * weight gradients dw[e] = a^T . dy[e].
+ *   a [R,K]; w_packed [E,N,K] (see pack_weights); y, dy [E,R,N]; dw [E,K,N]; bf16, K
+ *   and N multiples of 8 (backward: and at least 128)
+ */
+int mesh_moe_shared_linear(const void* a, const void* w_packed, void* y, int E,
+                           int R, int K, int N, int dtype, void* stream);
+size_t mesh_moe_shared_linear_backward_workspace_bytes(int E, int R, int K, int N);
+int mesh_moe_shared_linear_backward(const void* a, const void* dy, void* dw, int E,
+                                    int R, int K, int N, int dtype, void* workspace,
+                                    size_t workspace_bytes, void* stream);
 
 /*
  * RMS normalisation (sublayer_rms_norm, transformer/transformer.py:493-516):

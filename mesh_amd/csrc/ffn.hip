@@ -61,7 +61,8 @@ __device__ __forceinline__ uint32_t pack2_bf16(float a, float b, bool relu) {
 template <int BM, int BN, int BK, bool RELU, bool OUT_F32 = false>
 __global__ __launch_bounds__(256) void grouped_gemm_bf16_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-    void* __restrict__ Cvoid, int R, int N, int K, int tiles_m, int tiles_n) {
+    void* __restrict__ Cvoid, int R, int N, int K, int tiles_m, int tiles_n,
+    int64_t a_stride) {
   bf16_t* Cout = reinterpret_cast<bf16_t*>(Cvoid);
   using Cfg = GemmCfg<BM, BN, BK>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -83,7 +84,9 @@ __global__ __launch_bounds__(256) void grouped_gemm_bf16_kernel(
   const int tn = rem / tiles_m;
   const int tm = rem - tn * tiles_m;
   const int row0 = tm * BM, col0 = tn * BN;
-  const bf16_t* Ae = A + (int64_t)e * R * K;
+  // (a_stride: elements from one expert's rows to the next one's, 0 where all
+  // experts read the same rows)
+  const bf16_t* Ae = A + e * a_stride;
   const bf16_t* Be = B + (int64_t)e * N * K;
   bf16_t* Ce = Cout + (int64_t)e * R * N;
 
@@ -249,7 +252,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 template <int MT, int NT>
 __global__ __launch_bounds__(1024) void skinny_gemm_bf16_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
-    bf16_t* __restrict__ C, int R, int N, int K, int groups_n, int relu) {
+    bf16_t* __restrict__ C, int R, int N, int K, int groups_n, int relu,
+    int64_t a_stride) {
   constexpr int U = MT <= 2 ? 4 : 2;       // k steps of 32 loaded together
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -264,7 +268,7 @@ __global__ __launch_bounds__(1024) void skinny_gemm_bf16_kernel(
     bp[j] = B + ((int64_t)e * N + min(n0 + 16 * j + r16, N - 1)) * K + kq;
 #pragma unroll
   for (int i = 0; i < MT; ++i)
-    ap[i] = A + ((int64_t)e * R + min(16 * i + r16, R - 1)) * K + kq;
+    ap[i] = A + e * a_stride + (int64_t)min(16 * i + r16, R - 1) * K + kq;
   f32x4_t acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -464,7 +468,8 @@ __global__ __launch_bounds__(256) void stream_gemm_bf16_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
     bf16_t* __restrict__ C, int R, int N, int K, int tiles_n, int relu,
     const int32_t* __restrict__ row_map, int gather,
-    const bf16_t* __restrict__ zero_row) {
+    const bf16_t* __restrict__ zero_row,
+    int64_t a_stride) {
   using Cfg = StreamCfg<MT>;
   constexpr int BN = Cfg::BN, BK = Cfg::BK, NS = Cfg::NS;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(256) void stream_gemm_bf16_kernel(
   for (int j = 0; j < MT; ++j) {
     const int row = (wave + 4 * j) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ lds_swizzle(row);
-    const bf16_t* base = A + ((int64_t)e * R + min(row, R - 1)) * K;
+    const bf16_t* base = A + e * a_stride + (int64_t)min(row, R - 1) * K;
     if constexpr (MAPPED) {
       const int src = row_map[(int64_t)e * R + min(row, R - 1)];
       any |= src >= 0;
@@ -673,7 +678,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int32_t* __restrict__ tile_list = nullptr,
     const int32_t* __restrict__ row_count = nullptr,
     float mask_scale = 1.0f, float* __restrict__ partial = nullptr,
-    int whole_tiles = 0, int split = 1, int tile_rows = RingCfg::BM) {
+    int whole_tiles = 0, int split = 1, int tile_rows = RingCfg::BM,
+    int64_t a_stride = -1) {
   using Cfg = RingCfg;
   // row_count [E], optional: KMAJOR kernels take it as the reduction extent
   // per expert (k_extent)
@@ -822,7 +828,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         }
       }
     }
-    Ae = GATHER ? A : A + (int64_t)e * R * K;
+    // (a_stride 0: all experts read the same rows)
+    Ae = GATHER ? A : A + e * (a_stride < 0 ? (int64_t)R * K : a_stride);
     Be = B + (int64_t)e * N * K;
     Ce = Cout + (int64_t)e * R * N;
 #pragma unroll
@@ -1661,7 +1668,8 @@ int compute_units() {
 
 template <int BM, int BN, int BK>
 static int launch_mfma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
-                       int R, int N, int K, bool relu, hipStream_t st) {
+                       int R, int N, int K, bool relu, hipStream_t st,
+                       int64_t a_stride) {
   using Cfg = GemmCfg<BM, BN, BK>;
   const int tiles_m = (R + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   const int64_t blocks = (int64_t)tiles_m * tiles_n * E;
@@ -1671,12 +1679,12 @@ static int launch_mfma(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     auto k = grouped_gemm_bf16_kernel<BM, BN, BK, true>;
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<(unsigned)blocks, 256, Cfg::LDS_BYTES, st>>>(A, B, C, R, N, K, tiles_m,
-                                                      tiles_n);
+                                                      tiles_n, a_stride);
   } else {
     auto k = grouped_gemm_bf16_kernel<BM, BN, BK, false>;
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<(unsigned)blocks, 256, Cfg::LDS_BYTES, st>>>(A, B, C, R, N, K, tiles_m,
-                                                      tiles_n);
+                                                      tiles_n, a_stride);
   }
   MOE_CHECK_LAUNCH("expert_ffn (mfma)");
   return 0;
@@ -1689,7 +1697,8 @@ static int skinny_columns(int E, int N) {
 }
 
 static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
-                         int R, int N, int K, bool relu, hipStream_t st) {
+                         int R, int N, int K, bool relu, hipStream_t st,
+                         int64_t a_stride) {
   // 16 columns per block while no compute unit gets a second block, else 32
   // (half the token reads)
   const int nt = skinny_columns(E, N) / 16;
@@ -1709,7 +1718,7 @@ static int launch_skinny(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
   auto run = [&](auto k) -> int {
     MOE_ALLOW_LDS(k, lds);
     k<<<(unsigned)blocks, 64 * waves, lds, st>>>(A, B, C, R, N, K, groups_n,
-                                                 relu ? 1 : 0);
+                                                 relu ? 1 : 0, a_stride);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, few rows)");
     return 0;
   };
@@ -1772,7 +1781,9 @@ static bool stream_applies(int E, int R, int N, int K) {
 static int launch_stream(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                          int R, int N, int K, bool relu, hipStream_t st,
                          const int32_t* row_map = nullptr, bool gather = false,
-                         const bf16_t* zero_row = nullptr) {
+                         const bf16_t* zero_row = nullptr,
+                         int64_t a_stride = -1) {
+  if (a_stride < 0) a_stride = (int64_t)R * K;
   auto run = [&](auto k, auto cfg) -> int {
     using Cfg = decltype(cfg);
     const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
@@ -1782,7 +1793,7 @@ static int launch_stream(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<(unsigned)blocks, 256, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_n, relu ? 1 : 0, row_map, gather ? 1 : 0,
-        zero_row);
+        zero_row, a_stride);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, few rows per expert)");
     return 0;
   };
@@ -1858,7 +1869,7 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
                               int E, int R, int N, int K, hipStream_t st,
                               const int32_t* k_extent = nullptr,
-                              void* scratch = nullptr) {
+                              void* scratch = nullptr, int64_t a_stride = -1) {
   using Cfg = RingCfg;
   const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
@@ -1881,7 +1892,7 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     k<<<split_blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, units, nullptr, nullptr, nullptr,
         nullptr, nullptr, 1.0f, (float*)scratch, plan.whole_tiles, plan.split,
-        Cfg::BM);
+        Cfg::BM, a_stride);
     MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands, split)");
     split_reduce_kernel<<<(unsigned)tail * Cfg::TM * Cfg::TN, Cfg::THREADS, 0,
                           st>>>((const float*)scratch, C, R, N, tiles_m,
@@ -1893,7 +1904,7 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
   MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
   k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
       A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, Cfg::BM);
+      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, Cfg::BM, a_stride);
   MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
   return 0;
 }
@@ -1938,7 +1949,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                        const bf16_t* zero_row = nullptr,
                        const bf16_t* mask_src = nullptr,
                        const int32_t* tile_list = nullptr,
-                       float mask_scale = 1.0f) {
+                       float mask_scale = 1.0f, int64_t a_stride = -1) {
   using Cfg = RingCfg;
   const int cus = compute_units();
   if (cus == 0) return MESH_MOE_E_HIP;
@@ -1958,7 +1969,8 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,
-        mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1, tile_rows);
+        mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1, tile_rows,
+        a_stride);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, 256-column direct-to-LDS tiles)");
     return 0;
   };
@@ -2048,8 +2060,11 @@ static bool f32_nt_applies(const void* A, const void* B, const void* C, int R,
 static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
                         int N, int K, int act, int dtype, hipStream_t st,
                         const void* relu_mask_src = nullptr,
-                        bool* mask_applied = nullptr, float mask_scale = 1.0f) {
+                        bool* mask_applied = nullptr, float mask_scale = 1.0f,
+                        bool shared_a = false) {
   const bool relu = act == MESH_MOE_ACT_RELU;
+  // shared_a (bf16 on the matrix cores only): one A [R, K] for all experts
+  const int64_t a_stride = shared_a ? 0 : (int64_t)R * K;
   int rc;
   if (mask_applied) *mask_applied = false;
   if (dtype == MESH_MOE_F32) {
@@ -2082,10 +2097,10 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
                                  (bf16_t*)C, E, R, N, K, relu, st);
     else if (stream_applies(E, R, N, K))
       rc = launch_stream((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
-                         N, K, relu, st);
+                         N, K, relu, st, nullptr, false, nullptr, a_stride);
     else if (skinny_applies(E, R, N, K))
       rc = launch_skinny((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R,
-                         N, K, relu, st);
+                         N, K, relu, st, a_stride);
     else if (ring_shape(R, N, K) && (int64_t)R * K < (1LL << 31) &&
              (masks || !small_tiles_apply(E, R, N, K))) {
       // 256-column tiles in persistent blocks of 8 wavefronts (two per SIMD),
@@ -2093,14 +2108,14 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
       rc = launch_ring((const bf16_t*)A, (const bf16_t*)B, (bf16_t*)C, E, R, N,
                        K, relu, st, nullptr, nullptr,
                        masks ? (const bf16_t*)relu_mask_src : nullptr, nullptr,
-                       masks ? mask_scale : 1.0f);
+                       masks ? mask_scale : 1.0f, a_stride);
       if (masks) *mask_applied = rc == 0;
     } else if (R >= 1024 && N >= 1024 && !small_tiles_apply(E, R, N, K))
       rc = launch_mfma<256, 256, 64>((const bf16_t*)A, (const bf16_t*)B,
-                                     (bf16_t*)C, E, R, N, K, relu, st);
+                                     (bf16_t*)C, E, R, N, K, relu, st, a_stride);
     else
       rc = launch_mfma<128, 128, 64>((const bf16_t*)A, (const bf16_t*)B,
-                                     (bf16_t*)C, E, R, N, K, relu, st);
+                                     (bf16_t*)C, E, R, N, K, relu, st, a_stride);
   }
   if (rc != 0) return rc;
   if (act != MESH_MOE_ACT_RELU && act != MESH_MOE_ACT_LINEAR)
@@ -2145,7 +2160,8 @@ int batched_gemm_nt(const void* A, const void* B, void* C, int E, int R, int N,
   auto k = grouped_gemm_bf16_kernel<128, 128, 64, false, true>;
   MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
   k<<<(unsigned)blocks, 256, Cfg::LDS_BYTES, st>>>(
-      (const bf16_t*)A, (const bf16_t*)B, C, R, N, K, tiles_m, tiles_n);
+      (const bf16_t*)A, (const bf16_t*)B, C, R, N, K, tiles_m, tiles_n,
+      (int64_t)R * K);
   MOE_CHECK_LAUNCH("batched_gemm_nt (mfma, float32 result)");
   return 0;
 }
@@ -2991,4 +3007,59 @@ extern "C" int mesh_moe_compact_expert_ffn_backward(
   if (rc != 0) return rc;
   return launch_ring_kmajor((const bf16_t*)expert_in, dh, (bf16_t*)dwi, E, M,
                             H, R, st, rows_used);
+}
+
+// Several dense layers of one input: y[e] = a . w[e].  The experts of a grouped product
+// that all read the same rows (a_stride 0).  What bounds a projection of few rows is its
+// launch and a chip that one product does not fill: three products of 32 rows,
+// 1024 -> 1024, 14.6 us one by one and 5.4 in one launch, of 1024 rows, 768 -> 768,
+// 31.6 and 12.6, of 4096 rows 40.5 and 21.8, of 16384 rows, 1024 -> 1024 (256 tiles of
+// the ring each), 100.6 and 95.3.
+extern "C" int mesh_moe_shared_linear(const void* a, const void* w_packed, void* y,
+                                      int E, int R, int K, int N, int dtype,
+                                      void* stream) {
+  MOE_REQUIRE(a && w_packed && y, MESH_MOE_E_ARG, "shared_linear: null pointer");
+  MOE_REQUIRE(valid_dtype(dtype), MESH_MOE_E_ARG, "shared_linear: bad dtype %d",
+              dtype);
+  MOE_REQUIRE(E >= 1 && R >= 1 && K >= 1 && N >= 1, MESH_MOE_E_ARG,
+              "shared_linear: bad sizes E=%d R=%d K=%d N=%d", E, R, K, N);
+  MOE_REQUIRE(dtype == MESH_MOE_BF16 && K % 8 == 0 && N % 8 == 0 &&
+                  ((uintptr_t)a | (uintptr_t)w_packed | (uintptr_t)y) % 16 == 0,
+              MESH_MOE_E_UNSUPPORTED,
+              "shared_linear: needs bf16, sizes that are multiples of 8 and 16-byte "
+              "alignment (K=%d N=%d dtype=%d)", K, N, dtype);
+  return grouped_gemm(a, w_packed, y, E, R, N, K, MESH_MOE_ACT_LINEAR, dtype,
+                      (hipStream_t)stream, nullptr, nullptr, 1.0f, true);
+}
+
+extern "C" size_t mesh_moe_shared_linear_backward_workspace_bytes(int E, int R,
+                                                                  int K, int N) {
+  if (E < 1 || R < 1 || K < 1 || N < 1) return 0;
+  return kmajor_split_plan(E, K, N, R).bytes + 256;
+}
+
+// Their weight gradients: dw[e] = a^T . dy[e].  Nine tiles of 256 x 256 (768 -> 768) leave
+// most of the chip idle or are cut along a reduction that is then written and read as
+// partial sums; three times as many tiles need a third of the cuts.  With the three
+// products for dx: 4096 rows, 768 -> 768, 109.9 us one by one and 73.2, 16384 rows,
+// 1024 -> 1024, 260.5 and 206.9.
+extern "C" int mesh_moe_shared_linear_backward(const void* a, const void* dy,
+                                               void* dw, int E, int R, int K, int N,
+                                               int dtype, void* workspace,
+                                               size_t workspace_bytes,
+                                               void* stream) {
+  MOE_REQUIRE(a && dy && dw && workspace, MESH_MOE_E_ARG,
+              "shared_linear_backward: null pointer");
+  MOE_REQUIRE(E >= 1 && R >= 1 && K >= 1 && N >= 1, MESH_MOE_E_ARG,
+              "shared_linear_backward: bad sizes E=%d R=%d K=%d N=%d", E, R, K, N);
+  MOE_REQUIRE(kmajor_path_applies(a, dy, dw, K, N, R, dtype),
+              MESH_MOE_E_UNSUPPORTED,
+              "shared_linear_backward: needs bf16, K and N multiples of 8 and at "
+              "least 128, 16-byte alignment (K=%d N=%d dtype=%d)", K, N, dtype);
+  MOE_REQUIRE(workspace_bytes >=
+                  mesh_moe_shared_linear_backward_workspace_bytes(E, R, K, N),
+              MESH_MOE_E_ARG, "shared_linear_backward: workspace too small");
+  void* parts = (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  return launch_ring_kmajor((const bf16_t*)a, (const bf16_t*)dy, (bf16_t*)dw, E, K,
+                            N, R, (hipStream_t)stream, nullptr, parts, 0);
 }

@@ -111,6 +111,7 @@ class HipMeshImpl(mtf.MeshImpl):
       self._master = master.to(device=dev, dtype=variable.master_dtype).contiguous()
       self._slice = None
       self._derived = {}
+      self._together = {}
       self.copy_master_to_slices()
 
     variable = property(lambda self: self._variable)
@@ -188,6 +189,30 @@ class HipMeshImpl(mtf.MeshImpl):
         k, n = s.shape[-2], s.shape[-1]
         self._derived[key] = moe_hip.pack_weights(s.reshape(-1, k, n), dtype)
       return self._derived[key]
+
+    @staticmethod
+    def packed_together(variables, dtype):
+      """The packed copies of variables of one shape [K, N] as one tensor
+      [len(variables), N, K], of which packed() then gives the parts; None where
+      one of them has a packed copy of its own already."""
+      first = variables[0]
+      key, group = ("packed", dtype), ("packed_together", dtype)
+      if group not in first._together:
+        shape = first._slice.shape
+        if len(shape) != 2 or len(set(variables)) < len(variables) or any(
+            key in v._derived or v._slice.shape != shape for v in variables):
+          first._together[group] = None
+        else:
+          k, n = shape
+          joint = torch.empty((len(variables), n, k), dtype=dtype,
+                              device=first._slice.device)
+          for i, v in enumerate(variables):
+            v._derived[key] = joint[i:i + 1]
+            moe_hip.pack_weights(v._slice.reshape(1, k, n), dtype,
+                                 out=v._derived[key])
+          first._together[group] = (tuple(variables), joint)
+      found = first._together[group]
+      return found[1] if found and found[0] == tuple(variables) else None
 
   # -- execution -------------------------------------------------------------
   def slicewise(self, fn, *inputs):

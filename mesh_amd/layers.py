@@ -121,6 +121,57 @@ def get_dense_kernel_weights(x, new_dims, reduced_dims, expert_dims,
                             dtype=variable_dtype)
 
 
+class SharedInput(object):
+  """Dense layers without activation, of one input and of kernels of one shape:
+  their products, and the gradients of their kernels, are made in one launch
+  each."""
+
+  def __init__(self, layers):
+    x, kernel = layers[0].inputs
+    self.layers = list(layers)
+    self.gradients = {}        # {layer: its DenseGradOperation}
+    self._ahead = {}           # {first of them: every dy is there when it runs}
+    if all(op.inputs[0] is x and op.inputs[1].shape.to_integer_list ==
+           kernel.shape.to_integer_list and op.inputs[1].dtype == kernel.dtype and
+           op._activation is None and op.siblings is None   # pylint: disable=protected-access
+           for op in layers):
+      for op in layers:
+        op.siblings = self
+
+  def make_kernel_gradients(self, lowering, first):
+    """Called by the first of the gradient operations: {layer: its kernel
+    gradient} if every dy is there and they lie one after the other in memory (as
+    the attention's gradient leaves them), else {}."""
+    from mesh_amd import moe_hip
+    grads = [self.gradients.get(op) for op in self.layers]
+    operations = first.graph.operations
+    if first not in self._ahead:
+      at = operations.index(first)
+      self._ahead[first] = None not in grads and all(
+          operations.index(g.inputs[0].operation) < at for g in grads)
+    if not self._ahead[first]:
+      return {}
+
+    def rows_of(t):
+      return lowering.tensors[t].to_laid_out_tensor().tensor_list[0]
+    x = rows_of(first.inputs[1])
+    dys = [rows_of(g.inputs[0]) for g in grads]
+    d = dys[0]
+    n = d.shape[-1]
+    step = d.numel()
+    if not (moe_hip.shared_linear_backward_supported(x, n) and all(
+        t.is_contiguous() and t.dtype == x.dtype and t.shape == d.shape and
+        t.untyped_storage().data_ptr() == d.untyped_storage().data_ptr() and
+        t.storage_offset() == d.storage_offset() + i * step
+        for i, t in enumerate(dys))):
+      return {}
+    joint = d.as_strided((len(dys),) + tuple(d.shape), (step,) + d.stride())
+    made = lowering.mesh_impl(first).slicewise(
+        lambda rows: tuple(moe_hip.shared_linear_backward(rows, joint).unbind(0)),
+        lowering.tensors[first.inputs[1]])
+    return dict(zip(self.layers, made))
+
+
 class DenseOperation(mtf.Operation):
   """y = activation(x . kernel) over the last dim of x: the einsum (+ relu) of
   mtf.layers.dense without bias (mesh_tensorflow/layers.py:112-160) as one
@@ -132,9 +183,37 @@ class DenseOperation(mtf.Operation):
     self._activation = activation
     shape = mtf.Shape(x.shape.dims[:-1] + list(new_dims))
     self._outputs = [mtf.Tensor(self, shape, x.dtype)]
+    self.siblings = None       # a SharedInput
+
+  def _lower_siblings(self, lowering):
+    """All layers of one input in one launch, by the first of them.  False where
+    there is no kernel for that."""
+    from mesh_amd import moe_hip
+    layers = self.siblings.layers
+    if layers[0] is not self:
+      return False
+    mesh_impl = lowering.mesh_impl(self)
+    x = lowering.tensors[self.inputs[0]].to_laid_out_tensor().tensor_list[0]
+    n = self.outputs[0].shape.dims[-1].size
+    if not moe_hip.shared_linear_supported(x, n):
+      return False
+    variables = [lowering.variables[op.inputs[1].operation] for op in layers]
+    packed = variables[0].packed_together(variables, x.dtype)
+    if packed is None:
+      return False
+    outs = mesh_impl.slicewise(
+        lambda rows: tuple(moe_hip.shared_linear(rows, packed).unbind(0)),
+        lowering.tensors[self.inputs[0]])
+    for op, out in zip(layers, outs):
+      lowering.set_tensor_lowering(op.outputs[0], out)
+      lowering.done_ahead.add(op)
+    return True
 
   def lower(self, lowering):
     from mesh_amd import moe_hip
+    if self in lowering.done_ahead or (
+        self.siblings is not None and self._lower_siblings(lowering)):
+      return
     x, kernel = self.inputs
     mesh_impl = lowering.mesh_impl(self)
     packed = lowering.variables[kernel.operation].packed(x.dtype)
@@ -188,10 +267,37 @@ class DenseGradOperation(mtf.Operation):
                                 % (forward._activation,))  # pylint: disable=protected-access
     self._outputs = [mtf.Tensor(self, x.shape, x.dtype, index=0),
                      mtf.Tensor(self, kernel.shape, kernel.dtype, index=1)]
+    self._forward = forward
+    siblings = forward.siblings
+    if siblings is not None and not self._masks_dx:
+      siblings.gradients[forward] = self
+
+  def _kernel_gradient(self, lowering):
+    """This layer's part of what was made for all layers of its input, or None."""
+    siblings = self._forward.siblings
+    if siblings is None or siblings.gradients.get(self._forward) is not self:
+      return None
+    if self._forward is siblings.layers[-1]:
+      # (the backward walk meets the last layer first)
+      lowering.run_values[siblings] = siblings.make_kernel_gradients(lowering,
+                                                                     self)
+    return lowering.run_values.get(siblings, {}).pop(self._forward, None)
 
   def lower(self, lowering):
     from mesh_amd import moe_hip
     mesh_impl = lowering.mesh_impl(self)
+    made = self._kernel_gradient(lowering)
+    if made is not None:
+      k = self.inputs[1].shape.dims[-1].size
+      kernel_sizes = self.inputs[2].shape.to_integer_list
+      lowering.set_tensor_lowering(self.outputs[0], mesh_impl.slicewise(
+          lambda dy, x, w: moe_hip.dense(
+              dy, w.to(x.dtype).reshape(1, k, -1).contiguous()),
+          *[lowering.tensors[t] for t in self.inputs[:3]]))
+      lowering.set_tensor_lowering(self.outputs[1], mesh_impl.slicewise(
+          lambda dw, w: dw.reshape(kernel_sizes).to(w.dtype), made,
+          lowering.tensors[self.inputs[2]]))
+      return
     relu = self._relu and not self._dy_is_masked
     masks_dx = self._masks_dx
     k = self.inputs[1].shape.dims[-1].size

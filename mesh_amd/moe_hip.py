@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 38
+ABI_VERSION = 39
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -216,6 +216,14 @@ _SIGNATURES = {
     "mesh_moe_slot_combine": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
+    "mesh_moe_shared_linear": (ctypes.c_int, [
+        _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, _vp]),
+    "mesh_moe_shared_linear_backward_workspace_bytes": (ctypes.c_size_t, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "mesh_moe_shared_linear_backward": (ctypes.c_int, [
+        _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
     "mesh_moe_residual_rms_norm": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
         ctypes.c_double, ctypes.c_int, _vp]),
@@ -1479,6 +1487,50 @@ def dense(x, w_packed, activation=None):
   return y
 
 
+def shared_linear_supported(x, n):
+  """Whether shared_linear takes rows like x's and n columns per layer."""
+  k = x.shape[-1]
+  return (x.dtype == torch.bfloat16 and k % 8 == 0 and n % 8 == 0 and
+          x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def shared_linear(x, w_packed):
+  """x [..., K] times every packed kernel of [E, N, K] -> [E, ..., N]."""
+  lib = load_library()
+  e, n, k = w_packed.shape
+  y = torch.empty((e,) + tuple(x.shape[:-1]) + (n,), dtype=x.dtype,
+                  device=x.device)
+  with _stage("expert_linear"):
+    _check(lib.mesh_moe_shared_linear(
+        _dev(x, "a"), _dev(w_packed, "w_packed", x.dtype, (e, n, k)),
+        y.data_ptr(), e, x.numel() // k, k, n, dtype_code(x.dtype), _stream()),
+           "shared_linear")
+  return y
+
+
+def shared_linear_backward_supported(x, n):
+  """Whether shared_linear_backward takes rows like x's."""
+  return (shared_linear_supported(x, n) and x.shape[-1] >= 128 and n >= 128 and
+          x.numel() < 1 << 31 and x.numel() // x.shape[-1] * n < 1 << 31)
+
+
+def shared_linear_backward(x, dy):
+  """The weight gradients of shared_linear: x [..., K], dy [E, ..., N] ->
+  [E, K, N]."""
+  lib = load_library()
+  e, n, k = dy.shape[0], dy.shape[-1], x.shape[-1]
+  rows = x.numel() // k
+  dw = torch.empty((e, k, n), dtype=x.dtype, device=x.device)
+  ws_bytes = lib.mesh_moe_shared_linear_backward_workspace_bytes(e, rows, k, n)
+  ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=x.device)
+  with _stage("expert_linear_backward"):
+    _check(lib.mesh_moe_shared_linear_backward(
+        _dev(x, "a"), _dev(dy, "dy", x.dtype, (e,) + tuple(x.shape[:-1]) + (n,)),
+        dw.data_ptr(), e, rows, k, n, dtype_code(x.dtype), ws.data_ptr(), ws_bytes,
+        _stream()), "shared_linear_backward")
+  return dw
+
+
 def fused_attention_applies(q, num_heads):
   """Whether the fused attention kernels take q's shape and dtype."""
   b, l, hd = q.shape
@@ -1789,7 +1841,9 @@ def self_attention_backward(q, k, v, dout, num_heads, causal, fused=None,
         b, l, h, d, code, int(relative_bias is not None))
     if ws_bytes:
       ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device)
-      dq, dk, dv = (torch.empty_like(q) for _ in range(3))
+      # (one allocation: the projections' weight gradients are one launch then)
+      dq, dk, dv = torch.empty((3,) + tuple(q.shape), dtype=q.dtype,
+                               device=q.device).unbind(0)
       dvalues = None
       if relative_bias is not None:
         dvalues = torch.empty_like(relative_bias[0])

@@ -622,6 +622,7 @@ class Lowering(object):
     # Operations whose outputs this run already holds, because an operation in
     # front of them made them in the same kernel
     self.done_ahead = set()
+    self.run_values = {}   # what operations of one run leave for later ones
     for op in graph.operations:
       op.lower(self)
       for out in op.outputs:
@@ -635,6 +636,7 @@ class Lowering(object):
     self._feeds = dict(feeds or {})
     self.scalar_summaries = {}
     self.done_ahead = set()
+    self.run_values = {}
     try:
       for op in self.graph.operations:
         if not isinstance(op, Variable):

@@ -57,6 +57,7 @@ class AttentionParams(object):
     first = (query_heads_dims + [key_dim])[0].name
     combined = mtf.Dimension(first, self.num_heads * key_dim.size)
     self.combined_dim = combined
+    self._projections = {}     # {name: its DenseOperation}
     stddev = query_input_dim.size ** -0.5
     if fold_scaling_into_initializer:
       stddev *= key_dim.size ** -0.5
@@ -85,8 +86,16 @@ class AttentionParams(object):
                                initializer=normal(o_std), dtype=variable_dtype)
 
   def _project(self, x, w, name):
-    return mtf_layers.DenseOperation(x, w, [w.shape.dims[-1]], None,
-                                     name=name).outputs[0]
+    op = mtf_layers.DenseOperation(x, w, [w.shape.dims[-1]], None, name=name)
+    self._projections[name] = op
+    return op.outputs[0]
+
+  def share_projections(self):
+    """After compute_q, compute_k and compute_v of the same antecedent: one launch
+    makes all three."""
+    ops = [self._projections.get(n) for n in ("q_proj", "k_proj", "v_proj")]
+    if all(op is not None for op in ops):
+      mtf_layers.SharedInput(ops)
 
   def compute_q(self, query_antecedent):
     """[..., d_model] -> [..., heads * d_kv] (attention.py:481-497)."""

@@ -137,6 +137,7 @@ class SelfAttention(transformer.TransformerLayer):
     else:
       k = params.compute_k(x)
       v = params.compute_v(x)
+      params.share_projections()
     relative_values = self.relative_bias_values(context, params.num_heads)
     if context.mode == transformer.INCREMENTAL:
       # one position per batch entry: the step's key and value replace row

@@ -1759,3 +1759,86 @@ def test_layer_stack_second_run(packed, dtype):
   step.replay(feeds)
   for g in grads + [y]:
     assert torch.equal(lowering.export_to_tf_tensor(g), want[g]), g
+
+
+# few rows (the reduction cut over wavefronts), 128 x 128 tiles, the ring with whole and
+# with lower row tiles; column counts with a partial last tile; weight gradients whose
+# reduction is split and not
+@pytest.mark.parametrize("rows,k,n", [(1, 64, 16), (32, 1024, 1024), (64, 256, 264),
+                                      (100, 128, 136), (200, 64, 512),
+                                      (300, 768, 768), (2000, 128, 640),
+                                      (1111, 256, 256)])
+def test_shared_linear(hip, rows, k, n):
+  """The layers of one input in one launch against a launch each: products of the
+  same kernel have the same bits, weight gradients the sums in another order."""
+  gen = torch.Generator(device="cuda").manual_seed(rows + k + n)
+  x = torch.randn((rows, k), generator=gen, device="cuda").bfloat16()
+  w = (torch.randn((3, n, k), generator=gen, device="cuda") / k ** 0.5).bfloat16()
+  y = hip.shared_linear(x, w)
+  want = x.double() @ w.double().transpose(1, 2).contiguous()
+  # one rounding to bf16, and float32 sums below it
+  assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + k * 2.0 ** -24 * (
+      x.double().abs() @ w.double().abs().transpose(1, 2).contiguous())).all()
+  if not hip.shared_linear_backward_supported(x, n):
+    assert k < 128 or n < 128
+    return
+  dw = hip.shared_linear_backward(x, y)
+  xt, dy = x.double().t().contiguous(), y.double()
+  want = xt @ dy
+  assert ((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() + rows * 2.0 ** -24 * (
+      xt.abs() @ dy.abs())).all()
+
+
+def test_shared_projections_see_assigned_weights():
+  """The packed kernels that lie in one tensor follow assignments, eager and in a
+  captured step."""
+  b, l, m = 2, 64, 128
+  gen = torch.Generator(device="cuda").manual_seed(12)
+
+  def draw(*sizes):
+    return torch.randn(sizes, generator=gen, device="cuda").bfloat16()
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("batch", b), mtf.Dimension("length", l),
+          mtf.Dimension("d_model", m)]
+  xt, dyt = (mtf.import_tf_tensor(mesh, draw(b, l, m), mtf.Shape(dims))
+             for _ in range(2))
+  stack = transformer.make_layer_stack(
+      [(transformer_layers.SelfAttention, dict(num_heads=2, key_value_size=64))],
+      num_layers=1, block_scope=False)
+  model = transformer.Unitransformer(stack, d_model=m, name="decoder",
+                                     autoregressive=True)
+  bf16 = torch.bfloat16
+  y, _ = model.call_layers(xt, mtf.VariableDType(bf16, bf16, bf16), mode="train")
+  variables = list(graph.all_variables)
+  wrt = [xt] + [v.outputs[0] for v in variables]
+  results = [y] + mtf.gradients([y], wrt, grad_ys=[dyt])
+
+  def values():
+    return {v.name: draw(*v.shape.to_integer_list) * m ** -0.5 for v in variables}
+
+  def lower(init):
+    return mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()},
+                        initial_values={n: v.clone() for n, v in init.items()})
+
+  def out(low):
+    return [low.export_to_tf_tensor(t).clone() for t in results]
+
+  def same(got, want):
+    assert all(torch.equal(a, c) for a, c in zip(got, want))
+  first, second, third = values(), values(), values()
+  want = [out(lower(v)) for v in (first, second, third)]
+  low = lower(first)
+  same(out(low), want[0])
+  for op in variables:
+    low.variables[op].assign(second[op.name])
+  low.run()
+  same(out(low), want[1])
+  step = low.capture()
+  for init, expected in ((third, want[2]), (first, want[0]), (second, want[1])):
+    for op in variables:
+      low.variables[op].assign(init[op.name])
+    step.replay()
+    same(out(low), expected)
+  joint = [v for v in low.variables.values() if any(v._together.values())]
+  assert len(joint) == 1
