@@ -319,6 +319,82 @@ __global__ __launch_bounds__(256) void router_mfma_kernel(
                         min(TOK, tokens - t0));
 }
 
+// The same products for few tokens, in the same order (the bits of router_mfma_kernel): a
+// wavefront per 32 tokens and 32 experts, operands straight into registers.  A block of
+// 128 tokens that has the whole chip to itself is bound by its chain of K tiles, a
+// barrier and a round trip each; here two batches of four K tiles are in flight and
+// nobody waits for another wavefront: 64 tokens of 4096, 64 experts 31.9 -> 16.4 us.
+__global__ __launch_bounds__(64) void router_few_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ wp,
+    const float* __restrict__ bias, float* __restrict__ logits, int tokens,
+    int M, int E) {
+  constexpr int BK = 64, TILES = 4;
+  const int lane = threadIdx.x, fr = lane & 31, fc = lane >> 5;
+  const int t0 = blockIdx.x * 32, e0 = blockIdx.y * 32, b = blockIdx.z;
+  const int tok = t0 + fr;
+  const bf16_t* xr = x + ((int64_t)b * tokens + min(tok, tokens - 1)) * M + fc * 8;
+  const bf16_t* wr = wp + ((int64_t)b * E + min(e0 + fr, E - 1)) * M + fc * 8;
+  const int nk = M / BK;
+  const int rot = (t0 / 128) % nk;            // where router_mfma_kernel starts
+  struct Batch { rl_bf16x8_t x[TILES * 4], w[TILES * 4]; };
+  auto load = [&](Batch& f, int kt) {
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+      int kq = min(kt + i, nk - 1) + rot;     // (past the end: read, not used)
+      if (kq >= nk) kq -= nk;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        f.x[i * 4 + kk] =
+            *reinterpret_cast<const rl_bf16x8_t*>(xr + kq * BK + kk * 16);
+        f.w[i * 4 + kk] =
+            *reinterpret_cast<const rl_bf16x8_t*>(wr + kq * BK + kk * 16);
+      }
+    }
+  };
+  rl_f32x16_t acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+  auto multiply = [&](const Batch& f, int kt) {
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+      if (kt + i >= nk) return;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[i * 4 + kk],
+                                                      f.x[i * 4 + kk], acc, 0, 0, 0);
+    }
+  };
+  Batch even, odd;
+  int kt = 0;
+  load(even, 0);
+  for (; kt + 2 * TILES < nk; kt += 2 * TILES) {
+    load(odd, kt + TILES);
+    multiply(even, kt);
+    load(even, kt + 2 * TILES);
+    multiply(odd, kt + TILES);
+  }
+  if (kt + TILES < nk) {
+    load(odd, kt + TILES);
+    multiply(even, kt);
+    multiply(odd, kt + TILES);
+  } else {
+    multiply(even, kt);
+  }
+  if (tok >= tokens) return;
+  float* out = logits + ((int64_t)b * tokens + tok) * E;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int e = e0 + 8 * q + 4 * fc;        // E % 4 == 0: all four or none
+    if (e >= E) continue;
+    float4 v = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2],
+                           acc[4 * q + 3]);
+    if (bias != nullptr) {
+      v.x += bias[e]; v.y += bias[e + 1]; v.z += bias[e + 2]; v.w += bias[e + 3];
+    }
+    *reinterpret_cast<float4*>(out + e) = v;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Gating step 1: per token softmax, top-2, gate normalisation, second-place
 // policy; per block column sums of the balancing-loss proxies.
@@ -1771,6 +1847,17 @@ static int launch_router_mfma(const bf16_t* x, const bf16_t* wp,
   return 0;
 }
 
+// Whether a wavefront per 32 tokens and 32 experts beats a block per 128 tokens: while at
+// most two wavefronts share a compute unit.  In us, block / wavefront: 64 tokens of 1024,
+// 32 experts 7.6 / 6.0, 64 experts 9.9 / 6.0; 64 tokens of 4096, 64 experts 31.9 / 16.4;
+// 2048 tokens of 2048, 128 experts 27.4 / 10.0; 32 tokens of 64, 128 experts 3.6 / 3.0; two
+// per unit: 8192 tokens of 1024, 64 experts 11.4 / 10.9, of 4096 34.6 / 32.7; three and
+// four: 3 x 8192 of 1088, 16 experts 12.8 / 14.3, 8192 of 2048, 128 experts 28.2 / 32.3.
+static bool router_few_applies(int batch, int64_t tokens, int E) {
+  return batch * ((tokens + 31) / 32) * ((E + 31) / 32) <=
+         2 * (int64_t)compute_units();
+}
+
 extern "C" int mesh_moe_router_logits(const void* x, const void* w,
                                       const void* w_packed, const float* bias,
                                       float* logits, int batch, int64_t tokens,
@@ -1792,6 +1879,14 @@ extern "C" int mesh_moe_router_logits(const void* x, const void* w,
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wp = (const bf16_t*)w_packed;
     hipStream_t s2 = (hipStream_t)stream;
+    if (router_few_applies(batch, tokens, E)) {
+      dim3 grid((unsigned)((tokens + 31) / 32), (unsigned)((E + 31) / 32),
+                (unsigned)batch);
+      router_few_kernel<<<grid, 64, 0, s2>>>(xb, wp, bias, logits, (int)tokens, M,
+                                             E);
+      MOE_CHECK_LAUNCH("router_logits (mfma, few tokens)");
+      return 0;
+    }
     if (E <= 32)
       return launch_router_mfma<1>(xb, wp, bias, logits, batch, (int)tokens, M, E, s2);
     if (E <= 64)

@@ -138,6 +138,26 @@ def test_router_logits_edges(hip, shape, dtype):
   assert ((got - want).abs() <= bound).all()
 
 
+# a reduction of one K tile, of whole and of partly filled batches of tiles; tokens and
+# experts around the 32 of a wavefront; the row that the K tiles' rotation restarts at
+@pytest.mark.parametrize("tokens", [1, 31, 33, 200])
+@pytest.mark.parametrize("m,e", [(64, 4), (256, 36), (320, 32), (512, 64),
+                                 (576, 128), (1088, 100)])
+def test_router_logits_few_tokens(hip, tokens, m, e):
+  """Few tokens take a kernel of their own, with the bits that the same rows have in
+  a call with many."""
+  gen = torch.Generator(device="cuda").manual_seed(tokens + m + e)
+  x = torch.randn((40000, m), generator=gen, device="cuda").bfloat16()
+  w = torch.randn((m, e), generator=gen, device="cuda").bfloat16()
+  bias = torch.randn((e,), generator=gen, device="cuda")
+  packed = w.t().contiguous()
+  few = hip.router_logits(x[:tokens].clone(), w, bias, w_packed=packed)
+  assert torch.equal(few, hip.router_logits(x, w, bias, w_packed=packed)[:tokens])
+  batched = hip.router_logits(torch.stack([x[:tokens], x[:tokens] + 1]),
+                              torch.stack([w, w]), w_packed=torch.stack([packed] * 2))
+  assert torch.equal(batched[0], hip.router_logits(x, w, w_packed=packed)[:tokens])
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("shape", [(2, 1024, 512, 8), (3, 100, 72, 5),
                                    (1, 640, 1024, 128), (1, 15, 4, 17),
