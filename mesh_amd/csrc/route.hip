@@ -807,14 +807,11 @@ __host__ __device__ constexpr int select_row_floats(int E) {
 }                                        // for E = 8 n
 
 template <typename IT, int LANES>
-__global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
-    const float* __restrict__ logits, const IT* __restrict__ importance,
-    const float* __restrict__ second_uniform, GateParams p,
-    int32_t* __restrict__ idx, int32_t* __restrict__ pos,
-    float* __restrict__ gate, uint8_t* __restrict__ kept,
-    float* __restrict__ part1, float* __restrict__ part2) {
+__device__ __forceinline__ void gate_select_block(
+    const float* logits, const IT* importance, const float* second_uniform,
+    const GateParams& p, int32_t* idx, int32_t* pos, float* gate, uint8_t* kept,
+    float* part1, float* part2, float* smem) {
   constexpr int TOKENS = SELECT_THREADS / LANES;
-  extern __shared__ __attribute__((aligned(16))) float smem[];
   const int E = p.E, S = p.S;
   const int ld = select_row_floats(E);
   float* tile = smem;                                  // [TOKENS][ld]
@@ -834,10 +831,13 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   const bool sw = p.router == ROUTER_SWITCH;
 
   float m = -INFINITY;
+  // (here and below: the reads of four steps fly together)
+#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES) m = fmaxf(m, src[e]);
 #pragma unroll
   for (int d = 1; d < LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
   const float negm = -m;                                    // reduce_max
+#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES)
     row[e] = expf(src[e] + negm);
   __syncthreads();
@@ -845,6 +845,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   float s = 0.f;
   if (live) {
     int e = 0;
+#pragma unroll 4
     for (; e + 4 <= E; e += 4) {
       const float4 v = *reinterpret_cast<const float4*>(row + e);
       s += v.x; s += v.y; s += v.z; s += v.w;
@@ -864,6 +865,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
   const float neglse = -(logf(s) + m);                      // log + max
   float g1 = -1.f;
   int i1 = 0;
+#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES) {
     const float pe = expf(src[e] + neglse);                 // exp(log_softmax)
     row[e] = pe;
@@ -923,6 +925,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     const int masked = sel1 ? i1 : -1;                      // 1 + (-mask_1)
     float g2 = -1.f;
     int i2 = 0;
+#pragma unroll 4
     for (int e = lane; e < e_end; e += LANES) {
       const float q = row[e] * (e == masked ? 0.0f : 1.0f);
       if (q > g2) { g2 = q; i2 = e; }
@@ -930,6 +933,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     first_max(g2, i2);
     if (p.use_second_place_loss && live) {
       float qsum = 0.f;
+#pragma unroll 4
       for (int e = 0; e < E; ++e) qsum += row[e] * (e == masked ? 0.0f : 1.0f);
       qscale = 1.0f / (qsum + 1e-9f);                       // moe.py:1433-1434
     }
@@ -968,6 +972,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     __syncthreads();
     if (e < E && c < ranges) {
       float a = 0.f;
+#pragma unroll 4
       for (int r = c * per; r < min(ntok, (c + 1) * per); ++r)
         a += weights != nullptr ? tile[r * ld + e] * weights[r]
                                 : tile[r * ld + e];
@@ -976,6 +981,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     __syncthreads();
     if (tid < E) {
       float a = 0.f;
+#pragma unroll 8
       for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
       part[((int64_t)g * p.nblk + blk) * E + tid] = a;
     }
@@ -994,6 +1000,7 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
     __syncthreads();
     if (tid < 2) {
       float a = 0.f;
+#pragma unroll 8
       for (int r = 0; r < ntok; ++r) a += cols[tid * TOKENS + r];
       part2[((int64_t)g * p.nblk + blk) * E + tid] = a;
     }
@@ -1003,6 +1010,18 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
       row[e] = (row[e] * (sel1 && e == i1 ? 0.0f : 1.0f)) * qscale;
     column_sums(nullptr, part2);
   }
+}
+
+template <typename IT, int LANES>
+__global__ __launch_bounds__(SELECT_THREADS) void gate_select_kernel(
+    const float* __restrict__ logits, const IT* __restrict__ importance,
+    const float* __restrict__ second_uniform, GateParams p,
+    int32_t* __restrict__ idx, int32_t* __restrict__ pos,
+    float* __restrict__ gate, uint8_t* __restrict__ kept,
+    float* __restrict__ part1, float* __restrict__ part2) {
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  gate_select_block<IT, LANES>(logits, importance, second_uniform, p, idx, pos,
+                               gate, kept, part1, part2, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -1605,13 +1624,10 @@ __device__ __forceinline__ int cap_count(const int16_t* ch, int s_begin,
   return c;
 }
 
-__global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
-    GateParams p, const int32_t* __restrict__ idx, int32_t* __restrict__ pos,
-    float* __restrict__ gate, uint8_t* __restrict__ kept,
-    int32_t* __restrict__ fill, const float* __restrict__ part1,
-    const float* __restrict__ part2, float* __restrict__ gsum, int el, int ss,
-    float* __restrict__ loss) {
-  extern __shared__ __attribute__((aligned(16))) int32_t smem_i[];
+__device__ __forceinline__ void gate_capacity_group(
+    const GateParams& p, const int32_t* idx, int32_t* pos, float* gate,
+    uint8_t* kept, int32_t* fill, const float* part1, const float* part2,
+    float* gsum, int el, int ss, float* loss, int32_t* smem_i, int g) {
   const int S = p.S, E = p.E, C = p.C;
   int32_t* cnt = smem_i;                        // [nchunks][el] = CAP_THREADS
   int32_t* pre = cnt + CAP_THREADS;             // [nchunks][el]: first slots
@@ -1629,7 +1645,6 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
   float* lg = gl + S;                                         // [S]
   int32_t* lpos = reinterpret_cast<int32_t*>(lg + S);         // [S]
   int32_t* ebase = lpos + S;                                  // [el]
-  const int g = blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t base = (int64_t)g * S;
   const bool sw = p.router == ROUTER_SWITCH;
@@ -1672,6 +1687,7 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     cnt[chunk * el + e] = cap_count(ch, s_begin, s_end, e, vec);
     __syncthreads();
     int before = 0, total = 0;
+#pragma unroll 4
     for (int k = super * q; k < (super + 1) * q; ++k) {
       const int v = cnt[k * el + e];
       total += v;
@@ -1680,6 +1696,7 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     if (chunk == super * q) pre[super * el + e] = total;
     __syncthreads();
     total = 0;
+#pragma unroll 4
     for (int k = 0; k < nchunks / q; ++k) {
       const int v = pre[k * el + e];
       total += v;
@@ -1751,6 +1768,7 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     __syncthreads();
     if (chunk == 0 && e < E) {
       int total = 0;
+#pragma unroll 8
       for (int k = 0; k < nchunks; ++k) total += cnt[k * el + e];
       tot[2 * el + e] = total;
     }
@@ -1812,8 +1830,10 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
   __syncthreads();
   if (tid == 0) {
     float s1 = 0.f, s2 = 0.f;
+#pragma unroll 8
     for (int k = 0; k < E; ++k) s1 += prod[k];
     if (loss2 && !sw)
+#pragma unroll 8
       for (int k = 0; k < E; ++k) s2 += prod[el + k];
     gsum[g * GSUM] = s1;
     gsum[g * GSUM + 1] = s2;
@@ -1822,6 +1842,35 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
     // a single group's block needs no launch after it for the loss
     if (p.G == 1) gate_loss_value<false>(p, gsum, loss);
   }
+}
+
+__global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
+    GateParams p, const int32_t* __restrict__ idx, int32_t* __restrict__ pos,
+    float* __restrict__ gate, uint8_t* __restrict__ kept,
+    int32_t* __restrict__ fill, const float* __restrict__ part1,
+    const float* __restrict__ part2, float* __restrict__ gsum, int el, int ss,
+    float* __restrict__ loss) {
+  extern __shared__ __attribute__((aligned(16))) int32_t smem_i[];
+  gate_capacity_group(p, idx, pos, gate, kept, fill, part1, part2, gsum, el, ss,
+                      loss, smem_i, blockIdx.x);
+}
+
+// Both steps for a group that is one block of gate_select_kernel: what step 1 wrote is
+// read back by the same block.  (No pointer is __restrict__ here.)  Each step alone is
+// bound by being a launch.
+template <typename IT, int LANES>
+__global__ __launch_bounds__(SELECT_THREADS) void gate_small_groups_kernel(
+    const float* logits, const IT* importance, const float* second_uniform,
+    GateParams p, int32_t* idx, int32_t* pos, float* gate, uint8_t* kept,
+    int32_t* fill, float* part1, float* part2, float* gsum, int el, int ss,
+    float* loss) {
+  static_assert(SELECT_THREADS == CAP_THREADS, "one block does both steps");
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  gate_select_block<IT, LANES>(logits, importance, second_uniform, p, idx, pos,
+                               gate, kept, part1, part2, smem);
+  __syncthreads();
+  gate_capacity_group(p, idx, pos, gate, kept, fill, part1, part2, gsum, el, ss,
+                      loss, reinterpret_cast<int32_t*>(smem), blockIdx.y);
 }
 
 __global__ void gate_loss_kernel(GateParams p, const float* __restrict__ gsum,
@@ -1916,12 +1965,17 @@ extern "C" int mesh_moe_router_logits(const void* x, const void* w,
 }
 
 // Gating steps 2 and 3 (capacity positions, balancing loss) for every group.
-static int launch_capacity_and_loss(const GateParams& p, int32_t* idx,
-                                    int32_t* pos, float* gate, uint8_t* kept,
-                                    int32_t* fill, float* loss,
-                                    const float* part1, const float* part2,
-                                    float* gsum, hipStream_t st) {
-  int el = 2;
+static int launch_loss(const GateParams& p, const float* gsum, float* loss,
+                       hipStream_t st) {
+  if (p.G == 1) return 0;                // a single group's block made it
+  gate_loss_kernel<<<1, 64, 0, st>>>(p, gsum, loss);
+  MOE_CHECK_LAUNCH("gate_loss");
+  return 0;
+}
+
+// LDS of gate_capacity_group, its padded numbers of experts and of tokens.
+static size_t capacity_lds(const GateParams& p, int& el, int& ss) {
+  el = 2;
   while (el < p.E) el *= 2;
   // the id arrays padded to multiples of eight ids, for 16-byte reads, unless
   // a group as large as LDS takes leaves no room for it
@@ -1931,16 +1985,22 @@ static int launch_capacity_and_loss(const GateParams& p, int32_t* idx,
            (p.rank_by_gate ? sizeof(float) * (3 * (size_t)p.S + el) : 0);
   };
   const int padded = (p.S + 7) / 8 * 8;
-  const int ss = lds_bytes(padded) <= 160 * 1024 ? padded : p.S;
-  const size_t smem = lds_bytes(ss);
+  ss = lds_bytes(padded) <= 160 * 1024 ? padded : p.S;
+  return lds_bytes(ss);
+}
+
+static int launch_capacity_and_loss(const GateParams& p, int32_t* idx,
+                                    int32_t* pos, float* gate, uint8_t* kept,
+                                    int32_t* fill, float* loss,
+                                    const float* part1, const float* part2,
+                                    float* gsum, hipStream_t st) {
+  int el, ss;
+  const size_t smem = capacity_lds(p, el, ss);
   MOE_ALLOW_LDS(gate_capacity_kernel, smem);
   gate_capacity_kernel<<<p.G, CAP_THREADS, smem, st>>>(
       p, idx, pos, gate, kept, fill, part1, part2, gsum, el, ss, loss);
   MOE_CHECK_LAUNCH("gate_capacity");
-  if (p.G == 1) return 0;
-  gate_loss_kernel<<<1, 64, 0, st>>>(p, gsum, loss);
-  MOE_CHECK_LAUNCH("gate_loss");
-  return 0;
+  return launch_loss(p, gsum, loss, st);
 }
 
 static int check_gating_args(int G, int S, int E, int C, int policy,
@@ -2071,8 +2131,24 @@ static int run_gating(const GateParams& p, const float* logits,
     MOE_CHECK_LAUNCH("gate_select");
     return 0;
   };
+  int el, ss;
+  const size_t cap_smem = capacity_lds(p, el, ss);
+  // (with more groups than compute units the two kernels overlap better: 300 groups of
+  // 40 tokens, 16 experts 48.5 us apart and 49.2 in one, 1000 of 64, 128 experts 128 and
+  // 135; 64 of 64, 64 experts 18.5 and 17.5; one of 64 12.7 and 11.9)
+  const bool one_block = p.nblk == 1 && p.tt == 64 && G <= 128;
   auto run_lanes = [&](auto* imp) -> int {
     using IT = std::remove_const_t<std::remove_pointer_t<decltype(imp)>>;
+    if (one_block) {
+      auto k = gate_small_groups_kernel<IT, SELECT_THREADS / 64>;
+      const size_t both = smem > cap_smem ? smem : cap_smem;
+      MOE_ALLOW_LDS(k, both);
+      k<<<grid, SELECT_THREADS, both, st>>>(logits, imp, second_uniform, p, idx, pos,
+                                         gate, kept, fill, part1, part2, gsum, el,
+                                         ss, loss);
+      MOE_CHECK_LAUNCH("gate_small_groups");
+      return launch_loss(p, gsum, loss, st);
+    }
     switch (p.tt) {
       case 64: return run(gate_select_kernel<IT, 16>, imp);
       case 128: return run(gate_select_kernel<IT, 8>, imp);
@@ -2082,7 +2158,7 @@ static int run_gating(const GateParams& p, const float* logits,
   const int rc = importance && importance_dtype == MESH_MOE_BF16
                      ? run_lanes((const bf16_t*)importance)
                      : run_lanes((const float*)importance);
-  if (rc != 0) return rc;
+  if (rc != 0 || one_block) return rc;
   return launch_capacity_and_loss(p, idx, pos, gate, kept, fill, loss, part1,
                                   part2, gsum, st);
 }

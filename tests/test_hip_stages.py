@@ -138,6 +138,31 @@ def test_router_logits_edges(hip, shape, dtype):
   assert ((got - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("s,e", [(1, 2), (3, 512), (17, 5), (63, 16), (64, 64)])
+@pytest.mark.parametrize("router", ["top2", "switch"])
+def test_small_groups_gating(hip, router, s, e):
+  """Groups of at most 64 tokens are gated by one launch where they are few: the bits
+  of the launch per step that many groups take."""
+  gen = torch.Generator(device="cuda").manual_seed(s + e)
+  logits = torch.randn((200, s, e), generator=gen, device="cuda")
+  logits[0, s // 2] = 0.25                      # equal probabilities
+  importance = torch.randint(0, 3, (200, s), generator=gen, device="cuda") / 2
+  capacity = max(1, s // 4)
+  for imp in (None, importance):
+    def gating(g):
+      some = None if imp is None else imp[:g].contiguous()
+      if router == "switch":
+        return hip.switch_gating(logits[:g].contiguous(), capacity, importance=some,
+                                 z_loss=0.01, slots_by_gate=e % 2 == 0)
+      return hip.top2_gating(logits[:g].contiguous(), capacity, importance=some,
+                             policy="threshold", use_second_place_loss=True)
+    many = gating(200)
+    for g in (1, 2, 128):
+      few = gating(g)
+      for name in ("idx", "pos", "gate", "kept", "fill"):
+        assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
+
+
 # a reduction of one K tile, of whole and of partly filled batches of tiles; tokens and
 # experts around the 32 of a wavefront; the row that the K tiles' rotation restarts at
 @pytest.mark.parametrize("tokens", [1, 31, 33, 200])
