@@ -672,14 +672,13 @@ template <bool RELU, bool GATHER = false, bool KMAJOR = false,
 __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
     bf16_t* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
-    int total_tiles, const int32_t* __restrict__ row_map = nullptr,
-    const bf16_t* __restrict__ zero_row = nullptr,
-    const bf16_t* __restrict__ mask_src = nullptr,
-    const int32_t* __restrict__ tile_list = nullptr,
-    const int32_t* __restrict__ row_count = nullptr,
-    float mask_scale = 1.0f, float* __restrict__ partial = nullptr,
-    int whole_tiles = 0, int split = 1, int tile_rows = RingCfg::BM,
-    int64_t a_stride = -1) {
+    int total_tiles, const int32_t* __restrict__ row_map,
+    const bf16_t* __restrict__ zero_row,
+    const bf16_t* __restrict__ mask_src,
+    const int32_t* __restrict__ tile_list,
+    const int32_t* __restrict__ row_count,
+    float mask_scale, float* __restrict__ partial,
+    int whole_tiles, int split, int tile_rows, int64_t a_stride) {
   using Cfg = RingCfg;
   // row_count [E], optional: KMAJOR kernels take it as the reduction extent
   // per expert (k_extent)
@@ -828,8 +827,10 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         }
       }
     }
-    // (a_stride 0: all experts read the same rows)
-    Ae = GATHER ? A : A + e * (a_stride < 0 ? (int64_t)R * K : a_stride);
+    // (a_stride 0: all experts read the same rows, -1: each its own)
+    if constexpr (GATHER) Ae = A;
+    else if constexpr (LISTED || MASKED) Ae = A + (int64_t)e * R * K;
+    else Ae = A + e * (a_stride < 0 ? (int64_t)R * K : a_stride);
     Be = B + (int64_t)e * N * K;
     Ce = Cout + (int64_t)e * R * N;
 #pragma unroll
