@@ -831,13 +831,10 @@ __device__ __forceinline__ void gate_select_block(
   const bool sw = p.router == ROUTER_SWITCH;
 
   float m = -INFINITY;
-  // (here and below: the reads of four steps fly together)
-#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES) m = fmaxf(m, src[e]);
 #pragma unroll
   for (int d = 1; d < LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
   const float negm = -m;                                    // reduce_max
-#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES)
     row[e] = expf(src[e] + negm);
   __syncthreads();
@@ -845,7 +842,6 @@ __device__ __forceinline__ void gate_select_block(
   float s = 0.f;
   if (live) {
     int e = 0;
-#pragma unroll 4
     for (; e + 4 <= E; e += 4) {
       const float4 v = *reinterpret_cast<const float4*>(row + e);
       s += v.x; s += v.y; s += v.z; s += v.w;
@@ -865,7 +861,6 @@ __device__ __forceinline__ void gate_select_block(
   const float neglse = -(logf(s) + m);                      // log + max
   float g1 = -1.f;
   int i1 = 0;
-#pragma unroll 4
   for (int e = lane; e < e_end; e += LANES) {
     const float pe = expf(src[e] + neglse);                 // exp(log_softmax)
     row[e] = pe;
@@ -925,7 +920,6 @@ __device__ __forceinline__ void gate_select_block(
     const int masked = sel1 ? i1 : -1;                      // 1 + (-mask_1)
     float g2 = -1.f;
     int i2 = 0;
-#pragma unroll 4
     for (int e = lane; e < e_end; e += LANES) {
       const float q = row[e] * (e == masked ? 0.0f : 1.0f);
       if (q > g2) { g2 = q; i2 = e; }
@@ -933,7 +927,6 @@ __device__ __forceinline__ void gate_select_block(
     first_max(g2, i2);
     if (p.use_second_place_loss && live) {
       float qsum = 0.f;
-#pragma unroll 4
       for (int e = 0; e < E; ++e) qsum += row[e] * (e == masked ? 0.0f : 1.0f);
       qscale = 1.0f / (qsum + 1e-9f);                       // moe.py:1433-1434
     }
@@ -972,7 +965,6 @@ __device__ __forceinline__ void gate_select_block(
     __syncthreads();
     if (e < E && c < ranges) {
       float a = 0.f;
-#pragma unroll 4
       for (int r = c * per; r < min(ntok, (c + 1) * per); ++r)
         a += weights != nullptr ? tile[r * ld + e] * weights[r]
                                 : tile[r * ld + e];
@@ -981,7 +973,6 @@ __device__ __forceinline__ void gate_select_block(
     __syncthreads();
     if (tid < E) {
       float a = 0.f;
-#pragma unroll 8
       for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
       part[((int64_t)g * p.nblk + blk) * E + tid] = a;
     }
@@ -1000,7 +991,6 @@ __device__ __forceinline__ void gate_select_block(
     __syncthreads();
     if (tid < 2) {
       float a = 0.f;
-#pragma unroll 8
       for (int r = 0; r < ntok; ++r) a += cols[tid * TOKENS + r];
       part2[((int64_t)g * p.nblk + blk) * E + tid] = a;
     }
