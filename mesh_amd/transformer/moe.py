@@ -412,6 +412,14 @@ def _release_saved(saved):
     saved.clear()
 
 
+def _scaled_loss(loss, coef):
+  """loss * coef; a coefficient that is a Tensor of the graph (a schedule) is an
+  ordinary product."""
+  if isinstance(coef, mtf.Tensor):
+    return loss * coef
+  return ScaledLossOperation(loss, coef).outputs[0]
+
+
 class ScaledLossOperation(mtf.Operation):
   """The layer's loss times moe_loss_coef (transformer/moe.py:526-529), made by the
   layer's last kernel where that can (MoEV1Operation)."""
@@ -986,8 +994,7 @@ def transformer_moe_layer_v1(
         hidden_keep_prob=hidden_keep_prob).outputs
     outputs = [mtf.reshape(t, batch_and_length_dims + [output_dim])
                for t in (q, k)]
-    return outputs, ScaledLossOperation(
-        loss, hparams.moe_loss_coef).outputs[0]
+    return outputs, _scaled_loss(loss, hparams.moe_loss_coef)
   wo = mtf_layers.get_dense_kernel_weights(
       inputs, [output_dim], [hidden_dim], [experts_dim], None, name="wo",
       variable_dtype=variable_dtype)
@@ -996,8 +1003,7 @@ def transformer_moe_layer_v1(
       inputs, w_gate, wi, wo, nonpadding, output_dim, expert_capacity, gating,
       act_names, hidden_keep_prob=hidden_keep_prob).outputs
   output = mtf.reshape(output, batch_and_length_dims + [output_dim])
-  return output, ScaledLossOperation(
-      loss, hparams.moe_loss_coef).outputs[0]
+  return output, _scaled_loss(loss, hparams.moe_loss_coef)
 
 
 class MoEV2Operation(mtf.Operation):

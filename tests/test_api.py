@@ -415,6 +415,21 @@ def test_gradients_builds_the_backward_operation():
   assert any(isinstance(o, moe.MoEV2GradOperation) for o in g3.operations)
 
 
+@pytest.mark.parametrize("experts_attention", [False, True])
+def test_loss_coefficient_that_is_a_tensor(experts_attention):
+  """moe_loss_coef may be a Tensor of the graph (a schedule), with a gradient."""
+  _, mesh, x, dims = graph_input()
+  coef = mtf.import_tf_tensor(mesh, torch.tensor(0.5), mtf.Shape([]))
+  out_dim = mtf.Dimension("out", 8) if experts_attention else dims[-1]
+  _, loss = moe.transformer_moe_layer_v1(
+      x, out_dim, hparams(moe_loss_coef=coef,
+                          moe_use_experts_attention=experts_attention), True,
+      mtf.VariableDType(torch.float32))
+  assert loss.shape == mtf.Shape([])
+  grads = mtf.gradients([loss], [x, coef])
+  assert [g.shape for g in grads] == [x.shape, coef.shape]
+
+
 # ---- the transformer block around the layer -------------------------------------
 def _lm_moe_stack():
   from mesh_amd.transformer import transformer, transformer_layers
