@@ -159,7 +159,8 @@ class SharedInput(object):
     d = dys[0]
     n = d.shape[-1]
     step = d.numel()
-    if not (moe_hip.shared_linear_backward_supported(x, n) and all(
+    if not (moe_hip.shared_linear_backward_supported(x, n) and
+            d.data_ptr() % 16 == 0 and all(
         t.is_contiguous() and t.dtype == x.dtype and t.shape == d.shape and
         t.untyped_storage().data_ptr() == d.untyped_storage().data_ptr() and
         t.storage_offset() == d.storage_offset() + i * step

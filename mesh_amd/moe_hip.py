@@ -1438,12 +1438,14 @@ def rms_norm(x, scale, epsilon=1e-6):
   return out
 
 
-def residual_rms_norm_supported(x):
+def residual_rms_norm_supported(x, *others):
   """True if residual_rms_norm and the mask / addend of rms_norm_backward have a
-  kernel for rows like x's."""
+  kernel for rows like x's; `others`: what else the call reads in 16-byte pieces
+  (the other rows and the scale)."""
   m = x.shape[-1]
   return (x.dtype == torch.bfloat16 and m % 8 == 0 and m <= 4096 and
-          x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
+          x.numel() > 0 and all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                                for t in (x,) + others))
 
 
 def residual_rms_norm(x, residual, scale, epsilon=1e-6, row_mask=None):
