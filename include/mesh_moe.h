@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 39
+#define MESH_MOE_ABI_VERSION 40
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -903,13 +903,14 @@ int mesh_moe_rms_norm(const void* x, const void* scale, void* y, int64_t rows,
  * transformer/transformer.py:584-587) and the padding mask behind it
  * (sublayer_mask_padding, :469-489): sum = x + residual, y = rms_norm(sum) *
  * row_mask[row], each with the rounding it has as an operation of its own.
- * residual and sum [rows,M] may be NULL together, row_mask [rows] by itself; dtype
- * bf16, M % 8 == 0, M <= 4096, 16-byte aligned rows.  The backward call takes dy of
+ * residual and sum [rows,M] may be NULL together, row_mask [rows] by itself; norm
+ * [rows,M] (may be NULL) receives rms_norm(sum) without the mask; dtype bf16, M % 8
+ * == 0, M <= 4096, 16-byte aligned rows.  The backward call takes dy of
  * the masked result and adds `addend` [rows,M] (may be NULL) to dx.
  */
 int mesh_moe_residual_rms_norm(const void* x, const void* residual,
                                const void* scale, const void* row_mask, void* sum,
-                               void* y, int64_t rows, int M, double epsilon,
+                               void* norm, void* y, int64_t rows, int M, double epsilon,
                                int dtype, void* stream);
 int mesh_moe_residual_rms_norm_backward(
     const void* x, const void* scale, const void* dy, const void* row_mask,

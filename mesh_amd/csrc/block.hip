@@ -93,14 +93,15 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
 // With `residual` the row is x + residual, rounded to bf16, and is also written to
 // `sum`; with `row_mask` [rows] the result is multiplied by the row's value: the
 // residual sum and the padding mask around a norm, with the roundings they have as
-// operations of their own.  Bound by memory: 16384 x 1024, sum and norm 25.5 us (5.3
+// operations of their own; `norm_out` (or null) receives the norm without the mask.
+// Bound by memory: 16384 x 1024, sum and norm 25.5 us (5.3
 // TB/s; by themselves 17 + 13), 16000 x 768, sum, norm and mask 21 (12 + 11 + 14).
 template <int ITERS>
 __global__ __launch_bounds__(256) void rms_norm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,
     bf16_t* __restrict__ y, int64_t rows, int M, float inv_m, float eps,
     const bf16_t* __restrict__ residual, bf16_t* __restrict__ sum_out,
-    const bf16_t* __restrict__ row_mask) {
+    const bf16_t* __restrict__ row_mask, bf16_t* __restrict__ norm_out) {
   using T = bf16_t;
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -172,6 +173,8 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(
       o[j] = f32x2_to_bf16x2(round_to<T>(a * r) * sa, round_to<T>(b * r) * sb);
     }
     uint4 v = make_uint4(o[0], o[1], o[2], o[3]);
+    if (norm_out != nullptr)
+      store_streaming(reinterpret_cast<uint4*>(norm_out + row * M) + c, v);
     if (row_mask != nullptr) {
       float f[8];
       unpack16(v, f, T());
@@ -1115,18 +1118,19 @@ extern "C" int mesh_moe_attention_weights(const void* q, const void* k,
 static void launch_rms_norm_rows(const bf16_t* x, const bf16_t* scale, bf16_t* y,
                                  int64_t rows, int M, float inv_m, float eps,
                                  const bf16_t* residual, bf16_t* sum,
-                                 const bf16_t* row_mask, hipStream_t st) {
+                                 const bf16_t* row_mask, bf16_t* norm,
+                                 hipStream_t st) {
   auto k = M <= 1024 ? rms_norm_rows_kernel<2>
                      : M <= 2048 ? rms_norm_rows_kernel<4> : rms_norm_rows_kernel<8>;
   k<<<(unsigned)((rows + 3) / 4), 256, 0, st>>>(x, scale, y, rows, M, inv_m, eps,
-                                                residual, sum, row_mask);
+                                                residual, sum, row_mask, norm);
 }
 
 extern "C" int mesh_moe_residual_rms_norm(const void* x, const void* residual,
                                           const void* scale, const void* row_mask,
-                                          void* sum, void* y, int64_t rows, int M,
-                                          double epsilon, int dtype,
-                                          void* stream) {
+                                          void* sum, void* norm, void* y,
+                                          int64_t rows, int M, double epsilon,
+                                          int dtype, void* stream) {
   MOE_REQUIRE(x && scale && y && (residual == nullptr) == (sum == nullptr),
               MESH_MOE_E_ARG, "residual_rms_norm: null pointer");
   MOE_REQUIRE(valid_dtype(dtype), MESH_MOE_E_ARG,
@@ -1136,14 +1140,15 @@ extern "C" int mesh_moe_residual_rms_norm(const void* x, const void* residual,
   MOE_REQUIRE(dtype == MESH_MOE_BF16 && M % 8 == 0 && M <= 4096 &&
                   (rows + 3) / 4 <= 0x7fffffffLL &&
                   (((uintptr_t)x | (uintptr_t)residual | (uintptr_t)scale |
-                    (uintptr_t)sum | (uintptr_t)y) % 16 == 0),
+                    (uintptr_t)sum | (uintptr_t)norm | (uintptr_t)y) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,
               "residual_rms_norm: needs bf16 rows of 8 n <= 4096 elements on 16 "
               "bytes (M=%d dtype=%d)", M, dtype);
   launch_rms_norm_rows((const bf16_t*)x, (const bf16_t*)scale, (bf16_t*)y, rows, M,
                        round_bf16_host((float)(1.0 / (double)M)),
                        round_bf16_host((float)epsilon), (const bf16_t*)residual,
-                       (bf16_t*)sum, (const bf16_t*)row_mask, (hipStream_t)stream);
+                       (bf16_t*)sum, (const bf16_t*)row_mask, (bf16_t*)norm,
+                       (hipStream_t)stream);
   MOE_CHECK_LAUNCH("residual_rms_norm");
   return 0;
 }
@@ -1175,7 +1180,7 @@ extern "C" int mesh_moe_rms_norm(const void* x, const void* scale, void* y,
     bf16_t* yb = (bf16_t*)y;
     if (vec16 && M <= 4096)
       launch_rms_norm_rows(xb, sb, yb, rows, M, inv_m, eps, nullptr, nullptr,
-                           nullptr, st);
+                           nullptr, nullptr, st);
     else
       rms_norm_kernel<bf16_t><<<(unsigned)blocks, 256, 0, st>>>(xb, sb, yb, rows,
                                                                 M, inv_m, eps,

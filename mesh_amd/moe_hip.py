@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 39
+ABI_VERSION = 40
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -225,7 +225,7 @@ _SIGNATURES = {
         _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
     "mesh_moe_residual_rms_norm": (ctypes.c_int, [
-        _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
         ctypes.c_double, ctypes.c_int, _vp]),
     "mesh_moe_residual_rms_norm_backward": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
@@ -1443,20 +1443,28 @@ def residual_rms_norm_supported(x, *others):
   kernel for rows like x's; `others`: what else the call reads in 16-byte pieces
   (the other rows and the scale)."""
   m = x.shape[-1]
-  return (x.dtype == torch.bfloat16 and m % 8 == 0 and m <= 4096 and
-          x.numel() > 0 and all(t.is_contiguous() and t.data_ptr() % 16 == 0
-                                for t in (x,) + others))
+  if x.dtype != torch.bfloat16 or m % 8 or m > 4096 or not x.numel():
+    return False
+  at = 0
+  for t in (x,) + others:
+    if not t.is_contiguous():
+      return False
+    at |= t.data_ptr()
+  return at % 16 == 0
 
 
-def residual_rms_norm(x, residual, scale, epsilon=1e-6, row_mask=None):
+def residual_rms_norm(x, residual, scale, epsilon=1e-6, row_mask=None,
+                      want_norm=False):
   """rms_norm(x + residual) * row_mask in one pass: x, residual (or None) [..., M],
-  row_mask [...] (or None) -> (x + residual or x itself, result)."""
+  row_mask [...] (or None) -> (x + residual or x itself, result).  want_norm (with
+  a row_mask): also the norm without the mask, as a third result."""
   lib = load_library()
   m = x.shape[-1]
   rows = x.numel() // m
   shape = tuple(x.shape)
   total = x if residual is None else torch.empty_like(x)
   out = torch.empty_like(x)
+  norm = torch.empty_like(x) if want_norm else None
   with _stage("rms_norm"):
     _check(lib.mesh_moe_residual_rms_norm(
         _dev(x, "x"),
@@ -1464,9 +1472,10 @@ def residual_rms_norm(x, residual, scale, epsilon=1e-6, row_mask=None):
         _dev(scale, "scale", x.dtype, (m,)),
         None if row_mask is None else _dev(row_mask, "row_mask", x.dtype,
                                            shape[:-1]),
-        None if residual is None else total.data_ptr(), out.data_ptr(), rows, m,
+        None if residual is None else total.data_ptr(),
+        None if norm is None else norm.data_ptr(), out.data_ptr(), rows, m,
         float(epsilon), dtype_code(x.dtype), _stream()), "residual_rms_norm")
-  return total, out
+  return (total, out, norm) if want_norm else (total, out)
 
 
 def dense(x, w_packed, activation=None):

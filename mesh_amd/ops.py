@@ -1184,12 +1184,13 @@ def gradients(ys, xs, grad_ys=None, operations=None):
           for inp, grad in zip(op.inputs, input_grads):
             if inp in downstream and grad is not None:
               if inp in tensor_to_gradient:
-                # (an operation that can add to its result while it writes it)
+                # (an operation that can add to its result while it writes it;
+                # nobody else has seen that result yet)
                 add_to = getattr(grad.operation, "add_to_output", None)
-                total = add_to(grad, tensor_to_gradient[inp]) if add_to else None
-                if total is None:
-                  total = tensor_to_gradient[inp] + grad
-                tensor_to_gradient[inp] = total
+                if add_to and add_to(grad, tensor_to_gradient[inp]):
+                  tensor_to_gradient[inp] = grad
+                else:
+                  tensor_to_gradient[inp] = tensor_to_gradient[inp] + grad
               else:
                 tensor_to_gradient[inp] = grad
   finally:

@@ -1926,3 +1926,44 @@ def test_shared_projection_gradients_of_odd_views():
               2.0 ** -8 * want.abs() +
               rows * 2.0 ** -24 * (xt.abs() @ dy.abs())).all()
     low.run()
+
+
+def test_layer_stack_intermediates_are_those_of_the_run():
+  """Every tensor of a run holds what the run computed, whatever happens to the
+  variables and to the fed buffers after it."""
+  b, l, m = 2, 24, 64
+  gen = torch.Generator(device="cuda").manual_seed(33)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("batch", b), mtf.Dimension("length", l),
+          mtf.Dimension("d_model", m)]
+  ids = torch.ones((b, l), dtype=torch.int32, device="cuda")
+  ids[0, 15:] = 0
+  fed = [_bf16_at(gen, False, b, l, m) for _ in range(2)] + [ids]
+  xt, dyt = [mtf.import_tf_tensor(mesh, t, mtf.Shape(dims)) for t in fed[:2]]
+  idt = mtf.import_tf_tensor(mesh, ids, mtf.Shape(dims[:2]))
+  stack = transformer.make_layer_stack(
+      [(transformer_layers.DenseReluDense, dict(hidden_size=96)),
+       (transformer_layers.DenseReluDense, dict(hidden_size=32))],
+      num_layers=1, block_scope=False)
+  model = transformer.Unitransformer(stack, d_model=m, name="decoder",
+                                     autoregressive=True)
+  bf16 = torch.bfloat16
+  y, _ = model.call_layers(xt, mtf.VariableDType(bf16, bf16, bf16), mode="train",
+                           sequence_id=idt)
+  variables = list(graph.all_variables)
+  mtf.gradients([y], [xt] + [v.outputs[0] for v in variables], grad_ys=[dyt])
+  init = {v.name: _bf16_at(gen, False, *v.shape.to_integer_list)
+          for v in variables}
+  low = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()}, initial_values=init)
+  low.run()
+  tensors = [t for op in graph.operations for t in op.outputs
+             if op.inputs and not isinstance(op, mtf.Variable)]
+  before = {t: low.export_to_tf_tensor(t).clone() for t in tensors}
+  low.run()
+  for v in variables:
+    low.variables[v].assign(_bf16_at(gen, False, *v.shape.to_integer_list))
+  for t in fed:
+    t.zero_()
+  for t in tensors:
+    assert torch.equal(low.export_to_tf_tensor(t), before[t]), t
