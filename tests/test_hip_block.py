@@ -1967,3 +1967,26 @@ def test_layer_stack_intermediates_are_those_of_the_run():
     t.zero_()
   for t in tensors:
     assert torch.equal(low.export_to_tf_tensor(t), before[t]), t
+
+
+def test_norm_scale_that_the_graph_computes():
+  """A norm whose scale is not a variable but made by an operation behind the
+  residual sum: every run takes the scale of that run."""
+  gen = torch.Generator(device="cuda").manual_seed(34)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("rows", 12), mtf.Dimension("d_model", 64)]
+  x, residual = [mtf.import_tf_tensor(mesh, _bf16_at(gen, False, 12, 64),
+                                      mtf.Shape(dims)) for _ in range(2)]
+  factor = mtf.import_tf_tensor(mesh, _bf16_at(gen, False, 64),
+                                mtf.Shape(dims[1:]))
+  total = transformer.ResidualAddOperation(x, residual).outputs[0]
+  y = transformer.RmsNormOperation(total, factor * 2.0, 1e-6).outputs[0]
+  low = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()})
+  for _ in range(3):
+    value = _bf16_at(gen, False, 64)
+    low.run({factor: value})
+    want = B.rms_norm(H.to_np(low.export_to_tf_tensor(total)),
+                      H.to_np(2 * value), "bfloat16")
+    np.testing.assert_allclose(H.to_np(low.export_to_tf_tensor(y)), want,
+                               rtol=1.6e-2, atol=1e-3)
