@@ -898,31 +898,34 @@ def multiply(x1, x2, output_shape=None, name=None):
     def fn(a, b):
       return a * b.reshape(view).to(a.dtype)
 
-    reduced = [i for i, d in enumerate(big.shape.dims)
-               if d not in small.shape.dims]
-    small_sizes = small.shape.to_integer_list
-
-    def small_grad_fn(dy, a):
-      prod = dy.to(torch.float32) * a.to(torch.float32)
-      if reduced:
-        prod = prod.sum(dim=reduced)
-      return prod.reshape(small_sizes).to(small.dtype)
-
     def grad(op, dy):
-      # (a mask or another constant of the graph needs none: no reduction
-      # over the activations is built for it)
-      d_small = None
-      if _gradient_wanted(op.inputs[1]):
-        d_small = slicewise(small_grad_fn, [dy, op.inputs[0]],
-                            output_shape=small.shape, output_dtype=small.dtype,
-                            name="mul_grad_small")
-      return [multiply(dy, op.inputs[1]), d_small]
+      return [multiply(dy, op.inputs[1]), smaller_factor_gradient(op, dy)]
     return slicewise(
         fn, [big, small], output_shape=big.shape, output_dtype=big.dtype,
         name=name or "mul", grad_function=grad)
   c = _scalar_in(x1.dtype, x2)
   return cwise(lambda t: t * c, [x1], name=name or "scalar_mul",
                grad_function=lambda op, dy: [multiply(dy, x2)])
+
+
+def smaller_factor_gradient(op, dy):
+  """Inside the gradient of op, a product of its first input and a second one that
+  may lack some of the first one's dims: the gradient of the second.  None where
+  nobody asks for it (a mask or another constant of the graph: no reduction over the
+  activations is built for it)."""
+  big, small = op.inputs
+  if not _gradient_wanted(small):
+    return None
+  reduced = [i for i, d in enumerate(big.shape.dims) if d not in small.shape.dims]
+  small_sizes = small.shape.to_integer_list
+
+  def fn(dy, a):
+    prod = dy.to(torch.float32) * a.to(torch.float32)
+    if reduced:
+      prod = prod.sum(dim=reduced)
+    return prod.reshape(small_sizes).to(small.dtype)
+  return slicewise(fn, [dy, big], output_shape=small.shape,
+                   output_dtype=small.dtype, name="mul_grad_small")
 
 
 class ScalarSummaryOperation(Operation):

@@ -1990,3 +1990,28 @@ def test_norm_scale_that_the_graph_computes():
                       H.to_np(2 * value), "bfloat16")
     np.testing.assert_allclose(H.to_np(low.export_to_tf_tensor(y)), want,
                                rtol=1.6e-2, atol=1e-3)
+
+
+def test_padding_mask_has_a_gradient_where_it_is_asked_for():
+  """d mask = the sum of dy * x over the model dimension, as for any product of the
+  graph."""
+  gen = torch.Generator(device="cuda").manual_seed(35)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("batch", 3), mtf.Dimension("length", 20),
+          mtf.Dimension("d_model", 64)]
+  x, dy = [mtf.import_tf_tensor(mesh, _bf16_at(gen, False, 3, 20, 64),
+                                mtf.Shape(dims)) for _ in range(2)]
+  mask = mtf.import_tf_tensor(mesh, _bf16_at(gen, False, 3, 20),
+                              mtf.Shape(dims[:2]))
+  y = transformer.MaskPaddingOperation(x, mask).outputs[0]
+  dx, dmask = mtf.gradients([y], [x, mask], grad_ys=[dy])
+  low = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()})
+  xv, dyv, mv = [low.export_to_tf_tensor(t) for t in (x, dy, mask)]
+  assert torch.equal(low.export_to_tf_tensor(dx), dyv * mv[..., None])
+  want = (xv.double() * dyv.double()).sum(-1)
+  got = low.export_to_tf_tensor(dmask)
+  assert got.dtype == torch.bfloat16
+  # a bf16 rounding of a float32 sum of 64 products
+  assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -18 *
+          (xv.double() * dyv.double()).abs().sum(-1)).all()
