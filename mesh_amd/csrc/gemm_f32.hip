@@ -39,8 +39,11 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 //
 // A sum with an infinity, a NaN or an overflow in it is not what the terms give
 // (inf - inf, inf * 0).  Whatever such an operand touches comes out as an
-// infinity or a NaN; a wavefront that finds one among its results computes its
-// sub-tile again with float32 multiply-adds, in order of k.
+// infinity or a NaN; a wavefront that finds one among its sums (and the ones that it
+// shares k with) makes them again on v_mfma_f32_16x16x4_f32, operands straight from
+// memory.  8 x 1024 rows, K = 2048, 512 columns: 113 us, 440 with NaN everywhere;
+// weight gradients of these sizes 129 and 313.  (A chain of multiply-adds per element
+// took 15400 and 16600.)
 //
 // TM x TN MFMA tiles per wavefront; WN wavefronts along N times WK wavefronts
 // that share out the k of every K tile and add up their sums in the end.  All
@@ -135,6 +138,8 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
   constexpr int KS = Cfg::KS;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   bf16_t* As = reinterpret_cast<bf16_t*>(smem_raw);   // [2][3][BM][LDR]
+  __shared__ int again;           // WK > 1: the sums are made again
+  if (threadIdx.x == 0) again = 0;
   // an XCD works on a contiguous range of tiles, which share weight panels
   const int nblk = gridDim.x;
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -354,11 +359,96 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
     products(S0(), std::false_type(), 0);
     barrier();
   }
-  if constexpr (WK > 1) {
+  // 0 x is 0 only for finite x
+  float test[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        test[r] = __builtin_fmaf(acc[i][j][r], 0.f, test[r]);
+  bool redo = __any(!(test[0] + test[1] + test[2] + test[3] == 0.f));
+  auto sums_from_operands = [&]() {
+    // two MFMAs of 4 k at a time, which the wavefronts that share k take in turn: the
+    // q-th has k = 8 g + 2 (lane / 16) + q, with KMAJOR 8 g + 4 q + lane / 16
+    constexpr int NQ = 2;
+    const int groups = (K + 7) / 8;
+    int64_t a_at[TM], b_at[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      a_at[i] = (int64_t)min(row0 + i * 16 + (lane & 15), R - 1) * (KMAJOR ? 1 : K);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      b_at[j] = (int64_t)min(col0 + (wn * TN + j) * 16 + (lane & 15), N - 1) *
+                (KMAJOR ? 1 : K);
+    float fa[TM][NQ], fb[TN][NQ];
+    // (past the end of k: zeros in both operands)
+    auto load = [&](int g) {
+      if constexpr (KMAJOR) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+          const int k = 8 * g + 4 * q + (lane >> 4);
+          const int64_t kk = min(k, K - 1);
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            const float v = Ae[kk * R + a_at[i]];
+            fa[i][q] = k < K ? v : 0.f;
+          }
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const float v = Be[kk * N + b_at[j]];
+            fb[j][q] = k < K ? v : 0.f;
+          }
+        }
+      } else {
+        const int k = 8 * g + 2 * (lane >> 4), kk = min(k, K - 2);
+        auto load2 = [&](const float* p, float (&f)[NQ]) {
+          const float2 v = *reinterpret_cast<const float2*>(p);
+          f[0] = k < K ? v.x : 0.f;
+          f[1] = k < K ? v.y : 0.f;
+        };
+#pragma unroll
+        for (int i = 0; i < TM; ++i) load2(Ae + a_at[i] + kk, fa[i]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) load2(Be + b_at[j] + kk, fb[j]);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+    load(wk);
+    for (int g = wk; g < groups; g += WK) {
+      float ca[TM][NQ], cb[TN][NQ];
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) ca[i][q] = fa[i][q];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) cb[j][q] = fb[j][q];
+      }
+      load(g + WK);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[j][q], ca[i][q],
+                                                             acc[i][j], 0, 0, 0);
+    }
+  };
+  if constexpr (WK == 1) {
+    if (redo) sums_from_operands();
+  } else {
     // [wk - 1][wn][TM][TN][4][64], where the stages were
     float* parts = reinterpret_cast<float*>(smem_raw);
     constexpr int SUB = TM * TN * 256, PART = WN * SUB;
-    if (wk > 0) {
+    auto store_part = [&]() {
+      if (wk == 0) return;
       float* dst = parts + (wk - 1) * PART + wn * SUB + lane;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -367,8 +457,15 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             dst[((i * TN + j) * 4 + r) * 64] = acc[i][j][r];
-    }
+    };
+    if (redo) again = 1;
+    store_part();
     __syncthreads();
+    if (again) {
+      sums_from_operands();
+      store_part();
+      __syncthreads();
+    }
     if (wk > 0) return;
 #pragma unroll
     for (int w = 0; w < WK - 1; ++w) {
@@ -385,29 +482,6 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
   float* Ce = Cout + (int64_t)e * R * N;
   const float* mask = mask_src == nullptr ? nullptr : mask_src + (int64_t)e * R * N;
   const int col_w = col0 + wn * TN * 16;
-  // 0 x is 0 only for finite x
-  float test = 0.f;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) test = __builtin_fmaf(acc[i][j][r], 0.f, test);
-  if (__any(!(test == 0.f))) {
-    for (int at = lane; at < BM * TN * 16; at += 64) {
-      const int row = row0 + at / (TN * 16), col = col_w + at % (TN * 16);
-      if (row >= R || col >= N) continue;
-      const int64_t sa = KMAJOR ? R : 1, sb = KMAJOR ? N : 1;
-      const float* pa = Ae + (KMAJOR ? (int64_t)row : (int64_t)row * K);
-      const float* pb = Be + (KMAJOR ? (int64_t)col : (int64_t)col * K);
-      float sum = 0.f;
-      for (int k = 0; k < K; ++k) sum = __builtin_fmaf(pa[k * sa], pb[k * sb], sum);
-      const int64_t c = (int64_t)row * N + col;
-      Ce[c] = finish_f32(sum, relu, mask != nullptr, mask ? mask[c] : 1.f,
-                         mask_scale);
-    }
-    return;
-  }
   const int m_l = lane & 15, n_l = (lane >> 4) * 4;
 #pragma unroll
   for (int i = 0; i < TM; ++i)

@@ -94,3 +94,87 @@ def test_infinities_nan_and_overflow(hip, shape, activation):
   sure[1, 0, 4] = True
   assert torch.equal(got[sure].nan_to_num(7.0, 1e300, -1e300),
                      want[sure].nan_to_num(7.0, 1e300, -1e300))
+
+
+# [experts, rows, columns, k]: one for each tile of the table, in its order, as a
+# product and as a weight gradient summed over k + 1 rows (128 x 256, 160 x 256, 160 x
+# 128, 64 x 128, 80 x 64, 96 x 64, 32 x 32, 16 x 32, 32 x 64, 96 x 256, 64 x 256, 64 x
+# 128 with K tiles of 32, 16 x 128); rows, columns and k all leave a remainder
+TILE_SHAPES = [
+    (7, 1760, 280, 36), (16, 2276, 72, 48), (24, 1400, 72, 72), (24, 36, 660, 228),
+    (4, 2224, 68, 204), (16, 1288, 32, 220), (1, 2084, 40, 348), (1, 36, 40, 332),
+    (7, 36, 584, 328), (3, 2028, 548, 36), (4, 692, 1084, 40), (2, 712, 916, 92),
+    (8, 36, 1040, 328)]
+
+
+@pytest.mark.parametrize("form", ["product", "masked", "weight gradient"])
+@pytest.mark.parametrize("shape", TILE_SHAPES)
+def test_infinities_and_nan_in_every_tile(hip, shape, form):
+  """Non-finite values in both operands, at the k that the last K tile takes twice
+  among others, do to every sum what they do in float64; the other sums of their
+  tiles keep their values."""
+  e, r, n, k = shape
+  gen = torch.Generator(device="cuda").manual_seed(sum(shape))
+  if form == "weight gradient":
+    k += 1
+  a, w = _values(gen, e, r, k), _values(gen, e, n, k)
+  for t in (a, w):
+    for at, value in enumerate(("inf", "-inf", "nan") * 2):
+      row = int(torch.randint(t.shape[1], (), generator=gen, device="cuda"))
+      back = int(torch.randint(min(k, 300), (), generator=gen, device="cuda"))
+      t[at % e, row, k - 1 - back] = float(value)
+  wt = w.transpose(1, 2).contiguous()
+  want = a.double() @ wt.double()
+  if form == "product":
+    got = hip.expert_linear(a, w, "linear")
+  elif form == "masked":
+    mask = torch.randn((e, r, n), generator=gen, device="cuda")
+    got, _ = hip.expert_linear_backward(torch.zeros_like(mask), a, w,
+                                        da_relu_mask=mask)
+    want = torch.where(mask > 0, want, torch.zeros_like(want))
+  else:
+    _, got = hip.expert_linear_backward(
+        a.transpose(1, 2).contiguous(), wt, torch.empty(e, r, n, device="cuda"),
+        want_da=False)
+  finite = want.isfinite()
+  assert not finite.all() and finite.any()
+  # (a tile that is made again is added k by k; what the mask clears is 0)
+  bound = (k + 20) * 2.0 ** -24 * (a.double().abs() @ wt.double().abs())
+  bound = bound.nan_to_num(0.0, 0.0)
+  assert ((got.double() - want).abs() <= bound)[finite].all()
+  assert torch.equal(got.double()[~finite].nan_to_num(7.0, 1e300, -1e300),
+                     want[~finite].nan_to_num(7.0, 1e300, -1e300))
+
+
+def _time_us(call, reps=5):
+  call()
+  times = []
+  for _ in range(reps):
+    start, end = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    start.record()
+    call()
+    end.record()
+    end.synchronize()
+    times.append(start.elapsed_time(end) * 1e3)
+  return sorted(times)[reps // 2]
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+def test_products_of_nan_take_no_more_than_a_few_times_as_long(hip, kmajor):
+  """A diverged step, all of whose gradients are NaN, still ends in time."""
+  e, r, n, k = 8, 1024, 512, 2048
+  gen = torch.Generator(device="cuda").manual_seed(6)
+  if kmajor:
+    a, dy = _values(gen, e, k, r), _values(gen, e, k, n)
+    w = torch.empty(e, r, n, device="cuda")
+    call = lambda t: hip.expert_linear_backward(a, t, w, want_da=False)[1]
+  else:
+    a, dy = _values(gen, e, r, k), _values(gen, e, n, k)
+    call = lambda t: hip.expert_linear(a, t, "linear")
+  finite = _time_us(lambda: call(dy))
+  dy = torch.full_like(dy, float("nan"))
+  assert call(dy).isnan().all()
+  # (the products in terms, then on float32 MFMAs at less than half their rate)
+  nan = _time_us(lambda: call(dy))
+  print("finite %.1f us, NaN %.1f us" % (finite, nan))
+  assert nan < 10 * finite
