@@ -15,9 +15,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 // ---------------------------------------------------------------------------
 // Every float32 is the sum of three bf16 terms, x = x1 + x2 + x3: x1 is x
 // rounded to bf16, x2 the remainder rounded, and what is left then has at most
-// 8 significant bits.  (Exactly, down to 2^-133, the last bit of a bf16
-// denormal: what an operand loses below that is less than 2^-134 of the other
-// operand.)  A product a b is then the sum of nine exact products, of which
+// 8 significant bits, which bf16 holds exactly down to 2^-133, the last bit of its
+// denormals.  A product a b is then the sum of nine exact products, of which
 // a2 b3, a3 b2 and a3 b3, together below 2^-26 |a b|, are left out; the other six
 // run on v_mfma_f32_16x16x32_bf16, which adds exact products into float32: 96 cycles
 // of the matrix pipe for 16 x 16 outputs and k = 32 instead of 256 of
@@ -33,15 +32,16 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 // 160 rows, 512 -> 2048 241 -> 132; 33 rows x 128, K = 4096, 32 experts 50 -> 28.
 // Bound by the bf16 matrix pipes (and the power cap) in large launches; in small
 // ones by the latency of a block's first loads and of its last stores, and by
-// making terms, 11 vector instructions per pair of values, which run beside the
+// making terms, 12 vector instructions per pair of values, which run beside the
 // MFMAs.  What stays behind is reductions of few K tiles (K = 200 and 260: 8.4 ->
 // 9.0 and 6.8 -> 7.3).
 //
 // A sum with an infinity, a NaN or an overflow in it is not what the terms give
 // (inf - inf, inf * 0).  Whatever such an operand touches comes out as an
-// infinity or a NaN; a wavefront that finds one among its sums (and the ones that it
-// shares k with) makes them again on v_mfma_f32_16x16x4_f32, operands straight from
-// memory.  8 x 1024 rows, K = 2048, 512 columns: 113 us, 440 with NaN everywhere;
+// infinity or a NaN.  A block that finds one among its sums makes its tile again on
+// v_mfma_f32_16x16x4_f32, operands straight from memory.  So does one with an operand
+// whose third term is not whole (a value below 2^-110), which one more instruction per
+// pair of values finds out (1 % of a launch).  8 x 1024 rows, K = 2048, 512 columns: 113 us, 440 with NaN everywhere;
 // weight gradients of these sizes 129 and 313.  (A chain of multiply-adds per element
 // took 15400 and 16600.)
 //
@@ -95,25 +95,30 @@ __device__ __forceinline__ void for_each_index(F f) {
   for_each_index(f, std::make_integer_sequence<int, COUNT>());
 }
 
-// The three terms of two values, a's in the low halves.  (The remainders by
+// The three terms of two values, a's in the low halves.  `lost` collects the third
+// terms' bits: they are whole if its low half stays 0.  (The remainders by
 // v_dot2c_f32_bf16 would be one instruction each instead of two, but it waits for
 // the matrix pipe: 8 of them and 2 MFMAs take as long as both by themselves.)
-__device__ __forceinline__ void split_pair(float a, float b,
-                                           uint32_t (&t)[3]) {
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&t)[3],
+                                           uint32_t& lost) {
 #pragma unroll
   for (int n = 0; n < 3; ++n) {
     t[n] = f32x2_to_bf16x2(a, b);
-    if (n == 2) break;
+    if (n == 2) {
+      // (in C++ the compiler collects the values of many pairs before it ors them)
+      asm("v_or3_b32 %0, %0, %1, %2" : "+v"(lost) : "v"(a), "v"(b));
+      break;
+    }
     a = a - __uint_as_float(t[n] << 16);            // exact
     b = b - __uint_as_float(t[n] & 0xffff0000u);
   }
 }
 // the terms of 8 values as MFMA operands
-__device__ __forceinline__ void split_terms(const float (&f)[8],
-                                            uint4 (&t)[3]) {
+__device__ __forceinline__ void split_terms(const float (&f)[8], uint4 (&t)[3],
+                                            uint32_t& lost) {
   uint32_t w[4][3];
 #pragma unroll
-  for (int p = 0; p < 4; ++p) split_pair(f[2 * p], f[2 * p + 1], w[p]);
+  for (int p = 0; p < 4; ++p) split_pair(f[2 * p], f[2 * p + 1], w[p], lost);
 #pragma unroll
   for (int n = 0; n < 3; ++n)
     t[n] = make_uint4(w[0][n], w[1][n], w[2][n], w[3][n]);
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
   constexpr int KS = Cfg::KS;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   bf16_t* As = reinterpret_cast<bf16_t*>(smem_raw);   // [2][3][BM][LDR]
-  __shared__ int again;           // WK > 1: the sums are made again
+  __shared__ int again;           // the sums are made again
   if (threadIdx.x == 0) again = 0;
   // an XCD works on a contiguous range of tiles, which share weight panels
   const int nblk = gridDim.x;
@@ -216,13 +221,14 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
       for (int j = 0; j < TN; ++j) load8(bc, b_off[s][j], N, b_raw[SLOT % RAW][s][j]);
   };
   uint4 b_terms[2][KS][TN][3];
+  uint32_t lost = 0;
   // the terms of a loaded tile: A's into stage `slot`, B's into registers
   auto make_terms = [&](auto slot_c) {
     constexpr int SLOT = decltype(slot_c)::value;
 #pragma unroll
     for (int i = 0; i < Cfg::A_CHUNKS; ++i) {
       uint4 t[3];
-      split_terms(a_raw[SLOT % RAW][i], t);
+      split_terms(a_raw[SLOT % RAW][i], t, lost);
 #pragma unroll
       for (int n = 0; n < 3; ++n)
         *reinterpret_cast<uint4*>(As + SLOT * Cfg::STAGE + n * Cfg::PLANE +
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
     for (int s = 0; s < KS; ++s)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        split_terms(b_raw[SLOT % RAW][s][j], b_terms[SLOT][s][j]);
+        split_terms(b_raw[SLOT % RAW][s][j], b_terms[SLOT][s][j], lost);
   };
 
   f32x4_t acc[TM][TN];
@@ -274,7 +280,7 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
       constexpr int s = gb / TN, j = gb % TN;
       float(&raw)[8] = of_a ? a_raw[OTHER % RAW][ga] : b_raw[OTHER % RAW][s][j];
       uint32_t t[3];
-      split_pair(raw[2 * p], raw[2 * p + 1], t);
+      split_pair(raw[2 * p], raw[2 * p + 1], t, lost);
 #pragma unroll
       for (int n = 0; n < 3; ++n) w[n][p] = t[n];
       if constexpr (p == 3) {
@@ -368,7 +374,8 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         test[r] = __builtin_fmaf(acc[i][j][r], 0.f, test[r]);
-  bool redo = __any(!(test[0] + test[1] + test[2] + test[3] == 0.f));
+  if (!(test[0] + test[1] + test[2] + test[3] == 0.f) || (lost & 0xffffu) != 0)
+    again = 1;
   auto sums_from_operands = [&]() {
     // two MFMAs of 4 k at a time, which the wavefronts that share k take in turn: the
     // q-th has k = 8 g + 2 (lane / 16) + q, with KMAJOR 8 g + 4 q + lane / 16
@@ -442,7 +449,8 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
     }
   };
   if constexpr (WK == 1) {
-    if (redo) sums_from_operands();
+    __syncthreads();
+    if (again) sums_from_operands();
   } else {
     // [wk - 1][wn][TM][TN][4][64], where the stages were
     float* parts = reinterpret_cast<float*>(smem_raw);
@@ -458,7 +466,6 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
           for (int r = 0; r < 4; ++r)
             dst[((i * TN + j) * 4 + r) * 64] = acc[i][j][r];
     };
-    if (redo) again = 1;
     store_part();
     __syncthreads();
     if (again) {

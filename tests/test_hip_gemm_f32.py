@@ -178,3 +178,33 @@ def test_products_of_nan_take_no_more_than_a_few_times_as_long(hip, kmajor):
   nan = _time_us(lambda: call(dy))
   print("finite %.1f us, NaN %.1f us" % (finite, nan))
   assert nan < 10 * finite
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+@pytest.mark.parametrize("exponent", [-60, -100, -109, -112, -118, -124, -135])
+@pytest.mark.parametrize("shape", [(1, 40, 64, 1028), (3, 164, 260, 324),
+                                   (8, 320, 512, 2048)])
+def test_tiny_values_keep_their_bits(hip, shape, exponent, kmajor):
+  """A product with a selection of the columns gives back every value exactly, also
+  where its third term would lie below the last bit of a bf16 denormal; as either
+  operand, and with one tiny value in a thousand."""
+  e, r, n, k = shape
+  gen = torch.Generator(device="cuda").manual_seed(r - exponent)
+  scale = 2.0 ** 60                    # (the results are no denormals)
+  for share in (1.0, 1e-3):
+    a = torch.randn((e, r, k), generator=gen, device="cuda")
+    tiny = torch.rand((e, r, k), generator=gen, device="cuda") < share
+    a = torch.where(tiny, (a.double() * 2.0 ** exponent).float(), a)
+    at = torch.randint(0, k, (e, n), generator=gen, device="cuda")
+    pick = torch.zeros((e, n, k), device="cuda").scatter_(2, at[..., None], scale)
+    want = (a.double() * scale).float().gather(
+        2, at[:, None].expand(e, r, n).contiguous())
+    for first, second, result in ((a, pick, want),
+                                  (pick, a, want.transpose(1, 2).contiguous())):
+      if kmajor:
+        first, second = [t.transpose(1, 2).contiguous() for t in (first, second)]
+        _, got = hip.expert_linear_backward(
+            first, second, torch.empty_like(result), want_da=False)
+      else:
+        got = hip.expert_linear(first, second, "linear")
+      assert torch.equal(got, result)
