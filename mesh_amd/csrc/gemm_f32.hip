@@ -41,9 +41,9 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 // infinity or a NaN.  A block that finds one among its sums makes its tile again on
 // v_mfma_f32_16x16x4_f32, operands straight from memory.  So does one with an operand
 // whose third term is not whole (a value below 2^-110), which one more instruction per
-// pair of values finds out (1 % of a launch).  8 x 1024 rows, K = 2048, 512 columns: 113 us, 440 with NaN everywhere;
-// weight gradients of these sizes 129 and 313.  (A chain of multiply-adds per element
-// took 15400 and 16600.)
+// pair of values finds out (1 % of a launch).  8 x 1024 rows, K = 2048, 512 columns:
+// 113 us, 440 with NaN everywhere; weight gradients of these sizes 129 and 313.  (A
+// chain of multiply-adds per element took 15400 and 16600.)
 //
 // TM x TN MFMA tiles per wavefront; WN wavefronts along N times WK wavefronts
 // that share out the k of every K tile and add up their sums in the end.  All
@@ -131,6 +131,84 @@ __device__ __forceinline__ float finish_f32(float v, bool relu, bool masked,
   if (relu) v = fmaxf(v, 0.f);
   if (masked) v = m > 0.f ? v * mask_scale : 0.f;
   return v;
+}
+
+// The sums of TM x TN MFMA tiles from (row0, col0) on, straight from the operands of an
+// expert, on float32 MFMAs; the wavefronts wk of WK share k.  Any sizes.
+template <int TM, int TN, int WK, bool KMAJOR>
+__device__ __forceinline__ void sums_from_operands(
+    const float* __restrict__ Ae, const float* __restrict__ Be, int R, int N, int K,
+    int row0, int col0, int wk, f32x4_t (&acc)[TM][TN]) {
+  const int lane = threadIdx.x & 63;
+  // two MFMAs of 4 k at a time, which the wavefronts that share k take in turn: the
+  // q-th has k = 8 g + 2 (lane / 16) + q, with KMAJOR 8 g + 4 q + lane / 16
+  constexpr int NQ = 2;
+  const int groups = (K + 7) / 8;
+  int64_t a_at[TM], b_at[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+    a_at[i] = (int64_t)min(row0 + i * 16 + (lane & 15), R - 1) * (KMAJOR ? 1 : K);
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+    b_at[j] = (int64_t)min(col0 + j * 16 + (lane & 15), N - 1) * (KMAJOR ? 1 : K);
+  float fa[TM][NQ], fb[TN][NQ];
+  // (past the end of k: zeros in both operands)
+  auto load = [&](int g) {
+    if constexpr (KMAJOR) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const int k = 8 * g + 4 * q + (lane >> 4);
+        const int64_t kk = min(k, K - 1);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const float v = Ae[kk * R + a_at[i]];
+          fa[i][q] = k < K ? v : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const float v = Be[kk * N + b_at[j]];
+          fb[j][q] = k < K ? v : 0.f;
+        }
+      }
+    } else {
+      const int k = 8 * g + 2 * (lane >> 4), kk = min(k, K - 2);
+      auto load2 = [&](const float* p, float (&f)[NQ]) {
+        const float2 v = *reinterpret_cast<const float2*>(p);
+        f[0] = k < K ? v.x : 0.f;
+        f[1] = k < K ? v.y : 0.f;
+      };
+#pragma unroll
+      for (int i = 0; i < TM; ++i) load2(Ae + a_at[i] + kk, fa[i]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) load2(Be + b_at[j] + kk, fb[j]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+  load(wk);
+  for (int g = wk; g < groups; g += WK) {
+    float ca[TM][NQ], cb[TN][NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) ca[i][q] = fa[i][q];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) cb[j][q] = fb[j][q];
+    }
+    load(g + WK);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[j][q], ca[i][q],
+                                                           acc[i][j], 0, 0, 0);
+  }
 }
 
 template <int TM, int TN, int WN, int WK, int RAW, bool KMAJOR>
@@ -376,81 +454,13 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
         test[r] = __builtin_fmaf(acc[i][j][r], 0.f, test[r]);
   if (!(test[0] + test[1] + test[2] + test[3] == 0.f) || (lost & 0xffffu) != 0)
     again = 1;
-  auto sums_from_operands = [&]() {
-    // two MFMAs of 4 k at a time, which the wavefronts that share k take in turn: the
-    // q-th has k = 8 g + 2 (lane / 16) + q, with KMAJOR 8 g + 4 q + lane / 16
-    constexpr int NQ = 2;
-    const int groups = (K + 7) / 8;
-    int64_t a_at[TM], b_at[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-      a_at[i] = (int64_t)min(row0 + i * 16 + (lane & 15), R - 1) * (KMAJOR ? 1 : K);
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      b_at[j] = (int64_t)min(col0 + (wn * TN + j) * 16 + (lane & 15), N - 1) *
-                (KMAJOR ? 1 : K);
-    float fa[TM][NQ], fb[TN][NQ];
-    // (past the end of k: zeros in both operands)
-    auto load = [&](int g) {
-      if constexpr (KMAJOR) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          const int k = 8 * g + 4 * q + (lane >> 4);
-          const int64_t kk = min(k, K - 1);
-#pragma unroll
-          for (int i = 0; i < TM; ++i) {
-            const float v = Ae[kk * R + a_at[i]];
-            fa[i][q] = k < K ? v : 0.f;
-          }
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const float v = Be[kk * N + b_at[j]];
-            fb[j][q] = k < K ? v : 0.f;
-          }
-        }
-      } else {
-        const int k = 8 * g + 2 * (lane >> 4), kk = min(k, K - 2);
-        auto load2 = [&](const float* p, float (&f)[NQ]) {
-          const float2 v = *reinterpret_cast<const float2*>(p);
-          f[0] = k < K ? v.x : 0.f;
-          f[1] = k < K ? v.y : 0.f;
-        };
-#pragma unroll
-        for (int i = 0; i < TM; ++i) load2(Ae + a_at[i] + kk, fa[i]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) load2(Be + b_at[j] + kk, fb[j]);
-      }
-    };
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
-    load(wk);
-    for (int g = wk; g < groups; g += WK) {
-      float ca[TM][NQ], cb[TN][NQ];
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) ca[i][q] = fa[i][q];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) cb[j][q] = fb[j][q];
-      }
-      load(g + WK);
-#pragma unroll
-      for (int q = 0; q < NQ; ++q)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[j][q], ca[i][q],
-                                                             acc[i][j], 0, 0, 0);
-    }
+  auto sums_again = [&]() {
+    sums_from_operands<TM, TN, WK, KMAJOR>(Ae, Be, R, N, K, row0,
+                                           col0 + wn * TN * 16, wk, acc);
   };
   if constexpr (WK == 1) {
     __syncthreads();
-    if (again) sums_from_operands();
+    if (again) sums_again();
   } else {
     // [wk - 1][wn][TM][TN][4][64], where the stages were
     float* parts = reinterpret_cast<float*>(smem_raw);
@@ -469,7 +479,7 @@ __global__ __launch_bounds__(64 * WN * WK) void grouped_gemm_f32_split_kernel(
     store_part();
     __syncthreads();
     if (again) {
-      sums_from_operands();
+      sums_again();
       store_part();
       __syncthreads();
     }
@@ -563,9 +573,38 @@ static const SplitTile split_tiles[] = {
     split_tile<4, 2, 4, 1, 1>(1.85, 2.07, 0.26, 0.68),   // 64 x 128, K tiles of 32
     split_tile<1, 2, 4, 1, 2>(2.90, 0.50, 0.13, 0.48)};  // 16 x 128
 
+// The offsets of a tile's loads are 32 bits: of its rows' k, or (kmajor) of its k's
+// rows, the last of which lies 20 below the K tile's end.
+static bool split_tile_fits(const SplitTile& t, int R, int N, int K, bool kmajor) {
+  const int64_t most = 1LL << 30;
+  return kmajor ? (int64_t)(t.k - 20) * (R > N ? R : N) + 256 <= most
+                : (int64_t)(t.rows > t.cols ? t.rows : t.cols) * K <= most;
+}
+
+// Weight gradients of rows too long for that (from 89 million elements on): a
+// wavefront per 32 x 32 outputs, bound by memory.
+__global__ __launch_bounds__(64) void f32_long_rows_kernel(
+    const float* __restrict__ A, const float* __restrict__ B,
+    float* __restrict__ Cout, int R, int N, int K, int tiles_m) {
+  const int tm = blockIdx.x % tiles_m, tn = blockIdx.x / tiles_m, e = blockIdx.y;
+  f32x4_t acc[2][2];
+  sums_from_operands<2, 2, 1, true>(A + (int64_t)e * R * K, B + (int64_t)e * N * K,
+                                    R, N, K, tm * 32, tn * 32, 0, acc);
+  const int lane = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = tm * 32 + i * 16 + (lane & 15);
+      const int col = tn * 32 + j * 16 + (lane >> 4) * 4;
+      if (row < R && col < N)
+        *reinterpret_cast<f32x4_t*>(Cout + ((int64_t)e * R + row) * N + col) =
+            acc[i][j];
+    }
+}
+
 bool f32_gemm_applies(int R, int N, int K) {
-  // (offsets inside a tile are 32 bits)
-  const int most = 1 << 22;
+  const int most = 0x7fffffff - 1024;    // (room for the indexes of a last tile)
   return R >= 32 && N >= 32 && K >= 32 && R <= most && N <= most && K <= most;
 }
 
@@ -577,7 +616,7 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
   const SplitTile* best = nullptr;
   double best_cost = 0;
   for (const SplitTile& t : split_tiles) {
-    if (t.k > K) continue;
+    if (t.k > K || !split_tile_fits(t, R, N, K, kmajor)) continue;
     const int64_t blocks = (int64_t)E * ((R + t.rows - 1) / t.rows) *
                            ((N + t.cols - 1) / t.cols);
     const double n = (double)((blocks + cus - 1) / cus);
@@ -588,7 +627,20 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
       best_cost = cost;
     }
   }
-  return best->launch(A, B, C, E, R, N, K, kmajor, relu, mask_src, mask_scale, st);
+  if (best != nullptr)
+    return best->launch(A, B, C, E, R, N, K, kmajor, relu, mask_src, mask_scale, st);
+  if (!kmajor)
+    return f32_gemm_stable(A, B, C, E, R, N, K, relu, mask_src, mask_scale, st);
+  const int64_t tiles_m = ((int64_t)R + 31) / 32, tiles_n = ((int64_t)N + 31) / 32;
+  MOE_REQUIRE(!relu && mask_src == nullptr, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: no activation on sums of rows");
+  MOE_REQUIRE(tiles_m * tiles_n <= 0x7fffffffLL && E <= 65535,
+              MESH_MOE_E_UNSUPPORTED, "expert_ffn: too many tiles (%lld)",
+              (long long)(tiles_m * tiles_n));
+  f32_long_rows_kernel<<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)E), 64, 0,
+                         st>>>(A, B, C, R, N, K, (int)tiles_m);
+  MOE_CHECK_LAUNCH("expert_ffn (float32, long rows)");
+  return 0;
 }
 
 // ---------------------------------------------------------------------------

@@ -208,3 +208,62 @@ def test_tiny_values_keep_their_bits(hip, shape, exponent, kmajor):
       else:
         got = hip.expert_linear(first, second, "linear")
       assert torch.equal(got, result)
+
+
+@pytest.mark.parametrize("kmajor", [False, True])
+def test_products_of_many_rows_stay_on_the_matrix_cores(hip, kmajor):
+  """More than 2^22 rows (of a weight gradient: to sum over) cost per row what fewer
+  do."""
+  n = 256
+  gen = torch.Generator(device="cuda").manual_seed(7)
+
+  def run(rows):
+    a = torch.randn((1, rows, n), generator=gen, device="cuda")
+    if not kmajor:
+      w = torch.randn((1, n, n), generator=gen, device="cuda")
+      call = lambda: hip.expert_linear(a, w, "linear")
+      _assert_close(call()[:, -100:], a[:, -100:], w.transpose(1, 2).contiguous())
+    else:
+      w = torch.empty(1, n, n, device="cuda")
+      dy = torch.randn((1, rows, n), generator=gen, device="cuda")
+      call = lambda: hip.expert_linear_backward(a, dy, w, want_da=False)[1]
+      _assert_close(call(), a.transpose(1, 2).contiguous(), dy)
+    return _time_us(call)
+  few, many = run(1 << 22), run((1 << 22) + 4)
+  torch.cuda.empty_cache()
+  assert many < 1.5 * few
+
+
+def test_long_reductions(hip):
+  """A reduction of more than 2^25 elements, which no tile in terms takes."""
+  r, n, k = 33, 36, (1 << 25) + 4
+  gen = torch.Generator(device="cuda").manual_seed(8)
+  a = torch.zeros((1, r, k), device="cuda")
+  at = torch.randint(0, k, (64,), generator=gen, device="cuda")
+  at[0] = k - 1
+  a[0, :, at] = _values(gen, r, 64)
+  w = torch.zeros((1, n, k), device="cuda")
+  w[0, :, at] = _values(gen, n, 64)
+  got = hip.expert_linear(a, w, "linear")
+  x, y = a[:, :, at.unique()], w[:, :, at.unique()].transpose(1, 2)
+  # (64 sums that are not of zeros)
+  bound = 84 * 2.0 ** -24 * (x.double().abs() @ y.double().abs().contiguous())
+  assert ((got.double() - x.double() @ y.double().contiguous()).abs() <= bound).all()
+
+
+def test_weight_gradients_of_long_rows(hip):
+  """Rows too long for 32-bit offsets inside a K tile of 32."""
+  m, n, rows = 89478488, 32, 33
+  gen = torch.Generator(device="cuda").manual_seed(9)
+  a = torch.randn((1, rows, m), generator=gen, device="cuda")
+  dy = _values(gen, 1, rows, n)
+  _, got = hip.expert_linear_backward(a, dy, torch.empty(1, m, n, device="cuda"),
+                                      want_da=False)
+  at = torch.randint(0, m, (1000,), generator=gen, device="cuda")
+  at[:40] = torch.arange(m - 40, m, device="cuda")
+  x = a[:, :, at].transpose(1, 2).contiguous()
+  bound = (rows + 20) * 2.0 ** -24 * (x.double().abs() @ dy.double().abs())
+  close = (got[:, at].double() - x.double() @ dy.double()).abs() <= bound
+  del a, got
+  torch.cuda.empty_cache()
+  assert close.all()
