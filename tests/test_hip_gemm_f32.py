@@ -22,8 +22,10 @@ def _values(gen, *sizes):
 def _assert_close(got, a, b):
   """got [E,R,N] against a [E,R,K] . b [E,K,N].  Per 32 k six matrix products of
   exact terms and one addition to the sum, and a handful of additions where
-  wavefronts share k out; what the three dropped products of terms leave out is
-  below 2^-26 of |a b|."""
+  wavefronts share k out; what the three dropped products of terms leave out is at
+  most 2^-24 of |a b|, and far less for most values.  (The shapes on float32 MFMAs
+  round once per k, up to 260 times, in either direction: their sums stay inside it
+  too.)"""
   a, b = a.double(), b.double()
   roundings = a.shape[2] // 32 + 20
   bound = roundings * 2.0 ** -24 * (a.abs() @ b.abs())
@@ -32,7 +34,8 @@ def _assert_close(got, a, b):
 
 # rows and columns around the tiles' edges (16 to 160 rows, 32 to 256 columns), k
 # below, at and above one K tile of 32 to 256 and with remainders, few and many
-# tiles: every tile of the table is picked by one of them
+# tiles.  (Seven of them are products short enough for float32 MFMAs; TILE_SHAPES has
+# one for every tile in terms.)
 SHAPES = [
     (1, 32, 32, 32), (1, 33, 36, 36), (1, 33, 68, 60), (3, 47, 132, 64),
     (1, 64, 512, 512), (2, 65, 260, 100), (1, 37, 64, 2052), (1, 100, 96, 1028),
@@ -41,7 +44,18 @@ SHAPES = [
     (9, 161, 4096, 64), (1, 2000, 640, 320), (1, 5000, 36, 96), (12, 427, 1024, 128)]
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+# [experts, rows, columns, k]: one for each tile of the table, in its order, as a
+# product and as a weight gradient summed over k + 1 rows (128 x 256, 160 x 256, 160 x
+# 128, 64 x 128, 80 x 64, 96 x 64, 32 x 32, 16 x 32, 32 x 64, 96 x 256, 64 x 256, 64 x
+# 128 with K tiles of 32, 16 x 128); rows, columns and k all leave a remainder
+TILE_SHAPES = [
+    (7, 1760, 280, 36), (16, 2276, 72, 48), (24, 1400, 72, 72), (24, 36, 660, 228),
+    (4, 2224, 68, 204), (16, 1288, 32, 220), (1, 2084, 40, 348), (1, 36, 40, 332),
+    (7, 36, 584, 328), (3, 2028, 548, 36), (4, 692, 1084, 40), (2, 712, 916, 92),
+    (8, 36, 1040, 328)]
+
+
+@pytest.mark.parametrize("shape", SHAPES + TILE_SHAPES)
 def test_products(hip, shape):
   e, r, n, k = shape
   gen = torch.Generator(device="cuda").manual_seed(sum(shape))
@@ -50,7 +64,7 @@ def test_products(hip, shape):
   _assert_close(got, a, w.transpose(1, 2).contiguous())
 
 
-@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("shape", SHAPES + TILE_SHAPES)
 def test_products_summed_over_rows(hip, shape):
   """Weight gradients: both operands with the reduction outermost, any length."""
   e, m, n, rows = shape
@@ -62,7 +76,11 @@ def test_products_summed_over_rows(hip, shape):
   _assert_close(got, a.transpose(1, 2).contiguous(), dy)
 
 
-@pytest.mark.parametrize("shape", [(2, 70, 260, 100), (8, 320, 512, 1028)])
+# (the first is short enough for float32 MFMAs)
+NON_FINITE_SHAPES = [(2, 70, 260, 100), (8, 320, 512, 1028), (2, 70, 260, 1028)]
+
+
+@pytest.mark.parametrize("shape", NON_FINITE_SHAPES)
 @pytest.mark.parametrize("activation", ["linear", "relu"])
 def test_infinities_nan_and_overflow(hip, shape, activation):
   """What an infinity, a NaN or an overflow does to a sum is what it does in
@@ -94,17 +112,6 @@ def test_infinities_nan_and_overflow(hip, shape, activation):
   sure[1, 0, 4] = True
   assert torch.equal(got[sure].nan_to_num(7.0, 1e300, -1e300),
                      want[sure].nan_to_num(7.0, 1e300, -1e300))
-
-
-# [experts, rows, columns, k]: one for each tile of the table, in its order, as a
-# product and as a weight gradient summed over k + 1 rows (128 x 256, 160 x 256, 160 x
-# 128, 64 x 128, 80 x 64, 96 x 64, 32 x 32, 16 x 32, 32 x 64, 96 x 256, 64 x 256, 64 x
-# 128 with K tiles of 32, 16 x 128); rows, columns and k all leave a remainder
-TILE_SHAPES = [
-    (7, 1760, 280, 36), (16, 2276, 72, 48), (24, 1400, 72, 72), (24, 36, 660, 228),
-    (4, 2224, 68, 204), (16, 1288, 32, 220), (1, 2084, 40, 348), (1, 36, 40, 332),
-    (7, 36, 584, 328), (3, 2028, 548, 36), (4, 692, 1084, 40), (2, 712, 916, 92),
-    (8, 36, 1040, 328)]
 
 
 @pytest.mark.parametrize("form", ["product", "masked", "weight gradient"])
