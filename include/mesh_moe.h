@@ -265,9 +265,11 @@ int mesh_moe_pack_weights(const void* src, void* dst, int E, int K, int N,
  *   expert_in [E,R,M] dtype (R = rows per expert = groups * capacity)
  *   wi_packed [E,H,M] dtype; wo_packed [E,N,H] dtype  (see pack_weights)
  *   h [E,R,H] dtype (caller-provided scratch); y [E,R,N] dtype
- * bf16 with M and H multiples of 8 and float32 with M, H and N multiples of 4 run on
- * the matrix cores (float32 as three bf16 terms per value, with less error than
- * float32 multiply-adds), other shapes on a plain FMA tile kernel.
+ * bf16 with M and H multiples of 8 and float32 with M, H and N multiples of 4 and at
+ * least 32, R at least 32, run on the matrix cores, other shapes on a plain FMA tile
+ * kernel.  float32 is multiplied as three bf16 terms per value, with less error than
+ * float32 multiply-adds; short reductions of little work, and tiles that such terms do
+ * not serve (values below 2^-110, infinities, NaN), on the float32 matrix instructions.
  */
 int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
                         const void* wo_packed, void* h, void* y, int E, int R,
@@ -276,9 +278,11 @@ int mesh_moe_expert_ffn(const void* expert_in, const void* wi_packed,
 
 /*
  * mesh_moe_expert_ffn for callers that keep h, i.e. for a step whose gradient is
- * wanted: the same, except that float32 ReLU experts sum h in an order that stays as
- * it is from one version of the library to the next (which hidden units the ReLU
- * lets through hangs on sums that may be 0 up to rounding, and so do gradients).
+ * wanted: the same, except that float32 ReLU experts sum h on the float32 matrix
+ * instructions, in an order that stays as it is from one version of the library to the
+ * next (which hidden units the ReLU lets through hangs on sums that may be 0 up to
+ * rounding, and so do gradients).  Hidden tensors made by mesh_moe_expert_linear have
+ * no such promise.
  */
 int mesh_moe_expert_ffn_kept(const void* expert_in, const void* wi_packed,
                              const void* wo_packed, void* h, void* y, int E,

@@ -94,8 +94,8 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(
 // `sum`; with `row_mask` [rows] the result is multiplied by the row's value: the
 // residual sum and the padding mask around a norm, with the roundings they have as
 // operations of their own; `norm_out` (or null) receives the norm without the mask.
-// Bound by memory: 16384 x 1024, sum and norm 25.5 us (5.3
-// TB/s; by themselves 17 + 13), 16000 x 768, sum, norm and mask 21 (12 + 11 + 14).
+// Bound by memory: 16384 x 1024, sum and norm 23 us (5.8 TB/s; by themselves 17 + 13),
+// 16000 x 768, sum, norm and mask 18 (12 + 11 + 14), 21 with norm_out.
 template <int ITERS>
 __global__ __launch_bounds__(256) void rms_norm_rows_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ scale,

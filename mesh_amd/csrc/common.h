@@ -24,10 +24,10 @@ int batched_gemm_nt(const void* A, const void* B, void* C, int E, int R, int N,
                     int K, int dtype, bool out_f32, hipStream_t st);
 
 // Batched float32 products (gemm_f32.hip): C[e] = A[e] . B[e]^T with A [E,R,K], B
-// [E,N,K], K % 4 == 0, or (kmajor) A[e]^T . B[e] with A [E,K,R], B [E,K,N]; N % 4
-// == 0, operands on 16 bytes.  mask_src (null: none; shape of C): elements whose
-// mask_src element is not positive become 0, the others are multiplied by
-// mask_scale.
+// [E,N,K], K % 4 == 0, or (kmajor, neither mask nor relu) A[e]^T . B[e] with A [E,K,R],
+// B [E,K,N], R % 4 == 0; N % 4 == 0, operands on 16 bytes.  mask_src (null: none; shape
+// of C): elements whose mask_src element is not positive become 0, the others are
+// multiplied by mask_scale.
 bool f32_gemm_applies(int R, int N, int K);
 int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int K,
              bool kmajor, bool relu, const float* mask_src, float mask_scale,

@@ -17,8 +17,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 // rounded to bf16, x2 the remainder rounded, and what is left then has at most
 // 8 significant bits, which bf16 holds exactly down to 2^-133, the last bit of its
 // denormals.  A product a b is then the sum of nine exact products, of which
-// a2 b3, a3 b2 and a3 b3, together below 2^-26 |a b|, are left out; the other six
-// run on v_mfma_f32_16x16x32_bf16, which adds exact products into float32: 96 cycles
+// a2 b3, a3 b2 and a3 b3, together at most 2^-24 |a b| (2^-28 on average), are left
+// out; the other six run on v_mfma_f32_16x16x32_bf16, which adds exact products into float32: 96 cycles
 // of the matrix pipe for 16 x 16 outputs and k = 32 instead of 256 of
 // v_mfma_f32_32x32x2_f32.  The six are summed by themselves, small ones first, and
 // added to the accumulator once per 32 k, which rounds a sixteenth as often as
@@ -47,10 +47,10 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 //
 // TM x TN MFMA tiles per wavefront; WN wavefronts along N times WK wavefronts
 // that share out the k of every K tile and add up their sums in the end.  All
-// wavefronts of a block work on the same 32 TM rows of A: their terms are made
+// wavefronts of a block work on the same 16 TM rows of A: their terms are made
 // once, on the way from registers into LDS ([3][rows][BK] bf16, rows padded by 16
 // bytes so that fragment reads and writes spread over all banks).  A
-// wavefront's 32 TN columns of B belong to it and its WK partners alone: its
+// wavefront's 16 TN columns of B belong to it and its WK partners alone: its
 // lanes load them straight from memory in operand layout and make the terms in
 // registers.  Both operands of K tile t + 2 are on their way in registers, and
 // the terms of tile t + 1 are made beside the MFMAs of tile t.
@@ -647,14 +647,17 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
 // Sums that do not change: v_mfma_f32_32x32x2_f32, true float32 operands, the
 // order of k and the tiles these products have always had.
 //
-// For the hidden tensor that a training step keeps.  Its ReLU lets a unit through
-// or not by the sign of a sum, about one in ten million of these sums is 0 up to
-// rounding, and a unit that switches moves its column of the weight gradient by up
-// to 0.6 of the gradient's root mean square.  With other rounding a few units of a
-// step would switch, so that steps of two versions could not be compared; the more
-// exact kernel above is as good an answer, and not the same one.  (All other
-// products of a step are continuous in their operands and go there, short reductions
-// of little work excepted, which are faster here.)
+// For the hidden tensor of ReLU experts in a training step (mesh_moe_expert_ffn_kept).
+// Its ReLU lets a unit through or not by the sign of a sum, about one in ten million of
+// these sums is 0 up to rounding, and a unit that switches moves its column of the
+// weight gradient by up to 0.6 of the gradient's root mean square.  With other rounding
+// a few units of a step would switch, so that steps of two versions could not be
+// compared; the more exact kernel above is as good an answer, and not the same one.
+// The price: 60 us instead of 41 (8 experts x 320 rows, 512 -> 2048), and that a step
+// without gradients rounds h otherwise.  Hidden tensors that are made projection by
+// projection (dense layers, experts with dropout or several factors) have the sums of
+// the kernel above.
+// Also for short reductions of little work, which are faster here.
 //
 // Four wavefronts; K step 32.  The weight tile is the MFMA's first operand, so a
 // lane ends up with 4 consecutive output columns per register group.  One MFMA
