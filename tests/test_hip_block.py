@@ -2015,3 +2015,30 @@ def test_padding_mask_has_a_gradient_where_it_is_asked_for():
   # a bf16 rounding of a float32 sum of 64 products
   assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -18 *
           (xv.double() * dyv.double()).abs().sum(-1)).all()
+
+
+def test_gradient_of_the_norm_in_front_of_a_mask():
+  """Asked for, the masked gradient stays a tensor of the graph; the norm's input and
+  scale have the same gradients either way."""
+  gen = torch.Generator(device="cuda").manual_seed(36)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  dims = [mtf.Dimension("batch", 2), mtf.Dimension("length", 20),
+          mtf.Dimension("d_model", 64)]
+  x, dy = [mtf.import_tf_tensor(mesh, _bf16_at(gen, False, 2, 20, 64),
+                                mtf.Shape(dims)) for _ in range(2)]
+  keep = (torch.rand((2, 20), generator=gen, device="cuda") < 0.7).bfloat16()
+  mask = mtf.import_tf_tensor(mesh, keep, mtf.Shape(dims[:2]))
+  scale = mtf.get_variable(mesh, "scale", mtf.Shape(dims[2:]), dtype=torch.bfloat16)
+  norm = transformer.RmsNormOperation(x, scale, 1e-6).outputs[0]
+  y = transformer.MaskPaddingOperation(norm, mask).outputs[0]
+  without = mtf.gradients([y], [x, scale], grad_ys=[dy])
+  dnorm, *others = mtf.gradients([y], [norm, x, scale], grad_ys=[dy])
+  low = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()}, initial_values={
+      "scale": _bf16_at(gen, False, 64)})
+  for _ in range(2):
+    assert torch.equal(low.export_to_tf_tensor(dnorm),
+                       low.export_to_tf_tensor(dy) * keep[..., None])
+    for a, b in zip(without, others):
+      assert torch.equal(low.export_to_tf_tensor(a), low.export_to_tf_tensor(b))
+    low.run()
