@@ -842,7 +842,10 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         const int krow = (wave + Cfg::WAVES * j) * 2 + (lane >> 5);
         const int p = lane & 31;
         const int chunk = ((((p >> 2) ^ (krow & 3)) << 2) | (p & 3)) * 8;
-        a_off[j] = krow * R + min(row0 + chunk, R - 8);
+        // (TAILS: what lies past the tile's rows is not multiplied; its lanes
+        // fetch the tile's last piece again)
+        const int row_chunk = TAILS ? min(chunk, tile_rows - 8) : chunk;
+        a_off[j] = krow * R + min(row0 + row_chunk, R - 8);
         b_off[j] = krow * N + min(col0 + chunk, N - 8);
         continue;
       }
@@ -909,19 +912,27 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
 
   const int fr = lane & 31, fc = lane >> 5;
   int a_frag[BK / 16], b_frag[BK / 16];
-  if constexpr (KMAJOR) {
-    // byte offset of this lane's 8 bytes for 32-column block n of its
-    // wavefront's sub-tile, at step 0 / first half: a_frag[n], b_frag[n]
-    static_assert(Cfg::TM <= BK / 16 && Cfg::TN <= BK / 16, "offset arrays");
+  // KMAJOR: byte offset of this lane's 8 bytes for 32-column block n of its
+  // wavefront's sub-tile, at step 0 / first half: a_frag[n], b_frag[n].  The rows
+  // of the tile lie in LDS as they do in memory: the lower half's pieces (TAILS)
+  // follow the upper half's.
+  auto kmajor_inner = [&]() {
     const int t = lane & 15, g = lane >> 4;
-    const int inner = ((g & 1) * 16 + 4 * (t & 3)) * 2 +
-                      ((g >> 1) * 8 + (t >> 2)) * 512;
+    return ((g & 1) * 16 + 4 * (t & 3)) * 2 + ((g >> 1) * 8 + (t >> 2)) * 512;
+  };
+  auto set_a_frag = [&]() {
+    const int first = wm == 0 ? 0 : pieces0;
 #pragma unroll
     for (int n = 0; n < Cfg::TM; ++n)
-      a_frag[n] = (((wm * Cfg::TM + n) ^ (t >> 2)) * 64) + inner;
+      a_frag[n] = (((first + n) ^ ((lane & 15) >> 2)) * 64) + kmajor_inner();
+  };
+  if constexpr (KMAJOR) {
+    static_assert(Cfg::TM <= BK / 16 && Cfg::TN <= BK / 16, "offset arrays");
+    if constexpr (!TAILS) set_a_frag();
 #pragma unroll
     for (int n = 0; n < Cfg::TN; ++n)
-      b_frag[n] = (((wn * Cfg::TN + n) ^ (t >> 2)) * 64) + inner;
+      b_frag[n] =
+          (((wn * Cfg::TN + n) ^ ((lane & 15) >> 2)) * 64) + kmajor_inner();
   } else {
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
@@ -1103,6 +1114,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    if constexpr (KMAJOR && TAILS) set_a_frag();
     auto k_loop = [&](auto na_tag) {
       constexpr int NA = decltype(na_tag)::value;
 #pragma unroll
@@ -1865,6 +1877,52 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
   return (unsigned)(((tiles < cus ? tiles : cus) + 7) / 8 * 8);
 }
 
+// Rows per row tile (a multiple of 32, at most 256) for R rows per expert.
+// The persistent blocks take whole rounds of tiles, so what counts is rounds
+// times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
+// 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
+// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside
+// the K loop.  Rows are spread evenly over the row tiles: 640 rows per expert are
+// three tiles of 224 or four of 160, not 256 + 256 + 128.  Measured, tiles of
+// 256 and a shorter last one -> the rule's choice (both sides bit-identical):
+//   32 x 640 rows, 4096 x 1024 (384 tiles -> 512 of 160 rows)   203 -> 166 us
+//   16 x 705 rows, 768 x 3072 / 3072 x 768 (192 rows)       73 / 67 -> 60 / 55
+//   8 x 900 rows, 1536 x 4608 (192 rows)                        117 -> 100
+//   64 x 320 rows, 1024 x 4096 (160 rows; 128-row kernel before) 268 -> 207
+//   5000 rows, 1280 x 1280 (128 rows, 200 tiles instead of 100)  31 -> 25
+//   128 x 400 rows, 2048 x 8192 (224 rows)                     1729 -> 1680
+// K-major operands (weight gradients; R is then a width, K the rows summed over):
+// 0.48 + 0.12 per piece us per K tile, 3.3 + 0.75 per piece outside the K loop, whose
+// share is larger there (reductions of few K tiles; from 16 x 704 and 1280 rows):
+//   16 x 704 rows, 768 x 3072 / 3072 x 768 (192 rows)   76 / 75 -> 62.5 / 65
+//   16 x 1280 rows, 768 x 3072 (192 rows)                   115 -> 95
+//   24 x 512 rows, 512 x 1536 (192 rows)                    36.7 -> 31.9
+//   12 x 1000 rows, 1280 x 2560 (224 rows)                  94.6 -> 85
+// and the rule stays with 256 where that is the fastest (64 x 512 rows, 1024 x 4096
+// 316, 224 rows 328; 8 x 640 rows, 1024 x 4096 48, 192 rows 55).
+static int ring_tile_rows(int E, int R, int N, int K, int cus,
+                          bool kmajor = false) {
+  const int tiles_n = (N + RingCfg::BN - 1) / RingCfg::BN;
+  const int nk = (K + RingCfg::BK - 1) / RingCfg::BK;
+  int best_rows = RingCfg::BM;
+  double best = 0;
+  for (int rows = RingCfg::BM; rows >= 32; rows -= 32) {
+    const int tiles_m = (R + rows - 1) / rows;
+    const int even = ((R + tiles_m - 1) / tiles_m + 31) / 32 * 32;
+    const int64_t tiles = (int64_t)E * ((R + even - 1) / even) * tiles_n;
+    const int pieces = even / 32;
+    const double per_k_tile = kmajor ? 0.48 + 0.12 * pieces : 0.45 + 0.14 * pieces;
+    const double outside = kmajor ? 3.3 + 0.75 * pieces : 6.5;
+    const double cost = (double)((tiles + cus - 1) / cus) *
+                        (nk * (per_k_tile < 0.6 ? 0.6 : per_k_tile) + outside);
+    if (rows == RingCfg::BM || cost < 0.98 * best) {
+      best = cost;
+      best_rows = even;
+    }
+  }
+  return best_rows;
+}
+
 // scratch: kmajor_split_plan(...).bytes for the parts (null: nothing is split;
 // with k_extent nothing is)
 static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
@@ -1872,17 +1930,19 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
                               const int32_t* k_extent = nullptr,
                               void* scratch = nullptr, int64_t a_stride = -1) {
   using Cfg = RingCfg;
-  const int tiles_m = (R + Cfg::BM - 1) / Cfg::BM;
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  const SplitPlan plan =
+      scratch == nullptr || k_extent != nullptr ? SplitPlan()
+                                                : kmajor_split_plan(E, R, N, K);
+  const int tile_rows =
+      plan.split > 1 ? Cfg::BM : ring_tile_rows(E, R, N, K, cus, true);
+  const int tiles_m = (R + tile_rows - 1) / tile_rows;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n * E;
   MOE_REQUIRE(tiles <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
               "expert_ffn_backward: too many tiles (%lld)", (long long)tiles);
-  const int cus = compute_units();
-  if (cus == 0) return MESH_MOE_E_HIP;
   const unsigned blocks = ring_blocks(tiles, cus);
-  const SplitPlan plan =
-      scratch == nullptr || k_extent != nullptr ? SplitPlan()
-                                                : kmajor_split_plan(E, R, N, K);
   if (plan.split > 1) {
     const int tail = (int)tiles - plan.whole_tiles;
     const int units = plan.whole_tiles + tail * plan.split;
@@ -1901,47 +1961,18 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     MOE_CHECK_LAUNCH("expert_ffn_backward (sum of the parts)");
     return 0;
   }
-  auto k = grouped_gemm_bf16_ring_kernel<false, false, true>;
-  MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
-  k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
-      A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-      nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, Cfg::BM, a_stride);
-  MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
-  return 0;
-}
-
-// Rows per row tile (a multiple of 32, at most 256) for R rows per expert.
-// The persistent blocks take whole rounds of tiles, so what counts is rounds
-// times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
-// 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
-// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside
-// the K loop.  Rows are spread evenly over the row tiles: 640 rows per expert are
-// three tiles of 224 or four of 160, not 256 + 256 + 128.  Measured, tiles of
-// 256 and a shorter last one -> the rule's choice (both sides bit-identical):
-//   32 x 640 rows, 4096 x 1024 (384 tiles -> 512 of 160 rows)   203 -> 166 us
-//   16 x 705 rows, 768 x 3072 / 3072 x 768 (192 rows)       73 / 67 -> 60 / 55
-//   8 x 900 rows, 1536 x 4608 (192 rows)                        117 -> 100
-//   64 x 320 rows, 1024 x 4096 (160 rows; 128-row kernel before) 268 -> 207
-//   5000 rows, 1280 x 1280 (128 rows, 200 tiles instead of 100)  31 -> 25
-//   128 x 400 rows, 2048 x 8192 (224 rows)                     1729 -> 1680
-static int ring_tile_rows(int E, int R, int N, int K, int cus) {
-  const int tiles_n = (N + RingCfg::BN - 1) / RingCfg::BN;
-  const int nk = (K + RingCfg::BK - 1) / RingCfg::BK;
-  int best_rows = RingCfg::BM;
-  double best = 0;
-  for (int rows = RingCfg::BM; rows >= 32; rows -= 32) {
-    const int tiles_m = (R + rows - 1) / rows;
-    const int even = ((R + tiles_m - 1) / tiles_m + 31) / 32 * 32;
-    const int64_t tiles = (int64_t)E * ((R + even - 1) / even) * tiles_n;
-    const double per_k_tile = 0.45 + 0.14 * (even / 32);
-    const double cost = (double)((tiles + cus - 1) / cus) *
-                        (nk * (per_k_tile < 0.6 ? 0.6 : per_k_tile) + 6.5);
-    if (rows == RingCfg::BM || cost < 0.98 * best) {
-      best = cost;
-      best_rows = even;
-    }
-  }
-  return best_rows;
+  auto run = [&](auto k) -> int {
+    MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
+    k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
+        A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
+        nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, tile_rows, a_stride);
+    MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
+    return 0;
+  };
+  if (tile_rows != Cfg::BM)
+    return run(grouped_gemm_bf16_ring_kernel<false, false, true, false, false,
+                                             true>);
+  return run(grouped_gemm_bf16_ring_kernel<false, false, true>);
 }
 
 static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,

@@ -1700,6 +1700,30 @@ def test_weight_gradient_of_split_reductions(hip, shape):
 
 
 @pytest.mark.parametrize("shape", [
+    # the width is cut into tiles of 32 (the last one 8), 64 (8), 96 (40), 128, 160
+    # (104), 192, 224 and 256 rows
+    (2, 64, 200, 136), (6, 200, 520, 776), (10, 200, 520, 776), (6, 70, 1000, 776),
+    (90, 70, 264, 512), (16, 704, 768, 3072), (32, 160, 640, 1920),
+    (64, 130, 1024, 1024)], ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_row_tiles(hip, shape):
+  """Weight gradients whose output rows are spread over row tiles of 32 to 256.
+  The bound: one bf16 rounding, and for each of the two float32 sums of R
+  products R / 2 ulps of the sum of magnitudes."""
+  e, rows, k, n = shape
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(sum(shape))
+  a, dy, w = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16)
+              for s in ((e, rows, k), (e, rows, n), (e, k, n)))
+  dw = hip.expert_linear_backward(a, dy, w, want_da=False)[1]
+  for i in range(e):
+    at = a[i].float().t().contiguous()
+    want = at @ dy[i].float()
+    magnitude = at.abs() @ dy[i].float().abs()
+    bound = 2.0 ** -8 * want.abs() + rows * 2.0 ** -24 * magnitude
+    assert bool(((dw[i].float() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("shape", [
     (8, 320, 2048, 512), (8, 320, 512, 2048), (2, 33, 36, 100), (1, 32, 32, 32),
     (1, 2000, 260, 1028), (40, 65, 68, 132), (3, 161, 1000, 64), (5, 97, 64, 300)],
     ids=lambda s: "x".join(map(str, s)))
