@@ -31,7 +31,18 @@
 // keys of a step, so no data moves between lanes and V is never transposed in
 // memory.
 //
-// K and V tiles reach a two-stage LDS ring through global_load_lds_dwordx4; K
+// A tile's two halves of work are laid beside the other kind of its neighbours':
+// the exponentials of tile t between the MFMAs of tile t + 1's logits (a pair or two
+// after each), the maximum of t + 1 between the MFMAs of tile t's outputs.  (One
+// after the other, neither of the two wavefronts that a SIMD holds kept the matrix
+// pipe busy while the other one was at its softmax: busy 28 % of the time, vector
+// units 41 %.)  8 x 2048 positions, 8 heads of 128, causal 115 -> 99 us, without the
+// mask 166 -> 150; 2 x 4096, 16 heads of 64 102 -> 89; 16 packed rows of 1000, 12
+// heads of 64 58 -> 55.5.  What is left is the sum of both units' work (VALU 45 %,
+// MFMA 46 %) at 1.9 GHz of shader clock.
+//
+// K and V tiles reach a two-stage LDS ring through global_load_lds_dwordx4, K a tile
+// ahead of V; K
 // rows with XOR-swizzled 16-byte chunks, V rows with their 64-byte units
 // XOR-ed by the key index (bank conflicts of the transposing reads); the
 // queries of a wavefront stay in registers.  The transposing reads are inline
@@ -218,7 +229,7 @@ __device__ __forceinline__ void fa_visible_tiles(
 // it, which travels through LDS with the tile.
 template <int D, bool CAUSAL, bool STATS = false, bool SEQ = false,
           bool BIAS = false>
-__global__ __launch_bounds__(256, 2) void flash_attention_kernel(
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     const bf16_t* __restrict__ v, bf16_t* __restrict__ out, int L, int H,
     const bf16_t* __restrict__ dout, float* __restrict__ lse,
@@ -226,7 +237,8 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
     const float* __restrict__ tab) {
   using Cfg = FlashCfg<D>;
   extern __shared__ __attribute__((aligned(16))) unsigned char fa_smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   const int nq = (L + Cfg::BQ - 1) / Cfg::BQ;
   int tile_x, bh;
@@ -271,43 +283,46 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
       qf[s] = *reinterpret_cast<const fa_bf16x8_t*>(qr + s * 16);
   }
 
-  // direct-to-LDS loads of one K tile and one V tile: a lane's places in a tile
-  // (row and swizzled chunk) are offsets that never change, the tile's is a
-  // scalar; rows past the end repeat the last
+  // direct-to-LDS loads of a K tile and of a V tile: a lane's places in a tile (row
+  // and swizzled chunk) are byte offsets that never change, the tile's is a scalar;
+  // rows past the end repeat the last
   static_assert(Cfg::K_RPI == Cfg::V_RPI && Cfg::KCH == Cfg::VCH, "one row shape");
-  const uint32_t rs = (uint32_t)row_stride;
+  const uint32_t row_bytes = (uint32_t)row_stride * 2;
   uint32_t k_chunk[Cfg::K_INSTR], v_chunk[Cfg::K_INSTR], row_off[Cfg::K_INSTR];
 #pragma unroll
   for (int j = 0; j < Cfg::K_INSTR; ++j) {
     const int row = (wave * Cfg::K_INSTR + j) * Cfg::K_RPI + lane / Cfg::KCH;
     const int p = lane % Cfg::KCH;
-    k_chunk[j] = (uint32_t)(p ^ fa_kswz<Cfg::KCH>(row)) * 8;
+    k_chunk[j] = (uint32_t)(p ^ fa_kswz<Cfg::KCH>(row)) * 16;
     v_chunk[j] =
-        (uint32_t)((((p >> 2) ^ fa_vswz<Cfg::V_UNITS>(row)) << 2) | (p & 3)) * 8;
-    row_off[j] = (uint32_t)row * rs;
+        (uint32_t)((((p >> 2) ^ fa_vswz<Cfg::V_UNITS>(row)) << 2) | (p & 3)) * 16;
+    row_off[j] = (uint32_t)row * row_bytes;
   }
-  auto load_tile = [&](int kt, int buf) {
-    const int key0 = kt * Cfg::BK;
-    unsigned char* base = fa_smem + buf * Cfg::STAGE;
-    const bf16_t* kt0 = kb + (int64_t)key0 * row_stride;
-    const bf16_t* vt0 = vb + (int64_t)key0 * row_stride;
-    const uint32_t last_row = (uint32_t)(L - 1 - key0) * rs;
+  auto load_rows = [&](const bf16_t* src, int key0, const uint32_t* chunk,
+                       unsigned char* to) {
+    const char* first = (const char*)(src + (int64_t)key0 * row_stride);
+    const uint32_t last = key0 + Cfg::BK <= L
+                              ? 0xffffffffu : (uint32_t)(L - 1 - key0) * row_bytes;
 #pragma unroll
     for (int j = 0; j < Cfg::K_INSTR; ++j) {
-      const uint32_t row = min(row_off[j], last_row);
-      const int g = wave * Cfg::K_INSTR + j;
-      __builtin_amdgcn_global_load_lds((fa_glb_void_t*)(kt0 + (row + k_chunk[j])),
-                                       (fa_lds_void_t*)(base + g * 1024), 16, 0,
-                                       0);
+      const uint32_t row = min(row_off[j], last);
       __builtin_amdgcn_global_load_lds(
-          (fa_glb_void_t*)(vt0 + (row + v_chunk[j])),
-          (fa_lds_void_t*)(base + Cfg::K_BYTES + g * 1024), 16, 0, 0);
+          (fa_glb_void_t*)(first + (uint32_t)(row + chunk[j])),
+          (fa_lds_void_t*)(to + (wave * Cfg::K_INSTR + j) * 1024), 16, 0, 0);
     }
+  };
+  auto load_v = [&](int kt, int slot) {
+    load_rows(vb, kt * Cfg::BK, v_chunk,
+              fa_smem + 2 * Cfg::K_BYTES + slot * Cfg::V_BYTES);
+  };
+  auto load_k = [&](int kt, int slot) {
+    const int key0 = kt * Cfg::BK;
+    load_rows(kb, key0, k_chunk, fa_smem + slot * Cfg::K_BYTES);
     if constexpr (SEQ) {
       if (wave == 0)
         __builtin_amdgcn_global_load_lds(
             (fa_glb_void_t*)(seq_b + min(key0 + lane, L - 1)),
-            (fa_lds_void_t*)(fa_smem + Cfg::LDS_BYTES + buf * 256), 4, 0, 0);
+            (fa_lds_void_t*)(fa_smem + Cfg::LDS_BYTES + slot * 256), 4, 0, 0);
     }
     if constexpr (BIAS) {
       // entry i of the window: distance key0 - (q0 + BQ - 1) + i (+ L - 1)
@@ -316,7 +331,7 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
         const int d = key0 - (q0 + Cfg::BQ - 1) + (L - 1) + i;
         __builtin_amdgcn_global_load_lds(
             (fa_glb_void_t*)(tab_h + min(max(d, 0), 2 * L - 2)),
-            (fa_lds_void_t*)(fa_smem + Cfg::LDS_BYTES + 512 + buf * 768 +
+            (fa_lds_void_t*)(fa_smem + Cfg::LDS_BYTES + 512 + slot * 768 +
                              (wave - 1) * 256),
             4, 0, 0);
       }
@@ -333,176 +348,249 @@ __global__ __launch_bounds__(256, 2) void flash_attention_kernel(
   float m_run = NEG;      // running maximum of this lane's query
   float l_part = 0.f;     // sum over this half-wave's keys
 
-  load_tile(kt_begin, 0);
+  const int qw_first = q0 + wave * 32;
+  const int kt_count = n_ktiles - kt_begin;
+  load_k(kt_begin, 0);
+  load_v(kt_begin, 0);
+  if (kt_count > 1) load_k(kt_begin + 1, 1);
   __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
   __syncthreads();
 
-  const int qw_first = q0 + wave * 32;
-  const int kt_count = n_ktiles - kt_begin;
-  for (int it = 0; it < kt_count; ++it) {
-    const int kt = kt_begin + it, buf = it & 1;
-    if (kt + 1 < n_ktiles) load_tile(kt + 1, buf ^ 1);
+  // byte offsets of this lane's reads: K row l32 of a sub-tile, step s; V rows of
+  // step u, block dt (two transposing reads of 4 key rows x 16 d per 16 lanes; row
+  // krow + 16 u + 8 j has the same fa_vswz as krow)
+  uint32_t k_at[Cfg::DS], v_at[Cfg::DT];
+#pragma unroll
+  for (int s = 0; s < Cfg::DS; ++s)
+    k_at[s] = l32 * Cfg::K_ROW + (((2 * s + half) ^ fa_kswz<Cfg::KCH>(l32)) * 16);
+  {
+    const int t16 = lane & 15, g16 = lane >> 4;
+    const int krow = 4 * (g16 >> 1) + (t16 >> 2);        // + 16 u (+ 8)
+    const int dcol = (g16 & 1) * 16 + 4 * (t16 & 3);      // + 32 dt
+    const int sw = fa_vswz<Cfg::V_UNITS>(krow);
+#pragma unroll
+    for (int dt = 0; dt < Cfg::DT; ++dt) {
+      const int col = dt * 32 + dcol;                     // element index
+      v_at[dt] = (uint32_t)(size_t)(fa_lds_void_t*)fa_smem + 2 * Cfg::K_BYTES +
+                 krow * Cfg::V_ROW + (((col >> 5) ^ sw) << 6) + (col & 31) * 2;
+    }
+  }
+  constexpr int SM = 2 * Cfg::DS;                  // MFMAs of S^T of a tile
+  auto fence = [&]() { __builtin_amdgcn_sched_barrier(0); };
+
+  // MFMA j of a tile's logits, from the K tile in `slot`; the fragment of MFMA
+  // j + AHEAD is read in front of it
+  constexpr int AHEAD = D == 64 ? 2 : 3;
+  fa_bf16x8_t kf[AHEAD + 1];
+  auto read_k = [&](int slot, int j) {
+    kf[j % (AHEAD + 1)] = *reinterpret_cast<const fa_bf16x8_t*>(
+        fa_smem + k_at[j >> 1] + slot * Cfg::K_BYTES + (j & 1) * 32 * Cfg::K_ROW);
+  };
+  auto start_logits = [&](int slot, fa_f32x16_t (&acc_s)[2]) {
+    if constexpr (BIAS) {
+      // key kl + c of the tile against query 32 wave + l32 of the block
+      const float* bw = bias_s + slot * 192 + (Cfg::BQ - 1 - wave * 32 - l32);
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            acc_s[sub][4 * r4 + c] = bw[sub * 32 + 8 * r4 + 4 * half + c];
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) read_k(slot, j);
+  };
+  auto logits_mfma = [&](int slot, int j, fa_f32x16_t (&acc_s)[2]) {
+    if (j + AHEAD < SM) read_k(slot, j + AHEAD);
+    const fa_f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                              0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    acc_s[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        kf[j % (AHEAD + 1)], qf[j >> 1], !BIAS && j < 2 ? zero : acc_s[j & 1], 0, 0,
+        0);
+  };
+  // diagonal and last tiles, and those that hold other sequences: behind a branch
+  // that the tiles in between do not take
+  auto mask_logits = [&](int kt, int slot, fa_f32x16_t (&acc_s)[2]) {
     const int key0 = kt * Cfg::BK;
-    // (a wavefront whose queries all precede this tile still runs it: every
-    // weight comes out 0, which measured faster than skipping)
-    // mask: diagonal and last tiles only, behind a branch the tiles in between
-    // do not take
     bool need_mask =
         (CAUSAL && key0 + Cfg::BK - 1 > qw_first) || key0 + Cfg::BK > L;
-    const int32_t* sid_t = sid_s + buf * 64;
+    const int32_t* sid_t = sid_s + slot * 64;
     if constexpr (SEQ) {
       // (wave-uniform: any key of the tile or query of the wavefront with an
       // id other than the first query's)
       need_mask = need_mask || !own_uniform ||
                   __ballot(sid_t[lane] != own_first) != 0ull;
     }
-    {
-      const unsigned char* ks = fa_smem + buf * Cfg::STAGE;
-      // S^T: two sub-tiles of 32 keys
-      fa_f32x16_t acc_s[2];
+    if (need_mask) {
+      // (the empty asm keeps the compiler from turning the branch into 64
+      // selects that every tile would execute)
+      asm volatile("" ::: "memory");
 #pragma unroll
       for (int sub = 0; sub < 2; ++sub) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc_s[sub][r] = 0.f;
-        const int row = sub * 32 + l32;
-        const unsigned char* kr = ks + row * Cfg::K_ROW;
-        const int sw = fa_kswz<Cfg::KCH>(row);
-#pragma unroll
-        for (int s = 0; s < Cfg::DS; ++s) {
-          const fa_bf16x8_t kf = *reinterpret_cast<const fa_bf16x8_t*>(
-              kr + (((2 * s + half) ^ sw) * 16));
-          acc_s[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              kf, qf[s], acc_s[sub], 0, 0, 0);
-        }
-      }
-      if constexpr (BIAS) {
-        // key key0 + kl + c against query q0 + 32 wave + l32
-        const float* bw = bias_s + buf * 192 + (Cfg::BQ - 1 - wave * 32 - l32);
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-              acc_s[sub][4 * r4 + c] += bw[sub * 32 + 8 * r4 + 4 * half + c];
-      }
-      // mask and row maximum
-      if (need_mask) {
-        // (the empty asm keeps the compiler from turning the branch into 64
-        // selects that every tile would execute)
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-          for (int r4 = 0; r4 < 4; ++r4) {
-            const int kl = sub * 32 + 8 * r4 + 4 * half;     // key within tile
-            int kid[4] = {0, 0, 0, 0};
-            if constexpr (SEQ) {
-              const int4 i4 = *reinterpret_cast<const int4*>(sid_t + kl);
-              kid[0] = i4.x; kid[1] = i4.y; kid[2] = i4.z; kid[3] = i4.w;
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int key = key0 + kl + c;
-              const bool ok = key < L && (!CAUSAL || key <= my_q) &&
-                              (!SEQ || kid[c] == my_sid);
-              if (!ok) acc_s[sub][4 * r4 + c] = NEG;
-            }
+        for (int r4 = 0; r4 < 4; ++r4) {
+          const int kl = sub * 32 + 8 * r4 + 4 * half;     // key within tile
+          int kid[4] = {0, 0, 0, 0};
+          if constexpr (SEQ) {
+            const int4 i4 = *reinterpret_cast<const int4*>(sid_t + kl);
+            kid[0] = i4.x; kid[1] = i4.y; kid[2] = i4.z; kid[3] = i4.w;
           }
-        }
-      }
-      float mx = NEG;
 #pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc_s[sub][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = fa_exp2((m_run - m_new) * LOG2E);
-      // (a tile with no visible key before any visible key was met: the
-      // maximum is still the sentinel, and sentinel * log2e - sentinel * log2e
-      // would leave the product's rounding error, ~1e22, as the exponent)
-      const float mneg = m_new > 0.5f * NEG ? -m_new * LOG2E : -INFINITY;
-      m_run = m_new;
-      float psum = 0.f;
-      fa_bf16x8_t pf[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        uint32_t w[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int r = 8 * (u & 1) + 2 * c;
-          const float p0 = fa_exp2(fmaf(acc_s[u >> 1][r], LOG2E, mneg));
-          const float p1 = fa_exp2(fmaf(acc_s[u >> 1][r + 1], LOG2E, mneg));
-          psum += p0 + p1;
-          w[c] = f32x2_to_bf16x2(p0, p1);
-        }
-        fa_u32x4_t packed = {w[0], w[1], w[2], w[3]};
-        pf[u] = __builtin_bit_cast(fa_bf16x8_t, packed);
-      }
-      l_part = l_part * alpha + psum;
-      // the outputs are rescaled only when some query's maximum moved in this
-      // tile (after the first few tiles it rarely does): alpha is exactly 1
-      // otherwise and the 16 * D / 32 multiplications per lane drop out
-      if (__ballot(alpha != 1.0f) != 0ull) {
-#pragma unroll
-        for (int dt = 0; dt < Cfg::DT; ++dt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
-      }
-      // O^T += V^T . P: the V^T operand of step u, block dt is two
-      // transposing reads of 4 key rows x 16 d each (per 16 lanes)
-      {
-        const uint32_t lds0 = (uint32_t)(size_t)(fa_lds_void_t*)fa_smem;
-        const int t16 = lane & 15, g16 = lane >> 4;
-        const int krow = 4 * (g16 >> 1) + (t16 >> 2);        // + 16 u (+ 8)
-        const int dcol = (g16 & 1) * 16 + 4 * (t16 & 3);      // + 32 dt
-        // row krow + 16 u + 8 j has the same fa_vswz as krow (multiples of 4
-        // or 8 are added), so the unit swizzle is a per-lane constant
-        const int sw = fa_vswz<Cfg::V_UNITS>(krow);
-        uint32_t vaddr[Cfg::DT];
-#pragma unroll
-        for (int dt = 0; dt < Cfg::DT; ++dt) {
-          const int col = dt * 32 + dcol;                     // element index
-          vaddr[dt] = lds0 + buf * Cfg::STAGE + Cfg::K_BYTES +
-                      krow * Cfg::V_ROW + (((col >> 5) ^ sw) << 6) +
-                      (col & 31) * 2;
-        }
-        fa_i16x4_t vlo[2][4], vhi[2][4];
-        auto read_v = [&](int dt, int slot) {
-          const uint32_t a = vaddr[dt];
-          vlo[slot][0] = fa_lds_read_tr16<0 * Cfg::V_ROW>(a);
-          vhi[slot][0] = fa_lds_read_tr16<8 * Cfg::V_ROW>(a);
-          vlo[slot][1] = fa_lds_read_tr16<16 * Cfg::V_ROW>(a);
-          vhi[slot][1] = fa_lds_read_tr16<24 * Cfg::V_ROW>(a);
-          vlo[slot][2] = fa_lds_read_tr16<32 * Cfg::V_ROW>(a);
-          vhi[slot][2] = fa_lds_read_tr16<40 * Cfg::V_ROW>(a);
-          vlo[slot][3] = fa_lds_read_tr16<48 * Cfg::V_ROW>(a);
-          vhi[slot][3] = fa_lds_read_tr16<56 * Cfg::V_ROW>(a);
-        };
-        read_v(0, 0);
-#pragma unroll
-        for (int dt = 0; dt < Cfg::DT; ++dt) {
-          const int cur = dt & 1;
-          __builtin_amdgcn_sched_barrier(0);
-          __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0): block dt is here
-          __builtin_amdgcn_sched_barrier(0);
-          if (dt + 1 < Cfg::DT) read_v(dt + 1, cur ^ 1);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const fa_bf16x8_t vf = __builtin_bit_cast(
-                fa_bf16x8_t, __builtin_shufflevector(vlo[cur][u], vhi[cur][u], 0,
-                                                     1, 2, 3, 4, 5, 6, 7));
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                vf, pf[u], acc_o[dt], 0, 0, 0);
+          for (int c = 0; c < 4; ++c) {
+            const int key = key0 + kl + c;
+            const bool ok = key < L && (!CAUSAL || key <= my_q) &&
+                            (!SEQ || kid[c] == my_sid);
+            if (!ok) acc_s[sub][4 * r4 + c] = NEG;
           }
-          __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
-    // tile kt+1 has landed and everybody is done with tile kt
-    __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
-    __syncthreads();
+  };
+  // part i of 4 of the maximum of a tile's 32 logits
+  auto part_of_max = [&](int i, float mx, fa_f32x16_t (&acc_s)[2]) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      mx = fmaxf(mx, acc_s[i >> 1][8 * (i & 1) + r]);
+    return mx;
+  };
+  // The outputs are rescaled only when some query's maximum moved in this tile.
+  // (Weights relative to a maximum up to 2^8 too low would save nearly all of these
+  // multiplications, 99 -> 93 us at 8 x 2048, 8 heads of 128, causal, but a query's
+  // largest weight is then no longer 1, which bf16 holds exactly: 3 % more error.)
+  auto move_max = [&](float mx) {
+    const auto both = __builtin_amdgcn_permlane32_swap(
+        __float_as_uint(mx), __float_as_uint(mx), false, false);
+    mx = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+    const bool moves = mx > m_run;
+    if (__ballot(moves) != 0ull) {
+      const float m_new = moves ? mx : m_run;
+      const float alpha = fa_exp2((m_run - m_new) * LOG2E);
+      m_run = m_new;
+      l_part *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < Cfg::DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc_o[dt][r] *= alpha;
+    }
+  };
+
+  // Tile `it`: its weights, beside the MFMAs of the next tile's logits, then its
+  // share of the outputs, beside the next tile's maximum.
+  auto tile = [&](int it, auto slot_c, auto last_c, fa_f32x16_t (&acc_s)[2],
+                  fa_f32x16_t (&acc_n)[2]) {
+    constexpr int SLOT = decltype(slot_c)::value, OTHER = SLOT ^ 1;
+    constexpr bool LAST = decltype(last_c)::value;
+    const int kt = kt_begin + it;
+    if constexpr (!LAST) {
+      load_v(kt + 1, OTHER);
+      if (it + 2 < kt_count) load_k(kt + 2, SLOT);
+    }
+    // (no visible key so far: the maximum is still the sentinel, and sentinel *
+    // log2e - sentinel * log2e would leave the product's rounding error, ~1e22, as
+    // the exponent)
+    const float mneg = m_run > 0.5f * NEG ? -m_run * LOG2E : -INFINITY;
+    float psum = 0.f;
+    uint32_t w[16];
+    auto weights = [&](int i) {      // keys of registers 2 (i % 8) and + 1
+      const float p0 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7)], LOG2E, mneg));
+      const float p1 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7) + 1], LOG2E, mneg));
+      psum += p0 + p1;
+      w[i] = f32x2_to_bf16x2(p0, p1);
+      // (otherwise the compiler makes them where they are first used, behind the
+      // branch around the mask)
+      asm volatile("" : "+v"(w[i]), "+v"(psum));
+    };
+    if constexpr (!LAST) {
+      start_logits(OTHER, acc_n);
+      fence();
+#pragma unroll
+      for (int j = 0; j < SM; ++j) {
+        logits_mfma(OTHER, j, acc_n);
+#pragma unroll
+        for (int i = 16 * j / SM; i < 16 * (j + 1) / SM; ++i) weights(i);
+        fence();
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) weights(i);
+    }
+    l_part += psum;
+    fa_bf16x8_t pf[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      fa_u32x4_t packed = {w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]};
+      pf[u] = __builtin_bit_cast(fa_bf16x8_t, packed);
+    }
+    if constexpr (!LAST) mask_logits(kt + 1, OTHER, acc_n);
+    // O^T += V^T . P
+    fa_i16x4_t vlo[2][4], vhi[2][4];
+    auto read_v = [&](int dt, int to) {
+      constexpr int AT = SLOT * Cfg::V_BYTES;
+      const uint32_t a = v_at[dt];
+      vlo[to][0] = fa_lds_read_tr16<AT + 0 * Cfg::V_ROW>(a);
+      vhi[to][0] = fa_lds_read_tr16<AT + 8 * Cfg::V_ROW>(a);
+      vlo[to][1] = fa_lds_read_tr16<AT + 16 * Cfg::V_ROW>(a);
+      vhi[to][1] = fa_lds_read_tr16<AT + 24 * Cfg::V_ROW>(a);
+      vlo[to][2] = fa_lds_read_tr16<AT + 32 * Cfg::V_ROW>(a);
+      vhi[to][2] = fa_lds_read_tr16<AT + 40 * Cfg::V_ROW>(a);
+      vlo[to][3] = fa_lds_read_tr16<AT + 48 * Cfg::V_ROW>(a);
+      vhi[to][3] = fa_lds_read_tr16<AT + 56 * Cfg::V_ROW>(a);
+    };
+    float mx = NEG;
+    read_v(0, 0);
+#pragma unroll
+    for (int dt = 0; dt < Cfg::DT; ++dt) {
+      const int cur = dt & 1;
+      fence();
+      __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0): block dt is here
+      fence();
+      if (dt + 1 < Cfg::DT) read_v(dt + 1, cur ^ 1);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const fa_bf16x8_t vf = __builtin_bit_cast(
+            fa_bf16x8_t, __builtin_shufflevector(vlo[cur][u], vhi[cur][u], 0, 1, 2,
+                                                 3, 4, 5, 6, 7));
+        acc_o[dt] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[u], acc_o[dt], 0, 0, 0);
+        if constexpr (!LAST) {
+          if (u < 4 / Cfg::DT) mx = part_of_max(dt * (4 / Cfg::DT) + u, mx, acc_n);
+        }
+      }
+      fence();
+    }
+    if constexpr (!LAST) {
+      move_max(mx);
+      // the loads have landed and everybody is done with this tile
+      __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
+      __syncthreads();
+    }
+  };
+  fa_f32x16_t acc_a[2], acc_b[2];
+  start_logits(0, acc_a);
+#pragma unroll
+  for (int j = 0; j < SM; ++j) logits_mfma(0, j, acc_a);
+  mask_logits(kt_begin, 0, acc_a);
+  {
+    float mx = NEG;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = part_of_max(i, mx, acc_a);
+    move_max(mx);
+  }
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  // K tile 0's slot is loaded again at once: everybody is done with it
+  __syncthreads();
+  int it = 0;
+  for (; it + 2 < kt_count; it += 2) {
+    tile(it, S0(), std::false_type(), acc_a, acc_b);
+    tile(it + 1, S1(), std::false_type(), acc_b, acc_a);
+  }
+  if (it + 1 < kt_count) {
+    tile(it, S0(), std::false_type(), acc_a, acc_b);
+    tile(it + 1, S1(), std::true_type(), acc_b, acc_a);
+  } else {
+    tile(it, S0(), std::true_type(), acc_a, acc_b);
   }
 
   const float l_all = l_part + __shfl_xor(l_part, 32);

@@ -294,6 +294,70 @@ def test_self_attention_sequence_ids(hip, case, causal, act_dtype):
                                  err_msg="d%s fused=%s" % (name, fused))
 
 
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("case", [
+    (8, 64), (64, 128), (72, 64), (136, 128), (200, 64), (264, 64), (320, 128),
+    (392, 64)], ids=lambda c: "x".join(map(str, c)))
+def test_fused_attention_tile_counts(hip, case, causal, with_bias):
+  """One to seven tiles of keys, the last one whole or partly there, with logits
+  large enough that the running maximum moves in most tiles; forward, and the
+  gradients with and without the forward's outputs and denominators.  The bounds:
+  a weight and its gradient are rounded to bf16 once, each result once, and delta
+  may come from outputs that were rounded; 2^-8 of the sum of magnitudes each (a
+  rounding is at most half of that, and the float32 sums fit in the rest)."""
+  l, d = case
+  b, heads, nb = 2, 3, 8
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(l + d + causal + 2 * with_bias)
+  q, k, v, do = (torch.randn((b, l, heads * d), generator=gen, device="cuda")
+                 .to(torch.bfloat16) for _ in range(4))
+  q = q * (3.0 * d ** -0.5)
+  rel = None
+  at = torch.arange(l, device="cuda")
+  if with_bias:
+    bucket = B.relative_position_bucket(np.arange(-(l - 1), l), not causal, nb)
+    rel = (torch.randn((heads, nb), generator=gen, device="cuda").to(torch.bfloat16),
+           torch.from_numpy(bucket.astype(np.int32)).cuda())
+  four = lambda t: t.double().reshape(b, l, heads, d).transpose(1, 2).contiguous()
+  q4, k4, v4, do4 = (four(t) for t in (q, k, v, do))
+  logits = q4 @ k4.transpose(2, 3).contiguous()
+  if with_bias:
+    distance = at[None, :] - at[:, None] + l - 1
+    logits = logits + rel[0].double()[:, rel[1].long()[distance]]
+  if causal:
+    logits = logits.masked_fill(at[None, :] > at[:, None], float("-inf"))
+  w = torch.softmax(logits, -1)
+  want = w @ v4
+  spread = w @ v4.abs()
+  ulp = 2.0 ** -8
+  out, lse = hip.self_attention(q, k, v, heads, causal, relative_bias=rel,
+                                return_lse=True)
+  assert bool(((four(out) - want).abs() <= ulp * (spread + want.abs())).all())
+  assert bool(((lse.double().reshape(b, heads, l) - torch.logsumexp(logits, -1))
+               .abs() <= 2e-5).all())
+  dw = do4 @ v4.transpose(2, 3).contiguous()
+  ds = w * (dw - (do4 * want).sum(-1, keepdim=True))
+  slack = ds.abs() + w * (do4.abs() * (spread + want.abs())).sum(-1, keepdim=True)
+  t = lambda m: m.transpose(2, 3).contiguous()
+  wants = [(ds @ k4, slack @ k4.abs()), (t(ds) @ q4, t(slack) @ q4.abs()),
+           (t(w) @ do4, t(w) @ do4.abs())]
+  for saved in ({}, dict(out=out, lse=lse)):
+    grads = hip.self_attention_backward(q, k, v, do, heads, causal, fused=True,
+                                        relative_bias=rel, **saved)
+    for got, (value, magnitude) in zip(grads, wants):
+      bound = ulp * (magnitude + value.abs())
+      assert bool(((four(got) - value).abs() <= bound).all())
+    if with_bias:
+      at_bucket = torch.nn.functional.one_hot(rel[1].long(), nb).double()
+      by_distance = lambda m: torch.stack([
+          m.diagonal(int(e), dim1=2, dim2=3).sum((0, 2)) for e in range(1 - l, l)], -1)
+      value = by_distance(ds) @ at_bucket
+      magnitude = by_distance(slack) @ at_bucket
+      assert bool(((grads[3].double() - value).abs()
+                   <= ulp * (magnitude + value.abs())).all())
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_attention_at_the_block_benchmark_shape(hip, causal):
   """The fused attention kernels at the (batch, head) shape of the benchmark
