@@ -362,23 +362,16 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void lds_write_b64_asm(uint32_t addr, u32x2_t v) {
   asm volatile("ds_write_b64 %0, %1" :: "v"(addr), "v"(v) : "memory");
 }
-// Eight 16-byte reads, 8192 bytes apart, the even and the odd ones each from an
-// address of their own, and the wait for them: in one asm, whose outputs then
-// hold what the compiler takes them for.
-__device__ __forceinline__ void lds_read_pieces(u32x4_t (&p)[8], uint32_t even,
-                                                uint32_t odd) {
-  asm volatile("ds_read_b128 %0, %8\n\t"
-               "ds_read_b128 %1, %9 offset:8192\n\t"
-               "ds_read_b128 %2, %8 offset:16384\n\t"
-               "ds_read_b128 %3, %9 offset:24576\n\t"
-               "ds_read_b128 %4, %8 offset:32768\n\t"
-               "ds_read_b128 %5, %9 offset:40960\n\t"
-               "ds_read_b128 %6, %8 offset:49152\n\t"
-               "ds_read_b128 %7, %9 offset:57344\n\t"
+// Four 16-byte reads, 8192 bytes apart, and the wait for them: in one asm, whose
+// outputs then hold what the compiler takes them for.
+__device__ __forceinline__ void lds_read_lines(u32x4_t (&p)[4], uint32_t at) {
+  asm volatile("ds_read_b128 %0, %4\n\t"
+               "ds_read_b128 %1, %4 offset:8192\n\t"
+               "ds_read_b128 %2, %4 offset:16384\n\t"
+               "ds_read_b128 %3, %4 offset:24576\n\t"
                "s_waitcnt lgkmcnt(0)"
-               : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]), "=&v"(p[4]),
-                 "=&v"(p[5]), "=&v"(p[6]), "=&v"(p[7])
-               : "v"(even), "v"(odd)
+               : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3])
+               : "v"(at)
                : "memory");
 }
 
@@ -590,7 +583,7 @@ struct RingCfg {
   static constexpr int A_SLOTS = 2, B_SLOTS = 3;
   static constexpr int B_BASE = A_SLOTS * A_BYTES;
   static constexpr size_t LOOP_BYTES = (size_t)A_SLOTS * A_BYTES + (size_t)B_SLOTS * B_BYTES;
-  static constexpr size_t LDS_BYTES = LOOP_BYTES;  // the epilogue stages inside
+  static constexpr size_t LDS_BYTES = LOOP_BYTES;  // the output is staged inside
   static_assert(A_INSTR == 4 && B_INSTR == 4, "load schedule assumes 4 + 4");
 };
 
@@ -663,8 +656,13 @@ __device__ __forceinline__ void ring_tile_blocks(int rem, int tiles_m,
 // share a weight panel: with 400 rows per expert the weights were then read
 // twice from memory and the launches took 14 % longer.)
 // 512 bytes that stay zero (nothing writes them): where a K-major tile reaches
-// past the last reduction row, its rows are loaded from here
-static __device__ __attribute__((aligned(256))) bf16_t kmajor_zero_row[256];
+// past the last reduction row, its rows are loaded from here, and so is the second
+// K tile of a reduction that has one
+static __device__ __attribute__((aligned(256))) bf16_t ring_zero_row[256];
+
+// (the pieces of the kernel are lambdas over its registers: one that the compiler
+// left out of line would move them to memory)
+#define RING_INLINE __attribute__((always_inline))
 
 template <bool RELU, bool GATHER = false, bool KMAJOR = false,
           bool MASKED = false, bool LISTED = false, bool TAILS = false,
@@ -686,9 +684,9 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, WN = Cfg::WN;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
-  // PERSISTENT blocks: one per CU, each walks a strided list of tiles, so that
-  // block start-up and the first loads of a tile overlap the previous tile's
-  // epilogue.  Block b runs on XCD b % 8.  The P = blocks / 8 blocks of an XCD
+  // PERSISTENT blocks: one per CU, each walks a strided list of tiles, whose K tiles
+  // follow each other without a gap: the loads of a tile's last two K tiles are the
+  // next tile's first (see last_tile).  Block b runs on XCD b % 8.  The P = blocks / 8 blocks of an XCD
   // hold P consecutive logical tiles at any moment (shared panels in its L2),
   // and consecutive groups of P tiles go to consecutive XCDs: the whole chip
   // then works on the same one or two experts, whose token panels every XCD
@@ -696,47 +694,55 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // (1 % faster than giving each XCD a contiguous eighth of the tiles).
   const int nblk = gridDim.x;
   if constexpr (LISTED) total_tiles = tile_list[-1];
-  int tile, tile_end, tile_step;
   // TAILS: in its round k a block takes the tile k places further (cyclically)
   // among its XCD's P tiles of the round, so that it meets every row tile of
   // the experts in turn, full and partly empty ones: with a fixed place and an
   // even number of row tiles half of the blocks would only ever get the cheap
   // last row tiles and run ahead of the blocks they share weight panels with.
-  int round = 0;
   const int xcd_tiles = nblk >> 3;
-  const int xcd_first = (blockIdx.x & 7) * xcd_tiles;
-  const int xcd_local = blockIdx.x >> 3;
-  auto tile_of_round = [&](int k) {
-    const int place = xcd_local + k;
-    return k * nblk + xcd_first + (place >= xcd_tiles ? place % xcd_tiles : place);
+  int round_first = (blockIdx.x & 7) * xcd_tiles, place = blockIdx.x >> 3;
+  const int tile = round_first + place;
+  if (tile >= total_tiles) return;
+  // the block's tile of the round after the last one asked for
+  auto following_tile = [&]() {
+    round_first += nblk;
+    if (TAILS) place = place + 1 == xcd_tiles ? 0 : place + 1;
+    return round_first + place;
   };
-  tile = xcd_first + xcd_local;
-  tile_end = total_tiles;
-  tile_step = nblk;
-  if (tile >= tile_end) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int tiles_per_e = tiles_m * tiles_n;
-  // K tiles of the current tile's reduction: all of K, or with k_extent
-  // (KMAJOR) the expert's first k_extent[e] reduction rows only
-  int nk = KMAJOR ? (K + BK - 1) / BK : K / BK;
-  bool tile_empty = false;   // k_extent[e] == 0: the result is zero
-  // SPLIT: first K tile of the current unit, and its place among the partial
-  // results (-1: the unit is a whole tile)
-  int kt0 = 0, unit = -1;
 
-  // per-tile state
-  int row0, col0;
+  // what the K loop and the output of a tile need to know about it
+  struct Tile {
+    // K tiles of its reduction: all of K, or with k_extent (KMAJOR) the expert's
+    // first k_extent[e] reduction rows only
+    int nk;
+    int empty;           // k_extent[e] == 0: the result is zero
+    int unit;            // SPLIT: its place among the partial results (-1: a whole tile)
+    int row0, col0;
+    bf16_t* out;         // the expert's rows of C
+    // TAILS: 32-row pieces of this wavefront's sub-tile that hold rows of the
+    // tile, and of the sub-tiles of the upper half
+    int pieces, pieces0;
+  };
+
+  // the tile that is being loaded: two K tiles ahead of the one that is multiplied
   const bf16_t *Ae, *Be;
-  bf16_t* Ce;
-  typename std::conditional<GATHER, int64_t, int>::type a_off[Cfg::A_INSTR];
-  int b_off[Cfg::B_INSTR];
-  // TAILS: 32-row pieces of this wavefront's sub-tile that hold rows of the
-  // tile, and of the sub-tiles of the upper half
-  int pieces = Cfg::TM, pieces0 = Cfg::TM;
+  // Where a load's 16 bytes lie: a part that is the same for the wavefront, in
+  // scalar registers, and this lane's.  Load j fills the rows 8 (wave + WAVES j) + l / 8
+  // of an LDS tile (KMAJOR: 2 (wave + WAVES j) + l / 32).
+  //   a_row[j]   GATHER: the row of A (negative: zero_row); else (not KMAJOR) the
+  //              bytes to this lane's chunk of its row
+  //   a_lane, b_lane   KMAJOR: elements to this lane's chunk in the pair of rows;
+  //              else b_lane: bytes to its chunk in the eight rows
+  //   b_row[j]   not KMAJOR: elements to the first of the eight rows
+  uint32_t a_row[Cfg::A_INSTR], a_lane = 0, b_lane = 0;
+  int b_row[Cfg::B_INSTR];
+  int kt0 = 0;           // SPLIT: its first K tile
   // first row of row tile tm, and the place in it of LDS tile row `row`
   auto tile_row0 = [&](int tm) { return TAILS ? tm * tile_rows : tm * BM; };
   auto tile_pieces0 = [&](int tm) {
@@ -747,48 +753,57 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     return TAILS && row >= BM / 2 ? row - BM / 2 + 32 * p0 : row;
   };
   // logical tile -> expert, row tile, column tile
-  auto tile_coords = [&](int logical, int& e, int& tm, int& tn) {
-    if constexpr (LISTED) logical = tile_list[logical];
+  auto tile_coords = [&](int logical, int& e, int& tm, int& tn) RING_INLINE {
     e = logical / tiles_per_e;
     const int rem = logical - e * tiles_per_e;
     tn = rem / tiles_m;
     tm = rem - tn * tiles_m;
     if (!LISTED) ring_tile_blocks(rem, tiles_m, tiles_n, tm, tn);
   };
-  // GATHER: the slot -> token map entries of the four rows this lane loads in
-  // a tile.  fetch_map issues the four loads back to back and waits for them
-  // with everything else in flight (written as asm: the compiler would wait for
-  // each before issuing the next, four round trips per tile; the wait belongs
-  // to the same asm, whose outputs then hold what the compiler takes them for).
+  // the chunk that goes to 16-byte position l % 8 of the lane's rows: rows
+  // 8 (wave + 8 j) + l / 8, whose swizzle does not depend on j
+  static_assert(Cfg::WAVES % 2 == 0, "the swizzle of a lane's rows");
+  auto chunk_of = [&](int l) {
+    return ((l & 7) ^ lds_swizzle(wave * 8 + (l >> 3))) * 8;
+  };
+  const int a_chunk = chunk_of(lane);
+  if constexpr (!KMAJOR) b_lane = (uint32_t)((lane >> 3) * K + a_chunk) * 2;
+  // (What a step of the tile loop outside its K loop computes from the lane index, it
+  // computes from a copy that the compiler cannot see through: done once ahead of
+  // the tile loop it would be live across the K loop, which has no registers to
+  // spare.)
+  auto lane_again = [&]() {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  // GATHER: the slot -> token map entries of the four rows this lane loads in a
+  // tile.  They are asked for a whole tile ahead of their use.
   int map_src[Cfg::A_INSTR];
-  auto fetch_map = [&](int logical) {
+  auto fetch_map = [&](int logical) RING_INLINE {
     if constexpr (GATHER) {
       int e, tm, tn;
       tile_coords(logical, e, tm, tn);
       const int p0 = TAILS ? tile_pieces0(tm) : 0;
-      const int32_t* p[Cfg::A_INSTR];
+      const int s_lane = lane_again();
 #pragma unroll
       for (int j = 0; j < Cfg::A_INSTR; ++j) {
-        const int row = row_in_tile((wave + Cfg::WAVES * j) * 8 + (lane >> 3), p0);
-        p[j] = row_map + ((int64_t)e * R + min(tile_row0(tm) + row, R - 1));
+        const int row = row_in_tile((wave + Cfg::WAVES * j) * 8 + (s_lane >> 3), p0);
+        map_src[j] = row_map[(int64_t)e * R + min(tile_row0(tm) + row, R - 1)];
       }
-      static_assert(Cfg::A_INSTR == 4, "four map entries per lane");
-      asm volatile("global_load_dword %0, %4, off\n\t"
-                   "global_load_dword %1, %5, off\n\t"
-                   "global_load_dword %2, %6, off\n\t"
-                   "global_load_dword %3, %7, off\n\t"
-                   "s_waitcnt vmcnt(0)"
-                   : "=&v"(map_src[0]), "=&v"(map_src[1]), "=&v"(map_src[2]),
-                     "=&v"(map_src[3])
-                   : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3])
-                   : "memory");
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto set_tile = [&](int logical) {
+  // (logical: an entry of the tile list where there is one)
+  auto set_tile = [&](int logical) RING_INLINE {
+    Tile t;
+    const int s_lane = lane_again();
     int part = 0;
+    t.unit = -1;
     if constexpr (SPLIT) {
-      unit = logical - whole_tiles;
+      const int unit = logical - whole_tiles;
       if (unit >= 0) {
+        t.unit = unit;
         const int split_tiles = (total_tiles - whole_tiles) / split;
         part = unit / split_tiles;
         logical = whole_tiles + unit - part * split_tiles;
@@ -799,113 +814,106 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     if constexpr (TAILS) {
       const int valid = min(tile_rows, R - tm * tile_rows);
       const int blocks = (valid + 31) >> 5;
-      pieces0 = (blocks + 1) >> 1;
-      pieces = __builtin_amdgcn_readfirstlane(wm == 0 ? pieces0
-                                                      : blocks - pieces0);
+      t.pieces0 = (blocks + 1) >> 1;
+      t.pieces = wm == 0 ? t.pieces0 : blocks - t.pieces0;
+    } else {
+      t.pieces0 = t.pieces = Cfg::TM;
     }
-    row0 = tile_row0(tm);
-    col0 = tn * BN;
+    const int row0 = t.row0 = tile_row0(tm);
+    const int col0 = t.col0 = tn * BN;
+    int nk = KMAJOR ? (K + BK - 1) / BK : K / BK;
+    t.empty = false;
     if constexpr (KMAJOR && !SPLIT) {
       if (k_extent != nullptr) {
         const int used = k_extent[e];
-        tile_empty = used == 0;
-        nk = max(1, min((K + BK - 1) / BK, (used + BK - 1) / BK));
+        t.empty = used == 0;
+        nk = max(1, min(nk, (used + BK - 1) / BK));
       }
     }
     if constexpr (SPLIT) {
-      nk = (K + BK - 1) / BK;
-      tile_empty = false;
       kt0 = 0;
-      if (unit >= 0) {
+      if (t.unit >= 0) {
         const int all = nk;
         kt0 = (int)((int64_t)all * part / split);
         nk = (int)((int64_t)all * (part + 1) / split) - kt0;
         if (nk == 0) {     // fewer K tiles than parts
           nk = 1;
           kt0 = 0;
-          tile_empty = true;
+          t.empty = true;
         }
       }
     }
+    t.nk = nk;
     // (a_stride 0: all experts read the same rows, -1: each its own)
     if constexpr (GATHER) Ae = A;
     else if constexpr (LISTED || MASKED) Ae = A + (int64_t)e * R * K;
     else Ae = A + e * (a_stride < 0 ? (int64_t)R * K : a_stride);
     Be = B + (int64_t)e * N * K;
-    Ce = Cout + (int64_t)e * R * N;
+    t.out = Cout + (int64_t)e * R * N;
+    if constexpr (KMAJOR) {
+      // lane l fills 16-byte position l % 32 of its row with the chunk that
+      // belongs there under the unit swizzle
+      const int p = s_lane & 31, k_row = wave * 2 + (s_lane >> 5);
+      const int chunk = ((((p >> 2) ^ (k_row & 3)) << 2) | (p & 3)) * 8;
+      // (TAILS: what lies past the tile's rows is not multiplied; its lanes
+      // fetch the tile's last piece again)
+      const int row_chunk = TAILS ? min(chunk, tile_rows - 8) : chunk;
+      a_lane = k_row * R + min(row0 + row_chunk, R - 8);
+      b_lane = k_row * N + min(col0 + chunk, N - 8);
+    } else {
 #pragma unroll
-    for (int j = 0; j < Cfg::A_INSTR; ++j) {
-      if constexpr (KMAJOR) {
-        // instruction q = wave + WAVES * j fills tile rows 2q and 2q + 1; lane
-        // l fills 16-byte position l % 32 of its row with the chunk that
-        // belongs there under the unit swizzle
-        const int krow = (wave + Cfg::WAVES * j) * 2 + (lane >> 5);
-        const int p = lane & 31;
-        const int chunk = ((((p >> 2) ^ (krow & 3)) << 2) | (p & 3)) * 8;
-        // (TAILS: what lies past the tile's rows is not multiplied; its lanes
-        // fetch the tile's last piece again)
-        const int row_chunk = TAILS ? min(chunk, tile_rows - 8) : chunk;
-        a_off[j] = krow * R + min(row0 + row_chunk, R - 8);
-        b_off[j] = krow * N + min(col0 + chunk, N - 8);
-        continue;
+      for (int j = 0; j < Cfg::A_INSTR; ++j) {
+        const int row = (wave + Cfg::WAVES * j) * 8 + (s_lane >> 3);
+        if constexpr (GATHER)
+          a_row[j] = map_src[j];
+        else
+          a_row[j] = (uint32_t)(min(row0 + row_in_tile(row, t.pieces0), R - 1) * K +
+                                chunk_of(s_lane)) * 2;
+        // (N % 8 == 0: eight rows exist or they do not)
+        b_row[j] = min(col0 + (wave + Cfg::WAVES * j) * 8, N - 8) * K;
       }
-      const int row = (wave + Cfg::WAVES * j) * 8 + (lane >> 3);
-      const int chunk = (lane & 7) ^ lds_swizzle(row);
-      if constexpr (GATHER) {
-        const int src = map_src[j];
-        a_off[j] = (src >= 0 ? (int64_t)src * K : (int64_t)(zero_row - A)) +
-                   chunk * 8;
-      } else {
-        a_off[j] = min(row0 + row_in_tile(row, pieces0), R - 1) * K + chunk * 8;
-      }
-      b_off[j] = min(col0 + row, N - 1) * K + chunk * 8;
     }
+    return t;
   };
   // load j of the token (A, two slots at LDS offset 0) / weight (B, three
-  // slots behind them) tile kt; kt past the end re-fetches the last tile into
-  // a slot nobody reads any more
+  // slots behind them) tile kt; `zeros`: of a K tile of zeros instead
   constexpr int B_BASE = Cfg::B_BASE;
   // KMAJOR: load j of a tile fills reduction rows 2 (wave + WAVES j) and + 1
   // (lanes 32-63) of it; past the last reduction row they are zeros
   auto kmajor_past_end = [&](int kt, int j) {
     return (kt0 + kt) * BK + (wave + Cfg::WAVES * j) * 2 + (lane >> 5) >= K;
   };
-  auto load_a = [&](int kt, int j) {
-    const int slot = kt & 1;
-    kt = min(kt, nk - 1);
-    const bf16_t* src = Ae + (kt0 + kt) * (KMAJOR ? BK * R : BK) + a_off[j];
-    if constexpr (KMAJOR) {
-      if (kmajor_past_end(kt, j)) src = kmajor_zero_row + (lane & 31) * 8;
-    }
+  auto kmajor_row = [&](int kt, int j) {
+    return (int64_t)((kt0 + kt) * BK + Cfg::WAVES * j * 2);
+  };
+  auto load_a = [&](int kt, int slot, int j, bool zeros = false) RING_INLINE {
+    const bf16_t* src;
+    if constexpr (KMAJOR)
+      src = Ae + kmajor_row(kt, j) * R + a_lane;
+    else if constexpr (GATHER)
+      src = ((int)a_row[j] < 0 ? zero_row : Ae + (int64_t)(int)a_row[j] * K) +
+            (a_chunk + kt * BK);
+    else
+      src = (const bf16_t*)((const char*)(Ae + kt * BK) + a_row[j]);
+    if (zeros || (KMAJOR && kmajor_past_end(kt, j)))
+      src = ring_zero_row + ((KMAJOR ? lane : lane_again()) & 31) * 8;
     __builtin_amdgcn_global_load_lds(
         (glb_void_t*)src,
         (lds_void_t*)(smem_raw + slot * Cfg::A_BYTES +
                       (wave + Cfg::WAVES * j) * 1024), 16, 0, 0);
   };
-  auto load_b = [&](int kt, int slot, int j) {
-    kt = min(kt, nk - 1);
-    const bf16_t* src = Be + (kt0 + kt) * (KMAJOR ? BK * N : BK) + b_off[j];
-    if constexpr (KMAJOR) {
-      if (kmajor_past_end(kt, j)) src = kmajor_zero_row + (lane & 31) * 8;
-    }
+  auto load_b = [&](int kt, int slot, int j, bool zeros = false) RING_INLINE {
+    const bf16_t* src;
+    if constexpr (KMAJOR)
+      src = Be + kmajor_row(kt, j) * N + b_lane;
+    else
+      src = (const bf16_t*)((const char*)(Be + b_row[j] + kt * BK) + b_lane);
+    if (zeros || (KMAJOR && kmajor_past_end(kt, j)))
+      src = ring_zero_row + ((KMAJOR ? lane : lane_again()) & 31) * 8;
     __builtin_amdgcn_global_load_lds(
         (glb_void_t*)src,
         (lds_void_t*)(smem_raw + B_BASE + slot * Cfg::B_BYTES +
                       (wave + Cfg::WAVES * j) * 1024), 16, 0, 0);
-  };
-  // the first loads of a tile except weight tile 1, whose slot the epilogue of
-  // the previous tile still uses as staging area
-  auto prologue_head = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_a(0, j);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_b(0, 0, j);
-  };
-  auto prologue_tail = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_b(1, 1, j);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) load_a(1, j);
   };
 
   f32x16_t acc[Cfg::TM][Cfg::TN];
@@ -920,7 +928,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int t = lane & 15, g = lane >> 4;
     return ((g & 1) * 16 + 4 * (t & 3)) * 2 + ((g >> 1) * 8 + (t >> 2)) * 512;
   };
-  auto set_a_frag = [&]() {
+  auto set_a_frag = [&](int pieces0) {
     const int first = wm == 0 ? 0 : pieces0;
 #pragma unroll
     for (int n = 0; n < Cfg::TM; ++n)
@@ -928,7 +936,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   };
   if constexpr (KMAJOR) {
     static_assert(Cfg::TM <= BK / 16 && Cfg::TN <= BK / 16, "offset arrays");
-    if constexpr (!TAILS) set_a_frag();
+    if constexpr (!TAILS) set_a_frag(Cfg::TM);
 #pragma unroll
     for (int n = 0; n < Cfg::TN; ++n)
       b_frag[n] =
@@ -951,7 +959,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // compiler therefore does not know when the data arrives: wait_frags()
   // (lgkmcnt(0)) stands before the MFMAs that use it.
   const uint32_t lds0 = (uint32_t)(size_t)(lds_void_t*)smem_raw;
-  auto read_tr = [&](uint32_t at, int kk) {
+  auto read_tr = [&](uint32_t at, int kk) RING_INLINE {
     i16x4_t lo, hi;
     switch (kk) {
       case 0: lds_read_tr16_pair<0>(at, lo, hi); break;
@@ -962,35 +970,41 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     return __builtin_bit_cast(
         bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  auto wait_frags = [&]() {
+  auto wait_frags = [&]() RING_INLINE {
     if constexpr (KMAJOR) {
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0) only
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // fragment read n of a step: 0..TM-1 token rows, TM..TM+TN-1 weight rows
-  auto read_frag = [&](int aslot, int bslot, int kk, int buf, int n) {
-    if constexpr (KMAJOR) {
-      if (n < Cfg::TM)
-        fa[buf][n] = read_tr(lds0 + aslot * Cfg::A_BYTES + a_frag[n], kk);
-      else
-        fb[buf][n - Cfg::TM] = read_tr(
-            lds0 + B_BASE + bslot * Cfg::B_BYTES + b_frag[n - Cfg::TM], kk);
-      return;
-    }
-    if (n < Cfg::TM)
-      fa[buf][n] = *reinterpret_cast<const bf16x8_t*>(
-          smem_raw + aslot * Cfg::A_BYTES + a_frag[kk] + n * 32 * Cfg::ROW_BYTES);
+  // token fragment of piece n / weight fragment n of MFMA step kk
+  auto read_a = [&](int aslot, int kk, int n) RING_INLINE -> bf16x8_t {
+    if constexpr (KMAJOR)
+      return read_tr(lds0 + aslot * Cfg::A_BYTES + a_frag[n], kk);
     else
-      fb[buf][n - Cfg::TM] = *reinterpret_cast<const bf16x8_t*>(
-          smem_raw + B_BASE + bslot * Cfg::B_BYTES + b_frag[kk] +
-          (n - Cfg::TM) * 32 * Cfg::ROW_BYTES);
+      return *reinterpret_cast<const bf16x8_t*>(
+          smem_raw + aslot * Cfg::A_BYTES + a_frag[kk] + n * 32 * Cfg::ROW_BYTES);
   };
-  auto mfma = [&](int buf, int n) {
+  auto read_b = [&](int bslot, int kk, int n) RING_INLINE -> bf16x8_t {
+    if constexpr (KMAJOR)
+      return read_tr(lds0 + B_BASE + bslot * Cfg::B_BYTES + b_frag[n], kk);
+    else
+      return *reinterpret_cast<const bf16x8_t*>(
+          smem_raw + B_BASE + bslot * Cfg::B_BYTES + b_frag[kk] +
+          n * 32 * Cfg::ROW_BYTES);
+  };
+  // fragment read n of a step: 0..TM-1 token rows, TM..TM+TN-1 weight rows
+  auto read_frag = [&](int aslot, int bslot, int kk, int buf, int n) RING_INLINE {
+    if (n < Cfg::TM) fa[buf][n] = read_a(aslot, kk, n);
+    else fb[buf][n - Cfg::TM] = read_b(bslot, kk, n - Cfg::TM);
+  };
+  // (first: the sums begin)
+  auto mfma = [&](int buf, int n, bool first = false) RING_INLINE {
     const int i = n / Cfg::TN, j = n % Cfg::TN;
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[buf][j], fa[buf][i],
-                                                        acc[i][j], 0, 0, 0);
+    const f32x16_t none = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                           0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        fb[buf][j], fa[buf][i], first ? none : acc[i][j], 0, 0, 0);
   };
   // with NA of the wavefront's TM row pieces in use: is fragment read n /
   // MFMA n of a step needed?
@@ -1004,32 +1018,49 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // tile j = n % TN inner) first need them: a0 b0 b1 a1 a2 a3
   constexpr int RD[6] = {0, Cfg::TM, Cfg::TM + 1, 1, 2, 3};
 
-  // bslot = kt % 3, kept incrementally
-  int bslot = 0;
-  auto k_tile = [&](int kt, auto last_tag, auto na_tag) {
-    constexpr bool LAST = decltype(last_tag)::value;
+  // Output lines: 16 bytes per lane, eight rows of 128 bytes per store.  `base`
+  // is the first of the eight rows, `rows` how many of them are rows of the output
+  // (what the buffer's range drops; a store leaves in any case, the waits count
+  // on that), line_at this lane's place, out of range where the columns end.
+  constexpr int STORES = 4;       // per 32-row piece
+  constexpr uint32_t OUTSIDE = 0x80000000u;    // (8 rows of N < 2^25 end before)
+  auto store_line = [&](u32x4_t v, bf16_t* base, int rows, uint32_t line_at)
+      RING_INLINE {
+    rows = max(rows, 0);
+    asm("" : "+s"(rows));    // (scalar: not one clamp in the vector unit)
+    const int bytes = min(rows, 8) * N * 2;
+    __builtin_amdgcn_raw_buffer_store_b128(
+        v, __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000), line_at,
+        0, 0);
+  };
+  // slots of the K tile that is multiplied, and the K tile (of the tile that is
+  // being loaded) that its loads fetch
+  int aslot = 0, bslot = 0, lk = 2;
+  // FIRST: K tile 0
+  auto k_tile = [&](auto first_tag, auto na_tag) RING_INLINE {
+    constexpr bool FIRST = decltype(first_tag)::value;
     constexpr int NA = decltype(na_tag)::value;      // row pieces in use
     auto rd = [&](int as, int bs, int kk, int buf, int n) {
       if (frag_used(NA, n)) read_frag(as, bs, kk, buf, n);
     };
+    int kk_now = 0;
     auto mm = [&](int buf, int n) {
-      if (mfma_used(NA, n)) mfma(buf, n);
+      if (mfma_used(NA, n)) mfma(buf, n, FIRST && kk_now == 0);
     };
-    const int aslot = kt & 1;
-    const int bnext = bslot == 2 ? 0 : bslot + 1;       // slot of tile kt+1
-    const int bnext2 = bnext == 2 ? 0 : bnext + 1;      // slot of tile kt+2
+    const int bnext = bslot == 2 ? 0 : bslot + 1;       // slot of the next K tile
+    const int bnext2 = bnext == 2 ? 0 : bnext + 1;      // of the one after it
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
       const int cur = kk & 1, nxt = cur ^ 1;
-      // The loads a step carries: the four weight loads of tile kt+2 over
-      // steps 0..2, all four token loads of tile kt+2 right behind the
+      kk_now = kk;
+      // The loads a step carries: the four weight loads of the K tile after the
+      // next over steps 0..2, all four token loads of it right behind the
       // hand-over barrier that frees their slot (a full K tile ahead of use).
       auto load = [&](int which) {
-        if (LAST) return;
-        if (kk == 0) load_b(kt + 2, bnext2, which);
-        if (kk == 1 && which == 0) load_b(kt + 2, bnext2, 2);
-        if (kk == 2 && which == 0) load_b(kt + 2, bnext2, 3);
-        if (kk == 3) load_a(kt + 2, which);
+        if (kk == 0) load_b(lk, bnext2, which);
+        if (kk == 1 && which == 0) load_b(lk, bnext2, 2);
+        if (kk == 2 && which == 0) load_b(lk, bnext2, 3);
+        if (kk == 3) load_a(lk, aslot, which);
       };
       if (kk + 1 < KSTEPS) {
         // 6 fragment reads of step kk+1 (in the order its MFMAs need them),
@@ -1052,7 +1083,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         rd(aslot, bslot, kk + 1, nxt, RD[5]);
         mm(cur, 6); fence();
         mm(cur, 7); fence();
-      } else if (!LAST) {
+      } else {
         // this lane holds the last step's fragments (lgkmcnt 0); everything
         // but the four weight loads of tile kt+2 has landed (vmcnt 4)
         fence();
@@ -1071,236 +1102,333 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         }
         mm(cur, 6); fence();
         mm(cur, 7); fence();
-      } else {
-        wait_frags();
-#pragma unroll
-        for (int n = 0; n < 8; ++n) mm(cur, n);
       }
     }
+    aslot ^= 1;
     bslot = bnext;
+    ++lk;
   };
 
-  // Epilogue staging: two passes of 128 output rows (64 from each half of the
-  // tile, so that all eight wavefronts write), exactly the last two weight
-  // slots, which are free once the K loop is over.  Rows are 512 bytes, a
-  // multiple of the bank count, so 16-byte chunk c of staging row r lives at
-  // chunk c ^ (r & 31): the writes of a wavefront (32 rows x 8 bytes, twice)
-  // and its reads (2 rows x 32 chunks) both spread over all banks.
-  constexpr int EPI_ROWS = 128;
-  constexpr int EPI_ROW_BYTES = BN * 2;
-  constexpr int EPI_BASE = B_BASE + Cfg::B_BYTES;
-  static_assert(EPI_BASE + EPI_ROWS * EPI_ROW_BYTES <= (int)Cfg::LOOP_BYTES,
-                "epilogue staging exceeds the ring");
-  static_assert(BN == 256 && Cfg::WM == 2 && Cfg::TM == 4, "epilogue layout");
-  // (LDS byte address of the staging area: its accesses are written as asm)
-  const uint32_t cs0 = (uint32_t)(size_t)(lds_void_t*)smem_raw + EPI_BASE;
-  const int m_l = lane & 31;
-  const int half = lane >> 5;   // which 8 bytes of a 16-byte chunk
-  constexpr int CPR_C = BN / 8;  // 16-byte chunks per output row
-
-  fetch_map(tile);
-  set_tile(tile);
-  prologue_head();
-  prologue_tail();
-  for (;;) {
+  // The last K tile of a tile, its output, and the hand-over to the next tile.
+  //
+  // The K tile is multiplied piece by piece (32 rows of the wavefront's sub-tile):
+  // step 0 of all pieces, then steps 1 to 3 of one after the other, and while the
+  // matrix pipe is at piece i + 1, piece i is rounded (and relu), turned round in
+  // LDS and stored, 16 bytes per lane and whole 128-byte lines.  Each wavefront
+  // turns its pieces round by itself, without barriers, in the four kilobytes of
+  // the free weight slot that its own loads of the next tile's K tile 1 fill
+  // afterwards.  By then K tile 0 of the next tile has been on its way for a whole K
+  // tile, so the matrix pipes go on with it at once, and the stores have that
+  // much time before anything waits for them.
+  //
+  //
+  // A tile's output used to be staged by all wavefronts in two passes behind block
+  // barriers, with the ring drained and nothing multiplied, 6.5 us a tile.  Before and
+  // now, back to back: 16384 rows, 1024 -> 4096 126 -> 118 us, -> 1024 34.4 -> 31.3;
+  // 16 x 705 rows, 768 -> 3072 62 -> 53; 64 x 512 rows, 1024 -> 4096 270 -> 260; weight
+  // gradients of 64 x 512 rows 312 -> 293.  Without stores and staging the same
+  // launches take 103, 26.6, 46, 229 and 229: what is left is work, not waiting (a
+  // compute unit's 128 KB take 4.7 us when the whole chip stores, 2.7 if they stay in
+  // the L2s).  Twelve of the sixteen stores held back for the next three K tiles are no
+  // faster.  Turned round in registers (v_permlane32_swap, v_permlane16_swap) instead
+  // of LDS a store covers rows of 64 bytes, which cost the L2 1.4 times as long: weight
+  // gradients 293 -> 309.
+  const uint32_t lds_base = (uint32_t)(size_t)(lds_void_t*)smem_raw;
+  // The fragments of a tile's first step: read right behind the hand-over, or (TAILS:
+  // the wavefront's pieces in the next tile are another copy of the code) ahead of
+  // its first K tile.
+  auto first_frags = [&](int as, int bs, int na) RING_INLINE {
 #pragma unroll
-    for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-      for (int j = 0; j < Cfg::TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    // K tile 0 has landed: only tile 1 (4 + 4 loads) may still be in flight
-    wait_vmcnt<8>();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if constexpr (KMAJOR && TAILS) set_a_frag();
-    auto k_loop = [&](auto na_tag) {
-      constexpr int NA = decltype(na_tag)::value;
-#pragma unroll
-      for (int n = 0; n < 6; ++n)
-        if (frag_used(NA, RD[n])) read_frag(0, 0, 0, 0, RD[n]);
-      bslot = 0;
-      for (int kt = 0; kt + 1 < nk; ++kt) k_tile(kt, std::false_type{}, na_tag);
-      k_tile(nk - 1, std::true_type{}, na_tag);
+    for (int n = 0; n < 6; ++n)
+      if (frag_used(na, RD[n])) read_frag(as, bs, 0, 0, RD[n]);
+  };
+  auto last_tile = [&](const Tile& t, const Tile& after, bool has_next,
+                       auto na_tag) RING_INLINE {
+    constexpr int NA = decltype(na_tag)::value;
+    constexpr int TN = Cfg::TN;
+    static_assert(Cfg::TM == 4 && TN == 2 && KSTEPS == 4 && Cfg::WTN == 64,
+                  "a piece is 32 rows of 128 bytes");
+    const int bnext = bslot == 2 ? 0 : bslot + 1;       // K tile 0 of the next tile
+    const int bfree = bnext == 2 ? 0 : bnext + 1;       // K tile 1: free till then
+    bf16x8_t ga[2][KSTEPS - 1], gb[KSTEPS - 1][TN];
+    auto mm = [&](int i, int n) {
+      const int kk = n / TN, j = n % TN;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gb[kk][j], ga[i & 1][kk],
+                                                          acc[i][j], 0, 0, 0);
     };
-    if constexpr (TAILS) {
-      switch (pieces) {
-        case 0: k_loop(std::integral_constant<int, 0>{}); break;
-        case 1: k_loop(std::integral_constant<int, 1>{}); break;
-        case 2: k_loop(std::integral_constant<int, 2>{}); break;
-        case 3: k_loop(std::integral_constant<int, 3>{}); break;
-        default: k_loop(std::integral_constant<int, Cfg::TM>{}); break;
-      }
-    } else {
-      k_loop(std::integral_constant<int, Cfg::TM>{});
-    }
-
-    const int next = (TAILS && xcd_tiles != 0) ? tile_of_round(round + 1)
-                                               : tile + tile_step;
-    const bool has_next = next < tile_end;
-    // (the next tile's map entries travel while the ring drains)
-    if (has_next) fetch_map(next);
-    // Every wavefront is done with the ring and no direct-to-LDS load is in
-    // flight (the last hand-over re-fetched a tile nobody reads).
-    wait_vmcnt<0>();
-    asm volatile("" ::: "memory");
-    __syncthreads();
-    const int out_row0 = row0, out_col0 = col0, out_pieces0 = pieces0;
-    bf16_t* out_c = Ce;
-    const int out_unit = unit;
-    if constexpr (KMAJOR || SPLIT) {
-      // an expert without reduction rows: its one K tile held rows that
-      // nobody wrote
-      if (tile_empty) {
-#pragma unroll
-        for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-          for (int j = 0; j < Cfg::TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-      }
-    }
-    // staging row -> row of the output
-    auto out_row = [&](int pass, int srow) {
-      return out_row0 + (srow >> 6) * (TAILS ? 32 * out_pieces0 : 128) +
-             pass * 64 + (srow & 63);
-    };
-    // MASKED: the mask of a pass's pieces, all loads together and ahead of the
-    // staging.  (In front of its store, each was waited for by itself: what the
-    // mask costs a launch of 64 x 2048 rows, 1024 x 4096, is 108 us instead of 232,
-    // 16000 rows, 768 x 3072, 4 instead of 13.  Touching the mask's lines two K
-    // tiles earlier, for the L2, costs twice what it saves.)
-    constexpr int PIECES = EPI_ROWS * CPR_C / Cfg::THREADS;
-    u32x4_t mask[MASKED ? PIECES : 1];
-    auto load_mask = [&](int pass) {
+    const int e_lane = lane_again();
+    // Writes: row l % 32, 8-byte unit 2 c + l / 32 of it at unit (2 c + l / 32) ^
+    // (2 (row % 8) + row / 8 % 2); reads: row 8 n + l / 8, chunk l % 8, whose two
+    // units are exchanged where n is odd.  Both spread over all banks.
+    const uint32_t stage = lds_base + B_BASE + bfree * Cfg::B_BYTES + wave * 1024;
+    const int w_row = e_lane & 31;
+    const uint32_t w_at =
+        stage + (w_row >> 3) * (Cfg::WAVES * 1024) + (w_row & 7) * 128 +
+        (((e_lane >> 5) ^ ((w_row & 7) * 2) ^ ((w_row >> 3) & 1)) * 8);
+    const int r_row = e_lane >> 3, r_chunk = e_lane & 7;
+    const uint32_t r_at = stage + r_row * 128 + ((r_chunk ^ r_row) * 16);
+    const int first_row = t.row0 + (wm == 0 ? 0 : TAILS ? 32 * t.pieces0 : Cfg::WTM);
+    const int end_row = TAILS ? min(R, t.row0 + tile_rows) : R;
+    const int col = t.col0 + wn * Cfg::WTN + r_chunk * 8;
+    bf16_t* const out = t.out + (int64_t)first_row * N + t.col0 + wn * Cfg::WTN;
+    const uint32_t line_at =
+        col < N ? (uint32_t)(r_row * N + r_chunk * 8) * 2 : OUTSIDE;
+    u32x4_t mask[2][MASKED ? STORES : 1];
+    auto load_mask = [&](int i) {
       if constexpr (MASKED) {
-        int m_tid = tid;
-        asm volatile("" : "+v"(m_tid));
-        const bf16_t* m = mask_src + (out_c - Cout) +
-                          min(out_col0 + m_tid % CPR_C * 8, N - 8);
+        const bf16_t* m = mask_src + (t.out - Cout) + min(col, N - 8);
 #pragma unroll
-        for (int n = 0; n < PIECES; ++n)
-          mask[n] = *reinterpret_cast<const u32x4_t*>(
-              m + (int64_t)min(out_row(pass, m_tid / CPR_C + 16 * n), R - 1) * N);
+        for (int n = 0; n < STORES; ++n)
+          mask[i & 1][n] = *reinterpret_cast<const u32x4_t*>(
+              m + (int64_t)min(first_row + 32 * i + 8 * n + r_row, R - 1) * N);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    load_mask(0);
-    if (has_next) {
-      // the next tile's first loads fly while this tile is written out
-      set_tile(next);
-      prologue_head();
-    }
-    if constexpr (SPLIT) {
-      if (out_unit >= 0) {
+    const bool part = SPLIT && t.unit >= 0;
+    // piece i, two of its eight groups of 4 columns per lane
+    auto put = [&](int i, int g) {
+      if (part) return;
+#pragma unroll
+      for (int c = 2 * g; c < 2 * g + 2; ++c) {
+        const int j = c >> 2, q = c & 3;
+        u32x2_t v;
+        v.x = pack2_bf16(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], RELU);
+        v.y = pack2_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3], RELU);
+        lds_write_b64_asm(w_at ^ (16 * c), v);
+      }
+    };
+    u32x4_t line[STORES];
+    auto get = [&]() {
+      if (!part) lds_read_lines(line, r_at);
+    };
+    // line n of piece i as it goes to memory
+    auto finished = [&](int i, int n) {
+      u32x4_t v = line[n];
+      if (n & 1) v = __builtin_shufflevector(v, v, 2, 3, 0, 1);
+      if constexpr (MASKED) {
+        const u32x4_t hm = mask[i & 1][n];
+        if (mask_scale != 1.0f) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            v[q] = f32x2_to_bf16x2(
+                __builtin_bit_cast(float, v[q] << 16) * mask_scale,
+                __builtin_bit_cast(float, v[q] & 0xffff0000u) * mask_scale);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t keep =
+              (__builtin_bit_cast(float, hm[q] << 16) > 0.f ? 0xffffu : 0u) |
+              (__builtin_bit_cast(float, hm[q] & 0xffff0000u) > 0.f
+                   ? 0xffff0000u : 0u);
+          v[q] &= keep;
+        }
+      }
+      return v;
+    };
+    auto store = [&](int i) {
+      if (part) {
         // a part of a tile's reduction: the accumulators as they lie, 16
         // bytes per lane and register group; split_reduce_kernel adds the
         // parts and knows the layout
-        float* dst = partial + (int64_t)out_unit * (BM * BN) + tid * 4;
+        float* dst = partial + (int64_t)t.unit * (BM * BN) +
+                     (wave * 64 + e_lane) * 4;
 #pragma unroll
-        for (int i = 0; i < Cfg::TM; ++i)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-          for (int j = 0; j < Cfg::TN; ++j)
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<float4*>(
+                dst + ((i * TN + j) * 4 + q) * (Cfg::THREADS * 4)) =
+                make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
+                            acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        return;
+      }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-              *reinterpret_cast<float4*>(
-                  dst + ((i * Cfg::TN + j) * 4 + q) * (Cfg::THREADS * 4)) =
-                  make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1],
-                              acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-        if (!has_next) break;
-        tile = next;
-        ++round;
-        prologue_tail();
-        continue;
+      for (int n = 0; n < STORES; ++n) {
+        store_line(finished(i, n), out + (int64_t)(32 * i + 8 * n) * N,
+                   end_row - first_row - 32 * i - 8 * n, line_at);
+      }
+    };
+    auto zero_if_empty = [&](int i) {
+      if constexpr (KMAJOR || SPLIT) {
+        // an expert without reduction rows: its one K tile held rows that
+        // nobody wrote
+        if (t.empty) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        }
+      }
+    };
+
+    if constexpr (NA > 0) {
+      // step 0 of all pieces; meanwhile the fragments of piece 0's step 1
+      fence();
+      wait_frags();
+      ga[0][0] = read_a(aslot, 1, 0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) gb[0][j] = read_b(bslot, 1, j);
+      fence();
+#pragma unroll
+      for (int m = 0; m < NA * TN; ++m) { mfma(0, m); fence(); }
+      load_mask(0);
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        fence();
+        wait_frags();
+        if (i == 0) {
+          // (the fragments of piece 0's steps 2 and 3)
+#pragma unroll
+          for (int kk = 2; kk < KSTEPS; ++kk) {
+            ga[0][kk - 1] = read_a(aslot, kk, 0);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) gb[kk - 1][j] = read_b(bslot, kk, j);
+          }
+          fence();
+        }
+        mm(i, 0); fence();
+        mm(i, 1); fence();
+        if (i == 0) wait_frags();
+        if (i + 1 < NA) {
+#pragma unroll
+          for (int kk = 1; kk < KSTEPS; ++kk)
+            ga[(i + 1) & 1][kk - 1] = read_a(aslot, kk, i + 1);
+          fence();
+        }
+        if (i > 0) { zero_if_empty(i - 1); put(i - 1, 0); put(i - 1, 1); }
+        mm(i, 2); fence();
+        if (i > 0) { put(i - 1, 2); put(i - 1, 3); }
+        mm(i, 3); fence();
+        if (i > 0) get();
+        mm(i, 4); fence();
+        if (i > 0) store(i - 1);
+        mm(i, 5); fence();
+        if (i + 1 < NA) load_mask(i + 1);
       }
     }
-    // round (and relu), stage in LDS, coalesced 16-byte stores.  Nothing here
-    // waits for vector memory: the next tile's first loads and this tile's
-    // stores stay in flight.  (__syncthreads() waits for them at every
-    // barrier, and in front of an ordinary LDS access the compiler waits for
-    // the direct-to-LDS loads in flight, which might write the same LDS: the
-    // staging accesses are therefore asm.)
-    // (the staging addresses are formed from a copy of the thread index that
-    // the compiler cannot see through: computed once outside the tile loop
-    // they would be live across the K loop, which has no registers to spare)
-    int e_tid = tid;
-    asm volatile("" : "+v"(e_tid));
-    const int e_lane = e_tid & 63, e_wave = e_tid >> 6;
-    const int e_wm = e_wave / WN, e_wn = e_wave % WN;
-    const int e_ml = e_lane & 31, e_half = e_lane >> 5;
+    // Hand-over: the fragments of this tile are in registers, and all but the
+    // stores that came after the loads of the next tile's K tile 0 are done.
+    fence();
+    constexpr int LATER = NA > 1 ? STORES * (NA - 1) : 0;
+    __builtin_amdgcn_s_waitcnt((LATER & 15) | (0 << 8) | (7 << 4));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fence();
+    // (K tile 1 as a number that the compiler does not know: it would keep K tile 0's
+    // addresses to add to)
+    int kt1 = 1;
+    asm volatile("" : "+s"(kt1));
+    if (has_next) {
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
+      for (int j = 0; j < 4; ++j) load_a(kt1, aslot, j, after.nk < 2);
+    }
+    fence();
+    if constexpr (!TAILS) first_frags(aslot ^ 1, bnext, Cfg::TM);
+    fence();
+    if constexpr (NA > 0) {
+      zero_if_empty(NA - 1);
 #pragma unroll
-      for (int ii = 0; ii < 2; ++ii) {
-        const int i = pass * 2 + ii;
-        const int srow = e_wm * 64 + ii * 32 + e_ml;
+      for (int g = 0; g < 4; ++g) put(NA - 1, g);
+      get();
+      store(NA - 1);
+    }
+    wait_frags();
+    fence();
+    if (has_next) {
 #pragma unroll
-        for (int j = 0; j < Cfg::TN; ++j) {
+      for (int j = 0; j < 4; ++j) load_b(kt1, bfree, j, after.nk < 2);
+    }
+    fence();
+    aslot ^= 1;
+    bslot = bnext;
+    lk = 2;
+  };
+
+  // The block's next tile and the one after it: their numbers in the list where
+  // there is one, read ahead of their use.
+  auto entry_of = [&](int number) {
+    if constexpr (LISTED) return tile_list[min(number, total_tiles - 1)];
+    else return number;
+  };
+  Tile t = [&]() {
+    const int entry = entry_of(tile);
+    fetch_map(entry);
+    return set_tile(entry);
+  }();
+  int next = following_tile(), next2 = following_tile();
+  int next_entry = entry_of(next), next2_entry = entry_of(next2);
+  if (next < total_tiles) fetch_map(next_entry);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int chunk = (e_wn * Cfg::WTN + j * 32 + 8 * q) / 8;
-            u32x2_t v;
-            v.x = pack2_bf16(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], RELU);
-            v.y = pack2_bf16(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3], RELU);
-            lds_write_b64_asm(cs0 + srow * EPI_ROW_BYTES +
-                                  ((chunk ^ e_ml) * 16) + e_half * 8, v);
-          }
-        }
+  for (int j = 0; j < 4; ++j) load_a(0, 0, j);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) load_b(0, 0, j);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) load_b(1, 1, j, t.nk < 2);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) load_a(1, 1, j, t.nk < 2);
+  // K tile 0 has landed: only tile 1 (4 + 4 loads) may still be in flight
+  wait_vmcnt<8>();
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  if constexpr (!TAILS) first_frags(0, 0, Cfg::TM);
+  wait_frags();
+  for (;;) {
+    if constexpr (KMAJOR && TAILS) set_a_frag(t.pieces0);
+    const bool has_next = next < total_tiles;
+    Tile after = t;
+    auto tile_pass = [&](auto na_tag) RING_INLINE {
+      if constexpr (TAILS) {
+        first_frags(aslot, bslot, decltype(na_tag)::value);
+        wait_frags();
       }
-      lds_barrier();
-      // all staged pieces of this pass first, one wait, then the stores
-      static_assert(EPI_ROWS * CPR_C % Cfg::THREADS == 0, "whole pieces");
-      u32x4_t piece[PIECES];
-      // piece n: staging row (e_tid / CPR_C) + 16 n
-      static_assert(PIECES == 8 && Cfg::THREADS / CPR_C == 16 &&
-                        16 * EPI_ROW_BYTES == 8192, "offsets of the reads");
-      const uint32_t row_at = cs0 + e_tid / CPR_C * EPI_ROW_BYTES;
-      const uint32_t at = (e_tid % CPR_C) ^ (e_tid / CPR_C);
-      lds_read_pieces(piece, row_at + at * 16, row_at + (at ^ 16) * 16);
-#pragma unroll
-      for (int n = 0; n < PIECES; ++n) {
-        const int c = e_tid + n * Cfg::THREADS;
-        const int srow = c / CPR_C, chunk = c % CPR_C;
-        // 64 rows of each half of the tile
-        const int half_row = pass * 64 + (srow & 63);
-        const int grow = out_row(pass, srow);
-        const int gcol = out_col0 + chunk * 8;
-        // (TAILS: a half's rows past its pieces belong to the other half or to
-        // the next tile)
-        if (grow < (TAILS ? min(R, out_row0 + tile_rows) : R) && gcol < N &&
-            !(TAILS && srow < 64 && half_row >= 32 * out_pieces0)) {
-          u32x4_t v = piece[n];
-          if constexpr (MASKED) {
-            const u32x4_t hm = mask[n];
-            if (mask_scale != 1.0f) {
-#pragma unroll
-              for (int q = 0; q < 4; ++q)
-                v[q] = f32x2_to_bf16x2(
-                    __builtin_bit_cast(float, v[q] << 16) * mask_scale,
-                    __builtin_bit_cast(float, v[q] & 0xffff0000u) * mask_scale);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t keep =
-                  (__builtin_bit_cast(float, hm[q] << 16) > 0.f ? 0xffffu : 0u) |
-                  (__builtin_bit_cast(float, hm[q] & 0xffff0000u) > 0.f
-                       ? 0xffff0000u : 0u);
-              v[q] &= keep;
-            }
-          }
-          *reinterpret_cast<u32x4_t*>(out_c + (int64_t)grow * N + gcol) = v;
+      // The loads of the last two K tiles are the next tile's.  (Its map entries are
+      // older than the eight loads of a K tile that are in flight.  Without a next
+      // tile they are the first of this one again, which nobody reads.)
+      auto advance = [&]() RING_INLINE {
+        if (has_next) {
+          if constexpr (GATHER) wait_vmcnt<8>();
+          after = set_tile(next_entry);
+          if (next2 < total_tiles) fetch_map(next2_entry);
         }
+        lk = 0;
+      };
+      if (t.nk > 2) {
+        k_tile(std::true_type{}, na_tag);
+        for (int kt = 1; kt < t.nk - 2; ++kt) k_tile(std::false_type{}, na_tag);
+        advance();
+        k_tile(std::false_type{}, na_tag);
+      } else {
+        // (two K tiles at least: the second of one holds zeros)
+        advance();
+        k_tile(std::true_type{}, na_tag);
       }
-      if (pass == 0) load_mask(1);
-      lds_barrier();
+      last_tile(t, after, has_next, na_tag);
+    };
+    if constexpr (TAILS) {
+      switch (t.pieces) {
+        case 0: tile_pass(std::integral_constant<int, 0>{}); break;
+        case 1: tile_pass(std::integral_constant<int, 1>{}); break;
+        case 2: tile_pass(std::integral_constant<int, 2>{}); break;
+        case 3: tile_pass(std::integral_constant<int, 3>{}); break;
+        default: tile_pass(std::integral_constant<int, Cfg::TM>{}); break;
+      }
+    } else {
+      tile_pass(std::integral_constant<int, Cfg::TM>{});
     }
     if (!has_next) break;
-    tile = next;
-    ++round;
-    prologue_tail();   // the staging area is free again
+    t = after;
+    next = next2;
+    next_entry = next2_entry;
+    next2 = following_tile();
+    next2_entry = entry_of(next2);
   }
+  // no direct-to-LDS load may outlive the block
+  wait_vmcnt<0>();
 }
+
+#undef RING_INLINE
 
 // Sums the parts of the split tiles of a ring launch, in part order, rounds
 // once and writes the tiles.  One block per (tile, MFMA tile of the
@@ -1825,6 +1953,7 @@ static bool kmajor_path_applies(const void* A, const void* B, const void* C,
                                 int R, int N, int K, int dtype) {
   return dtype == MESH_MOE_BF16 && K >= 1 &&
          R % 8 == 0 && N % 8 == 0 && R >= 128 && N >= 128 &&
+         R < (1 << 25) && N < (1 << 25) &&   // 32-bit offsets within 32 rows
          (int64_t)R * K < (1LL << 31) && (int64_t)N * K < (1LL << 31) &&
          (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) == 0;
 }
@@ -1882,6 +2011,8 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 // times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
 // 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
 // expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside
+// (measured with the output staged behind the K loop; that it now runs beside
+// it changes none of the choices below)
 // the K loop.  Rows are spread evenly over the row tiles: 640 rows per expert are
 // three tiles of 224 or four of 160, not 256 + 256 + 128.  Measured, tiles of
 // 256 and a shorter last one -> the rule's choice (both sides bit-identical):

@@ -1723,6 +1723,50 @@ def test_weight_gradient_row_tiles(hip, shape):
     assert bool(((dw[i].float() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 1024])
+@pytest.mark.parametrize("e,rows,n", [(36, 300, 1288), (150, 130, 520),
+                                      (3, 5376, 1536)])
+def test_linear_tile_after_tile(hip, e, rows, n, k):
+  """More tiles than compute units, so that blocks go from one to the next: with
+  fewer K tiles than a block loads ahead, with rows and columns that end inside a
+  tile (whose neighbours' rows must stay as they are), with the ReLU and with its
+  mask.  The bound: one bf16 rounding, and for each of the two float32 sums of K
+  products K / 2 ulps of the sum of magnitudes."""
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(e + rows + n + k)
+  a, w, dy = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16)
+              for s in ((e, rows, k), (e, n, k), (e, rows, k)))
+  y = hip.expert_linear(a, w, "relu")
+  # dx = dy . v^T where y > 0, v [E, N, K]: the same product, masked
+  v = w
+  dx = hip.expert_linear_backward(y, dy, v, da_relu_mask=y)[0]
+  for i in range(e):
+    for got, lhs, keep in ((y, a, None), (dx, dy, y)):
+      want = lhs[i].float() @ w[i].float().t().contiguous()
+      magnitude = lhs[i].float().abs() @ w[i].float().abs().t().contiguous()
+      want = want.clamp(min=0) if keep is None else want * (keep[i] > 0)
+      bound = 2.0 ** -8 * want.abs() + k * 2.0 ** -24 * magnitude
+      assert bool(((got[i].float() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("rows", [1, 40, 64, 65, 128, 130, 192, 200])
+@pytest.mark.parametrize("e,k,n", [(30, 264, 2568), (12, 1280, 1288)])
+def test_weight_gradient_of_few_rows(hip, rows, e, k, n):
+  """Reductions of one to four K tiles, more tiles than compute units; the bound as
+  in the test above."""
+  gen = torch.Generator(device="cuda")
+  gen.manual_seed(rows + e)
+  a, dy, w = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16)
+              for s in ((e, rows, k), (e, rows, n), (e, k, n)))
+  dw = hip.expert_linear_backward(a, dy, w, want_da=False)[1]
+  for i in range(e):
+    at = a[i].float().t().contiguous()
+    want = at @ dy[i].float()
+    magnitude = at.abs() @ dy[i].float().abs()
+    bound = 2.0 ** -8 * want.abs() + rows * 2.0 ** -24 * magnitude
+    assert bool(((dw[i].float() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("shape", [
     (8, 320, 2048, 512), (8, 320, 512, 2048), (2, 33, 36, 100), (1, 32, 32, 32),
     (1, 2000, 260, 1028), (40, 65, 68, 132), (3, 161, 1000, 64), (5, 97, 64, 300)],
