@@ -5,6 +5,7 @@
 // float32 operation order of mtf.softmax (ops.py:5493-5541) and mtf.top_1
 // (ops.py:4937-4940).  The dense [G,S,E] masks and the S x S cumsum matmul
 // (ops.py:2761-2781) are replaced by a per-token record and integer counting.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -806,11 +807,14 @@ __host__ __device__ constexpr int select_row_floats(int E) {
   return (E + 3) / 4 * 4 + 4;            // 16-byte rows, odd in units of 16 bytes
 }                                        // for E = 8 n
 
-template <typename IT, int LANES>
+// TAIL: another block of the launch reads the records and partial sums (device-scope
+// stores, see st_dev); the choices also go to ch [3][TOKENS] in LDS (-1: not competing;
+// the third: what the loss counts), and `pos` is left to gate_rank_block.
+template <typename IT, int LANES, bool TAIL = false>
 __device__ __forceinline__ void gate_select_block(
     const float* logits, const IT* importance, const float* second_uniform,
     const GateParams& p, int32_t* idx, int32_t* pos, float* gate, uint8_t* kept,
-    float* part1, float* part2, float* smem) {
+    float* part1, float* part2, float* smem, int16_t* ch = nullptr) {
   constexpr int TOKENS = SELECT_THREADS / LANES;
   const int E = p.E, S = p.S;
   const int ld = select_row_floats(E);
@@ -829,6 +833,32 @@ __device__ __forceinline__ void gate_select_block(
   const float* src = logits + t * E;
   float* row = tile + tok * ld;
   const bool sw = p.router == ROUTER_SWITCH;
+  // the token's record (by one lane of a token that exists): choices, gates, the two
+  // `kept` bytes and what the loss counts
+  auto write_record = [&](int i1, int i2, float g1, float g2, unsigned k1,
+                          unsigned k2, int third) {
+    if constexpr (TAIL) {
+      st_dev(reinterpret_cast<unsigned long long*>(idx + t * 2), pack_i2(i1, i2));
+      st_dev(reinterpret_cast<unsigned long long*>(gate + t * 2), pack_f2(g1, g2));
+      st_dev(reinterpret_cast<uint16_t*>(kept + t * 2), (uint16_t)(k1 | k2 << 8));
+      ch[tok] = (k1 & 1) ? (int16_t)i1 : (int16_t)-1;
+      ch[TOKENS + tok] = (k2 & 1) ? (int16_t)i2 : (int16_t)-1;
+      ch[2 * TOKENS + tok] = (int16_t)third;
+    } else {
+      idx[t * 2 + 0] = i1;
+      idx[t * 2 + 1] = i2;
+      pos[t * 2 + 0] = 0;
+      pos[t * 2 + 1] = 0;
+      gate[t * 2 + 0] = g1;
+      gate[t * 2 + 1] = g2;
+      kept[t * 2 + 0] = (uint8_t)k1;
+      kept[t * 2 + 1] = (uint8_t)k2;
+    }
+  };
+  auto write_part = [&](float* at, float v) {
+    if constexpr (TAIL) st_dev(at, v);
+    else *at = v;
+  };
 
   float m = -INFINITY;
   for (int e = lane; e < e_end; e += LANES) m = fmaxf(m, src[e]);
@@ -896,14 +926,8 @@ __device__ __forceinline__ void gate_select_block(
       sel1 = (load_f32<IT>(importance + t) == 1.0f);
     if (!sel1) g1 = g1 * 0.0f;
     if (live && lane == 0) {
-      idx[t * 2 + 0] = i1;
-      idx[t * 2 + 1] = 0;
-      pos[t * 2 + 0] = 0;
-      pos[t * 2 + 1] = 0;
-      gate[t * 2 + 0] = g1;
-      gate[t * 2 + 1] = 0.0f;
-      kept[t * 2 + 0] = (sel1 ? 1 : 0) | 2;   // bit 1: counted by density_1
-      kept[t * 2 + 1] = 0;
+      // (bit 1: counted by density_1)
+      write_record(i1, 0, g1, 0.0f, (sel1 ? 1u : 0u) | 2u, 0u, i1);
       isone[tok] = 1.0f;
     }
   } else {
@@ -942,14 +966,8 @@ __device__ __forceinline__ void gate_select_block(
       } else if (p.policy == MESH_MOE_SECOND_RANDOM) {
         sel2 = sel2 && (second_uniform[t] < g2n * p.inv_threshold);
       }
-      idx[t * 2 + 0] = i1;
-      idx[t * 2 + 1] = i2;
-      pos[t * 2 + 0] = 0;
-      pos[t * 2 + 1] = 0;
-      gate[t * 2 + 0] = g1n;
-      gate[t * 2 + 1] = g2n;
-      kept[t * 2 + 0] = sel1 ? 1 : 0;
-      kept[t * 2 + 1] = (sel2 ? 1 : 0) | (sel2_loss ? 2 : 0);
+      write_record(i1, i2, g1n, g2n, sel1 ? 1u : 0u,
+                   (sel2 ? 1u : 0u) | (sel2_loss ? 2u : 0u), sel2_loss ? i2 : -1);
       isone[tok] = sel1 ? 1.0f : 0.0f;
     }
   }
@@ -974,7 +992,7 @@ __device__ __forceinline__ void gate_select_block(
     if (tid < E) {
       float a = 0.f;
       for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
-      part[((int64_t)g * p.nblk + blk) * E + tid] = a;
+      write_part(part + ((int64_t)g * p.nblk + blk) * E + tid, a);
     }
   };
   // density_1_proxy partial: sum over the block's tokens of p * (imp == 1)
@@ -992,7 +1010,7 @@ __device__ __forceinline__ void gate_select_block(
     if (tid < 2) {
       float a = 0.f;
       for (int r = 0; r < ntok; ++r) a += cols[tid * TOKENS + r];
-      part2[((int64_t)g * p.nblk + blk) * E + tid] = a;
+      write_part(part2 + ((int64_t)g * p.nblk + blk) * E + tid, a);
     }
   } else if (p.use_second_place_loss) {
     __syncthreads();
@@ -1141,9 +1159,40 @@ __device__ __forceinline__ void gate_rank_tile(
   }
 }
 
-// What the last block of group g does (all 256 threads; smem is the block's
-// whole dynamic LDS, free by now).  Same results, bit for bit, as
-// gate_capacity_kernel + gate_loss_kernel for slots in token order.
+// Ranks of the choices of a block of 64 tokens: gate_rank_tile with one wavefront per
+// choice.  ch [3][64] and cnt [3][E] in LDS; `live` tokens exist.
+__device__ __forceinline__ void gate_rank_block(
+    const int16_t* ch, int32_t* cnt, int E, bool loss2, int live, int64_t tok0,
+    int32_t* pos, int32_t* bcnt_blk) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < 3 * E; i += blockDim.x) cnt[i] = 0;
+  __syncthreads();
+  if (wave < 2 || (wave == 2 && loss2)) {
+    const int nbits = 32 - __builtin_clz((unsigned)max(E - 1, 1));
+    const int mine = lane < live ? ch[wave * 64 + lane] : -1;
+    // the lanes that name the same expert
+    unsigned long long match = __ballot(mine >= 0);
+    for (int b = 0; b < nbits; ++b) {
+      const bool bit = ((mine >> b) & 1) != 0;
+      const unsigned long long with = __ballot(bit);
+      match &= bit ? with : ~with;
+    }
+    const unsigned long long before = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const int rank = (int)__popcll(match & before);
+    if (mine >= 0 && rank == 0) cnt[wave * E + mine] = (int)__popcll(match);
+    if (wave < 2 && lane < live)
+      st_dev(pos + (tok0 + lane) * 2 + wave, mine >= 0 ? rank : 0);
+  }
+  __syncthreads();
+  for (int i = tid; i < 3 * E; i += blockDim.x) st_dev(bcnt_blk + i, cnt[i]);
+}
+
+// What the last block of group g does (all of its threads, 2 E at least; smem is the
+// block's whole dynamic LDS, free by now).  Same results, bit for bit, as
+// gate_capacity_kernel + gate_loss_kernel for slots in token order.  U: tokens per
+// thread and trip; PB: blocks whose sums are fetched together; the group's blocks are
+// 2^SHIFT tokens.
+template <int U, int PB, int SHIFT>
 __device__ __forceinline__ void gate_group_tail(
     unsigned char* smem, const GateParams& p, const FusedTail& ft, int g,
     const int32_t* __restrict__ idx, int32_t* __restrict__ pos,
@@ -1170,8 +1219,6 @@ __device__ __forceinline__ void gate_group_tail(
   // one round trip per dependent access: the loads of the three parts (token
   // records, partial sums of the loss, per-block counts) are issued together
   // before anything is used.
-  constexpr int U = 8;     // tokens per thread and trip
-  constexpr int PB = 16;   // blocks whose partial sums are fetched up front
   int2 ex[U], rk[U];
   float2 gt[U];
   uint16_t kk[U];
@@ -1197,15 +1244,15 @@ __device__ __forceinline__ void gate_group_tail(
   };
   // Loads return in the order they were issued: the per-block counts, which
   // the prefixes below need first, go out before the (many more) record loads.
-  auto load_counts = [&](int i, int (&cv)[PB]) {
+  auto load_counts = [&](int i, int b0, int (&cv)[PB]) {
     const int c = i / E, e = i - c * E;
 #pragma unroll
     for (int b = 0; b < PB; ++b)
-      cv[b] = (i < 3 * E && b < nblk && (c < 2 || loss2))
-                  ? ld_dev(bc + ((int64_t)b * 3 + c) * E + e) : 0;
+      cv[b] = (i < 3 * E && b0 + b < nblk && (c < 2 || loss2))
+                  ? ld_dev(bc + ((int64_t)(b0 + b) * 3 + c) * E + e) : 0;
   };
   int cv0[PB];
-  load_counts(tid, cv0);
+  load_counts(tid, 0, cv0);
   // thread e < E sums column e of part1, threads E .. 2E-1 column e of part2
   // (second-place loss: E columns; switch: columns 0 and 1), in block order
   const int pcol = tid < E ? tid : tid - E;
@@ -1224,25 +1271,22 @@ __device__ __forceinline__ void gate_group_tail(
     const int c = i / E, e = i - c * E;
     if (c == 2 && !loss2) { tot[i] = 0; continue; }
     uint16_t* pre = c == 0 ? pre1 : pre2;
-    int cv[PB];
-    if (i == tid) {
-#pragma unroll
-      for (int b = 0; b < PB; ++b) cv[b] = cv0[b];
-    } else {
-      load_counts(i, cv);
-    }
     int run = 0;
+    for (int b0 = 0; b0 < nblk; b0 += PB) {
+      int cv[PB];
+      if (i == tid && b0 == 0) {
 #pragma unroll
-    for (int b = 0; b < PB; ++b) {
-      if (b < nblk) {
-        if (c < 2) pre[b * E + e] = (uint16_t)run;
-        run += cv[b];
+        for (int b = 0; b < PB; ++b) cv[b] = cv0[b];
+      } else {
+        load_counts(i, b0, cv);
       }
-    }
-    for (int b = PB; b < nblk; ++b) {
-      const int v = ld_dev(bc + ((int64_t)b * 3 + c) * E + e);
-      if (c < 2) pre[b * E + e] = (uint16_t)run;
-      run += v;
+#pragma unroll
+      for (int b = 0; b < PB; ++b) {
+        if (b0 + b < nblk) {
+          if (c < 2) pre[(b0 + b) * E + e] = (uint16_t)run;
+          run += cv[b];
+        }
+      }
     }
     tot[i] = run;
   }
@@ -1251,7 +1295,14 @@ __device__ __forceinline__ void gate_group_tail(
 #pragma unroll
     for (int b = 0; b < PB; ++b)
       if (b < nblk) psum += pv[b];
-    for (int b = PB; b < nblk; ++b) psum += ld_dev(pcolumn + (int64_t)b * E);
+    for (int b0 = PB; b0 < nblk; b0 += PB) {
+#pragma unroll
+      for (int b = 0; b < PB; ++b)
+        pv[b] = b0 + b < nblk ? ld_dev(pcolumn + (int64_t)(b0 + b) * E) : 0.f;
+#pragma unroll
+      for (int b = 0; b < PB; ++b)
+        if (b0 + b < nblk) psum += pv[b];
+    }
   }
   __syncthreads();
   // Per-expert outputs and the group's share of the balancing loss come first:
@@ -1295,7 +1346,7 @@ __device__ __forceinline__ void gate_group_tail(
     for (int u = 0; u < U; ++u) {
       const int s = s0 + u * (int)blockDim.x;
       if (s >= S) continue;
-      const int blk = s >> 7;
+      const int blk = s >> SHIFT;
       uint16_t kout = 0;
       if (kk[u] & 1) {
         const int slot = pre1[blk * E + ex[u].x] + rk[u].x;
@@ -1510,7 +1561,7 @@ __global__ __launch_bounds__(256) void router_gate_kernel(
         arrive_is_last(ft.gctr + g, ft.call, (unsigned)p.nblk) ? 1 : 0;
   __syncthreads();
   if (!last_of_group) return;
-  gate_group_tail(rl_smem, p, ft, g, idx, pos, gate, kept, part1, part2);
+  gate_group_tail<8, 16, 7>(rl_smem, p, ft, g, idx, pos, gate, kept, part1, part2);
   (void)tokens_total;
 }
 
@@ -1863,6 +1914,47 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_small_groups_kernel(
                       loss, reinterpret_cast<int32_t*>(smem), blockIdx.y);
 }
 
+// Both steps and the loss from logits in memory, groups of any number of blocks of 64
+// tokens: every block ranks its own tokens, and the last one of a group finishes it as
+// in router_gate_kernel.  Apart, the three launches are a chain of round trips, and
+// step 2 counts the tokens of a whole group in one block.  2 x 1024 tokens, 8 experts
+// 15.5 -> 12.2 us, 6 x 1500, 16 experts 18.3 -> 16.2.
+template <typename IT>
+__global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
+    const float* __restrict__ logits, const IT* __restrict__ importance,
+    const float* __restrict__ second_uniform, GateParams p, int32_t* idx,
+    int32_t* pos, float* gate, uint8_t* kept, float* part1, float* part2,
+    FusedTail ft) {
+  constexpr int LANES = 16, TOKENS = SELECT_THREADS / LANES;
+  static_assert(TOKENS == 64, "gate_rank_block");
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  __shared__ int last_of_group;
+  const int g = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x;
+  if (tid == 0) {
+    // the first block of a group stamps the group's counter for this call
+    if (blk == 0) counter_prepare(ft.gctr + g, ft.call);
+    if (blk == 0 && g == 0) counter_prepare(ft.fctr, ft.call);
+  }
+  float* cols = smem + TOKENS * select_row_floats(p.E) + TOKENS;
+  int32_t* cnt = reinterpret_cast<int32_t*>(cols + SELECT_THREADS);   // [3][E]
+  int16_t* ch = reinterpret_cast<int16_t*>(cnt + 3 * p.E);            // [3][TOKENS]
+  gate_select_block<IT, LANES, true>(logits, importance, second_uniform, p, idx, pos,
+                                     gate, kept, part1, part2, smem, ch);
+  const bool loss2 = p.use_second_place_loss != 0 || p.router == ROUTER_SWITCH;
+  const int64_t tok0 = (int64_t)g * p.S + blk * TOKENS;
+  gate_rank_block(ch, cnt, p.E, loss2, min(TOKENS, p.S - blk * TOKENS), tok0, pos,
+                  ft.bcnt + ((int64_t)g * p.nblk + blk) * 3 * p.E);
+  wait_stores();
+  __syncthreads();
+  if (tid == 0)
+    last_of_group =
+        arrive_is_last(ft.gctr + g, ft.call, (unsigned)p.nblk) ? 1 : 0;
+  __syncthreads();
+  if (!last_of_group) return;
+  gate_group_tail<2, 16, 6>(reinterpret_cast<unsigned char*>(smem), p, ft, g, idx, pos,
+                            gate, kept, part1, part2);
+}
+
 __global__ void gate_loss_kernel(GateParams p, const float* __restrict__ gsum,
                                  float* __restrict__ loss) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -2100,6 +2192,14 @@ extern "C" size_t mesh_moe_gating_workspace_bytes(int G, int S, int E) {
          sizeof(unsigned long long) * ((size_t)G + 1) + 3 * 256;
 }
 
+// Number of a single-launch gating call: the arrival counters in the
+// workspace are read relative to it (see arrive_is_last).
+static unsigned long long next_call_number() {
+  static std::atomic<unsigned long long> counter{1};
+  unsigned long long n = counter.fetch_add(1, std::memory_order_relaxed);
+  return (n & ((1ull << 48) - 1)) | (1ull << 47);
+}
+
 // Gating from logits: step 1 (softmax / choices) then steps 2 and 3.
 static int run_gating(const GateParams& p, const float* logits,
                       const void* importance, int importance_dtype,
@@ -2123,12 +2223,51 @@ static int run_gating(const GateParams& p, const float* logits,
   };
   int el, ss;
   const size_t cap_smem = capacity_lds(p, el, ss);
-  // (with more groups than compute units the two kernels overlap better: 300 groups of
-  // 40 tokens, 16 experts 48.5 us apart and 49.2 in one, 1000 of 64, 128 experts 128 and
-  // 135; 64 of 64, 64 experts 18.5 and 17.5; one of 64 12.7 and 11.9)
-  const bool one_block = p.nblk == 1 && p.tt == 64 && G <= 128;
+  // A group of one block with nothing to wait for: one group (32 tokens, 32 experts
+  // 10.4 us, with the tail of gate_logits_kernel 10.8; 64 of 64 12.1 and 13.1), or slots
+  // by gate, which that kernel does not do, in up to 128 groups.
+  const bool one_block =
+      p.nblk == 1 && p.tt == 64 && (p.rank_by_gate ? G <= 128 : G == 1);
+  const size_t tail_smem = fused_tail_lds_bytes(p.nblk, E);
+  const size_t select_smem = smem + sizeof(int32_t) * 3 * (size_t)E +
+                             sizeof(int16_t) * 3 * 64;
+  // One launch, finished by the last block of every group, while its blocks (one per
+  // compute unit: 128 registers) are little more than one round of them, where groups
+  // are single blocks, and where they are so long that one block per group for all of
+  // step 2 is what takes the time.  Separate launches / one, us: 2 x 1024 tokens, 8
+  // experts 15.5 / 12.2; 16 x 1000, 64 experts 22.5 / 16.3; 8 x 2048, 128 experts 52.5 /
+  // 23.6; 48 x 333, 16 experts 20.8 / 17.7; 300 x 40 47 / 25; 16384 tokens 205 / 49; 6 x
+  // 8192 192 / 55.  On the other side 24 x 1000, 8 experts 18.7 / 19.3; 32 x 1000 20.4 /
+  // 33.6; 64 x 1000 30 / 46; 15 x 4096 40 / 52.  (In 64 registers, two blocks per
+  // compute unit: 64 x 1000 38.5, 2 x 1024 13.8.)
+  const int64_t all_blocks = (int64_t)G * p.nblk;
+  const bool one_launch =
+      p.tt == 64 && !p.rank_by_gate && !one_block && 2 * E <= SELECT_THREADS &&
+      tail_smem <= 60 * 1024 &&
+      (4 * all_blocks <= 5 * (int64_t)compute_units() || p.nblk == 1 || p.S >= 8192);
   auto run_lanes = [&](auto* imp) -> int {
     using IT = std::remove_const_t<std::remove_pointer_t<decltype(imp)>>;
+    if (one_launch) {
+      FusedTail ft;
+      uintptr_t at = ((uintptr_t)(gsum + (size_t)G * GSUM) + 255) & ~(uintptr_t)255;
+      ft.bcnt = (int32_t*)at;
+      at = (at + sizeof(int32_t) * 3 * (size_t)G * p.nblk * E + 255) & ~(uintptr_t)255;
+      ft.gctr = (unsigned long long*)at;
+      ft.fctr = ft.gctr + G;
+      ft.gsum = gsum;
+      ft.fill = fill;
+      ft.loss = loss;
+      ft.call = next_call_number();
+      auto k = gate_logits_kernel<IT>;
+      // (the last block of all stages the groups' terms of the loss)
+      const size_t terms = (size_t)G * GSUM <= 8192 ? sizeof(float) * G * GSUM : 0;
+      const size_t both = std::max(std::max(select_smem, tail_smem), terms);
+      MOE_ALLOW_LDS(k, both);
+      k<<<grid, SELECT_THREADS, both, st>>>(logits, imp, second_uniform, p, idx, pos,
+                                            gate, kept, part1, part2, ft);
+      MOE_CHECK_LAUNCH("gate_logits");
+      return 0;
+    }
     if (one_block) {
       auto k = gate_small_groups_kernel<IT, SELECT_THREADS / 64>;
       const size_t both = smem > cap_smem ? smem : cap_smem;
@@ -2148,17 +2287,9 @@ static int run_gating(const GateParams& p, const float* logits,
   const int rc = importance && importance_dtype == MESH_MOE_BF16
                      ? run_lanes((const bf16_t*)importance)
                      : run_lanes((const float*)importance);
-  if (rc != 0 || one_block) return rc;
+  if (rc != 0 || one_block || one_launch) return rc;
   return launch_capacity_and_loss(p, idx, pos, gate, kept, fill, loss, part1,
                                   part2, gsum, st);
-}
-
-// Number of a single-launch gating call: the arrival counters in the
-// workspace are read relative to it (see arrive_is_last).
-static unsigned long long next_call_number() {
-  static std::atomic<unsigned long long> counter{1};
-  unsigned long long n = counter.fetch_add(1, std::memory_order_relaxed);
-  return (n & ((1ull << 48) - 1)) | (1ull << 47);
 }
 
 // Shape limits of the fused projection + gating kernel.

@@ -163,6 +163,35 @@ def test_small_groups_gating(hip, router, s, e):
         assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
 
 
+# groups of one block of 64 tokens, of one and a token, of whole blocks, of more blocks
+# than are read together (16), the most experts
+@pytest.mark.parametrize("s,e", [(64, 16), (65, 5), (128, 64), (1000, 8), (1100, 33),
+                                 (130, 512)])
+@pytest.mark.parametrize("router", ["top2", "switch"])
+def test_gating_in_one_launch(hip, router, s, e):
+  """Few groups are gated by one launch, many by one per step: the same bits.  Twice,
+  since the launch's counters are left for the next call."""
+  gen = torch.Generator(device="cuda").manual_seed(s + e)
+  groups = 22000 // s if s > 64 else 400
+  logits = torch.randn((groups, s, e), generator=gen, device="cuda")
+  logits[0, s // 2] = 0.25                      # equal probabilities
+  importance = torch.randint(0, 3, (groups, s), generator=gen, device="cuda") / 2
+  capacity = max(1, s // 4)
+  for imp in (None, importance):
+    def gating(g):
+      some = None if imp is None else imp[:g].contiguous()
+      if router == "switch":
+        return hip.switch_gating(logits[:g].contiguous(), capacity, importance=some,
+                                 z_loss=0.01)
+      return hip.top2_gating(logits[:g].contiguous(), capacity, importance=some,
+                             policy="threshold", use_second_place_loss=True)
+    many = gating(groups)
+    for g in (1, 3, 3):
+      few = gating(g)
+      for name in ("idx", "pos", "gate", "kept", "fill"):
+        assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
+
+
 # a reduction of one K tile, of whole and of partly filled batches of tiles; tokens and
 # experts around the 32 of a wavefront; the row that the K tiles' rotation restarts at
 @pytest.mark.parametrize("tokens", [1, 31, 33, 200])
