@@ -529,6 +529,36 @@ def test_self_attention_relative_bias(hip, case, causal, act_dtype):
   assert np.abs(plain - got).max() > 1e-2
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("length", [8, 64, 72, 256, 264, 520])
+def test_key_and_value_gradients_of_one_launch(hip, length, causal):
+  """dk and dv of heads of 64 around the 64 queries of a tile and the 256 keys of a
+  block, against float64.  The bounds: one bf16 rounding of the result, one of every
+  weight W and dS in it (2^-9, doubled for the float32 sums in front of them), and
+  the rounding of the forward outputs in delta = dout . out."""
+  b, heads, d = 2, 3, 64
+  gen = torch.Generator(device="cuda").manual_seed(length)
+  q, k, v, do = (torch.randn((b, length, heads * d), generator=gen, device="cuda")
+                 .to(torch.bfloat16) for _ in range(4))
+  q = (q * 0.125).contiguous()
+  dk, dv = hip.self_attention_backward(q, k, v, do, heads, causal)[1:3]
+  split = lambda t: t.double().reshape(b, length, heads, d).transpose(1, 2)
+  qd, kd, vd, dod = (split(t).contiguous() for t in (q, k, v, do))
+  t = lambda x: x.transpose(2, 3).contiguous()
+  logits = qd @ t(kd)
+  if causal:
+    logits = logits.masked_fill(torch.ones((length, length), device="cuda").triu(1)
+                                .bool(), float("-inf"))
+  w = logits.softmax(-1)
+  out = w @ vd
+  ds = w * (dod @ t(vd) - (dod * out).sum(-1, keepdim=True))
+  ds_error = 2.0 ** -8 * (ds.abs() + w * (dod.abs() * out.abs()).sum(-1, keepdim=True))
+  for got, want, error in (
+      (dv, t(w) @ dod, 2.0 ** -8 * (t(w) @ dod.abs())),
+      (dk, t(ds) @ qd, t(ds_error) @ qd.abs())):
+    assert bool(((split(got) - want).abs() <= 2.0 ** -8 * want.abs() + error).all())
+
+
 def test_self_attention_rejections(hip):
   q = torch.zeros((1, 12, 16), dtype=torch.bfloat16, device="cuda")
   with pytest.raises(hip.MoeHipError, match="not divisible"):
