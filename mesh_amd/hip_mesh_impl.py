@@ -220,15 +220,17 @@ class HipMeshImpl(mtf.MeshImpl):
     (mesh_tensorflow/placement_mesh_impl.py:159-178)."""
     laid_out = self.LaidOutTensor
     args = []
-    for x in mtf.convert_args_to_laid_out_tensors(inputs):
+    for x in inputs:
+      if not isinstance(x, laid_out) and hasattr(x, "to_laid_out_tensor"):
+        x = x.to_laid_out_tensor()
       args.append(x.tensor_list[0] if isinstance(x, laid_out) else x)
-    if torch.cuda.current_device() == self._device_index:
+    if moe_hip.current_device() == self._device_index:
       ret = fn(*args)
     else:
       with torch.cuda.device(self._device):
         ret = fn(*args)
     if isinstance(ret, tuple):
-      return tuple(laid_out([t]) for t in ret)
+      return tuple([laid_out([t]) for t in ret])
     return laid_out([ret])
 
   def einsum(self, equation, *slices):
@@ -266,7 +268,10 @@ class HipMeshImpl(mtf.MeshImpl):
     return x
 
   def import_tf_tensor(self, x, tf_x):
-    t = torch.as_tensor(tf_x).to(device=self._device, dtype=x.dtype)
+    t = tf_x
+    if not (isinstance(t, torch.Tensor) and t.device == self._device and
+            t.dtype == x.dtype):
+      t = torch.as_tensor(t).to(device=self._device, dtype=x.dtype)
     return self.LaidOutTensor([t.contiguous()])
 
   def export_to_tf_tensor(self, x, laid_out_x):

@@ -300,14 +300,17 @@ def dtype_code(dtype):
   raise MoeHipError("unsupported dtype %s (float32 and bfloat16 only)" % dtype)
 
 
+_Tensor = torch.Tensor   # (a global less to look up in every check)
+
+
 def _dev(t, name, dtype=None, shape=None):
-  if not isinstance(t, torch.Tensor) or not t.is_cuda:
+  if not isinstance(t, _Tensor) or not t.is_cuda:
     raise MoeHipError("%s must be a GPU tensor" % name)
   if not t.is_contiguous():
     raise MoeHipError("%s must be contiguous" % name)
-  if dtype is not None and t.dtype != dtype:
+  if dtype is not None and t.dtype is not dtype:
     raise MoeHipError("%s: dtype %s, expected %s" % (name, t.dtype, dtype))
-  if shape is not None and t.shape != tuple(shape):
+  if shape is not None and t.shape != shape and t.shape != tuple(shape):
     raise MoeHipError("%s: shape %s, expected %s"
                       % (name, tuple(t.shape), tuple(shape)))
   return t.data_ptr()
@@ -318,10 +321,15 @@ def _dev(t, name, dtype=None, shape=None):
 _current_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
+# torch.cuda.current_device() without its check that the GPU is in use already (where
+# this is called it is: 0.13 instead of 0.24 us).
+current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def _stream():
   if _current_raw_stream is None:
     return torch.cuda.current_stream().cuda_stream
-  return _current_raw_stream(torch.cuda.current_device())
+  return _current_raw_stream(current_device())
 
 
 class StageTimer(object):

@@ -731,8 +731,8 @@ class Lowering(object):
     if correct_shape is None:
       correct_shape = self.mesh_impl(tensor).slice_shape(tensor.shape)
       self._slice_shapes[tensor] = correct_shape
-    actual_shape = list(laid_out_tensor.slice_shape)
-    if actual_shape != correct_shape:
+    actual_shape = laid_out_tensor.slice_shape
+    if actual_shape != correct_shape and list(actual_shape) != correct_shape:
       raise ValueError(
           "Wrong slice shape: correct_shape = %s actual shape = %s"
           % (correct_shape, actual_shape))
@@ -966,16 +966,16 @@ class ReshapeOperation(Operation):
       raise ValueError("Cannot reshape Tensor %s to shape %s - sizes differ."
                        % (x, new_shape))
     self._outputs = [Tensor(self, new_shape, x.dtype)]
+    self._sizes = tuple(new_shape.to_integer_list)
 
   def gradient(self, grad_ys):
     return [reshape(grad_ys[0], self.inputs[0].shape)]
 
   def lower(self, lowering):
     mesh_impl = lowering.mesh_impl(self)
-    new_shape = self.outputs[0].shape
     if mesh_impl.size != 1:
       raise NotImplementedError("reshape across a split mesh dimension")
-    sizes = new_shape.to_integer_list
+    sizes = self._sizes
     lowering.set_tensor_lowering(
         self.outputs[0],
         mesh_impl.slicewise(lambda t: t.reshape(sizes),

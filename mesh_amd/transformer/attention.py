@@ -384,18 +384,27 @@ class AttentionDecodeOperation(mtf.Operation):
     s_sizes = self.outputs[1].shape.to_integer_list
     channels, memory = q_sizes[-1], s_sizes[-2]
     heads = self._num_heads
+    flat = len(q_sizes) == 2
 
     bidirectional = self._rel_bidirectional
 
     def fn(q, k, v, old_k, old_v, position, *extra):
-      q2, k2, v2 = (t.reshape(-1, channels).contiguous() for t in (q, k, v))
-      kc, vc = (t.reshape(-1, memory, channels).contiguous()
-                for t in (old_k, old_v))
-      pos = position.reshape(-1).to(torch.int32).contiguous()
+      if flat:
+        # (one batch dimension: the tensors are what the library takes)
+        q2, k2, v2 = q.contiguous(), k.contiguous(), v.contiguous()
+        kc, vc = old_k.contiguous(), old_v.contiguous()
+        pos = position.to(torch.int32).contiguous()
+      else:
+        q2, k2, v2 = (t.reshape(-1, channels).contiguous() for t in (q, k, v))
+        kc, vc = (t.reshape(-1, memory, channels).contiguous()
+                  for t in (old_k, old_v))
+        pos = position.reshape(-1).to(torch.int32).contiguous()
       _, rel = _attention_extras(extra, None, 3 if extra else None, memory,
                                  bidirectional, q.dtype)
       out, new_k, new_v = moe_hip.attention_decode_states(
           q2, k2, v2, kc, vc, pos, heads, relative_bias=rel)
+      if flat:
+        return out, new_k, new_v
       return (out.reshape(q_sizes), new_k.reshape(s_sizes),
               new_v.reshape(s_sizes))
     outs = mesh_impl.slicewise(fn, *[lowering.tensors[t] for t in self.inputs])
