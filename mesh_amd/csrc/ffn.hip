@@ -1127,12 +1127,11 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // now, back to back: 16384 rows, 1024 -> 4096 126 -> 118 us, -> 1024 34.4 -> 31.3;
   // 16 x 705 rows, 768 -> 3072 62 -> 53; 64 x 512 rows, 1024 -> 4096 270 -> 260; weight
   // gradients of 64 x 512 rows 312 -> 293.  Without stores and staging the same
-  // launches take 103, 26.6, 46, 229 and 229: what is left is work, not waiting (a
-  // compute unit's 128 KB take 4.7 us when the whole chip stores, 2.7 if they stay in
-  // the L2s).  Twelve of the sixteen stores held back for the next three K tiles are no
-  // faster.  Turned round in registers (v_permlane32_swap, v_permlane16_swap) instead
-  // of LDS a store covers rows of 64 bytes, which cost the L2 1.4 times as long: weight
-  // gradients 293 -> 309.
+  // launches take 103, 26.6, 46, 229 and 229.  (A compute unit's 128 KB take 4.7 us when
+  // the whole chip stores, 2.7 if they stay in the L2s.)  Twelve of the sixteen stores
+  // held back for the next three K tiles are no faster.  Turned round in registers
+  // (v_permlane32_swap, v_permlane16_swap) instead of LDS a store covers rows of 64
+  // bytes, which cost the L2 1.4 times as long: weight gradients 293 -> 309.
   const uint32_t lds_base = (uint32_t)(size_t)(lds_void_t*)smem_raw;
   // The fragments of a tile's first step: read right behind the hand-over, or (TAILS:
   // the wavefront's pieces in the next tile are another copy of the code) ahead of
