@@ -2244,6 +2244,7 @@ static int run_gating(const GateParams& p, const float* logits,
   const bool one_launch =
       p.tt == 64 && !p.rank_by_gate && !one_block && 2 * E <= SELECT_THREADS &&
       tail_smem <= 60 * 1024 &&
+      G * GSUM <= 8192 &&      // (more groups' terms the last block reads one by one)
       (4 * all_blocks <= 5 * (int64_t)compute_units() || p.nblk == 1 || p.S >= 8192);
   auto run_lanes = [&](auto* imp) -> int {
     using IT = std::remove_const_t<std::remove_pointer_t<decltype(imp)>>;
@@ -2260,7 +2261,7 @@ static int run_gating(const GateParams& p, const float* logits,
       ft.call = next_call_number();
       auto k = gate_logits_kernel<IT>;
       // (the last block of all stages the groups' terms of the loss)
-      const size_t terms = (size_t)G * GSUM <= 8192 ? sizeof(float) * G * GSUM : 0;
+      const size_t terms = sizeof(float) * G * GSUM;
       const size_t both = std::max(std::max(select_smem, tail_smem), terms);
       MOE_ALLOW_LDS(k, both);
       k<<<grid, SELECT_THREADS, both, st>>>(logits, imp, second_uniform, p, idx, pos,

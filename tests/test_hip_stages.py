@@ -172,7 +172,7 @@ def test_gating_in_one_launch(hip, router, s, e):
   """Few groups are gated by one launch, many by one per step: the same bits.  Twice,
   since the launch's counters are left for the next call."""
   gen = torch.Generator(device="cuda").manual_seed(s + e)
-  groups = 22000 // s if s > 64 else 400
+  groups = 22000 // s if s > 64 else 2100       # (more than 2048 single blocks)
   logits = torch.randn((groups, s, e), generator=gen, device="cuda")
   logits[0, s // 2] = 0.25                      # equal probabilities
   importance = torch.randint(0, 3, (groups, s), generator=gen, device="cuda") / 2
