@@ -37,8 +37,8 @@
 // after the other, neither of the two wavefronts that a SIMD holds kept the matrix
 // pipe busy while the other one was at its softmax: busy 28 % of the time, vector
 // units 41 %.)  8 x 2048 positions, 8 heads of 128, causal 115 -> 99 us, without the
-// mask 166 -> 150; 2 x 4096, 16 heads of 64 102 -> 89; 16 packed rows of 1000, 12
-// heads of 64 58 -> 55.5.  What is left is the sum of both units' work (VALU 45 %,
+// mask 166 -> 150; 2 x 4096, 16 heads of 64 102 -> 89; with a relative bias 8 x 2048,
+// 16 heads of 64, causal 130 -> 125.  What is left is the sum of both units' work (VALU 45 %,
 // MFMA 46 %) at 1.9 GHz of shader clock.
 //
 // K and V tiles reach a two-stage LDS ring through global_load_lds_dwordx4, K a tile
@@ -348,11 +348,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
   float m_run = NEG;      // running maximum of this lane's query
   float l_part = 0.f;     // sum over this half-wave's keys
 
+  // Is a tile's softmax laid beside the next tile's logits?  Not for heads of 64 with
+  // ids and a bias, which do not fit into the registers of three wavefronts: up to 24 of
+  // them are spilled, and loads from there wait for the tiles that are on their way.
+  // Beside / one after the other, 16 packed rows of 1000, 12 heads, causal 53 / 47 us,
+  // not causal 89 / 75; 2 x 4096, 16 heads, not causal 69 / 58 (beside, in the registers
+  // of two wavefronts: 54, 87 and 67).  Heads of 128 with both have the registers (8 x
+  // 2048, 8 heads, not causal 84 / 87).
+  constexpr bool BESIDE = !(D == 64 && SEQ && BIAS);
   const int qw_first = q0 + wave * 32;
   const int kt_count = n_ktiles - kt_begin;
   load_k(kt_begin, 0);
   load_v(kt_begin, 0);
-  if (kt_count > 1) load_k(kt_begin + 1, 1);
+  if (BESIDE && kt_count > 1) load_k(kt_begin + 1, 1);
   __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
   __syncthreads();
 
@@ -386,18 +394,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     kf[j % (AHEAD + 1)] = *reinterpret_cast<const fa_bf16x8_t*>(
         fa_smem + k_at[j >> 1] + slot * Cfg::K_BYTES + (j & 1) * 32 * Cfg::K_ROW);
   };
-  auto start_logits = [&](int slot, fa_f32x16_t (&acc_s)[2]) {
-    if constexpr (BIAS) {
-      // key kl + c of the tile against query 32 wave + l32 of the block
-      const float* bw = bias_s + slot * 192 + (Cfg::BQ - 1 - wave * 32 - l32);
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            acc_s[sub][4 * r4 + c] = bw[sub * 32 + 8 * r4 + 4 * half + c];
-    }
+  auto start_logits = [&](int slot) {
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) read_k(slot, j);
   };
@@ -406,8 +403,27 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     const fa_f32x16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
                               0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     acc_s[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-        kf[j % (AHEAD + 1)], qf[j >> 1], !BIAS && j < 2 ? zero : acc_s[j & 1], 0, 0,
-        0);
+        kf[j % (AHEAD + 1)], qf[j >> 1], j < 2 ? zero : acc_s[j & 1], 0, 0, 0);
+  };
+  // (behind the products, as the backward kernels do it: the logits are then the
+  // same bits in both, and the sums of D products round at their own magnitude and
+  // not at the bias's, D / 16 times.  As the sums' first value the bias would cost
+  // 2 to 5 us less: 8 x 2048, 16 heads of 64, causal 119 us instead of 125.)
+  auto add_bias = [&](int slot, fa_f32x16_t (&acc_s)[2]) {
+    if constexpr (BIAS) {
+      // key kl + c of the tile against query 32 wave + l32 of the block
+      const float* bw = bias_s + slot * 192 + (Cfg::BQ - 1 - wave * 32 - l32);
+      fence();
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) {
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            acc_s[sub][4 * r4 + c] += bw[sub * 32 + 8 * r4 + 4 * half + c];
+        fence();
+      }
+    }
   };
   // diagonal and last tiles, and those that hold other sequences: behind a branch
   // that the tiles in between do not take
@@ -443,9 +459,17 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
                             (!SEQ || kid[c] == my_sid);
             if (!ok) acc_s[sub][4 * r4 + c] = NEG;
           }
+          fence();
         }
       }
     }
+  };
+  auto logits_of = [&](int kt, int slot, fa_f32x16_t (&acc_s)[2]) {
+    start_logits(slot);
+#pragma unroll
+    for (int j = 0; j < SM; ++j) logits_mfma(slot, j, acc_s);
+    add_bias(slot, acc_s);
+    mask_logits(kt, slot, acc_s);
   };
   // part i of 4 of the maximum of a tile's 32 logits
   auto part_of_max = [&](int i, float mx, fa_f32x16_t (&acc_s)[2]) {
@@ -475,16 +499,30 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     }
   };
 
+  auto max_of = [&](fa_f32x16_t (&acc_s)[2]) {
+    float mx = NEG;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = part_of_max(i, mx, acc_s);
+    return mx;
+  };
+
   // Tile `it`: its weights, beside the MFMAs of the next tile's logits, then its
-  // share of the outputs, beside the next tile's maximum.
+  // share of the outputs, beside the next tile's maximum.  (BESIDE; otherwise its
+  // logits and their maximum first, and nothing of the next tile but its loads.)
   auto tile = [&](int it, auto slot_c, auto last_c, fa_f32x16_t (&acc_s)[2],
                   fa_f32x16_t (&acc_n)[2]) {
     constexpr int SLOT = decltype(slot_c)::value, OTHER = SLOT ^ 1;
     constexpr bool LAST = decltype(last_c)::value;
     const int kt = kt_begin + it;
+    constexpr bool NEXT = BESIDE && !LAST;
     if constexpr (!LAST) {
       load_v(kt + 1, OTHER);
-      if (it + 2 < kt_count) load_k(kt + 2, SLOT);
+      if constexpr (!BESIDE) load_k(kt + 1, OTHER);
+      else if (it + 2 < kt_count) load_k(kt + 2, SLOT);
+    }
+    if constexpr (!BESIDE) {
+      logits_of(kt, SLOT, acc_s);
+      move_max(max_of(acc_s));
     }
     // (no visible key so far: the maximum is still the sentinel, and sentinel *
     // log2e - sentinel * log2e would leave the product's rounding error, ~1e22, as
@@ -501,8 +539,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
       // branch around the mask)
       asm volatile("" : "+v"(w[i]), "+v"(psum));
     };
-    if constexpr (!LAST) {
-      start_logits(OTHER, acc_n);
+    if constexpr (NEXT) {
+      start_logits(OTHER);
       fence();
 #pragma unroll
       for (int j = 0; j < SM; ++j) {
@@ -522,7 +560,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
       fa_u32x4_t packed = {w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]};
       pf[u] = __builtin_bit_cast(fa_bf16x8_t, packed);
     }
-    if constexpr (!LAST) mask_logits(kt + 1, OTHER, acc_n);
+    if constexpr (NEXT) {
+      add_bias(OTHER, acc_n);
+      mask_logits(kt + 1, OTHER, acc_n);
+    }
     // O^T += V^T . P
     fa_i16x4_t vlo[2][4], vhi[2][4];
     auto read_v = [&](int dt, int to) {
@@ -553,34 +594,28 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
                                                  3, 4, 5, 6, 7));
         acc_o[dt] =
             __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[u], acc_o[dt], 0, 0, 0);
-        if constexpr (!LAST) {
+        if constexpr (NEXT) {
           if (u < 4 / Cfg::DT) mx = part_of_max(dt * (4 / Cfg::DT) + u, mx, acc_n);
         }
       }
       fence();
     }
+    if constexpr (NEXT) move_max(mx);
     if constexpr (!LAST) {
-      move_max(mx);
       // the loads have landed and everybody is done with this tile
       __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
       __syncthreads();
     }
   };
   fa_f32x16_t acc_a[2], acc_b[2];
-  start_logits(0, acc_a);
-#pragma unroll
-  for (int j = 0; j < SM; ++j) logits_mfma(0, j, acc_a);
-  mask_logits(kt_begin, 0, acc_a);
-  {
-    float mx = NEG;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mx = part_of_max(i, mx, acc_a);
-    move_max(mx);
-  }
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
-  // K tile 0's slot is loaded again at once: everybody is done with it
-  __syncthreads();
+  if constexpr (BESIDE) {
+    logits_of(kt_begin, 0, acc_a);
+    move_max(max_of(acc_a));
+    // K tile 0's slot is loaded again at once: everybody is done with it
+    __syncthreads();
+  }
   int it = 0;
   for (; it + 2 < kt_count; it += 2) {
     tile(it, S0(), std::false_type(), acc_a, acc_b);

@@ -358,6 +358,78 @@ def test_fused_attention_tile_counts(hip, case, causal, with_bias):
                    <= ulp * (magnitude + value.abs())).all())
 
 
+@pytest.mark.parametrize("with_ids", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+def test_relative_bias_is_added_to_the_whole_logit(hip, d, causal, with_ids):
+  """Every 16 products of half of the keys add up to 2^-4, and the bias is 2^20, whose
+  last bit is 2^-3: the logits d / 16 * 2^-4 + 2^20 are exact if the bias is added to
+  the sum of all products, and 2^20 or too much if the sums start from it.  The weights
+  are ratios of exp(d / 16 * 2^-4) and 1; v is 1 for those keys and 0 for the others.
+  The bound: a weight and the result are rounded to bf16."""
+  b, l, heads, nb = 2, 200, 2, 8
+  first = (torch.arange(d, device="cuda") % 16 == 5).to(torch.bfloat16) / 4
+  odd = (torch.arange(l, device="cuda") % 3 == 1).to(torch.bfloat16)
+  q = first.repeat(b, l, heads).contiguous()
+  k = (odd[:, None] * first.repeat(heads)[None, :]).repeat(b, 1, 1).contiguous()
+  v = odd[:, None].repeat(b, 1, heads * d).contiguous()
+  bucket = B.relative_position_bucket(np.arange(-(l - 1), l), not causal, nb)
+  rel = (torch.full((heads, nb), 2.0 ** 20, device="cuda", dtype=torch.bfloat16),
+         torch.from_numpy(bucket.astype(np.int32)).cuda())
+  at = torch.arange(l, device="cuda")
+  ids = at // 70 if with_ids else torch.zeros_like(at)
+  sees = ids[:, None] == ids[None, :]
+  if causal:
+    sees = sees & (at[None, :] <= at[:, None])
+  weight = torch.exp(odd.double() * (d / 256.0))[None, :] * sees
+  want = (weight * odd.double()).sum(1) / weight.sum(1)
+  out = hip.self_attention(
+      q, k, v, heads, causal, relative_bias=rel,
+      sequence_id=ids.to(torch.int32).repeat(b, 1).contiguous() if with_ids else None)
+  assert bool(((out.double() - want[None, :, None]).abs()
+               <= 2.0 ** -7 * want[None, :, None]).all())
+
+
+@pytest.mark.parametrize("magnitude", [1.0, 16.0, 50.0])
+@pytest.mark.parametrize("d", [64, 128])
+def test_fused_attention_with_large_biases(hip, d, magnitude):
+  """Biases far larger than q . k; the logarithms of the denominators, the outputs and
+  dv against float64.  The bounds: a logit, its product with log2(e) and the maximum's
+  are rounded once each at their own magnitude, 2^-24 of it, and so is the sum with the
+  maximum; the rest as in test_fused_attention_tile_counts, and weights below the
+  smallest normal number (a key whose bias is 100 below another's) may come out 0."""
+  b, l, heads, nb = 2, 264, 3, 8
+  gen = torch.Generator(device="cuda").manual_seed(int(magnitude) + d)
+  q, k, v, do = (torch.randn((b, l, heads * d), generator=gen, device="cuda")
+                 .to(torch.bfloat16) for _ in range(4))
+  q = q * d ** -0.5
+  values = (torch.rand((heads, nb), generator=gen, device="cuda") * 2 - 1) * magnitude
+  bucket = B.relative_position_bucket(np.arange(-(l - 1), l), False, nb)
+  rel = (values.to(torch.bfloat16), torch.from_numpy(bucket.astype(np.int32)).cuda())
+  four = lambda t: t.double().reshape(b, l, heads, d).transpose(1, 2).contiguous()
+  q4, k4, v4, do4 = (four(t) for t in (q, k, v, do))
+  at = torch.arange(l, device="cuda")
+  logits = (q4 @ k4.transpose(2, 3).contiguous() +
+            rel[0].double()[:, rel[1].long()[at[None, :] - at[:, None] + l - 1]])
+  largest = float(logits.abs().max())
+  logits = logits.masked_fill(at[None, :] > at[:, None], float("-inf"))
+  out, lse = hip.self_attention(q, k, v, heads, True, relative_bias=rel,
+                                return_lse=True)
+  want = torch.logsumexp(logits, -1)
+  assert bool(((lse.double().reshape(b, heads, l) - want).abs()
+               <= 4 * 2.0 ** -24 * largest + 2e-6).all())
+  w = torch.softmax(logits, -1)
+  ulp = 2.0 ** -8
+  assert bool(((four(out) - w @ v4).abs()
+               <= ulp * (w @ v4.abs() + (w @ v4).abs())).all())
+  dv = hip.self_attention_backward(q, k, v, do, heads, True, fused=True,
+                                   relative_bias=rel, out=out, lse=lse)[2]
+  wt = w.transpose(2, 3).contiguous()
+  assert bool(((four(dv) - wt @ do4).abs()
+               <= ulp * (wt @ do4.abs() + (wt @ do4).abs()) +
+               2.0 ** -126 * do4.abs().sum(2, keepdim=True)).all())
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_attention_at_the_block_benchmark_shape(hip, causal):
   """The fused attention kernels at the (batch, head) shape of the benchmark
