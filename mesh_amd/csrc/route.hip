@@ -1191,8 +1191,11 @@ __device__ __forceinline__ void gate_rank_block(
 // block's whole dynamic LDS, free by now).  Same results, bit for bit, as
 // gate_capacity_kernel + gate_loss_kernel for slots in token order.  U: tokens per
 // thread and trip; PB: blocks whose sums are fetched together; the group's blocks are
-// 2^SHIFT tokens.
-template <int U, int PB, int SHIFT>
+// 2^SHIFT tokens.  LONG: so are those of every further PB blocks.  (Without: one by
+// one.  The loop over batches takes 44 registers in router_gate_kernel, whose groups
+// seldom have more than 16 blocks of 128 tokens: 174 instead of 130 registers, two
+// wavefronts per SIMD instead of three.)
+template <int U, int PB, int SHIFT, bool LONG>
 __device__ __forceinline__ void gate_group_tail(
     unsigned char* smem, const GateParams& p, const FusedTail& ft, int g,
     const int32_t* __restrict__ idx, int32_t* __restrict__ pos,
@@ -1271,21 +1274,37 @@ __device__ __forceinline__ void gate_group_tail(
     const int c = i / E, e = i - c * E;
     if (c == 2 && !loss2) { tot[i] = 0; continue; }
     uint16_t* pre = c == 0 ? pre1 : pre2;
+    int cv[PB];
+    if (i == tid) {
+#pragma unroll
+      for (int b = 0; b < PB; ++b) cv[b] = cv0[b];
+    } else {
+      load_counts(i, 0, cv);
+    }
     int run = 0;
-    for (int b0 = 0; b0 < nblk; b0 += PB) {
-      int cv[PB];
-      if (i == tid && b0 == 0) {
 #pragma unroll
-        for (int b = 0; b < PB; ++b) cv[b] = cv0[b];
-      } else {
-        load_counts(i, b0, cv);
+    for (int b = 0; b < PB; ++b) {
+      if (b < nblk) {
+        if (c < 2) pre[b * E + e] = (uint16_t)run;
+        run += cv[b];
       }
+    }
+    if constexpr (LONG) {
+      for (int b0 = PB; b0 < nblk; b0 += PB) {
+        load_counts(i, b0, cv);
 #pragma unroll
-      for (int b = 0; b < PB; ++b) {
-        if (b0 + b < nblk) {
-          if (c < 2) pre[(b0 + b) * E + e] = (uint16_t)run;
-          run += cv[b];
+        for (int b = 0; b < PB; ++b) {
+          if (b0 + b < nblk) {
+            if (c < 2) pre[(b0 + b) * E + e] = (uint16_t)run;
+            run += cv[b];
+          }
         }
+      }
+    } else {
+      for (int b = PB; b < nblk; ++b) {
+        const int v = ld_dev(bc + ((int64_t)b * 3 + c) * E + e);
+        if (c < 2) pre[b * E + e] = (uint16_t)run;
+        run += v;
       }
     }
     tot[i] = run;
@@ -1295,13 +1314,17 @@ __device__ __forceinline__ void gate_group_tail(
 #pragma unroll
     for (int b = 0; b < PB; ++b)
       if (b < nblk) psum += pv[b];
-    for (int b0 = PB; b0 < nblk; b0 += PB) {
+    if constexpr (LONG) {
+      for (int b0 = PB; b0 < nblk; b0 += PB) {
 #pragma unroll
-      for (int b = 0; b < PB; ++b)
-        pv[b] = b0 + b < nblk ? ld_dev(pcolumn + (int64_t)(b0 + b) * E) : 0.f;
+        for (int b = 0; b < PB; ++b)
+          pv[b] = b0 + b < nblk ? ld_dev(pcolumn + (int64_t)(b0 + b) * E) : 0.f;
 #pragma unroll
-      for (int b = 0; b < PB; ++b)
-        if (b0 + b < nblk) psum += pv[b];
+        for (int b = 0; b < PB; ++b)
+          if (b0 + b < nblk) psum += pv[b];
+      }
+    } else {
+      for (int b = PB; b < nblk; ++b) psum += ld_dev(pcolumn + (int64_t)b * E);
     }
   }
   __syncthreads();
@@ -1561,7 +1584,7 @@ __global__ __launch_bounds__(256) void router_gate_kernel(
         arrive_is_last(ft.gctr + g, ft.call, (unsigned)p.nblk) ? 1 : 0;
   __syncthreads();
   if (!last_of_group) return;
-  gate_group_tail<8, 16, 7>(rl_smem, p, ft, g, idx, pos, gate, kept, part1, part2);
+  gate_group_tail<8, 16, 7, false>(rl_smem, p, ft, g, idx, pos, gate, kept, part1, part2);
   (void)tokens_total;
 }
 
@@ -1951,8 +1974,8 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
         arrive_is_last(ft.gctr + g, ft.call, (unsigned)p.nblk) ? 1 : 0;
   __syncthreads();
   if (!last_of_group) return;
-  gate_group_tail<2, 16, 6>(reinterpret_cast<unsigned char*>(smem), p, ft, g, idx, pos,
-                            gate, kept, part1, part2);
+  gate_group_tail<2, 16, 6, true>(reinterpret_cast<unsigned char*>(smem), p, ft, g, idx,
+                                  pos, gate, kept, part1, part2);
 }
 
 __global__ void gate_loss_kernel(GateParams p, const float* __restrict__ gsum,
