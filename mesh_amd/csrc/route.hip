@@ -1065,16 +1065,27 @@ struct FusedTail {
   unsigned long long call;    // number of this call, < 2^48, never 0
 };
 
-// Puts a counter word into this call's state "no arrivals yet" if it holds
-// zero, which is what the last arrival of the previous use leaves behind.
-// Nobody waits for the result: a word that held something else (a workspace
-// used for the first time) is handled by the arrivals themselves.
-__device__ __forceinline__ void counter_prepare(unsigned long long* word,
-                                                unsigned long long call) {
-  unsigned long long zero = 0ull;
-  (void)__hip_atomic_compare_exchange_strong(
-      word, &zero, call << 16, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-      __HIP_MEMORY_SCOPE_AGENT);
+// Puts a counter word into this call's state "no arrivals yet", whatever it holds: zero
+// where the last arrival of a call left it, anything where the workspace's memory has
+// served something else since (between two passes of a training step it has).  One
+// thread of a block that arrives at the word itself; it hands the returned word to
+// counter_settle once its work is done (nobody waits for it before) and arrives behind
+// that.
+__device__ __forceinline__ unsigned long long counter_prepare(
+    unsigned long long* word, unsigned long long call) {
+  return __hip_atomic_exchange(word, call << 16, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Puts back the arrivals that came before counter_prepare.  Until then the word counts
+// too few, so no arrival takes itself for the last one, and this block's own arrival is
+// still to come.
+__device__ __forceinline__ void counter_settle(unsigned long long* word,
+                                               unsigned long long call,
+                                               unsigned long long prepared) {
+  if ((prepared >> 16) == call)
+    (void)__hip_atomic_fetch_add(word, prepared & 0xffffu, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // true for the last of `expected` arrivals; one thread per arrival.  The
@@ -1442,10 +1453,11 @@ __global__ __launch_bounds__(256) void router_gate_kernel(
   __shared__ int last_of_group;
   const int E = p.E;
   const int64_t tok0 = (int64_t)blockIdx.x * TOK;       // first token, flat
+  unsigned long long gctr_was = 0, fctr_was = 0;
   if (ft.bcnt != nullptr && threadIdx.x == 0) {
     // the first block of a group stamps the group's counter for this call
-    if (tok0 % p.S == 0) counter_prepare(ft.gctr + tok0 / p.S, ft.call);
-    if (blockIdx.x == 0) counter_prepare(ft.fctr, ft.call);
+    if (tok0 % p.S == 0) gctr_was = counter_prepare(ft.gctr + tok0 / p.S, ft.call);
+    if (blockIdx.x == 0) fctr_was = counter_prepare(ft.fctr, ft.call);
   }
   const int b = (int)(tok0 / tokens_per_batch);         // router weight set
   const bf16_t* xb = x + tok0 * M;
@@ -1577,6 +1589,10 @@ __global__ __launch_bounds__(256) void router_gate_kernel(
   // stores, see st_dev): once every wavefront's stores have completed, one
   // thread arrives at the group's counter; the last block to arrive finishes
   // the group.
+  if (threadIdx.x == 0) {
+    if (tok0 % p.S == 0) counter_settle(ft.gctr + g, ft.call, gctr_was);
+    if (blockIdx.x == 0) counter_settle(ft.fctr, ft.call, fctr_was);
+  }
   wait_stores();
   __syncthreads();
   if (tid == 0)
@@ -1940,8 +1956,10 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_small_groups_kernel(
 // Both steps and the loss from logits in memory, groups of any number of blocks of 64
 // tokens: every block ranks its own tokens, and the last one of a group finishes it as
 // in router_gate_kernel.  Apart, the three launches are a chain of round trips, and
-// step 2 counts the tokens of a whole group in one block.  2 x 1024 tokens, 8 experts
-// 15.5 -> 12.2 us, 6 x 1500, 16 experts 18.3 -> 16.2.
+// step 2 counts the tokens of a whole group in one block.  Kernel times apart / in one,
+// whatever the workspace held: 2 x 1024 tokens, 8 experts 6.5 + 11.3 + 2.5 / 13.7 us, 6 x
+// 1500, 16 experts 7.1 + 14 + 3.3 / 17.6.  (With counters that the arrivals themselves had
+// to put into this call's state, two more round trips: 16.5 and 24.5.)
 template <typename IT>
 __global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
     const float* __restrict__ logits, const IT* __restrict__ importance,
@@ -1953,10 +1971,11 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
   extern __shared__ __attribute__((aligned(16))) float smem[];
   __shared__ int last_of_group;
   const int g = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x;
+  // the first block of a group stamps the group's counter for this call
+  unsigned long long gctr_was = 0, fctr_was = 0;
   if (tid == 0) {
-    // the first block of a group stamps the group's counter for this call
-    if (blk == 0) counter_prepare(ft.gctr + g, ft.call);
-    if (blk == 0 && g == 0) counter_prepare(ft.fctr, ft.call);
+    if (blk == 0) gctr_was = counter_prepare(ft.gctr + g, ft.call);
+    if (blk == 0 && g == 0) fctr_was = counter_prepare(ft.fctr, ft.call);
   }
   float* cols = smem + TOKENS * select_row_floats(p.E) + TOKENS;
   int32_t* cnt = reinterpret_cast<int32_t*>(cols + SELECT_THREADS);   // [3][E]
@@ -1967,6 +1986,10 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
   const int64_t tok0 = (int64_t)g * p.S + blk * TOKENS;
   gate_rank_block(ch, cnt, p.E, loss2, min(TOKENS, p.S - blk * TOKENS), tok0, pos,
                   ft.bcnt + ((int64_t)g * p.nblk + blk) * 3 * p.E);
+  if (tid == 0) {
+    if (blk == 0) counter_settle(ft.gctr + g, ft.call, gctr_was);
+    if (blk == 0 && g == 0) counter_settle(ft.fctr, ft.call, fctr_was);
+  }
   wait_stores();
   __syncthreads();
   if (tid == 0)
@@ -2248,7 +2271,10 @@ static int run_gating(const GateParams& p, const float* logits,
   const size_t cap_smem = capacity_lds(p, el, ss);
   // A group of one block with nothing to wait for: one group (32 tokens, 32 experts
   // 10.4 us, with the tail of gate_logits_kernel 10.8; 64 of 64 12.1 and 13.1), or slots
-  // by gate, which that kernel does not do, in up to 128 groups.
+  // by gate, which that kernel does not do, in up to 128 groups.  (Two to 128 groups:
+  // kernel times with this kernel and the loss's / in one launch 2 x 64 tokens, 16
+  // experts 16.9 / 12.4 us, 32 x 40, 64 experts 20.6 / 16.8, 128 x 64, 128 experts 35.5 /
+  // 24.6.)
   const bool one_block =
       p.nblk == 1 && p.tt == 64 && (p.rank_by_gate ? G <= 128 : G == 1);
   const size_t tail_smem = fused_tail_lds_bytes(p.nblk, E);

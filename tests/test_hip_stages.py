@@ -192,6 +192,47 @@ def test_gating_in_one_launch(hip, router, s, e):
         assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
 
 
+@pytest.mark.parametrize("s,e", [(64, 16), (256, 8), (1024, 32), (8192, 4)])
+def test_gating_with_any_workspace(hip, monkeypatch, s, e):
+  """The launches that finish a group in its last block count arrivals in a workspace
+  that may hold anything: zeros, ones, what another call left.  One group and several,
+  from logits and beside the projection: the same bits."""
+  gen = torch.Generator(device="cuda").manual_seed(s + e)
+  m, capacity = 64, max(1, s // 4)
+  x = torch.randn((1, 3 * s, m), generator=gen, device="cuda").bfloat16()
+  w = hip.pack_weights(torch.randn((1, m, e), generator=gen, device="cuda").bfloat16(),
+                       torch.bfloat16)
+  logits = torch.randn((3, s, e), generator=gen, device="cuda")
+  plain, workspaces = torch.empty, []
+
+  def empty(*size, **kw):
+    t = plain(*size, **kw)
+    if kw.get("dtype") == torch.uint8 and t.dim() == 1:
+      if isinstance(held, int):
+        t.fill_(held)
+      else:
+        n = min(t.numel(), held.numel())
+        t[:n] = held[:n]
+      workspaces.append(t)
+    return t
+  monkeypatch.setattr(torch, "empty", empty)
+
+  def calls(g):
+    yield hip.top2_gating(logits[:g].contiguous(), capacity, policy="threshold",
+                          use_second_place_loss=True)
+    yield hip.switch_gating(logits[:g].contiguous(), capacity, z_loss=0.01)
+    if s % 128 == 0:
+      yield hip.router_top2_gating(x[:, :g * s].contiguous(), w, s, capacity)
+  for g in (1, 3):
+    held = 0
+    want = list(calls(g))
+    left = workspaces[-1].clone()
+    for held in (255, 1, 0x5a, left):
+      for got, right in zip(calls(g), want):
+        for name in ("idx", "pos", "gate", "kept", "fill", "loss"):
+          assert torch.equal(getattr(got, name), getattr(right, name)), name
+
+
 # a reduction of one K tile, of whole and of partly filled batches of tiles; tokens and
 # experts around the 32 of a wavefront; the row that the K tiles' rotation restarts at
 @pytest.mark.parametrize("tokens", [1, 31, 33, 200])
