@@ -240,6 +240,46 @@ def test_compact_backward_matches_oracle(hip, case):
                                err_msg=k)
 
 
+@pytest.mark.parametrize("m,hdim", [(704, 768), (320, 1024), (768, 2048)])
+def test_compact_weight_gradients_of_lower_row_tiles(hip, m, hdim):
+  """Weight gradients whose output rows are cut into tiles of 160 and 192, of experts
+  with no row, with one, and with counts around the K tiles of 64 (with their next tile's
+  loads in flight, a block goes from an expert of many rows to one of none and back).
+  Rows that nobody writes are NaN.  The bounds: one bf16 rounding of each result and of
+  dh, and an ulp for each of the products in a float32 sum."""
+  g, c, e, n = 2, 256, 16, 256
+  counts = torch.tensor([[0, 1, 63, 64, 0, 65, 128, 200, 256, 256, 0, 0, 129, 7, 192, 0],
+                         [0, 0, 0, 0, 256, 0, 1, 56, 0, 256, 1, 0, 127, 250, 63, 130]],
+                        dtype=torch.int32, device="cuda")
+  gen = torch.Generator(device="cuda").manual_seed(m + hdim)
+  r = hip.switch_gating(torch.randn((g, c, e), generator=gen, device="cuda"), c)
+  r.fill.copy_(counts)
+  row_offsets = (counts.t().cumsum(1) - counts.t()).to(torch.int32).contiguous()
+  def rand(*shape, scale=1.0):
+    return (torch.randn(shape, generator=gen, device="cuda") * scale).bfloat16()
+  xe, h, dy = rand(e, g * c, m), rand(e, g * c, hdim), rand(e, g * c, n)
+  wi, wo = rand(e, m, hdim, scale=m ** -0.5), rand(e, hdim, n, scale=n ** -0.5)
+  used = counts.sum(0).tolist()
+  for i in range(e):
+    for t in (xe, h, dy):
+      t[i, used[i]:-(-used[i] // 256) * 256] = 0
+      t[i, -(-used[i] // 256) * 256:] = float("nan")
+  _, dwi, dwo = hip.compact_expert_ffn_backward(xe, h, dy, wi, wo, r, row_offsets,
+                                                "relu")
+  for i in range(e):
+    x1, h1, dy1 = (t[i, :used[i]].double() for t in (xe, h, dy))
+    wt = wo[i].double().t().contiguous()
+    dh = (dy1 @ wt) * (h1 > 0)
+    dh_error = 2.0 ** -8 * dh.abs() + n * 2.0 ** -24 * (dy1.abs() @ wt.abs())
+    for got, lhs, rhs, error in ((dwi[i], x1, dh, dh_error),
+                                 (dwo[i], h1, dy1, torch.zeros_like(dy1))):
+      lhs = lhs.t().contiguous()
+      want = lhs @ rhs
+      bound = (2.0 ** -8 * want.abs() + lhs.abs() @ error +
+               used[i] * 2.0 ** -24 * (lhs.abs() @ rhs.abs()))
+      assert bool(((got.double() - want).abs() <= bound).all()), used[i]
+
+
 def test_compact_gradient_calls_edge_fills(hip):
   """Row counts per expert chosen by hand: none (its kernels' gradients are
   exactly zero), one, a whole 256-row tile, every row, and counts that end

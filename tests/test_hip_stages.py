@@ -142,37 +142,10 @@ def test_router_logits_edges(hip, shape, dtype):
 @pytest.mark.parametrize("router", ["top2", "switch"])
 def test_small_groups_gating(hip, router, s, e):
   """Groups of at most 64 tokens are gated by one launch where they are few: the bits
-  of the launch per step that many groups take."""
+  of the launch per step that many groups take (more than 2048; slots by gate: more
+  than 128)."""
   gen = torch.Generator(device="cuda").manual_seed(s + e)
-  logits = torch.randn((200, s, e), generator=gen, device="cuda")
-  logits[0, s // 2] = 0.25                      # equal probabilities
-  importance = torch.randint(0, 3, (200, s), generator=gen, device="cuda") / 2
-  capacity = max(1, s // 4)
-  for imp in (None, importance):
-    def gating(g):
-      some = None if imp is None else imp[:g].contiguous()
-      if router == "switch":
-        return hip.switch_gating(logits[:g].contiguous(), capacity, importance=some,
-                                 z_loss=0.01, slots_by_gate=e % 2 == 0)
-      return hip.top2_gating(logits[:g].contiguous(), capacity, importance=some,
-                             policy="threshold", use_second_place_loss=True)
-    many = gating(200)
-    for g in (1, 2, 128):
-      few = gating(g)
-      for name in ("idx", "pos", "gate", "kept", "fill"):
-        assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
-
-
-# groups of one block of 64 tokens, of one and a token, of whole blocks, of more blocks
-# than are read together (16), the most experts
-@pytest.mark.parametrize("s,e", [(64, 16), (65, 5), (128, 64), (1000, 8), (1100, 33),
-                                 (130, 512)])
-@pytest.mark.parametrize("router", ["top2", "switch"])
-def test_gating_in_one_launch(hip, router, s, e):
-  """Few groups are gated by one launch, many by one per step: the same bits.  Twice,
-  since the launch's counters are left for the next call."""
-  gen = torch.Generator(device="cuda").manual_seed(s + e)
-  groups = 22000 // s if s > 64 else 2100       # (more than 2048 single blocks)
+  groups = 2100
   logits = torch.randn((groups, s, e), generator=gen, device="cuda")
   logits[0, s // 2] = 0.25                      # equal probabilities
   importance = torch.randint(0, 3, (groups, s), generator=gen, device="cuda") / 2
@@ -182,14 +155,97 @@ def test_gating_in_one_launch(hip, router, s, e):
       some = None if imp is None else imp[:g].contiguous()
       if router == "switch":
         return hip.switch_gating(logits[:g].contiguous(), capacity, importance=some,
-                                 z_loss=0.01)
+                                 z_loss=0.01, slots_by_gate=e % 2 == 0)
       return hip.top2_gating(logits[:g].contiguous(), capacity, importance=some,
                              policy="threshold", use_second_place_loss=True)
     many = gating(groups)
-    for g in (1, 3, 3):
+    for g in (1, 2, 128):
       few = gating(g)
       for name in ("idx", "pos", "gate", "kept", "fill"):
         assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
+
+
+def _gating(hip, router, logits, importance, capacity):
+  if router == "switch":
+    return hip.switch_gating(logits, capacity, importance=importance, z_loss=0.01)
+  return hip.top2_gating(logits, capacity, importance=importance, policy="threshold",
+                         use_second_place_loss=True)
+
+
+# groups of one block of 64 tokens, of one and a token, of whole blocks, of more blocks
+# than are read together (16), the most experts; groups that are one launch however
+# many blocks they have, with an expert that most tokens choose
+@pytest.mark.parametrize("s,e", [(64, 16), (65, 5), (128, 64), (1000, 8), (1100, 33),
+                                 (130, 512), (8192, 16), (16384, 4)])
+@pytest.mark.parametrize("router", ["top2", "switch"])
+def test_gating_in_one_launch(hip, router, s, e):
+  """Few groups are gated by one launch, many by one per step: the same bits.  Twice,
+  since the launch's counters are left for the next call.  The many are the few over
+  and over, whose loss is the same mean: but for a rounding per group, and (both sides,
+  which may cut a group into blocks of 64 and of 128 tokens) per block and per token of
+  a block."""
+  gen = torch.Generator(device="cuda").manual_seed(s + e)
+  nblk = (s + 63) // 64
+  cus = torch.cuda.get_device_properties(0).multi_processor_count
+  # more than 2048 single blocks; tokens from which a block is 128 of them; else more
+  # than 5 / 4 blocks per compute unit
+  least = (2049 if nblk == 1 else -(-65536 // s) if s >= 8192 else
+           (5 * cus // 4) // nblk + 1)
+  copies = -(-least // 3)
+  few_logits = torch.randn((3, s, e), generator=gen, device="cuda")
+  few_logits[0, s // 2] = 0.25                  # equal probabilities
+  if s >= 8192:
+    few_logits[..., 0] += 2.5
+  few_importance = torch.randint(0, 3, (3, s), generator=gen, device="cuda") / 2
+  capacity = max(1, s // 4)
+  rel = 2 * (3 * copies + nblk + 128) * 2.0 ** -24
+  for with_importance in (False, True):
+    def gating(logits, importance):
+      return _gating(hip, router, logits, importance if with_importance else None,
+                     capacity)
+    many = gating(few_logits.repeat(copies, 1, 1), few_importance.repeat(copies, 1))
+    for g in (1, 3, 3):
+      few = gating(few_logits[:g].contiguous(), few_importance[:g].contiguous())
+      for name in ("idx", "pos", "gate", "kept", "fill"):
+        assert torch.equal(getattr(few, name), getattr(many, name)[:g]), name
+      if g == 3:
+        assert abs(float(few.loss) - float(many.loss)) <= rel * abs(float(many.loss))
+
+
+@pytest.mark.parametrize("router", ["top2", "switch"])
+def test_gating_loss_of_one_launch(hip, router):
+  """The loss of the launch that finishes groups in their last blocks, of 1, 16, 17 and
+  18 blocks (16 are added at a time), against the oracle's."""
+  for g, s, e in ((3, 50, 8), (2, 1024, 8), (2, 1025, 16), (3, 1100, 33)):
+    rng = np.random.default_rng(s + e)
+    logits = H.safe_logits(rng, g, s, e)
+    importance = (rng.integers(0, 3, (g, s)) / 2).astype(np.float32)
+    capacity = max(1, s // 4)
+    got = _gating(hip, router, torch.from_numpy(logits).cuda(),
+                  torch.from_numpy(importance).cuda(), capacity)
+    if router == "switch":
+      want = O.switch_gating(logits, capacity, importance=importance, train=True,
+                             z_loss=0.01, num_microbatches=1)
+    else:
+      want = O.top_2_gating(logits, capacity, importance=importance,
+                            policy="threshold", use_second_place_loss=True)
+    np.testing.assert_allclose(H.routing_to_np(got)["loss"], want["loss"], rtol=2e-5)
+
+
+@pytest.mark.parametrize("router", ["top2", "switch"])
+def test_gating_of_2048_groups(hip, router):
+  """2048 groups of one block are the most that one launch gates; 2049 take the launch
+  per step.  Every group is the same, so the loss is one group's, but for a rounding per
+  group."""
+  gen = torch.Generator(device="cuda").manual_seed(5)
+  logits = torch.randn((1, 40, 8), generator=gen, device="cuda").repeat(2049, 1, 1)
+  got = {g: _gating(hip, router, logits[:g].contiguous(), None, 10)
+         for g in (2, 2048, 2049)}
+  for g in (2, 2048):
+    for name in ("idx", "pos", "gate", "kept", "fill"):
+      assert torch.equal(getattr(got[g], name), getattr(got[2049], name)[:g]), name
+    want = float(got[2049].loss)
+    assert abs(float(got[g].loss) - want) <= 2 * 2049 * 2.0 ** -24 * abs(want)
 
 
 @pytest.mark.parametrize("s,e", [(64, 16), (256, 8), (1024, 32), (8192, 4)])
@@ -1329,6 +1385,35 @@ def test_dispatched_expert_ffn_equals_two_calls(hip, shape):
   if g * c == 256:
     r2 = hip.top2_gating(torch.from_numpy(logits).cuda(), c + 32)
     assert hip.dispatched_expert_ffn(x, r2, wi_p, wo_p, "relu") is None
+
+
+@pytest.mark.parametrize("m", [64, 128, 192, 320])
+@pytest.mark.parametrize("g,c", [(5, 80), (7, 91)])
+def test_dispatched_expert_ffn_tile_after_tile(hip, g, c, m):
+  """Rows fetched through the slot map by blocks that go from tile to tile (1024 of
+  them), whose map entries they ask for a tile ahead: row tiles of fewer than 256 rows,
+  the last one partly empty; reductions of one to five K tiles.  The second product's
+  weights are the identity, so that the result is the hidden tensor.  The bits of the
+  two calls, and against float64: one bf16 rounding, and K / 2 ulps of the sum of
+  magnitudes for the float32 sum of K products."""
+  s, e, h = 2048, 64, 2048
+  gen = torch.Generator(device="cuda").manual_seed(g + c + m)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  r = hip.top2_gating(mk(g, s, e), c)
+  assert int((r.fill < c).sum()) > 0                   # some empty slots
+  x = mk(g, s, m).to(torch.bfloat16)
+  wi = mk(e, h, m).to(torch.bfloat16)
+  wo = torch.eye(h, device="cuda", dtype=torch.bfloat16).repeat(e, 1, 1)
+  got = hip.dispatched_expert_ffn(x, r, wi, wo, "relu")
+  assert got is not None
+  xe = hip.dispatch(x, r).reshape(e, g * c, m)
+  assert torch.equal(got, hip.expert_ffn(xe, wi, wo, "relu"))
+  for i in range(0, e, 7):
+    t = wi[i].double().t().contiguous()
+    want = (xe[i].double() @ t).clamp(min=0)
+    magnitude = xe[i].double().abs() @ t.abs()
+    bound = 2.0 ** -8 * want + m * 2.0 ** -25 * magnitude
+    assert bool(((got[i].double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("case", [
