@@ -2706,6 +2706,7 @@ extern "C" int mesh_moe_compact_expert_ffn(
                   (int64_t)G * S <= 0x7fffffffLL &&
                   ring_path_applies((int)rows, H, M) &&
                   ring_path_applies((int)rows, N, H) &&
+                  rows * H < (1LL << 31) &&    // h's offsets within an expert
                   (((uintptr_t)x | (uintptr_t)wi_packed | (uintptr_t)wo_packed |
                     (uintptr_t)h | (uintptr_t)y) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,

@@ -357,6 +357,25 @@ def test_library_exports_every_declared_symbol():
   assert lib.mesh_moe_gating_workspace_bytes(32, 2048, 64) > 0
 
 
+def test_compact_experts_decline_a_hidden_tensor_beyond_32_bits():
+  """The second product on compacted rows reads the hidden tensor with 32-bit offsets
+  within an expert: 262144 rows of 8192 columns are declined, before anything is
+  launched (the callers then take the calls for all slots).  With 64 columns less it is
+  only the workspace's size that fails."""
+  if torch.cuda.is_available():
+    pytest.skip("pointers that are none")
+  lib = moe_hip.load_library()
+  g, s, e, c, m, n = 64, 4096, 1, 4096, 256, 256
+  p = 1 << 20
+
+  def call(h):
+    return lib.mesh_moe_compact_expert_ffn(
+        p, p, p, p, p, p, p, p, p, p, p, None, 1.0, None, p, 0, g, s, e, c, m, h, n,
+        moe_hip.ACTIVATIONS["relu"], moe_hip.BF16, None)
+  assert call(8192) == moe_hip.E_UNSUPPORTED
+  assert call(8192 - 64) not in (0, moe_hip.E_UNSUPPORTED)
+
+
 def test_product_does_not_import_the_oracle():
   pkg = os.path.join(ROOT, "mesh_amd")
   for dirpath, _, files in os.walk(pkg):
