@@ -375,15 +375,6 @@ __device__ __forceinline__ void lds_read_lines(u32x4_t (&p)[4], uint32_t at) {
                : "memory");
 }
 
-// Block barrier that publishes LDS writes and waits for nothing else: vector
-// memory loads and stores of this wavefront stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 __device__ __forceinline__ int lds_swizzle(int row) {
   return (row & 7) ^ ((row >> 3) & 1);
 }
@@ -1120,7 +1111,6 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // afterwards.  By then K tile 0 of the next tile has been on its way for a whole K
   // tile, so the matrix pipes go on with it at once, and the stores have that
   // much time before anything waits for them.
-  //
   //
   // A tile's output used to be staged by all wavefronts in two passes behind block
   // barriers, with the ring drained and nothing multiplied, 6.5 us a tile.  Before and
@@ -2009,27 +1999,32 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 // The persistent blocks take whole rounds of tiles, so what counts is rounds
 // times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
 // 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
-// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside
-// (measured with the output staged behind the K loop; that it now runs beside
-// it changes none of the choices below)
-// the K loop.  Rows are spread evenly over the row tiles: 640 rows per expert are
-// three tiles of 224 or four of 160, not 256 + 256 + 128.  Measured, tiles of
-// 256 and a shorter last one -> the rule's choice (both sides bit-identical):
-//   32 x 640 rows, 4096 x 1024 (384 tiles -> 512 of 160 rows)   203 -> 166 us
-//   16 x 705 rows, 768 x 3072 / 3072 x 768 (192 rows)       73 / 67 -> 60 / 55
-//   8 x 900 rows, 1536 x 4608 (192 rows)                        117 -> 100
-//   64 x 320 rows, 1024 x 4096 (160 rows; 128-row kernel before) 268 -> 207
-//   5000 rows, 1280 x 1280 (128 rows, 200 tiles instead of 100)  31 -> 25
-//   128 x 400 rows, 2048 x 8192 (224 rows)                     1729 -> 1680
+// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside the K
+// loop.  Rows are spread evenly over the row tiles: 640 rows per expert are three tiles
+// of 224 or four of 160, not 256 + 256 + 128.  (The terms are from when a tile's output
+// was staged behind its K loop; it now runs beside it, and a tile costs less outside.
+// What that moves is within 5 %: of 15 products timed with every height since, K 64 to
+// 4096, the rule's choice was the fastest or within 2 % of it in 13; 16 x 256 rows, 4096
+// x 1024 took 50.5 us with its 64 rows and 48.3 with 128, 48 x 180 rows, 768 x 1536 36.5
+// with its 192 and 35.3 with 96.)  Tiles of 256 and a shorter last one -> the rule's
+// choice (both sides bit-identical):
+//   32 x 640 rows, 4096 x 1024 (160 rows; of 224 188 us)             -> 171 us
+//   16 x 705 rows, 768 x 3072 (192 rows) / 3072 x 768 (160)  61 / 54 -> 50 / 50
+//   8 x 900 rows, 1536 x 4608 (192 rows)                        110 -> 91
+//   64 x 320 rows, 1024 x 4096 (160 rows; of 128 235 us)             -> 197
+//   16 x 705 rows, 512 x 768 (160 rows)                        15.0 -> 13.1
+//   5000 rows, 1280 x 1280 (128 rows)                          26.9 -> 21.7
 // K-major operands (weight gradients; R is then a width, K the rows summed over):
 // 0.48 + 0.12 per piece us per K tile, 3.3 + 0.75 per piece outside the K loop, whose
-// share is larger there (reductions of few K tiles; from 16 x 704 and 1280 rows):
-//   16 x 704 rows, 768 x 3072 / 3072 x 768 (192 rows)   76 / 75 -> 62.5 / 65
-//   16 x 1280 rows, 768 x 3072 (192 rows)                   115 -> 95
-//   24 x 512 rows, 512 x 1536 (192 rows)                    36.7 -> 31.9
-//   12 x 1000 rows, 1280 x 2560 (224 rows)                  94.6 -> 85
+// share is larger there (reductions of few K tiles; from 16 x 704 and 1280 rows, and
+// the same remark: in 12 timed since, 64 to 1280 rows, the rule's choice was the fastest
+// or within 2 % of it):
+//   16 x 704 rows, 768 x 3072 / 3072 x 768 (192 rows)       65 / 63 -> 51.5 / 52
+//   16 x 1280 rows, 768 x 3072 (192 rows)                       105 -> 85
+//   24 x 512 rows, 512 x 1536 (192 rows)                       32.5 -> 27.2
+//   12 x 1000 rows, 1280 x 2560 (224 rows)                     85.1 -> 76.9
 // and the rule stays with 256 where that is the fastest (64 x 512 rows, 1024 x 4096
-// 316, 224 rows 328; 8 x 640 rows, 1024 x 4096 48, 192 rows 55).
+// 287, 224 rows 301; 8 x 640 rows, 1024 x 4096 41.4, 192 rows 45).
 static int ring_tile_rows(int E, int R, int N, int K, int cus,
                           bool kmajor = false) {
   const int tiles_n = (N + RingCfg::BN - 1) / RingCfg::BN;
@@ -2183,16 +2178,18 @@ static bool ring_shape(int R, int N, int K) {
   return N >= 256 && R >= 128 && K % 64 == 0 && N % 8 == 0 &&
          (int64_t)N * K < (1LL << 31);
 }
-// Products for which the 128 x 128 tiles are faster than the ring's 256 columns
+// Products for which the 128 x 128 tiles are no slower than the ring's 256 columns
 // (same bits):
-// short reductions in at most two blocks per compute unit (the ring's first loads,
-// its hand-over and its epilogue through LDS take longer than the K loop: 30
-// experts, 384 x 512, K = 64: 7.0 against 8.7 us; 320 x 2048, K = 128: 5.6, 6.9;
-// from three blocks on the ring wins: 30 x 640 x 512, K = 128: 12.1, 10.6), and
-// one row tile per expert in a few blocks per compute unit, where a ring tile of
-// 128 rows has no second row tile to share its weights with (64 experts, 128 x
-// 1024: K = 256 14.8 against 17.2 us, K = 1024 33.9, 38.5; 256 experts, 128 x 512,
-// K = 512 38.5, 42.9; 64 experts, 128 x 4096, K = 1024 148, 137).
+// short reductions in at most two blocks per compute unit (the ring's first loads and
+// the output of its last tile, which has no next one beside it, take longer than the K
+// loop: 16 experts, 512 x 1024, K = 64 8.2 against 9.9 us; 30 experts, 384 x 512, K = 64
+// 8.0, 8.3; from three blocks on the ring wins: 30 x 640 x 512, K = 128 11.2, 8.7), and
+// one row tile per expert in a few blocks per compute unit, where a ring tile of 128
+// rows has no second row tile to share its weights with.  (There the lines were drawn
+// when a ring tile's output was staged behind its K loop, 64 experts, 128 x 1024: K = 256
+// 14.8 against 17.2 us, K = 1024 33.9, 38.5; the ring is now as fast or a little faster
+// on this side of them: 11.7, 10.9; 26.6, 26.1; 256 experts, 128 x 512, K = 512 32.7,
+// 31.7.)
 static bool small_tiles_apply(int E, int R, int N, int K) {
   const int64_t tiles =
       (int64_t)E * ((R + 127) / 128) * ((N + 127) / 128);
