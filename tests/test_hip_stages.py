@@ -289,6 +289,42 @@ def test_gating_with_any_workspace(hip, monkeypatch, s, e):
           assert torch.equal(getattr(got, name), getattr(right, name)), name
 
 
+def test_recorded_gating_with_any_workspace(hip):
+  """A recorded launch carries one call number into every replay, and its workspace is
+  written over between two of them (all of the recorded step's memory that is not an
+  output)."""
+  gen = torch.Generator(device="cuda").manual_seed(3)
+  g, s, e, c = 3, 1024, 8, 300
+  logits = torch.randn((g, s, e), generator=gen, device="cuda")
+  workspaces, plain = [], torch.empty
+
+  def empty(*size, **kw):
+    t = plain(*size, **kw)
+    if kw.get("dtype") == torch.uint8 and t.dim() == 1:
+      workspaces.append(t)
+    return t
+  want = hip.top2_gating(logits, c)               # (also loads what a launch needs)
+  torch.cuda.synchronize()
+  graph = torch.cuda.CUDAGraph()
+  torch.empty = empty
+  try:
+    with torch.cuda.graph(graph):
+      got = hip.top2_gating(logits, c)
+  finally:
+    torch.empty = plain
+  assert len(workspaces) == 1
+  for held in (0, 255, 1, None, 0x5a):
+    if held is not None:
+      workspaces[0].fill_(held)
+    for t in (got.idx, got.pos, got.gate, got.kept, got.fill, got.loss):
+      t.zero_()
+    graph.replay()
+    eager = hip.top2_gating(logits, c)
+    for name in ("idx", "pos", "gate", "kept", "fill", "loss"):
+      assert torch.equal(getattr(got, name), getattr(want, name)), (held, name)
+      assert torch.equal(getattr(eager, name), getattr(want, name)), (held, name)
+
+
 # a reduction of one K tile, of whole and of partly filled batches of tiles; tokens and
 # experts around the 32 of a wavefront; the row that the K tiles' rotation restarts at
 @pytest.mark.parametrize("tokens", [1, 31, 33, 200])
