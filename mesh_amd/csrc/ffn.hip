@@ -576,6 +576,9 @@ struct RingCfg {
   static constexpr size_t LOOP_BYTES = (size_t)A_SLOTS * A_BYTES + (size_t)B_SLOTS * B_BYTES;
   static constexpr size_t LDS_BYTES = LOOP_BYTES;  // the output is staged inside
   static_assert(A_INSTR == 4 && B_INSTR == 4, "load schedule assumes 4 + 4");
+  // row tiles of at most DEEP_ROWS rows: three slots for the token tile too
+  static constexpr int DEEP_ROWS = 160, DEEP_A_BYTES = DEEP_ROWS * ROW_BYTES;
+  static_assert(3 * DEEP_A_BYTES + B_SLOTS * B_BYTES <= LDS_BYTES, "three slots");
 };
 
 // Position of tile `rem` of an expert where its row tiles are many: 32
@@ -646,6 +649,17 @@ __device__ __forceinline__ void ring_tile_blocks(int rem, int tiles_m,
 // experts' last row tiles after all full ones separates the row tiles that
 // share a weight panel: with 400 rows per expert the weights were then read
 // twice from memory and the launches took 14 % longer.)
+//
+// DEEP (TAILS with row tiles of at most 160 rows): three token slots of 160 rows
+// instead of two of 256, and all seven loads of K tile t + 2 in steps 0 to 2 of K tile
+// t.  A low tile's MFMAs take half a microsecond a K tile, less than a load takes from
+// memory; with two slots the token loads wait for the hand-over that frees theirs and
+// are due at the next one.  (Loads alone, without the products: 32 x 640 rows, 4096 ->
+// 1024 159 of 168 us.)  Back to back, two slots / three, the same bits: 32 x 640 rows,
+// 4096 -> 1024 170 / 154 us; 64 x 320, 1024 -> 4096 197 / 183; 16 x 256, 4096 -> 1024
+// 52 / 41.5; 5000 rows, 1280 -> 1280 21.7 / 20.5; 16 x 708, 3072 -> 768 52.3 / 50.0.
+// (Weights ahead of the tokens, or the last load behind the hand-over: 1 to 3 % slower;
+// all loads in the first two steps: no change, as for the weights of the higher tiles.)
 // 512 bytes that stay zero (nothing writes them): where a K-major tile reaches
 // past the last reduction row, its rows are loaded from here, and so is the second
 // K tile of a reduction that has one
@@ -657,7 +671,7 @@ static __device__ __attribute__((aligned(256))) bf16_t ring_zero_row[256];
 
 template <bool RELU, bool GATHER = false, bool KMAJOR = false,
           bool MASKED = false, bool LISTED = false, bool TAILS = false,
-          bool SPLIT = false>
+          bool SPLIT = false, bool DEEP = false>
 __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
     bf16_t* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
@@ -673,6 +687,11 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // per expert (k_extent)
   const int32_t* k_extent = KMAJOR ? row_count : nullptr;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, WN = Cfg::WN;
+  static_assert(!DEEP || (TAILS && !KMAJOR && !LISTED && !SPLIT), "low row tiles");
+  constexpr int A_BYTES = DEEP ? Cfg::DEEP_A_BYTES : Cfg::A_BYTES;
+  constexpr int A_SLOTS = DEEP ? 3 : Cfg::A_SLOTS;
+  // loads of a token tile per wavefront (DEEP: the third is half a one)
+  constexpr int A_LOADS = DEEP ? 3 : Cfg::A_INSTR;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
 
   // PERSISTENT blocks: one per CU, each walks a strided list of tiles, whose K tiles
@@ -731,7 +750,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   //   a_lane, b_lane   KMAJOR: elements to this lane's chunk in the pair of rows;
   //              else b_lane: bytes to its chunk in the eight rows
   //   b_row[j]   not KMAJOR: elements to the first of the eight rows
-  uint32_t a_row[Cfg::A_INSTR], a_lane = 0, b_lane = 0;
+  uint32_t a_row[A_LOADS], a_lane = 0, b_lane = 0;
   int b_row[Cfg::B_INSTR];
   int kt0 = 0;           // SPLIT: its first K tile
   // first row of row tile tm, and the place in it of LDS tile row `row`
@@ -740,8 +759,18 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int valid = min(tile_rows, R - tm * tile_rows);
     return (((valid + 31) >> 5) + 1) >> 1;
   };
-  auto row_in_tile = [&](int row, int p0) {
-    return TAILS && row >= BM / 2 ? row - BM / 2 + 32 * p0 : row;
+  // (rows that are not multiplied: a row of the tile that another lane loads)
+  auto row_in_tile = [&](int row, int p0, int tm) {
+    if (!TAILS) return row;
+    const int last = min(tile_rows, R - tm * tile_rows) - 1;
+    if (DEEP) return min(row, last);
+    return row >= BM / 2 ? min(row - BM / 2 + 32 * p0, last)
+                         : min(row, min(32 * p0 - 1, last));
+  };
+  // LDS row that lane l's 16 bytes of load j belong to
+  auto lds_row = [&](int j, int l) {
+    return DEEP && j == 2 ? 128 + wave * 4 + ((l & 31) >> 3)
+                          : (wave + Cfg::WAVES * j) * 8 + (l >> 3);
   };
   // logical tile -> expert, row tile, column tile
   auto tile_coords = [&](int logical, int& e, int& tm, int& tn) RING_INLINE {
@@ -758,6 +787,9 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     return ((l & 7) ^ lds_swizzle(wave * 8 + (l >> 3))) * 8;
   };
   const int a_chunk = chunk_of(lane);
+  // (DEEP: of load 2, whose rows are four per wavefront)
+  auto chunk2_of = [&](int l) { return ((l & 7) ^ lds_swizzle(lds_row(2, l))) * 8; };
+  const int a_chunk2 = DEEP ? chunk2_of(lane) : 0;
   if constexpr (!KMAJOR) b_lane = (uint32_t)((lane >> 3) * K + a_chunk) * 2;
   // (What a step of the tile loop outside its K loop computes from the lane index, it
   // computes from a copy that the compiler cannot see through: done once ahead of
@@ -770,7 +802,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   };
   // GATHER: the slot -> token map entries of the four rows this lane loads in a
   // tile.  They are asked for a whole tile ahead of their use.
-  int map_src[Cfg::A_INSTR];
+  int map_src[A_LOADS];
   auto fetch_map = [&](int logical) RING_INLINE {
     if constexpr (GATHER) {
       int e, tm, tn;
@@ -778,8 +810,8 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       const int p0 = TAILS ? tile_pieces0(tm) : 0;
       const int s_lane = lane_again();
 #pragma unroll
-      for (int j = 0; j < Cfg::A_INSTR; ++j) {
-        const int row = row_in_tile((wave + Cfg::WAVES * j) * 8 + (s_lane >> 3), p0);
+      for (int j = 0; j < A_LOADS; ++j) {
+        const int row = row_in_tile(lds_row(j, s_lane), p0, tm);
         map_src[j] = row_map[(int64_t)e * R + min(tile_row0(tm) + row, R - 1)];
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -853,22 +885,25 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       b_lane = k_row * N + min(col0 + chunk, N - 8);
     } else {
 #pragma unroll
-      for (int j = 0; j < Cfg::A_INSTR; ++j) {
-        const int row = (wave + Cfg::WAVES * j) * 8 + (s_lane >> 3);
+      for (int j = 0; j < A_LOADS; ++j) {
+        const int row = lds_row(j, s_lane);
         if constexpr (GATHER)
           a_row[j] = map_src[j];
         else
-          a_row[j] = (uint32_t)(min(row0 + row_in_tile(row, t.pieces0), R - 1) * K +
-                                chunk_of(s_lane)) * 2;
+          a_row[j] = (uint32_t)(min(row0 + row_in_tile(row, t.pieces0, tm), R - 1) * K +
+                                (DEEP && j == 2 ? chunk2_of(s_lane)
+                                                : chunk_of(s_lane))) * 2;
+      }
+#pragma unroll
+      for (int j = 0; j < Cfg::B_INSTR; ++j)
         // (N % 8 == 0: eight rows exist or they do not)
         b_row[j] = min(col0 + (wave + Cfg::WAVES * j) * 8, N - 8) * K;
-      }
     }
     return t;
   };
-  // load j of the token (A, two slots at LDS offset 0) / weight (B, three
-  // slots behind them) tile kt; `zeros`: of a K tile of zeros instead
-  constexpr int B_BASE = Cfg::B_BASE;
+  // load j of the token (A, two slots at LDS offset 0, DEEP: three) / weight (B,
+  // three slots behind them) tile kt; `zeros`: of a K tile of zeros instead
+  constexpr int B_BASE = A_SLOTS * A_BYTES;
   // KMAJOR: load j of a tile fills reduction rows 2 (wave + WAVES j) and + 1
   // (lanes 32-63) of it; past the last reduction row they are zeros
   auto kmajor_past_end = [&](int kt, int j) {
@@ -883,14 +918,22 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       src = Ae + kmajor_row(kt, j) * R + a_lane;
     else if constexpr (GATHER)
       src = ((int)a_row[j] < 0 ? zero_row : Ae + (int64_t)(int)a_row[j] * K) +
-            (a_chunk + kt * BK);
+            ((DEEP && j == 2 ? a_chunk2 : a_chunk) + kt * BK);
     else
       src = (const bf16_t*)((const char*)(Ae + kt * BK) + a_row[j]);
     if (zeros || (KMAJOR && kmajor_past_end(kt, j)))
       src = ring_zero_row + ((KMAJOR ? lane : lane_again()) & 31) * 8;
+    if (DEEP && j == 2) {
+      if (lane < 32)
+        __builtin_amdgcn_global_load_lds(
+            (glb_void_t*)src,
+            (lds_void_t*)(smem_raw + slot * A_BYTES + 128 * Cfg::ROW_BYTES +
+                          wave * 512), 16, 0, 0);
+      return;
+    }
     __builtin_amdgcn_global_load_lds(
         (glb_void_t*)src,
-        (lds_void_t*)(smem_raw + slot * Cfg::A_BYTES +
+        (lds_void_t*)(smem_raw + slot * A_BYTES +
                       (wave + Cfg::WAVES * j) * 1024), 16, 0, 0);
   };
   auto load_b = [&](int kt, int slot, int j, bool zeros = false) RING_INLINE {
@@ -936,7 +979,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
 #pragma unroll
     for (int kk = 0; kk < BK / 16; ++kk) {
       const int col = ((kk * 2 + fc) ^ lds_swizzle(fr)) * 16;
-      a_frag[kk] = (wm * Cfg::WTM + fr) * Cfg::ROW_BYTES + col;
+      a_frag[kk] = ((DEEP ? 0 : wm * Cfg::WTM) + fr) * Cfg::ROW_BYTES + col;
       b_frag[kk] = (wn * Cfg::WTN + fr) * Cfg::ROW_BYTES + col;
     }
   }
@@ -968,13 +1011,16 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // DEEP: the lower half's rows follow the upper half's pieces
+  int a_half = 0;
   // token fragment of piece n / weight fragment n of MFMA step kk
   auto read_a = [&](int aslot, int kk, int n) RING_INLINE -> bf16x8_t {
     if constexpr (KMAJOR)
-      return read_tr(lds0 + aslot * Cfg::A_BYTES + a_frag[n], kk);
+      return read_tr(lds0 + aslot * A_BYTES + a_frag[n], kk);
     else
       return *reinterpret_cast<const bf16x8_t*>(
-          smem_raw + aslot * Cfg::A_BYTES + a_frag[kk] + n * 32 * Cfg::ROW_BYTES);
+          smem_raw + (aslot * A_BYTES + a_half) + a_frag[kk] +
+          n * 32 * Cfg::ROW_BYTES);
   };
   auto read_b = [&](int bslot, int kk, int n) RING_INLINE -> bf16x8_t {
     if constexpr (KMAJOR)
@@ -1028,6 +1074,10 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   // being loaded) that its loads fetch
   int aslot = 0, bslot = 0, lk = 2;
   // FIRST: K tile 0
+  auto next_a_slot = [&](int slot) {
+    if constexpr (A_SLOTS == 2) return slot ^ 1;
+    else return slot == A_SLOTS - 1 ? 0 : slot + 1;
+  };
   auto k_tile = [&](auto first_tag, auto na_tag) RING_INLINE {
     constexpr bool FIRST = decltype(first_tag)::value;
     constexpr int NA = decltype(na_tag)::value;      // row pieces in use
@@ -1040,6 +1090,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     };
     const int bnext = bslot == 2 ? 0 : bslot + 1;       // slot of the next K tile
     const int bnext2 = bnext == 2 ? 0 : bnext + 1;      // of the one after it
+    const int anext = next_a_slot(aslot), anext2 = next_a_slot(anext);
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
       const int cur = kk & 1, nxt = cur ^ 1;
@@ -1048,6 +1099,14 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       // next over steps 0..2, all four token loads of it right behind the
       // hand-over barrier that frees their slot (a full K tile ahead of use).
       auto load = [&](int which) {
+        if constexpr (DEEP) {
+          const int n = 2 * kk + which;       // 0 .. 6
+          if (kk == 3) return;
+          if (n < 3) load_a(lk, anext2, n);
+          else load_b(lk, bnext2, n - 3);
+          return;
+        }
+        if (which > 1 && kk < 3) return;
         if (kk == 0) load_b(lk, bnext2, which);
         if (kk == 1 && which == 0) load_b(lk, bnext2, 2);
         if (kk == 2 && which == 0) load_b(lk, bnext2, 3);
@@ -1073,12 +1132,14 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         mm(cur, 5); fence();
         rd(aslot, bslot, kk + 1, nxt, RD[5]);
         mm(cur, 6); fence();
+        if (DEEP && kk == 2) { load(2); fence(); }
         mm(cur, 7); fence();
       } else {
         // this lane holds the last step's fragments (lgkmcnt 0); everything
         // but the four weight loads of tile kt+2 has landed (vmcnt 4)
         fence();
-        __builtin_amdgcn_s_waitcnt((4 & 15) | (0 << 8) | (7 << 4));
+        constexpr int AHEAD = DEEP ? A_LOADS + Cfg::B_INSTR : Cfg::B_INSTR;
+        __builtin_amdgcn_s_waitcnt((AHEAD & 15) | (0 << 8) | (7 << 4));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -1087,7 +1148,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         // up with the other wavefronts' and hold this one's MFMAs back
 #pragma unroll
         for (int n = 0; n < 6; ++n) {
-          rd(aslot ^ 1, bnext, 0, nxt, RD[n]);
+          rd(anext, bnext, 0, nxt, RD[n]);
           if (n >= 2) load(n - 2);
           mm(cur, n); fence();
         }
@@ -1095,7 +1156,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         mm(cur, 7); fence();
       }
     }
-    aslot ^= 1;
+    aslot = anext;
     bslot = bnext;
     ++lk;
   };
@@ -1139,6 +1200,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
                   "a piece is 32 rows of 128 bytes");
     const int bnext = bslot == 2 ? 0 : bslot + 1;       // K tile 0 of the next tile
     const int bfree = bnext == 2 ? 0 : bnext + 1;       // K tile 1: free till then
+    const int anext = next_a_slot(aslot), afree = next_a_slot(anext);
     bf16x8_t ga[2][KSTEPS - 1], gb[KSTEPS - 1][TN];
     auto mm = [&](int i, int n) {
       const int kk = n / TN, j = n % TN;
@@ -1310,10 +1372,10 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     asm volatile("" : "+s"(kt1));
     if (has_next) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) load_a(kt1, aslot, j, after.nk < 2);
+      for (int j = 0; j < A_LOADS; ++j) load_a(kt1, afree, j, after.nk < 2);
     }
     fence();
-    if constexpr (!TAILS) first_frags(aslot ^ 1, bnext, Cfg::TM);
+    if constexpr (!TAILS) first_frags(anext, bnext, Cfg::TM);
     fence();
     if constexpr (NA > 0) {
       zero_if_empty(NA - 1);
@@ -1329,7 +1391,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       for (int j = 0; j < 4; ++j) load_b(kt1, bfree, j, after.nk < 2);
     }
     fence();
-    aslot ^= 1;
+    aslot = anext;
     bslot = bnext;
     lk = 2;
   };
@@ -1349,15 +1411,15 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   int next_entry = entry_of(next), next2_entry = entry_of(next2);
   if (next < total_tiles) fetch_map(next_entry);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) load_a(0, 0, j);
+  for (int j = 0; j < A_LOADS; ++j) load_a(0, 0, j);
 #pragma unroll
   for (int j = 0; j < 4; ++j) load_b(0, 0, j);
 #pragma unroll
   for (int j = 0; j < 4; ++j) load_b(1, 1, j, t.nk < 2);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) load_a(1, 1, j, t.nk < 2);
-  // K tile 0 has landed: only tile 1 (4 + 4 loads) may still be in flight
-  wait_vmcnt<8>();
+  for (int j = 0; j < A_LOADS; ++j) load_a(1, 1, j, t.nk < 2);
+  // K tile 0 has landed: only tile 1 may still be in flight
+  wait_vmcnt<A_LOADS + Cfg::B_INSTR>();
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -1365,6 +1427,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   wait_frags();
   for (;;) {
     if constexpr (KMAJOR && TAILS) set_a_frag(t.pieces0);
+    if constexpr (DEEP) a_half = wm == 0 ? 0 : t.pieces0 * 32 * Cfg::ROW_BYTES;
     const bool has_next = next < total_tiles;
     Tile after = t;
     auto tile_pass = [&](auto na_tag) RING_INLINE {
@@ -1377,7 +1440,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
       // tile they are the first of this one again, which nobody reads.)
       auto advance = [&]() RING_INLINE {
         if (has_next) {
-          if constexpr (GATHER) wait_vmcnt<8>();
+          if constexpr (GATHER) wait_vmcnt<A_LOADS + Cfg::B_INSTR>();
           after = set_tile(next_entry);
           if (next2 < total_tiles) fetch_map(next2_entry);
         }
@@ -1401,7 +1464,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         case 1: tile_pass(std::integral_constant<int, 1>{}); break;
         case 2: tile_pass(std::integral_constant<int, 2>{}); break;
         case 3: tile_pass(std::integral_constant<int, 3>{}); break;
-        default: tile_pass(std::integral_constant<int, Cfg::TM>{}); break;
+        default: tile_pass(std::integral_constant<int, DEEP ? 3 : Cfg::TM>{}); break;
       }
     } else {
       tile_pass(std::integral_constant<int, Cfg::TM>{});
@@ -1998,22 +2061,20 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 // Rows per row tile (a multiple of 32, at most 256) for R rows per expert.
 // The persistent blocks take whole rounds of tiles, so what counts is rounds
 // times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
-// 0.45 + 0.14 per piece us per K tile (from launches of 400 to 900 rows per
-// expert, K 768 to 4096, N 768 to 8192; no less than 0.6) and 6.5 us outside the K
-// loop.  Rows are spread evenly over the row tiles: 640 rows per expert are three tiles
-// of 224 or four of 160, not 256 + 256 + 128.  (The terms are from when a tile's output
-// was staged behind its K loop; it now runs beside it, and a tile costs less outside.
-// What that moves is within 5 %: of 15 products timed with every height since, K 64 to
-// 4096, the rule's choice was the fastest or within 2 % of it in 13; 16 x 256 rows, 4096
-// x 1024 took 50.5 us with its 64 rows and 48.3 with 128, 48 x 180 rows, 768 x 1536 36.5
-// with its 192 and 35.3 with 96.)  Tiles of 256 and a shorter last one -> the rule's
-// choice (both sides bit-identical):
-//   32 x 640 rows, 4096 x 1024 (160 rows; of 224 188 us)             -> 171 us
-//   16 x 705 rows, 768 x 3072 (192 rows) / 3072 x 768 (160)  61 / 54 -> 50 / 50
-//   8 x 900 rows, 1536 x 4608 (192 rows)                        110 -> 91
-//   64 x 320 rows, 1024 x 4096 (160 rows; of 128 235 us)             -> 197
-//   16 x 705 rows, 512 x 768 (160 rows)                        15.0 -> 13.1
-//   5000 rows, 1280 x 1280 (128 rows)                          26.9 -> 21.7
+// 0.40 + 0.13 per piece us per K tile (0.20 + 0.14 with three token slots, no less than
+// 0.6 and 0.5) and 5 us outside the K loop.  Rows are spread evenly over the row tiles:
+// 640 rows per expert are three tiles of 224 or four of 160, not 256 + 256 + 128.  The
+// terms are fitted to 18 products of 1 to 128 experts, 180 to 16000 rows, K 512 to 8192,
+// N 512 to 8192, timed with six heights each: the rule's choice is 0.3 % slower than the
+// best of them on average and 2.2 % at worst (16 x 1250 rows, 768 x 3072: 256 rows 90.0
+// us, 160 88.1).  Tiles of 256 and a shorter last one -> the rule's choice (both sides
+// bit-identical):
+//   32 x 640 rows, 4096 x 1024 (160 rows; of 224 186 us)       197 -> 155 us
+//   16 x 708 rows, 768 x 3072 (192 rows) / 3072 x 768 (160)  67 / 56 -> 53 / 51
+//   8 x 900 rows, 1536 x 4608 (192 rows)                        111 -> 93
+//   64 x 320 rows, 1024 x 4096 (160 rows; of 128 206 us)       200 -> 182
+//   16 x 700 rows, 512 x 512 (96 rows)                         14.1 -> 10.7
+//   5000 rows, 1280 x 1280 (128 rows)                          26.6 -> 20.4
 // K-major operands (weight gradients; R is then a width, K the rows summed over):
 // 0.48 + 0.12 per piece us per K tile, 3.3 + 0.75 per piece outside the K loop, whose
 // share is larger there (reductions of few K tiles; from 16 x 704 and 1280 rows, and
@@ -2036,10 +2097,14 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
     const int even = ((R + tiles_m - 1) / tiles_m + 31) / 32 * 32;
     const int64_t tiles = (int64_t)E * ((R + even - 1) / even) * tiles_n;
     const int pieces = even / 32;
-    const double per_k_tile = kmajor ? 0.48 + 0.12 * pieces : 0.45 + 0.14 * pieces;
-    const double outside = kmajor ? 3.3 + 0.75 * pieces : 6.5;
+    const bool deep = !kmajor && even <= RingCfg::DEEP_ROWS;
+    const double per_k_tile = kmajor ? 0.48 + 0.12 * pieces
+                              : deep ? 0.20 + 0.14 * pieces
+                                     : 0.40 + 0.13 * pieces;
+    const double least = deep ? 0.5 : 0.6;
+    const double outside = kmajor ? 3.3 + 0.75 * pieces : 5.0;
     const double cost = (double)((tiles + cus - 1) / cus) *
-                        (nk * (per_k_tile < 0.6 ? 0.6 : per_k_tile) + outside);
+                        (nk * (per_k_tile < least ? least : per_k_tile) + outside);
     if (rows == RingCfg::BM || cost < 0.98 * best) {
       best = cost;
       best_rows = even;
@@ -2134,6 +2199,9 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
 #define MOE_RING(RELU_, GATHER_, MASKED_, LISTED_, TAILS_)                     \
   run(grouped_gemm_bf16_ring_kernel<RELU_, GATHER_, false, MASKED_, LISTED_,   \
                                     TAILS_>)
+#define MOE_RING_DEEP(RELU_, GATHER_, MASKED_)                                 \
+  run(grouped_gemm_bf16_ring_kernel<RELU_, GATHER_, false, MASKED_, false,     \
+                                    true, false, true>)
   if (tile_list != nullptr) {
     if (mask_src != nullptr) return MOE_RING(false, false, true, true, false);
     // the first GEMM gathers its rows, the second does not
@@ -2146,14 +2214,17 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
   // row tiles of fewer than 256 rows, or an expert's last one partly empty: the
   // instantiation that skips empty 32-row pieces
   const bool tails = R % tile_rows != 0 || tile_rows != Cfg::BM;
+  const bool deep = tile_rows <= Cfg::DEEP_ROWS;
 #define MOE_RING_T(RELU_, GATHER_, MASKED_)                                    \
-  (tails ? MOE_RING(RELU_, GATHER_, MASKED_, false, true)                      \
-         : MOE_RING(RELU_, GATHER_, MASKED_, false, false))
+  (deep    ? MOE_RING_DEEP(RELU_, GATHER_, MASKED_)                            \
+   : tails ? MOE_RING(RELU_, GATHER_, MASKED_, false, true)                    \
+           : MOE_RING(RELU_, GATHER_, MASKED_, false, false))
   if (mask_src != nullptr) return MOE_RING_T(false, false, true);
   if (row_map != nullptr)
     return relu ? MOE_RING_T(true, true, false) : MOE_RING_T(false, true, false);
   return relu ? MOE_RING_T(true, false, false) : MOE_RING_T(false, false, false);
 #undef MOE_RING_T
+#undef MOE_RING_DEEP
 #undef MOE_RING
 }
 

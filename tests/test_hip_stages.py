@@ -1866,6 +1866,36 @@ def test_linear_row_tiles(hip, shape):
   assert torch.equal(da, hip.expert_linear(dy, w))
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 448])
+@pytest.mark.parametrize("e,rows,n", [(130, 129, 520), (200, 257, 520),
+                                      (64, 260, 1024), (20, 290, 264), (9, 150, 264)])
+def test_linear_three_token_slots(hip, e, rows, n, k):
+  """Row tiles of 32 to 160 rows, whose token tiles have three slots: tiles of one
+  to five pieces, last rows of a tile one and 97 to 129 rows in, fewer K tiles than
+  slots, blocks with one tile and with several; with ReLU and with its mask."""
+  _check_linear(hip, (e, rows, k, n), "relu")
+  gen = torch.Generator(device="cuda").manual_seed(e + rows)
+  dy, w, y = (torch.randn(s, generator=gen, device="cuda").to(torch.bfloat16)
+              for s in ((e, rows, k), (e, n, k), (e, rows, n)))
+  masked = hip.expert_linear_backward(y, dy, w, da_relu_mask=y)[0]
+  assert torch.equal(masked, hip.expert_linear(dy, w) * (y > 0))
+
+
+@pytest.mark.parametrize("e,g,c,h", [(32, 5, 128, 1024), (32, 5, 127, 1024),
+                                     (16, 2, 128, 512)])
+def test_gathered_rows_with_three_token_slots(hip, e, g, c, h):
+  """The same tiles with rows fetched through the slot map: the bits of dispatch and
+  two products."""
+  s, m = 512, 1024
+  gen = torch.Generator(device="cuda").manual_seed(g + c)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  r = hip.top2_gating(mk(g, s, e), c)
+  x, wi, wo = (t.to(torch.bfloat16) for t in (mk(g, s, m), mk(e, h, m), mk(e, m, h)))
+  got = hip.dispatched_expert_ffn(x, r, wi, wo, "relu")
+  xe = hip.dispatch(x, r).reshape(e, g * c, m)
+  assert torch.equal(got, hip.expert_ffn(xe, wi, wo, "relu"))
+
+
 @pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
                                    (2, 6144, 776, 256), (29, 3000, 520, 760)],
                          ids=lambda s: "x".join(map(str, s)))
