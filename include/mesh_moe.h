@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 40
+#define MESH_MOE_ABI_VERSION 41
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -407,6 +407,27 @@ int mesh_moe_combine_loss(const void* y, const int32_t* idx, const int32_t* pos,
                           const int32_t* row_offsets, const float* loss,
                           double loss_coef, void* out, void* loss_out, int G, int S,
                           int E, int C, int N, int dtype, void* stream);
+
+/*
+ * The forward pass of transformer_moe_layer_v1 with _top_2_gating and one expert layer
+ * (transformer/moe.py:191-525, :1312-1513) in one call: router projection, gating,
+ * dispatch, the two expert products and combine, with the results of the calls above.
+ *   x [G,S,M] dtype; w_gate [M,E] and w_gate_packed [E,M] dtype; wi_packed [E,H,M],
+ *   wo_packed [E,N,H]; importance as in mesh_moe_top2_gating; the operands' addresses
+ *   multiples of 16 (else MESH_MOE_E_UNSUPPORTED, nothing launched)
+ *   policy      as in mesh_moe_top2_gating, not MESH_MOE_SECOND_RANDOM
+ *   out [G,S,N] dtype; loss_out [2] dtype as in mesh_moe_combine_loss
+ */
+size_t mesh_moe_top2_layer_workspace_bytes(int G, int S, int E, int C, int M, int H,
+                                           int N, int dtype);
+int mesh_moe_top2_layer(const void* x, const void* w_gate, const void* w_gate_packed,
+                        const void* wi_packed, const void* wo_packed,
+                        const void* importance, int importance_dtype, void* out,
+                        void* loss_out, void* workspace, size_t workspace_bytes,
+                        int G, int S, int E, int C, int M, int H, int N,
+                        int activation, int dtype, int policy, double threshold,
+                        int use_second_place_loss, int num_microbatches,
+                        double loss_coef, void* stream);
 
 /*
  * "No token left behind" gating (_ntlb_gating, transformer/moe.py:804-940)

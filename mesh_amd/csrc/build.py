@@ -11,7 +11,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCES = ["abi.hip", "route.hip", "dispatch.hip", "ffn.hip", "gemm_f32.hip",
            "backward.hip", "expert_choice.hip", "ntlb.hip", "summaries.hip",
-           "block.hip", "attention.hip"]
+           "block.hip", "attention.hip", "layer.hip"]
 LIB_NAME = "libmesh_moe_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 

@@ -38,6 +38,11 @@ int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int 
                     int K, bool relu, const float* mask_src, float mask_scale,
                     hipStream_t st);
 
+// ffn.hip: whether the expert feed-forward calls that fold the dispatch into their
+// first product take these sizes
+bool dispatched_ffn_shapes(int G, int S, int E, int C, int M, int H, int dtype);
+bool compact_ffn_shapes(int G, int S, int E, int C, int M, int H, int N, int dtype);
+
 // Fused self-attention (attention.hip): q, k, v, out [B,L,H*D] bf16.
 bool flash_attention_supported(int L, int H, int D, int dtype, const void* q,
                                const void* k, const void* v, const void* out);

@@ -2648,6 +2648,27 @@ __global__ __launch_bounds__(LIST_THREADS) void compact_lists_kernel(
   write_tile_list(lists, used, blockIdx.x);
 }
 
+// The conditions of mesh_moe_dispatched_expert_ffn and mesh_moe_compact_expert_ffn on
+// sizes (operands are to lie on 16 bytes besides)
+static bool dispatched_sizes_fit(int G, int S, int C, int dtype) {
+  return dtype == MESH_MOE_BF16 && (int64_t)G * C <= 0x7fffffffLL &&
+         (int64_t)G * S <= 0x7fffffffLL;
+}
+static bool dispatched_few_rows(int G, int S, int E, int C, int M, int H) {
+  const int64_t rows = (int64_t)G * C;
+  return rows <= STREAM_ROWS && (int64_t)G * S <= MAP_SCAN_TOKENS &&
+         stream_applies(E, (int)rows, H, M) && many_column_tiles(E, H);
+}
+bool dispatched_ffn_shapes(int G, int S, int E, int C, int M, int H, int dtype) {
+  return dispatched_sizes_fit(G, S, C, dtype) &&
+         (dispatched_few_rows(G, S, E, C, M, H) || ring_path_applies(G * C, H, M));
+}
+bool compact_ffn_shapes(int G, int S, int E, int C, int M, int H, int N, int dtype) {
+  return dispatched_sizes_fit(G, S, C, dtype) && E <= 1024 &&
+         ring_path_applies(G * C, H, M) && ring_path_applies(G * C, N, H) &&
+         (int64_t)G * C * H < (1LL << 31);    // h's offsets within an expert
+}
+
 }  // namespace mesh_moe
 
 extern "C" size_t mesh_moe_dispatched_expert_ffn_workspace_bytes(int G, int E,
@@ -2671,12 +2692,9 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
               MESH_MOE_E_ARG, "dispatched_expert_ffn: unknown activation %d",
               activation);
   const int64_t rows = (int64_t)G * C;
-  const bool few_rows =
-      rows <= STREAM_ROWS && (int64_t)G * S <= MAP_SCAN_TOKENS &&
-      stream_applies(E, (int)rows, H, M) && many_column_tiles(E, H) &&
-      ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
-  MOE_REQUIRE(dtype == MESH_MOE_BF16 && rows <= 0x7fffffffLL &&
-                  (int64_t)G * S <= 0x7fffffffLL &&
+  const bool few_rows = dispatched_few_rows(G, S, E, C, M, H) &&
+                        ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
+  MOE_REQUIRE(dispatched_sizes_fit(G, S, C, dtype) &&
                   (few_rows || ring_path_applies((int)rows, H, M)) &&
                   (((uintptr_t)x | (uintptr_t)wi_packed | (uintptr_t)h) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,
@@ -2770,11 +2788,7 @@ extern "C" int mesh_moe_compact_expert_ffn(
               MESH_MOE_E_ARG, "compact_expert_ffn: unknown activation %d",
               activation);
   const int64_t rows = (int64_t)G * C;
-  MOE_REQUIRE(dtype == MESH_MOE_BF16 && rows <= 0x7fffffffLL && E <= 1024 &&
-                  (int64_t)G * S <= 0x7fffffffLL &&
-                  ring_path_applies((int)rows, H, M) &&
-                  ring_path_applies((int)rows, N, H) &&
-                  rows * H < (1LL << 31) &&    // h's offsets within an expert
+  MOE_REQUIRE(compact_ffn_shapes(G, S, E, C, M, H, N, dtype) &&
                   (((uintptr_t)x | (uintptr_t)wi_packed | (uintptr_t)wo_packed |
                     (uintptr_t)h | (uintptr_t)y) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,

@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 40
+ABI_VERSION = 41
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -224,6 +224,14 @@ _SIGNATURES = {
     "mesh_moe_shared_linear_backward": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
+    "mesh_moe_top2_layer_workspace_bytes": (ctypes.c_size_t, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "mesh_moe_top2_layer": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int, _vp, _vp, _vp, ctypes.c_size_t,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_double, ctypes.c_int, ctypes.c_int, ctypes.c_double, _vp]),
     "mesh_moe_residual_rms_norm": (ctypes.c_int, [
         _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int,
         ctypes.c_double, ctypes.c_int, _vp]),
@@ -1040,6 +1048,60 @@ def combine(y, r, group_size, out=None, row_offsets=None, loss_coef=None):
         _dev(r.kept, "kept", torch.uint8, (g, s, 2)), op, g, s, e, c, n, code,
         _stream()), "combine")
   return out
+
+
+def timing():
+  """Whether a StageTimer is installed: it sees the stages' calls one by one."""
+  return _timer is not None
+
+
+def top2_layer(x, w_gate, w_gate_packed, wi_packed, wo_packed, groups, group_size,
+               capacity, out_sizes, activation="relu", importance=None, policy="all",
+               threshold=0.2, use_second_place_loss=False, num_microbatches=None,
+               loss_coef=1.0):
+  """The whole forward pass of a top-2 layer in one library call: x of
+  groups * group_size rows [.., M], w_gate [M, E], w_gate_packed [1, E, M], wi_packed
+  [E, H, M], wo_packed [E, N, H], importance [groups, group_size] values or None ->
+  (out of sizes out_sizes, loss, loss * loss_coef), or None where an operand does not
+  lie on 16 bytes in one piece (the caller then makes the calls one by one)."""
+  lib = load_library()
+  if activation not in ACTIVATIONS:
+    raise ValueError("unsupported expert activation %r" % (activation,))
+  e, h, m = wi_packed.shape
+  n = wo_packed.shape[1]
+  dt, dev = x.dtype, x.device
+  if not (x.is_contiguous() and w_gate.is_contiguous() and
+          (importance is None or importance.is_contiguous())):
+    return None
+  xp = _dev(x, "x")
+  if x.numel() != groups * group_size * m:
+    raise MoeHipError("x: shape %s, expected %d x %d rows of %d"
+                      % (tuple(x.shape), groups, group_size, m))
+  wgp = _dev(w_gate_packed, "w_gate_packed", dt, (1, e, m))
+  wip = _dev(wi_packed, "wi_packed", dt)
+  wop = _dev(wo_packed, "wo_packed", dt, (e, n, h))
+  if (xp | wgp | wip | wop) % 16:
+    return None
+  ip, icode = None, F32
+  if importance is not None:
+    icode = dtype_code(importance.dtype)
+    ip = _dev(importance, "importance")
+    if importance.numel() != groups * group_size:
+      raise MoeHipError("importance: shape %s, expected %s"
+                        % (tuple(importance.shape), (groups, group_size)))
+  code = dtype_code(dt)
+  sizes = (groups, group_size, e, int(capacity), m, h, n)
+  ws_bytes = lib.mesh_moe_top2_layer_workspace_bytes(*sizes, code)
+  ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=dev)
+  out = torch.empty(out_sizes, dtype=dt, device=dev)
+  losses = torch.empty((2,), dtype=dt, device=dev)
+  _check(lib.mesh_moe_top2_layer(
+      xp, _dev(w_gate, "w_gate", dt), wgp, wip, wop, ip, icode, out.data_ptr(),
+      losses.data_ptr(), ws.data_ptr(), ws_bytes, *sizes, ACTIVATIONS[activation],
+      code, POLICIES[policy], float(threshold), int(use_second_place_loss),
+      int(num_microbatches or 1), float(loss_coef), _stream()), "top2_layer")
+  loss, scaled = losses.unbind(0)
+  return out, loss, scaled
 
 
 # ----------------------------------------------------------------------------

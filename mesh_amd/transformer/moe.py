@@ -517,13 +517,48 @@ class MoEV1Operation(mtf.Operation):
     by_input = dict(zip(grad_op.wrt, grad_op.outputs))
     return [by_input.get(t) for t in self.inputs]
 
+  def _lower_whole(self, lowering, x, w_gate, packed):
+    """Everything in one library call, where nothing but the outputs is asked for.
+    False where the calls are to be made one by one."""
+    gating = self._gating
+    if (type(gating) is not _GatingSpec or gating.policy == "random" or
+        self._save_for_backward or self._k_wo is not None or self._more_wi or
+        self._hidden_keep_prob is not None or self.scaled_loss is None or
+        moe_hip.timing()):
+      return False
+    o, g, s, _ = x.shape.to_integer_list
+    sizes = (o, g, s, self.outputs[0].shape.dims[-1].size)
+
+    def fn(x_s, wg_s, imp_s=None):
+      made = moe_hip.top2_layer(
+          x_s, wg_s, *packed, o * g, s, self._capacity, sizes,
+          activation=self._activation, importance=imp_s, policy=gating.policy,
+          threshold=gating.threshold,
+          use_second_place_loss=gating.use_second_place_loss,
+          num_microbatches=gating.num_microbatches,
+          loss_coef=self.scaled_loss.coef)
+      return made or ()
+    args = [lowering.tensors[x], lowering.tensors[w_gate]]
+    if self._has_importance:
+      args.append(lowering.tensors[self.inputs[4]])
+    made = lowering.mesh_impl(self).slicewise(fn, *args)
+    if not made:
+      return False
+    for t, v in zip(self.outputs + [self.scaled_loss.outputs[0]], made):
+      lowering.set_tensor_lowering(t, v)
+    lowering.done_ahead.add(self.scaled_loss)
+    lowering.operations[self] = {}
+    return True
+
   def lower(self, lowering):
-    mesh_impl = lowering.mesh_impl(self)
     x, w_gate, wi, wo = self.inputs[:4]
     dt = x.dtype
     wi_p = _packed(lowering, wi, dt)
     wo_p = _packed(lowering, wo, dt)
     wg_p = _packed(lowering, w_gate, dt)               # [1, E, M]
+    if self._lower_whole(lowering, x, w_gate, (wg_p, wi_p, wo_p)):
+      return
+    mesh_impl = lowering.mesh_impl(self)
     kwo_p = (_packed(lowering, self._k_wo, dt) if self._k_wo is not None
              else None)
     more_wi_p = [_packed(lowering, t, dt) for t in self._more_wi]

@@ -1605,6 +1605,59 @@ def test_v2_random_configs_match_oracle():
           err_msg=str((k, case)))
 
 
+@pytest.mark.parametrize("case", [
+    # batch, length, M, H, E, group, capacity factor, dtype, nonpadding, second place
+    (2, 64, 16, 64, 8, 32, 1.25, "float32", False, False),
+    (3, 50, 24, 40, 5, 64, 1.0, "float32", True, True),
+    (2, 512, 128, 256, 8, 512, 1.25, "float32", False, False),
+    (2, 64, 16, 64, 8, 32, 1.25, "bfloat16", True, False),
+    (40, 1, 256, 2048, 64, 1024, 2.0, "bfloat16", False, False),   # few rows
+    (3, 100, 256, 512, 4, 300, 2.0, "bfloat16", True, True),       # gathered rows
+    (4, 512, 128, 512, 8, 512, 1.25, "bfloat16", True, False),
+    (2, 1024, 256, 512, 4, 1024, 1.0, "bfloat16", False, True)],   # compacted rows
+    ids=lambda c: "x".join(map(str, c[:6])) + "-" + c[7])
+def test_v1_in_one_call_equals_its_calls(case):
+  """A forward-only top-2 layer is one library call; with a timer on the stages it is
+  made call by call.  The same bits, and both against the oracle's tests above."""
+  from mesh_amd import moe_hip
+  b, l, m, hdim, e, group, cf, act_dtype, padded, loss2 = case
+  rng = np.random.default_rng(b + l + m + e)
+  w = dict(w_gate=H.normal_weights(rng, (m, e), m),
+           wi=H.normal_weights(rng, (e, m, hdim), m),
+           wo=H.normal_weights(rng, (e, hdim, m), hdim))
+  hp, _ = make_hparams(moe_num_experts=e, moe_hidden_size=hdim, moe_group_size=group,
+                       moe_capacity_factor_eval=cf, moe_use_second_place_loss=loss2,
+                       moe_second_policy_eval="threshold" if loss2 else "all")
+  xs = [O.cast_act(rng.standard_normal((b, l, m)).astype(np.float32), act_dtype)
+        for _ in range(2)]
+  npad = (rng.random((b, l)) < 0.8).astype(np.float32) if padded else None
+  _, _, lowering, (xt, y) = run_v1(xs[0], w, hp, False, act_dtype, nonpadding=npad)
+  outputs = [t for op in lowering.graph.operations for t in op.outputs]
+  xv = torch.from_numpy(xs[1]).to(H.ACT_TORCH[act_dtype]).cuda()
+  got = []
+  for timed in (False, True):
+    if timed:
+      with moe_hip.StageTimer() as timer:
+        lowering.run({xt: xv})
+      assert len(timer.routing) == 1
+    else:
+      lowering.run({xt: xv})
+    got.append([lowering.export_to_tf_tensor(t) for t in outputs])
+  for one, calls in zip(*got):
+    assert one.dtype == calls.dtype and one.shape == calls.shape
+    assert torch.equal(one, calls)
+  # a view off 16 bytes, and one with other strides: the calls one by one
+  for odd in (torch.empty(xv.numel() + 1, dtype=xv.dtype, device="cuda")[1:],
+              torch.empty((m, b * l), dtype=xv.dtype, device="cuda").t()):
+    odd = odd.reshape(xv.shape) if odd.dim() == 1 else odd.unflatten(0, (b, l))
+    odd.copy_(xv)
+    if act_dtype == "float32" or not odd.is_contiguous():
+      lowering.run({xt: odd})
+      np.testing.assert_allclose(H.to_np(lowering.export_to_tf_tensor(y)),
+                                 H.to_np(got[0][outputs.index(y)]), rtol=2e-2,
+                                 atol=1e-2)
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 def test_captured_step_replays_match_eager(act_dtype):
   """Lowering.capture(): a HIP-graph replay gives what an eager run gives, on
