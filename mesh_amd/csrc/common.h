@@ -42,6 +42,36 @@ int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int 
 // first product take these sizes
 bool dispatched_ffn_shapes(int G, int S, int E, int C, int M, int H, int dtype);
 bool compact_ffn_shapes(int G, int S, int E, int C, int M, int H, int N, int dtype);
+// The token of every expert's row (-1: an empty one, which reads as zeros), for a first
+// product that fetches its rows through it, and the zeros.
+struct SlotMap {
+  int32_t* map = nullptr;       // [E][G * C]
+  uint16_t* zero_row = nullptr; // [zeros], bf16
+  int zeros = 0;
+};
+// where it lies in the workspace of mesh_moe_dispatched_expert_ffn
+SlotMap slot_map_in(void* workspace, int G, int E, int C, int M);
+// mesh_moe_dispatched_expert_ffn (arguments checked by it) with the fill counts, or null.
+// map_made: the map is there.
+int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
+                   const float* gate, const uint8_t* kept, const int32_t* fill,
+                   bool map_made, const void* wi_packed, const void* wo_packed, void* h,
+                   void* y, void* workspace, size_t workspace_bytes, int G, int S,
+                   int E, int C, int M, int H, int N, int activation, int dtype,
+                   void* stream);
+// whether those calls take the kernels for few rows, which read the map at once
+bool dispatched_few_rows(int G, int S, int E, int C, int M, int H);
+
+// route.hip: mesh_moe_top2_gating, which makes the slot map of one group of at most 64
+// tokens (gating_makes_map) in the same launch where one is given
+bool gating_makes_map(int G, int S);
+int top2_gating(const float* logits, const void* importance, int importance_dtype,
+                int importance_from_slot_gate, const float* second_uniform, int G,
+                int S, int E, int C, int policy, double threshold,
+                int use_second_place_loss, int num_microbatches, int32_t* idx,
+                int32_t* pos, float* gate, uint8_t* kept, int32_t* fill, float* loss,
+                void* workspace, size_t workspace_bytes, void* stream,
+                const SlotMap& slots);
 
 // Fused self-attention (attention.hip): q, k, v, out [B,L,H*D] bf16.
 bool flash_attention_supported(int L, int H, int D, int dtype, const void* q,

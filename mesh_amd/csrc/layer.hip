@@ -13,7 +13,7 @@ namespace {
 struct LayerSpace {
   size_t logits, idx, pos, gate, kept, fill, loss, gating, gating_bytes;
   size_t row_offsets, ffn, ffn_bytes, h, y, expert_in, bytes;
-  bool fused_router, compact, dispatched;
+  bool fused_router, compact, dispatched, map_by_gating;
 };
 
 // Which calls the layer is made of (those of mesh_amd/transformer/moe.py for operands
@@ -26,6 +26,8 @@ LayerSpace layer_space(int G, int S, int E, int C, int M, int H, int N, int dtyp
   w.fused_router = bf16 && M % 64 == 0 && E % 4 == 0 && E <= 128 && S % 128 == 0;
   w.compact = rows % 256 == 0 && compact_ffn_shapes(G, S, E, C, M, H, N, dtype);
   w.dispatched = !w.compact && dispatched_ffn_shapes(G, S, E, C, M, H, dtype);
+  w.map_by_gating = w.dispatched && !w.fused_router && gating_makes_map(G, S) &&
+                    dispatched_few_rows(G, S, E, C, M, H);
   auto take = [&](size_t n) {
     const size_t at = w.bytes;
     w.bytes += (n + 255) & ~(size_t)255;
@@ -107,10 +109,11 @@ extern "C" int mesh_moe_top2_layer(
     rc = mesh_moe_router_logits(x, w_gate, w_gate_packed, nullptr, logits, 1, tokens,
                                 M, E, dtype, stream);
     if (rc == 0)
-      rc = mesh_moe_top2_gating(logits, importance, importance_dtype, 0, nullptr, G,
-                                S, E, C, policy, threshold, use_second_place_loss,
-                                num_microbatches, idx, pos, gate, kept, fill, loss,
-                                at + w.gating, w.gating_bytes, stream);
+      rc = top2_gating(logits, importance, importance_dtype, 0, nullptr, G, S, E, C,
+                       policy, threshold, use_second_place_loss, num_microbatches, idx,
+                       pos, gate, kept, fill, loss, at + w.gating, w.gating_bytes,
+                       stream, w.map_by_gating ? slot_map_in(at + w.ffn, G, E, C, M)
+                                               : SlotMap());
   }
   if (rc != 0) return rc;
   void *h = at + w.h, *y = at + w.y;
@@ -122,9 +125,9 @@ extern "C" int mesh_moe_top2_layer(
                                      nullptr, at + w.ffn, w.ffn_bytes, G, S, E, C, M,
                                      H, N, activation, dtype, stream);
   } else if (w.dispatched) {
-    rc = mesh_moe_dispatched_expert_ffn(x, idx, pos, gate, kept, wi_packed, wo_packed,
-                                        h, y, at + w.ffn, w.ffn_bytes, G, S, E, C, M,
-                                        H, N, activation, dtype, stream);
+    rc = dispatched_ffn(x, idx, pos, gate, kept, fill, w.map_by_gating, wi_packed,
+                        wo_packed, h, y, at + w.ffn, w.ffn_bytes, G, S, E, C, M, H, N,
+                        activation, dtype, stream);
   } else {
     void* expert_in = at + w.expert_in;
     rc = mesh_moe_dispatch(x, idx, pos, gate, kept, fill, expert_in, nullptr, G, S, E,

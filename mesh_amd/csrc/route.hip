@@ -807,10 +807,13 @@ __host__ __device__ constexpr int select_row_floats(int E) {
   return (E + 3) / 4 * 4 + 4;            // 16-byte rows, odd in units of 16 bytes
 }                                        // for E = 8 n
 
-// TAIL: another block of the launch reads the records and partial sums (device-scope
-// stores, see st_dev); the choices also go to ch [3][TOKENS] in LDS (-1: not competing;
-// the third: what the loss counts), and `pos` is left to gate_rank_block.
-template <typename IT, int LANES, bool TAIL = false>
+// Where step 1 leaves the records and the partial sums of the loss.  RECORD_TAIL: another
+// block of the launch reads them (device-scope stores, see st_dev); the choices also go
+// to ch [3][TOKENS] in LDS (-1: not competing; the third: what the loss counts), and
+// `pos` is left to gate_rank_block.  RECORD_LDS: the same block finishes them; idx [64][2],
+// gate [64][2], ch and the parts [E] are LDS, pos and kept are left to it.
+constexpr int RECORD_MEMORY = 0, RECORD_TAIL = 1, RECORD_LDS = 2;
+template <typename IT, int LANES, int RECORD = RECORD_MEMORY>
 __device__ __forceinline__ void gate_select_block(
     const float* logits, const IT* importance, const float* second_uniform,
     const GateParams& p, int32_t* idx, int32_t* pos, float* gate, uint8_t* kept,
@@ -830,14 +833,42 @@ __device__ __forceinline__ void gate_select_block(
   // experts this lane walks: none for a token that does not exist
   const int e_end = live ? E : 0;
   const int64_t t = (int64_t)g * S + t0 + (live ? tok : 0);
+  // A block that has the chip to itself reads its logits from memory once, where they fit
+  // REGS registers, and several experts of a sum at a time.  (gate_logits_kernel has no
+  // registers to spare: 2 x 1024 tokens, 8 experts 11.6 us, with the same 12.4.)
+  constexpr bool ALONE = RECORD == RECORD_LDS;
+  constexpr int REGS = ALONE ? 8 : 1;
   const float* src = logits + t * E;
+  const bool in_regs = ALONE && E <= REGS * LANES;
+  float x[REGS];
+#pragma unroll
+  for (int i = 0; i < REGS; ++i)
+    x[i] = in_regs && lane + i * LANES < e_end ? src[lane + i * LANES] : -INFINITY;
+  // fn(expert, logit) for the experts of this lane, in ascending order
+  auto for_logits = [&](auto fn) {
+    if (in_regs) {
+#pragma unroll
+      for (int i = 0; i < REGS; ++i)
+        if (lane + i * LANES < e_end) fn(lane + i * LANES, x[i]);
+    } else {
+      for (int e = lane; e < e_end; e += LANES) fn(e, src[e]);
+    }
+  };
   float* row = tile + tok * ld;
   const bool sw = p.router == ROUTER_SWITCH;
   // the token's record (by one lane of a token that exists): choices, gates, the two
   // `kept` bytes and what the loss counts
   auto write_record = [&](int i1, int i2, float g1, float g2, unsigned k1,
                           unsigned k2, int third) {
-    if constexpr (TAIL) {
+    if constexpr (RECORD == RECORD_LDS) {
+      idx[tok * 2] = i1;
+      idx[tok * 2 + 1] = i2;
+      gate[tok * 2] = g1;
+      gate[tok * 2 + 1] = g2;
+      ch[tok] = (k1 & 1) ? (int16_t)i1 : (int16_t)-1;
+      ch[TOKENS + tok] = (k2 & 1) ? (int16_t)i2 : (int16_t)-1;
+      ch[2 * TOKENS + tok] = (int16_t)third;
+    } else if constexpr (RECORD == RECORD_TAIL) {
       st_dev(reinterpret_cast<unsigned long long*>(idx + t * 2), pack_i2(i1, i2));
       st_dev(reinterpret_cast<unsigned long long*>(gate + t * 2), pack_f2(g1, g2));
       st_dev(reinterpret_cast<uint16_t*>(kept + t * 2), (uint16_t)(k1 | k2 << 8));
@@ -856,25 +887,31 @@ __device__ __forceinline__ void gate_select_block(
     }
   };
   auto write_part = [&](float* at, float v) {
-    if constexpr (TAIL) st_dev(at, v);
+    if constexpr (RECORD == RECORD_TAIL) st_dev(at, v);
     else *at = v;
   };
+  const int64_t part_at = RECORD == RECORD_LDS ? 0 : ((int64_t)g * p.nblk + blk) * E;
 
   float m = -INFINITY;
-  for (int e = lane; e < e_end; e += LANES) m = fmaxf(m, src[e]);
+  for_logits([&](int, float v) { m = fmaxf(m, v); });
 #pragma unroll
   for (int d = 1; d < LANES; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
   const float negm = -m;                                    // reduce_max
-  for (int e = lane; e < e_end; e += LANES)
-    row[e] = expf(src[e] + negm);
+  for_logits([&](int e, float v) { row[e] = expf(v + negm); });
   __syncthreads();
   // exp, reduce_sum: in expert order
   float s = 0.f;
   if (live) {
     int e = 0;
-    for (; e + 4 <= E; e += 4) {
-      const float4 v = *reinterpret_cast<const float4*>(row + e);
+    auto add4 = [&](int at) {
+      const float4 v = *reinterpret_cast<const float4*>(row + at);
       s += v.x; s += v.y; s += v.z; s += v.w;
+    };
+    if constexpr (ALONE) {
+#pragma unroll 4
+      for (; e + 4 <= E; e += 4) add4(e);
+    } else {
+      for (; e + 4 <= E; e += 4) add4(e);
     }
     for (; e < E; ++e) s += row[e];
   }
@@ -891,11 +928,11 @@ __device__ __forceinline__ void gate_select_block(
   const float neglse = -(logf(s) + m);                      // log + max
   float g1 = -1.f;
   int i1 = 0;
-  for (int e = lane; e < e_end; e += LANES) {
-    const float pe = expf(src[e] + neglse);                 // exp(log_softmax)
+  for_logits([&](int e, float v) {
+    const float pe = expf(v + neglse);                      // exp(log_softmax)
     row[e] = pe;
     if (pe > g1) { g1 = pe; i1 = e; }                       // first argmax
-  }
+  });
   first_max(g1, i1);
   __syncthreads();
   bool sel1 = live;
@@ -991,8 +1028,13 @@ __device__ __forceinline__ void gate_select_block(
     __syncthreads();
     if (tid < E) {
       float a = 0.f;
-      for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
-      write_part(part + ((int64_t)g * p.nblk + blk) * E + tid, a);
+      if constexpr (ALONE) {
+#pragma unroll 8
+        for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
+      } else {
+        for (int k = 0; k < ranges; ++k) a += cols[k * el + tid];
+      }
+      write_part(part + part_at + tid, a);
     }
   };
   // density_1_proxy partial: sum over the block's tokens of p * (imp == 1)
@@ -1010,7 +1052,7 @@ __device__ __forceinline__ void gate_select_block(
     if (tid < 2) {
       float a = 0.f;
       for (int r = 0; r < ntok; ++r) a += cols[tid * TOKENS + r];
-      write_part(part2 + ((int64_t)g * p.nblk + blk) * E + tid, a);
+      write_part(part2 + part_at + tid, a);
     }
   } else if (p.use_second_place_loss) {
     __syncthreads();
@@ -1171,10 +1213,11 @@ __device__ __forceinline__ void gate_rank_tile(
 }
 
 // Ranks of the choices of a block of 64 tokens: gate_rank_tile with one wavefront per
-// choice.  ch [3][64] and cnt [3][E] in LDS; `live` tokens exist.
-__device__ __forceinline__ void gate_rank_block(
-    const int16_t* ch, int32_t* cnt, int E, bool loss2, int live, int64_t tok0,
-    int32_t* pos, int32_t* bcnt_blk) {
+// choice.  ch [3][64] and cnt [3][E] in LDS; `live` tokens exist; ranked(token, choice,
+// rank among the block's choosers of that expert).
+template <typename F>
+__device__ __forceinline__ void gate_rank_choices(const int16_t* ch, int32_t* cnt, int E,
+                                                  bool loss2, int live, F&& ranked) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < 3 * E; i += blockDim.x) cnt[i] = 0;
   __syncthreads();
@@ -1191,11 +1234,17 @@ __device__ __forceinline__ void gate_rank_block(
     const unsigned long long before = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     const int rank = (int)__popcll(match & before);
     if (mine >= 0 && rank == 0) cnt[wave * E + mine] = (int)__popcll(match);
-    if (wave < 2 && lane < live)
-      st_dev(pos + (tok0 + lane) * 2 + wave, mine >= 0 ? rank : 0);
+    if (wave < 2 && lane < live) ranked(lane, wave, mine >= 0 ? rank : 0);
   }
   __syncthreads();
-  for (int i = tid; i < 3 * E; i += blockDim.x) st_dev(bcnt_blk + i, cnt[i]);
+}
+__device__ __forceinline__ void gate_rank_block(
+    const int16_t* ch, int32_t* cnt, int E, bool loss2, int live, int64_t tok0,
+    int32_t* pos, int32_t* bcnt_blk) {
+  gate_rank_choices(ch, cnt, E, loss2, live, [&](int token, int choice, int rank) {
+    st_dev(pos + (tok0 + token) * 2 + choice, rank);
+  });
+  for (int i = threadIdx.x; i < 3 * E; i += blockDim.x) st_dev(bcnt_blk + i, cnt[i]);
 }
 
 // What the last block of group g does (all of its threads, 2 E at least; smem is the
@@ -1935,9 +1984,9 @@ __global__ __launch_bounds__(CAP_THREADS) void gate_capacity_kernel(
                       loss, smem_i, blockIdx.x);
 }
 
-// Both steps for a group that is one block of gate_select_kernel: what step 1 wrote is
-// read back by the same block.  (No pointer is __restrict__ here.)  Each step alone is
-// bound by being a launch.
+// Both steps for a group that is one block of gate_select_kernel, slots by gate: what
+// step 1 wrote is read back by the same block.  (No pointer is __restrict__ here.)  Each
+// step alone is bound by being a launch.
 template <typename IT, int LANES>
 __global__ __launch_bounds__(SELECT_THREADS) void gate_small_groups_kernel(
     const float* logits, const IT* importance, const float* second_uniform,
@@ -1951,6 +2000,87 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_small_groups_kernel(
   __syncthreads();
   gate_capacity_group(p, idx, pos, gate, kept, fill, part1, part2, gsum, el, ss,
                       loss, reinterpret_cast<int32_t*>(smem), blockIdx.y);
+}
+
+// Everything for one group of at most 64 tokens, slots in token order, in one block: the
+// records, ranks and sums stay in LDS until they are final.  With `map` also what the
+// first expert product asks for: the token of every slot, -1 for empty ones (a kept
+// choice whose bf16 gate is 0 owns none, as in slot_map_rows_kernel), and a row of m
+// zeros.  Same results, bit for bit, as gate_select_kernel + gate_capacity_kernel.
+// Bound by being a launch and a chain of block barriers.  Both steps in one block, the
+// second on what the first left in memory / here: 32 tokens, 32 experts 10.0 / 6.4 us,
+// 64 of 64 11.8 / 8.3, 17 of 128 13.1 / 8.9; the slot map was another launch, 3.4 to 4.9.
+template <typename IT>
+__global__ __launch_bounds__(SELECT_THREADS) void gate_one_group_kernel(
+    const float* __restrict__ logits, const IT* __restrict__ importance,
+    const float* __restrict__ second_uniform, GateParams p, int32_t* __restrict__ idx,
+    int32_t* __restrict__ pos, float* __restrict__ gate, uint8_t* __restrict__ kept,
+    int32_t* __restrict__ fill, float* __restrict__ loss, int32_t* __restrict__ map,
+    bf16_t* __restrict__ zero_row, int m) {
+  constexpr int LANES = 16, TOKENS = SELECT_THREADS / LANES;
+  static_assert(TOKENS == 64, "gate_rank_choices");
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  __shared__ int32_t ids[TOKENS * 2], rank[TOKENS * 2];
+  __shared__ float gates[TOKENS * 2], terms[GSUM];
+  __shared__ int16_t ch[3 * TOKENS];
+  const int E = p.E, S = p.S, C = p.C, tid = threadIdx.x;
+  const bool sw = p.router == ROUTER_SWITCH;
+  const bool loss2 = p.use_second_place_loss != 0 || sw;
+  float* part1 = smem + TOKENS * select_row_floats(E) + TOKENS + SELECT_THREADS;  // [E]
+  float* part2 = part1 + E;                                        // [max(E, 2)]
+  int32_t* cnt = reinterpret_cast<int32_t*>(part2 + max(E, 2));    // [3][E]
+  float* prod = reinterpret_cast<float*>(cnt + 3 * E);             // [2][E]
+  if (map != nullptr)
+    for (int i = tid; i < m; i += SELECT_THREADS) zero_row[i] = 0;
+  gate_select_block<IT, LANES, RECORD_LDS>(logits, importance, second_uniform, p, ids,
+                                           nullptr, gates, nullptr, part1, part2, smem,
+                                           ch);
+  __syncthreads();
+  gate_rank_choices(ch, cnt, E, loss2, S, [&](int token, int choice, int r) {
+    rank[token * 2 + choice] = r;
+  });
+  if (tid < S * 2) {
+    const int t = tid >> 1, choice = tid & 1;
+    const int e = ids[tid];
+    const bool competes = ch[choice * TOKENS + t] >= 0;
+    int slot = rank[tid];
+    if (choice == 1 && competes) slot += min(cnt[e], C);
+    const bool ok = competes && slot < C;
+    const float v = ok ? gates[tid] : gates[tid] * 0.0f;
+    idx[tid] = e;
+    pos[tid] = slot;
+    gate[tid] = v;
+    kept[tid] = ok ? 1 : 0;
+    if (map != nullptr && ok)
+      map[(int64_t)e * C + slot] = round_to<bf16_t>(v) == 0.0f ? -1 : t;
+  }
+  if (tid < E) {
+    const int t1 = cnt[tid], t2 = cnt[E + tid];
+    const int k1 = min(t1, C), used = k1 + min(t2, C - k1);
+    fill[tid] = used;
+    const float inv_s = (float)(1.0 / (double)S);
+    // density_1: competing first choices (top-2) or every token's arg-max (switch)
+    const int dens = sw ? cnt[2 * E + tid] : t1;
+    prod[tid] = (part1[tid] * inv_s) * ((float)dens * inv_s);
+    if (loss2 && !sw)
+      prod[E + tid] = (part2[tid] * inv_s) * ((float)cnt[2 * E + tid] * inv_s);
+    if (map != nullptr)
+      for (int slot = used; slot < C; ++slot) map[(int64_t)tid * C + slot] = -1;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < E; ++k) s1 += prod[k];
+    if (loss2 && !sw)
+#pragma unroll 8
+      for (int k = 0; k < E; ++k) s2 += prod[E + k];
+    terms[0] = s1;
+    terms[1] = s2;
+    terms[2] = sw && E > 1 ? part2[1] : 0.f;
+    terms[3] = sw ? part2[0] : 0.f;
+    gate_loss_value<false>(p, terms, loss);
+  }
 }
 
 // Both steps and the loss from logits in memory, groups of any number of blocks of 64
@@ -1980,8 +2110,8 @@ __global__ __launch_bounds__(SELECT_THREADS) void gate_logits_kernel(
   float* cols = smem + TOKENS * select_row_floats(p.E) + TOKENS;
   int32_t* cnt = reinterpret_cast<int32_t*>(cols + SELECT_THREADS);   // [3][E]
   int16_t* ch = reinterpret_cast<int16_t*>(cnt + 3 * p.E);            // [3][TOKENS]
-  gate_select_block<IT, LANES, true>(logits, importance, second_uniform, p, idx, pos,
-                                     gate, kept, part1, part2, smem, ch);
+  gate_select_block<IT, LANES, RECORD_TAIL>(logits, importance, second_uniform, p, idx,
+                                            pos, gate, kept, part1, part2, smem, ch);
   const bool loss2 = p.use_second_place_loss != 0 || p.router == ROUTER_SWITCH;
   const int64_t tok0 = (int64_t)g * p.S + blk * TOKENS;
   gate_rank_block(ch, cnt, p.E, loss2, min(TOKENS, p.S - blk * TOKENS), tok0, pos,
@@ -2246,12 +2376,17 @@ static unsigned long long next_call_number() {
   return (n & ((1ull << 48) - 1)) | (1ull << 47);
 }
 
+// Whether the gating of one group can make the slot map of the first expert product.
+namespace mesh_moe {
+bool gating_makes_map(int G, int S) { return G == 1 && S <= 64; }
+}  // namespace mesh_moe
+
 // Gating from logits: step 1 (softmax / choices) then steps 2 and 3.
 static int run_gating(const GateParams& p, const float* logits,
                       const void* importance, int importance_dtype,
                       const float* second_uniform, int32_t* idx, int32_t* pos,
                       float* gate, uint8_t* kept, int32_t* fill, float* loss,
-                      void* workspace, hipStream_t st) {
+                      void* workspace, hipStream_t st, const SlotMap& slots = {}) {
   const int G = p.G, E = p.E;
   uintptr_t wsp = ((uintptr_t)workspace + 255) & ~(uintptr_t)255;
   float* part1 = (float*)wsp;
@@ -2270,13 +2405,16 @@ static int run_gating(const GateParams& p, const float* logits,
   int el, ss;
   const size_t cap_smem = capacity_lds(p, el, ss);
   // A group of one block with nothing to wait for: one group (32 tokens, 32 experts
-  // 10.4 us, with the tail of gate_logits_kernel 10.8; 64 of 64 12.1 and 13.1), or slots
-  // by gate, which that kernel does not do, in up to 128 groups.  (Two to 128 groups:
-  // kernel times with this kernel and the loss's / in one launch 2 x 64 tokens, 16
+  // 6.4 us, with the tail of gate_logits_kernel 10.8; 64 of 64 8.3 and 13.1), or
+  // slots by gate, which those two do not do, in up to 128 groups.  (Two to 128 groups:
+  // kernel times of step 1, step 2 and the loss / in one launch 2 x 64 tokens, 16
   // experts 16.9 / 12.4 us, 32 x 40, 64 experts 20.6 / 16.8, 128 x 64, 128 experts 35.5 /
   // 24.6.)
+  const bool one_group = gating_makes_map(G, p.S) && p.tt == 64 && !p.rank_by_gate;
   const bool one_block =
-      p.nblk == 1 && p.tt == 64 && (p.rank_by_gate ? G <= 128 : G == 1);
+      one_group || (p.nblk == 1 && p.tt == 64 && p.rank_by_gate && G <= 128);
+  MOE_REQUIRE(slots.map == nullptr || one_group, MESH_MOE_E_UNSUPPORTED,
+              "gating: a slot map from more than one block of tokens");
   const size_t tail_smem = fused_tail_lds_bytes(p.nblk, E);
   const size_t select_smem = smem + sizeof(int32_t) * 3 * (size_t)E +
                              sizeof(int16_t) * 3 * 64;
@@ -2316,6 +2454,18 @@ static int run_gating(const GateParams& p, const float* logits,
       k<<<grid, SELECT_THREADS, both, st>>>(logits, imp, second_uniform, p, idx, pos,
                                             gate, kept, part1, part2, ft);
       MOE_CHECK_LAUNCH("gate_logits");
+      return 0;
+    }
+    if (one_group) {
+      auto k = gate_one_group_kernel<IT>;
+      // (the parts, counts and terms per expert behind what step 1 needs)
+      const size_t lds = smem + sizeof(float) * (2 * (size_t)E + 3 * (size_t)E +
+                                                 2 * (size_t)E);
+      MOE_ALLOW_LDS(k, lds);
+      k<<<1, SELECT_THREADS, lds, st>>>(logits, imp, second_uniform, p, idx, pos, gate,
+                                        kept, fill, loss, slots.map, slots.zero_row,
+                                        slots.zeros);
+      MOE_CHECK_LAUNCH("gate_one_group");
       return 0;
     }
     if (one_block) {
@@ -2478,13 +2628,14 @@ extern "C" int mesh_moe_top2_gating_static_scratch(
                               loss, ptr, STATIC_SCRATCH_BYTES, stream);
 }
 
-extern "C" int mesh_moe_top2_gating(
-    const float* logits, const void* importance, int importance_dtype,
-    int importance_from_slot_gate, const float* second_uniform, int G, int S,
-    int E, int C, int policy,
-    double threshold, int use_second_place_loss, int num_microbatches,
-    int32_t* idx, int32_t* pos, float* gate, uint8_t* kept, int32_t* fill,
-    float* loss, void* workspace, size_t workspace_bytes, void* stream) {
+namespace mesh_moe {
+int top2_gating(const float* logits, const void* importance, int importance_dtype,
+                int importance_from_slot_gate, const float* second_uniform, int G,
+                int S, int E, int C, int policy, double threshold,
+                int use_second_place_loss, int num_microbatches, int32_t* idx,
+                int32_t* pos, float* gate, uint8_t* kept, int32_t* fill, float* loss,
+                void* workspace, size_t workspace_bytes, void* stream,
+                const SlotMap& slots) {
   MOE_REQUIRE(logits && idx && pos && gate && kept && fill && loss && workspace,
               MESH_MOE_E_ARG, "top2_gating: null pointer");
   if (int rc = check_gating_args(G, S, E, C, policy, second_uniform, importance,
@@ -2496,7 +2647,21 @@ extern "C" int mesh_moe_top2_gating(
                                   select_tokens(G, S, E));
   return run_gating(p, logits, importance, importance_dtype, second_uniform,
                     idx, pos, gate, kept, fill, loss, workspace,
-                    (hipStream_t)stream);
+                    (hipStream_t)stream, slots);
+}
+}  // namespace mesh_moe
+
+extern "C" int mesh_moe_top2_gating(
+    const float* logits, const void* importance, int importance_dtype,
+    int importance_from_slot_gate, const float* second_uniform, int G, int S,
+    int E, int C, int policy,
+    double threshold, int use_second_place_loss, int num_microbatches,
+    int32_t* idx, int32_t* pos, float* gate, uint8_t* kept, int32_t* fill,
+    float* loss, void* workspace, size_t workspace_bytes, void* stream) {
+  return top2_gating(logits, importance, importance_dtype, importance_from_slot_gate,
+                     second_uniform, G, S, E, C, policy, threshold,
+                     use_second_place_loss, num_microbatches, idx, pos, gate, kept,
+                     fill, loss, workspace, workspace_bytes, stream, SlotMap());
 }
 
 extern "C" int mesh_moe_router_top2_gating(

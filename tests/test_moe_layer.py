@@ -1634,18 +1634,26 @@ def test_v1_in_one_call_equals_its_calls(case):
   _, _, lowering, (xt, y) = run_v1(xs[0], w, hp, False, act_dtype, nonpadding=npad)
   outputs = [t for op in lowering.graph.operations for t in op.outputs]
   xv = torch.from_numpy(xs[1]).to(H.ACT_TORCH[act_dtype]).cuda()
-  got = []
-  for timed in (False, True):
-    if timed:
-      with moe_hip.StageTimer() as timer:
+  router = {v.name: lv for v, lv in lowering.variables.items()}[
+      "moe/top_2_gating/kernel"]
+  # (a router that is sure of its first choice: second gates of 0, whose slots are
+  # kept and hold no token)
+  for scale in (100.0, 1.0):
+    router.assign(w["w_gate"] * np.float32(scale))
+    got = []
+    for timed in (False, True):
+      if timed:
+        with moe_hip.StageTimer() as timer:
+          lowering.run({xt: xv})
+        (record,) = timer.routing
+        zeros = (record.kept > 0) & (record.gate.to(xv.dtype) == 0)
+        assert loss2 or bool(zeros.any()) == (scale > 1.0)
+      else:
         lowering.run({xt: xv})
-      assert len(timer.routing) == 1
-    else:
-      lowering.run({xt: xv})
-    got.append([lowering.export_to_tf_tensor(t) for t in outputs])
-  for one, calls in zip(*got):
-    assert one.dtype == calls.dtype and one.shape == calls.shape
-    assert torch.equal(one, calls)
+      got.append([lowering.export_to_tf_tensor(t) for t in outputs])
+    for one, calls in zip(*got):
+      assert one.dtype == calls.dtype and one.shape == calls.shape
+      assert torch.equal(one, calls)
   # a view off 16 bytes, and one with other strides: the calls one by one
   for odd in (torch.empty(xv.numel() + 1, dtype=xv.dtype, device="cuda")[1:],
               torch.empty((m, b * l), dtype=xv.dtype, device="cuda").t()):
