@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 41
+#define MESH_MOE_ABI_VERSION 42
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -906,6 +906,9 @@ int mesh_moe_broadcast_dropout(const void* x, const void* uniform,
  * weight gradients dw[e] = a^T . dy[e].
  *   a [R,K]; w_packed [E,N,K] (see pack_weights); y, dy [E,R,N]; dw [E,K,N]; bf16, K
  *   and N multiples of 8 (backward: and at least 128)
+ * and the gradient of their input, dx [R,K] = sum over e of dy[e] . w[e]^T, summed in
+ * float32 (w: E pointers, on the host, to [K,N] on the device), for the sizes that
+ * ..._backward_input_supported returns 1 for
  */
 int mesh_moe_shared_linear(const void* a, const void* w_packed, void* y, int E,
                            int R, int K, int N, int dtype, void* stream);
@@ -913,6 +916,11 @@ size_t mesh_moe_shared_linear_backward_workspace_bytes(int E, int R, int K, int 
 int mesh_moe_shared_linear_backward(const void* a, const void* dy, void* dw, int E,
                                     int R, int K, int N, int dtype, void* workspace,
                                     size_t workspace_bytes, void* stream);
+int mesh_moe_shared_linear_backward_input_supported(int E, int R, int K, int N,
+                                                    int dtype);
+int mesh_moe_shared_linear_backward_input(const void* dy, const void* const* w,
+                                          void* dx, int E, int R, int K, int N,
+                                          int dtype, void* stream);
 
 /*
  * RMS normalisation (sublayer_rms_norm, transformer/transformer.py:493-516):

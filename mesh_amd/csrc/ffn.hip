@@ -665,13 +665,21 @@ __device__ __forceinline__ void ring_tile_blocks(int rem, int tiles_m,
 // K tile of a reduction that has one
 static __device__ __attribute__((aligned(256))) bf16_t ring_zero_row[256];
 
+// A reduction in up to three parts (SEGMENTS), C = A0 . B0^T + A1 . B1^T + ...: K is one
+// part's, and part i of an operand lies where its K tiles, counted through, are off by
+// a_at[i] and b_at[i] elements.
+struct RingSegments {
+  int count = 1, tiles = 0;       // parts, K tiles of each
+  int64_t a_at[3] = {}, b_at[3] = {};
+};
+
 // (the pieces of the kernel are lambdas over its registers: one that the compiler
 // left out of line would move them to memory)
 #define RING_INLINE __attribute__((always_inline))
 
 template <bool RELU, bool GATHER = false, bool KMAJOR = false,
           bool MASKED = false, bool LISTED = false, bool TAILS = false,
-          bool SPLIT = false, bool DEEP = false>
+          bool SPLIT = false, bool DEEP = false, bool SEGMENTS = false>
 __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kernel(
     const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
     bf16_t* __restrict__ Cout, int R, int N, int K, int tiles_m, int tiles_n,
@@ -681,13 +689,15 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int32_t* __restrict__ tile_list,
     const int32_t* __restrict__ row_count,
     float mask_scale, float* __restrict__ partial,
-    int whole_tiles, int split, int tile_rows, int64_t a_stride) {
+    int whole_tiles, int split, int tile_rows, int64_t a_stride,
+    RingSegments segments) {
   using Cfg = RingCfg;
   // row_count [E], optional: KMAJOR kernels take it as the reduction extent
   // per expert (k_extent)
   const int32_t* k_extent = KMAJOR ? row_count : nullptr;
   constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, WN = Cfg::WN;
   static_assert(!DEEP || (TAILS && !KMAJOR && !LISTED && !SPLIT), "low row tiles");
+  static_assert(!SEGMENTS || (TAILS && !KMAJOR && !GATHER && !LISTED && !MASKED), "");
   constexpr int A_BYTES = DEEP ? Cfg::DEEP_A_BYTES : Cfg::A_BYTES;
   constexpr int A_SLOTS = DEEP ? 3 : Cfg::A_SLOTS;
   // loads of a token tile per wavefront (DEEP: the third is half a one)
@@ -845,6 +855,7 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     const int row0 = t.row0 = tile_row0(tm);
     const int col0 = t.col0 = tn * BN;
     int nk = KMAJOR ? (K + BK - 1) / BK : K / BK;
+    if constexpr (SEGMENTS) nk *= segments.count;
     t.empty = false;
     if constexpr (KMAJOR && !SPLIT) {
       if (k_extent != nullptr) {
@@ -912,15 +923,20 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   auto kmajor_row = [&](int kt, int j) {
     return (int64_t)((kt0 + kt) * BK + Cfg::WAVES * j * 2);
   };
+  // SEGMENTS: elements from where K tile kt would follow K tile 0 to where it lies
+  auto segment_of = [&](int kt) {
+    return kt < segments.tiles ? 0 : kt < 2 * segments.tiles ? 1 : 2;
+  };
   auto load_a = [&](int kt, int slot, int j, bool zeros = false) RING_INLINE {
     const bf16_t* src;
+    const int64_t jump = SEGMENTS ? segments.a_at[segment_of(kt)] : 0;
     if constexpr (KMAJOR)
       src = Ae + kmajor_row(kt, j) * R + a_lane;
     else if constexpr (GATHER)
       src = ((int)a_row[j] < 0 ? zero_row : Ae + (int64_t)(int)a_row[j] * K) +
             ((DEEP && j == 2 ? a_chunk2 : a_chunk) + kt * BK);
     else
-      src = (const bf16_t*)((const char*)(Ae + kt * BK) + a_row[j]);
+      src = (const bf16_t*)((const char*)(Ae + (jump + kt * BK)) + a_row[j]);
     if (zeros || (KMAJOR && kmajor_past_end(kt, j)))
       src = ring_zero_row + ((KMAJOR ? lane : lane_again()) & 31) * 8;
     if (DEEP && j == 2) {
@@ -938,10 +954,11 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
   };
   auto load_b = [&](int kt, int slot, int j, bool zeros = false) RING_INLINE {
     const bf16_t* src;
+    const int64_t jump = SEGMENTS ? segments.b_at[segment_of(kt)] : 0;
     if constexpr (KMAJOR)
       src = Be + kmajor_row(kt, j) * N + b_lane;
     else
-      src = (const bf16_t*)((const char*)(Be + b_row[j] + kt * BK) + b_lane);
+      src = (const bf16_t*)((const char*)(Be + b_row[j] + (jump + kt * BK)) + b_lane);
     if (zeros || (KMAJOR && kmajor_past_end(kt, j)))
       src = ring_zero_row + ((KMAJOR ? lane : lane_again()) & 31) * 8;
     __builtin_amdgcn_global_load_lds(
@@ -2143,7 +2160,7 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     k<<<split_blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, units, nullptr, nullptr, nullptr,
         nullptr, nullptr, 1.0f, (float*)scratch, plan.whole_tiles, plan.split,
-        Cfg::BM, a_stride);
+        Cfg::BM, a_stride, RingSegments());
     MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands, split)");
     split_reduce_kernel<<<(unsigned)tail * Cfg::TM * Cfg::TN, Cfg::THREADS, 0,
                           st>>>((const float*)scratch, C, R, N, tiles_m,
@@ -2155,7 +2172,8 @@ static int launch_ring_kmajor(const bf16_t* A, const bf16_t* B, bf16_t* C,
     MOE_ALLOW_LDS(k, Cfg::LDS_BYTES);
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, nullptr, nullptr,
-        nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, tile_rows, a_stride);
+        nullptr, nullptr, k_extent, 1.0f, nullptr, 0, 1, tile_rows, a_stride,
+        RingSegments());
     MOE_CHECK_LAUNCH("expert_ffn_backward (mfma, K-major operands)");
     return 0;
   };
@@ -2171,13 +2189,15 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
                        const bf16_t* zero_row = nullptr,
                        const bf16_t* mask_src = nullptr,
                        const int32_t* tile_list = nullptr,
-                       float mask_scale = 1.0f, int64_t a_stride = -1) {
+                       float mask_scale = 1.0f, int64_t a_stride = -1,
+                       const RingSegments& segments = RingSegments()) {
   using Cfg = RingCfg;
   const int cus = compute_units();
   if (cus == 0) return MESH_MOE_E_HIP;
   // (listed tiles are 256 rows high)
   const int tile_rows =
-      tile_list != nullptr ? Cfg::BM : ring_tile_rows(E, R, N, K, cus);
+      tile_list != nullptr ? Cfg::BM
+                           : ring_tile_rows(E, R, N, K * segments.count, cus);
   const int tiles_m = (R + tile_rows - 1) / tile_rows;
   const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n * E;
@@ -2192,7 +2212,7 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
     k<<<blocks, Cfg::THREADS, Cfg::LDS_BYTES, st>>>(
         A, B, C, R, N, K, tiles_m, tiles_n, (int)tiles, row_map, zero_row,
         mask_src, tile_list, nullptr, mask_scale, nullptr, 0, 1, tile_rows,
-        a_stride);
+        a_stride, segments);
     MOE_CHECK_LAUNCH("expert_ffn (mfma, 256-column direct-to-LDS tiles)");
     return 0;
   };
@@ -2215,6 +2235,11 @@ static int launch_ring(const bf16_t* A, const bf16_t* B, bf16_t* C, int E,
   // instantiation that skips empty 32-row pieces
   const bool tails = R % tile_rows != 0 || tile_rows != Cfg::BM;
   const bool deep = tile_rows <= Cfg::DEEP_ROWS;
+  if (segments.count > 1)       // (whole tiles too)
+    return deep ? run(grouped_gemm_bf16_ring_kernel<false, false, false, false, false,
+                                                    true, false, true, true>)
+                : run(grouped_gemm_bf16_ring_kernel<false, false, false, false, false,
+                                                    true, false, false, true>);
 #define MOE_RING_T(RELU_, GATHER_, MASKED_)                                    \
   (deep    ? MOE_RING_DEEP(RELU_, GATHER_, MASKED_)                            \
    : tails ? MOE_RING(RELU_, GATHER_, MASKED_, false, true)                    \
@@ -3370,4 +3395,47 @@ extern "C" int mesh_moe_shared_linear_backward(const void* a, const void* dy,
   void* parts = (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
   return launch_ring_kmajor((const bf16_t*)a, (const bf16_t*)dy, (bf16_t*)dw, E, K,
                             N, R, (hipStream_t)stream, nullptr, parts, 0);
+}
+
+// The gradient of that input, dx = sum over e of dy[e] . w[e]^T, as one product whose
+// reduction has E parts, added in float32.  One by one every part is written, and read
+// again by a sum of its own that rounds it: three parts of 16000 rows, 768 -> 768, are
+// three products of 24 us and two sums of 12, and a training step of such a block took
+// 1924 us, now 1888.  What other kernels than the ring make (few rows, short reductions)
+// is left to them.
+extern "C" int mesh_moe_shared_linear_backward_input_supported(int E, int R, int K,
+                                                               int N, int dtype) {
+  return dtype == MESH_MOE_BF16 && (E == 2 || E == 3) && R >= 1 && K >= 1 && N >= 1 &&
+         ring_shape(R, K, N) && (int64_t)R * N < (1LL << 31) &&
+         (int64_t)N * E <= 0x7fffffff && !stream_applies(1, R, K, N * E) &&
+         !skinny_applies(1, R, K, N * E) && !small_tiles_apply(1, R, K, N * E);
+}
+
+extern "C" int mesh_moe_shared_linear_backward_input(const void* dy,
+                                                     const void* const* w, void* dx,
+                                                     int E, int R, int K, int N,
+                                                     int dtype, void* stream) {
+  MOE_REQUIRE(dy && w && dx, MESH_MOE_E_ARG,
+              "shared_linear_backward_input: null pointer");
+  MOE_REQUIRE(mesh_moe_shared_linear_backward_input_supported(E, R, K, N, dtype),
+              MESH_MOE_E_UNSUPPORTED,
+              "shared_linear_backward_input: needs bf16, two or three layers and a "
+              "product of the 256-column tiles (E=%d R=%d K=%d N=%d dtype=%d)", E, R, K,
+              N, dtype);
+  uintptr_t bits = (uintptr_t)dy | (uintptr_t)dx;
+  RingSegments parts;
+  parts.count = E;
+  parts.tiles = N / RingCfg::BK;
+  for (int i = 0; i < E; ++i) {
+    MOE_REQUIRE(w[i], MESH_MOE_E_ARG, "shared_linear_backward_input: null pointer");
+    bits |= (uintptr_t)w[i];
+    parts.a_at[i] = (int64_t)i * R * N - (int64_t)i * N;
+    parts.b_at[i] = ((intptr_t)w[i] - (intptr_t)w[0]) / (intptr_t)sizeof(bf16_t) -
+                    (int64_t)i * N;
+  }
+  MOE_REQUIRE(bits % 16 == 0, MESH_MOE_E_UNSUPPORTED,
+              "shared_linear_backward_input: operands off 16 bytes");
+  return launch_ring((const bf16_t*)dy, (const bf16_t*)w[0], (bf16_t*)dx, 1, R, K, N,
+                     false, (hipStream_t)stream, nullptr, nullptr, nullptr, nullptr,
+                     1.0f, -1, parts);
 }

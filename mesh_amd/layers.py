@@ -123,8 +123,8 @@ def get_dense_kernel_weights(x, new_dims, reduced_dims, expert_dims,
 
 class SharedInput(object):
   """Dense layers without activation, of one input and of kernels of one shape:
-  their products, and the gradients of their kernels, are made in one launch
-  each."""
+  their products, the gradients of their kernels, and that of their input are made in
+  one launch each."""
 
   def __init__(self, layers):
     x, kernel = layers[0].inputs
@@ -138,11 +138,10 @@ class SharedInput(object):
       for op in layers:
         op.siblings = self
 
-  def make_kernel_gradients(self, lowering, first):
-    """Called by the first of the gradient operations: {layer: its kernel
-    gradient} if every dy is there and they lie one after the other in memory (as
-    the attention's gradient leaves them), else {}."""
-    from mesh_amd import moe_hip
+  def _joint_gradients(self, lowering, first):
+    """Called by the first of the gradient operations: the gradients of all layers'
+    outputs as one tensor [layers, ...], if every one is there and they lie one after
+    the other in memory (as the attention's gradient leaves them), else None."""
     grads = [self.gradients.get(op) for op in self.layers]
     operations = first.graph.operations
     if first not in self._ahead:
@@ -150,27 +149,49 @@ class SharedInput(object):
       self._ahead[first] = None not in grads and all(
           operations.index(g.inputs[0].operation) < at for g in grads)
     if not self._ahead[first]:
-      return {}
-
-    def rows_of(t):
-      return lowering.tensors[t].to_laid_out_tensor().tensor_list[0]
-    x = rows_of(first.inputs[1])
-    dys = [rows_of(g.inputs[0]) for g in grads]
+      return None
+    dys = [_rows_of(lowering, g.inputs[0]) for g in grads]
     d = dys[0]
-    n = d.shape[-1]
     step = d.numel()
-    if not (moe_hip.shared_linear_backward_supported(x, n) and
-            d.data_ptr() % 16 == 0 and all(
-        t.is_contiguous() and t.dtype == x.dtype and t.shape == d.shape and
+    if not all(
+        t.is_contiguous() and t.dtype == d.dtype and t.shape == d.shape and
         t.untyped_storage().data_ptr() == d.untyped_storage().data_ptr() and
         t.storage_offset() == d.storage_offset() + i * step
-        for i, t in enumerate(dys))):
+        for i, t in enumerate(dys)):
+      return None
+    return d.as_strided((len(dys),) + tuple(d.shape), (step,) + d.stride())
+
+  def make_gradients(self, lowering, first):
+    """Called by the first of the gradient operations: {layer: its kernel gradient}
+    and, under the operation whose dx is the sum over all layers, that sum; without the
+    sum, or {}, where there is no kernel for it."""
+    from mesh_amd import moe_hip
+    joint = self._joint_gradients(lowering, first)
+    if joint is None:
       return {}
-    joint = d.as_strided((len(dys),) + tuple(d.shape), (step,) + d.stride())
-    made = lowering.mesh_impl(first).slicewise(
+    x = _rows_of(lowering, first.inputs[1])
+    if not (x.dtype == joint.dtype and joint.data_ptr() % 16 == 0 and
+            moe_hip.shared_linear_backward_supported(x, joint.shape[-1])):
+      return {}
+    mesh_impl = lowering.mesh_impl(first)
+    made = dict(zip(self.layers, mesh_impl.slicewise(
         lambda rows: tuple(moe_hip.shared_linear_backward(rows, joint).unbind(0)),
-        lowering.tensors[first.inputs[1]])
-    return dict(zip(self.layers, made))
+        lowering.tensors[first.inputs[1]])))
+    last = first.sums_up_in(self.layers)
+    if last is not None:
+      n = joint.shape[-1]
+      kernels = [
+          _rows_of(lowering, self.gradients[op].inputs[2]).to(joint.dtype).reshape(
+              -1, n).contiguous() for op in self.layers]
+      if moe_hip.shared_linear_backward_input_supported(joint, kernels):
+        made[last] = mesh_impl.slicewise(
+            lambda _: moe_hip.shared_linear_backward_input(joint, kernels),
+            lowering.tensors[first.inputs[0]])
+    return made
+
+
+def _rows_of(lowering, tensor):
+  return lowering.tensors[tensor].to_laid_out_tensor().tensor_list[0]
 
 
 class DenseOperation(mtf.Operation):
@@ -268,35 +289,79 @@ class DenseGradOperation(mtf.Operation):
                                 % (forward._activation,))  # pylint: disable=protected-access
     self._outputs = [mtf.Tensor(self, x.shape, x.dtype, index=0),
                      mtf.Tensor(self, kernel.shape, kernel.dtype, index=1)]
+    self._dx, self._dw = self._outputs
     self._forward = forward
+    self._adds = self.added_by = None    # layers of the same input (add_to_output)
     siblings = forward.siblings
     if siblings is not None and not self._masks_dx:
       siblings.gradients[forward] = self
 
-  def _kernel_gradient(self, lowering):
-    """This layer's part of what was made for all layers of its input, or None."""
+  def add_to_output(self, output, addend):
+    """Makes dx the sum of what it was and addend, the dx of another layer of the same
+    input, before anything reads it; False where this operation cannot.  Nothing else
+    reads addend: it leaves the graph."""
+    other, siblings = addend.operation, self._forward.siblings
+    # pylint: disable=protected-access
+    if (output is not self._dx or self._adds is not None or siblings is None or
+        siblings.gradients.get(self._forward) is not self or
+        not isinstance(other, DenseGradOperation) or addend is not other._dx or
+        other.added_by is not None or
+        siblings.gradients.get(other._forward) is not other):
+      return False
+    self._adds, other.added_by = other, self
+    other._outputs.remove(addend)
+    return True
+
+  def sums_up_in(self, layers):
+    """The operation whose dx is the sum of those of all `layers`, or None."""
+    last = self
+    while last.added_by is not None:
+      last = last.added_by
+    summed, op = [], last
+    while op is not None:
+      summed.append(op._forward)         # pylint: disable=protected-access
+      op = op._adds                      # pylint: disable=protected-access
+    return last if set(summed) == set(layers) else None
+
+  def _made_ahead(self, lowering):
+    """What the first gradient operation of layers with one input made for all."""
     siblings = self._forward.siblings
     if siblings is None or siblings.gradients.get(self._forward) is not self:
-      return None
+      return {}
     if self._forward is siblings.layers[-1]:
       # (the backward walk meets the last layer first)
-      lowering.run_values[siblings] = siblings.make_kernel_gradients(lowering,
-                                                                     self)
-    return lowering.run_values.get(siblings, {}).pop(self._forward, None)
+      lowering.run_values[siblings] = siblings.make_gradients(lowering, self)
+    return lowering.run_values.get(siblings, {})
+
+  def _set_dx(self, lowering, value):
+    """Lowers dx: `value` is what this layer gives to it."""
+    if self._adds is not None:
+      value = lowering.mesh_impl(self).slicewise(
+          lambda one, dx: one + dx, lowering.run_values.pop(self._adds), value)
+    if self.added_by is not None:
+      lowering.run_values[self] = value
+    else:
+      lowering.set_tensor_lowering(self._dx, value)
 
   def lower(self, lowering):
     from mesh_amd import moe_hip
     mesh_impl = lowering.mesh_impl(self)
-    made = self._kernel_gradient(lowering)
-    if made is not None:
+    made = self._made_ahead(lowering)
+    last = self._forward.siblings and self.sums_up_in(self._forward.siblings.layers)
+    whole = last is not None and last in made
+    dw = made.pop(self._forward, None)
+    if dw is not None:
       k = self.inputs[1].shape.dims[-1].size
       kernel_sizes = self.inputs[2].shape.to_integer_list
-      lowering.set_tensor_lowering(self.outputs[0], mesh_impl.slicewise(
-          lambda dy, x, w: moe_hip.dense(
-              dy, w.to(x.dtype).reshape(1, k, -1).contiguous()),
-          *[lowering.tensors[t] for t in self.inputs[:3]]))
-      lowering.set_tensor_lowering(self.outputs[1], mesh_impl.slicewise(
-          lambda dw, w: dw.reshape(kernel_sizes).to(w.dtype), made,
+      if not whole:
+        self._set_dx(lowering, mesh_impl.slicewise(
+            lambda dy, x, w: moe_hip.dense(
+                dy, w.to(x.dtype).reshape(1, k, -1).contiguous()),
+            *[lowering.tensors[t] for t in self.inputs[:3]]))
+      elif last is self:
+        lowering.set_tensor_lowering(self._dx, made.pop(self))
+      lowering.set_tensor_lowering(self._dw, mesh_impl.slicewise(
+          lambda dw, w: dw.reshape(kernel_sizes).to(w.dtype), dw,
           lowering.tensors[self.inputs[2]]))
       return
     relu = self._relu and not self._dy_is_masked
@@ -312,8 +377,8 @@ class DenseGradOperation(mtf.Operation):
       return dx, dw.reshape(kernel_sizes).to(w.dtype)
     dx, dw = mesh_impl.slicewise(
         fn, *[lowering.tensors[t] for t in self.inputs])
-    lowering.set_tensor_lowering(self.outputs[0], dx)
-    lowering.set_tensor_lowering(self.outputs[1], dw)
+    self._set_dx(lowering, dx)
+    lowering.set_tensor_lowering(self._dw, dw)
 
 
 def _activation_name(activation):

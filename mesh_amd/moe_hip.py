@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 41
+ABI_VERSION = 42
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -224,6 +224,11 @@ _SIGNATURES = {
     "mesh_moe_shared_linear_backward": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
+    "mesh_moe_shared_linear_backward_input_supported": (ctypes.c_int, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "mesh_moe_shared_linear_backward_input": (ctypes.c_int, [
+        _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, _vp]),
     "mesh_moe_top2_layer_workspace_bytes": (ctypes.c_size_t, [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int]),
@@ -1610,6 +1615,33 @@ def shared_linear_backward(x, dy):
         dw.data_ptr(), e, rows, k, n, dtype_code(x.dtype), ws.data_ptr(), ws_bytes,
         _stream()), "shared_linear_backward")
   return dw
+
+
+def shared_linear_backward_input_supported(dy, kernels):
+  """Whether shared_linear_backward_input takes dy [E, ..., N] and these kernels."""
+  e, n, k = dy.shape[0], dy.shape[-1], kernels[0].shape[0]
+  rows = dy[0].numel() // n
+  return (len(kernels) == e and rows < 1 << 31 and dy.is_contiguous() and
+          dy.dtype == torch.bfloat16 and dy.data_ptr() % 16 == 0 and
+          all(w.dtype == dy.dtype and w.shape == (k, n) and w.is_contiguous() and
+              w.device == dy.device and w.data_ptr() % 16 == 0 for w in kernels) and
+          load_library().mesh_moe_shared_linear_backward_input_supported(
+              e, rows, k, n, BF16) == 1)
+
+
+def shared_linear_backward_input(dy, kernels):
+  """The gradient of shared_linear's input: dy [E, ..., N], kernels E times [K, N] ->
+  [..., K], the sum over the layers in float32."""
+  lib = load_library()
+  e, n, k = dy.shape[0], dy.shape[-1], kernels[0].shape[0]
+  rows = dy[0].numel() // n
+  dx = torch.empty(tuple(dy.shape[1:-1]) + (k,), dtype=dy.dtype, device=dy.device)
+  pointers = (ctypes.c_void_p * e)(*[_dev(w, "w", dy.dtype, (k, n)) for w in kernels])
+  with _stage("expert_linear_backward"):
+    _check(lib.mesh_moe_shared_linear_backward_input(
+        _dev(dy, "dy"), ctypes.addressof(pointers), dx.data_ptr(), e, rows, k, n,
+        dtype_code(dy.dtype), _stream()), "shared_linear_backward_input")
+  return dx
 
 
 def fused_attention_applies(q, num_heads):

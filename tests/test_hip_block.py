@@ -1956,6 +1956,72 @@ def test_shared_linear(hip, rows, k, n):
       xt.abs() @ dy.abs())).all()
 
 
+# two and three parts of one K tile and of several; row tiles with three token slots,
+# lower and whole ones, a last one of one row; a partial last column tile
+@pytest.mark.parametrize("e,rows,k,n", [(2, 136, 256, 192), (3, 129, 264, 128),
+                                        (3, 700, 768, 768), (3, 9000, 520, 64),
+                                        (2, 16385, 256, 320), (3, 16384, 1024, 128)])
+def test_shared_linear_input_gradient(hip, e, rows, k, n):
+  """The parts of the reduction one after the other: the bits of one product over
+  operands that lie side by side."""
+  gen = torch.Generator(device="cuda").manual_seed(rows + k + n)
+  dy = torch.randn((e, rows, n), generator=gen, device="cuda").bfloat16()
+  kernels = [(torch.randn((k, n), generator=gen, device="cuda") / k ** 0.5).bfloat16()
+             for _ in range(e)][::-1]
+  assert hip.shared_linear_backward_input_supported(dy, kernels)
+  got = hip.shared_linear_backward_input(dy, kernels)
+  want = hip.dense(torch.cat(list(dy), 1), torch.cat(kernels, 1)[None].contiguous())
+  assert torch.equal(got, want)
+  assert not hip.shared_linear_backward_input_supported(dy, kernels[1:])
+  assert not hip.shared_linear_backward_input_supported(dy[:, :64].contiguous(),
+                                                        kernels)
+
+
+def test_input_gradient_of_shared_projections(monkeypatch):
+  """dx of layers of one input, summed in one product, against the sum of their
+  gradients: float32 sums instead of up to three bf16 roundings; a second step and one
+  that is asked for twice."""
+  rows, k, n = 300, 256, 192
+  gen = torch.Generator(device="cuda").manual_seed(5)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  rdim, kdim, ndim = (mtf.Dimension("rows", rows), mtf.Dimension("k", k),
+                      mtf.Dimension("n", n))
+  x = mtf.import_tf_tensor(mesh, _bf16_at(gen, False, rows, k),
+                           mtf.Shape([rdim, kdim]))
+  kernels = [mtf.get_variable(mesh, name, mtf.Shape([kdim, ndim]),
+                              dtype=torch.bfloat16) for name in "qkv"]
+  layers = [mtf_layers.DenseOperation(x, w, [ndim], None, name="dense_" + w.name)
+            for w in kernels]
+  mtf_layers.SharedInput(layers)
+  joint = _bf16_at(gen, False, 3, rows, n)
+  dys = [mtf.import_tf_tensor(mesh, part, mtf.Shape([rdim, ndim]))
+         for part in joint.unbind(0)]
+  init = {name: _bf16_at(gen, False, k, n) for name in "qkv"}
+  outs = [op.outputs[0] for op in layers]
+  first, = mtf.gradients(outs, [x], grad_ys=dys)
+  second, = mtf.gradients(outs, [x], grad_ys=dys)
+  some, = mtf.gradients(outs[1:], [x], grad_ys=dys[1:])
+  products = [joint[i].double() @ init[name].double().t().contiguous()
+              for i, name in enumerate("qkv")]
+  sizes = [joint[i].double().abs() @ init[name].double().abs().t().contiguous()
+           for i, name in enumerate("qkv")]
+  for joined in (True, False):
+    if not joined:
+      monkeypatch.setattr("mesh_amd.moe_hip.shared_linear_backward_input_supported",
+                          lambda *_: False)
+    low = mtf.Lowering(graph, {mesh: mtf.HipMeshImpl()}, initial_values=init)
+    for _ in range(2):
+      for grad, of in ((first, [0, 1, 2]), (second, [0, 1, 2]), (some, [1, 2])):
+        want = sum(products[i] for i in of)
+        # a rounding to bf16 of each product and of each sum, float32 sums below them
+        bound = sum(2.0 ** -7 * products[i].abs() + 3 * n * 2.0 ** -24 * sizes[i]
+                    for i in of) + 2.0 ** -8 * want.abs()
+        diff = (low.export_to_tf_tensor(grad).double() - want).abs()
+        assert (diff <= bound).all()
+      low.run()
+
+
 def test_shared_projections_see_assigned_weights():
   """The packed kernels that lie in one tensor follow assignments, eager and in a
   captured step."""
