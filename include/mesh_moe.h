@@ -964,11 +964,12 @@ size_t mesh_moe_self_attention_workspace_bytes(int B, int L, int H, int D,
  * transformer_layers.py:289-296 via attention.py:830-842), float32 softmax,
  * weights cast to dtype, outputs = weights . v.
  *   q, k, v, out [B,L,H*D] dtype (heads and d_kv combined as the reference's
- *   combine_dims does); any L and D (bf16 shapes whose L or D is not a
- *   multiple of 8 run their two products on a plain tile kernel).
- * bf16 with D = 64 or 128 runs one fused kernel (logits stay on chip, the
+ *   combine_dims does); any L and D (bf16 shapes of the three-step form whose L or D
+ *   is not a multiple of 8 run their two products on a plain tile kernel).
+ * bf16 with D = 64 or 128 and L >= 8 runs one fused kernel (logits stay on chip, the
  * division by the softmax sum comes after the weights are rounded; no scratch
- * but the bias table below).  Other cases run the three-step form whose logits
+ * but the bias table below, and room for copies of operands off 16 bytes, which are
+ * taken where L is no multiple of 8).  Other cases run the three-step form whose logits
  * and weights of all heads live in the workspace (B*H*L*L*(4 + sizeof dtype)
  * bytes).
  * sequence_id [B,L] int32 or NULL: with it a query sees only the keys that
@@ -1025,7 +1026,7 @@ size_t mesh_moe_self_attention_backward_workspace_bytes(int B, int L, int H,
  *   dW = dout . v^T,  delta = sum_k dW W,  dS = W (dW - delta) cast to dtype,
  *   dv = W^T . dout,  dq = dS . k,  dk = dS^T . q.
  *   q, k, v, dout, dq, dk, dv [B,L,H*D] dtype.
- * bf16 with D = 64 or 128 and L a multiple of 8 only (MESH_MOE_E_UNSUPPORTED
+ * bf16 with D = 64 or 128 and L at least 8 only (MESH_MOE_E_UNSUPPORTED
  * otherwise: compose mesh_moe_attention_weights, mesh_moe_softmax_backward and
  * mesh_moe_expert_linear_backward instead).  Nothing of size L x L reaches
  * memory; the workspace holds two float32 [B*H, L] vectors.  Four launches:

@@ -227,8 +227,16 @@ __device__ __forceinline__ void fa_visible_tiles(
 // the float32 logits: tab [H, 2L-1] holds, per head, the bias of every distance
 // key - query + L - 1.  A tile's logits need a window of BK + BQ - 1 entries of
 // it, which travels through LDS with the tile.
+// DIVIDED: the weights are divided by their sum before they are rounded, as the
+// reference and the three-step form do it.  That takes the maximum and the sum first, in
+// a walk over the keys of its own.  For lengths that are no multiple of 8, which had the
+// three-step form: rounded in the other order a weight is as exact, but nearly every
+// output moves by a bit of bf16, and units of a ReLU behind the attention whose sum is
+// next to zero switch (570 tokens: a value of the next layer's weight gradient by 0.9 of
+// the gradient's root mean square), so that steps of two versions could not be compared.
+// The first walk costs 9 us for 7 x 1385 tokens, 8 heads of 64, causal.
 template <int D, bool CAUSAL, bool STATS = false, bool SEQ = false,
-          bool BIAS = false>
+          bool BIAS = false, bool DIVIDED = false>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
     const bf16_t* __restrict__ v, bf16_t* __restrict__ out, int L, int H,
@@ -359,8 +367,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
   const int qw_first = q0 + wave * 32;
   const int kt_count = n_ktiles - kt_begin;
   load_k(kt_begin, 0);
-  load_v(kt_begin, 0);
-  if (BESIDE && kt_count > 1) load_k(kt_begin + 1, 1);
+  if constexpr (!DIVIDED) {
+    load_v(kt_begin, 0);
+    if (BESIDE && kt_count > 1) load_k(kt_begin + 1, 1);
+  }
   __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
   __syncthreads();
 
@@ -482,10 +492,14 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
   // (Weights relative to a maximum up to 2^8 too low would save nearly all of these
   // multiplications, 99 -> 93 us at 8 x 2048, 8 heads of 128, causal, but a query's
   // largest weight is then no longer 1, which bf16 holds exactly: 3 % more error.)
-  auto move_max = [&](float mx) {
+  auto both_halves_max = [&](float mx) {
     const auto both = __builtin_amdgcn_permlane32_swap(
         __float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+    return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+  };
+  auto move_max = [&](float mx) {
+    if constexpr (DIVIDED) return;          // m_run is what the first walk found
+    mx = both_halves_max(mx);
     const bool moves = mx > m_run;
     if (__ballot(moves) != 0ull) {
       const float m_new = moves ? mx : m_run;
@@ -506,6 +520,10 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     return mx;
   };
 
+  // (no visible key so far: the maximum is still the sentinel, and sentinel * log2e -
+  // sentinel * log2e would leave the product's rounding error, ~1e22, as the exponent)
+  auto exponent_of_max = [&](float m) { return m > 0.5f * NEG ? -m * LOG2E : -INFINITY; };
+
   // Tile `it`: its weights, beside the MFMAs of the next tile's logits, then its
   // share of the outputs, beside the next tile's maximum.  (BESIDE; otherwise its
   // logits and their maximum first, and nothing of the next tile but its loads.)
@@ -524,10 +542,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
       logits_of(kt, SLOT, acc_s);
       move_max(max_of(acc_s));
     }
-    // (no visible key so far: the maximum is still the sentinel, and sentinel *
-    // log2e - sentinel * log2e would leave the product's rounding error, ~1e22, as
-    // the exponent)
-    const float mneg = m_run > 0.5f * NEG ? -m_run * LOG2E : -INFINITY;
+    const float mneg = exponent_of_max(m_run);
     float psum = 0.f;
     uint32_t w[16];
     auto weights = [&](int i) {      // keys of registers 2 (i % 8) and + 1
@@ -608,6 +623,29 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     }
   };
   fa_f32x16_t acc_a[2], acc_b[2];
+  if constexpr (DIVIDED) {
+    for (int it = 0; it < kt_count; ++it) {
+      if (it + 1 < kt_count) load_k(kt_begin + it + 1, (it + 1) & 1);
+      logits_of(kt_begin + it, it & 1, acc_a);
+      const float m_new = fmaxf(m_run, both_halves_max(max_of(acc_a)));
+      const float mneg = exponent_of_max(m_new);
+      float psum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 32; ++i)
+        psum += fa_exp2(fmaf(acc_a[i >> 4][i & 15], LOG2E, mneg));
+      l_part = l_part * fa_exp2((m_run - m_new) * LOG2E) + psum;
+      m_run = m_new;
+      __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
+      __syncthreads();
+    }
+    // exp(logit - m_run) is the divided weight
+    m_run += logf(l_part + __shfl_xor(l_part, 32));
+    load_k(kt_begin, 0);
+    load_v(kt_begin, 0);
+    if (BESIDE && kt_count > 1) load_k(kt_begin + 1, 1);
+    __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
+    __syncthreads();
+  }
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   if constexpr (BESIDE) {
@@ -628,7 +666,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     tile(it, S0(), std::true_type(), acc_a, acc_b);
   }
 
-  const float l_all = l_part + __shfl_xor(l_part, 32);
+  const float l_all = DIVIDED ? 1.0f : l_part + __shfl_xor(l_part, 32);
   const float inv = 1.0f / l_all;
   if constexpr (STATS) {
     const bf16_t* drow = dout + ((int64_t)b * L + min(my_q, L - 1)) * row_stride +
@@ -674,7 +712,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
   }
 }
 
-template <int D, bool CAUSAL, bool SEQ, bool BIAS>
+template <int D, bool CAUSAL, bool SEQ, bool BIAS, bool DIVIDED>
 static int launch_flash_one(const bf16_t* q, const bf16_t* k, const bf16_t* v,
                             bf16_t* out, int B, int L, int H,
                             const int32_t* seq, const float* tab, float* lse,
@@ -682,7 +720,7 @@ static int launch_flash_one(const bf16_t* q, const bf16_t* k, const bf16_t* v,
   using Cfg = FlashCfg<D>;
   constexpr int LDS = Cfg::LDS_BYTES + 512 + 1536;  // + key ids, bias windows
   dim3 grid((unsigned)((L + Cfg::BQ - 1) / Cfg::BQ), (unsigned)(B * H));
-  auto kern = flash_attention_kernel<D, CAUSAL, false, SEQ, BIAS>;
+  auto kern = flash_attention_kernel<D, CAUSAL, false, SEQ, BIAS, DIVIDED>;
   MOE_ALLOW_LDS(kern, LDS);
   kern<<<grid, Cfg::THREADS, LDS, st>>>(q, k, v, out, L, H, nullptr, lse,
                                         nullptr, seq, tab);
@@ -709,9 +747,13 @@ static int launch_flash(const bf16_t* q, const bf16_t* k, const bf16_t* v,
                         hipStream_t st) {
   return flash_dispatch(causal != 0, seq != nullptr, tab != nullptr,
                         [&](auto c, auto s, auto bi) {
-    return launch_flash_one<D, decltype(c)::value, decltype(s)::value,
-                            decltype(bi)::value>(q, k, v, out, B, L, H, seq, tab,
-                                                 lse, st);
+    constexpr bool C = decltype(c)::value, S = decltype(s)::value,
+                   BI = decltype(bi)::value;
+    if (L % 8 != 0)
+      return launch_flash_one<D, C, S, BI, true>(q, k, v, out, B, L, H, seq, tab, lse,
+                                                 st);
+    return launch_flash_one<D, C, S, BI, false>(q, k, v, out, B, L, H, seq, tab, lse,
+                                                st);
   });
 }
 
@@ -741,10 +783,13 @@ static size_t relative_table_bytes(int L, int H) {
   return ((size_t)H * (2 * (size_t)L - 1) * sizeof(float) + 255) & ~(size_t)255;
 }
 
+// (Any length: a row is a multiple of 16 bytes, tiles are masked and clamped at its end.
+// Lengths that are no multiple of 8 took the three-step form, whose logits and weights
+// go through memory: a block of two attentions over 7 x 1385 tokens, 8 heads of 64, 2097
+// us a pass, now 340, a training step of one over 9 x 961 tokens 2747 and 825.)
 bool flash_attention_supported(int L, int H, int D, int dtype, const void* q,
                                const void* k, const void* v, const void* out) {
   return dtype == MESH_MOE_BF16 && (D == 64 || D == 128) && L >= 8 &&
-         L % 8 == 0 &&
          (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 ==
           0) && (int64_t)L * H * D < (1LL << 31);
 }

@@ -1190,13 +1190,34 @@ extern "C" int mesh_moe_rms_norm(const void* x, const void* scale, void* y,
   return 0;
 }
 
+// Operands off 16 bytes are refused where L is a multiple of 8; other lengths have always
+// been taken from anywhere, and are copied.
+static size_t aligned_copy_bytes(int B, int L, int H, int D) {
+  return ((size_t)B * L * H * D * sizeof(bf16_t) + 255) & ~(size_t)255;
+}
+__global__ __launch_bounds__(256) void copy_bf16_kernel(const bf16_t* __restrict__ from,
+                                                        bf16_t* __restrict__ to,
+                                                        int64_t n) {
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += step)
+    to[i] = from[i];
+}
+static int copy_bf16(const void* from, void* to, int64_t n, hipStream_t st) {
+  const int64_t blocks = (n + 255) / 256;
+  copy_bf16_kernel<<<(unsigned)(blocks < 65536 ? blocks : 65536), 256, 0, st>>>(
+      (const bf16_t*)from, (bf16_t*)to, n);
+  MOE_CHECK_LAUNCH("self_attention (aligned copy)");
+  return 0;
+}
+
 extern "C" size_t mesh_moe_self_attention_workspace_bytes(int B, int L, int H,
                                                           int D, int dtype,
                                                           int relative_bias) {
   if (B < 1 || L < 1 || H < 1 || D < 1 || !valid_dtype(dtype)) return 0;
   if (flash_attention_supported(L, H, D, dtype, nullptr, nullptr, nullptr,
                                 nullptr))
-    return flash_attention_workspace_bytes(B, L, H, D, relative_bias != 0);
+    return flash_attention_workspace_bytes(B, L, H, D, relative_bias != 0) +
+           (L % 8 != 0 ? 4 * aligned_copy_bytes(B, L, H, D) : 0);
   const size_t b = dtype_size(dtype);
   const size_t hd = (size_t)B * H * L * D, ll = (size_t)B * H * L * L;
   return 4 * hd * b + ll * 4 + ll * b + 7 * 256;
@@ -1232,16 +1253,29 @@ extern "C" int mesh_moe_self_attention(const void* q, const void* k,
   if (flash_attention_supported(L, H, D, dtype, nullptr, nullptr, nullptr,
                                 nullptr)) {
     // fused kernel: the logits stay on chip
-    MOE_REQUIRE(flash_attention_supported(L, H, D, dtype, q, k, v, out),
-                MESH_MOE_E_UNSUPPORTED,
+    const bool aligned = flash_attention_supported(L, H, D, dtype, q, k, v, out);
+    MOE_REQUIRE(aligned || L % 8 != 0, MESH_MOE_E_UNSUPPORTED,
                 "self_attention: q, k, v, out must be 16-byte aligned");
+    if (!aligned) {
+      const int64_t n = (int64_t)B * L * H * D;
+      const size_t each = aligned_copy_bytes(B, L, H, D);
+      char* at = (char*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+      const void* from[3] = {q, k, v};
+      for (int i = 0; i < 3; ++i)
+        if (int rc = copy_bf16(from[i], at + i * each, n, st)) return rc;
+      if (int rc = flash_attention(at, at + each, at + 2 * each, at + 3 * each, B, L, H,
+                                   D, causal ? 1 : 0, sequence_id, rel_values,
+                                   rel_bucket, num_buckets, lse, at + 4 * each, st))
+        return rc;
+      return copy_bf16(at + 3 * each, out, n, st);
+    }
     return flash_attention(q, k, v, out, B, L, H, D, causal ? 1 : 0,
                            sequence_id, rel_values, rel_bucket, num_buckets,
                            lse, workspace, st);
   }
   MOE_REQUIRE(lse == nullptr, MESH_MOE_E_UNSUPPORTED,
               "self_attention: lse is written by the fused kernel only (bf16, "
-              "d_kv 64 or 128, L a multiple of 8)");
+              "d_kv 64 or 128, L at least 8)");
   if (dtype == MESH_MOE_F32)
     return run_attention<float>((const float*)q, (const float*)k,
                                 (const float*)v, (float*)out, B, L, H, D,
@@ -1598,7 +1632,7 @@ extern "C" int mesh_moe_self_attention_backward(
                   flash_attention_supported(L, H, D, dtype, dq, dk, dv, dout),
               MESH_MOE_E_UNSUPPORTED,
               "self_attention_backward: the fused kernels take bf16, d_kv 64 or "
-              "128, L a multiple of 8 and 16-byte aligned tensors (L=%d D=%d)",
+              "128, L at least 8 and 16-byte aligned tensors (L=%d D=%d)",
               L, D);
   MOE_REQUIRE(workspace_bytes >= flash_attention_backward_workspace_bytes(
                                      B, L, H, rel_values != nullptr),

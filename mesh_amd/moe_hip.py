@@ -1930,7 +1930,7 @@ def self_attention_backward(q, k, v, dout, num_heads, causal, fused=None,
                             sequence_id=None, relative_bias=None, out=None,
                             lse=None):
   """Backward of self_attention: q, k, v, dout [B, L, H*D] -> (dq, dk, dv).
-  Shapes the fused kernels take (bf16, d_kv 64 or 128, L a multiple of 8) run
+  Shapes the fused kernels take (bf16, d_kv 64 or 128, L at least 8) run
   mesh_moe_self_attention_backward: nothing [L, L] reaches memory.  Otherwise
   (or with fused=False) the weights are recomputed ([B*H, L, L]) and every
   product runs on the grouped GEMM with one (batch, head) pair per group:
@@ -1953,6 +1953,11 @@ def self_attention_backward(q, k, v, dout, num_heads, causal, fused=None,
     ws_bytes = lib.mesh_moe_self_attention_backward_workspace_bytes(
         b, l, h, d, code, int(relative_bias is not None))
     if ws_bytes:
+      if l % 8:
+        # (the fused kernels need 16 bytes; these lengths are taken from anywhere)
+        q, k, v, dout, out = (
+            t.clone() if t is not None and t.data_ptr() % 16 else t
+            for t in (q, k, v, dout, out))
       ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device)
       # (one allocation: the projections' weight gradients are one launch then)
       dq, dk, dv = torch.empty((3,) + tuple(q.shape), dtype=q.dtype,

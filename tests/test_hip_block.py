@@ -164,8 +164,8 @@ def _packed_sequence_ids(rng, b, l, mean_len):
                          ids=lambda c: "x".join(map(str, c)))
 def test_self_attention_sequence_ids_in_any_order(hip, case, causal, with_bias):
   """Ids that come back later in the row, that are equal modulo 64, negative
-  ones and a single position of its own, at lengths of a single tile or that the
-  fused kernels do not take (no multiple of 8: the three-step form)."""
+  ones and a single position of its own, at lengths of a single tile or that end one
+  to three positions into a tile."""
   l, d = case
   b, heads, nb = 3, 1, 8
   rng = np.random.default_rng(l + d + causal)
@@ -599,6 +599,61 @@ def test_self_attention_relative_bias(hip, case, causal, act_dtype):
   # not the same as no bias
   plain = H.to_np(hip.self_attention(g(q), g(k), g(v), heads, causal))
   assert np.abs(plain - got).max() > 1e-2
+
+
+@pytest.mark.parametrize("with_ids_and_bias", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("length,d", [(9, 64), (63, 128), (65, 64), (127, 64),
+                                      (129, 128), (257, 64), (257, 128), (771, 64)])
+def test_fused_attention_of_any_length(hip, length, d, causal, with_ids_and_bias):
+  """Lengths that end one to seven positions before or behind a tile's last one, with
+  and without kept denominators, and operands off 16 bytes: against the oracle and, as
+  far from float64, the three-step form."""
+  b, heads, nb = 2, 2, 8
+  rng = np.random.default_rng(length + d + causal)
+  mk = lambda *sizes: O.cast_act(
+      (rng.standard_normal(sizes) * 0.5).astype(np.float32), "bfloat16")
+  q, k, v, do = (mk(b, length, heads * d) for _ in range(4))
+  ids = values = sid = rel = None
+  if with_ids_and_bias:
+    ids = _packed_sequence_ids(rng, b, length, max(4, length // 3))
+    values = mk(heads, nb)
+    bucket = B.relative_position_bucket(np.arange(-(length - 1), length), not causal,
+                                        nb)
+    sid = torch.from_numpy(ids).cuda()
+    rel = (H.to_gpu(values, "bfloat16"), torch.from_numpy(bucket.astype(np.int32)).cuda())
+  args = [H.to_gpu(t, "bfloat16") for t in (q, k, v, do)]
+  assert hip.fused_attention_applies(args[0], heads)
+  kw = dict(sequence_id=sid, relative_bias=rel)
+  out, lse = hip.self_attention(*args[:3], heads, causal, return_lse=True, **kw)
+  want = B._attention_core(q, k, v, heads, causal, "bfloat16", sequence_id=ids,
+                           relative_values=values)
+  np.testing.assert_allclose(H.to_np(out), want, **_tol("bfloat16"))
+  exact = B._attention_core(q, k, v, heads, causal, "float32", sequence_id=ids,
+                            relative_values=values)
+  weights = H.to_np(hip.attention_weights(*args[:2], heads, causal, sid, rel))
+  v4 = v.reshape(b, length, heads, d)
+  three = O.cast_act(np.einsum("bhlm,bmhd->blhd", weights.reshape(
+      b, heads, length, length), v4).astype(np.float32), "bfloat16").reshape(q.shape)
+  error = lambda t: np.linalg.norm(t - exact)
+  # (both round every weight and every output once: the same error but for chance)
+  assert error(H.to_np(out)) <= 1.1 * error(three)
+  want = B.attention_core_backward(q, k, v, do, heads, causal, "bfloat16",
+                                   sequence_id=ids, relative_values=values)
+  def off_16(t):
+    moved = torch.empty(t.numel() + 8, dtype=t.dtype, device="cuda")
+    moved = moved[1:1 + t.numel()].view(t.shape)
+    moved.copy_(t)
+    return moved
+  moved = [off_16(t) for t in args]
+  assert torch.equal(hip.self_attention(*moved[:3], heads, causal, **kw), out)
+  for grads in (
+      hip.self_attention_backward(*args, heads, causal, fused=True, **kw),
+      hip.self_attention_backward(*args, heads, causal, out=out, lse=lse, **kw),
+      hip.self_attention_backward(*moved, heads, causal, **kw)):
+    for gt, wnt in zip(grads, want):
+      scale = max(1.0, float(np.abs(wnt).max()))
+      np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
 
 
 @pytest.mark.parametrize("causal", [False, True])
