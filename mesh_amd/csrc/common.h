@@ -32,6 +32,14 @@ bool f32_gemm_applies(int R, int N, int K);
 int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int K,
              bool kmajor, bool relu, const float* mask_src, float mask_scale,
              hipStream_t st);
+// A[e] . B[e]^T for fewer than 32 rows of A, A[e]^T . B[e] over fewer than 32 rows of both
+// (16-byte alignment): chains of multiply-adds in ascending k.
+bool f32_few_rows_applies(int R, int N, int K);
+int f32_few_rows(const float* A, const float* B, float* C, int E, int R, int N, int K,
+                 bool relu, const float* mask_src, float mask_scale, hipStream_t st);
+bool f32_few_k_applies(int R, int N, int K);
+int f32_few_k(const float* A, const float* B, float* C, int E, int R, int N, int K,
+              hipStream_t st);
 // A[e] . B[e]^T (the operands and limits of f32_gemm) with sums whose bits do not
 // change from one version of f32_gemm to the next.
 int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int N,

@@ -2338,6 +2338,13 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
         rc = f32_gemm((const float*)A, (const float*)B, (float*)C, E, R, N, K, false,
                       relu, mask, mask_scale, st);
       if (masks) *mask_applied = rc == 0;
+    } else if (f32_few_rows_applies(R, N, K) &&
+               ((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0) {
+      const bool masks = relu_mask_src != nullptr && mask_applied != nullptr &&
+                         !relu && ((uintptr_t)relu_mask_src % 16) == 0;
+      rc = f32_few_rows((const float*)A, (const float*)B, (float*)C, E, R, N, K, relu,
+                        masks ? (const float*)relu_mask_src : nullptr, mask_scale, st);
+      if (masks) *mask_applied = rc == 0;
     } else
       rc = launch_simple<float>((const float*)A, (const float*)B, (float*)C, E,
                                 R, N, K, relu, st);
@@ -2378,13 +2385,20 @@ static int grouped_gemm(const void* A, const void* B, void* C, int E, int R,
   return 0;
 }
 
-// C[e] = A[e]^T . B[e] in float32, A [K, R] and B [K, N]: what f32_gemm takes with
-// operands as they lie.
+// C[e] = A[e]^T . B[e] in float32, A [K, R] and B [K, N]: what f32_gemm and f32_few_k take
+// with operands as they lie.
 static bool f32_kmajor_applies(const void* A, const void* B, const void* C,
                                int R, int N, int K, int dtype) {
   return dtype == MESH_MOE_F32 && R % 4 == 0 && N % 4 == 0 &&
-         f32_gemm_applies(R, N, K) &&
+         (f32_gemm_applies(R, N, K) || f32_few_k_applies(R, N, K)) &&
          ((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) % 16 == 0;
+}
+static int f32_kmajor(const void* A, const void* B, void* C, int E, int R, int N, int K,
+                      hipStream_t st) {
+  if (f32_few_k_applies(R, N, K))
+    return f32_few_k((const float*)A, (const float*)B, (float*)C, E, R, N, K, st);
+  return f32_gemm((const float*)A, (const float*)B, (float*)C, E, R, N, K, true, false,
+                  nullptr, 1.f, st);
 }
 
 // Batched C[e] = A[e] . B[e]^T for the other source files (attention): `dtype`
@@ -3094,8 +3108,7 @@ extern "C" int mesh_moe_expert_linear_backward(
                               E, K, N, R, st, nullptr,
                               (void*)up((uintptr_t)workspace));
   if (f32_kmajor_applies(a, dy, dw, K, N, R, dtype))
-    return f32_gemm((const float*)a, (const float*)dy, (float*)dw, E, K, N, R, true,
-                    false, nullptr, 1.f, st);
+    return f32_kmajor(a, dy, dw, E, K, N, R, st);
   const size_t es = dtype_size(dtype);
   unsigned char* tr_a = (unsigned char*)up((uintptr_t)workspace);
   unsigned char* tr_dy =
@@ -3205,11 +3218,9 @@ extern "C" int mesh_moe_expert_ffn_backward(
   }
   if (f32_kmajor_applies(h, dy, dwo, H, N, R, dtype) &&
       f32_kmajor_applies(expert_in, dh, dwi, M, H, R, dtype)) {
-    rc = f32_gemm((const float*)h, (const float*)dy, (float*)dwo, E, H, N, R, true,
-                  false, nullptr, 1.f, st);
+    rc = f32_kmajor(h, dy, dwo, E, H, N, R, st);
     if (rc != 0) return rc;
-    return f32_gemm((const float*)expert_in, (const float*)dh, (float*)dwi, E, M, H,
-                    R, true, false, nullptr, 1.f, st);
+    return f32_kmajor(expert_in, dh, dwi, E, M, H, R, st);
   }
   // otherwise: both operands transposed to token-contiguous copies first
   rc = mesh_moe_pack_weights(h, tr_h, E, R, H, dtype, dtype, stream);

@@ -644,6 +644,243 @@ int f32_gemm(const float* A, const float* B, float* C, int E, int R, int N, int 
 }
 
 // ---------------------------------------------------------------------------
+// Few rows per expert (fewer than 32), C[e] = act(A[e] . B[e]^T): small batches, whose
+// time is that of reading the weights.  A wavefront takes all rows and 16 TN columns and
+// walks k by itself on v_mfma_f32_16x16x4_f32, whose sums are a chain of multiply-adds in
+// ascending k: the bits of grouped_gemm_simple_kernel, which had these products on 64 x
+// 64 tiles of plain multiply-adds.  (So a hidden tensor that is kept for a gradient has
+// one set of sums, see below.)  A lane loads 16 bytes, four consecutive k of its row; an
+// MFMA wants one k of each lane group, so the four registers and the four groups change
+// places (v_permlane32_swap, v_permlane16_swap).  DEPTH groups of 16 k are on their way.
+// A layer of 85 tokens, 8 experts, 832 -> 1664 -> 832 (21 rows each) 364 -> 89 us, of
+// which the two products are 18 and 32; 407 tokens, 48 experts, 640 -> 2560, a training
+// step 1558 -> 587, its four products 82 to 123 us for 315 MB of weights each.  What is
+// left to the read rate is rows of one stride that all wavefronts walk in step (another
+// first k per wavefront would be another order of the sums).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void swap_groups(float (&v)[4]) {
+  auto swap32 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b),
+                                                    false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  };
+  auto swap16 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b),
+                                                    false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  };
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
+
+template <int RT, int TN>
+__global__ __launch_bounds__(256) void f32_few_rows_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ Cout,
+    int R, int N, int K, int col_blocks, int relu, const float* __restrict__ mask_src,
+    float mask_scale) {
+  constexpr int DEPTH = RT + TN == 2 ? 10 : RT + TN == 3 ? 8 : 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int e = blockIdx.x / col_blocks;
+  const int col0 = ((blockIdx.x - e * col_blocks) * 4 + wave) * 16 * TN;
+  if (col0 >= N) return;
+  const int c = lane & 15, g = lane >> 4;
+  // (rows and columns past the end are read as the last one and not stored)
+  const float *a_row[RT], *b_row[TN];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+    a_row[i] = A + ((int64_t)e * R + min(16 * i + c, R - 1)) * K;
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+    b_row[j] = B + ((int64_t)e * N + min(col0 + 16 * j + c, N - 1)) * K;
+  f32x4_t a_raw[DEPTH][RT], b_raw[DEPTH][TN];
+  auto load = [&](int chunk, auto slot_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+    const int k = min(16 * chunk + 4 * g, K - 4);
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      b_raw[SLOT][j] = *reinterpret_cast<const f32x4_t*>(b_row[j] + k);
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+      a_raw[SLOT][i] = *reinterpret_cast<const f32x4_t*>(a_row[i] + k);
+  };
+  f32x4_t acc[RT][TN];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+  auto multiply = [&](int chunk, auto slot_c, auto whole_c) {
+    constexpr int SLOT = decltype(slot_c)::value;
+    constexpr bool WHOLE = decltype(whole_c)::value;
+    float a[RT][4], b[TN][4];
+    const bool mine = 16 * chunk + 4 * g < K;
+    auto take = [&](f32x4_t v, float (&to)[4]) {
+      // (the four values stay together till here: taken apart where they are loaded,
+      // the compiler waits for them there)
+      asm volatile("" : "+v"(v));
+      to[0] = v[0]; to[1] = v[1]; to[2] = v[2]; to[3] = v[3];
+      if constexpr (!WHOLE)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) to[q] = mine ? to[q] : 0.f;
+      swap_groups(to);
+    };
+#pragma unroll
+    for (int i = 0; i < RT; ++i) take(a_raw[SLOT][i], a[i]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) take(b_raw[SLOT][j], b[j]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][q], a[i][q], acc[i][j],
+                                                           0, 0, 0);
+  };
+  // (a branch between the loads would wait for all of them)
+  const int chunks = (K + 15) / 16;
+  int first = 0;
+  for_each_index<DEPTH>([&](auto u) { load(decltype(u)::value, u); });
+  for (; first + DEPTH <= K / 16; first += DEPTH)
+    for_each_index<DEPTH>([&](auto u) {
+      const int chunk = first + decltype(u)::value;
+      multiply(chunk, u, std::true_type());
+      load(chunk + DEPTH, u);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  for_each_index<DEPTH>([&](auto u) {
+    const int chunk = first + decltype(u)::value;
+    if (chunk < chunks) multiply(chunk, u, std::false_type());
+  });
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int row = 16 * i + c, col = col0 + 16 * j + 4 * g;
+      if (row >= R || col >= N) continue;
+      const int64_t at = ((int64_t)e * R + row) * N + col;
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[q] = acc[i][j][q];
+        if (relu) v[q] = v[q] > 0.f ? v[q] : 0.f;
+      }
+      if (mask_src != nullptr) {
+        const float4 m = *reinterpret_cast<const float4*>(mask_src + at);
+        const float mv[4] = {m.x, m.y, m.z, m.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = finish_f32(v[q], false, true, mv[q], mask_scale);
+      }
+      *reinterpret_cast<float4*>(Cout + at) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+bool f32_few_rows_applies(int R, int N, int K) {
+  return R >= 1 && R < 32 && N >= 16 && K >= 16 && N % 4 == 0 && K % 4 == 0;
+}
+
+int f32_few_rows(const float* A, const float* B, float* C, int E, int R, int N, int K,
+                 bool relu, const float* mask_src, float mask_scale, hipStream_t st) {
+  const int cus = compute_units();
+  if (cus == 0) return MESH_MOE_E_HIP;
+  // two column tiles per wavefront, which share the rows' loads, once every SIMD has two
+  // wavefronts anyway
+  const bool two = (int64_t)E * ((N + 15) / 16) >= (int64_t)16 * cus;
+  const int col_blocks = (N + (two ? 127 : 63)) / (two ? 128 : 64);
+  const int64_t blocks = (int64_t)E * col_blocks;
+  MOE_REQUIRE(blocks <= 0x7fffffffLL, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: too many tiles (%lld)", (long long)blocks);
+  auto run = [&](auto k) {
+    k<<<(unsigned)blocks, 256, 0, st>>>(A, B, C, R, N, K, col_blocks, relu ? 1 : 0,
+                                        mask_src, mask_scale);
+    MOE_CHECK_LAUNCH("expert_ffn (float32, few rows)");
+    return 0;
+  };
+  if (R <= 16) return two ? run(f32_few_rows_kernel<1, 2>) : run(f32_few_rows_kernel<1, 1>);
+  return two ? run(f32_few_rows_kernel<2, 2>) : run(f32_few_rows_kernel<2, 1>);
+}
+
+// Their weight gradients, C[e] = A[e]^T . B[e] over fewer than 32 rows (A [K][R], B
+// [K][N]): bound by the stores.  A wavefront makes 64 x 64 outputs from one load of 16
+// bytes per operand and four rows; the register of a load picks the column, so that a
+// lane ends up with four consecutive outputs and a store is four whole rows of 256 bytes.
+// The sums are chains of multiply-adds over 16 or 32 rows (zeros behind the last one):
+// the bits of grouped_gemm_simple_kernel on transposed copies, which these were before.
+// 48 experts, 10 rows, 640 x 2560: 65 us, 4.8 TB/s.
+template <int KS>
+__global__ __launch_bounds__(256) void f32_few_k_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ Cout,
+    int R, int N, int K, int tiles_m, int tiles_n) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tiles = tiles_m * tiles_n, e = blockIdx.x / tiles;
+  const int rem = blockIdx.x - e * tiles, tm = rem / tiles_n, tn = rem - tm * tiles_n;
+  const int row0 = tm * 64, col0 = (tn * 4 + wave) * 64;
+  if (col0 >= N) return;
+  const int c = lane & 15, g = lane >> 4;
+  const float* a_at = A + (int64_t)e * K * R + min(row0 + 4 * c, R - 4);
+  const float* b_at = B + (int64_t)e * K * N + min(col0 + 4 * c, N - 4);
+  float4 a[KS], b[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int64_t k = min(4 * s + g, K - 1);
+    a[s] = *reinterpret_cast<const float4*>(a_at + k * R);
+    b[s] = *reinterpret_cast<const float4*>(b_at + k * N);
+  }
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const bool there = 4 * s + g < K;
+    const float av[4] = {there ? a[s].x : 0.f, there ? a[s].y : 0.f,
+                         there ? a[s].z : 0.f, there ? a[s].w : 0.f};
+    const float bv[4] = {there ? b[s].x : 0.f, there ? b[s].y : 0.f,
+                         there ? b[s].z : 0.f, there ? b[s].w : 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+  }
+  const int col = col0 + 4 * c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = row0 + 16 * g + 4 * r + i;
+      if (row < R && col < N)
+        *reinterpret_cast<float4*>(Cout + ((int64_t)e * R + row) * N + col) =
+            make_float4(acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]);
+    }
+}
+
+bool f32_few_k_applies(int R, int N, int K) {
+  return K >= 1 && K < 32 && R >= 16 && N >= 16 && R % 4 == 0 && N % 4 == 0;
+}
+
+int f32_few_k(const float* A, const float* B, float* C, int E, int R, int N, int K,
+              hipStream_t st) {
+  const int64_t tiles_m = ((int64_t)R + 63) / 64, tiles_n = ((int64_t)N + 255) / 256;
+  MOE_REQUIRE((int64_t)E * tiles_m <= 0x7fffffffLL / tiles_n, MESH_MOE_E_UNSUPPORTED,
+              "expert_ffn: too many tiles (%lld a expert)", (long long)(tiles_m * tiles_n));
+  const unsigned blocks = (unsigned)(E * tiles_m * tiles_n);
+  auto k = K <= 16 ? f32_few_k_kernel<4> : f32_few_k_kernel<8>;
+  k<<<blocks, 256, 0, st>>>(A, B, C, R, N, K, (int)tiles_m, (int)tiles_n);
+  MOE_CHECK_LAUNCH("expert_ffn (float32, sums over few rows)");
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
 // Sums that do not change: v_mfma_f32_32x32x2_f32, true float32 operands, the
 // order of k and the tiles these products have always had.
 //

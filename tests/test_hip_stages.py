@@ -1866,6 +1866,46 @@ def test_linear_row_tiles(hip, shape):
   assert torch.equal(da, hip.expert_linear(dy, w))
 
 
+def _off_16(t):
+  moved = torch.empty(t.numel() + 4, dtype=t.dtype, device="cuda")
+  moved = moved[1:1 + t.numel()].view(t.shape)
+  moved.copy_(t)
+  return moved
+
+
+# one and two row tiles; one and two column tiles per wavefront; partial row and column
+# tiles; reductions that end inside a group of 16 and are shorter than the loads ahead
+@pytest.mark.parametrize("rows", [1, 3, 16, 17, 31])
+@pytest.mark.parametrize("e,k,n", [(3, 16, 20), (2, 20, 16), (5, 52, 260), (2, 832, 132),
+                                   (70, 192, 1000), (140, 100, 512)])
+def test_float32_few_rows(hip, e, k, n, rows):
+  """Fewer than 32 float32 rows per expert: products, masked ones and weight gradients
+  have the bits of the kernel that takes operands off 16 bytes, which adds with one
+  chain of multiply-adds; also where products underflow."""
+  gen = torch.Generator(device="cuda").manual_seed(e + k + n + rows)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  for scale in (1.0, 2.0 ** -70):
+    a, w, dy = mk(e, rows, k) * scale, mk(e, n, k) * scale, mk(e, rows, n) * scale
+    for act in ("linear", "relu"):
+      assert torch.equal(hip.expert_linear(a, w, act),
+                         hip.expert_linear(_off_16(a), w, act))
+    wt = w.transpose(1, 2).contiguous()
+    mask = mk(e, rows, k)
+    got = hip.expert_linear_backward(a, dy, wt, da_relu_mask=mask)
+    want = hip.expert_linear_backward(_off_16(a), _off_16(dy), wt, da_relu_mask=mask)
+    for g, x in zip(got, want):
+      assert torch.equal(g, x)
+    assert bool((got[0][mask <= 0] == 0).all())
+  # (and they are the products: float32 sums of k and of the rows)
+  a, w, dy = (t.double() for t in (a, w, dy))
+  t = lambda x: x.transpose(1, 2).contiguous()
+  y = hip.expert_linear(a.float(), w.float()).double()
+  assert ((y - a @ t(w)).abs() <= k * 2.0 ** -24 * (a.abs() @ t(w).abs()) + 1e-43).all()
+  dw = got[1].double()
+  assert ((dw - t(a) @ dy).abs() <=
+          rows * 2.0 ** -24 * (t(a).abs() @ dy.abs()) + 1e-43).all()
+
+
 @pytest.mark.parametrize("k", [64, 128, 192, 448])
 @pytest.mark.parametrize("e,rows,n", [(130, 129, 520), (200, 257, 520),
                                       (64, 260, 1024), (20, 290, 264), (9, 150, 264)])
