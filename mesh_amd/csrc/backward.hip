@@ -1076,7 +1076,7 @@ __global__ __launch_bounds__(256) void gating_backward_rows_kernel(
 // the staged ones are multiplied.  Every block writes its sums to its token
 // chunk's [M, E] plane of the workspace and router_wgrad_reduce_kernel adds
 // the planes in chunk order: the same bits on every run.
-// Needs M % 4 == 0, E % 4 == 0 and 16-byte aligned rows.
+// Needs M % 4 == 0 and 16-byte aligned rows of x.
 //
 // The product is short of blocks, not of bandwidth: 2048 tokens per block
 // left 30 blocks of 64 dependent steps for 9000 x 768 tokens and 16 experts
@@ -1096,6 +1096,26 @@ __device__ __forceinline__ uint4 load_or_zero(const uint4* p, bool in) {
   uint4 v = make_uint4(0, 0, 0, 0);
   if (in) v = *p;
   return v;
+}
+
+// Eight d(logits) of a token from expert e on, zeros past the last expert.  Rows of E % 4
+// == 0 experts start on 16 bytes; others are read one by one, which 32 tokens at a time
+// with the next ones on their way hide.
+__device__ __forceinline__ void load_dlogits8(const float* __restrict__ row, int e, int E,
+                                              bool in, uint4& a, uint4& b) {
+  if (E % 4 == 0) {
+    a = load_or_zero(reinterpret_cast<const uint4*>(row + e), in && e < E);
+    b = load_or_zero(reinterpret_cast<const uint4*>(row + e + 4), in && e + 4 < E);
+    return;
+  }
+  uint32_t v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    v[q] = 0;
+    if (in && e + q < E) v[q] = __float_as_uint(row[e + q]);
+  }
+  a = make_uint4(v[0], v[1], v[2], v[3]);
+  b = make_uint4(v[4], v[5], v[6], v[7]);
 }
 
 // Tokens per block of the two kernels below: about 512 blocks (two per compute
@@ -1139,11 +1159,7 @@ __global__ __launch_bounds__(256) void router_wgrad_mfma_kernel(
       xraw[u] = load_or_zero(
           reinterpret_cast<const uint4*>(x + t * M + m0 + sc * 16 + u * VN),
           t < t1 && m0 + sc * 16 + u * VN < M);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-      draw[u] = load_or_zero(
-          reinterpret_cast<const uint4*>(dlogits + t * E + e0 + sc * 8 + u * 4),
-          t < t1 && e0 + sc * 8 + u * 4 < E);
+    load_dlogits8(dlogits + t * E, e0 + sc * 8, E, t < t1, draw[0], draw[1]);
   };
   load(t0);
   for (int64_t tb = t0; tb < t1; tb += WM_KT) {
@@ -1244,11 +1260,9 @@ __global__ __launch_bounds__(256) void router_wgrad_bf16_kernel(
     const bool in = t < t1;
     const int m = m0 + sc * 16, e = e0 + sc * 8;
     const uint4* xp = reinterpret_cast<const uint4*>(x + t * M + m);
-    const uint4* dp = reinterpret_cast<const uint4*>(dlogits + t * E + e);
     xv0 = load_or_zero(xp, in && m < M);
     xv1 = load_or_zero(xp + 1, in && m + 8 < M);
-    da = load_or_zero(dp, in && e < E);
-    db = load_or_zero(dp + 1, in && e + 4 < E);
+    load_dlogits8(dlogits + t * E, e, E, in, da, db);
   };
   load(t0);
   for (int64_t tb = t0; tb < t1; tb += WB_KT) {
@@ -1815,10 +1829,12 @@ extern "C" int mesh_moe_gating_backward(
       dgate, d_loss, counts, n_one, dlogits, st);
 }
 
-// the matrix-core kernels take the sizes (operands still have to be aligned)
+// The matrix-core kernels take the sizes (operands still have to be aligned).  (Experts
+// that are no multiple of 4 took the kernel with atomics, 64 experts at a time: 6664 tokens
+// of 1280, 2 experts, 634 us, now 11 + 5.)
 static bool router_wgrad_mfma_applies(int64_t tokens, int M, int E, int dtype) {
   const int chunk = router_wgrad_chunk(tokens, M, E, dtype);
-  return ((size_t)M * dtype_size(dtype)) % 16 == 0 && E % 4 == 0 &&
+  return ((size_t)M * dtype_size(dtype)) % 16 == 0 &&
          (tokens + chunk - 1) / chunk <= 65535 && (E + 63) / 64 <= 65535;
 }
 

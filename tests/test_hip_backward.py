@@ -523,6 +523,21 @@ def test_router_backward_weights_sizes(hip, shape, act_dtype):
   test_router_backward_weights(hip, shape, act_dtype)
 
 
+@pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("shape", [(6664, 1280, 2), (33, 8, 1), (700, 136, 3),
+                                   (2000, 256, 7), (500, 128, 65)])
+def test_router_backward_weights_of_any_expert_count(hip, shape, act_dtype):
+  """Rows of d(logits) that do not start on 16 bytes; the same bits on every run."""
+  test_router_backward_weights(hip, shape, act_dtype)
+  t, m, e = shape
+  gen = torch.Generator(device="cuda").manual_seed(e)
+  x = torch.randn((t, m), generator=gen, device="cuda").to(
+      torch.float32 if act_dtype == "float32" else torch.bfloat16)
+  dl = torch.randn((t, e), generator=gen, device="cuda")
+  assert torch.equal(hip.router_backward_weights(x, dl),
+                     hip.router_backward_weights(x, dl))
+
+
 @pytest.mark.parametrize("e", [8, 512])
 def test_router_backward_weights_float32_sums_stay_short(hip, e):
   """No float32 sum runs over more than 512 tokens before the chunks' sums are
