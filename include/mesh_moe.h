@@ -342,6 +342,17 @@ int mesh_moe_dispatched_expert_ffn(
     const uint8_t* kept, const void* wi_packed, const void* wo_packed, void* h,
     void* y, void* workspace, size_t workspace_bytes, int G, int S, int E, int C,
     int M, int H, int N, int activation, int dtype, void* stream);
+/* The same where every expert has `outer` kernels, wi_packed [E*outer,H,M] and wo_packed
+ * [E*outer,N,H], kernel e * outer + o for the groups from o * G / outer on (the inner level
+ * of transformer_moe_layer_v2, transformer/moe.py:743-793): y [E*outer, G/outer*C, N].
+ * fill [G,E] as the gating left it.  No kernel for at most 64 rows per expert. */
+int mesh_moe_dispatched_outer_expert_ffn(
+    const void* x, const int32_t* idx, const int32_t* pos, const float* gate,
+    const uint8_t* kept, const int32_t* fill, const void* wi_packed,
+    const void* wo_packed, void* h, void* y, void* workspace, size_t workspace_bytes,
+    int G, int S, int E, int C, int outer, int M, int H, int N, int activation, int dtype,
+    void* stream);
+
 
 /*
  * Combine: out[g,s,:] = w1 * y[idx1,g,pos1,:] + w2 * y[idx2,g,pos2,:] with

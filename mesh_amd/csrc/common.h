@@ -66,7 +66,7 @@ int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
                    bool map_made, const void* wi_packed, const void* wo_packed, void* h,
                    void* y, void* workspace, size_t workspace_bytes, int G, int S,
                    int E, int C, int M, int H, int N, int activation, int dtype,
-                   void* stream);
+                   void* stream, int outer = 1);
 // whether those calls take the kernels for few rows, which read the map at once
 bool dispatched_few_rows(int G, int S, int E, int C, int M, int H);
 

@@ -2759,7 +2759,7 @@ int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
                    bool map_made, const void* wi_packed, const void* wo_packed, void* h,
                    void* y, void* workspace, size_t workspace_bytes, int G, int S,
                    int E, int C, int M, int H, int N, int activation, int dtype,
-                   void* stream) {
+                   void* stream, int outer) {
   MOE_REQUIRE(x && idx && pos && gate && kept && wi_packed && wo_packed && h &&
                   y && workspace, MESH_MOE_E_ARG,
               "dispatched_expert_ffn: null pointer");
@@ -2769,8 +2769,13 @@ int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
                   activation <= MESH_MOE_ACT_SWISH,
               MESH_MOE_E_ARG, "dispatched_expert_ffn: unknown activation %d",
               activation);
-  const int64_t rows = (int64_t)G * C;
-  const bool few_rows = dispatched_few_rows(G, S, E, C, M, H) &&
+  MOE_REQUIRE(outer >= 1 && G % outer == 0 && (int64_t)E * outer <= 0x7fffffff,
+              MESH_MOE_E_ARG, "dispatched_expert_ffn: %d groups in %d outer parts", G,
+              outer);
+  // outer > 1: every expert has that many kernels, one for G / outer groups in a row, and
+  // its rows lie in that order anyway
+  const int64_t rows = (int64_t)G / outer * C;
+  const bool few_rows = outer == 1 && dispatched_few_rows(G, S, E, C, M, H) &&
                         ((uintptr_t)wo_packed | (uintptr_t)y) % 16 == 0;
   MOE_REQUIRE(dispatched_sizes_fit(G, S, C, dtype) &&
                   (few_rows || ring_path_applies((int)rows, H, M)) &&
@@ -2819,23 +2824,23 @@ int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
         pair_blocks, expert_blocks);
     MOE_CHECK_LAUNCH("dispatched_expert_ffn (slot map)");
   } else {
-    const int64_t n_map = (int64_t)E * R;
+    const int64_t n_map = (int64_t)E * G * C;
     const unsigned cb = (unsigned)((n_map + 255) / 256 < 4096 ? (n_map + 255) / 256
                                                               : 4096);
     slot_map_clear_kernel<<<cb, 256, 0, st>>>(map, n_map, zero_row, M);
     MOE_CHECK_LAUNCH("dispatched_expert_ffn (clear)");
     slot_map_kernel<<<(unsigned)pair_blocks, 256, 0, st>>>(
-        idx, pos, gate, kept, map, (int64_t)G * S, S, C, rows);
+        idx, pos, gate, kept, map, (int64_t)G * S, S, C, (int64_t)G * C);
     MOE_CHECK_LAUNCH("dispatched_expert_ffn (slot map)");
   }
   int rc = launch_ring((const bf16_t*)x, (const bf16_t*)wi_packed, (bf16_t*)h,
-                       E, R, H, M, relu, st, map, zero_row);
+                       E * outer, R, H, M, relu, st, map, zero_row);
   if (rc != 0) return rc;
   if (!relu && activation != MESH_MOE_ACT_LINEAR) {
-    rc = launch_activation(h, (int64_t)E * R * H, activation, dtype, st);
+    rc = launch_activation(h, (int64_t)E * outer * R * H, activation, dtype, st);
     if (rc != 0) return rc;
   }
-  return grouped_gemm(h, wo_packed, y, E, R, N, H, MESH_MOE_ACT_LINEAR, dtype,
+  return grouped_gemm(h, wo_packed, y, E * outer, R, N, H, MESH_MOE_ACT_LINEAR, dtype,
                       st);
 }
 
@@ -2849,6 +2854,20 @@ extern "C" int mesh_moe_dispatched_expert_ffn(
   return dispatched_ffn(x, idx, pos, gate, kept, nullptr, false, wi_packed, wo_packed,
                         h, y, workspace, workspace_bytes, G, S, E, C, M, H, N,
                         activation, dtype, stream);
+}
+
+// (The inner level of the hierarchical layer, forward: the dispatch in front of its
+// experts wrote and read every slot row once more.  8 x 16 experts, 40960 tokens of 2048
+// in 40 groups, 71 us of 3570.)
+extern "C" int mesh_moe_dispatched_outer_expert_ffn(
+    const void* x, const int32_t* idx, const int32_t* pos, const float* gate,
+    const uint8_t* kept, const int32_t* fill, const void* wi_packed,
+    const void* wo_packed, void* h, void* y, void* workspace, size_t workspace_bytes,
+    int G, int S, int E, int C, int outer, int M, int H, int N, int activation, int dtype,
+    void* stream) {
+  return dispatched_ffn(x, idx, pos, gate, kept, fill, false, wi_packed, wo_packed, h, y,
+                        workspace, workspace_bytes, G, S, E, C, M, H, N, activation,
+                        dtype, stream, outer);
 }
 
 static size_t compact_ffn_tiles(int E, int R, int H, int N) {

@@ -224,6 +224,10 @@ _SIGNATURES = {
     "mesh_moe_shared_linear_backward": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp, ctypes.c_size_t, _vp]),
+    "mesh_moe_dispatched_outer_expert_ffn": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]),
     "mesh_moe_shared_linear_backward_input_supported": (ctypes.c_int, [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "mesh_moe_shared_linear_backward_input": (ctypes.c_int, [
@@ -885,11 +889,13 @@ E_UNSUPPORTED = -2
 
 
 def dispatched_expert_ffn(x, r, wi_packed, wo_packed, activation="relu",
-                          h=None):
+                          h=None, outer=1):
   """dispatch + expert_ffn without materialising expert_in: x [G, S, M], the
   Routing r -> y [E, G*C, N], or None where the library has no such kernel for
   the case (the caller then makes the two calls).  h [E, G*C, H], if given,
-  receives the hidden tensor.  With at most 64 rows per expert the rows of y and
+  receives the hidden tensor.  With kernels [E * outer, ...] every expert has `outer`
+  of them, one for each G / outer groups in a row: y [E * outer, G / outer * C, N].
+  With at most 64 rows per expert the rows of y and
   h of an expert that no token goes to are unspecified (combine reads none of
   them)."""
   lib = load_library()
@@ -902,20 +908,29 @@ def dispatched_expert_ffn(x, r, wi_packed, wo_packed, activation="relu",
   if dt != torch.bfloat16:
     return None
   dev = x.device
+  if g % outer:
+    return None
+  rows = g // outer * c
+  e_w = e * outer
   if h is None:
-    h = torch.empty((e, g * c, hdim), dtype=dt, device=dev)
-  _dev(h, "h", dt, (e, g * c, hdim))
-  y = torch.empty((e, g * c, n), dtype=dt, device=dev)
+    h = torch.empty((e_w, rows, hdim), dtype=dt, device=dev)
+  _dev(h, "h", dt, (e_w, rows, hdim))
+  y = torch.empty((e_w, rows, n), dtype=dt, device=dev)
   ws_bytes = lib.mesh_moe_dispatched_expert_ffn_workspace_bytes(g, e, c, m)
   ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=dev)
+  routing = (_dev(x, "x"), _dev(r.idx, "idx", torch.int32, (g, s, 2)),
+             r.pos.data_ptr(), r.gate.data_ptr(), r.kept.data_ptr())
+  buffers = (_dev(wi_packed, "wi_packed", dt, (e_w, hdim, m)),
+             _dev(wo_packed, "wo_packed", dt, (e_w, n, hdim)), h.data_ptr(),
+             y.data_ptr(), ws.data_ptr(), ws_bytes)
+  how = (m, hdim, n, ACTIVATIONS[activation], dtype_code(dt), _stream())
   with _stage("expert_ffn"):
-    rc = lib.mesh_moe_dispatched_expert_ffn(
-        _dev(x, "x"), _dev(r.idx, "idx", torch.int32, (g, s, 2)),
-        r.pos.data_ptr(), r.gate.data_ptr(), r.kept.data_ptr(),
-        _dev(wi_packed, "wi_packed", dt, (e, hdim, m)),
-        _dev(wo_packed, "wo_packed", dt, (e, n, hdim)), h.data_ptr(),
-        y.data_ptr(), ws.data_ptr(), ws_bytes, g, s, e, c, m, hdim, n,
-        ACTIVATIONS[activation], dtype_code(dt), _stream())
+    if outer > 1:
+      rc = lib.mesh_moe_dispatched_outer_expert_ffn(
+          *routing, _dev(r.fill, "fill", torch.int32, (g, e)), *buffers, g, s, e, c,
+          outer, *how)
+    else:
+      rc = lib.mesh_moe_dispatched_expert_ffn(*routing, *buffers, g, s, e, c, *how)
   if rc == E_UNSUPPORTED:
     return None
   _check(rc, "dispatched_expert_ffn")

@@ -1113,14 +1113,18 @@ class MoEV2Operation(mtf.Operation):
       logits_y = None
       if save:
         ry, logits_y = ry
-      ein_y = moe_hip.dispatch(inputs_y.reshape(x_e * h0, t_, m_), ry)
       # experts: weights are [y, x, ...]; rows of (y, x) are its h0*d slots
-      h = None
-      if save:
-        h = torch.empty((y_e * x_e, h0 * d_, wi_p.shape[1]), dtype=dt,
-                        device=xg.device)
-      yy = moe_hip.expert_ffn(ein_y.reshape(y_e * x_e, h0 * d_, m_), wi_p,
-                              wo_p, "relu", h=h, for_gradient=save)
+      h = yy = ein_y = None
+      if not save:
+        yy = moe_hip.dispatched_expert_ffn(inputs_y.reshape(x_e * h0, t_, m_), ry, wi_p,
+                                           wo_p, "relu", outer=x_e)
+      if yy is None:
+        ein_y = moe_hip.dispatch(inputs_y.reshape(x_e * h0, t_, m_), ry)
+        if save:
+          h = torch.empty((y_e * x_e, h0 * d_, wi_p.shape[1]), dtype=dt,
+                          device=xg.device)
+        yy = moe_hip.expert_ffn(ein_y.reshape(y_e * x_e, h0 * d_, m_), wi_p,
+                                wo_p, "relu", h=h, for_gradient=save)
       out_y = moe_hip.combine(yy.reshape(y_e, x_e * h0, d_, n_), ry, t_)
       out = moe_hip.combine(out_y.reshape(x_e, ag, c_, n_), rx, s_)
       loss = (rx.loss.to(dt) + ry.loss.to(dt)).reshape(())

@@ -1936,6 +1936,24 @@ def test_gathered_rows_with_three_token_slots(hip, e, g, c, h):
   assert torch.equal(got, hip.expert_ffn(xe, wi, wo, "relu"))
 
 
+@pytest.mark.parametrize("e,g,c,outer", [(4, 6, 65, 2), (16, 40, 80, 8), (3, 12, 64, 4),
+                                         (2, 4, 256, 1), (5, 9, 43, 3)])
+def test_gathered_rows_of_kernels_per_part(hip, e, g, c, outer):
+  """Several kernels per expert, each for a run of groups: the bits of dispatch and two
+  products, rows that are dropped, empty or have a gate of zero among them."""
+  s, m, h = 192, 256, 512
+  gen = torch.Generator(device="cuda").manual_seed(g + c)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  importance = (mk(g, s) > -0.5).float()
+  r = hip.top2_gating(mk(g, s, e), c, importance=importance)
+  x, wi, wo = (t.to(torch.bfloat16) for t in (
+      mk(g, s, m), mk(e * outer, h, m), mk(e * outer, m, h)))
+  got = hip.dispatched_expert_ffn(x, r, wi, wo, "relu", outer=outer)
+  xe = hip.dispatch(x, r).reshape(e * outer, g // outer * c, m)
+  assert torch.equal(got, hip.expert_ffn(xe, wi, wo, "relu"))
+  assert hip.dispatched_expert_ffn(x, r, wi, wo, "relu", outer=g + 1) is None
+
+
 @pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
                                    (2, 6144, 776, 256), (29, 3000, 520, 760)],
                          ids=lambda s: "x".join(map(str, s)))
