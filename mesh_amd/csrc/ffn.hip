@@ -2092,6 +2092,12 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 //   64 x 320 rows, 1024 x 4096 (160 rows; of 128 206 us)       200 -> 182
 //   16 x 700 rows, 512 x 512 (96 rows)                         14.1 -> 10.7
 //   5000 rows, 1280 x 1280 (128 rows)                          26.6 -> 20.4
+// In launches of three rounds of 256-row tiles and more the power limiter sets the pace,
+// and low tiles move more bytes per product: the terms for three token slots then count
+// 1.10 times.  (24 such products timed without that factor, 160 or 128 rows against the
+// 192 to 256 that the terms give the others: chosen for less than a tenth they were 1 to
+// 13 % slower, 16 x 1408 rows, 1920 -> 7680 563 -> 606 us, 48 x 501, 7296 -> 2624 869 ->
+// 982; for more, 1 % slower to 4 % faster.)
 // K-major operands (weight gradients; R is then a width, K the rows summed over):
 // 0.48 + 0.12 per piece us per K tile, 3.3 + 0.75 per piece outside the K loop, whose
 // share is larger there (reductions of few K tiles; from 16 x 704 and 1280 rows, and
@@ -2107,6 +2113,8 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
                           bool kmajor = false) {
   const int tiles_n = (N + RingCfg::BN - 1) / RingCfg::BN;
   const int nk = (K + RingCfg::BK - 1) / RingCfg::BK;
+  const bool long_launch =
+      (int64_t)E * ((R + RingCfg::BM - 1) / RingCfg::BM) * tiles_n >= 3 * (int64_t)cus;
   int best_rows = RingCfg::BM;
   double best = 0;
   for (int rows = RingCfg::BM; rows >= 32; rows -= 32) {
@@ -2120,7 +2128,8 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
                                      : 0.40 + 0.13 * pieces;
     const double least = deep ? 0.5 : 0.6;
     const double outside = kmajor ? 3.3 + 0.75 * pieces : 5.0;
-    const double cost = (double)((tiles + cus - 1) / cus) *
+    const double limited = deep && long_launch ? 1.10 : 1.0;
+    const double cost = limited * (double)((tiles + cus - 1) / cus) *
                         (nk * (per_k_tile < least ? least : per_k_tile) + outside);
     if (rows == RingCfg::BM || cost < 0.98 * best) {
       best = cost;
