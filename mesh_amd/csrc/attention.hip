@@ -666,7 +666,9 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     tile(it, S0(), std::true_type(), acc_a, acc_b);
   }
 
-  const float l_all = DIVIDED ? 1.0f : l_part + __shfl_xor(l_part, 32);
+  // (DIVIDED: a query all of whose logits are -inf, or one inf or NaN, has no weights: NaN)
+  const float l_all =
+      DIVIDED ? 1.0f + (m_run - m_run) : l_part + __shfl_xor(l_part, 32);
   const float inv = 1.0f / l_all;
   if constexpr (STATS) {
     const bf16_t* drow = dout + ((int64_t)b * L + min(my_q, L - 1)) * row_stride +

@@ -656,6 +656,40 @@ def test_fused_attention_of_any_length(hip, length, d, causal, with_ids_and_bias
       np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("length", [24, 25, 131])
+def test_fused_attention_of_infinite_logits(hip, length, d):
+  """Causal.  Key 0 has a logit of -inf for every query: query 0, which sees nothing
+  else, gets NaN, the others the weights of their other keys.  A key with a NaN, and one
+  with a logit of +inf, make NaN of the queries that see them."""
+  gen = torch.Generator(device="cuda").manual_seed(length)
+  q, k, v = (torch.randn((1, length, d), generator=gen, device="cuda") for _ in range(3))
+  q = q.abs() * d ** -0.5
+  at = length - 3
+  for value in (None, float("nan"), float("inf")):
+    k[0, 0] = 0.0
+    k[0, 0, 5] = float("-inf")
+    if value is not None:
+      k[0, at] = 0.0
+      k[0, at, 7] = value
+    got, lse = hip.self_attention(*(t.bfloat16() for t in (q, k, v)), 1, True,
+                                  return_lse=True)
+    first_bad = length if value is None else at
+    assert bool(got[0, 0].isnan().all()) and not bool(lse[0, 0].isfinite())
+    assert bool(got[0, 1:first_bad].isfinite().all())
+    assert bool(got[0, first_bad:].isnan().all())
+    kd = k.bfloat16().double()[0].clone()
+    kd[0, 5] = 0.0
+    logits = q.bfloat16().double()[0] @ kd.t()
+    logits[:, 0] = float("-inf")
+    logits = logits.masked_fill(torch.ones((length, length), device="cuda").triu(1)
+                                .bool(), float("-inf"))[1:first_bad, :first_bad]
+    want = logits.softmax(-1) @ v.bfloat16().double()[0, :first_bad]
+    # a rounding to bf16 of every weight and of the sum
+    assert ((got[0, 1:first_bad].double() - want).abs() <= 2.0 ** -7 * (
+        logits.softmax(-1) @ v.bfloat16().double()[0, :first_bad].abs())).all()
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("length", [8, 64, 72, 256, 264, 520])
 def test_key_and_value_gradients_of_one_launch(hip, length, causal):
