@@ -130,7 +130,7 @@ class SharedInput(object):
     x, kernel = layers[0].inputs
     self.layers = list(layers)
     self.gradients = {}        # {layer: its DenseGradOperation}
-    self._ahead = {}           # {first of them: every dy is there when it runs}
+    self._ahead = {}           # {all of them: every dy is there when the last runs}
     if all(op.inputs[0] is x and op.inputs[1].shape.to_integer_list ==
            kernel.shape.to_integer_list and op.inputs[1].dtype == kernel.dtype and
            op._activation is None and op.siblings is None   # pylint: disable=protected-access
@@ -142,13 +142,13 @@ class SharedInput(object):
     """Called by the first of the gradient operations: the gradients of all layers'
     outputs as one tensor [layers, ...], if every one is there and they lie one after
     the other in memory (as the attention's gradient leaves them), else None."""
-    grads = [self.gradients.get(op) for op in self.layers]
+    grads = tuple(self.gradients.get(op) for op in self.layers)
     operations = first.graph.operations
-    if first not in self._ahead:
+    if grads not in self._ahead:
       at = operations.index(first)
-      self._ahead[first] = None not in grads and all(
+      self._ahead[grads] = None not in grads and all(
           operations.index(g.inputs[0].operation) < at for g in grads)
-    if not self._ahead[first]:
+    if not self._ahead[grads]:
       return None
     dys = [_rows_of(lowering, g.inputs[0]) for g in grads]
     d = dys[0]
@@ -313,15 +313,17 @@ class DenseGradOperation(mtf.Operation):
     return True
 
   def sums_up_in(self, layers):
-    """The operation whose dx is the sum of those of all `layers`, or None."""
+    """The operation whose dx is the sum of those of all `layers`, or None.  None too
+    where a later mtf.gradients has made another gradient operation of one of the
+    layers: what is made ahead is made for, and from the dy of, that one."""
     last = self
     while last.added_by is not None:
       last = last.added_by
-    summed, op = [], last
+    known, summed, op = self._forward.siblings.gradients, {}, last
     while op is not None:
-      summed.append(op._forward)         # pylint: disable=protected-access
+      summed[op._forward] = op           # pylint: disable=protected-access
       op = op._adds                      # pylint: disable=protected-access
-    return last if set(summed) == set(layers) else None
+    return last if summed == {layer: known.get(layer) for layer in layers} else None
 
   def _made_ahead(self, lowering):
     """What the first gradient operation of layers with one input made for all."""

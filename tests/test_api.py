@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import mesh_amd as mtf
+from mesh_amd import layers
 from mesh_amd import moe_hip
 from mesh_amd.transformer import moe
 
@@ -432,6 +433,73 @@ def test_gradients_builds_the_backward_operation():
   grads3 = mtf.gradients([y3, l3], [x3] + v3)
   assert [g.shape for g in grads3] == [t.shape for t in [x3] + v3]
   assert any(isinstance(o, moe.MoEV2GradOperation) for o in g3.operations)
+
+
+class _CpuMesh(mtf.HipMeshImpl):
+  """One slice on the CPU, for graphs whose kernels a test replaces by torch."""
+
+  def __init__(self):
+    mtf.MeshImpl.__init__(self, [], {})
+    self._device, self._device_index = torch.device("cpu"), None
+
+
+@pytest.mark.parametrize("second_dys", ["same", "in_place", "apart"])
+@pytest.mark.parametrize("again", ["q", "k", "v", "qk", "kv", "qv", "qkv"])
+def test_shared_input_gradients_asked_for_again(monkeypatch, again, second_dys):
+  """Gradients of three layers of one input, then those of some of them once more, with
+  the same dys, with ones that lie beside the first call's others, or elsewhere: every
+  sum is made of its own call's, in the first run and in later ones."""
+  rows, k, n = 3, 4, 5
+  t = lambda x: x.transpose(-1, -2)
+  for name, fn in dict(
+      current_device=lambda: None,
+      pack_weights=lambda w, dtype, out=None: t(w).to(dtype) if out is None else
+      out.copy_(t(w)),
+      dense=lambda x, w, activation=None: x @ t(w[0]),
+      dense_backward=lambda x, w, dy, y=None, dx_relu_mask=False: (dy @ t(w), t(x) @ dy),
+      shared_linear_supported=lambda x, n: True,
+      shared_linear=lambda x, w: x @ t(w),
+      shared_linear_backward_supported=lambda x, n: True,
+      shared_linear_backward=lambda x, dy: t(x) @ dy,
+      shared_linear_backward_input_supported=lambda dy, kernels: True,
+      shared_linear_backward_input=lambda dy, kernels: sum(
+          d @ t(w) for d, w in zip(dy, kernels))).items():
+    monkeypatch.setattr(moe_hip, name, fn)
+  gen = torch.Generator().manual_seed(1)
+  mk = lambda *sizes: torch.randn(sizes, generator=gen, dtype=torch.float64)
+  graph = mtf.Graph()
+  mesh = mtf.Mesh(graph, "mesh")
+  rdim, kdim, ndim = (mtf.Dimension("rows", rows), mtf.Dimension("k", k),
+                      mtf.Dimension("n", n))
+  x = mtf.import_tf_tensor(mesh, mk(rows, k), mtf.Shape([rdim, kdim]))
+  weights = [mtf.get_variable(mesh, name, mtf.Shape([kdim, ndim]),
+                              dtype=torch.float64) for name in "qkv"]
+  ops = [layers.DenseOperation(x, w, [ndim], None) for w in weights]
+  layers.SharedInput(ops)
+  of = ["qkv".index(c) for c in again]
+  joint, other = mk(3, rows, n), mk(3, rows, n)
+  values = [[other[i] if i in of and second_dys == "in_place" else joint[i]
+             for i in range(3)],
+            [other[i] if second_dys == "apart" else joint[i] for i in range(3)]]
+  dys = [[mtf.import_tf_tensor(mesh, value, mtf.Shape([rdim, ndim])) for value in call]
+         for call in values]
+  wrt = [x] + weights
+  first = mtf.gradients([op.outputs[0] for op in ops], wrt, grad_ys=dys[0])
+  second = mtf.gradients([ops[i].outputs[0] for i in of], wrt,
+                         grad_ys=[dys[1][i] for i in of])
+  init = {name: mk(k, n) for name in "qkv"}
+  low = mtf.Lowering(graph, {mesh: _CpuMesh()}, initial_values=init)
+  value = low.export_to_tf_tensor
+  for _ in range(2):
+    for grads, dy, parts in ((first, values[0], [0, 1, 2]), (second, values[1], of)):
+      dx = sum(dy[i] @ t(init["qkv"[i]]) for i in parts)
+      torch.testing.assert_close(value(grads[0]), dx)
+      for i in range(3):
+        if i in parts:
+          torch.testing.assert_close(value(grads[1 + i]), t(value(x)) @ dy[i])
+        else:
+          assert grads[1 + i] is None
+    low.run()
 
 
 @pytest.mark.parametrize("experts_attention", [False, True])
