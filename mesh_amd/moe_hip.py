@@ -1083,14 +1083,15 @@ def top2_layer(x, w_gate, w_gate_packed, wi_packed, wo_packed, groups, group_siz
   groups * group_size rows [.., M], w_gate [M, E], w_gate_packed [1, E, M], wi_packed
   [E, H, M], wo_packed [E, N, H], importance [groups, group_size] values or None ->
   (out of sizes out_sizes, loss, loss * loss_coef), or None where an operand does not
-  lie on 16 bytes in one piece (the caller then makes the calls one by one)."""
+  lie on 16 bytes in one piece or w_gate is of another dtype than x (the caller then
+  makes the calls one by one; not all of them read w_gate)."""
   lib = load_library()
   if activation not in ACTIVATIONS:
     raise ValueError("unsupported expert activation %r" % (activation,))
   e, h, m = wi_packed.shape
   n = wo_packed.shape[1]
   dt, dev = x.dtype, x.device
-  if not (x.is_contiguous() and w_gate.is_contiguous() and
+  if not (x.is_contiguous() and w_gate.is_contiguous() and w_gate.dtype == dt and
           (importance is None or importance.is_contiguous())):
     return None
   xp = _dev(x, "x")

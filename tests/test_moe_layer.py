@@ -1666,6 +1666,23 @@ def test_v1_in_one_call_equals_its_calls(case):
                                  atol=1e-2)
 
 
+def test_v1_forward_with_variables_of_another_activation_dtype():
+  """bf16 tokens, float32 variables, sizes whose router projection is fused with the
+  gating and reads the packed kernel only: the layer of bf16 variables."""
+  b, l, m, hdim, e = 2, 128, 64, 128, 4
+  rng = np.random.default_rng(23)
+  w = dict(w_gate=H.normal_weights(rng, (m, e), m),
+           wi=H.normal_weights(rng, (e, m, hdim), m),
+           wo=H.normal_weights(rng, (e, hdim, m), hdim))
+  hp, _ = make_hparams(moe_num_experts=e, moe_hidden_size=hdim, moe_group_size=l,
+                       moe_capacity_factor_eval=1.25)
+  x = O.cast_act(rng.standard_normal((b, l, m)).astype(np.float32), "bfloat16")
+  got = [run_v1(x, w, hp, False, "bfloat16", variable_dtype=vdt)[:2]
+         for vdt in (None, mtf.VariableDType(torch.float32))]
+  np.testing.assert_array_equal(got[0][0], got[1][0])
+  assert got[0][1] == got[1][1]
+
+
 @pytest.mark.parametrize("act_dtype", ["float32", "bfloat16"])
 def test_captured_step_replays_match_eager(act_dtype):
   """Lowering.capture(): a HIP-graph replay gives what an eager run gives, on
