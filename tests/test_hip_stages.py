@@ -1954,6 +1954,30 @@ def test_gathered_rows_of_kernels_per_part(hip, e, g, c, outer):
   assert hip.dispatched_expert_ffn(x, r, wi, wo, "relu", outer=g + 1) is None
 
 
+@pytest.mark.parametrize("c", [43, 64, 65, 700])
+def test_gathered_rows_of_mostly_empty_slots(hip, c):
+  """Experts without a token, with one and with as many as there are: every empty slot
+  is known as one, whatever the map's memory held."""
+  e, g, outer, s, m, h = 3, 6, 2, 96, 256, 512
+  gen = torch.Generator(device="cuda").manual_seed(c)
+  mk = lambda *sh: torch.randn(sh, generator=gen, device="cuda")
+  logits = mk(g, s, e) - 30.0 * torch.arange(e, device="cuda")
+  importance = (mk(g, s) > 0).float()
+  importance[1] = 0.0
+  importance[2] = 0.0
+  importance[2, 5] = 1.0
+  r = hip.top2_gating(logits, c, importance=importance)
+  x, wi, wo = (t.to(torch.bfloat16) for t in (
+      mk(g, s, m), mk(e * outer, h, m), mk(e * outer, m, h)))
+  xe = hip.dispatch(x, r).reshape(e * outer, g // outer * c, m)
+  want = hip.expert_ffn(xe, wi, wo, "relu")
+  for _ in range(2):
+    # (memory that the call's workspace is likely to get)
+    torch.full((1 << 20,), 7, dtype=torch.int32, device="cuda")
+    assert torch.equal(hip.dispatched_expert_ffn(x, r, wi, wo, "relu", outer=outer),
+                       want)
+
+
 @pytest.mark.parametrize("shape", [(1, 4000, 264, 520), (1, 1025, 128, 256),
                                    (2, 6144, 776, 256), (29, 3000, 520, 760)],
                          ids=lambda s: "x".join(map(str, s)))
