@@ -2080,12 +2080,17 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 // times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
 // 0.40 + 0.13 per piece us per K tile (0.20 + 0.14 with three token slots, no less than
 // 0.6 and 0.5) and 5 us outside the K loop.  Rows are spread evenly over the row tiles:
-// 640 rows per expert are three tiles of 224 or four of 160, not 256 + 256 + 128.  The
-// terms are fitted to 18 products of 1 to 128 experts, 180 to 16000 rows, K 512 to 8192,
-// N 512 to 8192, timed with six heights each: the rule's choice is 0.3 % slower than the
-// best of them on average and 2.2 % at worst (16 x 1250 rows, 768 x 3072: 256 rows 90.0
-// us, 160 88.1).  Tiles of 256 and a shorter last one -> the rule's choice (both sides
-// bit-identical):
+// 640 rows per expert are three tiles of 224 or four of 160, not 256 + 256 + 128.  In more
+// than one round the row tiles of an expert do not run side by side, and each reads its
+// weights again: no less than 9 TB/s takes for all of them.  (Without that term three low
+// tiles in two rounds were chosen over one tile in one where the weights set the pace: 32
+// x 240 rows, 2304 -> 1152 68 us, one tile 58; 32 x 166, 4608 -> 1152 125 and 99.  One
+// round of low tiles reads them once from memory: 12 x 152, 4608 -> 1536 61 in tiles of
+// 64, 64 in tiles of 96.)  Of 394 products of 1 to 128 experts, 128 to 16000 rows, K and N
+// 512 to 8192, timed with every height from 64 on, the rule's choice is 0.3 % slower than
+// the best one on average, by more than 3 % in 16 and by 9 % at worst (24 x 417 rows, 8192
+// -> 2048: 224 rows 370 us, 128 338).  Tiles of 256 and a shorter last one -> the rule's
+// choice (both sides bit-identical):
 //   32 x 640 rows, 4096 x 1024 (160 rows; of 224 186 us)       197 -> 155 us
 //   16 x 708 rows, 768 x 3072 (192 rows) / 3072 x 768 (160)  67 / 56 -> 53 / 51
 //   8 x 900 rows, 1536 x 4608 (192 rows)                        111 -> 93
@@ -2115,6 +2120,7 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
   const int nk = (K + RingCfg::BK - 1) / RingCfg::BK;
   const bool long_launch =
       (int64_t)E * ((R + RingCfg::BM - 1) / RingCfg::BM) * tiles_n >= 3 * (int64_t)cus;
+  const double weights_once = (double)E * N * K * sizeof(bf16_t) / 9e6;
   int best_rows = RingCfg::BM;
   double best = 0;
   for (int rows = RingCfg::BM; rows >= 32; rows -= 32) {
@@ -2129,8 +2135,10 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
     const double least = deep ? 0.5 : 0.6;
     const double outside = kmajor ? 3.3 + 0.75 * pieces : 5.0;
     const double limited = deep && long_launch ? 1.10 : 1.0;
-    const double cost = limited * (double)((tiles + cus - 1) / cus) *
-                        (nk * (per_k_tile < least ? least : per_k_tile) + outside);
+    double cost = limited * (double)((tiles + cus - 1) / cus) *
+                  (nk * (per_k_tile < least ? least : per_k_tile) + outside);
+    if (!kmajor && tiles > cus && cost < tiles_m * weights_once)
+      cost = tiles_m * weights_once;
     if (rows == RingCfg::BM || cost < 0.98 * best) {
       best = cost;
       best_rows = even;
