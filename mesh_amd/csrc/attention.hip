@@ -355,6 +355,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
   constexpr float LOG2E = 1.4426950408889634f;
   float m_run = NEG;      // running maximum of this lane's query
   float l_part = 0.f;     // sum over this half-wave's keys
+  float inv_sum = 1.f;    // DIVIDED: 1 / sum over all keys
 
   // Is a tile's softmax laid beside the next tile's logits?  Not for heads of 64 with
   // ids and a bias, which do not fit into the registers of three wavefronts: up to 24 of
@@ -546,9 +547,14 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     float psum = 0.f;
     uint32_t w[16];
     auto weights = [&](int i) {      // keys of registers 2 (i % 8) and + 1
-      const float p0 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7)], LOG2E, mneg));
-      const float p1 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7) + 1], LOG2E, mneg));
-      psum += p0 + p1;
+      float p0 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7)], LOG2E, mneg));
+      float p1 = fa_exp2(fmaf(acc_s[i >> 3][2 * (i & 7) + 1], LOG2E, mneg));
+      if constexpr (DIVIDED) {
+        p0 *= inv_sum;
+        p1 *= inv_sum;
+      } else {
+        psum += p0 + p1;
+      }
       w[i] = f32x2_to_bf16x2(p0, p1);
       // (otherwise the compiler makes them where they are first used, behind the
       // branch around the mask)
@@ -568,7 +574,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
 #pragma unroll
       for (int i = 0; i < 16; ++i) weights(i);
     }
-    l_part += psum;
+    if constexpr (!DIVIDED) l_part += psum;
     fa_bf16x8_t pf[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -633,13 +639,19 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
 #pragma unroll
       for (int i = 0; i < 32; ++i)
         psum += fa_exp2(fmaf(acc_a[i >> 4][i & 15], LOG2E, mneg));
-      l_part = l_part * fa_exp2((m_run - m_new) * LOG2E) + psum;
+      // (the exponents' own difference: the sum then has the rounding of the maximum's
+      // exponent that the weights have, and it divides out.  Without a key so far the sum
+      // is 0, or NaN that stays.)
+      l_part = psum + (m_run > 0.5f * NEG
+                           ? l_part * fa_exp2(mneg - exponent_of_max(m_run))
+                           : l_part);
       m_run = m_new;
       __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0)
       __syncthreads();
     }
-    // exp(logit - m_run) is the divided weight
-    m_run += logf(l_part + __shfl_xor(l_part, 32));
+    // (no weights, all of them or one inf or NaN: NaN)
+    l_part += __shfl_xor(l_part, 32);
+    inv_sum = 1.0f / l_part;
     load_k(kt_begin, 0);
     load_v(kt_begin, 0);
     if (BESIDE && kt_count > 1) load_k(kt_begin + 1, 1);
@@ -666,10 +678,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void flash_attention_kernel(
     tile(it, S0(), std::true_type(), acc_a, acc_b);
   }
 
-  // (DIVIDED: a query all of whose logits are -inf, or one inf or NaN, has no weights: NaN)
-  const float l_all =
-      DIVIDED ? 1.0f + (m_run - m_run) : l_part + __shfl_xor(l_part, 32);
-  const float inv = 1.0f / l_all;
+  const float l_all = DIVIDED ? l_part : l_part + __shfl_xor(l_part, 32);
+  const float inv = DIVIDED ? 1.0f : 1.0f / l_all;
   if constexpr (STATS) {
     const bf16_t* drow = dout + ((int64_t)b * L + min(my_q, L - 1)) * row_stride +
                          (int64_t)h * D;

@@ -690,6 +690,25 @@ def test_fused_attention_of_infinite_logits(hip, length, d):
         logits.softmax(-1) @ v.bfloat16().double()[0, :first_bad].abs())).all()
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("length", [24, 25, 131, 200])
+def test_fused_attention_of_huge_logits(hip, length, d):
+  """Logits of up to 2^21, whole multiples of 2^10 and exact in float32, several keys of
+  the same one among them: a query's largest weights are equal parts of 1, whatever the
+  maximum's exponent rounds to."""
+  gen = torch.Generator(device="cuda").manual_seed(length)
+  whole = lambda n: torch.randint(-4, 5, (1, n, d), generator=gen, device="cuda").float()
+  q, k = whole(length) * 2.0 ** 5, whole(length) * 2.0 ** 5
+  k[0, length // 2:] = k[0, :length - length // 2].clone()
+  v = torch.randn((1, length, d), generator=gen, device="cuda")
+  q, k, v = (t.bfloat16() for t in (q, k, v))
+  got = hip.self_attention(q, k, v, 1, False)[0].double()
+  weights = (q.double()[0] @ k.double()[0].t().contiguous()).softmax(-1)
+  # a rounding to bf16 of every weight and of the sum, float32 sums below them
+  assert ((got - weights @ v.double()[0]).abs() <=
+          (2.0 ** -7 + 2.0 ** -14) * (weights @ v.double()[0].abs())).all()
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("length", [8, 64, 72, 256, 264, 520])
 def test_key_and_value_gradients_of_one_launch(hip, length, causal):
