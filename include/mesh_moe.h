@@ -29,7 +29,8 @@
 extern "C" {
 #endif
 
-#define MESH_MOE_ABI_VERSION 42
+/* (counted up with every change of a declaration, and of what a call accepts) */
+#define MESH_MOE_ABI_VERSION 43
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0

@@ -3,6 +3,7 @@ defaults, dimension and variable names, error types, and that the C-ABI library
 loads and exports every symbol the header declares."""
 
 import ctypes
+import hashlib
 import inspect
 import os
 import re
@@ -356,6 +357,21 @@ def test_library_exports_every_declared_symbol():
   assert lib.mesh_moe_abi_version() == moe_hip.ABI_VERSION
   lib.mesh_moe_gating_workspace_bytes.restype = ctypes.c_size_t
   assert lib.mesh_moe_gating_workspace_bytes(32, 2048, 64) > 0
+
+
+# {version: what the declarations of the header hash to}
+_DECLARATIONS = {42: "ff364a62b8f3b800", 43: "fb4ec3a91e893039"}
+
+
+def test_abi_version_counts_the_declarations():
+  """A library built between two changes of the header is told by its version."""
+  header = open(os.path.join(ROOT, "include", "mesh_moe.h")).read()
+  code = re.sub(r"/\*.*?\*/", " ", header, flags=re.DOTALL)
+  code = re.sub(r"(MESH_MOE_ABI_VERSION) \d+", r"\1", code)
+  digest = hashlib.sha256(" ".join(code.split()).encode()).hexdigest()[:16]
+  assert _DECLARATIONS.get(moe_hip.ABI_VERSION) == digest
+  assert max(_DECLARATIONS) == moe_hip.ABI_VERSION
+  assert len(set(_DECLARATIONS.values())) == len(_DECLARATIONS)
 
 
 def test_compact_experts_decline_a_hidden_tensor_beyond_32_bits():
