@@ -30,7 +30,7 @@ extern "C" {
 #endif
 
 /* (counted up with every change of a declaration, and of what a call accepts) */
-#define MESH_MOE_ABI_VERSION 43
+#define MESH_MOE_ABI_VERSION 44
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -162,9 +162,11 @@ int mesh_moe_top2_gating_static_scratch(
  * of mesh_moe_top2_gating; batch * tokens == G * S and each weight set covers
  * whole groups.  The workspace may hold anything on entry.
  * Returns MESH_MOE_E_UNSUPPORTED (nothing launched) unless dtype is bf16,
- * M % 64 == 0, E % 4 == 0, E <= 128 and S % 128 == 0; callers then use the two
- * separate entry points.
+ * M % 64 == 0, E % 4 == 0, E <= 128 and S % 128 == 0
+ * (mesh_moe_fused_router_supported: 1 or 0); callers then use the two separate entry
+ * points.
  */
+int mesh_moe_fused_router_supported(int M, int E, int S, int dtype);
 int mesh_moe_router_top2_gating(
     const void* x, const void* w_packed, const float* bias, float* logits,
     int batch, int64_t tokens, int M, int dtype, const void* importance,
@@ -364,6 +366,11 @@ int mesh_moe_dispatched_outer_expert_ffn(
 int mesh_moe_combine(const void* y, const int32_t* idx, const int32_t* pos,
                      const float* gate, const uint8_t* kept, void* out, int G,
                      int S, int E, int C, int N, int dtype, void* stream);
+
+/* 1 where a layer with two choices per token is better off with
+ * mesh_moe_compact_expert_ffn than with the padded rows (if that call takes its sizes),
+ * which is what mesh_moe_top2_layer does; 0 elsewhere. */
+int mesh_moe_top2_compacts(int G, int C);
 
 /* Bytes of scratch mesh_moe_compact_expert_ffn needs. */
 size_t mesh_moe_compact_expert_ffn_workspace_bytes(int G, int E, int C, int M,

@@ -50,6 +50,8 @@ int f32_gemm_stable(const float* A, const float* B, float* C, int E, int R, int 
 // first product take these sizes
 bool dispatched_ffn_shapes(int G, int S, int E, int C, int M, int H, int dtype);
 bool compact_ffn_shapes(int G, int S, int E, int C, int M, int H, int N, int dtype);
+// whether a layer with two choices per token takes the calls on compacted rows
+bool top2_compacts(int G, int C);
 // The token of every expert's row (-1: an empty one, which reads as zeros), for a first
 // product that fetches its rows through it, and the zeros.
 struct SlotMap {
@@ -70,7 +72,9 @@ int dispatched_ffn(const void* x, const int32_t* idx, const int32_t* pos,
 // whether those calls take the kernels for few rows, which read the map at once
 bool dispatched_few_rows(int G, int S, int E, int C, int M, int H);
 
-// route.hip: mesh_moe_top2_gating, which makes the slot map of one group of at most 64
+// route.hip: sizes that the gating calls with the router projection inside take
+bool fused_router_shapes(int M, int E, int S, int dtype);
+// mesh_moe_top2_gating, which makes the slot map of one group of at most 64
 // tokens (gating_makes_map) in the same launch where one is given
 bool gating_makes_map(int G, int S);
 int top2_gating(const float* logits, const void* importance, int importance_dtype,

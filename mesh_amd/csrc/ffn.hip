@@ -2756,8 +2756,17 @@ bool compact_ffn_shapes(int G, int S, int E, int C, int M, int H, int N, int dty
          ring_path_applies(G * C, H, M) && ring_path_applies(G * C, N, H) &&
          (int64_t)G * C * H < (1LL << 31);    // h's offsets within an expert
 }
+// Two choices per token fill nearly all slots.  Compacted rows then save a tile nowhere,
+// the empty slots only move to the end of each expert's rows: 1.5 % faster forward, 1 %
+// forward and backward (64 experts of 2048 slots, 4096 -> 16384) where an expert's slots
+// are whole tiles.  Of others the padded layout shortens an expert's last row tile.
+bool top2_compacts(int G, int C) { return (int64_t)G * C % RingCfg::BM == 0; }
 
 }  // namespace mesh_moe
+
+extern "C" int mesh_moe_top2_compacts(int G, int C) {
+  return top2_compacts(G, C) ? 1 : 0;
+}
 
 extern "C" size_t mesh_moe_dispatched_expert_ffn_workspace_bytes(int G, int E,
                                                                  int C, int M) {

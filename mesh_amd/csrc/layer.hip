@@ -22,9 +22,8 @@ LayerSpace layer_space(int G, int S, int E, int C, int M, int H, int N, int dtyp
   LayerSpace w = {};
   const size_t size = dtype_size(dtype), rows = (size_t)G * C;
   const size_t tokens = (size_t)G * S;
-  const bool bf16 = dtype == MESH_MOE_BF16;
-  w.fused_router = bf16 && M % 64 == 0 && E % 4 == 0 && E <= 128 && S % 128 == 0;
-  w.compact = rows % 256 == 0 && compact_ffn_shapes(G, S, E, C, M, H, N, dtype);
+  w.fused_router = fused_router_shapes(M, E, S, dtype);
+  w.compact = top2_compacts(G, C) && compact_ffn_shapes(G, S, E, C, M, H, N, dtype);
   w.dispatched = !w.compact && dispatched_ffn_shapes(G, S, E, C, M, H, dtype);
   w.map_by_gating = w.dispatched && !w.fused_router && gating_makes_map(G, S) &&
                     dispatched_few_rows(G, S, E, C, M, H);

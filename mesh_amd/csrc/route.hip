@@ -2493,6 +2493,17 @@ static int run_gating(const GateParams& p, const float* logits,
 }
 
 // Shape limits of the fused projection + gating kernel.
+namespace mesh_moe {
+bool fused_router_shapes(int M, int E, int S, int dtype) {
+  return dtype == MESH_MOE_BF16 && M % 64 == 0 && E % 4 == 0 && E <= 128 &&
+         S % 128 == 0;
+}
+}  // namespace mesh_moe
+
+extern "C" int mesh_moe_fused_router_supported(int M, int E, int S, int dtype) {
+  return fused_router_shapes(M, E, S, dtype) ? 1 : 0;
+}
+
 static int check_fused_router_args(const char* who, const void* x,
                                    const void* w_packed, int batch,
                                    int64_t tokens, int M, int dtype, int G,
@@ -2503,8 +2514,7 @@ static int check_fused_router_args(const char* who, const void* x,
   // (the one-launch tail keeps per-block slot prefixes in 16 bits)
   MOE_REQUIRE(S <= GATE_MAX_GROUP, MESH_MOE_E_UNSUPPORTED,
               "%s: group size S=%d > %d", who, S, GATE_MAX_GROUP);
-  MOE_REQUIRE(dtype == MESH_MOE_BF16 && M % 64 == 0 && E % 4 == 0 && E <= 128 &&
-                  S % 128 == 0 && tokens % S == 0 &&
+  MOE_REQUIRE(fused_router_shapes(M, E, S, dtype) && tokens % S == 0 &&
                   (int64_t)128 * M < (1LL << 31) &&
                   (((uintptr_t)x | (uintptr_t)w_packed) % 16 == 0),
               MESH_MOE_E_UNSUPPORTED,

@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 43
+ABI_VERSION = 44
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -233,6 +233,9 @@ _SIGNATURES = {
     "mesh_moe_shared_linear_backward_input": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, _vp]),
+    "mesh_moe_fused_router_supported": (ctypes.c_int, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "mesh_moe_top2_compacts": (ctypes.c_int, [ctypes.c_int, ctypes.c_int]),
     "mesh_moe_top2_layer_workspace_bytes": (ctypes.c_size_t, [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int, ctypes.c_int, ctypes.c_int]),
@@ -577,8 +580,9 @@ def top2_gating_static_scratch(logits, capacity, out, importance=None,
 
 def fused_gating_supported(x, num_experts, group_size):
   """True if mesh_moe_router_top2_gating has a kernel for this case."""
-  return (x.dtype == torch.bfloat16 and x.shape[-1] % 64 == 0 and
-          num_experts % 4 == 0 and num_experts <= 128 and group_size % 128 == 0)
+  return (x.dtype == torch.bfloat16 and
+          load_library().mesh_moe_fused_router_supported(
+              x.shape[-1], num_experts, group_size, BF16) == 1)
 
 
 def router_top2_gating(x, w_packed, group_size, capacity, importance=None,
@@ -1068,6 +1072,11 @@ def combine(y, r, group_size, out=None, row_offsets=None, loss_coef=None):
         _dev(r.kept, "kept", torch.uint8, (g, s, 2)), op, g, s, e, c, n, code,
         _stream()), "combine")
   return out
+
+
+def top2_compacts(groups, capacity):
+  """Whether a layer with two choices per token takes compact_expert_ffn."""
+  return load_library().mesh_moe_top2_compacts(groups, capacity) == 1
 
 
 def timing():

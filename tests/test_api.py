@@ -360,7 +360,8 @@ def test_library_exports_every_declared_symbol():
 
 
 # {version: what the declarations of the header hash to}
-_DECLARATIONS = {42: "ff364a62b8f3b800", 43: "fb4ec3a91e893039"}
+_DECLARATIONS = {42: "ff364a62b8f3b800", 43: "fb4ec3a91e893039",
+                 44: "9247610a552442fd"}
 
 
 def test_abi_version_counts_the_declarations():
@@ -372,6 +373,30 @@ def test_abi_version_counts_the_declarations():
   assert _DECLARATIONS.get(moe_hip.ABI_VERSION) == digest
   assert max(_DECLARATIONS) == moe_hip.ABI_VERSION
   assert len(set(_DECLARATIONS.values())) == len(_DECLARATIONS)
+
+
+def test_rules_of_the_layer_in_one_call_are_the_librarys(monkeypatch):
+  """Which calls a top-2 layer is made of stands in one place: the layer that makes them
+  one by one asks the library, whose one call follows the same rules."""
+  lib = moe_hip.load_library()
+  x = lambda m, dt=torch.bfloat16: torch.empty((1, 1, m), dtype=dt, device="meta")
+  for m in (32, 64, 96, 128):
+    for e in (2, 4, 126, 128, 132):
+      for s in (64, 128, 192, 256):
+        want = m % 64 == 0 and e % 4 == 0 and e <= 128 and s % 128 == 0
+        assert lib.mesh_moe_fused_router_supported(m, e, s, moe_hip.BF16) == want
+        assert not lib.mesh_moe_fused_router_supported(m, e, s, moe_hip.F32)
+        assert moe_hip.fused_gating_supported(x(m), e, s) == want
+        assert not moe_hip.fused_gating_supported(x(m, torch.float32), e, s)
+  for g, c in ((1, 255), (1, 256), (2, 128), (3, 128), (1 << 16, 1 << 15)):
+    assert moe_hip.top2_compacts(g, c) == (g * c % 256 == 0)
+
+  class Other(object):
+    mesh_moe_fused_router_supported = staticmethod(lambda *_: 1)
+    mesh_moe_top2_compacts = staticmethod(lambda *_: 1)
+  monkeypatch.setattr(moe_hip, "load_library", lambda: Other)
+  assert moe_hip.fused_gating_supported(x(33), 3, 5)
+  assert moe_hip.top2_compacts(1, 3)
 
 
 def test_compact_experts_decline_a_hidden_tensor_beyond_32_bits():
