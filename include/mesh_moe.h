@@ -30,7 +30,7 @@ extern "C" {
 #endif
 
 /* (counted up with every change of a declaration, and of what a call accepts) */
-#define MESH_MOE_ABI_VERSION 44
+#define MESH_MOE_ABI_VERSION 45
 
 /* element types of activations / weights */
 #define MESH_MOE_F32 0
@@ -970,9 +970,12 @@ int mesh_moe_residual_rms_norm_backward(
     double epsilon, int dtype, void* workspace, size_t workspace_bytes,
     void* stream);
 
-/* Bytes of scratch mesh_moe_self_attention needs. */
+/* Bytes of scratch mesh_moe_self_attention needs; the second, where q, k, v and out lie
+ * on 16 bytes (without the room for copies that do). */
 size_t mesh_moe_self_attention_workspace_bytes(int B, int L, int H, int D,
                                                int dtype, int relative_bias);
+size_t mesh_moe_self_attention_aligned_workspace_bytes(int B, int L, int H, int D,
+                                                       int dtype, int relative_bias);
 
 /*
  * Multi-head dot-product self-attention after the q/k/v projections

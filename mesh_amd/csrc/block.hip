@@ -1210,17 +1210,27 @@ static int copy_bf16(const void* from, void* to, int64_t n, hipStream_t st) {
   return 0;
 }
 
-extern "C" size_t mesh_moe_self_attention_workspace_bytes(int B, int L, int H,
-                                                          int D, int dtype,
-                                                          int relative_bias) {
+static size_t self_attention_workspace(int B, int L, int H, int D, int dtype,
+                                       int relative_bias, bool aligned) {
   if (B < 1 || L < 1 || H < 1 || D < 1 || !valid_dtype(dtype)) return 0;
   if (flash_attention_supported(L, H, D, dtype, nullptr, nullptr, nullptr,
                                 nullptr))
     return flash_attention_workspace_bytes(B, L, H, D, relative_bias != 0) +
-           (L % 8 != 0 ? 4 * aligned_copy_bytes(B, L, H, D) : 0);
+           (L % 8 != 0 && !aligned ? 4 * aligned_copy_bytes(B, L, H, D) : 0);
   const size_t b = dtype_size(dtype);
   const size_t hd = (size_t)B * H * L * D, ll = (size_t)B * H * L * L;
   return 4 * hd * b + ll * 4 + ll * b + 7 * 256;
+}
+
+extern "C" size_t mesh_moe_self_attention_workspace_bytes(int B, int L, int H,
+                                                          int D, int dtype,
+                                                          int relative_bias) {
+  return self_attention_workspace(B, L, H, D, dtype, relative_bias, false);
+}
+
+extern "C" size_t mesh_moe_self_attention_aligned_workspace_bytes(
+    int B, int L, int H, int D, int dtype, int relative_bias) {
+  return self_attention_workspace(B, L, H, D, dtype, relative_bias, true);
 }
 
 extern "C" int mesh_moe_self_attention(const void* q, const void* k,
@@ -1246,14 +1256,14 @@ extern "C" int mesh_moe_self_attention(const void* q, const void* k,
               MESH_MOE_E_ARG,
               "self_attention: rel_values, rel_bucket and num_buckets go "
               "together");
-  MOE_REQUIRE(workspace_bytes >= mesh_moe_self_attention_workspace_bytes(
-                                     B, L, H, D, dtype, rel_values != nullptr),
+  const bool aligned = flash_attention_supported(L, H, D, dtype, q, k, v, out);
+  MOE_REQUIRE(workspace_bytes >= self_attention_workspace(B, L, H, D, dtype,
+                                                          rel_values != nullptr, aligned),
               MESH_MOE_E_ARG, "self_attention: workspace too small");
   hipStream_t st = (hipStream_t)stream;
   if (flash_attention_supported(L, H, D, dtype, nullptr, nullptr, nullptr,
                                 nullptr)) {
     // fused kernel: the logits stay on chip
-    const bool aligned = flash_attention_supported(L, H, D, dtype, q, k, v, out);
     MOE_REQUIRE(aligned || L % 8 != 0, MESH_MOE_E_UNSUPPORTED,
                 "self_attention: q, k, v, out must be 16-byte aligned");
     if (!aligned) {

@@ -22,7 +22,7 @@ BF16 = 1
 POLICIES = {"all": 0, "none": 1, "threshold": 2, "random": 3}
 ACTIVATIONS = {None: 0, "linear": 0, "relu": 1, "gelu": 2, "sigmoid": 3,
                "tanh": 4, "swish": 5}
-ABI_VERSION = 44
+ABI_VERSION = 45
 
 _vp = ctypes.c_void_p
 _SIGNATURES = {
@@ -253,6 +253,9 @@ _SIGNATURES = {
     "mesh_moe_rms_norm": (ctypes.c_int, [
         _vp, _vp, _vp, ctypes.c_int64, ctypes.c_int, ctypes.c_double,
         ctypes.c_int, _vp]),
+    "mesh_moe_self_attention_aligned_workspace_bytes": (ctypes.c_size_t, [
+        ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+        ctypes.c_int]),
     "mesh_moe_self_attention_workspace_bytes": (ctypes.c_size_t, [
         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
         ctypes.c_int]),
@@ -1696,8 +1699,10 @@ def self_attention(q, k, v, num_heads, causal, sequence_id=None,
   lse = None
   if return_lse:
     lse = torch.empty((b * num_heads, l), dtype=torch.float32, device=q.device)
-  ws_bytes = lib.mesh_moe_self_attention_workspace_bytes(
-      b, l, num_heads, d, code, int(relative_bias is not None))
+  workspace_of = (lib.mesh_moe_self_attention_workspace_bytes
+                  if (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16 else
+                  lib.mesh_moe_self_attention_aligned_workspace_bytes)
+  ws_bytes = workspace_of(b, l, num_heads, d, code, int(relative_bias is not None))
   ws = torch.empty((max(ws_bytes, 1),), dtype=torch.uint8, device=q.device)
   with _stage("self_attention"):
     _check(lib.mesh_moe_self_attention(

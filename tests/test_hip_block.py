@@ -656,6 +656,29 @@ def test_fused_attention_of_any_length(hip, length, d, causal, with_ids_and_bias
       np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
 
 
+@pytest.mark.parametrize("length", [1000, 1001])
+def test_fused_attention_holds_no_room_for_copies(hip, length):
+  """Operands on 16 bytes need no copies, whatever the length: beside what is returned
+  the call holds no tensor of their size, and the public size covers both cases."""
+  heads, d = 8, 64
+  q, k, v = (torch.randn((4, length, heads * d), device="cuda").bfloat16()
+             for _ in range(3))
+  size = q.numel() * q.element_size()
+  torch.cuda.synchronize()
+  before = torch.cuda.memory_allocated()
+  torch.cuda.reset_peak_memory_stats()
+  out = hip.self_attention(q, k, v, heads, True)
+  torch.cuda.synchronize()
+  assert size <= torch.cuda.max_memory_allocated() - before <= size * 1.25
+  moved = torch.empty(q.numel() + 1, dtype=q.dtype, device="cuda")[1:].view(q.shape)
+  moved.copy_(q)
+  if length % 8:
+    assert torch.equal(hip.self_attention(moved, k, v, heads, True), out)
+  else:
+    with pytest.raises(hip.MoeHipError, match="16-byte"):
+      hip.self_attention(moved, k, v, heads, True)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("length", [24, 25, 131])
 def test_fused_attention_of_infinite_logits(hip, length, d):
