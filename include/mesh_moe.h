@@ -348,14 +348,14 @@ int mesh_moe_dispatched_expert_ffn(
 /* The same where every expert has `outer` kernels, wi_packed [E*outer,H,M] and wo_packed
  * [E*outer,N,H], kernel e * outer + o for the groups from o * G / outer on (the inner level
  * of transformer_moe_layer_v2, transformer/moe.py:743-793): y [E*outer, G/outer*C, N].
- * fill [G,E] as the gating left it.  No kernel for at most 64 rows per expert. */
+ * fill [G,E] as the gating left it.  Only where the first GEMM of G/outer*C rows, 128 at
+ * least, fits the 256 x 256 kernel. */
 int mesh_moe_dispatched_outer_expert_ffn(
     const void* x, const int32_t* idx, const int32_t* pos, const float* gate,
     const uint8_t* kept, const int32_t* fill, const void* wi_packed,
     const void* wo_packed, void* h, void* y, void* workspace, size_t workspace_bytes,
     int G, int S, int E, int C, int outer, int M, int H, int N, int activation, int dtype,
     void* stream);
-
 
 /*
  * Combine: out[g,s,:] = w1 * y[idx1,g,pos1,:] + w2 * y[idx2,g,pos2,:] with
@@ -988,10 +988,11 @@ size_t mesh_moe_self_attention_aligned_workspace_bytes(int B, int L, int H, int 
  *   q, k, v, out [B,L,H*D] dtype (heads and d_kv combined as the reference's
  *   combine_dims does); any L and D (bf16 shapes of the three-step form whose L or D
  *   is not a multiple of 8 run their two products on a plain tile kernel).
- * bf16 with D = 64 or 128 and L >= 8 runs one fused kernel (logits stay on chip, the
- * division by the softmax sum comes after the weights are rounded; no scratch
- * but the bias table below, and room for copies of operands off 16 bytes, which are
- * taken where L is no multiple of 8).  Other cases run the three-step form whose logits
+ * bf16 with D = 64 or 128 and L >= 8 runs one fused kernel (logits stay on chip; no
+ * scratch but the bias table below, and room for copies of operands off 16 bytes, which
+ * are taken where L is no multiple of 8).  Where L is a multiple of 8 the division by the
+ * softmax sum comes after the weights are rounded; other lengths divide first, as the
+ * three-step form does, and walk the keys twice for it.  Other cases run the three-step form whose logits
  * and weights of all heads live in the workspace (B*H*L*L*(4 + sizeof dtype)
  * bytes).
  * sequence_id [B,L] int32 or NULL: with it a query sees only the keys that

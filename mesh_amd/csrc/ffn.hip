@@ -1112,9 +1112,11 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
     for (int kk = 0; kk < KSTEPS; ++kk) {
       const int cur = kk & 1, nxt = cur ^ 1;
       kk_now = kk;
-      // The loads a step carries: the four weight loads of the K tile after the
-      // next over steps 0..2, all four token loads of it right behind the
-      // hand-over barrier that frees their slot (a full K tile ahead of use).
+      // The loads a step carries.  Two token slots: the four weight loads of the K
+      // tile after the next over steps 0..2, all four token loads of it in step 3,
+      // behind the hand-over barrier that frees their slot (a full K tile ahead of
+      // use).  DEEP: all seven of them over steps 0..2, into slots that the hand-over
+      // barrier of the K tile before freed (step 3 carries none).
       auto load = [&](int which) {
         if constexpr (DEEP) {
           const int n = 2 * kk + which;       // 0 .. 6
@@ -1152,8 +1154,9 @@ __global__ __launch_bounds__(RingCfg::THREADS) void grouped_gemm_bf16_ring_kerne
         if (DEEP && kk == 2) { load(2); fence(); }
         mm(cur, 7); fence();
       } else {
-        // this lane holds the last step's fragments (lgkmcnt 0); everything
-        // but the four weight loads of tile kt+2 has landed (vmcnt 4)
+        // this lane holds the last step's fragments (lgkmcnt 0); everything but the
+        // loads of tile kt+2 that are out has landed: the four weight loads, whose
+        // token loads follow this barrier (vmcnt 4), DEEP all seven (vmcnt 7)
         fence();
         constexpr int AHEAD = DEEP ? A_LOADS + Cfg::B_INSTR : Cfg::B_INSTR;
         __builtin_amdgcn_s_waitcnt((AHEAD & 15) | (0 << 8) | (7 << 4));
