@@ -1069,7 +1069,9 @@ size_t mesh_moe_self_attention_backward_workspace_bytes(int B, int L, int H,
  * out [B,L,H*D] dtype and lse [B*H,L] float32 (both or neither): what
  * mesh_moe_self_attention wrote for the same arguments.  With them the first
  * of the four launches is replaced by a small one (delta = sum_d dout out from
- * the rounded outputs); without them the denominators are recomputed.
+ * the rounded outputs); without them the denominators are recomputed.  Where L is no
+ * multiple of 8 delta is sum_k dW W / sum_k W in float32 in both cases, from a pass over
+ * the keys of its own.
  */
 int mesh_moe_self_attention_backward(const void* q, const void* k, const void* v,
                                      const void* dout, void* dq, void* dk,

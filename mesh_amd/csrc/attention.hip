@@ -860,7 +860,14 @@ int flash_attention(const void* q, const void* k, const void* v, void* out,
 // streamed tile that is read both ways (K in BWD_DQ, Q in BWD_DK, Q and dout in
 // BWD_DKV) is loaded into LDS twice, once per swizzle.
 // ---------------------------------------------------------------------------
-enum { BWD_DQ = 0, BWD_DK = 1, BWD_DV = 2, BWD_DKV = 3 };
+// Before them, for lengths that are no multiple of 8:
+//   BWD_DELTA  a lane owns a query; walks key tiles: delta = sum W dW / sum W
+// A sum dout . out of outputs that are rounded to bf16 is further off than the weights and
+// their gradients of the three-step form, which these lengths had: 2 x 1001 positions, 4
+// heads of 64, logits around 64, dq was 0.91 % off float64 with it, three-step 0.59, now
+// 0.24; around 4 0.40, 0.34 and 0.24.  The pass is bound as the others by its products and
+// exponentials: 7 x 1385 positions, 8 heads of 64, causal, all gradients 107 -> 132 us.
+enum { BWD_DQ = 0, BWD_DK = 1, BWD_DV = 2, BWD_DKV = 3, BWD_DELTA = 4 };
 
 template <int D>
 struct FlashBwdCfg {
@@ -877,7 +884,7 @@ struct FlashBwdCfg {
   static constexpr int STATS_BYTES = BIAS_AT + 320 * 4;
   static constexpr int RING = 512;                  // floats, see dwin below
   static constexpr int copies(int what) {
-    return what == BWD_DV ? 2 : what == BWD_DKV ? 4 : 3;
+    return what == BWD_DV || what == BWD_DELTA ? 2 : what == BWD_DKV ? 4 : 3;
   }
   static constexpr int stage_bytes(int what) {
     return copies(what) * TILE + STATS_BYTES;
@@ -889,7 +896,8 @@ struct FlashBwdCfg {
 
 // BIAS: the logits are recomputed with the relative attention bias (tab as
 // in the forward kernel); BWD_DQ also sums its dS along the diagonals into
-// dtab [H, 2L-1] (float atomics), the gradient of tab.
+// dtab [H, 2L-1] (float atomics), the gradient of tab.  grad: what WHAT says, bf16 rows;
+// BWD_DELTA delta_out instead.
 template <int D, bool CAUSAL, int WHAT, bool SEQ, bool BIAS>
 __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
@@ -897,9 +905,11 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     const float* __restrict__ lse, const float* __restrict__ delta,
     bf16_t* __restrict__ grad, bf16_t* __restrict__ grad_v, int L, int H,
     const int32_t* __restrict__ seq, const float* __restrict__ tab,
-    float* __restrict__ dtab) {
+    float* __restrict__ dtab, float* __restrict__ delta_out) {
   using Cfg = FlashBwdCfg<D>;
-  constexpr bool OWN_Q = WHAT == BWD_DQ, BOTH = WHAT == BWD_DKV;
+  constexpr bool DELTA = WHAT == BWD_DELTA;
+  constexpr bool OWN_Q = WHAT == BWD_DQ || DELTA, BOTH = WHAT == BWD_DKV;
+  constexpr bool SUM_BIAS = BIAS && WHAT == BWD_DQ;
   constexpr int NCOPY = Cfg::copies(WHAT);
   constexpr int STAGE = Cfg::stage_bytes(WHAT);
   constexpr float LOG2E = 1.4426950408889634f;
@@ -947,7 +957,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
   float my_lse2 = 0.f, my_delta = 0.f;
   if constexpr (OWN_Q) {
     my_lse2 = lse_b[my_c] * LOG2E;
-    my_delta = delta_b[my_c];
+    if constexpr (!DELTA) my_delta = delta_b[my_c];
   }
   const int32_t* seq_b = SEQ ? seq + (int64_t)b * L : nullptr;
   int my_sid = 0, own_first = 0;
@@ -993,6 +1003,8 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     load_copy(str1, row0, base, std::false_type());
     if constexpr (WHAT == BWD_DV) {
       load_copy(str2, row0, base + Cfg::TILE, std::true_type());
+    } else if constexpr (DELTA) {
+      load_copy(str2, row0, base + Cfg::TILE, std::false_type());
     } else {
       load_copy(str1, row0, base + Cfg::TILE, std::true_type());
       load_copy(str2, row0, base + 2 * Cfg::TILE, std::false_type());
@@ -1045,7 +1057,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
   // later).
   float* dwin = reinterpret_cast<float*>(fb_smem + 2 * STAGE);
   float* dtab_h = nullptr;
-  if constexpr (BIAS && OWN_Q) {
+  if constexpr (SUM_BIAS) {
     dtab_h = dtab + (int64_t)h * (2 * L - 1);
     if (tid < Cfg::RING) dwin[tid] = 0.f;
   }
@@ -1057,6 +1069,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     if (val != 0.f && d >= 0 && d <= 2 * L - 2) atomicAdd(dtab_h + d, val);
   };
   float ra0 = 0.f, ra1 = 0.f, ra2 = 0.f;
+  float sum_w = 0.f, sum_wd = 0.f;         // DELTA: over this half-wave's keys
   const int rot_m = l32 + 4 * half;        // lane m takes key column c from lane
   const int rot_hb = half << 7;            // (m + c) mod 32 of its half-wave
 
@@ -1091,7 +1104,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     if (t + 1 < t_end) load_tile(t + 1, buf ^ 1);
     const int row0 = t * Cfg::BT;
     const unsigned char* t1r = fb_smem + buf * STAGE;
-    const unsigned char* t2r = t1r + 2 * Cfg::TILE;           // all but BWD_DV
+    const unsigned char* t2r = t1r + (DELTA ? 1 : 2) * Cfg::TILE;   // all but BWD_DV
     const uint32_t ttr = lds0 + buf * STAGE + Cfg::TILE;      // the copy read transposed
     const float* st = reinterpret_cast<const float*>(t1r + NCOPY * Cfg::TILE);
     bool need_mask =
@@ -1109,7 +1122,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
       bw = reinterpret_cast<const float*>(t1r + NCOPY * Cfg::TILE + Cfg::BIAS_AT) +
            (OWN_Q ? Cfg::BOWN - 1 - (wave * 32 + l32)
                   : wave * 32 + l32 + Cfg::BT - 1);
-    if constexpr (BIAS && OWN_Q) {
+    if constexpr (SUM_BIAS) {
       if (t > t_begin && wave == ((t - 1) & 7)) flush_dwin(t - 1);
     }
 
@@ -1149,8 +1162,14 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
       }
       // weights (and their gradient) of this lane's own entity against the
       // 16 streamed rows SUB * 32 + 8 (r / 4) + 4 half + r % 4
-      float w[16], wv[BOTH ? 16 : 1];
-      if constexpr (OWN_Q) {
+      float w[16], wv[BOTH || DELTA ? 16 : 1];
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          w[r] = fa_exp2(fmaf(acc_s[r], LOG2E, -my_lse2));
+          wv[r] = w[r] * acc_dp[r];
+        }
+      } else if constexpr (OWN_Q) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float p = fa_exp2(fmaf(acc_s[r], LOG2E, -my_lse2));
@@ -1193,12 +1212,20 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
                             (!CAUSAL || (OWN_Q ? sr <= my : my <= sr)) &&
                             (!SEQ || sid4[c] == my_sid);
             if (!ok) w[4 * r4 + c] = 0.f;
-            if constexpr (BOTH)
+            if constexpr (BOTH || DELTA)
               if (!ok) wv[4 * r4 + c] = 0.f;
           }
         }
       }
-      if constexpr (BIAS && OWN_Q) {
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          sum_w += w[r];
+          sum_wd += wv[r];
+        }
+        return;
+      }
+      if constexpr (SUM_BIAS) {
         if (ow_last >= L) {          // rows past the end carry no gradient
           asm volatile("" ::: "memory");
 #pragma unroll
@@ -1270,7 +1297,7 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     };
     do_sub(std::integral_constant<int, 0>());
     do_sub(std::integral_constant<int, 1>());
-    if constexpr (BIAS && OWN_Q) {
+    if constexpr (SUM_BIAS) {
       // the lower half-wave hands in n = 0 (e = -m), the upper one n = 1
       // (e = 32 - m), each the sum of both halves' accumulators
       const float got = __shfl_xor(half == 0 ? ra1 : ra0, 32);
@@ -1285,7 +1312,13 @@ __global__ __launch_bounds__(512) void flash_attention_backward_kernel(
     __builtin_amdgcn_s_waitcnt(0x0070 | (15 << 8));   // vmcnt(0): tile t+1 is here
     __syncthreads();
   }
-  if constexpr (BIAS && OWN_Q) {
+  if constexpr (DELTA) {
+    sum_w += __shfl_xor(sum_w, 32);
+    sum_wd += __shfl_xor(sum_wd, 32);
+    if (my < L && half == 0) delta_out[(int64_t)bh * L + my] = sum_wd / sum_w;
+    return;
+  }
+  if constexpr (SUM_BIAS) {
     // n = 2 of the last tile, then what its window still holds: five chunks
     if (t_end > t_begin) {
       const int rel = t_end * Cfg::BT + Cfg::BOWN - 1 - 32 * wave - l32;
@@ -1320,7 +1353,8 @@ static int launch_flash_backward_one(const bf16_t* q, const bf16_t* k,
                                      const float* lse, const float* delta,
                                      bf16_t* grad, bf16_t* grad_v, int B, int L,
                                      int H, const int32_t* seq, const float* tab,
-                                     float* dtab, hipStream_t st) {
+                                     float* dtab, hipStream_t st,
+                                     float* delta_out = nullptr) {
   using Cfg = FlashBwdCfg<D>;
   constexpr int LDS = 2 * Cfg::stage_bytes(WHAT) +
                       (BIAS && WHAT == BWD_DQ ? Cfg::RING * 4 : 0);
@@ -1328,7 +1362,7 @@ static int launch_flash_backward_one(const bf16_t* q, const bf16_t* k,
   auto kern = flash_attention_backward_kernel<D, CAUSAL, WHAT, SEQ, BIAS>;
   MOE_ALLOW_LDS(kern, LDS);
   kern<<<grid, Cfg::THREADS, LDS, st>>>(q, k, v, dout, lse, delta, grad, grad_v,
-                                        L, H, seq, tab, dtab);
+                                        L, H, seq, tab, dtab, delta_out);
   MOE_CHECK_LAUNCH("self_attention_backward (fused)");
   return 0;
 }
@@ -1393,7 +1427,8 @@ __global__ __launch_bounds__(256) void attention_delta_kernel(
 
 // lse_saved / out_saved: the forward pass's softmax denominators and outputs
 // when the caller kept them; otherwise a pass in the forward kernel's shape
-// recomputes the denominators (and delta from the unrounded outputs).
+// recomputes the denominators (and delta from the unrounded outputs).  Lengths that are
+// no multiple of 8 have their delta from BWD_DELTA in both cases.
 template <int D, bool CAUSAL, bool SEQ, bool BIAS>
 static int launch_flash_backward(const bf16_t* q, const bf16_t* k,
                                  const bf16_t* v, const bf16_t* dout,
@@ -1403,12 +1438,9 @@ static int launch_flash_backward(const bf16_t* q, const bf16_t* k,
                                  float* dtab, const bf16_t* out_saved,
                                  const float* lse_saved, hipStream_t st) {
   using Cfg = FlashCfg<D>;
-  if (out_saved != nullptr) {
-    const int64_t items = (int64_t)B * L * H;
-    attention_delta_kernel<D><<<(unsigned)((items * 16 + 255) / 256), 256, 0,
-                                st>>>(dout, out_saved, delta, items, L, H);
-    MOE_CHECK_LAUNCH("self_attention_backward (delta)");
-  } else {
+  const bool exact_delta = L % 8 != 0;
+  const float* lse_use = out_saved != nullptr ? lse_saved : lse;
+  if (out_saved == nullptr) {
     constexpr int LDS = Cfg::LDS_BYTES + 512 + 1536;
     dim3 grid((unsigned)((L + Cfg::BQ - 1) / Cfg::BQ), (unsigned)(B * H));
     auto stats = flash_attention_kernel<D, CAUSAL, true, SEQ, BIAS>;
@@ -1416,8 +1448,18 @@ static int launch_flash_backward(const bf16_t* q, const bf16_t* k,
     stats<<<grid, Cfg::THREADS, LDS, st>>>(q, k, v, nullptr, L, H, dout, lse,
                                            delta, seq, tab);
     MOE_CHECK_LAUNCH("self_attention_backward (lse, delta)");
+  } else if (!exact_delta) {
+    const int64_t items = (int64_t)B * L * H;
+    attention_delta_kernel<D><<<(unsigned)((items * 16 + 255) / 256), 256, 0,
+                                st>>>(dout, out_saved, delta, items, L, H);
+    MOE_CHECK_LAUNCH("self_attention_backward (delta)");
   }
-  const float* lse_use = out_saved != nullptr ? lse_saved : lse;
+  if (exact_delta) {
+    const int rc = launch_flash_backward_one<D, CAUSAL, BWD_DELTA, SEQ, BIAS>(
+        q, k, v, dout, lse_use, nullptr, nullptr, nullptr, B, L, H, seq, tab, nullptr,
+        st, delta);
+    if (rc != 0) return rc;
+  }
   return launch_flash_backward_all<D, CAUSAL, SEQ, BIAS>(
       q, k, v, dout, dq, dk, dv, lse_use, delta, B, L, H, seq, tab, dtab, st);
 }

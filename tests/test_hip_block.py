@@ -656,6 +656,60 @@ def test_fused_attention_of_any_length(hip, length, d, causal, with_ids_and_bias
       np.testing.assert_allclose(H.to_np(gt), wnt, rtol=3e-2, atol=3e-2 * scale)
 
 
+@pytest.mark.parametrize("with_ids_and_bias", [False, True])
+@pytest.mark.parametrize("scale", [0.5, 8.0, 60.0])
+@pytest.mark.parametrize("length,d,causal", [(65, 64, True), (257, 128, False),
+                                             (259, 64, False), (601, 128, True)])
+def test_gradients_of_any_length_are_as_exact_as_three_steps(hip, length, d, causal,
+                                                             scale, with_ids_and_bias):
+  """Lengths that are no multiple of 8, logits of a standard deviation of 4 to 700: the
+  fused backward, with kept denominators and outputs and without, is no further from
+  float64 than the three-step form that these lengths had."""
+  b, heads, nb = 2, 2, 8
+  rng = np.random.default_rng(length)
+  mk = lambda s, *sizes: O.cast_act(
+      (rng.standard_normal(sizes) * s).astype(np.float32), "bfloat16")
+  q, k = (mk(scale ** 0.5, b, length, heads * d) for _ in range(2))
+  v, do = (mk(1.0, b, length, heads * d) for _ in range(2))
+  sid = rel = None
+  to64 = lambda t: torch.from_numpy(np.asarray(t, np.float64)).reshape(
+      b, length, heads, d).transpose(1, 2).contiguous().requires_grad_()
+  q64, k64, v64 = to64(q), to64(k), to64(v)
+  logits = q64 @ k64.transpose(-1, -2)
+  values64 = None
+  if with_ids_and_bias:
+    ids = _packed_sequence_ids(rng, b, length, max(4, length // 3))
+    values = mk(1.0, heads, nb)
+    bucket = B.relative_position_bucket(np.arange(-(length - 1), length), not causal,
+                                        nb)
+    sid = torch.from_numpy(ids).cuda()
+    rel = (H.to_gpu(values, "bfloat16"), torch.from_numpy(bucket.astype(np.int32)).cuda())
+    values64 = torch.from_numpy(values.astype(np.float64)).requires_grad_()
+    at = torch.arange(length)
+    distance = at[None, :] - at[:, None] + length - 1
+    logits = logits + values64[:, torch.from_numpy(bucket).long()[distance]]
+    ids = torch.from_numpy(ids)
+    logits = logits.masked_fill(ids[:, None, :, None] != ids[:, None, None, :],
+                                float("-inf"))
+  if causal:
+    logits = logits.masked_fill(torch.ones(length, length).triu(1).bool(), float("-inf"))
+  out64 = logits.softmax(-1) @ v64
+  out64.backward(to64(do).detach())
+  want = [t.grad.transpose(1, 2).reshape(b, length, -1) for t in (q64, k64, v64)]
+  if values64 is not None:
+    want.append(values64.grad)
+  args = [H.to_gpu(t, "bfloat16") for t in (q, k, v, do)]
+  kw = dict(sequence_id=sid, relative_bias=rel)
+  out, lse = hip.self_attention(*args[:3], heads, causal, return_lse=True, **kw)
+  error = lambda grads: [float((g.double().cpu() - w).norm()) for g, w in zip(grads, want)]
+  three = error(hip.self_attention_backward(*args, heads, causal, fused=False, **kw))
+  for kept in (dict(), dict(out=out, lse=lse)):
+    fused = error(hip.self_attention_backward(*args, heads, causal, fused=True, **kept,
+                                              **kw))
+    # (dv has the same roundings in both: the same error but for chance)
+    assert all(f <= 1.05 * t for f, t in zip(fused, three)), (kept.keys(), fused, three)
+
+
 @pytest.mark.parametrize("length", [1000, 1001])
 def test_fused_attention_holds_no_room_for_copies(hip, length):
   """Operands on 16 bytes need no copies, whatever the length: beside what is returned
