@@ -10,6 +10,7 @@ raises, and so does every call.
 """
 
 import ctypes
+import functools
 import os
 
 import torch
@@ -581,11 +582,17 @@ def top2_gating_static_scratch(logits, capacity, out, importance=None,
   return out
 
 
+# (asked once for each set of sizes: a call of the library takes 0.6 us of an eager step)
+@functools.lru_cache(maxsize=1024)
+def _fused_router_sizes(m, num_experts, group_size):
+  return load_library().mesh_moe_fused_router_supported(
+      m, num_experts, group_size, BF16) == 1
+
+
 def fused_gating_supported(x, num_experts, group_size):
   """True if mesh_moe_router_top2_gating has a kernel for this case."""
   return (x.dtype == torch.bfloat16 and
-          load_library().mesh_moe_fused_router_supported(
-              x.shape[-1], num_experts, group_size, BF16) == 1)
+          _fused_router_sizes(x.shape[-1], num_experts, group_size))
 
 
 def router_top2_gating(x, w_packed, group_size, capacity, importance=None,
@@ -1077,6 +1084,7 @@ def combine(y, r, group_size, out=None, row_offsets=None, loss_coef=None):
   return out
 
 
+@functools.lru_cache(maxsize=1024)
 def top2_compacts(groups, capacity):
   """Whether a layer with two choices per token takes compact_expert_ffn."""
   return load_library().mesh_moe_top2_compacts(groups, capacity) == 1

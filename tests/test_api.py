@@ -395,8 +395,13 @@ def test_rules_of_the_layer_in_one_call_are_the_librarys(monkeypatch):
     mesh_moe_fused_router_supported = staticmethod(lambda *_: 1)
     mesh_moe_top2_compacts = staticmethod(lambda *_: 1)
   monkeypatch.setattr(moe_hip, "load_library", lambda: Other)
-  assert moe_hip.fused_gating_supported(x(33), 3, 5)
-  assert moe_hip.top2_compacts(1, 3)
+  rules = (moe_hip._fused_router_sizes, moe_hip.top2_compacts)
+  try:
+    assert moe_hip.fused_gating_supported(x(33), 3, 5)
+    assert moe_hip.top2_compacts(1, 3)
+  finally:
+    for rule in rules:
+      rule.cache_clear()
 
 
 def test_compact_experts_decline_a_hidden_tensor_beyond_32_bits():
