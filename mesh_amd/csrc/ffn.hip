@@ -2082,18 +2082,21 @@ static unsigned ring_blocks(int64_t tiles, int cus) {
 // The persistent blocks take whole rounds of tiles, so what counts is rounds
 // times the time of a tile, and a tile of fewer 32-row pieces is cheaper: about
 // 0.40 + 0.13 per piece us per K tile (0.20 + 0.14 with three token slots, no less than
-// 0.6 and 0.5) and 5 us outside the K loop.  Rows are spread evenly over the row tiles:
-// 640 rows per expert are three tiles of 224 or four of 160, not 256 + 256 + 128.  In more
-// than one round the row tiles of an expert do not run side by side, and each reads its
-// weights again: no less than 9 TB/s takes for all of them.  (Without that term three low
-// tiles in two rounds were chosen over one tile in one where the weights set the pace: 32
-// x 240 rows, 2304 -> 1152 68 us, one tile 58; 32 x 166, 4608 -> 1152 125 and 99.  One
-// round of low tiles reads them once from memory: 12 x 152, 4608 -> 1536 61 in tiles of
-// 64, 64 in tiles of 96.)  Of 394 products of 1 to 128 experts, 128 to 16000 rows, K and N
-// 512 to 8192, timed with every height from 64 on, the rule's choice is 0.3 % slower than
-// the best one on average, by more than 3 % in 16 and by 9 % at worst (24 x 417 rows, 8192
-// -> 2048: 224 rows 370 us, 128 338).  Tiles of 256 and a shorter last one -> the rule's
-// choice (both sides bit-identical):
+// 0.6 and 0.5) and 5 us outside the K loop, 4.5 of a single piece.  Rows are spread
+// evenly over the row tiles: 640 rows per expert are three tiles of 224 or four of 160,
+// not 256 + 256 + 128.  In more than one round the row tiles of an expert do not run
+// side by side, and each reads its weights again: no less than 9 TB/s takes for all of
+// them.  (Without that term three low tiles in two rounds were chosen over one tile in
+// one where the weights set the pace: 32 x 240 rows, 2304 -> 1152 68 us, one tile 58;
+// 32 x 166, 4608 -> 1152 125 and 99.  One round of low tiles reads them once from
+// memory: 12 x 152, 4608 -> 1536 61 in tiles of 64, 64 in tiles of 96.  70 products
+// whose tiles of 32 rows fit into one round, which 64 were chosen for: with K below
+// 1600 all are 4 to 8 % faster in 32, 2 x 570 rows, 832 -> 384 9.6 us and 8.9; others
+// between 17 % faster and 3.5 % slower.)  Of 394 products of 1 to 128 experts, 128 to
+// 16000 rows, K and N 512 to 8192, timed with every height from 64 on, the rule's
+// choice is 0.3 % slower than the best one on average, by more than 3 % in 16 and by 9
+// % at worst (24 x 417 rows, 8192 -> 2048: 224 rows 370 us, 128 338).  Tiles of 256 and
+// a shorter last one -> the rule's choice (both sides bit-identical):
 //   32 x 640 rows, 4096 x 1024 (160 rows; of 224 186 us)       197 -> 155 us
 //   16 x 708 rows, 768 x 3072 (192 rows) / 3072 x 768 (160)  67 / 56 -> 53 / 51
 //   8 x 900 rows, 1536 x 4608 (192 rows)                        111 -> 93
@@ -2136,7 +2139,7 @@ static int ring_tile_rows(int E, int R, int N, int K, int cus,
                               : deep ? 0.20 + 0.14 * pieces
                                      : 0.40 + 0.13 * pieces;
     const double least = deep ? 0.5 : 0.6;
-    const double outside = kmajor ? 3.3 + 0.75 * pieces : 5.0;
+    const double outside = kmajor ? 3.3 + 0.75 * pieces : pieces == 1 ? 4.5 : 5.0;
     const double limited = deep && long_launch ? 1.10 : 1.0;
     double cost = limited * (double)((tiles + cus - 1) / cus) *
                   (nk * (per_k_tile < least ? least : per_k_tile) + outside);
